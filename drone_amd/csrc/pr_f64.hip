@@ -7,6 +7,7 @@
 // iteration) and accumulates d_k, so one iteration touches: row_ptr 8N, col_idx 4E, gather source 8N,
 // inv_outdeg 8N, c_k 8N  =  4E + 32N bytes.
 #include "pr_rowblock.h"
+#include "pr_sell.h"
 #include "relabel.h"
 #include "spmv_merge.h"
 
@@ -118,7 +119,9 @@ struct drone_pr_plan {
     const double *inv_user = nullptr;  // caller's inverse out-degree, caller's vertex order
     Relabel rl;                        // hot-first copy of the CSR; all work vectors use its id space
     double *inv = nullptr;             // inverse out-degree in internal order
-    int deterministic = 0;             // 1: merge-path tiles (bit-reproducible); 0: source-sorted row blocks
+    bool sell = false;                 // small matrix: one launch per iteration (pr_sell.h), bit-reproducible in any mode
+    SellRows sr;
+    int deterministic = 0;             // else 1: merge-path tiles (bit-reproducible); 0: source-sorted row blocks
     RowBlocks rb;
     int units = 0;                     // tiles or blocks of the active mode
     MergeTiling mt;
@@ -161,6 +164,9 @@ extern "C" int drone_pr_plan_create_ex(drone_pr_plan **out, int64_t n, int64_t n
     hipStream_t s = as_stream(stream);
     const auto build = [&]() -> int {
         DRONE_HIP_TRY(hipGetDevice(&p->device));
+        // the two tuning overrides ask for row blocks of any size
+        p->sell = (flags & (DRONE_PR_SHARED_BLOCKS | DRONE_PR_WHOLE_BLOCKS)) == 0 && sell_suits(n, nnz);
+        if (p->sell) return sell_create(&p->sr, n, nnz, row_ptr, col_idx, s);
         int rc = relabel_create(&p->rl, n, nnz, row_ptr, col_idx, inv_outdeg, s);
         if (rc != DRONE_OK) return rc;
         p->rows = n;
@@ -214,6 +220,7 @@ extern "C" int drone_pr_plan_create_ex(drone_pr_plan **out, int64_t n, int64_t n
 extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
 {
     if (!p) return DRONE_OK;
+    sell_destroy(&p->sr);
     merge_tiling_destroy(&p->mt);
     merge_scratch_destroy(&p->ms);
     row_blocks_destroy(&p->rb);
@@ -294,6 +301,16 @@ extern "C" int drone_pr_run_f64(drone_pr_plan *p, double alpha, int iters, doubl
         return DRONE_OK;
     }
     // the caller may have refreshed inv_outdeg since the plan was made: re-read it every run (8N bytes)
+    if (p->sell) {
+        int rc = sell_begin(p->sr, p->inv_user, s);
+        for (int it = 0; it < iters && rc == DRONE_OK; ++it) {
+            const bool prof = p->prof_n < p->prof_cap;
+            if (prof) DRONE_HIP_TRY(hipEventRecord(p->ev0[p->prof_n], s));
+            rc = sell_iterate(p->sr, it, alpha, it == iters - 1 ? rank_out : nullptr, s);
+            if (prof) DRONE_HIP_TRY(hipEventRecord(p->ev1[p->prof_n++], s));
+        }
+        return rc;
+    }
     { int rc = relabel_gather_f64(p->rl, p->inv_user, p->inv, s); if (rc != DRONE_OK) return rc; }
     pr_f64_init_kernel<<<p->init_blocks, kSpmvBlock, 0, s>>>(p->n, p->inv, inv_n, p->c[0], p->init_part);
     reduce_stat_kernel<0><<<1, kSpmvBlock, 0, s>>>(p->init_part, p->init_blocks, p->dang);

@@ -1,0 +1,60 @@
+// fp64 pull PageRank of small and mid-size matrices: one launch per iteration.
+//
+// Such an iteration is bound by latency, not by bytes: R-MAT scale 12 / 16 (53 K / 955 K entries) took 17.1 / 18.7 us as
+// two launches of the row-block path (zero 128 KB of accumulators, sweep, epilogue; then the fix-up with its two-level
+// tickets for the dangling mass), where a launch that follows another on a stream costs 2.3 us and the bytes less than
+// one.  Here a row belongs to one wavefront (or, a hub row, to one work-group), so nothing straddles and nothing is left
+// to fix up, and the dangling mass travels as one partial per work-group that EVERY work-group of the next launch adds
+// up for itself - a few KB out of L2, in flight beside the entries.
+//
+// Layout.  Rows are sorted by length, longest first, and that order is the plan's vertex order (sources are renumbered
+// alike, so an iteration writes the next gather source with coalesced stores).  A row of L entries gets P = 1 ... 64
+// lanes, the power of two that leaves a lane at most kSellDepth entries; 64 / P neighbouring rows form a slice, one
+// wavefront.  A slice's entries are stored step by step, 64 consecutive source ids per step (lane = row in slice * P + q
+// takes the row's entries q, q + P, ...), padded to the longest row of the slice - the first, and its neighbours in the
+// sort are about as long - with the id of a source that is always 0.  Rows of more than 64 * kSellWaveSteps entries are
+// hubs: a work-group each, T consecutive ids per step.  Every sum has a fixed order, so the results are bitwise repeatable.
+//
+// Measured, R-MAT edge factor 16, us per iteration (row blocks before, this): 1 K vertices 11.6 -> 4.05, 4 K 17.1 -> 4.7,
+// 16 K 18.3 -> 4.9, 64 K 19.4 -> 9.1, 131 K 24.0 -> 14.2, 262 K 32.1 -> 24.3, 524 K 43.8 -> 41.3; the plan takes
+// 0.13 ... 1.2 ms instead of 0.3 ... 2.7 ms.  Below 16 K vertices it is a launch (2.3 us) plus one chain of slice
+// descriptor, ids, gathers and the partials' sum out of a cold L2; at 64 K and more the rate of gathers that hit L2.
+// Lanes of 4 or 16 entries (kSellDepth) instead of 8: 10.0 / 9.3 us at 64 K.
+#pragma once
+#include "common.h"
+
+namespace drone {
+
+constexpr int kSellClasses = 7;      // P = 64, 32, ..., 1
+constexpr int kSellDepth = 8;        // most entries of a lane in a slice with P < 64; gathers in flight per lane
+constexpr int kSellWaveSteps = 16;   // most steps of a slice with P = 64: longer rows are hubs
+
+struct SellRows {
+    int64_t n = 0, nnz = 0;
+    int threads = 256;               // work-group size of the iteration, 256 or 512
+    int hubs = 0, slices = 0, blocks = 0;
+    int row_begin[kSellClasses + 1] = {};    // first row of the class (row_begin[kSellClasses] = n)
+    int slice_begin[kSellClasses + 1] = {};  // first slice of the class
+    int32_t *order = nullptr;        // device [n]: row -> caller's id
+    int32_t *hub_step = nullptr;     // device [hubs + 1]: first step (of `threads` ids) of a hub row in hub_col
+    int4 *slice = nullptr;           // device [slices]: {first step (of 64 ids) in col, steps, first row, rows << 3 | log2 P}
+    int32_t *hub_col = nullptr;
+    int32_t *col = nullptr;
+    double *c[2] = {nullptr, nullptr};     // device [n + 1]: gather sources; [n] stays 0
+    double *inv = nullptr;           // device [n]: inverse out-degrees in row order, refreshed by every run
+    double *part[2] = {nullptr, nullptr};  // device: dangling mass per work-group, of this iteration and the one before
+    int init_blocks = 0;
+    DeviceArena arena;               // everything above
+    DeviceArena entries;             // hub_col and col, whose sizes are known last
+};
+
+// Whether the layout suits the matrix (n rows, nnz entries).
+bool sell_suits(int64_t n, int64_t nnz);
+int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, const int32_t *col, hipStream_t stream);
+void sell_destroy(SellRows *sr);
+// The two kinds of launch of a run: sell_begin reads the caller's inverse out-degrees, makes the first gather source and
+// its dangling mass; sell_iterate is one iteration (it = 0, 1, ...), the last of which passes rank_out.
+int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t stream);
+int sell_iterate(const SellRows &sr, int it, double alpha, double *rank_out, hipStream_t stream);
+
+}  // namespace drone

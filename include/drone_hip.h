@@ -153,11 +153,13 @@ int drone_pr_plan_create(drone_pr_plan **plan, int64_t n, int64_t nnz, const int
 /* Same with flags.  By default the aggregation runs over row blocks whose entries are sorted by source
  * (fastest; row sums are added in LDS in no fixed order, so the last bits may differ between runs, as
  * with the reference's float atomics).  DRONE_PR_DETERMINISTIC selects the merge-path kernel, whose
- * results are bitwise reproducible. */
+ * results are bitwise reproducible.  Small matrices (rows + entries up to 9 Mi) get a layout of their own in
+ * either mode, one launch per iteration and bitwise reproducible. */
 #define DRONE_PR_DETERMINISTIC 1
 /* Tuning overrides of the default mode.  Row blocks of a large matrix (about 50 M entries and more) are shared by up
  * to four work-groups, which then find more entries per cache line of the gather source; small matrices keep one
- * work-group per block.  DRONE_PR_SHARED_BLOCKS forces sharing, DRONE_PR_WHOLE_BLOCKS forbids it.  (The sweep keeps
+ * work-group per block.  DRONE_PR_SHARED_BLOCKS forces sharing, DRONE_PR_WHOLE_BLOCKS forbids it; either also asks for row
+ * blocks where the matrix is small.  (The sweep keeps
  * four 64-entry batches in flight per wavefront, six where a work-group sweeps a million entries;
  * DRONE_PR_SWEEP_DEPTH=4 or 6 in the environment at plan creation fixes that choice.) */
 #define DRONE_PR_SHARED_BLOCKS 2
