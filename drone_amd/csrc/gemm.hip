@@ -20,11 +20,13 @@
 // dense-core shape of the SpMM) 133 TFLOP/s = 84 % of the 157 TFLOP/s fp32 MFMA peak.
 // A long reduction with a small output (the weight gradient: K = vertex count) is split over grid.z; the
 // partial tiles go to a scratch buffer and are summed in split order by a second kernel.
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
 
 #include "common.h"
+#include "gemm_direct.h"
 
 namespace drone {
 namespace {
@@ -809,18 +811,25 @@ void launch_tall(int M, int N, int K, float alpha, const float *A, int lda, cons
     const unsigned grid = (unsigned)std::min<int64_t>(kTallGroups, ceil_div(all_steps, kTallWaves));
     sgemm_tall_kernel<KQ, NT, TB><<<grid, kTallWaves * kWave, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
 }
-bool sgemm_tall(int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
+// Whether an instance of sgemm_tall_kernel covers the product.
+bool tall_covers(int transB, int M, int N, int K, const float *A, int lda, const float *C, int ldc)
+{
+    const int kq = (K + 15) / 16;
+    // Enough rows for its 256 x 12 wavefronts: 41 columns x 128 take 12.0 us (10.5 by sgemm_direct_kernel) at 30,000 rows, 15.1
+    // (16.1) at 50,000.  The lanes read whole 16-byte pieces of A's rows up to column 16 kq, and write C's in such pieces.
+    if (M < 32768 || K < 1 || N > 128 || lda < 16 * kq || lda % 4 != 0 || (reinterpret_cast<uintptr_t>(A) & 15) != 0 ||
+        ldc % 4 != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0)
+        return false;
+    return transB ? (kq == 3 || kq == 4 || kq == 8) && N > 48 : kq == 4 || kq == 8;
+}
+void sgemm_tall(int transB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
                 float *C, int ldc, hipStream_t s)
 {
     const int kq = (K + 15) / 16, nt = N <= 48 ? 3 : N <= 64 ? 4 : 8;
-    // the lanes read whole 16-byte pieces of A's rows up to column 16 kq, and write C's rows in 16-byte pieces
-    if (M < 8192 || K < 1 || N > 128 || lda < 16 * kq || lda % 4 != 0 || (reinterpret_cast<uintptr_t>(A) & 15) != 0 ||
-        ldc % 4 != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0)
-        return false;
 #define DRONE_TALL(KQ_, NT_, TB_)                                                            \
     if (kq == KQ_ && nt == NT_ && (transB != 0) == TB_) {                                    \
         launch_tall<KQ_, NT_, TB_>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);         \
-        return true;                                                                         \
+        return;                                                                              \
     }
     DRONE_TALL(8, 3, false)
     DRONE_TALL(8, 4, false)
@@ -835,7 +844,127 @@ bool sgemm_tall(int transB, int M, int N, int K, float alpha, const float *A, in
     DRONE_TALL(3, 4, true)
     DRONE_TALL(4, 4, true)
 #undef DRONE_TALL
-    return false;
+}
+
+// How many ways the tiled kernel splits the reduction: when the output has too few tiles to fill 256 CUs and K is long.
+int tiled_splits(int tiles, int K)
+{
+    if (tiles >= 256 || K < 4096) return 1;
+    // two work-groups per CU in one round, and at least 1024 reduction steps per work-group.  Measured on the
+    // weight gradients of the 232,965-vertex model (ms for 128 x 41 / 602 x 128 outputs): 1024 work-groups of at
+    // least 512 steps 0.153 / 0.443; 512 and 512: 0.153 / 0.414; 256 and 1024: 0.106 / 0.516; 512 and 1024:
+    // 0.106 / 0.411; 512 and 2048: 0.123 / 0.414.
+    return std::max(1, std::min(512 / tiles, (int)ceil_div(K, 1024)));
+}
+
+// Which products sgemm_direct_kernel takes, and in which shape (ks = 0: the tiled kernel).  The shapes were chosen by
+// timing all instances on some 150 layer products (2 ... 128 columns, inner dimensions 2 ... 700, 1,000 ... 233,000 rows)
+// and their weight gradients; the choice between the kernels compares two estimates that were fitted to the same runs.
+struct DirectShape {
+    int mt = 0, nt = 0, ks = 0, splits = 1;
+};
+DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
+{
+    DirectShape d;
+    if (K < 1 || (ta && tb) || (ta && M < 2)) return d;
+    const auto blocks = [&]() { return ceil_div(M, 16 * d.mt) * ceil_div(N, 16 * d.nt); };
+    if (ta) {
+        if (N <= 16) { d.mt = M <= 16 ? 1 : 2; d.nt = 1; d.ks = 16; }
+        else if (N <= 32) { d.mt = 2; d.nt = 2; d.ks = 16; }
+        else if (ceil_div(N, 64) * 64 * 4 > ceil_div(N, 32) * 32 * 5) { d.mt = M >= 64 ? 4 : 2; d.nt = 2; d.ks = 8; }
+        else { d.mt = 2; d.nt = 4; d.ks = 8; }
+        // about 512 work-groups, none of them with less than five groups of 16 steps per wavefront
+        d.splits = (int)std::max<int64_t>(1, std::min<int64_t>({512 / blocks(), K / (80 * d.ks), 128}));
+    } else {
+        const int n16 = (int)ceil_div(N, 16);
+        d.mt = 1;
+        d.nt = n16 <= 4 ? n16 : n16 <= 6 ? 3 : n16 == 7 ? 7 : 4;
+        const int64_t waves = blocks();
+        if (K >= 384 && d.nt != 7) {
+            // the wavefronts of a work-group share a row block: less of op(B) is read per product
+            d.ks = 8;
+            if (waves >= 1024 && d.nt != 3) d.mt = 2;
+        } else if (waves >= 1024) {
+            d.ks = 1;
+            if (waves >= 4096) d.mt = 2;
+        } else {
+            if (d.nt == 7) d.nt = 4;
+            if (K < 256 && d.nt > 2 && waves < 512) d.nt = 2;
+            d.ks = K >= 384 ? 8 : K >= 64 ? 4 : 1;
+        }
+    }
+    // us: matrix instructions at the rate the kernel reaches on padded blocks, or its memory traffic
+    const double in = 4.0 * ((double)M * K + (double)K * N), out = 4.0 * M * N;
+    const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
+    const double direct_us = std::max(padded / 75e6, in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
+    // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.5 for a 128-wide one)
+    const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
+    const double tiled_us = std::max(ceil_div((int64_t)tiles * splits, 256) * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.5),
+                                     in / 2.0e6 + out / 2.4e6) + (splits > 1 ? 5 : 0);
+    if (tiled_us < direct_us) d.ks = 0;
+    return d;
+}
+
+template <int MT, int NT, bool AK, bool BK, int KS>
+void launch_direct(const DirectShape &d, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+                   float beta, float *C, int ldc, int k_chunk, float *partial, hipStream_t s)
+{
+    constexpr int kWaves = KS > 4 ? KS : 4;
+    const dim3 grid((unsigned)(ceil_div(N, 16 * NT) * ceil_div(M, 16 * MT * (kWaves / KS))), 1, (unsigned)d.splits);
+    const size_t lds = KS > 1 ? sizeof(float) * kWaves * MT * NT * 4 * kWave : 0;
+    sgemm_direct_kernel<MT, NT, AK, BK, KS><<<grid, kWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+}
+
+int sgemm_direct(DirectShape d, bool may_allocate, bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
+                 int lda, const float *B, int ldb, float beta, float *C, int ldc, hipStream_t s)
+{
+    const int k_chunk = (int)ceil_div(ceil_div(K, d.splits), 16) * 16;
+    d.splits = (int)ceil_div(K, k_chunk);
+    float *partial = nullptr;
+    if (d.splits > 1) {
+        const int rc = split_scratch(may_allocate, (size_t)d.splits * M * N, s, M, N, K, d.splits, &partial);
+        if (rc != DRONE_OK) return rc;
+    }
+    bool done = false;
+#define DRONE_DIRECT(MT_, NT_, AK_, BK_, KS_)                                                              \
+    if (d.mt == MT_ && d.nt == NT_ && d.ks == KS_ && ta != AK_ && tb == BK_) {                              \
+        launch_direct<MT_, NT_, AK_, BK_, KS_>(d, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial, s); \
+        done = true;                                                                                      \
+    }
+#define DRONE_DIRECT_ROWS(MT_, NT_, KS_) DRONE_DIRECT(MT_, NT_, true, false, KS_) DRONE_DIRECT(MT_, NT_, true, true, KS_)
+    DRONE_DIRECT_ROWS(1, 1, 1)
+    DRONE_DIRECT_ROWS(1, 2, 1)
+    DRONE_DIRECT_ROWS(1, 3, 1)
+    DRONE_DIRECT_ROWS(1, 4, 1)
+    DRONE_DIRECT_ROWS(1, 7, 1)
+    DRONE_DIRECT_ROWS(2, 1, 1)
+    DRONE_DIRECT_ROWS(2, 2, 1)
+    DRONE_DIRECT_ROWS(2, 3, 1)
+    DRONE_DIRECT_ROWS(2, 4, 1)
+    DRONE_DIRECT_ROWS(2, 7, 1)
+    DRONE_DIRECT_ROWS(1, 1, 4)
+    DRONE_DIRECT_ROWS(1, 2, 4)
+    DRONE_DIRECT_ROWS(1, 3, 4)
+    DRONE_DIRECT_ROWS(1, 4, 4)
+    DRONE_DIRECT_ROWS(1, 1, 8)
+    DRONE_DIRECT_ROWS(1, 2, 8)
+    DRONE_DIRECT_ROWS(1, 3, 8)
+    DRONE_DIRECT_ROWS(1, 4, 8)
+    DRONE_DIRECT_ROWS(2, 1, 8)
+    DRONE_DIRECT_ROWS(2, 2, 8)
+    DRONE_DIRECT_ROWS(2, 4, 8)
+    DRONE_DIRECT(1, 1, false, false, 16)
+    DRONE_DIRECT(2, 1, false, false, 16)
+    DRONE_DIRECT(2, 2, false, false, 16)
+    DRONE_DIRECT(2, 2, false, false, 8)
+    DRONE_DIRECT(4, 2, false, false, 8)
+    DRONE_DIRECT(2, 4, false, false, 8)
+#undef DRONE_DIRECT_ROWS
+#undef DRONE_DIRECT
+    DRONE_REQUIRE(done, "no instance of the direct kernel for this shape");
+    if (d.splits > 1) launch_reduce(M, N, d.splits, partial, alpha, beta, C, ldc, s);
+    DRONE_HIP_TRY(hipGetLastError());
+    return DRONE_OK;
 }
 
 int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,
@@ -848,29 +977,23 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
     if (M == 0 || N == 0) return DRONE_OK;
     DRONE_REQUIRE(C != nullptr && (K == 0 || (A && B)), "null operand");
     hipStream_t s = as_stream(stream);
-    // (the skinny kernel's lanes read four floats of A's row and two of B's at once, also the lanes past M and N)
-    if (transA && !transB && M <= 128 && N <= 64 && K >= 8192 && lda >= (M + 3) / 4 * 4 && ldb >= (N + 1) / 2 * 2)
-        return sgemm_tn_skinny(may_allocate, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
-    if (!transA && K <= 128 && sgemm_tall(transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s)) {
+    if (!transA && K <= 128 && tall_covers(transB, M, N, K, A, lda, C, ldc)) {
+        sgemm_tall(transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
         DRONE_HIP_TRY(hipGetLastError());
         return DRONE_OK;
     }
+    // (the skinny kernel's lanes read four floats of A's row and two of B's at once, also the lanes past M and N.  128 x 41
+    // outputs: 24.6 us (17.9 by sgemm_direct_kernel) over 30,000 rows, 24.0 (24.5) over 50,000, 31 (39) over 100,000; outputs
+    // of 32 rows and fewer are better off with the direct kernel at any length, 43 x 22 and 43 x 41 are not)
+    if (transA && !transB && M > 32 && M <= 128 && N <= 64 && K >= 40000 && lda >= (M + 3) / 4 * 4 && ldb >= (N + 1) / 2 * 2)
+        return sgemm_tn_skinny(may_allocate, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+    const DirectShape direct = direct_shape(transA != 0, transB != 0, M, N, K);
+    if (direct.ks > 0)
+        return sgemm_direct(direct, may_allocate, transA != 0, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
     const bool narrow = N <= 64;
     const int bn = narrow ? 64 : 128;
     const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, bn));
-    // split the reduction when the output has too few tiles to fill 256 CUs and K is long
-    int splits = 1;
-    if (tiles < 256 && K >= 4096) {
-        // two work-groups per CU in one round, and at least 1024 reduction steps per work-group.  Measured on the
-        // weight gradients of the 232,965-vertex model (ms for 128 x 41 / 602 x 128 outputs): 1024 work-groups of at
-        // least 512 steps 0.153 / 0.443; 512 and 512: 0.153 / 0.414; 256 and 1024: 0.106 / 0.516; 512 and 1024:
-        // 0.106 / 0.411; 512 and 2048: 0.123 / 0.414.
-        splits = 512 / tiles;
-        if (splits < 1) splits = 1;
-        const int max_splits = (int)ceil_div(K, 1024);
-        if (splits > max_splits) splits = max_splits;
-        if (splits > 512) splits = 512;
-    }
+    int splits = tiled_splits(tiles, K);
     int k_chunk = (int)ceil_div(ceil_div(K > 0 ? K : 1, splits), BK) * BK;
     splits = (int)ceil_div(K > 0 ? K : 1, k_chunk);
     float *partial = nullptr;
