@@ -18,11 +18,15 @@
 // -1 untouched), which is all the exchange and countActive (common.cu:17-31) look at.  The round number
 // stored in g->active by the reference depends on its thread schedule and is not reproduced.
 //
-// A full sweep costs E however few vertices changed, so rounds with a sparse frontier run the other way round:
-// one wavefront per frontier vertex walks its out-edges and lowers the targets with atomicMin (what the
-// reference does for every round), appending each newly lowered vertex once to the next frontier.  The direction
-// is chosen per round from the number of out-edges of the frontier: push below E / 16, pull above.  Both
-// directions move towards the same fixed point, so switching between them does not change the result.
+// A full sweep costs E however few vertices changed, so a round with a sparse frontier runs the other way round: the
+// frontier is a list of vertices, the list's out-edges are dealt out evenly whatever vertices they belong to, the targets
+// are lowered, and each newly lowered vertex goes once into the next list.  Which kernel takes a round depends on the
+// number of out-edges of the list: up to kSmallEdges one work-group in LDS, which stays for the following rounds
+// (push_rounds_small_kernel), up to E / kPullShare the whole GPU (push_round_kernel), above that a sweep - over the open
+// vertices only where it is known which these are (pull_open_kernel).  All move towards the same fixed point, so
+// switching between them does not change the result.  Every kernel leaves the list's size in device memory for the next
+// (TraverseState), so the host enqueues several rounds per wait.
+#include <algorithm>
 #include <chrono>
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -76,56 +80,100 @@ struct SsspEpi {
     __device__ __forceinline__ void fix(int r, MinF32 s, double &stat) const { lower(r, s.v, stat); }
 };
 
+// The same over lengths that are all 1.0, as build_graph leaves them: 4 bytes per edge less.
+struct SsspUnitEpi : SsspEpi {
+    __device__ __forceinline__ MinF32 load(int c, int64_t) const { return MinF32{dist[c] + 1.0f}; }
+};
+
+// Where a traversal stands.  Its launches hand it on in device memory, so that several rounds can be enqueued before the host
+// has to know how the first of them went: every kernel that runs rounds looks at `listed` and leaves lists that are not for
+// it alone.
+struct TraverseState {
+    unsigned long long listed;  // vertices that still have to propagate << 32 | their out-edges
+    int mark;                   // of the next round, cc.cu:37 `active[v] = step + 1`: positive, and different in every round
+    int rounds;                 // rounds completed
+    int which;                  // which of the two list buffers holds the list
+    double not_one;             // lengths other than 1.0
+};
+// Pinned memory; `state` is as the last launch before the wait left it.
+struct Report {
+    TraverseState state;
+    double visited;  // vertices with active != 0, if the list is empty
+};
+// Two lists of vertices, and where each listed vertex's out-edges start in the list's concatenated out-edges.
+struct Lists {
+    int *vertex[2], *offset[2];
+};
+// A list of no vertices that no round may take for its own: all of them still have to propagate.
+__host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
+
 // cc.cu:10-20
-__global__ void cc_init_kernel(int n, int *__restrict__ active, int *__restrict__ cc, int *__restrict__ ubm)
+__global__ void cc_init_kernel(int n, int *__restrict__ active, int *__restrict__ cc, int *__restrict__ ubm,
+                               TraverseState *__restrict__ state)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         active[i] = 0;
         cc[i] = i;
         ubm[i] = 0;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 1, 0, 0, 0.0};  // cc.cu:16
 }
 
-// sssp.cu:23-38
-__global__ void sssp_init_kernel(int n, int start, int *__restrict__ active, float *__restrict__ dist,
-                                 int *__restrict__ ubm)
+// sssp.cu:23-38, and the list of the first round: the start vertex if this subgraph holds it (sssp.cu:30) and it has
+// out-edges.
+__global__ void sssp_init_kernel(int n, const int *__restrict__ global_to_local, int start_id, int *__restrict__ active,
+                                 float *__restrict__ dist, int *__restrict__ ubm, const int *__restrict__ index,
+                                 int *__restrict__ list, int *__restrict__ offset, TraverseState *__restrict__ state)
 {
+    const int start = global_to_local[start_id];
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         active[i] = i == start ? 0 : -1;
         dist[i] = i == start ? 0.0f : kUnreached;
         ubm[i] = 0;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const int degree = start >= 0 ? index[start + 1] - index[start] : 0;
+        list[0] = start;
+        offset[0] = 0;
+        *state = TraverseState{degree > 0 ? (1ull << 32) + (unsigned long long)degree : 0ull, 1, 0, 0, 0.0};
+    }
 }
 
-// cc.cu:391-404 / sssp.cu:483-496; block_part[b] = vertices a message activated
-__global__ __launch_bounds__(kSpmvBlock) void process_messages_kernel(int n, int *__restrict__ active,
-                                                                      int *__restrict__ ubm,
-                                                                      double *__restrict__ block_part)
+// Ends a counting kernel: the last work-group adds the work-groups' counts and leaves the sum in *out.
+__device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
 {
-    __shared__ double s_red[kSpmvBlock / kWave];
-    double cnt = 0.0;
+    const double total = block_sum_256(mine, s_red);
+    unsigned int one = 0;
+    if (threadIdx.x == 0) one = publish_part(block_part + blockIdx.x, total);
+    if (!last_block_done(ticket, one)) return;
+    const double all = block_sum_of_parts(block_part, (int)gridDim.x, s_red);
+    if (threadIdx.x == 0) *out = all;
+}
+
+// cc.cu:391-404 / sssp.cu:483-496
+__global__ __launch_bounds__(kSpmvBlock) void process_messages_kernel(int n, int *__restrict__ active, int *__restrict__ ubm)
+{
     for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < n; i += gridDim.x * kSpmvBlock) {
         if (ubm[i] != 0) {
             active[i] = 0;
             ubm[i] = 0;
-            cnt += 1.0;
         } else {
             active[i] = -1;
         }
     }
-    const double total = block_sum_256(cnt, s_red);
-    if (threadIdx.x == 0) block_part[blockIdx.x] = total;
 }
 
-// common.cu:17-31 without the single-address atomics
-__global__ __launch_bounds__(kSpmvBlock) void count_active_kernel(int n, const int *__restrict__ active,
-                                                                  double *__restrict__ block_part)
+// Ends what the host enqueues before it waits: tells it where the traversal stands and, if nothing is left to propagate or
+// `always`, counts the vertices with active != 0 (common.cu:17-31, without atomics on one address).
+__global__ __launch_bounds__(kSpmvBlock) void report_kernel(int n, bool always, const int *__restrict__ active, const TraverseState *state,
+                                                            double *block_part, unsigned int *ticket, Report *report)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
+    if (blockIdx.x == 0 && threadIdx.x == 0) report->state = *state;
+    if (!always && state->listed != 0) return;
     double cnt = 0.0;
     for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < n; i += gridDim.x * kSpmvBlock) cnt += active[i] != 0;
-    const double total = block_sum_256(cnt, s_red);
-    if (threadIdx.x == 0) block_part[blockIdx.x] = total;
+    publish_sum(cnt, s_red, block_part, ticket, &report->visited);
 }
 
 __global__ void iota_kernel(int *out, int n)
@@ -133,19 +181,21 @@ __global__ void iota_kernel(int *out, int n)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = i;
 }
 
-__global__ __launch_bounds__(kSpmvBlock) void count_not_one_kernel(int n, const float *__restrict__ len,
-                                                                   double *__restrict__ block_part)
+// *out = lengths other than 1.0 (len is 16-byte aligned).
+__global__ __launch_bounds__(kSpmvBlock) void count_not_one_kernel(int n, const float *__restrict__ len, double *block_part,
+                                                                   unsigned int *ticket, double *out)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
     double cnt = 0.0;
-    for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < n; i += gridDim.x * kSpmvBlock) cnt += len[i] != 1.0f;
-    const double total = block_sum_256(cnt, s_red);
-    if (threadIdx.x == 0) block_part[blockIdx.x] = total;
-}
-
-__global__ void fill_f32_kernel(float *out, float v, int n)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = v;
+    const float4 *len4 = reinterpret_cast<const float4 *>(len);
+    const int quads = n / 4;
+#pragma unroll 4
+    for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += gridDim.x * kSpmvBlock) {
+        const float4 v = len4[i];
+        cnt += (double)((v.x != 1.0f) + (v.y != 1.0f) + (v.z != 1.0f) + (v.w != 1.0f));
+    }
+    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) cnt += len[4 * quads + threadIdx.x] != 1.0f;
+    publish_sum(cnt, s_red, block_part, ticket, out);
 }
 
 __global__ void gather_len_kernel(int n, const int *__restrict__ eid, const float *__restrict__ len,
@@ -154,19 +204,19 @@ __global__ void gather_len_kernel(int n, const int *__restrict__ eid, const floa
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = len[eid[i]];
 }
 
-// Launches of at most this many work-groups hand their counters to the host themselves (publish_counters); larger
-// ones - push rounds over a long list of hubs - leave them to a copy.
-constexpr int kPublishMaxBlocks = 16384;
+constexpr int kListBlocks = 2048;  // most work-groups of the kernels that build a list
+constexpr int kSumBlocks = 512;   // most work-groups of the counting kernels
 
 // Per-call scratch of the traversals, hung off CCValues::ext / SSSPValues::ext.
 struct TraverseExt {
     double *stat = nullptr;        // device scalar
-    double *block_part = nullptr;  // device [blocks]
-    int blocks = 0;
-    int *frontier[2] = {nullptr, nullptr};  // device [n] each: vertex lists of the push rounds
-    unsigned long long *counters = nullptr; // device [2]: {vertices << 32 | out-edges, largest out-degree} of the list being built; zero between launches
-    unsigned int *ticket = nullptr;         // device [ticket_words(kPublishMaxBlocks)]: counters of last_block_done, zero between launches
-    unsigned long long *host = nullptr;     // pinned [4]: where the kernels' last work-groups leave the statistic / the counters (+ rounds run)
+    double *block_part = nullptr;  // device [kSumBlocks]: parts of the counting kernels
+    int blocks = 0;                // work-groups of the passes over the vertices
+    Lists lists{};                 // device [n] each; vertices with out-edges only
+    unsigned long long *counters = nullptr; // device: vertices << 32 | out-edges of the list being built; zero between launches
+    unsigned int *ticket = nullptr;         // device [ticket_words(kListBlocks)]: counters of last_block_done, zero between launches
+    TraverseState *state = nullptr;         // device
+    Report *report = nullptr;               // pinned
 };
 
 double seconds_since(std::chrono::steady_clock::time_point t0)
@@ -180,21 +230,29 @@ void die(const char *what)
     exit(EXIT_FAILURE);
 }
 
+void allow_small_lds();  // of push_rounds_small_kernel, on the current device
+
 TraverseExt *traverse_ext_create(int n)
 {
+    allow_small_lds();
     TraverseExt *t = new TraverseExt();
     t->blocks = (int)ceil_div(n > 0 ? n : 1, kSpmvBlock * 4);
     if (t->blocks > 4096) t->blocks = 4096;
     DRONE_HIP_OR_DIE(hipMalloc(&t->stat, sizeof(double)));
-    DRONE_HIP_OR_DIE(hipMalloc(&t->block_part, sizeof(double) * (size_t)t->blocks));
-    DRONE_HIP_OR_DIE(hipMalloc(&t->frontier[0], sizeof(int) * (size_t)(n > 0 ? n : 1)));
-    DRONE_HIP_OR_DIE(hipMalloc(&t->frontier[1], sizeof(int) * (size_t)(n > 0 ? n : 1)));
-    DRONE_HIP_OR_DIE(hipMalloc(&t->counters, sizeof(unsigned long long) * 2));
-    DRONE_HIP_OR_DIE(hipMemset(t->counters, 0, sizeof(unsigned long long) * 2));
-    DRONE_HIP_OR_DIE(hipMalloc(&t->ticket, sizeof(unsigned int) * ticket_words(kPublishMaxBlocks)));
-    DRONE_HIP_OR_DIE(hipMemset(t->ticket, 0, sizeof(unsigned int) * ticket_words(kPublishMaxBlocks)));
+    DRONE_HIP_OR_DIE(hipMalloc(&t->block_part, sizeof(double) * (size_t)kSumBlocks));
+    const size_t cnt = ((size_t)(n > 0 ? n : 1) + 63) & ~(size_t)63;
+    DRONE_HIP_OR_DIE(hipMalloc(&t->lists.vertex[0], sizeof(int) * 4 * cnt));  // one allocation
+    t->lists.vertex[1] = t->lists.vertex[0] + cnt;
+    t->lists.offset[0] = t->lists.vertex[1] + cnt;
+    t->lists.offset[1] = t->lists.offset[0] + cnt;
+    DRONE_HIP_OR_DIE(hipMalloc(&t->counters, sizeof(unsigned long long)));
+    DRONE_HIP_OR_DIE(hipMemset(t->counters, 0, sizeof(unsigned long long)));
+    DRONE_HIP_OR_DIE(hipMalloc(&t->state, sizeof(TraverseState)));
+    DRONE_HIP_OR_DIE(hipMalloc(&t->ticket, sizeof(unsigned int) * ticket_words(kListBlocks)));
+    DRONE_HIP_OR_DIE(hipMemset(t->ticket, 0, sizeof(unsigned int) * ticket_words(kListBlocks)));
     DRONE_HIP_OR_DIE(hipStreamSynchronize(nullptr));  // the kernels that count may run on any stream
-    DRONE_HIP_OR_DIE(hipHostMalloc(&t->host, sizeof(unsigned long long) * 4));
+    DRONE_HIP_OR_DIE(hipHostMalloc(&t->report, sizeof(Report)));
+    *t->report = Report{};
     return t;
 }
 
@@ -204,310 +262,779 @@ void traverse_ext_destroy(void *ext)
     if (!t) return;
     (void)hipFree(t->stat);
     (void)hipFree(t->block_part);
-    (void)hipFree(t->frontier[0]);
-    (void)hipFree(t->frontier[1]);
+    (void)hipFree(t->lists.vertex[0]);
     (void)hipFree(t->counters);
     (void)hipFree(t->ticket);
-    (void)hipHostFree(t->host);
+    (void)hipFree(t->state);
+    (void)hipHostFree(t->report);
     delete t;
 }
 
-// Where a sweep's fix-up leaves its statistic for the host.
-double *stat_landing(TraverseExt *t) { return reinterpret_cast<double *>(t->host); }
+int sum_blocks(int64_t n, int per_lane = 4) { return (int)std::min<int64_t>(std::max<int64_t>(ceil_div(n, (int64_t)kSpmvBlock * per_lane), 1), kSumBlocks); }
 
-// The statistic of the last sweep (or of reduce_parts): its kernel wrote it to pinned memory, so waiting is enough.
-double read_stat(TraverseExt *t, hipStream_t s)
+void launch_report(Graph *g, TraverseExt *t, bool always, hipStream_t s)
 {
-    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
-    return *stat_landing(t);
-}
-
-double reduce_parts(TraverseExt *t, hipStream_t s)
-{
-    reduce_stat_kernel<0><<<1, kSpmvBlock, 0, s>>>(t->block_part, t->blocks, stat_landing(t));
-    return read_stat(t, s);
+    const int n = getLocalVertexSize(g);
+    report_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, always, g->active, t->state, t->block_part, t->ticket, t->report);
 }
 
 int count_active(Graph *g, TraverseExt *t, hipStream_t s)
 {
-    count_active_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(getLocalVertexSize(g), g->active, t->block_part);
-    return (int)reduce_parts(t, s);
+    launch_report(g, t, true, s);
+    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+    return (int)t->report->visited;
 }
 
 // ---- push direction ---------------------------------------------------------------------------------------
+// A value's place in the integers' order: what LDS atomics compare.
+__device__ __forceinline__ int order_of(int v) { return v; }
+__device__ __forceinline__ int order_of(float v)
+{
+    const int b = __float_as_int(v);
+    return b ^ ((b >> 31) & 0x7FFFFFFF);
+}
+
+__device__ __forceinline__ int value_of_order(int o, int) { return o; }
+__device__ __forceinline__ float value_of_order(int o, float) { return __int_as_float(o ^ ((o >> 31) & 0x7FFFFFFF)); }
+
 struct CcPush {
+    using Value = int;
     int *cc;
     __device__ __forceinline__ int load(int v) const { return __atomic_load_n(cc + v, __ATOMIC_RELAXED); }
+    __device__ __forceinline__ int at(int v) const { return cc[v]; }
+    __device__ __forceinline__ void store(int v, int x) const { cc[v] = x; }
     __device__ __forceinline__ int relax(int val, int) const { return val; }
-    __device__ __forceinline__ bool lower(int t, int nv) const { return atomicMin(cc + t, nv) > nv; }  // cc.cu:35-36
+    __device__ __forceinline__ int lower(int t, int nv) const { return atomicMin(cc + t, nv); }  // cc.cu:35-36
+    static __device__ __forceinline__ bool activates(int old, int nv) { return old > nv; }
 };
 
 struct SsspPush {
+    using Value = float;
     float *dist;
     const float *__restrict__ len;  // out-edge order (g->edgeLen)
     __device__ __forceinline__ float load(int v) const
     {
         return __uint_as_float(__atomic_load_n(reinterpret_cast<unsigned int *>(dist + v), __ATOMIC_RELAXED));
     }
+    __device__ __forceinline__ float at(int v) const { return dist[v]; }
+    __device__ __forceinline__ void store(int v, float x) const { dist[v] = x; }
     __device__ __forceinline__ float relax(float val, int e) const { return val + len[e]; }
-    __device__ __forceinline__ bool lower(int t, float nv) const
+    // sssp.cu:11-21 fatomicMin without its compare-and-swap loop: floats of one sign order like their bits, a negative
+    // float's bits are the larger the smaller it is.  Returns the value found.
+    __device__ __forceinline__ float lower(int t, float nv) const
     {
-        // sssp.cu:11-21 fatomicMin: compare-and-swap until the stored value is not larger; returns the value seen
-        // first.  The target counts as updated past the tolerance (sssp.cu:64).
-        unsigned int *addr = reinterpret_cast<unsigned int *>(dist + t);
-        const float first = __uint_as_float(__atomic_load_n(addr, __ATOMIC_RELAXED));
-        float old = first;
-        while (old > nv) {
-            const unsigned int seen = atomicCAS(addr, __float_as_uint(old), __float_as_uint(nv));
-            if (seen == __float_as_uint(old)) break;
-            old = __uint_as_float(seen);
-        }
-        return first > nv + kRelaxEps;
+        if (__float_as_int(nv) >= 0) return __int_as_float(atomicMin(reinterpret_cast<int *>(dist + t), __float_as_int(nv)));
+        return __uint_as_float(atomicMax(reinterpret_cast<unsigned int *>(dist + t), __float_as_uint(nv)));
     }
+    // The target counts as updated past the tolerance (sssp.cu:64).
+    static __device__ __forceinline__ bool activates(float old, float nv) { return old > nv + kRelaxEps; }
 };
 
-// Appends v for every lane with `take` to the list and adds the lanes' out-degrees to the counters.  The vertex
-// count and the edge sum share one 64-bit word (both stay below 2^31), so a wavefront issues one atomic that returns
-// its position in the list; the largest degree is only written when it grows.  Must be reached by all lanes.
-__device__ __forceinline__ void frontier_append(bool take, int v, int degree, int *__restrict__ list,
-                                                unsigned long long *__restrict__ counters)
-{
-    const unsigned long long mask = __ballot(take);
-    if (mask == 0) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    unsigned long long sum = take ? (unsigned long long)degree : 0ull;
-    int mx = take ? degree : 0;
-#pragma unroll
-    for (int m = kWave / 2; m > 0; m >>= 1) {
-        sum += __shfl_xor(sum, m, kWave);
-        const int o = __shfl_xor(mx, m, kWave);
-        mx = o > mx ? o : mx;
-    }
-    const int leader = __ffsll((long long)mask) - 1;
-    unsigned long long base = 0;
-    if (lane == leader) {
-        base = atomicAdd(counters, ((unsigned long long)__popcll(mask) << 32) + sum) >> 32;
-        if ((unsigned long long)mx > __atomic_load_n(counters + 1, __ATOMIC_RELAXED)) {
-            // waited for, like the add above: publish_counters reads the word once every work-group has its ticket
-            const unsigned long long seen = atomicMax(counters + 1, (unsigned long long)mx);
-            asm volatile("" ::"v"((unsigned int)seen));
-        }
-    }
-    base = __shfl(base, leader, kWave);
-    if (take) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = v;
-}
-
-// The last work-group of a launch that built a list hands {count << 32 | edges, largest degree} to the host (pinned
-// memory) and clears the counters for the next launch.  ticket == nullptr: the host copies and clears them.
-// The two counter words are all it reads of the other work-groups' work, and they are only ever updated by returning
+// Ends a round: the last work-group of a launch that built list `which` leaves the state for the next launch and clears the
+// counter.  The counter is all it reads of the other work-groups' work, and it is only ever updated by returning
 // agent-scope atomics (see publish_part in spmv_merge.h); the list itself is plain stores, read by the next launch.
-__device__ __forceinline__ void publish_counters(unsigned long long *counters, unsigned int *ticket,
-                                                 unsigned long long *host)
+// Every work-group has read *state by the time the last one gets here.
+__device__ __forceinline__ void end_round(TraverseState *state, int mark, int rounds, int which, unsigned long long *counters,
+                                          unsigned int *ticket)
 {
-    if (ticket == nullptr) return;
     __syncthreads();  // every wavefront of the work-group has issued its appends (their atomics return before they go on)
     if (!last_block_done(ticket, 1u) || threadIdx.x != 0) return;
-    host[0] = __hip_atomic_exchange(counters, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    host[1] = __hip_atomic_exchange(counters + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    state->listed = __hip_atomic_exchange(counters, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    state->mark = mark;
+    state->rounds = rounds;
+    state->which = which;
 }
 
-// list <- vertices whose active flag equals `value`.  A work-group first compacts its matches in LDS, then the
-// first wavefront appends them, so the shared counter sees one atomic per 256 vertices that hold a match.
-__global__ __launch_bounds__(kSpmvBlock) void collect_frontier_kernel(int n, const int *__restrict__ active, int value,
-                                                                      const int *__restrict__ index, int *__restrict__ list,
-                                                                      unsigned long long *counters, unsigned int *ticket,
-                                                                      unsigned long long *host)
-{
-    __shared__ int s_v[kSpmvBlock];
-    __shared__ int s_count;
-    for (int base = blockIdx.x * kSpmvBlock; base < n; base += gridDim.x * kSpmvBlock) {
-        if (threadIdx.x == 0) s_count = 0;
-        __syncthreads();
-        const int v = base + threadIdx.x;
-        if (v < n && active[v] == value) s_v[atomicAdd(&s_count, 1)] = v;
-        __syncthreads();
-        const int cnt = s_count;
-        if (threadIdx.x < kWave) {
-            for (int k = 0; k < cnt; k += kWave) {  // cnt is the same for the whole wavefront
-                const bool take = k + (int)threadIdx.x < cnt;
-                const int u = take ? s_v[k + threadIdx.x] : 0;
-                frontier_append(take, u, take ? index[u + 1] - index[u] : 0, list, counters);
+// A work-group's part of the next list: vertices and their out-degrees gathered in LDS, appended with ONE atomic on the
+// shared counter.  (One atomic per wavefront with something to append cost 9 ns each, all on one address: 150 us for a
+// million frontier edges.)
+template <int CAP>
+struct ListBuffer {
+    int vertex[CAP], degree_before[CAP];
+    unsigned long long held;  // vertices << 32 | out-edges
+    unsigned long long base;
+
+    __device__ __forceinline__ void add(int v, int degree)
+    {
+        const unsigned long long p = atomicAdd(&held, (1ull << 32) + (unsigned long long)degree);
+        vertex[p >> 32] = v;
+        degree_before[p >> 32] = (int)(p & 0xFFFFFFFFull);
+    }
+    // by all threads, between barriers; leaves the buffer empty
+    __device__ __forceinline__ void flush(int *__restrict__ list, int *__restrict__ offset, unsigned long long *counters)
+    {
+        if (threadIdx.x == 0) {
+            unsigned long long at = 0;
+            if (held) {
+                at = atomicAdd(counters, held);
+                asm volatile("" ::"v"((unsigned int)at));  // waited for: end_round counts on it
             }
+            base = at;
         }
         __syncthreads();
-    }
-    publish_counters(counters, ticket, host);
-}
-
-// One wavefront per (frontier vertex, chunk of kPushChunk out-edges); blockIdx.y is the chunk, so a hub's edges are
-// spread over many wavefronts and a wavefront whose chunk lies past the vertex's degree leaves at once.  A target
-// lowered in this round is appended to `next` once: its active flag is swapped to this round's mark, and only the
-// lane that changes it appends.
-constexpr int kPushChunk = 1024;
-
-template <typename Push>
-__global__ __launch_bounds__(256) void push_round_kernel(int count, const int *__restrict__ frontier,
-                                                         const int *__restrict__ index, const int *__restrict__ dst,
-                                                         Push push, int *__restrict__ active, int mark,
-                                                         int *__restrict__ next, unsigned long long *counters,
-                                                         unsigned int *ticket, unsigned long long *host)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    const int waves = gridDim.x * (blockDim.x / kWave);
-    for (int i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < count; i += waves) {
-        const int v = frontier[i];
-        const int e0 = index[v] + blockIdx.y * kPushChunk;
-        int e1 = index[v + 1];
-        if (e0 >= e1) continue;  // the same for all lanes
-        if (e1 > e0 + kPushChunk) e1 = e0 + kPushChunk;
-        const auto val = push.load(v);
-        for (int eb = e0; eb < e1; eb += kWave) {
-            const int e = eb + lane;
-            bool take = false;
-            int t = 0;
-            if (e < e1) {
-                t = dst[e];
-                take = push.lower(t, push.relax(val, e)) && atomicExch(active + t, mark) != mark;
-            }
-            frontier_append(take, t, take ? index[t + 1] - index[t] : 0, next, counters);
+        const int count = (int)(held >> 32);
+        const int v0 = (int)(base >> 32), e0 = (int)(base & 0xFFFFFFFFull);
+        for (int i = threadIdx.x; i < count; i += blockDim.x) {
+            list[v0 + i] = vertex[i];
+            offset[v0 + i] = e0 + degree_before[i];
         }
-    }
-    publish_counters(counters, ticket, host);
-}
-
-// Push rounds of a short list inside ONE launch: a single work-group walks the list, builds the next one (counters in
-// LDS) and goes on with it for as long as it stays short - at most kSmallCount vertices with kSmallEdges out-edges -
-// and is not empty, up to max_rounds rounds.  Round k of the launch marks with mark + k.  A path of 20,000 vertices
-// then costs one launch and a barrier per hop instead of a launch and a host round trip per hop.  The lists alternate
-// between a and b; the host learns the rounds run and the last list's counters from pinned memory:
-// host[0] = count << 32 | out-edges, host[1] = largest out-degree, host[2] = rounds (the list is b after an odd number).
-constexpr int kSmallCount = 256;
-constexpr int kSmallEdges = 8192;
-
-template <typename Push>
-__global__ __launch_bounds__(256) void push_rounds_small_kernel(int count, int *a, int *b, const int *__restrict__ index,
-                                                                const int *__restrict__ dst, Push push, int *active,
-                                                                int mark, int max_rounds, unsigned long long *host)
-{
-    __shared__ unsigned long long s_counters[2];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int waves = blockDim.x / kWave;
-    int rounds = 0;
-    unsigned long long packed = 0, max_degree = 0;
-    for (;;) {
-        if (threadIdx.x < 2) s_counters[threadIdx.x] = 0ull;
         __syncthreads();
-        for (int i = threadIdx.x / kWave; i < count; i += waves) {
-            const int v = a[i];
-            const int e0 = index[v], e1 = index[v + 1];
-            const auto val = push.load(v);
-            for (int eb = e0; eb < e1; eb += kWave) {
-                const int e = eb + lane;
-                bool take = false;
-                int t = 0;
-                if (e < e1) {
-                    t = dst[e];
-                    take = push.lower(t, push.relax(val, e)) && atomicExch(active + t, mark) != mark;
-                }
-                frontier_append(take, t, take ? index[t + 1] - index[t] : 0, b, s_counters);
-            }
-        }
-        __syncthreads();  // the next list and its counters are complete (the work-group's own writes are visible to it)
-        ++rounds;
-        packed = s_counters[0];
-        max_degree = s_counters[1];
-        count = (int)(packed >> 32);
-        int *const swap = a;
-        a = b;
-        b = swap;
-        if (count == 0 || count > kSmallCount || (packed & 0xFFFFFFFFull) > (unsigned long long)kSmallEdges ||
-            rounds == max_rounds)
-            break;
-        ++mark;
-        __syncthreads();  // everyone has read the counters before they are cleared
+        if (threadIdx.x == 0) held = 0ull;
+        __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        host[0] = packed;
-        host[1] = max_degree;
-        host[2] = (unsigned long long)rounds;
-    }
-}
-
-struct Frontier {
-    unsigned long long count = 0, edges = 0, max_degree = 0;
 };
 
-Frontier read_counters(TraverseExt *t, hipStream_t s, bool published)
+// List 0 <- vertices with out-edges whose active flag equals `value`; every work-group takes a contiguous range.
+constexpr int kCollectBuffer = 2048, kCollectStep = 4 * kSpmvBlock;
+__global__ __launch_bounds__(kSpmvBlock) void collect_frontier_kernel(int n, const int *__restrict__ active, int value,
+                                                                      const int *__restrict__ index, Lists lists,
+                                                                      unsigned long long *counters, unsigned int *ticket,
+                                                                      TraverseState *state, int next_mark, int rounds)
 {
-    if (!published) {
-        DRONE_HIP_OR_DIE(hipMemcpyAsync(t->host, t->counters, sizeof(unsigned long long) * 2, hipMemcpyDeviceToHost, s));
-        DRONE_HIP_OR_DIE(hipMemsetAsync(t->counters, 0, sizeof(unsigned long long) * 2, s));
+    __shared__ ListBuffer<kCollectBuffer> s_buf;
+    if (threadIdx.x == 0) s_buf.held = 0ull;
+    __syncthreads();
+    const int per_block = (int)(((int64_t)n + gridDim.x - 1) / gridDim.x);
+    const int begin = blockIdx.x * per_block, end = begin + per_block < n ? begin + per_block : n;
+    for (int64_t base = begin; base < end; base += kCollectStep) {
+        bool take[kCollectStep / kSpmvBlock];
+#pragma unroll
+        for (int k = 0; k < kCollectStep / kSpmvBlock; ++k) {
+            const int64_t v = base + k * kSpmvBlock + threadIdx.x;
+            take[k] = v < end && active[v] == value;
+        }
+#pragma unroll
+        for (int k = 0; k < kCollectStep / kSpmvBlock; ++k)
+            if (take[k]) {
+                const int v = (int)base + k * kSpmvBlock + (int)threadIdx.x;
+                const int degree = index[v + 1] - index[v];
+                if (degree > 0) s_buf.add(v, degree);
+            }
+        __syncthreads();
+        const bool full = (int)(s_buf.held >> 32) > kCollectBuffer - kCollectStep || base + kCollectStep >= end;
+        __syncthreads();  // everyone has read it before anyone adds again
+        if (full) s_buf.flush(lists.vertex[0], lists.offset[0], counters);
     }
-    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));  // else publish_counters has written them
-    return Frontier{t->host[0] >> 32, t->host[0] & 0xFFFFFFFFull, t->host[1]};
+    end_round(state, next_mark, rounds, 0, counters, ticket);
 }
 
-Frontier collect_frontier(Graph *g, TraverseExt *t, int value, int *list, hipStream_t s)
+// One push round over a list: a work-group takes kChunk consecutive edges of the list's concatenated out-edges at a time,
+// whatever vertices they belong to (hubs are spread, short rows packed).  A target is first looked at with a plain load:
+// a value that is not above the new one there never will be (values only fall), whatever the load's age, so only real
+// improvements pay for atomics, which are carried out at the memory side.  A target lowered in this round is appended to
+// `next` once: its active flag is swapped to this round's mark, and only the lane that changes it appends.
+// Lists of at most `above` edges are push_rounds_small_kernel's, of more than `limit` a sweep's: left alone.
+// (One wavefront per vertex and 1,024-edge piece, pieces along grid.y, launched 400,000 work-groups for a list of 50,000
+// vertices with one hub of 39,000 edges: 70 us per round on the 11.5 M-edge graph, 9 us this way.)
+constexpr int kPushThreads = 256;
+constexpr int kPushBlocks = 1024;
+constexpr int kPushWideEdges = 1 << 19;  // from here on a chunk has eight edges per lane, below one: 256 work-groups either way
+
+template <typename Value, int PER>
+struct PushShared {
+    int start[kPushThreads * PER], edge[kPushThreads * PER];
+    Value val[kPushThreads * PER];
+    ListBuffer<kPushThreads * PER> buf;
+    int first, entries;
+};
+
+template <typename Push, int PER>
+__device__ __forceinline__ void push_chunks(PushShared<typename Push::Value, PER> &sh, int count, int edges, int mark,
+                                            const int *__restrict__ list, const int *__restrict__ offset,
+                                            const int *__restrict__ index, const int *__restrict__ dst, const Push &push,
+                                            int *__restrict__ active, int *__restrict__ next, int *__restrict__ next_offset,
+                                            unsigned long long *counters)
+{
+    using Value = typename Push::Value;
+    constexpr int kChunk = kPushThreads * PER;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int64_t chunks = ((int64_t)edges + kChunk - 1) / kChunk;
+    for (int64_t chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
+        const int j0 = (int)(chunk * kChunk), j1 = edges - j0 < kChunk ? edges : j0 + kChunk;
+        if (tid < kWave) {  // the listed vertex that holds edge j0, 64 probes at a time
+            int lo = 0, hi = count;  // offset[lo] <= j0, and offset[hi] > j0 (offset[count] would be `edges`)
+            while (hi - lo > 1) {
+                const int step = (hi - lo + kWave - 1) / kWave, at = lo + (lane + 1) * step;
+                const unsigned long long below = __ballot(at < hi && offset[at < hi ? at : lo] <= j0);
+                lo += __popcll(below) * step;
+                hi = lo + step < hi ? lo + step : hi;
+            }
+            if (lane == 0) {
+                sh.first = lo;
+                sh.entries = 0;
+                sh.buf.held = 0ull;
+            }
+        }
+        __syncthreads();
+        const int first = sh.first;
+        int mine = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {  // every listed vertex has an edge: at most kChunk of them
+            const int i = tid + k * kPushThreads;
+            if (first + i < count) {
+                const int start = offset[first + i] - j0;
+                if (start < j1 - j0) {
+                    const int v = list[first + i];
+                    sh.start[i] = start;
+                    sh.edge[i] = index[v] - start;
+                    sh.val[i] = push.load(v);
+                    mine = i + 1;
+                }
+            }
+        }
+        if (mine) atomicMax(&sh.entries, mine);
+        __syncthreads();
+        const int entries = sh.entries;
+        int t[PER], e[PER];
+        Value nv[PER], old[PER];
+        bool live[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int j = tid + k * kPushThreads;
+            int lo = 0, hi = entries;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (sh.start[mid] <= j) lo = mid; else hi = mid;
+            }
+            live[k] = j < j1 - j0;
+            if (!live[k]) lo = 0;
+            e[k] = sh.edge[lo] + (live[k] ? j : 0);  // past the list's end: its edge j0 once more
+            nv[k] = sh.val[lo];
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            t[k] = dst[e[k]];
+            nv[k] = push.relax(nv[k], e[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) old[k] = push.at(t[k]);
+#pragma unroll
+        for (int k = 0; k < PER; ++k) live[k] = live[k] && nv[k] < old[k];
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            if (live[k]) old[k] = push.lower(t[k], nv[k]);
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            if (live[k]) live[k] = Push::activates(old[k], nv[k]) && atomicExch(active + t[k], mark) != mark;
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            if (live[k]) {
+                const int degree = index[t[k] + 1] - index[t[k]];
+                if (degree > 0) sh.buf.add(t[k], degree);
+            }
+        __syncthreads();
+        sh.buf.flush(next, next_offset, counters);
+    }
+}
+
+template <typename Push>
+__global__ __launch_bounds__(kPushThreads) void push_round_kernel(TraverseState *state, unsigned long long above, unsigned long long limit,
+                                                                  Lists lists, const int *__restrict__ index,
+                                                                  const int *__restrict__ dst, Push push, int *__restrict__ active,
+                                                                  unsigned long long *counters, unsigned int *ticket)
+{
+    using Value = typename Push::Value;
+    __shared__ union Shared {
+        PushShared<Value, 8> wide;
+        PushShared<Value, 1> narrow;
+    } s_push;
+    const TraverseState now = *state;
+    const unsigned long long edges = now.listed & 0xFFFFFFFFull;
+    if (edges <= above || edges > limit) return;
+    const int count = (int)(now.listed >> 32), w = now.which & 1;
+    if (edges >= (unsigned long long)kPushWideEdges)
+        push_chunks<Push, 8>(s_push.wide, count, (int)edges, now.mark, lists.vertex[w], lists.offset[w], index, dst, push, active,
+                             lists.vertex[w ^ 1], lists.offset[w ^ 1], counters);
+    else
+        push_chunks<Push, 1>(s_push.narrow, count, (int)edges, now.mark, lists.vertex[w], lists.offset[w], index, dst, push, active,
+                             lists.vertex[w ^ 1], lists.offset[w ^ 1], counters);
+    end_round(state, now.mark + 1, now.rounds + 1, w ^ 1, counters, ticket);
+}
+
+// One sweep over the in-edges of the vertices that can still fall (the "open" ones): a vertex's in-neighbours are looked
+// at until one settles it.  Most of a sweep over all edges is spent on vertices that have their final value; and of those
+// that have not, most find a settling neighbour in a few steps (the bottom-up step of breadth-first search).  It is bound
+// by the chains of dependent loads (value, row bounds, neighbour, its value), so rows are spread: a work-group takes
+// 64-row pieces from all over the graph (vertices of high degree often sit side by side), rows of up to kPullLane entries
+// get a lane, of up to kPullGroup 16 lanes, of up to kPullWave a wavefront, longer ones the work-group.  Lowered vertices are
+// listed for the next round on the way.  1 M vertices, 11.5 M edges: 26 us for either of the two sweeps of a shortest-path
+// run, 91 for the sweep over all edges; 72 with rows side by side in one work-group and wavefronts for all rows above 16
+// entries.
+struct CcPull {  // no label is below 0
+    using Value = int;
+    int *cc;
+    __device__ __forceinline__ bool begin(const TraverseState &) { return true; }
+    __device__ __forceinline__ int at(int v) const { return cc[v]; }
+    __device__ __forceinline__ void store(int v, int x) const { cc[v] = x; }
+    __device__ __forceinline__ bool open(int v) const { return v > 0; }
+    __device__ __forceinline__ int offer(int u, int) const { return cc[u]; }  // what in-neighbour u offers
+    __device__ __forceinline__ bool settles(int x) const { return x <= 0; }
+};
+struct LevelPull {  // rounds of unit lengths from one start vertex: round k reaches the vertices at distance k, for good
+    using Value = float;
+    float *dist;
+    float level = 0.0f;
+    // beyond 2^24 levels are no longer exact
+    static constexpr int kMostRounds = (1 << 24) - 1;
+    __device__ __forceinline__ bool begin(const TraverseState &s)
+    {
+        level = (float)(s.rounds + 1);
+        return s.not_one == 0.0 && s.rounds < kMostRounds;
+    }
+    __device__ __forceinline__ float at(int v) const { return dist[v]; }
+    __device__ __forceinline__ void store(int v, float x) const { dist[v] = x; }
+    __device__ __forceinline__ bool open(float v) const { return v >= kUnreached; }
+    __device__ __forceinline__ float offer(int u, float otherwise) const { return dist[u] == level - 1.0f ? level : otherwise; }
+    __device__ __forceinline__ bool settles(float x) const { return x == level; }
+};
+constexpr int kPullThreads = 1024, kPullBlocks = 512;  // all resident at once: an append to the shared counter each
+constexpr int kPullList = 2048;
+constexpr int kPullLane = 8, kPullGroup = 256, kPullWave = 4096;
+
+template <typename Pull>
+__global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *state, unsigned long long limit, int n,
+                                                                 const int *__restrict__ in_index,
+                                                                 const int *__restrict__ in_src, Pull pull,
+                                                                 int *__restrict__ active, const int *__restrict__ index,
+                                                                 Lists lists, unsigned long long *counters, unsigned int *ticket)
+{
+    using Value = typename Pull::Value;
+    constexpr int kWaves = kPullThreads / kWave;
+    __shared__ ListBuffer<kPullList> s_buf;
+    __shared__ int s_group[kPullThreads], s_wave[kPullThreads], s_block[kPullThreads];
+    __shared__ int s_groups, s_waves, s_blocks, s_best;
+    const TraverseState now = *state;
+    if ((now.listed & 0xFFFFFFFFull) <= limit || !pull.begin(now)) return;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    if (tid == 0) s_buf.held = 0ull;
+    const auto lower = [&](int r, Value was, Value to) {
+        if (!(to < was)) return;
+        pull.store(r, to);
+        active[r] = now.mark;
+        const int degree = index[r + 1] - index[r];
+        if (degree > 0) s_buf.add(r, degree);
+    };
+    // G lanes a row
+    const auto walk = [&](auto lanes, const int *rows, int count) {
+        constexpr int G = decltype(lanes)::value;
+        const int l = tid & (G - 1);
+        for (int i = tid / G; i < count; i += kPullThreads / G) {
+            const int row = rows[i];
+            const unsigned int e0 = in_index[row], e1 = in_index[row + 1];
+            const Value was = pull.at(row);
+            Value best = was;
+            for (unsigned int base = e0; base < e1; base += 2 * G) {
+                int u[2];
+                Value x[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const unsigned int e = base + k * G + l;
+                    u[k] = in_src[e < e1 ? e : e1 - 1];
+                }
+#pragma unroll
+                for (int k = 0; k < 2; ++k) x[k] = pull.offer(u[k], was);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) best = x[k] < best ? x[k] : best;
+                const unsigned long long settled = __ballot(pull.settles(best));
+                if (G == kWave ? settled != 0 : ((settled >> (lane & ~(G - 1))) & ((1ull << (G & 63)) - 1)) != 0) break;
+            }
+#pragma unroll
+            for (int m = G / 2; m > 0; m >>= 1) {
+                const Value o = __shfl_xor(best, m, kWave);
+                best = o < best ? o : best;
+            }
+            if (l == 0) lower(row, was, best);
+        }
+    };
+    const int64_t pieces = ((int64_t)n + kWave - 1) / kWave, per_pass = (int64_t)kWaves * gridDim.x;
+    for (int64_t pass = 0; pass < pieces; pass += per_pass) {
+        if (tid == 0) s_groups = s_waves = s_blocks = 0;
+        __syncthreads();
+        const int64_t r64 = (pass + (int64_t)wave * gridDim.x + blockIdx.x) * kWave + lane;
+        if (r64 < n) {
+            const int r = (int)r64;
+            const Value was = pull.at(r);
+            if (pull.open(was)) {
+                const unsigned int e0 = in_index[r], e1 = in_index[r + 1];
+                if (e1 - e0 <= kPullLane) {
+                    Value best = was;
+                    for (unsigned int e = e0; e < e1 && !pull.settles(best); e += 4) {
+                        int u[4];
+                        Value x[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) u[k] = in_src[e + k < e1 ? e + k : e1 - 1];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) x[k] = pull.offer(u[k], was);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) best = x[k] < best ? x[k] : best;
+                    }
+                    lower(r, was, best);
+                } else if (e1 - e0 <= kPullGroup) {
+                    s_group[atomicAdd(&s_groups, 1)] = r;
+                } else if (e1 - e0 <= kPullWave) {
+                    s_wave[atomicAdd(&s_waves, 1)] = r;
+                } else {
+                    s_block[atomicAdd(&s_blocks, 1)] = r;
+                }
+            }
+        }
+        __syncthreads();
+        walk(std::integral_constant<int, kWave>{}, s_wave, s_waves);
+        walk(std::integral_constant<int, 16>{}, s_group, s_groups);
+        for (int i = 0; i < s_blocks; ++i) {  // the same count for all: s_blocks is settled
+            const int row = s_block[i];
+            const unsigned int e0 = in_index[row], e1 = in_index[row + 1];
+            const Value was = pull.at(row);
+            if (tid == 0) s_best = order_of(was);
+            __syncthreads();
+            Value best = was;
+            for (unsigned int base = e0; base < e1; base += 4 * kPullThreads) {
+                int u[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const unsigned int e = base + k * kPullThreads + tid;
+                    u[k] = in_src[e < e1 ? e : e1 - 1];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const Value x = pull.offer(u[k], was);
+                    best = x < best ? x : best;
+                }
+                if (__syncthreads_or(pull.settles(best))) break;
+            }
+            if (best < was) atomicMin(&s_best, order_of(best));
+            __syncthreads();
+            if (tid == 0) lower(row, was, value_of_order(s_best, was));
+            __syncthreads();
+        }
+        __syncthreads();
+        const bool full = (int)(s_buf.held >> 32) > kPullList - kPullThreads;
+        __syncthreads();  // everyone has read it before anyone adds again
+        if (full) s_buf.flush(lists.vertex[0], lists.offset[0], counters);
+    }
+    __syncthreads();
+    s_buf.flush(lists.vertex[0], lists.offset[0], counters);
+    end_round(state, now.mark + 1, now.rounds + 1, 0, counters, ticket);
+}
+
+// Push rounds of a short list inside ONE launch: a single work-group keeps the list in LDS, builds the next one there and
+// goes on with it for as long as it has at most kSmallEdges out-edges and is not empty, up to max_rounds rounds.
+// What bounds it is a hop's chain of dependent loads - the edge's target, then the target's value and its row's bounds - so
+// everything else stays out of the chain: the lists and the round's new values live in LDS (a hash table finds a target that
+// several edges lower), no global atomics (only this work-group writes), and a round's values are stored beside the next
+// round's first loads.  Edges are dealt out one per lane across the listed vertices.  While a list has no more edges than a
+// wavefront has lanes, the first wavefront goes on alone, without barriers.  A hop of a 20,000-vertex path 2.0 -> 0.95 us, a
+// round of a 593 x 130 grid 50 -> 2.6 us (lists in global memory, atomics, a wavefront per listed vertex before).
+// Ordering: a value or flag is stored by a plain store before a point that waits for it (a barrier, or the lone
+// wavefront's own wait), and read behind that point by the same work-group, i.e. through the same L1.
+// Longer lists are left alone.  It runs rounds until `most_rounds` of the call are done.
+constexpr int kSmallEdges = 4096, kSmallThreads = 1024;
+constexpr int kSmallSlots = 2 * kSmallEdges;  // of the hash table: at most half full
+constexpr size_t kSmallLds = sizeof(int) * (5 * kSmallEdges + 2 * kSmallSlots);
+
+template <typename Push>
+struct SmallRounds {
+    using Value = typename Push::Value;
+    int *s_start, *s_edge, *s_vertex, *s_val, *s_slot_vertex, *s_slot_val;
+    Value *s_old;
+    unsigned long long *s_counters;  // [2]: of the current list and of the one being built, by turns
+    int *s_ends;                     // [2]: lowered vertices without out-edges: kept from the list's far end
+    const int *__restrict__ index;
+    const int *__restrict__ dst;
+    Push push;
+    int *active;
+    int first_mark;
+
+    __device__ __forceinline__ void store(int i, int mark) const
+    {
+        const int v = s_vertex[i];
+        const Value nv = value_of_order(s_val[i], Value{});
+        push.store(v, nv);
+        if (Push::activates(s_old[i], nv)) active[v] = mark;
+    }
+
+    // T = lanes that take part: the work-group, or its first wavefront.
+    template <int T>
+    static __device__ __forceinline__ void meet()
+    {
+        if constexpr (T == kWave) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
+    }
+
+    // Runs rounds while the list has at most `most` edges; rounds / pending: how many ran, whether the list's values are
+    // still to be stored.  Starts and ends behind a meeting point.
+    template <int T, int PER>
+    __device__ __forceinline__ void run(int most, int max_rounds, int &rounds, bool &pending) const
+    {
+        const int tid = threadIdx.x;
+        for (;;) {
+            const int now = rounds & 1, n = (int)(s_counters[now] >> 32), m = (int)(s_counters[now] & 0xFFFFFFFFull), ends = s_ends[now];
+            if (n + ends == 0 || m > most || n > PER * T || ends > PER * T || rounds >= max_rounds) break;
+            if (T > kWave && m <= kWave && n <= kWave && ends <= kWave && m > 0) break;  // a wavefront's work
+            int t[PER], e[PER];
+            Value nv[PER];
+            // the edges' targets, and beside them the stores of the last round's values
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const int j = tid + k * T;
+                if (j < m) {
+                    int lo = 0, hi = n;
+                    while (hi - lo > 1) {
+                        const int mid = (lo + hi) >> 1;
+                        if (s_start[mid] <= j) lo = mid; else hi = mid;
+                    }
+                    e[k] = s_edge[lo] + (j - s_start[lo]);
+                    t[k] = dst[e[k]];
+                    nv[k] = push.relax(value_of_order(s_val[lo], Value{}), e[k]);
+                }
+            }
+            if (pending) {
+                for (int i = tid; i < n; i += T) store(i, first_mark + rounds - 1);
+                for (int i = tid; i < ends; i += T) store(kSmallEdges - 1 - i, first_mark + rounds - 1);
+            }
+            meet<T>();  // the list has been read and its values are stored
+            Value old[PER];
+            int r0[PER], r1[PER];
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                if (tid + k * T < m) {
+                    old[k] = push.at(t[k]);
+                    r0[k] = index[t[k]];
+                    r1[k] = index[t[k] + 1];
+                }
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                if (tid + k * T < m && nv[k] < old[k]) {
+                    unsigned int slot = ((unsigned int)t[k] * 0x9E3779B1u) >> 19;
+                    static_assert(kSmallSlots == 1 << 13, "the hash keeps 13 bits");
+                    int found;
+                    while ((found = atomicCAS(&s_slot_vertex[slot], -1, t[k])) != -1 && found != t[k]) slot = (slot + 1) & (kSmallSlots - 1);
+                    if (found == -1) {  // first edge to lower it
+                        int i;
+                        if (r1[k] > r0[k]) {
+                            const unsigned long long p = atomicAdd(&s_counters[now ^ 1], (1ull << 32) + (unsigned long long)(r1[k] - r0[k]));
+                            i = (int)(p >> 32);
+                            s_start[i] = (int)(p & 0xFFFFFFFFull);
+                            s_edge[i] = r0[k];
+                        } else {
+                            i = kSmallEdges - 1 - atomicAdd(&s_ends[now ^ 1], 1);
+                        }
+                        s_vertex[i] = t[k];
+                        s_old[i] = old[k];
+                        s_val[i] = (int)slot;
+                    }
+                    atomicMin(&s_slot_val[slot], order_of(nv[k]));
+                }
+            meet<T>();  // the next list is complete
+            const int n2 = (int)(s_counters[now ^ 1] >> 32), ends2 = s_ends[now ^ 1];
+            const auto settle = [&](int i) {  // the vertex's value out of its slot, which is emptied
+                const int slot = s_val[i];
+                s_val[i] = s_slot_val[slot];
+                s_slot_val[slot] = INT_MAX;
+                s_slot_vertex[slot] = -1;
+            };
+            for (int i = tid; i < n2; i += T) settle(i);
+            for (int i = tid; i < ends2; i += T) settle(kSmallEdges - 1 - i);
+            if (tid == 0) {
+                s_counters[now] = 0ull;
+                s_ends[now] = 0;
+            }
+            pending = true;
+            ++rounds;
+            meet<T>();
+        }
+    }
+};
+
+template <typename Push>
+__global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(TraverseState *state, Lists lists, const int *__restrict__ index,
+                                                                         const int *__restrict__ dst, Push push, int *active,
+                                                                         int most_rounds)
+{
+    extern __shared__ int s_small[];
+    __shared__ unsigned long long s_counters[2];
+    __shared__ int s_ends[2], s_rounds, s_pending;
+    SmallRounds<Push> sr;
+    sr.s_start = s_small;
+    sr.s_edge = sr.s_start + kSmallEdges;
+    sr.s_vertex = sr.s_edge + kSmallEdges;
+    sr.s_val = sr.s_vertex + kSmallEdges;
+    sr.s_old = reinterpret_cast<typename Push::Value *>(sr.s_val + kSmallEdges);
+    sr.s_slot_vertex = sr.s_val + 2 * kSmallEdges;
+    sr.s_slot_val = sr.s_slot_vertex + kSmallSlots;
+    sr.s_counters = s_counters;
+    sr.s_ends = s_ends;
+    sr.index = index;
+    sr.dst = dst;
+    sr.push = push;
+    sr.active = active;
+    const int tid = threadIdx.x;
+    const TraverseState start = *state;
+    if ((start.listed & 0xFFFFFFFFull) > (unsigned long long)kSmallEdges || start.listed == 0) return;
+    const int count = (int)(start.listed >> 32), edges = (int)(start.listed & 0xFFFFFFFFull), mark = start.mark;
+    const int max_rounds = most_rounds - start.rounds;
+    int *list = lists.vertex[start.which & 1], *offset = lists.offset[start.which & 1];
+    sr.first_mark = mark;
+    for (int i = tid; i < kSmallSlots; i += kSmallThreads) {
+        sr.s_slot_vertex[i] = -1;
+        sr.s_slot_val[i] = INT_MAX;
+    }
+    for (int i = tid; i < count; i += kSmallThreads) {
+        const int v = list[i];
+        sr.s_start[i] = offset[i];
+        sr.s_edge[i] = index[v];
+        sr.s_val[i] = order_of(push.at(v));
+    }
+    if (tid == 0) {
+        s_counters[0] = ((unsigned long long)count << 32) + (unsigned long long)edges;
+        s_counters[1] = 0ull;
+        s_ends[0] = s_ends[1] = 0;
+    }
+    __syncthreads();
+    int rounds = 0;
+    bool pending = false;
+    for (;;) {
+        const int now = rounds & 1, n = (int)(s_counters[now] >> 32), m = (int)(s_counters[now] & 0xFFFFFFFFull), ends = s_ends[now];
+        if (n + ends == 0 || m > kSmallEdges || rounds >= max_rounds) break;
+        if (m > 0 && m <= kWave && n <= kWave && ends <= kWave) {
+            if (tid < kWave) {
+                sr.template run<kWave, 1>(kWave, max_rounds, rounds, pending);
+                if (tid == 0) {
+                    s_rounds = rounds;
+                    s_pending = pending;
+                }
+            }
+            __syncthreads();
+            rounds = s_rounds;
+            pending = s_pending != 0;
+            __syncthreads();
+        } else {
+            sr.template run<kSmallThreads, kSmallEdges / kSmallThreads>(kSmallEdges, max_rounds, rounds, pending);
+        }
+    }
+    const int now = rounds & 1, n = (int)(s_counters[now] >> 32), ends = s_ends[now];
+    if (pending) {
+        for (int i = tid; i < n; i += kSmallThreads) {
+            sr.store(i, mark + rounds - 1);
+            list[i] = sr.s_vertex[i];
+            offset[i] = sr.s_start[i];
+        }
+        for (int i = tid; i < ends; i += kSmallThreads) sr.store(kSmallEdges - 1 - i, mark + rounds - 1);
+    }
+    if (tid == 0) {
+        state->listed = s_counters[now];
+        state->mark = mark + rounds;
+        state->rounds = start.rounds + rounds;
+    }
+}
+
+__global__ void set_state_kernel(TraverseState *state, TraverseState to) { *state = to; }
+
+void allow_small_lds()
+{
+    for (const void *kernel : {reinterpret_cast<const void *>(&push_rounds_small_kernel<CcPush>),
+                               reinterpret_cast<const void *>(&push_rounds_small_kernel<SsspPush>)})
+        DRONE_HIP_OR_DIE(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+}
+
+// A list with at most this many out-edges is pushed along them; for a longer one a sweep costs less: a push costs
+// the list's out-edges and two atomics per vertex it lowers, a sweep up to all edges but nothing per vertex.
+constexpr unsigned kPullShare = 16;
+unsigned long long push_limit(const GraphExt *x) { return std::max((unsigned long long)x->edges / kPullShare, (unsigned long long)kSmallEdges); }
+
+// List 0 <- the vertices with active == value.
+void launch_collect(Graph *g, TraverseExt *t, int value, int next_mark, int rounds, hipStream_t s)
 {
     const int n = getLocalVertexSize(g);
-    collect_frontier_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, value, g->index, list, t->counters, t->ticket,
-                                                            t->host);
-    return read_counters(t, s, true);
+    collect_frontier_kernel<<<std::min(t->blocks, 512), kSpmvBlock, 0, s>>>(n, g->active, value, g->index, t->lists, t->counters,
+                                                                           t->ticket, t->state, next_mark, rounds);
 }
 
-// Runs rounds until nothing changes.  `fr` describes the vertices that still have to propagate and sit in
-// t->frontier[0] (count 0 with all_active = true means "every vertex": the first round is a sweep).  Returns the
-// number of rounds, or -1 when the bound of n + 1 rounds is exceeded (a cycle of negative length).
-template <typename V, typename Epi, typename Push>
-int run_to_fixed_point(Graph *g, TraverseExt *t, Epi epi, Push push, Frontier fr, bool all_active, hipStream_t s)
+template <typename Pull>
+void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
+    pull_open_kernel<Pull><<<(unsigned)std::min<int64_t>(ceil_div(x->n, kPullThreads), kPullBlocks), kPullThreads, 0, s>>>(
+        t->state, push_limit(x), x->n, x->in_index, x->in_src, pull, g->active, g->index, t->lists, t->counters, t->ticket);
+}
+
+// Runs rounds until nothing changes, from what *t->state says is left to propagate.  What it takes of `run`:
+//   run.push                 the relaxation along out-edges
+//   run.sweep(mark)          launches a sweep over all in-edges that marks what it lowers
+//   run.speculates(state)    whether pull() may be launched before its round is known to come
+//   run.can_pull(state)      whether pull() may do the next round
+//   run.pull()               launches a sweep over the open vertices that lists what it lowers
+// Returns the number of rounds, or -1 when the bound of n + 1 rounds is exceeded (a cycle of negative length).
+//
+// A wait for the GPU costs ~12 us and a launch that finds nothing to do ~3, so the host enqueues the kinds of rounds that
+// usually follow each other - a list grows past what one work-group takes, then past what is worth pushing, and shrinks
+// again - and only then waits.  Breadth-first distances over 1 M vertices and 11.5 M edges: 550 us with a wait per round and sweeps
+// over all edges, 269 with the kernels here and a wait per round, 128 with the rounds enqueued together; labels of
+// 500,009 vertices 880, 440, 244.
+template <typename Run>
+int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, bool all_active, hipStream_t s)
+{
+    using Push = decltype(run.push);
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
     const int n = x->n;
-    const unsigned long long push_limit = (unsigned long long)x->edges / 16;
-    int cur = 0, rounds = 0, mark = 0;
-    bool pull = all_active || fr.edges > push_limit;
-    if (!pull && fr.count == 0) return 0;
+    const unsigned long long limit = push_limit(x);
+    const auto small = [&] {
+        push_rounds_small_kernel<Push><<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, g->dst, run.push, g->active, n + 2);
+    };
+    const auto push = [&](int times) {  // there are such lists at all if limit > kSmallEdges
+        const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div((int64_t)limit, kPushThreads), kPushBlocks);
+        for (int i = 0; i < times && limit > (unsigned long long)kSmallEdges; ++i)
+            push_round_kernel<Push><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, limit, t->lists, g->index, g->dst, run.push,
+                                                                  g->active, t->counters, t->ticket);
+    };
+    TraverseState now{};
+    bool known = false;
+    int sweeps = 1;  // per wait: doubles while nothing else is to be done
+    const auto pull_maybe = [&](int times) {
+        for (int i = 0; i < times && run.speculates(now) && (unsigned long long)x->edges > limit; ++i) run.pull();
+    };
+    if (all_active) {
+        run.sweep(1);  // nothing is final yet: all edges once
+        now = TraverseState{everything(), 2, 1, 0, 0.0};
+        set_state_kernel<<<1, 1, 0, s>>>(t->state, now);
+        known = true;
+    }
     for (;;) {
-        if (rounds > n + 1) return -1;
-        ++rounds;
-        ++mark;  // cc.cu:37 `active[v] = step + 1`: positive, and different in every round
-        if (pull) {
-            epi.mark = mark;
-            spmv_merge_launch<V, int, kIpt, Epi>(x->mt, x->ms, x->in_index, x->in_src, epi, t->stat, s, stat_landing(t));
-            DRONE_HIP_OR_DIE(hipGetLastError());
-            const double changed = read_stat(t, s);
-            if (changed == 0.0) return rounds;
-            if (changed <= (double)n / 16) {  // few enough to be worth listing
-                cur = 0;
-                fr = collect_frontier(g, t, mark, t->frontier[0], s);
-                pull = fr.edges > push_limit;
-            }
-        } else if (fr.count <= (unsigned long long)kSmallCount && fr.edges <= (unsigned long long)kSmallEdges) {
-            const int left = n + 3 - rounds;  // rounds this launch may run: the bound of n + 1 trips at the next check
-            push_rounds_small_kernel<Push><<<1, 256, 0, s>>>((int)fr.count, t->frontier[cur], t->frontier[cur ^ 1], g->index, g->dst,
-                                                           push, g->active, mark, left, t->host);
-            DRONE_HIP_OR_DIE(hipGetLastError());
-            DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
-            const int ran = (int)t->host[2];
-            fr = Frontier{t->host[0] >> 32, t->host[0] & 0xFFFFFFFFull, t->host[1]};
-            rounds += ran - 1;
-            mark += ran - 1;
-            cur ^= ran & 1;
-            if (fr.count == 0) return rounds;
-            pull = fr.edges > push_limit;
+        const unsigned long long edges = now.listed & 0xFFFFFFFFull;
+        int sweeps_next = 1;
+        if (!known || edges <= (unsigned long long)kSmallEdges) {
+            small();
+            push(1);
+            pull_maybe(2);
+            push(2);
+            small();
+        } else if (edges <= limit) {
+            push(3);
+            small();
+        } else if (run.can_pull(now)) {
+            run.pull();
+            pull_maybe(1);
+            push(3);
+            small();
         } else {
-            const int waves_per_block = 256 / kWave;
-            const int gx = (int)(ceil_div((int64_t)fr.count, waves_per_block) < 16384 ? ceil_div((int64_t)fr.count, waves_per_block) : 16384);
-            const int gy = (int)ceil_div((int64_t)(fr.max_degree > 0 ? fr.max_degree : 1), kPushChunk);
-            const bool publish = (int64_t)gx * gy <= kPublishMaxBlocks;
-            push_round_kernel<Push><<<dim3(gx, gy), 256, 0, s>>>((int)fr.count, t->frontier[cur], g->index, g->dst, push, g->active,
-                                                         mark, t->frontier[cur ^ 1], t->counters, publish ? t->ticket : nullptr, t->host);
-            DRONE_HIP_OR_DIE(hipGetLastError());
-            fr = read_counters(t, s, publish);
-            cur ^= 1;
-            if (fr.count == 0) return rounds;
-            pull = fr.edges > push_limit;  // a sweep covers whatever the listed vertices still had to propagate
+            for (int i = 0; i < sweeps; ++i) run.sweep(now.mark + i);
+            launch_collect(g, t, now.mark + sweeps - 1, now.mark + sweeps, now.rounds + sweeps, s);
+            push(1);
+            small();
+            sweeps_next = std::min(2 * sweeps, 8);
         }
+        sweeps = sweeps_next;
+        launch_report(g, t, false, s);
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+        now = t->report->state;
+        known = true;
+        if (now.listed == 0) return now.rounds;
+        if (now.rounds > n + 1) return -1;
     }
 }
 
@@ -549,22 +1076,69 @@ void ensure_in_edge_ids(Graph *g, hipStream_t s)
     (void)hipFree(iota);
 }
 
-// Brings x->in_len (edge lengths in in-edge order) up to date with g->edgeLen.  build_graph leaves every length at
-// 1.0 and few callers change that, so a streaming check for "all ones" comes first: it avoids the random gather
-// through in_eid, which costs more than a whole sweep.
-void refresh_in_edge_lengths(Graph *g, TraverseExt *t, hipStream_t s)
-{
-    GraphExt *x = static_cast<GraphExt *>(g->ext);
-    if (x->edges == 0) return;
-    count_not_one_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(x->edges, g->edgeLen, t->block_part);
-    if (reduce_parts(t, s) == 0.0) {
-        if (!x->in_len_ones) fill_f32_kernel<<<1024, 256, 0, s>>>(x->in_len, 1.0f, x->edges);
-        x->in_len_ones = true;
-        return;
+struct CcRun {
+    Graph *g;
+    TraverseExt *t;
+    int *cc;
+    hipStream_t s;
+    CcPush push{cc};
+    bool speculates(const TraverseState &) const { return true; }
+    bool can_pull(const TraverseState &) const { return true; }
+    void pull() { launch_pull(g, t, CcPull{cc}, s); }
+    void sweep(int mark)
+    {
+        GraphExt *x = static_cast<GraphExt *>(g->ext);
+        spmv_merge_launch<MinI32, int, kIpt>(x->mt, x->ms, x->in_index, x->in_src, CcEpi{cc, g->active, mark}, t->stat, s);
     }
-    gather_len_kernel<<<1024, 256, 0, s>>>(x->edges, x->in_eid, g->edgeLen, x->in_len);
-    x->in_len_ones = false;
-}
+};
+
+// levels: the rounds start from one vertex, so over unit lengths round k reaches the vertices at distance k.  Whether all
+// lengths are 1.0 (as build_graph leaves them) is counted on the device, at the start of such a call and otherwise when a
+// sweep first needs to know it, as are the lengths in in-edge order, whose random gather costs more than a whole sweep.
+struct SsspRun {
+    Graph *g;
+    TraverseExt *t;
+    float *dist;
+    hipStream_t s;
+    bool levels;
+    SsspPush push{dist, g->edgeLen};
+    bool counted = false, gathered = false;
+
+    void count_lengths()
+    {
+        GraphExt *x = static_cast<GraphExt *>(g->ext);
+        count_not_one_kernel<<<sum_blocks(x->edges, 16), kSpmvBlock, 0, s>>>(x->edges, g->edgeLen, t->block_part, t->ticket, &t->state->not_one);
+        counted = true;
+    }
+    bool unit_lengths()  // between waits
+    {
+        if (!counted) {
+            count_lengths();
+            launch_report(g, t, false, s);
+            DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+        }
+        return t->report->state.not_one == 0.0;
+    }
+    bool speculates(const TraverseState &now) const { return levels && now.not_one == 0.0; }
+    bool can_pull(const TraverseState &now) { return levels && now.rounds < LevelPull::kMostRounds && unit_lengths(); }
+    void pull() { launch_pull(g, t, LevelPull{dist}, s); }
+    void sweep(int mark)
+    {
+        GraphExt *x = static_cast<GraphExt *>(g->ext);
+        if (unit_lengths()) {
+            spmv_merge_launch<MinF32, int, kIpt>(x->mt, x->ms, x->in_index, x->in_src, SsspUnitEpi{{dist, nullptr, g->active, mark}},
+                                                 t->stat, s);
+            return;
+        }
+        if (!gathered) {
+            ensure_in_edge_ids(g, s);
+            gather_len_kernel<<<1024, 256, 0, s>>>(x->edges, x->in_eid, g->edgeLen, x->in_len);
+            gathered = true;
+        }
+        spmv_merge_launch<MinF32, int, kIpt>(x->mt, x->ms, x->in_index, x->in_src, SsspEpi{dist, x->in_len, g->active, mark},
+                                             t->stat, s);
+    }
+};
 
 template <typename Policy, typename T>
 void exchange_values(Graph *g, T *vals, int **send_id, int **recv_id, T **send_val, T **recv_val, int workerId,
@@ -609,16 +1183,16 @@ extern "C" Response CC_PEVal(Graph *g, CCValues *values, int workerId, int worke
         values->ext = traverse_ext_create(n);
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    cc_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, values->ccValue, g->updateByMessage);
-    if (n > 0)  // every vertex starts active (cc.cu:16): the first round is a sweep
-        run_to_fixed_point<MinI32>(g, t, CcEpi{values->ccValue, g->active, 1}, CcPush{values->ccValue}, Frontier{}, true, s);
+    cc_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, values->ccValue, g->updateByMessage, t->state);
+    CcRun run{g, t, values->ccValue, s};
+    if (n > 0) run_to_fixed_point(g, t, run, true, s);
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
     exchange_values<CcExchange>(g, values->ccValue, &values->sendID, &values->recvID, &values->sendCCValue,
                                 &values->recvCCValue, workerId, workerNum, comm, &res);
     res.SendTime = (float)seconds_since(t1);
-    res.VisitedSize = count_active(g, t, s);
+    res.VisitedSize = workerNum <= 1 && t->report->state.listed == 0 ? (int)t->report->visited : count_active(g, t, s);
     return res;
 }
 
@@ -635,18 +1209,17 @@ extern "C" Response CC_IncEVal(Graph *g, CCValues *values, int workerId, int wor
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
     const int n = getLocalVertexSize(g);
-    process_messages_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage, t->block_part);
-    if (reduce_parts(t, s) > 0.0) {  // cc.cu:425: no message, no round
-        const Frontier fr = collect_frontier(g, t, 0, t->frontier[0], s);  // the vertices a message activated
-        run_to_fixed_point<MinI32>(g, t, CcEpi{values->ccValue, g->active, 1}, CcPush{values->ccValue}, fr, false, s);
-    }
+    process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
+    launch_collect(g, t, 0, 1, 0, s);  // cc.cu:425: the vertices a message activated propagate
+    CcRun run{g, t, values->ccValue, s};
+    run_to_fixed_point(g, t, run, false, s);
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
     exchange_values<CcExchange>(g, values->ccValue, &values->sendID, &values->recvID, &values->sendCCValue,
                                 &values->recvCCValue, workerId, workerNum, comm, &res);
     res.SendTime = (float)seconds_since(t1);
-    res.VisitedSize = count_active(g, t, s);
+    res.VisitedSize = workerNum <= 1 && t->report->state.listed == 0 ? (int)t->report->visited : count_active(g, t, s);
     return res;
 }
 
@@ -676,31 +1249,25 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
         set_error(DRONE_ERR_INVALID, "SSSP_PEVal: startId %d is outside [0, %d)", startId, nglobal);
         die("SSSP_PEVal");
     }
-    int start = -1;  // sssp.cu:405-406
-    DRONE_HIP_OR_DIE(hipMemcpy(&start, g->Global2Local + startId, sizeof(int), hipMemcpyDeviceToHost));
     ensure_aggregation_ready(g);
     ensure_flags(g);
-    ensure_in_edge_ids(g, s);
-    GraphExt *x = static_cast<GraphExt *>(g->ext);
     if (!values->ext) {  // sssp.cu:408-411
         DRONE_HIP_OR_DIE(hipMalloc(&values->distance, sizeof(float) * (size_t)(n > 0 ? n : 1)));
         values->ext = traverse_ext_create(n);
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    refresh_in_edge_lengths(g, t, s);
-    sssp_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, start, g->active, values->distance, g->updateByMessage);
-    if (start >= 0) {  // sssp.cu:30: only the worker that holds the start vertex has anything to do
-        const Frontier fr = collect_frontier(g, t, 0, t->frontier[0], s);  // the start vertex
-        report_rounds(run_to_fixed_point<MinF32>(g, t, SsspEpi{values->distance, x->in_len, g->active, 1},
-                                                 SsspPush{values->distance, g->edgeLen}, fr, false, s), "SSSP_PEVal");
-    }
+    sssp_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage,
+                                                     g->index, t->lists.vertex[0], t->lists.offset[0], t->state);
+    SsspRun run{g, t, values->distance, s, true};
+    run.count_lengths();
+    report_rounds(run_to_fixed_point(g, t, run, false, s), "SSSP_PEVal");
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
     exchange_values<SsspExchange>(g, values->distance, &values->sendID, &values->recvID, &values->sendDis,
                                   &values->recvDis, workerId, workerNum, comm, &res);
     res.SendTime = (float)seconds_since(t1);
-    res.VisitedSize = count_active(g, t, s);
+    res.VisitedSize = workerNum <= 1 && t->report->state.listed == 0 ? (int)t->report->visited : count_active(g, t, s);
     return res;
 }
 
@@ -716,21 +1283,18 @@ extern "C" Response SSSP_IncEVal(Graph *g, SSSPValues *values, int workerId, int
         die("SSSP_IncEVal");
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    GraphExt *x = static_cast<GraphExt *>(g->ext);
     const int n = getLocalVertexSize(g);
-    process_messages_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage, t->block_part);
-    if (reduce_parts(t, s) > 0.0) {
-        const Frontier fr = collect_frontier(g, t, 0, t->frontier[0], s);
-        report_rounds(run_to_fixed_point<MinF32>(g, t, SsspEpi{values->distance, x->in_len, g->active, 1},
-                                                 SsspPush{values->distance, g->edgeLen}, fr, false, s), "SSSP_IncEVal");
-    }
+    process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
+    launch_collect(g, t, 0, 1, 0, s);
+    SsspRun run{g, t, values->distance, s, false};
+    report_rounds(run_to_fixed_point(g, t, run, false, s), "SSSP_IncEVal");
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
     exchange_values<SsspExchange>(g, values->distance, &values->sendID, &values->recvID, &values->sendDis,
                                   &values->recvDis, workerId, workerNum, comm, &res);
     res.SendTime = (float)seconds_since(t1);
-    res.VisitedSize = count_active(g, t, s);
+    res.VisitedSize = workerNum <= 1 && t->report->state.listed == 0 ? (int)t->report->visited : count_active(g, t, s);
     return res;
 }
 
