@@ -65,6 +65,22 @@ struct SsspExchange {
     }
 };
 
+// ---- workers of one loopback group: they share the address space and, as a rule, the GPU
+// What a worker shows the others when they meet to synchronise rows in place.
+struct RowsOffer {
+    Graph *g = nullptr;
+    float *data = nullptr;
+    int ld = 0, K = 0;
+    bool compress = false;
+    std::vector<uint64_t> planned_with;  // DirectRows::with
+    bool agrees = false;                 // its tables agree with the others'; set between the meeting and a barrier
+};
+bool loopback_is(const drone_transport *tr, int workerNum);
+// Shows `mine` and waits for everybody.  An error if somebody is in another kind of step.
+int loopback_rows_meet(drone_transport *tr, int workerId, const RowsOffer &mine);
+RowsOffer &loopback_offer(drone_transport *tr, int worker);
+int loopback_barrier(drone_transport *tr);
+
 // Builds the static lists on first use (reads the routing tables back from the device).
 int routes_prepare(Graph *g, int workerNum);
 void routes_release(RouteLists *r);

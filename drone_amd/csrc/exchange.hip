@@ -2,9 +2,11 @@
 #include "exchange.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <condition_variable>
 #include <mutex>
+#include <thread>
 #include <rocprim/device/device_scan.hpp>
 
 using namespace drone;
@@ -250,6 +252,8 @@ int drone::routes_prepare(Graph *g, int workerNum)
     DRONE_HIP_TRY(hipHostMalloc(&r.chunk_count_h, sizeof(int) * ((size_t)most_chunks + 1)));
     DRONE_HIP_TRY(hipMemset(r.chunk_count, 0, sizeof(int) * ((size_t)most_chunks + 1)));
     r.unknown_reported = 0;
+    static std::atomic<uint64_t> last_id{0};
+    r.id = ++last_id;
     r.workers = workerNum;
     r.ready = true;
     return DRONE_OK;
@@ -353,15 +357,17 @@ struct drone_loopback {
     std::mutex mu;
     std::condition_variable cv;
     int waiting = 0;
-    uint64_t generation = 0;
-    bool broken = false;
-    static constexpr int kMaxArrays = 4;
+    std::atomic<uint64_t> generation{0};
+    std::atomic<bool> broken{false};
+    static constexpr int kMaxArrays = 4, kSpinMicroseconds = 100;
     struct Slot {
         const int *send_len = nullptr, *send_index = nullptr;
         int n_arrays = 0;
         const void *send[kMaxArrays] = {};
         size_t elem_bytes[kMaxArrays] = {};
         float *scalar = nullptr;
+        bool in_rows = false;  // the worker is in loopback_rows_meet, not in an exchange
+        RowsOffer rows;
     };
     std::vector<Slot> slot;
     struct Endpoint {
@@ -372,6 +378,8 @@ struct drone_loopback {
     float *scalars = nullptr, *sums = nullptr;  // pinned [workers] each: staging of the all-reduce
 
     // Returns false when a peer did not arrive in time (the group is then unusable).
+    // Workers mostly arrive within microseconds of each other, and being woken from a condition variable takes tens of
+    // them: a worker first looks for a while whether the last one has come (if each has a core to itself).
     bool barrier()
     {
         std::unique_lock<std::mutex> lk(mu);
@@ -384,6 +392,13 @@ struct drone_loopback {
             return true;
         }
         auto arrived = [&] { return generation != gen || broken; };
+        if (workers <= (int)std::thread::hardware_concurrency()) {
+            lk.unlock();
+            const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kSpinMicroseconds);
+            while (!arrived() && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+            lk.lock();
+            if (arrived()) return !broken;
+        }
         if (timeout_ms > 0) {
             if (!cv.wait_for(lk, std::chrono::milliseconds(timeout_ms), arrived)) {
                 broken = true;
@@ -417,6 +432,7 @@ int loopback_exchange(void *ctx, int workerId, int workerNum, const int *send_le
     mine.send_len = send_len;
     mine.send_index = send_index;
     mine.n_arrays = n_arrays;
+    mine.in_rows = false;
     for (int a = 0; a < n_arrays; ++a) {
         mine.send[a] = send[a];
         mine.elem_bytes[a] = elem_bytes[a];
@@ -427,9 +443,9 @@ int loopback_exchange(void *ctx, int workerId, int workerNum, const int *send_le
         recv_len[w] = 0;
         if (w == workerId) continue;
         const drone_loopback::Slot &src = grp->slot[w];
-        const int len = src.send_len[workerId];
-        if (len <= 0) continue;
-        if (src.n_arrays != n_arrays) {
+        const int len = src.in_rows ? 0 : src.send_len[workerId];
+        if (len <= 0 && !src.in_rows) continue;
+        if (src.in_rows || src.n_arrays != n_arrays) {
             set_error(DRONE_ERR_INVALID, "loopback transport: workers %d and %d are in different exchange steps", workerId, w);
             rc = DRONE_ERR_INVALID;
             break;
@@ -483,6 +499,36 @@ int loopback_allreduce(void *ctx, int workerId, int workerNum, float *device_sca
 }
 
 }  // namespace
+
+bool drone::loopback_is(const drone_transport *tr, int workerNum)
+{
+    return tr->exchange == loopback_exchange && static_cast<drone_loopback::Endpoint *>(tr->ctx)->group->workers == workerNum;
+}
+
+RowsOffer &drone::loopback_offer(drone_transport *tr, int worker)
+{
+    return static_cast<drone_loopback::Endpoint *>(tr->ctx)->group->slot[(size_t)worker].rows;
+}
+
+int drone::loopback_barrier(drone_transport *tr)
+{
+    return static_cast<drone_loopback::Endpoint *>(tr->ctx)->group->barrier() ? DRONE_OK : loopback_fail("rows");
+}
+
+int drone::loopback_rows_meet(drone_transport *tr, int workerId, const RowsOffer &mine)
+{
+    drone_loopback *grp = static_cast<drone_loopback::Endpoint *>(tr->ctx)->group;
+    grp->slot[(size_t)workerId].rows = mine;
+    grp->slot[(size_t)workerId].in_rows = true;
+    if (!grp->barrier()) return loopback_fail("rows");
+    for (const drone_loopback::Slot &s : grp->slot)
+        if (!s.in_rows || s.rows.K != mine.K || s.rows.compress != mine.compress) {
+            set_error(DRONE_ERR_INVALID, "loopback transport: the workers are in different exchange steps");
+            if (!grp->barrier()) return loopback_fail("rows");
+            return DRONE_ERR_INVALID;
+        }
+    return DRONE_OK;
+}
 
 extern "C" int drone_loopback_create(drone_loopback **group, int workerNum, int timeout_ms)
 {

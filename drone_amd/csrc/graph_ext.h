@@ -13,6 +13,7 @@ namespace drone {
 // Static send lists of the replica exchange and the scratch of one pack step.
 struct RouteLists {
     bool ready = false;
+    uint64_t id = 0;               // never given out twice
     int workers = 0;
     int mirror_items = 0;          // = MirrorSize
     int master_items = 0;          // = MirrorWorkerSize: one item per (master, worker holding a mirror of it)
@@ -41,8 +42,19 @@ struct RouteLists {
 };
 constexpr int kExchangeChunk = 1024;
 
+// The row synchronisation between workers that can reach each other's rows: what this worker does as a master.
+struct DirectRows {
+    std::vector<uint64_t> with;   // RouteLists::id of all workers it was made for; empty: not made
+    bool usable = false;          // the workers' tables agree with each other
+    int masters = 0;              // masters with a mirror somewhere
+    int *master_row = nullptr;    // device [masters]: local id
+    int *first = nullptr;         // device [masters + 1]: their mirrors, ascending by worker
+    int2 *mirror = nullptr;       // device [first[masters]]: worker, local id there
+};
+
 // Staging of the K-wide row synchronisation (grow-only).
 struct RowSync {
+    DirectRows direct;
     int capacity = 0;        // rows
     size_t row_elems = 0;    // capacity * K the row buffers were sized for
     int *send_id = nullptr, *recv_id = nullptr;
@@ -50,7 +62,8 @@ struct RowSync {
     uint8_t *send_u8 = nullptr, *recv_u8 = nullptr;
     float *send_maxmin = nullptr, *recv_maxmin = nullptr;
 };
-void row_sync_release(RowSync *rs);
+void row_sync_release(RowSync *rs);  // staging only
+void direct_rows_release(DirectRows *d);
 
 struct GraphExt {
     int n = 0;

@@ -317,6 +317,7 @@ void drone::graph_ext_release(GraphExt *x)
     if (x->rank64) (void)hipFree(x->rank64);
     routes_release(&x->routes);
     row_sync_release(&x->row_sync);
+    direct_rows_release(&x->row_sync.direct);
     if (x->in_eid) (void)hipFree(x->in_eid);
     if (x->in_len) (void)hipFree(x->in_len);
     *x = GraphExt{};
