@@ -2,41 +2,52 @@
 // getHandle()/run() (cuda_gcn/src/gcn.h:10-12, gcn.cu:22-52) plus the per-epoch calls of its main loop
 // (gcn.cu:96-106 -> CUDAGCN::run_epoch, cuda_gcn.cu:356-379), so a host in any language can drive a training
 // run.  Data loading is out: the caller hands over device arrays.
+#include <algorithm>
 #include <cstring>
-#include <vector>
 
 #include "../../include/drone_gcn_modules.hpp"
-#include "common.h"
+#include "spmv_merge.h"
 
 using namespace drone;
 
 namespace {
-// cuda_kernel.cu:463-467
-__global__ void set_truth_kernel(int *__restrict__ truth, const int *__restrict__ split, const int *__restrict__ label,
-                                 int current_split, int n)
+constexpr int kTruthBlocks = 256;  // work-groups at most
+
+// cuda_kernel.cu:463-467; count (optional): the labelled rows, which the mean-reduced gradient is divided by.
+__global__ __launch_bounds__(kSpmvBlock) void set_truth_kernel(int *__restrict__ truth, const int *__restrict__ split,
+                                                              const int *__restrict__ label, int current_split, int n,
+                                                              int *count, double *part, unsigned int *ticket)
 {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id < n) truth[id] = split[id] == current_split ? label[id] : -1;
+    __shared__ double s_red[kSpmvBlock / kWave];
+    double labelled = 0.0;
+    for (int64_t id = (int64_t)blockIdx.x * kSpmvBlock + threadIdx.x; id < n; id += (int64_t)gridDim.x * kSpmvBlock) {
+        const int t = split[id] == current_split ? label[id] : -1;
+        truth[id] = t;
+        labelled += t >= 0;
+    }
+    if (!count) return;
+    const double total = block_sum_256(labelled, s_red);
+    unsigned int one = 0;
+    if (threadIdx.x == 0) one = publish_part(part + blockIdx.x, total);
+    if (!last_block_done(ticket, one)) return;
+    const double all = block_sum_of_parts(part, (int)gridDim.x, s_red);
+    if (threadIdx.x == 0) *count = (int)all;
 }
 }  // namespace
 
 void drone_gcn_mod::GCN::set_truth(int current_split)
 {
     const int n = params.localVertexSize;
-    set_truth_kernel<<<(n + 255) / 256, 256, 0, static_cast<hipStream_t>(s)>>>(truth, split, label, current_split, n);
-    DRONE_GCN_HIP(hipGetLastError());
-    if (params.mean_gradient && current_split != truth_split) {
-        // number of labelled rows, needed on the host to scale the loss gradient; recounted only when the
-        // split changes (labels and split ids are fixed for the handle's lifetime)
-        std::vector<int> h((size_t)n);
-        DRONE_GCN_HIP(hipMemcpyAsync(h.data(), truth, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost,
-                                     static_cast<hipStream_t>(s)));
-        DRONE_GCN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(s)));
-        truth_count = 0;
-        for (int v : h) truth_count += v >= 0;
-        ce->grad_scale = truth_count > 0 ? 1.0f / (float)truth_count : 1.0f;
+    const size_t part_bytes = sizeof(double) * kTruthBlocks, ticket_bytes = sizeof(unsigned int) * ticket_words(kTruthBlocks);
+    if (truth_count && !truth_scratch) {
+        DRONE_GCN_HIP(hipMalloc(&truth_scratch, part_bytes + ticket_bytes));
+        DRONE_GCN_HIP(hipMemset(truth_scratch, 0, part_bytes + ticket_bytes));
+        DRONE_GCN_HIP(hipStreamSynchronize(nullptr));
     }
-    truth_split = current_split;
+    double *part = static_cast<double *>(truth_scratch);
+    set_truth_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), kTruthBlocks), kSpmvBlock, 0, static_cast<hipStream_t>(s)>>>(
+        truth, split, label, current_split, n, truth_count, part, reinterpret_cast<unsigned int *>(part + kTruthBlocks));
+    DRONE_GCN_HIP(hipGetLastError());
 }
 
 struct drone_gcn {

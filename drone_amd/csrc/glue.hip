@@ -1,11 +1,12 @@
 // Element-wise and per-row kernels on the measured GCN step, semantics as in cuda_gcn/src/cuda/cuda_kernel.cu:
 // ReLU (:384-399), dropout with an explicit keep mask (:403-420), soft-max cross-entropy (:295-379 with the
 // host logic of cuda_module.cu:406-483), Adam (:450-460), plus SGD, accuracy (cuda_gcn.cu:226-246) and arg-max.
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
 
-#include "common.h"
+#include "spmv_merge.h"
 
 namespace drone {
 namespace {
@@ -28,19 +29,49 @@ __device__ __forceinline__ uint64_t splitmix64_dev(uint64_t x)
     return x ^ (x >> 31);
 }
 
+// Four elements per lane when the count and the addresses allow 16-byte accesses (a float and a mask byte at a time: 10 us for
+// 16,000 rows of 64, four: 5).
+template <int V>
 __global__ void relu_forward_kernel(float *__restrict__ x, uint8_t *__restrict__ mask, int64_t n, int training)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const bool keep = x[i] > 0;
-        if (training) mask[i] = keep;
-        if (!keep) x[i] = 0;
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q * V < n; q += (int64_t)gridDim.x * blockDim.x) {
+        if constexpr (V == 4) {
+            float4 t = reinterpret_cast<const float4 *>(x)[q];
+            if (training) reinterpret_cast<uchar4 *>(mask)[q] = make_uchar4(t.x > 0, t.y > 0, t.z > 0, t.w > 0);
+            if (!(t.x > 0)) t.x = 0;
+            if (!(t.y > 0)) t.y = 0;
+            if (!(t.z > 0)) t.z = 0;
+            if (!(t.w > 0)) t.w = 0;
+            reinterpret_cast<float4 *>(x)[q] = t;
+        } else {
+            const bool keep = x[q] > 0;
+            if (training) mask[q] = keep;
+            if (!keep) x[q] = 0;
+        }
     }
 }
 
+template <int V>
 __global__ void relu_backward_kernel(float *__restrict__ g, const uint8_t *__restrict__ mask, int64_t n)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        if (!mask[i]) g[i] = 0;
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q * V < n; q += (int64_t)gridDim.x * blockDim.x) {
+        if constexpr (V == 4) {
+            float4 t = reinterpret_cast<const float4 *>(g)[q];
+            const uchar4 m = reinterpret_cast<const uchar4 *>(mask)[q];
+            if (!m.x) t.x = 0;
+            if (!m.y) t.y = 0;
+            if (!m.z) t.z = 0;
+            if (!m.w) t.w = 0;
+            reinterpret_cast<float4 *>(g)[q] = t;
+        } else {
+            if (!mask[q]) g[q] = 0;
+        }
+    }
+}
+
+inline bool four_wide(const float *x, const uint8_t *mask, int64_t n)
+{
+    return n % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(mask) % 4 == 0;
 }
 
 // keep[i] = u(seed, step, i) >= p with u uniform in [0,1): a pure function of its arguments
@@ -134,25 +165,65 @@ __global__ void relu_dropout_backward_kernel(float *__restrict__ g, const uint8_
 // flight: with one group, every step of the loop was a chain of two memory round trips (logits, then the store of the
 // gradient behind them) and the kernel took 49 us for 232,965 x 41, twice what its 90 MB cost.
 constexpr int kCeGroups = 2;
+constexpr int kLossRowBlocks = 2048, kLossWeightBlocks = 64;  // most work-groups for the rows, for the weights
+constexpr int kLossBlocks = kLossRowBlocks + kLossWeightBlocks;
+
+// Parts of the work-groups: [0] loss, [1] labelled rows, [2] correct rows, [3] counted rows, [4] sum of squares.
+struct LossScratch {
+    double *part;          // [5][kLossBlocks]
+    unsigned int *ticket;  // counters of last_block_done, zero between launches
+    static constexpr size_t bytes() { return sizeof(double) * 5 * kLossBlocks + sizeof(unsigned int) * (kLossBlocks / kTicketGroup + 2) * kTicketStride; }
+};
+
+// A work-group's part of sum x[i]^2, in double: every lane four independent chains (one chain of dependent loads and fp64 adds
+// in a single work-group took 117 us for the 77,056 weights of a 602 x 128 layer).  Valid in thread 0.
+__device__ __forceinline__ double squares_part(const float *__restrict__ x, int64_t n, int block, int blocks, double *s_red)
+{
+    const int64_t step = (int64_t)blocks * kThreads;
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    int64_t i = (int64_t)block * kThreads + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {
+        const float a = x[i], b = x[i + step], c = x[i + 2 * step], d = x[i + 3 * step];
+        t[0] += (double)a * (double)a;
+        t[1] += (double)b * (double)b;
+        t[2] += (double)c * (double)c;
+        t[3] += (double)d * (double)d;
+    }
+    for (; i < n; i += step) t[0] += (double)x[i] * (double)x[i];
+    return block_sum_256((t[0] + t[1]) + (t[2] + t[3]), s_red);
+}
+
+// The loss, the gradient, and what is reported with them, in one launch: the last work-group adds the parts of all.
+// Work-groups past row_blocks add up the squares of the weights meanwhile.  A training step and the report of its loss
+// spent five launches and three copies on this (cross-entropy and its finish, accuracy and the clearing of its counts,
+// sum of squares; ~5 us each where the graph is small): an epoch with its evaluation on 2,708
+// vertices 310 -> 190 us.
 template <int L>
-__global__ __launch_bounds__(kThreads) void cross_entropy_kernel(int n, int classes, const float *__restrict__ logits,
-                                                                 int ld, const int *__restrict__ truth,
-                                                                 float *__restrict__ grad, int ldg, float grad_scale,
-                                                                 double *__restrict__ block_loss,
-                                                                 int *__restrict__ block_count)
+__global__ __launch_bounds__(kThreads) void loss_kernel(drone_loss_pass p, int row_blocks, LossScratch scratch)
 {
     constexpr int R = kWave / L, kWaves = kThreads / kWave, U = kCeGroups;
-    __shared__ double s_loss[kWaves];
-    __shared__ int s_cnt[kWaves];
+    __shared__ double s_red[5][kWaves], s_part[5];
+    const int n = p.n, classes = p.classes, ld = p.ld, ldg = p.ldg;
+    const float *__restrict__ logits = p.logits;
+    const int *__restrict__ truth = p.truth;
+    float *__restrict__ grad = p.grad;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int li = lane % L, sub = lane / L;
     const int per_lane = (classes + L - 1) / L;  // more than 4 only in the 64-lane instance
     double loss = 0.0;
-    int cnt = 0;
-    for (int row0 = (blockIdx.x * kWaves + wave) * R * U; row0 < n; row0 += gridDim.x * kWaves * R * U) {
+    int cnt = 0, correct = 0, counted = 0;
+    double squares = 0.0;
+    if ((int)blockIdx.x >= row_blocks)
+        squares = squares_part(p.weights, p.weight_count, (int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks, s_red[4]);
+    const int mean_over = p.mean_over && grad ? *p.mean_over : 0;
+    const float grad_scale = p.mean_over ? (mean_over > 0 ? 1.0f / (float)mean_over : 1.0f) : p.grad_scale;
+    for (int64_t base = ((int64_t)blockIdx.x * kWaves + wave) * R * U; base < n && (int)blockIdx.x < row_blocks;
+         base += (int64_t)row_blocks * kWaves * R * U) {
+        const int row0 = (int)base;
         if (per_lane <= 4) {
             float z[U][4];
             int t[U];
+            bool skip[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int row = row0 + u * R + sub;
@@ -160,6 +231,7 @@ __global__ __launch_bounds__(kThreads) void cross_entropy_kernel(int n, int clas
 #pragma unroll
                 for (int k = 0; k < 4; ++k) z[u][k] = li + k * L < classes ? src[li + k * L] : -INFINITY;
                 t[u] = row < n ? truth[row] : -1;
+                skip[u] = p.skip && row < n && p.skip[row] != -1;
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -200,6 +272,10 @@ __global__ __launch_bounds__(kThreads) void cross_entropy_kernel(int n, int clas
                 if (li == 0 && labelled) {
                     loss += (double)(logf(sum) - (zt - mx));
                     cnt += 1;
+                    if (!skip[u]) {
+                        counted += 1;
+                        correct += !(mx > zt);
+                    }
                 }
             }
         } else {
@@ -230,48 +306,37 @@ __global__ __launch_bounds__(kThreads) void cross_entropy_kernel(int n, int clas
                 if (li == 0 && labelled) {
                     loss += (double)(logf(sum) - (z[t] - mx));
                     cnt += 1;
+                    if (!p.skip || p.skip[row] == -1) {
+                        counted += 1;
+                        correct += !(mx > z[t]);
+                    }
                 }
             }
         }
     }
+    // (whole numbers below 2^53: exact)
+    const double parts[5] = {block_sum_256(loss, s_red[0]), block_sum_256((double)cnt, s_red[1]),
+                             block_sum_256((double)correct, s_red[2]), block_sum_256((double)counted, s_red[3]), squares};
+    if (threadIdx.x == 0) {
 #pragma unroll
-    for (int m = kWave / 2; m > 0; m >>= 1) {
-        loss += __shfl_xor(loss, m, kWave);
-        cnt += __shfl_xor(cnt, m, kWave);
+        for (int k = 0; k < 5; ++k) s_part[k] = parts[k];
     }
-    if (lane == 0) { s_loss[wave] = loss; s_cnt[wave] = cnt; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double l = 0.0;
-        int c = 0;
-        for (int w = 0; w < kWaves; ++w) { l += s_loss[w]; c += s_cnt[w]; }
-        block_loss[blockIdx.x] = l;
-        block_count[blockIdx.x] = c;
-    }
-}
-
-// loss_out = sum(block_loss) / sum(block_count) (mean over labelled rows), count_out = sum(block_count)
-__global__ __launch_bounds__(kThreads) void cross_entropy_finish_kernel(int blocks, const double *__restrict__ block_loss,
-                                                                        const int *__restrict__ block_count,
-                                                                        float *__restrict__ loss_out,
-                                                                        int *__restrict__ count_out)
-{
-    __shared__ double s_l[kThreads];
-    __shared__ int s_c[kThreads];
-    double l = 0.0;
-    int c = 0;
-    for (int i = threadIdx.x; i < blocks; i += kThreads) { l += block_loss[i]; c += block_count[i]; }
-    s_l[threadIdx.x] = l;
-    s_c[threadIdx.x] = c;
-    __syncthreads();
-    for (int m = kThreads / 2; m > 0; m >>= 1) {
-        if (threadIdx.x < m) { s_l[threadIdx.x] += s_l[threadIdx.x + m]; s_c[threadIdx.x] += s_c[threadIdx.x + m]; }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        if (loss_out) *loss_out = (float)(s_l[0] / (double)s_c[0]);
-        if (count_out) *count_out = s_c[0];
-    }
+    unsigned int one = 0;
+    // five lanes, one instruction: it has returned for all of them when it has for thread 0
+    if (threadIdx.x < 5) one = publish_part(scratch.part + threadIdx.x * kLossBlocks + blockIdx.x, s_part[threadIdx.x]);
+    if (!last_block_done(scratch.ticket, one)) return;
+    double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += kThreads)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) sum[k] += load_agent(scratch.part + k * kLossBlocks + i);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) sum[k] = block_sum_256(sum[k], s_red[k]);
+    if (threadIdx.x != 0) return;
+    const float mean = (float)(sum[0] / sum[1]);  // over the labelled rows
+    if (p.loss) *p.loss = mean;
+    if (p.labelled) *p.labelled = (int)sum[1];
+    if (p.report) *p.report = drone_loss_report{mean, (float)sum[4], (int)sum[1], (int)sum[2], (int)sum[3]};
 }
 
 // cuda_gcn.cu:226-246: a labelled row is wrong iff some logit is strictly greater than the true-class logit; rows of
@@ -390,20 +455,29 @@ __global__ __launch_bounds__(1024) void sum_squares_kernel(const float *__restri
     }
 }
 
-__global__ void sgd_kernel(float *__restrict__ w, const float *__restrict__ g, int64_t n, float lr)
+// One launch for all tensors of an optimiser step: blockIdx.y is the tensor.
+constexpr int kStepTensors = 4;
+struct StepTensors {
+    drone_step_tensor t[kStepTensors];
+};
+__global__ void sgd_kernel(StepTensors tensors, float lr)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    const drone_step_tensor t = tensors.t[blockIdx.y];
+    float *__restrict__ w = t.w;
+    const float *__restrict__ g = t.grad;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < t.n; i += (int64_t)gridDim.x * blockDim.x)
         w[i] -= lr * g[i];
 }
 
 // cuda_kernel.cu:450-460
-__global__ void adam_kernel(float *__restrict__ w, const float *__restrict__ grad, float *__restrict__ m,
-                            float *__restrict__ v, int64_t n, int decay, float weight_decay, float beta1, float beta2,
-                            float eps, float step_size)
+__global__ void adam_kernel(StepTensors tensors, float weight_decay, float beta1, float beta2, float eps, float step_size)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const drone_step_tensor t = tensors.t[blockIdx.y];
+    float *__restrict__ w = t.w, *__restrict__ m = t.m, *__restrict__ v = t.v;
+    const float *__restrict__ grad = t.grad;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < t.n; i += (int64_t)gridDim.x * blockDim.x) {
         float g = grad[i];
-        if (decay) g += weight_decay * w[i];
+        if (t.decay) g += weight_decay * w[i];
         const float mi = (float)(beta1 * m[i] + (1.0 - beta1) * g);
         const float vi = (float)(beta2 * v[i] + (1.0 - beta2) * g * g);
         m[i] = mi;
@@ -418,10 +492,10 @@ __global__ void fill_f32_kernel(float *__restrict__ x, int64_t n, float value)
         x[i] = value;
 }
 
-// scratch for the cross-entropy block partials (2048 blocks), one per (device, stream): calls on one stream are
+// LossScratch, one per (device, stream): calls on one stream are
 // ordered and share it, calls on different streams may overlap
 std::mutex g_mutex;
-std::map<std::pair<int, hipStream_t>, void *> g_ce_ws;
+std::map<std::pair<int, hipStream_t>, void *> g_loss_scratch;
 
 }  // namespace
 }  // namespace drone
@@ -433,7 +507,8 @@ extern "C" int drone_relu_forward_f32(float *x, uint8_t *mask, int64_t n, int tr
     clear_error();
     DRONE_REQUIRE(n >= 0 && (n == 0 || x) && (!training || mask || n == 0), "null operand");
     if (n == 0) return DRONE_OK;
-    relu_forward_kernel<<<grid_for(n), kThreads, 0, as_stream(stream)>>>(x, mask, n, training);
+    if (four_wide(x, mask, n)) relu_forward_kernel<4><<<grid_for(n / 4, 1), kThreads, 0, as_stream(stream)>>>(x, mask, n, training);
+    else relu_forward_kernel<1><<<grid_for(n), kThreads, 0, as_stream(stream)>>>(x, mask, n, training);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
@@ -443,7 +518,8 @@ extern "C" int drone_relu_backward_f32(float *grad, const uint8_t *mask, int64_t
     clear_error();
     DRONE_REQUIRE(n >= 0 && (n == 0 || (grad && mask)), "null operand");
     if (n == 0) return DRONE_OK;
-    relu_backward_kernel<<<grid_for(n), kThreads, 0, as_stream(stream)>>>(grad, mask, n);
+    if (four_wide(grad, mask, n)) relu_backward_kernel<4><<<grid_for(n / 4, 1), kThreads, 0, as_stream(stream)>>>(grad, mask, n);
+    else relu_backward_kernel<1><<<grid_for(n), kThreads, 0, as_stream(stream)>>>(grad, mask, n);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
@@ -515,35 +591,58 @@ extern "C" int drone_relu_dropout_backward_f32(float *grad, const uint8_t *mask,
     return DRONE_OK;
 }
 
-extern "C" int drone_cross_entropy_f32(int n, int classes, const float *logits, int ld, const int *truth, float *grad,
-                                       int ldg, float grad_scale, float *loss_out, int *count_out,
-                                       drone_stream_t stream)
+extern "C" int drone_loss_pass_f32(const drone_loss_pass *pass, drone_stream_t stream)
 {
     clear_error();
-    DRONE_REQUIRE(n > 0 && classes > 0 && logits && truth && ld >= classes, "operands");
-    DRONE_REQUIRE(grad == nullptr || ldg >= classes, "ldg < classes");
+    DRONE_REQUIRE(pass != nullptr, "null pass");
+    const drone_loss_pass &p = *pass;
+    DRONE_REQUIRE(p.n > 0 && p.classes > 0 && p.logits && p.truth && p.ld >= p.classes, "operands");
+    DRONE_REQUIRE(p.grad == nullptr || p.ldg >= p.classes, "ldg < classes");
+    DRONE_REQUIRE(p.weight_count >= 0 && (p.weights || p.weight_count == 0), "weights");
     int dev = 0;
     DRONE_HIP_TRY(hipGetDevice(&dev));
-    int blocks = (int)ceil_div(n, kThreads / kWave);
-    if (blocks > 2048) blocks = 2048;
     hipStream_t s = as_stream(stream);
     void *ws = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        void *&slot = g_ce_ws[std::make_pair(dev, s)];
-        if (!slot) DRONE_HIP_TRY(hipMalloc(&slot, 2048 * (sizeof(double) + sizeof(int))));
+        void *&slot = g_loss_scratch[std::make_pair(dev, s)];
+        if (!slot) {
+            DRONE_HIP_TRY(hipMalloc(&slot, LossScratch::bytes()));
+            fill_f32_kernel<<<64, kThreads, 0, s>>>(static_cast<float *>(slot), (int64_t)(LossScratch::bytes() / sizeof(float)), 0.0f);
+        }
         ws = slot;
     }
-    double *bl = static_cast<double *>(ws);
-    int *bc = reinterpret_cast<int *>(bl + 2048);
-    if (classes <= 16) cross_entropy_kernel<4><<<blocks, kThreads, 0, s>>>(n, classes, logits, ld, truth, grad, ldg, grad_scale, bl, bc);
-    else if (classes <= 32) cross_entropy_kernel<8><<<blocks, kThreads, 0, s>>>(n, classes, logits, ld, truth, grad, ldg, grad_scale, bl, bc);
-    else if (classes <= 64) cross_entropy_kernel<16><<<blocks, kThreads, 0, s>>>(n, classes, logits, ld, truth, grad, ldg, grad_scale, bl, bc);
-    else if (classes <= 128) cross_entropy_kernel<32><<<blocks, kThreads, 0, s>>>(n, classes, logits, ld, truth, grad, ldg, grad_scale, bl, bc);
-    else cross_entropy_kernel<64><<<blocks, kThreads, 0, s>>>(n, classes, logits, ld, truth, grad, ldg, grad_scale, bl, bc);
-    cross_entropy_finish_kernel<<<1, kThreads, 0, s>>>(blocks, bl, bc, loss_out, count_out);
+    double *part = static_cast<double *>(ws);
+    const LossScratch scratch{part, reinterpret_cast<unsigned int *>(part + 5 * kLossBlocks)};
+    const int lanes = p.classes <= 16 ? 4 : p.classes <= 32 ? 8 : p.classes <= 64 ? 16 : p.classes <= 128 ? 32 : 64;  // per row
+    const int row_blocks = (int)std::min<int64_t>(ceil_div(p.n, kThreads / lanes * kCeGroups), kLossRowBlocks);
+    const int weight_blocks = (int)std::min<int64_t>(ceil_div(p.weight_count, kThreads * 8), kLossWeightBlocks);
+    const int blocks = row_blocks + weight_blocks;
+    if (lanes == 4) loss_kernel<4><<<blocks, kThreads, 0, s>>>(p, row_blocks, scratch);
+    else if (lanes == 8) loss_kernel<8><<<blocks, kThreads, 0, s>>>(p, row_blocks, scratch);
+    else if (lanes == 16) loss_kernel<16><<<blocks, kThreads, 0, s>>>(p, row_blocks, scratch);
+    else if (lanes == 32) loss_kernel<32><<<blocks, kThreads, 0, s>>>(p, row_blocks, scratch);
+    else loss_kernel<64><<<blocks, kThreads, 0, s>>>(p, row_blocks, scratch);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
+}
+
+extern "C" int drone_cross_entropy_f32(int n, int classes, const float *logits, int ld, const int *truth, float *grad,
+                                       int ldg, float grad_scale, float *loss_out, int *count_out,
+                                       drone_stream_t stream)
+{
+    drone_loss_pass p{};
+    p.n = n;
+    p.classes = classes;
+    p.logits = logits;
+    p.ld = ld;
+    p.truth = truth;
+    p.grad = grad;
+    p.ldg = ldg;
+    p.grad_scale = grad_scale;
+    p.loss = loss_out;
+    p.labelled = count_out;
+    return drone_loss_pass_f32(&p, stream);
 }
 
 extern "C" int drone_sum_squares_f32(const float *x, int64_t n, float *out, drone_stream_t stream)
@@ -572,29 +671,58 @@ extern "C" int drone_accuracy_f32(int n, int classes, const float *logits, int l
     return DRONE_OK;
 }
 
-extern "C" int drone_sgd_step_f32(float *w, const float *g, int64_t n, float lr, drone_stream_t stream)
+namespace {
+int steps_grid(const drone_step_tensor *t, int tensors, StepTensors *out)
+{
+    int64_t most = 0;
+    for (int i = 0; i < tensors; ++i) {
+        out->t[i] = t[i];
+        most = std::max(most, t[i].n);
+    }
+    return grid_for(most);
+}
+}  // namespace
+
+extern "C" int drone_sgd_steps_f32(const drone_step_tensor *t, int tensors, float lr, drone_stream_t stream)
 {
     clear_error();
-    DRONE_REQUIRE(n >= 0 && (n == 0 || (w && g)), "null operand");
-    if (n == 0) return DRONE_OK;
-    sgd_kernel<<<grid_for(n), kThreads, 0, as_stream(stream)>>>(w, g, n, lr);
+    DRONE_REQUIRE(t && tensors >= 1 && tensors <= kStepTensors, "tensors");
+    for (int i = 0; i < tensors; ++i) DRONE_REQUIRE(t[i].n >= 0 && (t[i].n == 0 || (t[i].w && t[i].grad)), "null operand");
+    StepTensors all{};
+    const int grid = steps_grid(t, tensors, &all);
+    sgd_kernel<<<dim3(grid, tensors), kThreads, 0, as_stream(stream)>>>(all, lr);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
 
+extern "C" int drone_sgd_step_f32(float *w, const float *g, int64_t n, float lr, drone_stream_t stream)
+{
+    const drone_step_tensor t{w, g, nullptr, nullptr, n, 0};
+    return drone_sgd_steps_f32(&t, 1, lr, stream);
+}
+
 // cuda_module.cu:590-600: step_count is the value after the increment.
+extern "C" int drone_adam_steps_f32(const drone_step_tensor *t, int tensors, float weight_decay, float lr, float beta1,
+                                    float beta2, float eps, int step_count, drone_stream_t stream)
+{
+    clear_error();
+    DRONE_REQUIRE(t && tensors >= 1 && tensors <= kStepTensors && step_count >= 1, "tensors / step_count");
+    for (int i = 0; i < tensors; ++i)
+        DRONE_REQUIRE(t[i].n >= 0 && (t[i].n == 0 || (t[i].w && t[i].grad && t[i].m && t[i].v)), "operands");
+    const float step_size = lr * sqrtf(1 - powf(beta2, (float)step_count)) / (1 - powf(beta1, (float)step_count));
+    StepTensors all{};
+    const int grid = steps_grid(t, tensors, &all);
+    adam_kernel<<<dim3(grid, tensors), kThreads, 0, as_stream(stream)>>>(all, weight_decay, beta1, beta2, eps, step_size);
+    DRONE_HIP_TRY(hipGetLastError());
+    return DRONE_OK;
+}
+
 extern "C" int drone_adam_step_f32(float *w, const float *g, float *m, float *v, int64_t n, int decay,
                                    float weight_decay, float lr, float beta1, float beta2, float eps, int step_count,
                                    drone_stream_t stream)
 {
-    clear_error();
-    DRONE_REQUIRE(n >= 0 && (n == 0 || (w && g && m && v)) && step_count >= 1, "operands");
-    if (n == 0) return DRONE_OK;
-    const float step_size = lr * sqrtf(1 - powf(beta2, (float)step_count)) / (1 - powf(beta1, (float)step_count));
-    adam_kernel<<<grid_for(n), kThreads, 0, as_stream(stream)>>>(w, g, m, v, n, decay, weight_decay, beta1, beta2, eps,
-                                                               step_size);
-    DRONE_HIP_TRY(hipGetLastError());
-    return DRONE_OK;
+    const drone_step_tensor t{w, g, m, v, n, decay};
+    return drone_adam_steps_f32(&t, 1, weight_decay, lr, beta1, beta2, eps, step_count, stream);
 }
 
 extern "C" int drone_fill_f32(float *x, int64_t n, float value, drone_stream_t stream)

@@ -344,6 +344,11 @@ public:
     float *d_loss = nullptr;  // device scalars
     int *d_count = nullptr;
     float grad_scale = 1.0f;  // 1 = the reference's sum-reduced gradient
+    const int *mean_over = nullptr;  // device: scale the gradient by 1 / *mean_over instead
+    // what is reported with the loss (drone_loss_pass); null / 0: nothing
+    const int *skip = nullptr;
+    const Variable *l2_weight = nullptr;
+    drone_loss_report *report = nullptr;
     CrossEntropyLoss(Variable *logits_, const int *truth_, int num_classes_, std::string name, drone_stream_t stream)
         : logits(logits_), truth(truth_), num_classes(num_classes_), s(stream)
     {
@@ -354,8 +359,22 @@ public:
     ~CrossEntropyLoss() override { (void)hipFree(d_loss); (void)hipFree(d_count); }
     void forward(bool training) override
     {
-        DRONE_GCN_CHECK(drone_cross_entropy_f32(logits->rows, num_classes, logits->data, logits->ld, truth,
-                                                training ? logits->grad : nullptr, logits->ld, grad_scale, d_loss, d_count, s));
+        drone_loss_pass p = {};
+        p.n = logits->rows;
+        p.classes = num_classes;
+        p.logits = logits->data;
+        p.ld = p.ldg = logits->ld;
+        p.truth = truth;
+        p.grad = training ? logits->grad : nullptr;
+        p.grad_scale = grad_scale;
+        p.mean_over = mean_over;
+        p.skip = skip;
+        p.weights = l2_weight ? l2_weight->data : nullptr;
+        p.weight_count = l2_weight ? (int64_t)l2_weight->rows * l2_weight->ld : 0;
+        p.loss = d_loss;
+        p.labelled = d_count;
+        p.report = report;
+        DRONE_GCN_CHECK(drone_loss_pass_f32(&p, s));
     }
     void backward() override {}
 };
@@ -393,10 +412,11 @@ public:
     void step() override
     {
         step_count++;
-        for (auto &sl : vars)
-            DRONE_GCN_CHECK(drone_adam_step_f32(sl.var->data, sl.var->grad, sl.m, sl.v, (int64_t)sl.var->rows * sl.var->ld,
-                                                sl.decay, params.weight_decay, params.lr, params.beta1, params.beta2,
-                                                params.eps, step_count, s));
+        std::vector<drone_step_tensor> t;
+        for (auto &sl : vars) t.push_back({sl.var->data, sl.var->grad, sl.m, sl.v, (int64_t)sl.var->rows * sl.var->ld, sl.decay});
+        for (size_t i = 0; i < t.size(); i += 4)
+            DRONE_GCN_CHECK(drone_adam_steps_f32(&t[i], (int)(t.size() - i < 4 ? t.size() - i : 4), params.weight_decay, params.lr,
+                                                 params.beta1, params.beta2, params.eps, step_count, s));
     }
 };
 
@@ -409,7 +429,10 @@ public:
     SGD(std::vector<Variable *> vs, float lr_, drone_stream_t stream) : vars(std::move(vs)), lr(lr_), s(stream) {}
     void step() override
     {
-        for (auto *v : vars) DRONE_GCN_CHECK(drone_sgd_step_f32(v->data, v->grad, (int64_t)v->rows * v->ld, lr, s));
+        std::vector<drone_step_tensor> t;
+        for (auto *v : vars) t.push_back({v->data, v->grad, nullptr, nullptr, (int64_t)v->rows * v->ld, 0});
+        for (size_t i = 0; i < t.size(); i += 4)
+            DRONE_GCN_CHECK(drone_sgd_steps_f32(&t[i], (int)(t.size() - i < 4 ? t.size() - i : 4), lr, s));
     }
 };
 
@@ -454,15 +477,15 @@ public:
     GraphSum *graphsum1 = nullptr, *graphsum2 = nullptr;
     Replicas replicas;
     const int *mirror2worker = nullptr;    // device [N] (Graph::Mirror2Worker) with replicas, else null
-    float *l2_sum = nullptr;               // device scalar: sum of W1^2 (cuda_gcn.cu:254-260)
     CrossEntropyLoss *ce = nullptr;
     ReLU *relu = nullptr;              // layer 1 without dropout
     ReLUDropout *relu_drop = nullptr;  // layer 1 with dropout
     int input_cols = 0;          // inner dimension of layer 1's products: input_dim rounded up (padded_inner_dim)
     float *x_padded = nullptr;   // the model's zero-padded copy of X, when it needs one
     int *truth = nullptr;   // device [N]: label on rows of the current split, -1 elsewhere
-    int truth_split = -1, truth_count = 0;
-    int *counts = nullptr;  // device [2]: correct, labelled
+    int *truth_count = nullptr;  // device: labelled rows of the current split, kept with mean_gradient
+    void *truth_scratch = nullptr;
+    drone_loss_report *report = nullptr;  // pinned: what the last forward pass reports
     const int *label = nullptr, *split = nullptr;  // device, borrowed
     drone_stream_t s;
 
@@ -520,8 +543,9 @@ public:
         const int max_dim = p.hidden_dim > p.output_dim ? p.hidden_dim : p.output_dim;
         adj.reset(new Adjacency(N, nnz, rp, ci, in_degree, out_degree, max_dim, s));
         DRONE_GCN_HIP(hipMalloc(&truth, sizeof(int) * (size_t)N));
-        DRONE_GCN_HIP(hipMalloc(&counts, sizeof(int) * 2));
-        DRONE_GCN_HIP(hipMalloc(&l2_sum, sizeof(float)));
+        if (p.mean_gradient) DRONE_GCN_HIP(hipMalloc(&truth_count, sizeof(int)));
+        DRONE_GCN_HIP(hipHostMalloc(&report, sizeof(drone_loss_report)));
+        *report = drone_loss_report{};
         const Replicas *r = cut ? &replicas : nullptr;
 
         if (p.fold_input_aggregation) {
@@ -553,6 +577,13 @@ public:
         modules.emplace_back(graphsum2);
         ce = new CrossEntropyLoss(output, truth, p.output_dim, "CrossEntropy", s);
         modules.emplace_back(ce);
+        // cuda_gcn.cu:298-299, 314-315: what train_epoch / eval report besides the loss - the accuracy over the labelled
+        // rows that are not mirrors (:226-246) and the L2 penalty weight_decay * sum(W1^2) / 2 (:254-260), from the
+        // weights as they are before the optimiser step - comes out of the loss's launch
+        ce->mean_over = truth_count;
+        ce->skip = mirror2worker;
+        ce->l2_weight = layer1_weight;
+        ce->report = report;
         if (p.use_adam) {
             AdamParams ap;
             ap.lr = p.learning_rate;
@@ -568,50 +599,35 @@ public:
     {
         (void)hipFree(x_padded);
         (void)hipFree(truth);
-        (void)hipFree(counts);
-        (void)hipFree(l2_sum);
+        (void)hipFree(truth_count);
+        (void)hipFree(truth_scratch);
+        (void)hipHostFree(report);
     }
 
     void set_truth(int current_split);  // cuda_gcn.cu:211-223; defined in gcn_model.hip (needs a kernel)
-    // The modules in order, then the counts and sums read_metrics() reports (cuda_gcn.cu:298-299 takes them right
-    // after the forward pass too).
+    // The modules in order.
     void forward(bool training)
     {
         for (auto &m : modules) m->forward(training);
-        metrics_async();
     }
     void backward() { for (int i = (int)modules.size() - 1; i >= 0; --i) modules[i]->backward(); }
 
     // Enqueues one training step (cuda_gcn.cu:287-306 without the host read-backs): forward, accuracy counts,
-    // backward, optimiser.  Loss and counts stay on the device until read_metrics().
+    // backward, optimiser.  Loss and counts lie in `report` once the stream has been waited for: read_metrics().
     void train_step_async()
     {
         forward(true);
         backward();
         optimizer->step();
     }
-    // cuda_gcn.cu:298-299, 314-315: what train_epoch / eval report besides the loss - the accuracy over the labelled
-    // rows that are not mirrors (:226-246) and the L2 penalty weight_decay * sum(W1^2) / 2 (:254-260) - taken from the
-    // weights as they are before the optimiser step, left on the device.
-    void metrics_async()
-    {
-        DRONE_GCN_HIP(hipMemsetAsync(counts, 0, sizeof(int) * 2, static_cast<hipStream_t>(s)));
-        DRONE_GCN_CHECK(drone_accuracy_f32(params.localVertexSize, params.output_dim, output->data, output->ld, truth,
-                                           mirror2worker, nullptr, counts, s));
-        DRONE_GCN_CHECK(drone_sum_squares_f32(layer1_weight->data, (int64_t)layer1_weight->rows * layer1_weight->ld, l2_sum, s));
-    }
     // {loss + L2 penalty, accuracy} of the last forward pass, as CUDAGCN::train_epoch / eval return them.
     // cross_entropy (optional): the mean cross-entropy alone.
     std::pair<float, float> read_metrics(float *cross_entropy = nullptr)
     {
-        float loss = 0.0f, l2 = 0.0f;
-        int c[2] = {0, 0};
         DRONE_GCN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(s)));
-        DRONE_GCN_HIP(hipMemcpy(&loss, ce->d_loss, sizeof(float), hipMemcpyDeviceToHost));
-        DRONE_GCN_HIP(hipMemcpy(&l2, l2_sum, sizeof(float), hipMemcpyDeviceToHost));
-        DRONE_GCN_HIP(hipMemcpy(c, counts, sizeof(int) * 2, hipMemcpyDeviceToHost));
-        if (cross_entropy) *cross_entropy = loss;
-        return {loss + params.weight_decay * l2 / 2, c[1] ? (float)c[0] / (float)c[1] : 0.0f};
+        if (cross_entropy) *cross_entropy = report->loss;
+        return {report->loss + params.weight_decay * report->sum_squares / 2,
+                report->counted ? (float)report->correct / (float)report->counted : 0.0f};
     }
     std::pair<float, float> train_epoch()
     {

@@ -202,7 +202,7 @@ int drone_pr_run_workers_f64(Graph *g, PRValues *values, int workerId, int worke
  * int32 offsets / int32 columns / fp32 values, base 0 - the descriptors of cuda_module.cu:166-194.
  * Calls are asynchronous on `stream`.  Apart from plan creation, the transpose (a set-up step) and
  * grow-only scratch kept per (device, stream) by drone_sgemm_rm_f32 (split reductions) and
- * drone_cross_entropy_f32, nothing allocates; calls on different streams may overlap, except that two products with
+ * drone_cross_entropy_f32 / drone_loss_pass_f32, nothing allocates; calls on different streams may overlap, except that two products with
  * the SAME plan share the plan's partial-row scratch and must not run at the same time.  drone_spmm_csr_f32 only
  * launches kernels and records / waits for events between `stream` and the plan's own side stream, so it can be
  * recorded into a HIP graph on a capturing stream (drone_sgemm_rm_f32 as well once its scratch has grown to the
@@ -318,6 +318,30 @@ int drone_relu_dropout_backward_f32(float *grad, const uint8_t *mask, const uint
  * *loss_out (device) = mean loss over labelled rows, *count_out (device) = their number. */
 int drone_cross_entropy_f32(int n, int classes, const float *logits, int ld, const int *truth, float *grad,
                             int ldg, float grad_scale, float *loss_out, int *count_out, drone_stream_t stream);
+/* One launch for a pass's loss and for what CUDAGCN::train_epoch / eval report with it (cuda_gcn.cu:226-260, 298-299):
+ * drone_cross_entropy_f32, the counts of drone_accuracy_f32 from the same logits, and drone_sum_squares_f32 of `weights`.
+ * Pointers are device pointers unless noted; those marked optional may be NULL. */
+typedef struct drone_loss_report {
+    float loss, sum_squares;
+    int labelled, correct, counted;
+} drone_loss_report;
+typedef struct drone_loss_pass {
+    int n, classes;
+    const float *logits;
+    int ld;
+    const int *truth;
+    float *grad; /* optional */
+    int ldg;
+    float grad_scale;
+    const int *mean_over; /* optional: grad_scale is 1 / *mean_over instead (1 if that is 0) */
+    const int *skip;      /* optional */
+    const float *weights; /* optional */
+    int64_t weight_count;
+    float *loss;               /* optional */
+    int *labelled;             /* optional */
+    drone_loss_report *report; /* optional; device or pinned host memory */
+} drone_loss_pass;
+int drone_loss_pass_f32(const drone_loss_pass *pass, drone_stream_t stream);
 /* cuda_gcn.cu:226-246: a labelled row is correct unless some logit is strictly greater than the true-class
  * logit; rows with skip[row] != -1 are not counted (:234 passes Mirror2Worker, so a replicated vertex is counted
  * on its master's worker only; skip may be NULL).  counts[0] += correct, counts[1] += counted (device ints,
@@ -333,6 +357,17 @@ int drone_sgd_step_f32(float *w, const float *g, int64_t n, float lr, drone_stre
 int drone_adam_step_f32(float *w, const float *g, float *m, float *v, int64_t n, int decay,
                         float weight_decay, float lr, float beta1, float beta2, float eps, int step_count,
                         drone_stream_t stream);
+/* The same for up to four tensors in one launch.  m, v and decay (nonzero: weight_decay * w joins the gradient) are Adam's. */
+typedef struct drone_step_tensor {
+    float *w;
+    const float *grad;
+    float *m, *v;
+    int64_t n;
+    int decay;
+} drone_step_tensor;
+int drone_sgd_steps_f32(const drone_step_tensor *t, int tensors, float lr, drone_stream_t stream);
+int drone_adam_steps_f32(const drone_step_tensor *t, int tensors, float weight_decay, float lr, float beta1, float beta2,
+                         float eps, int step_count, drone_stream_t stream);
 int drone_fill_f32(float *x, int64_t n, float value, drone_stream_t stream);
 
 /* ---- whole-model handle: the C surface of cuda_gcn (cuda_gcn/src/gcn.h:10-12 getHandle/run, and the
