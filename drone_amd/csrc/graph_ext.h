@@ -65,6 +65,12 @@ struct RowSync {
 void row_sync_release(RowSync *rs);  // staging only
 void direct_rows_release(DirectRows *d);
 
+// A vertex's row of the out-edge CSR and the targets of its first edges (-1 past the row's end).
+constexpr int kFirstEdges = 4;
+struct alignas(32) FirstEdges {
+    int begin, degree, dst[kFirstEdges], pad[2];
+};
+
 struct GraphExt {
     int n = 0;
     int edges = 0;
@@ -86,6 +92,7 @@ struct GraphExt {
     double *rank64 = nullptr;
     RouteLists routes;
     RowSync row_sync;
+    FirstEdges *first_edges = nullptr;  // device [n], or null: see ensure_first_edges in traverse.hip
     // SSSP: edge lengths in in-edge order
     int *in_eid = nullptr;    // device [edges]: position in the out-edge CSR (g->dst / g->edgeLen) of each in-edge
     float *in_len = nullptr;  // device [edges]: g->edgeLen in in-edge order, refreshed at every SSSP_PEVal

@@ -318,6 +318,7 @@ void drone::graph_ext_release(GraphExt *x)
     routes_release(&x->routes);
     row_sync_release(&x->row_sync);
     direct_rows_release(&x->row_sync.direct);
+    if (x->first_edges) (void)hipFree(x->first_edges);
     if (x->in_eid) (void)hipFree(x->in_eid);
     if (x->in_len) (void)hipFree(x->in_len);
     *x = GraphExt{};

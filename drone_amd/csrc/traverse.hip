@@ -717,20 +717,41 @@ __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *
     end_round(state, now.mark + 1, now.rounds + 1, 0, counters, ticket);
 }
 
+// Index and head of a vertex's out-edges, for the rounds of a lone wavefront: one access gives what a hop needs to go on from
+// the vertex, where row bounds and then targets are two that wait for each other.
+__global__ void first_edges_kernel(int n, const int *__restrict__ index, const int *__restrict__ dst, FirstEdges *__restrict__ first)
+{
+    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+        FirstEdges f{index[v], index[v + 1] - index[v], {-1, -1, -1, -1}, {0, 0}};
+#pragma unroll
+        for (int k = 0; k < kFirstEdges; ++k)
+            if (k < f.degree) f.dst[k] = dst[f.begin + k];
+        first[v] = f;
+    }
+}
+
 // Push rounds of a short list inside ONE launch: a single work-group keeps the list in LDS, builds the next one there and
 // goes on with it for as long as it has at most kSmallEdges out-edges and is not empty, up to max_rounds rounds.
 // What bounds it is a hop's chain of dependent loads - the edge's target, then the target's value and its row's bounds - so
 // everything else stays out of the chain: the lists and the round's new values live in LDS (a hash table finds a target that
 // several edges lower), no global atomics (only this work-group writes), and a round's values are stored beside the next
 // round's first loads.  Edges are dealt out one per lane across the listed vertices.  While a list has no more edges than a
-// wavefront has lanes, the first wavefront goes on alone, without barriers.  A hop of a 20,000-vertex path 2.0 -> 0.95 us, a
-// round of a 593 x 130 grid 50 -> 2.6 us (lists in global memory, atomics, a wavefront per listed vertex before).
+// wavefront has lanes, the first wavefront goes on alone, without barriers (run_lone).  A hop of a 20,000-vertex path
+// 2.0 -> 0.40 us, a round of a 593 x 130 grid 50 -> 2.6 us (lists in global memory, atomics, a wavefront per listed vertex before).
 // Ordering: a value or flag is stored by a plain store before a point that waits for it (a barrier, or the lone
 // wavefront's own wait), and read behind that point by the same work-group, i.e. through the same L1.
-// Longer lists are left alone.  It runs rounds until `most_rounds` of the call are done.
+// Longer lists are left alone.  It runs rounds until n + 2 of the call are done.
 constexpr int kSmallEdges = 4096, kSmallThreads = 1024;
 constexpr int kSmallSlots = 2 * kSmallEdges;  // of the hash table: at most half full
 constexpr size_t kSmallLds = sizeof(int) * (5 * kSmallEdges + 2 * kSmallSlots);
+
+constexpr int kWarmBytes = 3 << 20;  // of the 4 MB of an XCD's L2
+
+struct LoneShared {
+    int4 edge[kWave];  // {target or -1, edge, place of the value it starts from, -} of the next round's lanes
+    int least[kWave];
+    int tag[256];
+};
 
 template <typename Push>
 struct SmallRounds {
@@ -739,6 +760,8 @@ struct SmallRounds {
     Value *s_old;
     unsigned long long *s_counters;  // [2]: of the current list and of the one being built, by turns
     int *s_ends;                     // [2]: lowered vertices without out-edges: kept from the list's far end
+    LoneShared *s_lone;
+    const FirstEdges *__restrict__ first;  // null where the graph has none
     const int *__restrict__ index;
     const int *__restrict__ dst;
     Push push;
@@ -753,28 +776,16 @@ struct SmallRounds {
         if (Push::activates(s_old[i], nv)) active[v] = mark;
     }
 
-    // T = lanes that take part: the work-group, or its first wavefront.
-    template <int T>
-    static __device__ __forceinline__ void meet()
+    // The work-group runs rounds until the list is too long for it or fits a wavefront; rounds / pending: how many ran,
+    // whether the list's values are still to be stored.  Starts and ends behind a barrier.
+    __device__ __forceinline__ void run(int max_rounds, int &rounds, bool &pending) const
     {
-        if constexpr (T == kWave) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-            __builtin_amdgcn_wave_barrier();
-        } else {
-            __syncthreads();
-        }
-    }
-
-    // Runs rounds while the list has at most `most` edges; rounds / pending: how many ran, whether the list's values are
-    // still to be stored.  Starts and ends behind a meeting point.
-    template <int T, int PER>
-    __device__ __forceinline__ void run(int most, int max_rounds, int &rounds, bool &pending) const
-    {
+        constexpr int T = kSmallThreads, PER = kSmallEdges / T;
         const int tid = threadIdx.x;
         for (;;) {
             const int now = rounds & 1, n = (int)(s_counters[now] >> 32), m = (int)(s_counters[now] & 0xFFFFFFFFull), ends = s_ends[now];
-            if (n + ends == 0 || m > most || n > PER * T || ends > PER * T || rounds >= max_rounds) break;
-            if (T > kWave && m <= kWave && n <= kWave && ends <= kWave && m > 0) break;  // a wavefront's work
+            if (n + ends == 0 || m > kSmallEdges || rounds >= max_rounds) break;
+            if (m <= kWave && ends <= kWave && m > 0) break;  // a wavefront's work
             int t[PER], e[PER];
             Value nv[PER];
             // the edges' targets, and beside them the stores of the last round's values
@@ -796,7 +807,7 @@ struct SmallRounds {
                 for (int i = tid; i < n; i += T) store(i, first_mark + rounds - 1);
                 for (int i = tid; i < ends; i += T) store(kSmallEdges - 1 - i, first_mark + rounds - 1);
             }
-            meet<T>();  // the list has been read and its values are stored
+            __syncthreads();  // the list has been read and its values are stored
             Value old[PER];
             int r0[PER], r1[PER];
 #pragma unroll
@@ -829,7 +840,7 @@ struct SmallRounds {
                     }
                     atomicMin(&s_slot_val[slot], order_of(nv[k]));
                 }
-            meet<T>();  // the next list is complete
+            __syncthreads();  // the next list is complete
             const int n2 = (int)(s_counters[now ^ 1] >> 32), ends2 = s_ends[now ^ 1];
             const auto settle = [&](int i) {  // the vertex's value out of its slot, which is emptied
                 const int slot = s_val[i];
@@ -845,19 +856,180 @@ struct SmallRounds {
             }
             pending = true;
             ++rounds;
-            meet<T>();
+            __syncthreads();
+        }
+    }
+
+    // Inclusive sum over the wavefront's lanes, all of them active.
+    static __device__ __forceinline__ int wave_scan(int v)
+    {
+        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // from 1, 2, 4, 8 lanes below in the row of 16
+        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of the row below to rows 1 and 3
+        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
+        return v;
+    }
+    // Orders the lanes' accesses to LDS and memory, which the hardware carries out in a wavefront's program order.
+    static __device__ __forceinline__ void lanes_meet()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    // The first wavefront runs rounds alone, an edge per lane, while they have at most 64 edges.  A round is a chain: the
+    // targets' values and first edges come from memory in one access, lanes with the same target agree on the least value
+    // (not if only one lane lowers anything), and each lowered vertex hands its edges to the lanes of the next round through
+    // LDS.  Against a list in LDS, searched, hashed and settled like the work-group's, and row bounds and targets fetched one
+    // after the other: a hop of a 20,000-vertex path 0.95 -> 0.57 us,
+    // 0.40 with the single lowering lane's edges passed on in registers and the L2 warm.
+    // warm(), run by the other wavefronts beside it, brings the vertices' first edges into this XCD's L2 if they fit: a
+    // launch finds it cold.  (Only what nobody writes.)
+    // Ends with the list in LDS and all values stored.
+    __device__ __forceinline__ void run_lone(int max_rounds, int &rounds, bool &pending) const
+    {
+        const int lane = threadIdx.x, now = rounds & 1;
+        const int n = (int)(s_counters[now] >> 32), ends = s_ends[now];
+        int m = (int)(s_counters[now] & 0xFFFFFFFFull), t = 0, e = 0, count = 0;
+        Value from{}, nv{};
+        if (lane < m) {
+            int lo = 0, hi = n;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (s_start[mid] <= lane) lo = mid; else hi = mid;
+            }
+            e = s_edge[lo] + (lane - s_start[lo]);
+            t = dst[e];
+            from = value_of_order(s_val[lo], Value{});
+        }
+        if (pending) {
+            if (lane < n) store(lane, first_mark + rounds - 1);
+            if (lane < ends) store(kSmallEdges - 1 - lane, first_mark + rounds - 1);
+            pending = false;
+        }
+        lanes_meet();
+        for (;;) {
+            Value old{};
+            FirstEdges f{0, 0, {-1, -1, -1, -1}, {0, 0}};
+            if (lane < m) {
+                old = push.at(t);
+                if (first) {
+                    f = first[t];
+                } else {
+                    f.begin = index[t];
+                    f.degree = index[t + 1] - f.begin;
+                }
+                nv = push.relax(from, e);
+            }
+            bool lowers = lane < m && nv < old;
+            const int mark = first_mark + rounds++;
+            const unsigned long long lowering = __ballot(lowers);
+            if (__popcll(lowering) > 1) {
+                int leader = lane;
+                bool open = lowers;
+                int *tag = s_lone->tag + (((unsigned int)t * 0x9E3779B1u) >> 24);
+                static_assert(sizeof(s_lone->tag) == sizeof(int) << 8, "the hash keeps 8 bits");
+                while (__ballot(open)) {  // one lane of each tag's is settled, and with it all that have its target
+                    if (open) __hip_atomic_store(tag, lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    lanes_meet();
+                    const int who = open ? __hip_atomic_load(tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : lane;
+                    lanes_meet();
+                    if (__shfl(t, who, kWave) == t && open) {
+                        leader = who;
+                        open = false;
+                    }
+                }
+                if (__ballot(leader != lane)) {
+                    s_lone->least[lane] = INT_MAX;
+                    lanes_meet();
+                    if (lowers) atomicMin(&s_lone->least[leader], order_of(nv));
+                    lanes_meet();
+                    if (lowers) nv = value_of_order(s_lone->least[leader], Value{});
+                    lowers = lowers && leader == lane;
+                    lanes_meet();
+                }
+            }
+            if (lowers) {
+                push.store(t, nv);
+                if (Push::activates(old, nv)) active[t] = mark;
+            }
+            if (__popcll(lowering) == 1 && rounds < max_rounds) {  // its edges go to the first lanes, out of registers
+                const int who = __ffsll(lowering) - 1, degree = __builtin_amdgcn_readlane(f.degree, who);
+                if (degree <= kWave) {
+                    count = degree > 0;
+                    m = degree;
+                    if (m == 0) break;
+                    e = __builtin_amdgcn_readlane(f.begin, who) + lane;
+                    from = value_of_order(__builtin_amdgcn_readlane(order_of(nv), who), Value{});
+                    t = -1;
+#pragma unroll
+                    for (int k = 0; k < kFirstEdges; ++k) {
+                        const int d = __builtin_amdgcn_readlane(f.dst[k], who);
+                        if (lane == k) t = d;
+                    }
+                    if (t < 0 && lane < m) t = dst[e];
+                    lanes_meet();
+                    continue;
+                }
+            }
+            const int take = lowers ? f.degree : 0;
+            const int upto = wave_scan(take), before = upto - take;
+            m = __builtin_amdgcn_readlane(upto, kWave - 1);
+            const unsigned long long taking = __ballot(take > 0);
+            count = __popcll(taking);
+            if (m == 0 || m > kWave || rounds >= max_rounds) {  // over, or not for this wavefront: the list goes back to LDS
+                if (take > 0) {
+                    const int i = __popcll(taking & ((1ull << lane) - 1));
+                    s_start[i] = before;
+                    s_edge[i] = f.begin;
+                    s_vertex[i] = t;
+                    s_val[i] = order_of(nv);
+                }
+                break;
+            }
+#pragma unroll
+            for (int k = 0; k < kFirstEdges; ++k)
+                if (k < take) s_lone->edge[before + k] = make_int4(f.dst[k], f.begin + k, order_of(nv), 0);
+            for (int k = kFirstEdges; __ballot(k < take); ++k)
+                if (k < take) s_lone->edge[before + k] = make_int4(-1, f.begin + k, order_of(nv), 0);
+            lanes_meet();
+            const int4 mine = s_lone->edge[lane];
+            lanes_meet();
+            if (lane < m) {
+                e = mine.y;
+                t = mine.x >= 0 ? mine.x : dst[e];
+                from = value_of_order(mine.z, Value{});
+            }
+        }
+        if (lane == 0) {
+            s_counters[rounds & 1] = ((unsigned long long)count << 32) + (unsigned long long)(unsigned int)m;
+            s_counters[(rounds & 1) ^ 1] = 0ull;
+            s_ends[0] = s_ends[1] = 0;
+        }
+    }
+
+    // Touches the lines of the vertices' first edges, until *stop.
+    __device__ __forceinline__ void warm(int n, const int *stop) const
+    {
+        constexpr int kPerLine = 128 / sizeof(FirstEdges);
+        if (!first || (int64_t)n * (int)sizeof(FirstEdges) > kWarmBytes) return;
+        for (int v = ((int)threadIdx.x - kWave) * kPerLine; v < n; v += (kSmallThreads - kWave) * kPerLine) {
+            if (__hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) return;
+            asm volatile("" ::"v"(first[v].begin));  // the load stays
         }
     }
 };
 
 template <typename Push>
 __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(TraverseState *state, Lists lists, const int *__restrict__ index,
-                                                                         const int *__restrict__ dst, Push push, int *active,
-                                                                         int most_rounds)
+                                                                         const int *__restrict__ dst, const FirstEdges *__restrict__ first,
+                                                                         Push push, int *active, int n_all)
 {
     extern __shared__ int s_small[];
+    __shared__ LoneShared s_lone;
     __shared__ unsigned long long s_counters[2];
-    __shared__ int s_ends[2], s_rounds, s_pending;
+    __shared__ int s_ends[2], s_rounds, s_pending, s_done;
     SmallRounds<Push> sr;
     sr.s_start = s_small;
     sr.s_edge = sr.s_start + kSmallEdges;
@@ -868,6 +1040,8 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     sr.s_slot_val = sr.s_slot_vertex + kSmallSlots;
     sr.s_counters = s_counters;
     sr.s_ends = s_ends;
+    sr.s_lone = &s_lone;
+    sr.first = first;
     sr.index = index;
     sr.dst = dst;
     sr.push = push;
@@ -876,7 +1050,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     const TraverseState start = *state;
     if ((start.listed & 0xFFFFFFFFull) > (unsigned long long)kSmallEdges || start.listed == 0) return;
     const int count = (int)(start.listed >> 32), edges = (int)(start.listed & 0xFFFFFFFFull), mark = start.mark;
-    const int max_rounds = most_rounds - start.rounds;
+    const int max_rounds = n_all + 2 - start.rounds;  // the host tells a cycle of negative length by n + 2
     int *list = lists.vertex[start.which & 1], *offset = lists.offset[start.which & 1];
     sr.first_mark = mark;
     for (int i = tid; i < kSmallSlots; i += kSmallThreads) {
@@ -893,36 +1067,42 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
         s_counters[0] = ((unsigned long long)count << 32) + (unsigned long long)edges;
         s_counters[1] = 0ull;
         s_ends[0] = s_ends[1] = 0;
+        s_done = 0;
     }
     __syncthreads();
     int rounds = 0;
-    bool pending = false;
+    bool pending = false, warmed = false;
     for (;;) {
         const int now = rounds & 1, n = (int)(s_counters[now] >> 32), m = (int)(s_counters[now] & 0xFFFFFFFFull), ends = s_ends[now];
         if (n + ends == 0 || m > kSmallEdges || rounds >= max_rounds) break;
-        if (m > 0 && m <= kWave && n <= kWave && ends <= kWave) {
+        if (m > 0 && m <= kWave && ends <= kWave) {
             if (tid < kWave) {
-                sr.template run<kWave, 1>(kWave, max_rounds, rounds, pending);
+                sr.run_lone(max_rounds, rounds, pending);
                 if (tid == 0) {
                     s_rounds = rounds;
                     s_pending = pending;
+                    __hip_atomic_store(&s_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 }
+            } else if (!warmed) {
+                sr.warm(n_all, &s_done);
             }
+            warmed = true;  // or found that it was not worth it
             __syncthreads();
             rounds = s_rounds;
             pending = s_pending != 0;
             __syncthreads();
         } else {
-            sr.template run<kSmallThreads, kSmallEdges / kSmallThreads>(kSmallEdges, max_rounds, rounds, pending);
+            sr.run(max_rounds, rounds, pending);
         }
     }
     const int now = rounds & 1, n = (int)(s_counters[now] >> 32), ends = s_ends[now];
-    if (pending) {
+    if (rounds > 0)
         for (int i = tid; i < n; i += kSmallThreads) {
-            sr.store(i, mark + rounds - 1);
             list[i] = sr.s_vertex[i];
             offset[i] = sr.s_start[i];
         }
+    if (pending) {
+        for (int i = tid; i < n; i += kSmallThreads) sr.store(i, mark + rounds - 1);
         for (int i = tid; i < ends; i += kSmallThreads) sr.store(kSmallEdges - 1 - i, mark + rounds - 1);
     }
     if (tid == 0) {
@@ -983,7 +1163,8 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, bool all_active, hipS
     const int n = x->n;
     const unsigned long long limit = push_limit(x);
     const auto small = [&] {
-        push_rounds_small_kernel<Push><<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, g->dst, run.push, g->active, n + 2);
+        push_rounds_small_kernel<Push><<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, g->dst, x->first_edges, run.push,
+                                                                            g->active, n);
     };
     const auto push = [&](int times) {  // there are such lists at all if limit > kSmallEdges
         const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div((int64_t)limit, kPushThreads), kPushBlocks);
@@ -1158,6 +1339,22 @@ void exchange_values(Graph *g, T *vals, int **send_id, int **recv_id, T **send_v
     if (rc != DRONE_OK) die("exchange");
 }
 
+// The vertices' first edges, for graphs of at most kFirstEdgesPer edges per vertex: there lists of few edges last for many rounds
+// (roads, grids, chains); where vertices have more, a list outgrows a wavefront within a few rounds.  Without them
+// (no memory) rounds take an access more.
+constexpr int kFirstEdgesPer = 8;
+void ensure_first_edges(Graph *g, hipStream_t s)
+{
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
+    if (x->first_edges || x->n == 0 || (int64_t)x->edges > (int64_t)kFirstEdgesPer * x->n) return;
+    if (hipMalloc(&x->first_edges, sizeof(FirstEdges) * (size_t)x->n) != hipSuccess) {
+        (void)hipGetLastError();
+        x->first_edges = nullptr;
+        return;
+    }
+    first_edges_kernel<<<(unsigned)std::min<int64_t>(ceil_div(x->n, 256), 2048), 256, 0, s>>>(x->n, g->index, g->dst, x->first_edges);
+}
+
 void ensure_flags(Graph *g)
 {
     const size_t cnt = (size_t)(getLocalVertexSize(g) > 0 ? getLocalVertexSize(g) : 1);
@@ -1177,6 +1374,7 @@ extern "C" Response CC_PEVal(Graph *g, CCValues *values, int workerId, int worke
     Response res = {};
     const int n = getLocalVertexSize(g);
     ensure_aggregation_ready(g);
+    ensure_first_edges(g, s);
     ensure_flags(g);
     if (!values->ext) {  // cc.cu:349-351: the state is allocated by this call
         DRONE_HIP_OR_DIE(hipMalloc(&values->ccValue, sizeof(int) * (size_t)(n > 0 ? n : 1)));
@@ -1250,6 +1448,7 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
         die("SSSP_PEVal");
     }
     ensure_aggregation_ready(g);
+    ensure_first_edges(g, s);
     ensure_flags(g);
     if (!values->ext) {  // sssp.cu:408-411
         DRONE_HIP_OR_DIE(hipMalloc(&values->distance, sizeof(float) * (size_t)(n > 0 ? n : 1)));

@@ -48,6 +48,9 @@ def _rows(lengths, sources):
 
 CASES = {
     "lone": lambda: _layers([1] + [63, 64, 65] * 3, 1, 1),
+    # few edges per vertex on average, many per vertex, for the lone wavefront; lists that leave it and come back
+    "chain": lambda: _layers([1] * 40 + [2, 5, 1, 9, 13, 1, 64, 1, 65, 1, 4, 16, 16, 3] * 3, 4, 6),
+    "chain_many": lambda: _layers([1] * 40 + [2, 5, 1, 9, 13, 1, 64, 1, 65, 1, 4, 16, 16, 3] * 3 + [300, 3000, 3000], 12, 7),
     "group": lambda: _layers([1, 31, 65, 255, 1024, 1025, 2048, 64, 1365, 1366, 1, 1], 3, 2),
     "edge4096": lambda: _layers([1, 4096, 4096, 4097, 4097, 2, 4096, 4095], 1, 3),
     "device": lambda: _layers([1, 3000, 9000, 9001, 9000, 300, 70_000, 69_999, 40, 1], 2, 4),
