@@ -15,7 +15,7 @@
 // L2 (B is hundreds of MB, an XCD's L2 is 4 MB).  They are therefore cut by COLUMN BAND: columns are ranked by
 // how often they occur, a band is the set of columns whose feature rows fill about 3 MB (kBandBytes), the first
 // kHotBands bands are kept apart and everything colder shares one last band.  The plan holds a copy of the
-// long rows' entries stably sorted by (band, row) and the resulting pieces (<= kChunk entries each) as a work
+// long rows' entries stably sorted by (band, row) and the resulting pieces (<= piece_entries()) as a work
 // list in that order.  Work-groups are dispatched in list order, so at any moment the resident wavefronts
 // work inside one band whose feature rows stay in L2.  A piece writes its partial row to plan-owned scratch;
 // a second kernel adds each long row's partials in (band, position) order - no atomics, bitwise repeatable.
@@ -34,6 +34,7 @@
 // 2.62; 0.12: 4.45 / 2.59; 0.16: 4.58 / 2.67).  Graphs without such a core (every chunk below the threshold) get no
 // dense part.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <numeric>
 #include <vector>
@@ -88,7 +89,26 @@ namespace drone {
 namespace {
 
 constexpr int kSplitRow = 512;          // rows with more non-zeros are cut into band pieces (256: 4.58 / 2.87 ms, 512: 4.45 / 2.60, 1024: 5.03 / 2.76 for K = 128 / 41 on the 229 M-entry graph)
-constexpr int kChunk = 1024;            // most non-zeros in one piece (256 ... 4096 all within 2 %: 4.26 / 4.28 / 4.24 / 4.29 / 4.35 ms, K = 128)
+// Most entries in one piece: what a wavefront would get of the whole matrix if it were dealt out evenly over the 8,192
+// wavefronts the GPU holds, within these bounds.  A piece is a serial chain of 16 ... 128 entries per step, and in a small
+// matrix the longest one is what the launch waits for.  us with pieces of at most 1,024 / 256 / 128 entries: training step
+// on 30,011 vertices (0.7 M entries) 393 / 292 / 280, forward + transposed product of 20 K vertices and 0.3 M entries at
+// K = 128 163 / 87 / 74, 0.1 M vertices and 1 M entries at K = 64 125 / 85 / 80, 0.2 M vertices and 3 M entries at K = 32
+// 133 / 120 / 126, 1 M vertices and 15 M entries at K = 41 816 / 670 / 664; the 232,965-vertex step 8,818 / 8,721.
+// The partial rows of a row are added one after the other, eight at a time: a row of very many entries gets longer pieces, so
+// that neither chain outgrows the other (16 entries against 8 pieces per round trip).
+constexpr int kLeastPiece = 128, kMostPiece = 256, kHubPiece = 1024;
+int piece_entries(int64_t nnz, int row_len)
+{
+    const int64_t share = std::min<int64_t>(std::max<int64_t>(nnz / 8192, kLeastPiece), kMostPiece);
+    const int64_t hub = std::min<int64_t>((int64_t)std::sqrt(2.0 * (double)row_len), kHubPiece);
+    return (int)(ceil_div(std::max(share, hub), kWave) * kWave);
+}
+// Up to so many entries in long rows there is one band: most of the pieces are resident at once, so their order keeps nothing
+// in L2 and the bands only make them shorter.  us with bands / without: 0.2 M vertices, 3 M entries (K = 32) 120 / 114,
+// training step on 0.1 M vertices and 7 M entries 596 / 575, 0.4 M vertices, 6 M entries (K = 100) 582 / 578; above it
+// 1 M vertices, 16 M entries (K = 128) 2,026 / 2,346, the 232,965-vertex step 8,721 / 11,437.
+constexpr int64_t kOneBandEntries = 4 << 20;
 constexpr int kHotBands = 20;           // bands kept apart; colder columns share one more band
 constexpr size_t kBandBytes = 3u << 20; // feature rows of one band (three quarters of an XCD's L2)
 // Band size x hot bands, ms for K = 128 / 41 on the 229 M-entry graph: 1 MB x 48: 4.90 / 3.02; 2 MB x 24: 4.44 / 2.59;
@@ -751,6 +771,8 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
     int num_bands = (int)ceil_div(p->n_cols, band_cols);
     if (num_bands > kHotBands + 1) num_bands = kHotBands + 1;
     if (num_bands < 1) num_bands = 1;
+    if (long_nnz <= kOneBandEntries) num_bands = 1;
+    const auto piece_of_row = [&](int i) { return piece_entries(p->nnz, long_offset[i + 1] - long_offset[i]); };
     p->band_cols = band_cols;
     p->num_bands = num_bands;
     DRONE_REQUIRE(((int64_t)num_bands + 1) * num_long < (int64_t)UINT32_MAX, "too many long rows for 32-bit band keys");
@@ -890,7 +912,10 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
         std::vector<int> pieces_of_row((size_t)num_long, 0);
         const auto is_dense_run = [&](unsigned k) { return h_keys[k] / (unsigned)num_long == (unsigned)num_bands; };
         for (unsigned k = 0; k < runs; ++k)
-            if (!is_dense_run(k)) pieces_of_row[h_keys[k] % (unsigned)num_long] += (int)ceil_div(h_counts[k], kChunk);
+            if (!is_dense_run(k)) {
+                const int i = (int)(h_keys[k] % (unsigned)num_long);
+                pieces_of_row[i] += (int)ceil_div(h_counts[k], piece_of_row(i));
+            }
         std::vector<int> first_slot((size_t)num_long + 1, 0);
         for (int i = 0; i < num_long; ++i) first_slot[i + 1] = first_slot[i] + pieces_of_row[i];
         const int num_pieces = first_slot[num_long];
@@ -910,9 +935,10 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
                 pos = end;
                 continue;
             }
-            for (int64_t b = pos; b < end; b += kChunk) {
+            const int piece = piece_of_row(i);
+            for (int64_t b = pos; b < end; b += piece) {
                 pb.push_back((int)b);
-                pe.push_back((int)(b + kChunk < end ? b + kChunk : end));
+                pe.push_back((int)(b + piece < end ? b + piece : end));
                 ps.push_back(cursor[i]++);
             }
             pos = end;
