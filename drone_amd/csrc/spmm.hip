@@ -10,7 +10,7 @@
 // one per lane, and handed to the groups by cross-lane reads.
 //
 // Schedule: rows of at most kSplitRow non-zeros are taken in row order, a wavefront per chunk of consecutive rows
-// that hold at most 64 entries together (spmm_chunks_kernel).  Longer rows carry
+// that hold at most 64 entries together (sum_chunk; fewer in small matrices).  Longer rows carry
 // most of the non-zeros of power-law graphs and gather from all over B; run row by row their accesses miss
 // L2 (B is hundreds of MB, an XCD's L2 is 4 MB).  They are therefore cut by COLUMN BAND: columns are ranked by
 // how often they occur, a band is the set of columns whose feature rows fill about 3 MB (kBandBytes), the first
@@ -103,6 +103,15 @@ int piece_entries(int64_t nnz, int row_len)
     const int64_t share = std::min<int64_t>(std::max<int64_t>(nnz / 8192, kLeastPiece), kMostPiece);
     const int64_t hub = std::min<int64_t>((int64_t)std::sqrt(2.0 * (double)row_len), kHubPiece);
     return (int)(ceil_div(std::max(share, hub), kWave) * kWave);
+}
+// Most entries in one chunk of short rows: the same share, so that a small matrix occupies more of the GPU.  us with chunks of
+// up to 64 / 32 / 16 / 8 entries: epoch on 2,708 vertices 186 / 173 / 166 / 162, step on 9,000 vertices and 70 K entries
+// 121 / 109 / 111 / 108, 30,011 vertices and 0.7 M entries 262 / 257 / 265 / 268, 0.2 M vertices and 3 M entries 108 / 115 /
+// 117 / 129.
+constexpr int kLeastChunk = 16;
+int chunk_entries(int64_t n_rows, int64_t nnz)
+{
+    return (int)std::min<int64_t>(std::max<int64_t>(ceil_div((n_rows + nnz) / 8192, 16) * 16, kLeastChunk), kWave);
 }
 // Up to so many entries in long rows there is one band: most of the pieces are resident at once, so their order keeps nothing
 // in L2 and the bands only make them shorter.  us with bands / without: 0.2 M vertices, 3 M entries (K = 32) 120 / 114,
@@ -267,13 +276,13 @@ struct RowSegments {
     __device__ __forceinline__ float *out(int first, int j) const { return C + (size_t)(first + j) * ldc; }
 };
 template <int G, int VEC, typename Segments>
-__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_chunks_kernel(
-    int num_chunks, const int *__restrict__ chunk_first, const int *__restrict__ chunk_last, Segments seg,
-    const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
+__device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *__restrict__ chunk_first,
+                                          const int *__restrict__ chunk_last, Segments seg, const int *__restrict__ ci,
+                                          const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
 {
     constexpr int P = kWave / G;
     constexpr int U = 8;  // feature-row loads in flight per lane group (4 / 6 / 8 measured the same)
-    const int c = blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
+    const int c = block * kRowsPerBlock + threadIdx.x / kWave;
     if (c >= num_chunks) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int li = lane % G, sub = lane / G;
@@ -394,12 +403,12 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_chunks_kernel(
 // One piece per lane group (two or four pieces side by side in a wavefront, nothing folded across groups) lost too:
 // 4.78 / 3.00 ms for K = 128 / 41 against 4.44 / 2.60 - the wavefront runs as long as its longest piece.
 template <int G, int VEC>
-__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_pieces_kernel(
-    int num_pieces, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
-    const int *__restrict__ piece_slot, const int *__restrict__ ci, const float *__restrict__ val,
-    const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
+__device__ __forceinline__ void sum_piece(int block, int num_pieces, const int *__restrict__ piece_begin,
+                                          const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
+                                          const int *__restrict__ ci, const float *__restrict__ val,
+                                          const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
 {
-    const int s = blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
+    const int s = block * kRowsPerBlock + threadIdx.x / kWave;
     if (s >= num_pieces) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int li = lane % G, sub = lane / G;
@@ -410,6 +419,42 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_pieces_kernel(
         row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, kbase, active, acc);
         if (sub == 0 && active) store_row<VEC>(partial + (size_t)piece_slot[s] * ldp, kbase, K, acc, 1.0f, 0.0f);
     }
+}
+
+template <int G, int VEC>
+__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_pieces_kernel(
+    int num_pieces, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
+    const int *__restrict__ piece_slot, const int *__restrict__ ci, const float *__restrict__ val,
+    const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
+{
+    sum_piece<G, VEC>(blockIdx.x, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
+}
+
+template <int G, int VEC, typename Segments>
+__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_chunks_kernel(
+    int num_chunks, const int *__restrict__ chunk_first, const int *__restrict__ chunk_last, Segments seg,
+    const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
+{
+    sum_chunk<G, VEC>(blockIdx.x, num_chunks, chunk_first, chunk_last, seg, ci, val, B, ldb, K);
+}
+
+// Both in one launch, the pieces first: the chunks fill the GPU while the last pieces end, and a launch is saved.  us
+// against one launch each: training step on 30,011 vertices 280 / 263, 20 K vertices and 0.3 M entries at K = 128 74 / 57,
+// 1 M vertices and 15 M entries at K = 41 678 / 619, forward and backward over a vertex cut 757 / 715.  Not beside a bit
+// core: pieces alone take 8 wavefronts per SIMD instead of 6 (76 registers here), and the product of 3 M vertices at
+// K = 64 took 2,369 / 2,442.
+template <int G, int VEC>
+__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_gather_kernel(
+    int num_pieces, int piece_blocks, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
+    const int *__restrict__ piece_slot, const int *__restrict__ ci2, const float *__restrict__ val2,
+    float *__restrict__ partial, int ldp, int num_chunks, const int *__restrict__ chunk_first,
+    const int *__restrict__ chunk_last, RowSegments seg, const int *__restrict__ ci, const float *__restrict__ val,
+    const float *__restrict__ B, int ldb, int K)
+{
+    if ((int)blockIdx.x < piece_blocks)
+        sum_piece<G, VEC>(blockIdx.x, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
+    else
+        sum_chunk<G, VEC>(blockIdx.x - piece_blocks, num_chunks, chunk_first, chunk_last, seg, ci, val, B, ldb, K);
 }
 
 // C[row,:] = alpha * (sum of the row's partial pieces, in slot = (band, position) order) + beta * C[row,:]
@@ -704,14 +749,21 @@ template <int G, int VEC>
 void launch_spmm(const drone_spmm_plan *plan, const int *rp, const int *ci, const float *v, const float *B, int ldb,
                  float *C, int ldc, int K, float alpha, float beta, hipStream_t s)
 {
-    if (plan->num_pieces > 0) {
-        spmm_pieces_kernel<G, VEC><<<(int)ceil_div(plan->num_pieces, kRowsPerBlock), kWave * kRowsPerBlock, 0, s>>>(
-            plan->num_pieces, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2, B, ldb,
-            plan->partial, plan->max_k, K);
+    const int piece_blocks = (int)ceil_div(plan->num_pieces, kRowsPerBlock), chunk_blocks = (int)ceil_div(plan->num_chunks, kRowsPerBlock);
+    const RowSegments rows{rp, C, ldc, alpha, beta};
+    if (piece_blocks > 0 && chunk_blocks > 0 && plan->bits.tiles == 0) {
+        spmm_gather_kernel<G, VEC><<<(unsigned)piece_blocks + (unsigned)chunk_blocks, kWave * kRowsPerBlock, 0, s>>>(
+            plan->num_pieces, piece_blocks, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2,
+            plan->partial, plan->max_k, plan->num_chunks, plan->chunk_r0, plan->chunk_r1, rows, ci, v, B, ldb, K);
+    } else {
+        if (piece_blocks > 0)
+            spmm_pieces_kernel<G, VEC><<<piece_blocks, kWave * kRowsPerBlock, 0, s>>>(
+                plan->num_pieces, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2, B, ldb,
+                plan->partial, plan->max_k, K);
+        if (chunk_blocks > 0)
+            spmm_chunks_kernel<G, VEC, RowSegments><<<chunk_blocks, kWave * kRowsPerBlock, 0, s>>>(
+                plan->num_chunks, plan->chunk_r0, plan->chunk_r1, rows, ci, v, B, ldb, K);
     }
-    if (plan->num_chunks > 0)
-        spmm_chunks_kernel<G, VEC, RowSegments><<<(int)ceil_div(plan->num_chunks, kRowsPerBlock), kWave * kRowsPerBlock, 0, s>>>(
-            plan->num_chunks, plan->chunk_r0, plan->chunk_r1, RowSegments{rp, C, ldc, alpha, beta}, ci, v, B, ldb, K);
     if (plan->num_long > 0) {  // also when every entry of the long rows went to the dense part: C = beta * C there
         const int ldp = plan->max_k;
         // the partial rows are read in 16-byte pieces up to column 4 ceil(K / 4): they must hold that many floats
@@ -1068,6 +1120,7 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
     }
     // chunks of the short rows
     std::vector<int> h_c0, h_c1;
+    const int most = chunk_entries(n_rows, nnz);
     {
         int first = -1, entries = 0;
         const auto close = [&](int end) {
@@ -1087,7 +1140,7 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
                 h_c0.push_back(r);
                 h_c1.push_back(r + 1);
             } else {
-                if (first >= 0 && (entries + len > kWave || r - first >= kWave - 1)) close(r);
+                if (first >= 0 && (entries + len > most || r - first >= kWave - 1)) close(r);
                 if (first < 0) first = r;
                 entries += len;
             }

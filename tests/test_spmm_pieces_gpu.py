@@ -1,5 +1,6 @@
 """Long rows of the aggregation at the lengths where their pieces change: 512 entries (a row is cut at all), 128 and 256 (a
-piece), 38,000 and 600,000 (a hub's pieces grow with it, up to 1,024), and 4,194,304 entries in long rows (column bands)."""
+piece), 38,000 and 600,000 (a hub's pieces grow with it, up to 1,024), and 4,194,304 entries in long rows (column bands); and
+short rows at the sizes of their chunks."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -12,6 +13,10 @@ CASES = {
     "hub": (SHORT + [32_768, 33_000, 40_000, 300_000, 700_001], 700_001),
     "at_one_band": ([8192] * 512, 20_000),
     "bands": (SHORT + [8192] * 512, 70_001),
+    # chunks of at most 16 entries, 16, 17 and 64 in a row; 32; no long row at all
+    "chunks16": ([0, 1, 2, 13, 14, 15, 16, 17, 3, 0, 0, 63, 64, 65, 7, 9] * 9 + [600], 3001),
+    "chunks32": ([0, 1, 15, 16, 17, 31, 32, 33, 2] * 1500 + [513, 700], 20_011),
+    "no_long": ([1, 7, 16, 0, 40, 512] * 3, 1001),
     "bands_hub": ([8191] * 300 + [600, 513, 40_000, 300_000, 1_900_000], 1_900_003),
 }
 
