@@ -5,9 +5,8 @@
 // and atomicMin's its label / distance into the targets) until nothing changes, with a device synchronise per
 // round.
 //
-// Here a dense round is one sweep of the merge-path aggregation over the IN-edge CSR with min as the combining
-// operator: value[v] <- min(value[v], min over in-edges u->v of f(value[u])), f = identity for labels and
-// + edge length for distances.  No atomics, hub rows are spread over tiles, and the sweep updates in place,
+// Here a dense round of distances is one sweep of the merge-path aggregation over the IN-edge CSR with min as the combining
+// operator: value[v] <- min(value[v], min over in-edges u->v of value[u] + length).  No atomics, hub rows are spread over tiles, and the sweep updates in place,
 // so a change can travel several hops in one sweep.  Both iterations descend monotonically towards the least
 // fixed point below the starting state.  Labels, and distances over unit or integer lengths, are identical to the
 // reference's.  With real-valued lengths the reference can stop short of the fixed point: it stores every lower
@@ -39,24 +38,6 @@ namespace {
 constexpr int kIpt = 8;  // the tiling ensure_aggregation_ready() builds
 constexpr float kUnreached = 1e8f;  // sssp.cu:33
 constexpr float kRelaxEps = 1e-6f;  // sssp.cu:64
-
-struct CcEpi {
-    int *cc;  // read through load() and lowered in place: a sweep may see values it has already lowered
-    int *active;
-    int mark;
-
-    __device__ __forceinline__ MinI32 load(int c, int64_t) const { return MinI32{cc[c]}; }
-    __device__ __forceinline__ void lower(int r, int v, double &stat) const
-    {
-        if (v < cc[r]) {  // cc.cu:35-39
-            cc[r] = v;
-            active[r] = mark;
-            stat += 1.0;
-        }
-    }
-    __device__ __forceinline__ void row(int r, MinI32 s, double &stat) const { lower(r, s.v, stat); }
-    __device__ __forceinline__ void fix(int r, MinI32 s, double &stat) const { lower(r, s.v, stat); }
-};
 
 struct SsspEpi {
     float *dist;  // updated in place, as above
@@ -107,16 +88,30 @@ struct Lists {
 // A list of no vertices that no round may take for its own: all of them still have to propagate.
 __host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
 
-// cc.cu:10-20
-__global__ void cc_init_kernel(int n, int *__restrict__ active, int *__restrict__ cc, int *__restrict__ ubm,
-                               TraverseState *__restrict__ state)
+// cc.cu:10-20 and, in place of the first round, labels from further away: a vertex follows its first in-neighbour, that one's
+// first, and so on for as long as the numbers fall and for at most kCcHops hops, and takes the number it arrives at.  It
+// arrives there against the edges' direction, so the label is one that propagation would bring; rows are in ascending order,
+// so the first in-neighbour is the least.  All vertices still have to propagate: the next round looks at every in-edge of
+// every vertex that can fall.  500,009 vertices, 11.5 M edges: 17.5 us instead of
+// 64 for the sweep over all edges that stood here, and the rounds after it start nearer: labels of the graph 241 -> 123 us.
+constexpr int kCcHops = 32;
+__global__ void cc_init_kernel(int n, const int *__restrict__ in_index, const int *__restrict__ in_src, int *__restrict__ active,
+                               int *__restrict__ cc, int *__restrict__ ubm, TraverseState *__restrict__ state)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        active[i] = 0;
-        cc[i] = i;
+        int label = i;
+        for (int hop = 0; hop < kCcHops && label > 0; ++hop) {
+            const int e0 = in_index[label], e1 = in_index[label + 1];
+            if (e0 == e1) break;
+            const int u = in_src[e0];
+            if (u >= label) break;
+            label = u;
+        }
+        active[i] = label < i;  // the mark of round 1, cc.cu:16
+        cc[i] = label;
         ubm[i] = 0;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 1, 0, 0, 0.0};  // cc.cu:16
+    if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 2, 1, 0, 0.0};
 }
 
 // sssp.cu:23-38, and the list of the first round: the start vertex if this subgraph holds it (sssp.cu:30) and it has
@@ -1112,8 +1107,6 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     }
 }
 
-__global__ void set_state_kernel(TraverseState *state, TraverseState to) { *state = to; }
-
 void allow_small_lds()
 {
     for (const void *kernel : {reinterpret_cast<const void *>(&push_rounds_small_kernel<CcPush>),
@@ -1142,11 +1135,12 @@ void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
         t->state, push_limit(x), x->n, x->in_index, x->in_src, pull, g->active, g->index, t->lists, t->counters, t->ticket);
 }
 
-// Runs rounds until nothing changes, from what *t->state says is left to propagate.  What it takes of `run`:
+// Runs rounds until nothing changes, from what *t->state says is left to propagate (`now`, if known).  What it takes of `run`:
 //   run.push                 the relaxation along out-edges
 //   run.sweep(mark)          launches a sweep over all in-edges that marks what it lowers
 //   run.speculates(state)    whether pull() may be launched before its round is known to come
-//   run.can_pull(state)      whether pull() may do the next round
+//   Run::kSweeps             whether there are rounds that pull() cannot do:
+//   run.can_pull(state)      whether it may do the next one
 //   run.pull()               launches a sweep over the open vertices that lists what it lowers
 // Returns the number of rounds, or -1 when the bound of n + 1 rounds is exceeded (a cycle of negative length).
 //
@@ -1156,7 +1150,7 @@ void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
 // over all edges, 269 with the kernels here and a wait per round, 128 with the rounds enqueued together; labels of
 // 500,009 vertices 880, 440, 244.
 template <typename Run>
-int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, bool all_active, hipStream_t s)
+int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bool known, hipStream_t s)
 {
     using Push = decltype(run.push);
     GraphExt *x = static_cast<GraphExt *>(g->ext);
@@ -1172,21 +1166,17 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, bool all_active, hipS
             push_round_kernel<Push><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, limit, t->lists, g->index, g->dst, run.push,
                                                                   g->active, t->counters, t->ticket);
     };
-    TraverseState now{};
-    bool known = false;
     int sweeps = 1;  // per wait: doubles while nothing else is to be done
     const auto pull_maybe = [&](int times) {
         for (int i = 0; i < times && run.speculates(now) && (unsigned long long)x->edges > limit; ++i) run.pull();
     };
-    if (all_active) {
-        run.sweep(1);  // nothing is final yet: all edges once
-        now = TraverseState{everything(), 2, 1, 0, 0.0};
-        set_state_kernel<<<1, 1, 0, s>>>(t->state, now);
-        known = true;
-    }
     for (;;) {
         const unsigned long long edges = now.listed & 0xFFFFFFFFull;
         int sweeps_next = 1;
+        const auto can_pull = [&] {
+            if constexpr (Run::kSweeps) return run.can_pull(now);
+            else return true;
+        };
         if (!known || edges <= (unsigned long long)kSmallEdges) {
             small();
             push(1);
@@ -1196,12 +1186,12 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, bool all_active, hipS
         } else if (edges <= limit) {
             push(3);
             small();
-        } else if (run.can_pull(now)) {
+        } else if (can_pull()) {
             run.pull();
             pull_maybe(1);
             push(3);
             small();
-        } else {
+        } else if constexpr (Run::kSweeps) {
             for (int i = 0; i < sweeps; ++i) run.sweep(now.mark + i);
             launch_collect(g, t, now.mark + sweeps - 1, now.mark + sweeps, now.rounds + sweeps, s);
             push(1);
@@ -1264,13 +1254,8 @@ struct CcRun {
     hipStream_t s;
     CcPush push{cc};
     bool speculates(const TraverseState &) const { return true; }
-    bool can_pull(const TraverseState &) const { return true; }
+    static constexpr bool kSweeps = false;
     void pull() { launch_pull(g, t, CcPull{cc}, s); }
-    void sweep(int mark)
-    {
-        GraphExt *x = static_cast<GraphExt *>(g->ext);
-        spmv_merge_launch<MinI32, int, kIpt>(x->mt, x->ms, x->in_index, x->in_src, CcEpi{cc, g->active, mark}, t->stat, s);
-    }
 };
 
 // levels: the rounds start from one vertex, so over unit lengths round k reaches the vertices at distance k.  Whether all
@@ -1284,6 +1269,7 @@ struct SsspRun {
     bool levels;
     SsspPush push{dist, g->edgeLen};
     bool counted = false, gathered = false;
+    static constexpr bool kSweeps = true;
 
     void count_lengths()
     {
@@ -1373,7 +1359,6 @@ extern "C" Response CC_PEVal(Graph *g, CCValues *values, int workerId, int worke
     hipStream_t s = comm ? static_cast<hipStream_t>(comm->s) : nullptr;
     Response res = {};
     const int n = getLocalVertexSize(g);
-    ensure_aggregation_ready(g);
     ensure_first_edges(g, s);
     ensure_flags(g);
     if (!values->ext) {  // cc.cu:349-351: the state is allocated by this call
@@ -1381,9 +1366,10 @@ extern "C" Response CC_PEVal(Graph *g, CCValues *values, int workerId, int worke
         values->ext = traverse_ext_create(n);
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    cc_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->active, values->ccValue, g->updateByMessage, t->state);
+    const GraphExt *x = static_cast<const GraphExt *>(g->ext);
+    cc_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, x->in_index, x->in_src, g->active, values->ccValue, g->updateByMessage, t->state);
     CcRun run{g, t, values->ccValue, s};
-    if (n > 0) run_to_fixed_point(g, t, run, true, s);
+    if (n > 0) run_to_fixed_point(g, t, run, TraverseState{everything(), 2, 1, 0, 0.0}, true, s);
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1410,7 +1396,7 @@ extern "C" Response CC_IncEVal(Graph *g, CCValues *values, int workerId, int wor
     process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
     launch_collect(g, t, 0, 1, 0, s);  // cc.cu:425: the vertices a message activated propagate
     CcRun run{g, t, values->ccValue, s};
-    run_to_fixed_point(g, t, run, false, s);
+    run_to_fixed_point(g, t, run, TraverseState{}, false, s);
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1459,7 +1445,7 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
                                                      g->index, t->lists.vertex[0], t->lists.offset[0], t->state);
     SsspRun run{g, t, values->distance, s, true};
     run.count_lengths();
-    report_rounds(run_to_fixed_point(g, t, run, false, s), "SSSP_PEVal");
+    report_rounds(run_to_fixed_point(g, t, run, TraverseState{}, false, s), "SSSP_PEVal");
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1486,7 +1472,7 @@ extern "C" Response SSSP_IncEVal(Graph *g, SSSPValues *values, int workerId, int
     process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
     launch_collect(g, t, 0, 1, 0, s);
     SsspRun run{g, t, values->distance, s, false};
-    report_rounds(run_to_fixed_point(g, t, run, false, s), "SSSP_IncEVal");
+    report_rounds(run_to_fixed_point(g, t, run, TraverseState{}, false, s), "SSSP_IncEVal");
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();

@@ -51,6 +51,9 @@ CASES = {
     # few edges per vertex on average, many per vertex, for the lone wavefront; lists that leave it and come back
     "chain": lambda: _layers([1] * 40 + [2, 5, 1, 9, 13, 1, 64, 1, 65, 1, 4, 16, 16, 3] * 3, 4, 6),
     "chain_many": lambda: _layers([1] * 40 + [2, 5, 1, 9, 13, 1, 64, 1, 65, 1, 4, 16, 16, 3] * 3 + [300, 3000, 3000], 12, 7),
+    # labels that come from as far as a first round looks, from one hop further and from much further away
+    "falling": lambda: (np.concatenate([np.arange(31), 100 + np.arange(32), 200 + np.arange(33), 300 + np.arange(500), [0, 0, 0]]).astype(np.int32),
+                        np.concatenate([np.arange(1, 32), 101 + np.arange(32), 201 + np.arange(33), 301 + np.arange(500), [100, 200, 300]]).astype(np.int32)),
     "group": lambda: _layers([1, 31, 65, 255, 1024, 1025, 2048, 64, 1365, 1366, 1, 1], 3, 2),
     "edge4096": lambda: _layers([1, 4096, 4096, 4097, 4097, 2, 4096, 4095], 1, 3),
     "device": lambda: _layers([1, 3000, 9000, 9001, 9000, 300, 70_000, 69_999, 40, 1], 2, 4),
