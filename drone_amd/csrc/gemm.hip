@@ -46,25 +46,42 @@ struct alignas(4) Float4U {
 
 // Loads a (BK x EXT) k-major tile of op(X) into registers: element (k, i) for k in [0,BK), i in [0,EXT).
 // K_CONTIG: memory holds X[i][k] (k contiguous) - lanes walk k fastest; else X[k][i] - lanes walk i fastest.
-// A tile that lies wholly inside the matrix is fetched as 16-byte loads without bounds checks (`full`, uniform
-// over the work-group); edge tiles take dword loads with a check per element.  The two paths distribute the
-// elements over the lanes differently, so store() must be told which one filled the registers.
-template <int EXT, bool K_CONTIG>
+// A tile with all BK steps of the reduction is fetched as 16-byte loads without masks (`full`, uniform over the
+// work-group), also where it reaches past the matrix in i (not INSIDE): what stands there only reaches outputs that
+// nobody stores, so a lane past the end reads the last row again, or slides back to the row's last four elements and puts
+// those of its own that exist in their place (store(): doing it here would wait for the load).  The last, partial tile of
+// the reduction takes dword loads with a check per element.  The two paths distribute the elements over the lanes
+// differently, so store() must be told which one filled the registers.  With checked dword loads for every tile that
+// reaches past the matrix, 30,011 x 301 x 100 took 41 us (36 now), 602 x 128 over 232,965 rows 384 (336), 1,000 x 3,000 x
+// 1,001 transposed 350 (208).
+template <int EXT, bool K_CONTIG, bool INSIDE>
 struct TileLoader {
     static constexpr int PER = BK * EXT / 256;
     static constexpr int VPER = PER / 4;
     float r[PER];
+    // How far this lane's piece of i slid back, modulo 4 (a piece that lies wholly outside: any).
+    static __device__ __forceinline__ int slid(int t, int i0, int i_end)
+    {
+        const int i = i0 + 4 * (t % (EXT / 4));
+        return K_CONTIG || INSIDE || i + 4 <= i_end ? 0 : (i + 4 - i_end) & 3;
+    }
     __device__ __forceinline__ void load(int t, const float *__restrict__ X, int ld, int i0, int i_end, int k0, int k_end, bool full)
     {
+        const auto fetch = [&](int p, const float *src) {
+            const Float4U q = *reinterpret_cast<const Float4U *>(src);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[4 * p + j] = q.v[j];
+        };
         if (full) {
 #pragma unroll
             for (int p = 0; p < VPER; ++p) {
-                const float *src;
-                if constexpr (K_CONTIG) src = X + (size_t)(i0 + t / (BK / 4) + p * (1024 / BK)) * ld + k0 + 4 * (t % (BK / 4));
-                else src = X + (size_t)(k0 + t / (EXT / 4) + p * (1024 / EXT)) * ld + i0 + 4 * (t % (EXT / 4));
-                const Float4U q = *reinterpret_cast<const Float4U *>(src);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) r[4 * p + j] = q.v[j];
+                if constexpr (K_CONTIG) {
+                    const int i = i0 + t / (BK / 4) + p * (1024 / BK);
+                    fetch(p, X + (size_t)(INSIDE || i < i_end ? i : i_end - 1) * ld + k0 + 4 * (t % (BK / 4)));
+                } else {
+                    const int i = i0 + 4 * (t % (EXT / 4));
+                    fetch(p, X + (size_t)(k0 + t / (EXT / 4) + p * (1024 / EXT)) * ld + (INSIDE || i + 4 <= i_end ? i : i_end - 4));
+                }
             }
             return;
         }
@@ -79,7 +96,7 @@ struct TileLoader {
             r[p] = v;
         }
     }
-    __device__ __forceinline__ void store(int t, float *s /* [BK][EXT+PAD] */, bool full) const
+    __device__ __forceinline__ void store(int t, float *s /* [BK][EXT+PAD] */, bool full, int slid) const
     {
         if (full) {
 #pragma unroll
@@ -90,7 +107,12 @@ struct TileLoader {
                     for (int j = 0; j < 4; ++j) s[(k + j) * (EXT + PAD) + i] = r[4 * p + j];
                 } else {
                     const int k = t / (EXT / 4) + p * (1024 / EXT), i = 4 * (t % (EXT / 4));
-                    *reinterpret_cast<float4 *>(s + k * (EXT + PAD) + i) = make_float4(r[4 * p], r[4 * p + 1], r[4 * p + 2], r[4 * p + 3]);
+                    float4 v = make_float4(r[4 * p], r[4 * p + 1], r[4 * p + 2], r[4 * p + 3]);
+                    if constexpr (!INSIDE) {
+                        if (slid & 1) v.x = v.y, v.y = v.z, v.z = v.w;
+                        if (slid & 2) v.x = v.z, v.y = v.w;
+                    }
+                    *reinterpret_cast<float4 *>(s + k * (EXT + PAD) + i) = v;
                 }
             }
             return;
@@ -127,31 +149,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 
     if (threadIdx.x >= 256) {
         // ---- loader wavefronts: tile i + 1 goes to LDS while tile i is multiplied, tile i + 2 is in flight ----
-        TileLoader<BM, !TA> la;
-        TileLoader<BN, TB> lb;
-        const bool rows_inside = m0 + BM <= M, cols_inside = n0 + BN <= N;  // the tile's extent in m / n lies inside C
-        auto fetch = [&](int i) {
-            const int k0 = kb + i * BK;
-            const bool full = k0 + BK <= ke;
-            la.load(t, A, lda, m0, M, k0, ke, full && rows_inside);
-            lb.load(t, B, ldb, n0, N, k0, ke, full && cols_inside);
-        };
-        auto put = [&](int i) {
-            const bool full = kb + (i + 1) * BK <= ke;
-            la.store(t, sA[i & 1], full && rows_inside);
-            lb.store(t, sB[i & 1], full && cols_inside);
-        };
-        if (tiles > 0) {
-            fetch(0);
-            put(0);
-        }
-        if (tiles > 1) fetch(1);
-        __syncthreads();
-        for (int i = 0; i < tiles; ++i) {
-            if (i + 1 < tiles) put(i + 1);
-            if (i + 2 < tiles) fetch(i + 2);
+        const auto run = [&](auto inside) {
+            constexpr bool kInside = decltype(inside)::value;
+            TileLoader<BM, !TA, kInside> la;
+            TileLoader<BN, TB, kInside> lb;
+            const bool wide_a = !TA || M >= 4, wide_b = TB || N >= 4;  // there is a piece of four to slide back to
+            const int slid_a = la.slid(t, m0, M), slid_b = lb.slid(t, n0, N);
+            auto fetch = [&](int i) {
+                const int k0 = kb + i * BK;
+                const bool full = k0 + BK <= ke;
+                la.load(t, A, lda, m0, M, k0, ke, full && wide_a);
+                lb.load(t, B, ldb, n0, N, k0, ke, full && wide_b);
+            };
+            auto put = [&](int i) {
+                const bool full = kb + (i + 1) * BK <= ke;
+                la.store(t, sA[i & 1], full && wide_a, slid_a);
+                lb.store(t, sB[i & 1], full && wide_b, slid_b);
+            };
+            if (tiles > 0) {
+                fetch(0);
+                put(0);
+            }
+            if (tiles > 1) fetch(1);
             __syncthreads();
-        }
+            for (int i = 0; i < tiles; ++i) {
+                if (i + 1 < tiles) put(i + 1);
+                if (i + 2 < tiles) fetch(i + 2);
+                __syncthreads();
+            }
+        };
+        // the tile's extent in m / n lies inside C
+        if (m0 + BM <= M && n0 + BN <= N) run(std::true_type{});
+        else run(std::false_type{});
         return;
     }
 
@@ -897,9 +926,9 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
     const double in = 4.0 * ((double)M * K + (double)K * N), out = 4.0 * M * N;
     const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
     const double direct_us = std::max(padded / 75e6, in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
-    // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.5 for a 128-wide one)
+    // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.25 for a 128-wide one)
     const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
-    const double tiled_us = std::max(ceil_div((int64_t)tiles * splits, 256) * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.5),
+    const double tiled_us = std::max(ceil_div((int64_t)tiles * splits, 256) * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.25),
                                      in / 2.0e6 + out / 2.4e6) + (splits > 1 ? 5 : 0);
     if (tiled_us < direct_us) d.ks = 0;
     return d;
