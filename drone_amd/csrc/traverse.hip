@@ -92,8 +92,8 @@ __host__ __device__ __forceinline__ unsigned long long everything() { return (1u
 // first, and so on for as long as the numbers fall and for at most kCcHops hops, and takes the number it arrives at.  It
 // arrives there against the edges' direction, so the label is one that propagation would bring; rows are in ascending order,
 // so the first in-neighbour is the least.  All vertices still have to propagate: the next round looks at every in-edge of
-// every vertex that can fall.  500,009 vertices, 11.5 M edges: 17.5 us instead of
-// 64 for the sweep over all edges that stood here, and the rounds after it start nearer: labels of the graph 241 -> 123 us.
+// every vertex that can fall.  500,009 vertices, 11.5 M edges: 17.5 us instead of 64 for the sweep over all edges that
+// stood here, and the rounds after it start nearer: labels of the graph 241 -> 123 us.
 constexpr int kCcHops = 32;
 __global__ void cc_init_kernel(int n, const int *__restrict__ in_index, const int *__restrict__ in_src, int *__restrict__ active,
                                int *__restrict__ cc, int *__restrict__ ubm, TraverseState *__restrict__ state)
@@ -877,8 +877,8 @@ struct SmallRounds {
     // targets' values and first edges come from memory in one access, lanes with the same target agree on the least value
     // (not if only one lane lowers anything), and each lowered vertex hands its edges to the lanes of the next round through
     // LDS.  Against a list in LDS, searched, hashed and settled like the work-group's, and row bounds and targets fetched one
-    // after the other: a hop of a 20,000-vertex path 0.95 -> 0.57 us,
-    // 0.40 with the single lowering lane's edges passed on in registers and the L2 warm.
+    // after the other: a hop of a 20,000-vertex path 0.95 -> 0.57 us, 0.40 with the single lowering lane's edges passed on
+    // in registers and the L2 warm.  (Four edges per lane, up to 256: a 40 x 1,000 grid took 3.0 ms instead of 2.3.)
     // warm(), run by the other wavefronts beside it, brings the vertices' first edges into this XCD's L2 if they fit: a
     // launch finds it cold.  (Only what nobody writes.)
     // Ends with the list in LDS and all values stored.
@@ -1148,7 +1148,7 @@ void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
 // usually follow each other - a list grows past what one work-group takes, then past what is worth pushing, and shrinks
 // again - and only then waits.  Breadth-first distances over 1 M vertices and 11.5 M edges: 550 us with a wait per round and sweeps
 // over all edges, 269 with the kernels here and a wait per round, 128 with the rounds enqueued together; labels of
-// 500,009 vertices 880, 440, 244.
+// 500,009 vertices 880, 440, 244 (123 since their first round follows chains, see cc_init_kernel).
 template <typename Run>
 int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bool known, hipStream_t s)
 {
