@@ -9,10 +9,11 @@
 // operator: value[v] <- min(value[v], min over in-edges u->v of value[u] + length).  No atomics, hub rows are spread over tiles, and the sweep updates in place,
 // so a change can travel several hops in one sweep.  Both iterations descend monotonically towards the least
 // fixed point below the starting state.  Labels, and distances over unit or integer lengths, are identical to the
-// reference's.  With real-valued lengths the reference can stop short of the fixed point: it stores every lower
-// distance but re-activates a vertex only when the improvement exceeds 1e-6 (sssp.cu:62-68), so an improvement
-// below that is not carried on; the sweeps here carry every improvement on and end at the exact fixed point, at
-// most 1e-6 per hop below the reference's value.  g->active keeps the
+// reference's.  With real-valued lengths both can stop short of the fixed point: every lower distance is stored, but a
+// vertex propagates only when the improvement exceeds 1e-6 (sssp.cu:62-68).  That rule is the same in every kind of
+// round here: a vertex goes on the next list, and gets its mark, if the round lowered it past the tolerance.  A sweep
+// looks at all in-edges, so it takes a smaller improvement along where the reference leaves it; results lie at most
+// 1e-6 per hop below the reference's value.  g->active keeps the
 // reference's three classes (> 0 lowered by propagation in this call, 0 activated by a message or initial,
 // -1 untouched), which is all the exchange and countActive (common.cu:17-31) look at.  The round number
 // stored in g->active by the reference depends on its thread schedule and is not reproduced.
@@ -300,6 +301,7 @@ struct CcPush {
     __device__ __forceinline__ void store(int v, int x) const { cc[v] = x; }
     __device__ __forceinline__ int relax(int val, int) const { return val; }
     __device__ __forceinline__ int lower(int t, int nv) const { return atomicMin(cc + t, nv); }  // cc.cu:35-36
+    static constexpr bool kTolerance = false;  // every lowered label propagates
     static __device__ __forceinline__ bool activates(int old, int nv) { return old > nv; }
 };
 
@@ -322,6 +324,7 @@ struct SsspPush {
         return __uint_as_float(atomicMax(reinterpret_cast<unsigned int *>(dist + t), __float_as_uint(nv)));
     }
     // The target counts as updated past the tolerance (sssp.cu:64).
+    static constexpr bool kTolerance = true;
     static __device__ __forceinline__ bool activates(float old, float nv) { return old > nv + kRelaxEps; }
 };
 
@@ -754,7 +757,7 @@ struct SmallRounds {
     int *s_start, *s_edge, *s_vertex, *s_val, *s_slot_vertex, *s_slot_val;
     Value *s_old;
     unsigned long long *s_counters;  // [2]: of the current list and of the one being built, by turns
-    int *s_ends;                     // [2]: lowered vertices without out-edges: kept from the list's far end
+    int *s_ends;                     // [2]: lowered vertices that do not propagate (no out-edges, or within the tolerance): kept from the list's far end
     LoneShared *s_lone;
     const FirstEdges *__restrict__ first;  // null where the graph has none
     const int *__restrict__ index;
@@ -812,30 +815,46 @@ struct SmallRounds {
                     r0[k] = index[t[k]];
                     r1[k] = index[t[k] + 1];
                 }
+            const auto keep = [&](int k, bool goes) {
+                unsigned int slot = ((unsigned int)t[k] * 0x9E3779B1u) >> 19;
+                static_assert(kSmallSlots == 1 << 13, "the hash keeps 13 bits");
+                int found;
+                while ((found = atomicCAS(&s_slot_vertex[slot], -1, t[k])) != -1 && found != t[k]) slot = (slot + 1) & (kSmallSlots - 1);
+                if (found == -1) {  // first edge to lower it
+                    int i;
+                    if (goes && r1[k] > r0[k]) {
+                        const unsigned long long p = atomicAdd(&s_counters[now ^ 1], (1ull << 32) + (unsigned long long)(r1[k] - r0[k]));
+                        i = (int)(p >> 32);
+                        s_start[i] = (int)(p & 0xFFFFFFFFull);
+                        s_edge[i] = r0[k];
+                    } else {
+                        i = kSmallEdges - 1 - atomicAdd(&s_ends[now ^ 1], 1);
+                    }
+                    s_vertex[i] = t[k];
+                    s_old[i] = old[k];
+                    s_val[i] = (int)slot;
+                }
+                atomicMin(&s_slot_val[slot], order_of(nv[k]));
+            };
+            bool slight = false;
 #pragma unroll
             for (int k = 0; k < PER; ++k)
                 if (tid + k * T < m && nv[k] < old[k]) {
-                    unsigned int slot = ((unsigned int)t[k] * 0x9E3779B1u) >> 19;
-                    static_assert(kSmallSlots == 1 << 13, "the hash keeps 13 bits");
-                    int found;
-                    while ((found = atomicCAS(&s_slot_vertex[slot], -1, t[k])) != -1 && found != t[k]) slot = (slot + 1) & (kSmallSlots - 1);
-                    if (found == -1) {  // first edge to lower it
-                        int i;
-                        if (r1[k] > r0[k]) {
-                            const unsigned long long p = atomicAdd(&s_counters[now ^ 1], (1ull << 32) + (unsigned long long)(r1[k] - r0[k]));
-                            i = (int)(p >> 32);
-                            s_start[i] = (int)(p & 0xFFFFFFFFull);
-                            s_edge[i] = r0[k];
-                        } else {
-                            i = kSmallEdges - 1 - atomicAdd(&s_ends[now ^ 1], 1);
-                        }
-                        s_vertex[i] = t[k];
-                        s_old[i] = old[k];
-                        s_val[i] = (int)slot;
-                    }
-                    atomicMin(&s_slot_val[slot], order_of(nv[k]));
+                    if (Push::activates(old[k], nv[k])) keep(k, true);
+                    else slight = true;
                 }
-            __syncthreads();  // the next list is complete
+            if constexpr (Push::kTolerance) {
+                // Targets that no edge lowers past the tolerance: their value is stored and goes no further.  After the
+                // others, so that a target that one edge lowers a little and another by more is on the list.
+                if (__syncthreads_or(slight)) {
+#pragma unroll
+                    for (int k = 0; k < PER; ++k)
+                        if (tid + k * T < m && nv[k] < old[k] && !Push::activates(old[k], nv[k])) keep(k, false);
+                    __syncthreads();
+                }
+            } else {
+                __syncthreads();
+            }  // the next list is complete
             const int n2 = (int)(s_counters[now ^ 1] >> 32), ends2 = s_ends[now ^ 1];
             const auto settle = [&](int i) {  // the vertex's value out of its slot, which is emptied
                 const int slot = s_val[i];
@@ -880,7 +899,8 @@ struct SmallRounds {
     // after the other: a hop of a 20,000-vertex path 0.95 -> 0.57 us, 0.40 with the single lowering lane's edges passed on
     // in registers and the L2 warm.  (Four edges per lane, up to 256: a 40 x 1,000 grid took 3.0 ms instead of 2.3.)
     // warm(), run by the other wavefronts beside it, brings the vertices' first edges into this XCD's L2 if they fit: a
-    // launch finds it cold.  (Only what nobody writes.)
+    // launch finds it cold.  (Only what nobody writes.)  A branch that is taken costs the lone wavefront a refill of its
+    // instructions, so the common case is the one that falls through (without the hints a hop takes 0.41 us).
     // Ends with the list in LDS and all values stored.
     __device__ __forceinline__ void run_lone(int max_rounds, int &rounds, bool &pending) const
     {
@@ -920,7 +940,7 @@ struct SmallRounds {
             bool lowers = lane < m && nv < old;
             const int mark = first_mark + rounds++;
             const unsigned long long lowering = __ballot(lowers);
-            if (__popcll(lowering) > 1) {
+            if (__builtin_expect(__popcll(lowering) > 1, 0)) {
                 int leader = lane;
                 bool open = lowers;
                 int *tag = s_lone->tag + (((unsigned int)t * 0x9E3779B1u) >> 24);
@@ -945,16 +965,15 @@ struct SmallRounds {
                     lanes_meet();
                 }
             }
-            if (lowers) {
-                push.store(t, nv);
-                if (Push::activates(old, nv)) active[t] = mark;
-            }
-            if (__popcll(lowering) == 1 && rounds < max_rounds) {  // its edges go to the first lanes, out of registers
-                const int who = __ffsll(lowering) - 1, degree = __builtin_amdgcn_readlane(f.degree, who);
-                if (degree <= kWave) {
+            const bool goes = lowers && Push::activates(old, nv);
+            if (lowers) push.store(t, nv);
+            if (goes) active[t] = mark;
+            if (__builtin_expect(__popcll(lowering) == 1 && rounds < max_rounds, 1)) {  // its edges go to the first lanes, out of registers
+                const int who = __ffsll(lowering) - 1, degree = __builtin_amdgcn_readlane(goes ? f.degree : 0, who);
+                if (__builtin_expect(degree <= kWave, 1)) {
                     count = degree > 0;
                     m = degree;
-                    if (m == 0) break;
+                    if (__builtin_expect(m == 0, 0)) break;
                     e = __builtin_amdgcn_readlane(f.begin, who) + lane;
                     from = value_of_order(__builtin_amdgcn_readlane(order_of(nv), who), Value{});
                     t = -1;
@@ -968,7 +987,7 @@ struct SmallRounds {
                     continue;
                 }
             }
-            const int take = lowers ? f.degree : 0;
+            const int take = goes ? f.degree : 0;
             const int upto = wave_scan(take), before = upto - take;
             m = __builtin_amdgcn_readlane(upto, kWave - 1);
             const unsigned long long taking = __ballot(take > 0);

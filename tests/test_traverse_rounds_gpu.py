@@ -109,3 +109,69 @@ def test_rounds_at_their_edges(oracle, name):
             assert res.VisitedSize == np.count_nonzero(cc != np.arange(n))
     finally:
         w.close()
+
+
+def _near_ties(copies, filler):
+    """A start vertex and `copies` of x -> y -> z, where x falls in the first round and once more in the third: by less than
+    the tolerance of 1e-6, by more, or by both along two edges.  Edges with lengths; filler: as many edges that nothing reaches."""
+    e = []
+    for i in range(copies):
+        a, b, c, d, x, y, z = range(1 + 7 * i, 8 + 7 * i)
+        e += [(0, a, 1.0), (a, c, 0.5), (c, x, 0.5), (x, y, 1.0), (y, z, 1.0)]
+        e.append((0, x, [2 + 2 ** -21, 2 + 2 ** -18, 2 + 2 ** -18][i % 3]))  # c brings 2.0: 4.8e-7, 3.8e-6 below
+        if i % 3 == 2:
+            e += [(0, b, 1.0), (b, d, 0.5), (d, x, 0.5 + 2 ** -18 - 2 ** -21)]  # 4.8e-7 below
+    base = 1 + 7 * copies
+    at = np.arange(filler)
+    u, v, w = (np.array(c) for c in zip(*e))
+    u = np.concatenate([u, base + at % 1000])
+    v = np.concatenate([v, base + 1000 + at // 1000])
+    w = np.concatenate([w, np.ones(filler)]).astype(np.float32)
+    perm = np.random.default_rng(copies).permutation(int(max(u.max(), v.max())) + 1)
+    return perm[u].astype(np.int32), perm[v].astype(np.int32), w
+
+
+@pytest.mark.parametrize("kind,copies,filler", [("lone", 3, 0), ("lone", 13, 0), ("group", 40, 0), ("group", 1200, 0),
+                                                ("device", 3000, 200_000), ("sweep", 6000, 0)])
+def test_improvements_within_the_tolerance(oracle, kind, copies, filler):
+    """Every kind of listed round stores an improvement of at most 1e-6 and does not carry it on, as sssp.cu:62-68: the same
+    distances and flags as the oracle's, whichever kernel runs the round.  A sweep takes it along."""
+    from drone_amd.traverse import SSSPWorkerCUDA
+    u, v, length = _near_ties(copies, filler)
+    nglobal, start = int(max(u.max(), v.max())) + 1, int(u[0])
+    n, g2l, l2g, index, dst = oracle.build_graph(nglobal, u, v)
+    by_edge = {(a, b): w for a, b, w in zip(u.tolist(), v.tolist(), length.tolist())}
+    src = np.repeat(np.arange(n), np.diff(index))
+    local = np.array([by_edge[e] for e in zip(l2g[src].tolist(), l2g[dst].tolist())], np.float32)
+    st = oracle.SSSPState(index, dst, local)
+    st.peval(int(g2l[start]))
+    exact = _bellman(index, dst, int(g2l[start]), local)
+    assert (exact < st.val).sum() == 2 * ((copies + 2) // 3)  # y and z of the copies that fall by little
+    w = SSSPWorkerCUDA(nglobal, u, v, startId=start)
+    try:
+        w.set_edge_len(local)
+        for _ in range(2):
+            res = w.peval()
+            got = w.read()
+            if kind == "sweep":
+                assert (exact <= got).all() and (got <= st.val).all()
+            else:
+                np.testing.assert_array_equal(got, st.val)
+                np.testing.assert_array_equal(np.sign(w.flags()["active"]), np.sign(st.active))
+            assert res.VisitedSize == st.visited()
+    finally:
+        w.close()
+
+
+def test_cycle_that_falls_within_the_tolerance():
+    """A cycle whose length is negative by less than the tolerance ends after one turn, without an error (sssp.cu:64)."""
+    from drone_amd import _lib
+    from drone_amd.traverse import SSSPWorkerCUDA
+    w = SSSPWorkerCUDA(3, np.array([0, 1, 2], np.int32), np.array([1, 2, 0], np.int32), startId=0)
+    try:
+        w.set_edge_len(np.array([1.0, 1.0, -2 - 2 ** -21], np.float32))
+        w.peval()
+        assert _lib.lib().drone_last_error() == 0
+        np.testing.assert_array_equal(w.read(), np.array([-2 ** -21, 1.0, 2.0], np.float32))
+    finally:
+        w.close()
