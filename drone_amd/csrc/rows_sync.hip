@@ -133,8 +133,8 @@ struct WorkerRows {
 };
 
 // Sums the rows of this worker's masters and their mirrors (ascending by worker) and writes the sums to all of them, the
-// mirrors' through the compressed form if the rows would travel in it.  G lanes per master.  A vertex has one master, so
-// no other worker touches these rows.
+// mirrors' through the compressed form if the rows would travel in it.  G lanes per master.  A master here is no mirror of
+// another worker's and its mirrors name this worker alone (direct_match_kernel), so no other worker touches these rows.
 template <bool kCompressed, int G>
 __global__ __launch_bounds__(kWave * kRowsPerBlock) void rows_direct_kernel(
     int masters, const int *__restrict__ master_row, const int *__restrict__ first, const int2 *__restrict__ mirror, int me, int K,
@@ -193,15 +193,16 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock) void rows_direct_kernel(
 }
 
 // row[i] = local id on the mirror's worker of the i-th (master, mirror worker) item of one worker's group; *bad counts items
-// that are no mirror of a master here.
+// that are no mirror of a master here, and those whose master here is itself a mirror: its row would be summed by its own
+// master's worker at the same time.
 __global__ void direct_match_kernel(int items, const int *__restrict__ item_vertex, const int *__restrict__ l2g,
-                                    const int *__restrict__ peer_g2l, int peer_nglobal, const int *__restrict__ peer_m2w, int me,
-                                    int *__restrict__ row, int *__restrict__ bad)
+                                    const int *__restrict__ own_m2w, const int *__restrict__ peer_g2l, int peer_nglobal,
+                                    const int *__restrict__ peer_m2w, int me, int *__restrict__ row, int *__restrict__ bad)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
         const int gid = l2g[item_vertex[i]];
         const int l = gid >= 0 && gid < peer_nglobal ? peer_g2l[gid] : -1;
-        if (l < 0 || peer_m2w[l] != me) atomicAdd(bad, 1);
+        if (l < 0 || peer_m2w[l] != me || own_m2w[item_vertex[i]] != -1) atomicAdd(bad, 1);
         row[i] = l;
     }
 }
@@ -370,7 +371,7 @@ int ensure_row_staging(RowSync *rs, int capacity, int K)
 }
 
 // Makes `d` for the workers of the offers.  agrees: every item of this worker's lists is a mirror there that names this worker
-// as its master's, no item comes twice, and the mirrors there are no more than these.
+// as its master's, its master here is no mirror, no item comes twice, and the mirrors there are no more than these.
 int direct_rows_make(DirectRows *d, Graph *g, drone_transport *tr, int me, int workerNum, hipStream_t s, bool *agrees)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
@@ -388,8 +389,8 @@ int direct_rows_make(DirectRows *d, Graph *g, drone_transport *tr, int me, int w
             if (count == 0) continue;
             const Graph *p = loopback_offer(tr, w).g;
             direct_match_kernel<<<(unsigned)std::min<int64_t>(ceil_div(count, 256), 2048), 256, 0, s>>>(
-                count, r.master_vertex + r.master_off[w], g->Local2Global, p->Global2Local, *p->globalVertexSize, p->Mirror2Worker,
-                me, r.pos + r.master_off[w], r.unknown);
+                count, r.master_vertex + r.master_off[w], g->Local2Global, g->Mirror2Worker, p->Global2Local, *p->globalVertexSize,
+                p->Mirror2Worker, me, r.pos + r.master_off[w], r.unknown);
         }
         DRONE_HIP_TRY(hipGetLastError());
         DRONE_HIP_TRY(hipMemcpyAsync(r.unknown_h, r.unknown, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -54,3 +54,52 @@ def test_rows_direct(oracle, W, Ks, agree, compress):
             lib().drone_graph_destroy(w.g)
             w.g = None
         lb.close()
+
+
+@pytest.mark.parametrize("compress", [False, True])
+def test_chains_of_masters_take_the_general_path(oracle, compress):
+    """Tables that agree item by item, but where a worker's master is itself a mirror of another's (C's mirror names A, A's own
+    row is a mirror of B's): two workers would write A's row at once, so nothing is summed in place."""
+    import torch
+    from drone_amd import gcn, rmat
+    from drone_amd._lib import lib
+    from drone_amd.pagerank import Loopback, run_workers
+    from drone_amd.traverse import _WorkerCUDA
+    n, W, K = 1 << 9, 3, 37
+    u, v = rmat.clean_directed_np(*rmat.rmat_edges(9, 8 << 9, seed=5))
+    parts, master = vertex_cut(u, v, W, 5)
+    lists = [({int(x): [] for x in p["master_vertex"]}, dict(zip(p["mirror_vertex"].tolist(), p["master_worker"].tolist()))) for p in parts]
+    for w, (_, mirrors) in enumerate(lists):
+        for x, b in mirrors.items():
+            lists[b][0][x].append(w)
+    chained = 0
+    for x, b in master.items():
+        if len(lists[b][0].get(x, [])) == 2:
+            a, c = lists[b][0][x]
+            lists[b][0][x], lists[a][0][x], lists[c][1][x] = [a], [c], a
+            chained += 1
+    assert chained > 50
+    for p, (masters, mirrors) in zip(parts, lists):
+        p.update(master_vertex=np.array(sorted(masters), np.int32), mirror_number=np.array([len(masters[x]) for x in sorted(masters)], np.int32),
+                 mirror_workers=np.array([w for x in sorted(masters) for w in masters[x]], np.int32),
+                 mirror_vertex=np.array(sorted(mirrors), np.int32), master_worker=np.array([mirrors[x] for x in sorted(mirrors)], np.int32))
+    local = [oracle.build_graph(n, p["u"], p["v"])[2] for p in parts]
+    tops = [oracle.Part(l2g, n, p["master_vertex"], p["mirror_number"], p["mirror_workers"], p["mirror_vertex"], p["master_worker"])
+            for l2g, p in zip(local, parts)]
+    rng = np.random.default_rng(7)
+    lb = Loopback(W, timeout_ms=60000)
+    ws = [_WorkerCUDA(n, p["u"], p["v"], workerId=i, workerNum=W, routes=p, loopback=lb) for i, p in enumerate(parts)]
+    try:
+        host = [rng.standard_normal((len(l2g), K)).astype(np.float32) for l2g in local]
+        rows = [torch.from_numpy(h.copy()).cuda() for h in host]
+        torch.cuda.synchronize()
+        want = oracle.graphsum_sync_rows(tops, host, compress=compress)
+        got = run_workers([(lambda i=i: gcn.graphsum_sync_rows(ws[i].g, rows[i], i, W, ws[i].comm, compress)) for i in range(W)])
+        for i in range(W):
+            assert got[i] == (want[0][i], want[1][i])
+            np.testing.assert_array_equal(rows[i].cpu().numpy(), host[i])
+    finally:
+        for w in ws:
+            lib().drone_graph_destroy(w.g)
+            w.g = None
+        lb.close()
