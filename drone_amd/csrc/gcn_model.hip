@@ -13,10 +13,11 @@ using namespace drone;
 namespace {
 constexpr int kTruthBlocks = 256;  // work-groups at most
 
-// cuda_kernel.cu:463-467; count (optional): the labelled rows, which the mean-reduced gradient is divided by.
+// cuda_kernel.cu:463-467; count (optional): the labelled rows, which the mean-reduced gradient is divided by, also in pinned
+// memory for the host.
 __global__ __launch_bounds__(kSpmvBlock) void set_truth_kernel(int *__restrict__ truth, const int *__restrict__ split,
                                                               const int *__restrict__ label, int current_split, int n,
-                                                              int *count, double *part, unsigned int *ticket)
+                                                              int *count, int *count_h, double *part, unsigned int *ticket)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
     double labelled = 0.0;
@@ -31,23 +32,31 @@ __global__ __launch_bounds__(kSpmvBlock) void set_truth_kernel(int *__restrict__
     if (threadIdx.x == 0) one = publish_part(part + blockIdx.x, total);
     if (!last_block_done(ticket, one)) return;
     const double all = block_sum_of_parts(part, (int)gridDim.x, s_red);
-    if (threadIdx.x == 0) *count = (int)all;
+    if (threadIdx.x == 0) *count = *count_h = (int)all;
 }
 }  // namespace
 
-void drone_gcn_mod::GCN::set_truth(int current_split)
+void drone_gcn_mod::GCN::choose_truth(int current_split)
 {
     const int n = params.localVertexSize;
+    // recounted only when the split changes (labels and split ids are fixed for the handle's lifetime)
+    const bool counts_rows = params.mean_gradient && current_split != truth_split;
     const size_t part_bytes = sizeof(double) * kTruthBlocks, ticket_bytes = sizeof(unsigned int) * ticket_words(kTruthBlocks);
-    if (truth_count && !truth_scratch) {
+    if (counts_rows && !truth_scratch) {
         DRONE_GCN_HIP(hipMalloc(&truth_scratch, part_bytes + ticket_bytes));
         DRONE_GCN_HIP(hipMemset(truth_scratch, 0, part_bytes + ticket_bytes));
         DRONE_GCN_HIP(hipStreamSynchronize(nullptr));
     }
     double *part = static_cast<double *>(truth_scratch);
     set_truth_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), kTruthBlocks), kSpmvBlock, 0, static_cast<hipStream_t>(s)>>>(
-        truth, split, label, current_split, n, truth_count, part, reinterpret_cast<unsigned int *>(part + kTruthBlocks));
+        truth, split, label, current_split, n, counts_rows ? labelled : nullptr, labelled_h, part,
+        reinterpret_cast<unsigned int *>(part + kTruthBlocks));
     DRONE_GCN_HIP(hipGetLastError());
+    truth_split = current_split;
+    if (counts_rows) {
+        ce->mean_over = labelled;
+        truth_pending = true;
+    }
 }
 
 struct drone_gcn {

@@ -12,6 +12,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <cstddef>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -341,23 +342,16 @@ class CrossEntropyLoss : public Module {
     int num_classes;
     drone_stream_t s;
 public:
-    float *d_loss = nullptr;  // device scalars
-    int *d_count = nullptr;
+    float *d_loss = nullptr;  // pinned scalar that the device writes: GCN::read_metrics() reads it without a copy
+    int *d_count = nullptr;   // device scalar
     float grad_scale = 1.0f;  // 1 = the reference's sum-reduced gradient
     const int *mean_over = nullptr;  // device: scale the gradient by 1 / *mean_over instead
     // what is reported with the loss (drone_loss_pass); null / 0: nothing
     const int *skip = nullptr;
     const Variable *l2_weight = nullptr;
     drone_loss_report *report = nullptr;
-    CrossEntropyLoss(Variable *logits_, const int *truth_, int num_classes_, std::string name, drone_stream_t stream)
-        : logits(logits_), truth(truth_), num_classes(num_classes_), s(stream)
-    {
-        ModuleName = std::move(name);
-        DRONE_GCN_HIP(hipMalloc(&d_loss, sizeof(float)));
-        DRONE_GCN_HIP(hipMalloc(&d_count, sizeof(int)));
-    }
-    ~CrossEntropyLoss() override { (void)hipFree(d_loss); (void)hipFree(d_count); }
-    void forward(bool training) override
+    // What forward() enqueues.
+    drone_loss_pass pass(bool training) const
     {
         drone_loss_pass p = {};
         p.n = logits->rows;
@@ -374,6 +368,20 @@ public:
         p.loss = d_loss;
         p.labelled = d_count;
         p.report = report;
+        return p;
+    }
+    CrossEntropyLoss(Variable *logits_, const int *truth_, int num_classes_, std::string name, drone_stream_t stream)
+        : logits(logits_), truth(truth_), num_classes(num_classes_), s(stream)
+    {
+        ModuleName = std::move(name);
+        DRONE_GCN_HIP(hipHostMalloc(&d_loss, sizeof(float)));
+        *d_loss = 0.0f;
+        DRONE_GCN_HIP(hipMalloc(&d_count, sizeof(int)));
+    }
+    ~CrossEntropyLoss() override { (void)hipHostFree(d_loss); (void)hipFree(d_count); }
+    void forward(bool training) override
+    {
+        const drone_loss_pass p = pass(training);
         DRONE_GCN_CHECK(drone_loss_pass_f32(&p, s));
     }
     void backward() override {}
@@ -483,9 +491,16 @@ public:
     int input_cols = 0;          // inner dimension of layer 1's products: input_dim rounded up (padded_inner_dim)
     float *x_padded = nullptr;   // the model's zero-padded copy of X, when it needs one
     int *truth = nullptr;   // device [N]: label on rows of the current split, -1 elsewhere
-    int *truth_count = nullptr;  // device: labelled rows of the current split, kept with mean_gradient
+    int truth_split = -1, truth_count = 0;  // the split chosen last and, with mean_gradient, its labelled rows
+    // What a forward pass reports besides the loss, for the device and, once the stream has been waited for, for the host:
+    // pinned memory, so read_metrics() copies nothing.
+    drone_loss_report *report = nullptr;
+    float *l2_sum = nullptr;  // = &report->sum_squares: sum of W1^2 (cuda_gcn.cu:254-260)
+    int *counts = nullptr;    // = &report->correct: [2], correct and counted rows
+    int *labelled = nullptr;  // device: the labelled rows as set_truth's kernel counts them
+    int *labelled_h = nullptr;  // pinned: the same
+    bool truth_pending = false; // counted, but truth_count and ce->grad_scale do not hold it yet
     void *truth_scratch = nullptr;
-    drone_loss_report *report = nullptr;  // pinned: what the last forward pass reports
     const int *label = nullptr, *split = nullptr;  // device, borrowed
     drone_stream_t s;
 
@@ -543,9 +558,13 @@ public:
         const int max_dim = p.hidden_dim > p.output_dim ? p.hidden_dim : p.output_dim;
         adj.reset(new Adjacency(N, nnz, rp, ci, in_degree, out_degree, max_dim, s));
         DRONE_GCN_HIP(hipMalloc(&truth, sizeof(int) * (size_t)N));
-        if (p.mean_gradient) DRONE_GCN_HIP(hipMalloc(&truth_count, sizeof(int)));
+        DRONE_GCN_HIP(hipMalloc(&labelled, sizeof(int)));
+        DRONE_GCN_HIP(hipHostMalloc(&labelled_h, sizeof(int)));
         DRONE_GCN_HIP(hipHostMalloc(&report, sizeof(drone_loss_report)));
         *report = drone_loss_report{};
+        l2_sum = &report->sum_squares;
+        counts = &report->correct;
+        static_assert(offsetof(drone_loss_report, counted) == offsetof(drone_loss_report, correct) + sizeof(int), "counts[1]");
         const Replicas *r = cut ? &replicas : nullptr;
 
         if (p.fold_input_aggregation) {
@@ -580,7 +599,6 @@ public:
         // cuda_gcn.cu:298-299, 314-315: what train_epoch / eval report besides the loss - the accuracy over the labelled
         // rows that are not mirrors (:226-246) and the L2 penalty weight_decay * sum(W1^2) / 2 (:254-260), from the
         // weights as they are before the optimiser step - comes out of the loss's launch
-        ce->mean_over = truth_count;
         ce->skip = mirror2worker;
         ce->l2_weight = layer1_weight;
         ce->report = report;
@@ -599,21 +617,41 @@ public:
     {
         (void)hipFree(x_padded);
         (void)hipFree(truth);
-        (void)hipFree(truth_count);
+        (void)hipFree(labelled);
+        (void)hipHostFree(labelled_h);
         (void)hipFree(truth_scratch);
         (void)hipHostFree(report);
     }
 
-    void set_truth(int current_split);  // cuda_gcn.cu:211-223; defined in gcn_model.hip (needs a kernel)
-    // The modules in order.
+    // cuda_gcn.cu:211-223.  With mean_gradient a change of the split waits for the stream: truth_count and ce->grad_scale
+    // are the new split's when it returns (on a capturing stream they follow at the next read_metrics()).
+    void set_truth(int current_split)
+    {
+        choose_truth(current_split);
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (truth_pending) DRONE_GCN_HIP(hipStreamIsCapturing(static_cast<hipStream_t>(s), &capturing));
+        if (!truth_pending || capturing != hipStreamCaptureStatusNone) return;
+        DRONE_GCN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(s)));
+        settle_truth();
+    }
+    // The modules in order; the loss's launch leaves the counts and sums read_metrics() reports (cuda_gcn.cu:298-299 takes
+    // them right after the forward pass too).
     void forward(bool training)
     {
         for (auto &m : modules) m->forward(training);
     }
+    // The counts and the sum of squares once more, from the logits, truth and weights as they are now.
+    void metrics_async()
+    {
+        drone_loss_pass p = ce->pass(false);
+        p.loss = nullptr;
+        p.labelled = nullptr;
+        DRONE_GCN_CHECK(drone_loss_pass_f32(&p, s));
+    }
     void backward() { for (int i = (int)modules.size() - 1; i >= 0; --i) modules[i]->backward(); }
 
     // Enqueues one training step (cuda_gcn.cu:287-306 without the host read-backs): forward, accuracy counts,
-    // backward, optimiser.  Loss and counts lie in `report` once the stream has been waited for: read_metrics().
+    // backward, optimiser.  Loss and counts stay where they are until read_metrics().
     void train_step_async()
     {
         forward(true);
@@ -625,21 +663,35 @@ public:
     std::pair<float, float> read_metrics(float *cross_entropy = nullptr)
     {
         DRONE_GCN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(s)));
-        if (cross_entropy) *cross_entropy = report->loss;
-        return {report->loss + params.weight_decay * report->sum_squares / 2,
-                report->counted ? (float)report->correct / (float)report->counted : 0.0f};
+        settle_truth();
+        const float loss = *ce->d_loss;
+        if (cross_entropy) *cross_entropy = loss;
+        return {loss + params.weight_decay * *l2_sum / 2, counts[1] ? (float)counts[0] / (float)counts[1] : 0.0f};
     }
     std::pair<float, float> train_epoch()
     {
-        set_truth(1);
+        choose_truth(1);
         train_step_async();
         return read_metrics();
     }
     std::pair<float, float> eval(int current_split)  // cuda_gcn.cu:308-318
     {
-        set_truth(current_split);
+        choose_truth(current_split);
         forward(false);
         return read_metrics();
+    }
+
+private:
+    // Enqueues the new truth.  With mean_gradient a change of the split also counts its labelled rows, and until
+    // settle_truth() the loss takes that count from the device: train_epoch() and eval() need no wait before their own.
+    void choose_truth(int current_split);  // defined in gcn_model.hip (needs a kernel)
+    void settle_truth()  // behind a wait for the stream
+    {
+        if (!truth_pending) return;
+        truth_pending = false;
+        truth_count = *labelled_h;
+        ce->grad_scale = truth_count > 0 ? 1.0f / (float)truth_count : 1.0f;
+        ce->mean_over = nullptr;
     }
 };
 
