@@ -66,27 +66,21 @@ class Loopback:
 def run_workers(calls):
     """Runs one callable per worker, each on its own thread (the foreign calls release the GIL), and returns their
     results in order.  The first exception is re-raised."""
-    import _thread
-    out, err, ended = [None] * len(calls), [None] * len(calls), [_thread.allocate_lock() for _ in calls]
+    import threading
+    out, err = [None] * len(calls), [None] * len(calls)
 
     def body(i):
         try:
             out[i] = calls[i]()
         except BaseException as e:  # noqa: BLE001
             err[i] = e
-        finally:
-            ended[i].release()
 
-    # without the bookkeeping of threading.Thread, and the first worker on the caller's thread: a thread that is started and
-    # waited for costs as much as a kernel or two, and the last worker can only begin when all of them have been started
-    for lock in ended:
-        lock.acquire()
-    for i in range(1, len(calls)):
-        _thread.start_new_thread(body, (i,))
-    if calls:
-        body(0)
-    for lock in ended:
-        lock.acquire()
+    # none on the caller's: the entry points make their subgraph's GPU the calling thread's current one
+    ts = [threading.Thread(target=body, args=(i,)) for i in range(len(calls))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
     for e in err:
         if e is not None:
             raise e
