@@ -497,6 +497,30 @@ __global__ void fill_f32_kernel(float *__restrict__ x, int64_t n, float value)
 std::mutex g_mutex;
 std::map<std::pair<int, hipStream_t>, void *> g_loss_scratch;
 
+// Zeroed on a stream of its own and waited for: the caller's may be recording a graph, and then a fill on it would run at
+// the replays instead of now.
+int loss_scratch_create(void **out)
+{
+    void *p = nullptr;
+    hipStream_t once = nullptr;
+    DRONE_HIP_TRY(hipMalloc(&p, LossScratch::bytes()));
+    hipError_t e = hipStreamCreateWithFlags(&once, hipStreamNonBlocking);
+    if (e == hipSuccess) {
+        fill_f32_kernel<<<64, kThreads, 0, once>>>(static_cast<float *>(p), (int64_t)(LossScratch::bytes() / sizeof(float)), 0.0f);
+        e = hipGetLastError();
+        const hipError_t waited = hipStreamSynchronize(once);
+        if (e == hipSuccess) e = waited;
+        (void)hipStreamDestroy(once);
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        set_error(DRONE_ERR_HIP, "scratch of the loss: %s", hipGetErrorString(e));
+        return DRONE_ERR_HIP;
+    }
+    *out = p;
+    return DRONE_OK;
+}
+
 }  // namespace
 }  // namespace drone
 
@@ -607,8 +631,8 @@ extern "C" int drone_loss_pass_f32(const drone_loss_pass *pass, drone_stream_t s
         std::lock_guard<std::mutex> lock(g_mutex);
         void *&slot = g_loss_scratch[std::make_pair(dev, s)];
         if (!slot) {
-            DRONE_HIP_TRY(hipMalloc(&slot, LossScratch::bytes()));
-            fill_f32_kernel<<<64, kThreads, 0, s>>>(static_cast<float *>(slot), (int64_t)(LossScratch::bytes() / sizeof(float)), 0.0f);
+            const int rc = loss_scratch_create(&slot);
+            if (rc != DRONE_OK) return rc;
         }
         ws = slot;
     }

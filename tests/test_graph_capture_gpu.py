@@ -83,3 +83,39 @@ def test_pagerank_iterations_in_a_hip_graph(T, deterministic):
         else:
             assert float(((out - eager).abs() / eager).max()) <= 1e-12, it
     plan.close()
+
+
+def test_first_loss_on_a_stream_is_recorded(T):
+    """The first loss of a stream is recorded, not run: the scratch it makes has to be ready for the calls that are run before
+    (and between) the replays."""
+    from drone_amd._lib import check, lib
+    n, classes = 5000, 7
+    gen = T.Generator(device="cuda").manual_seed(3)
+    z = T.randn(n, classes, generator=gen, device="cuda")
+    truth = T.randint(0, classes, (n,), generator=gen, device="cuda", dtype=T.int32)
+    want = float(T.nn.functional.cross_entropy(z.double(), truth.long()))
+    loss, count = T.zeros(1, device="cuda"), T.zeros(1, dtype=T.int32, device="cuda")
+    junk = T.full((1 << 20,), -1, dtype=T.int32, device="cuda")
+    T.cuda.synchronize()
+    del junk
+    T.cuda.empty_cache()
+    side, graph = T.cuda.Stream(), T.cuda.CUDAGraph()
+
+    def call():
+        check(lib().drone_cross_entropy_f32(n, classes, z.data_ptr(), classes, truth.data_ptr(), None, classes, 1.0, loss.data_ptr(),
+                                            count.data_ptr(), side.cuda_stream))
+
+    def result():
+        T.cuda.synchronize()
+        got = float(loss), int(count)
+        loss.zero_(), count.zero_()
+        T.cuda.synchronize()
+        assert got[1] == n and abs(got[0] - want) <= 1e-6 * want  # fp32 exp and log of values near 1, summed in fp64
+
+    with T.cuda.graph(graph, stream=side, capture_error_mode="relaxed"):
+        call()
+    for _ in range(3):
+        call()
+        result()
+        graph.replay()
+        result()
