@@ -758,6 +758,7 @@ struct SmallRounds {
     Value *s_old;
     unsigned long long *s_counters;  // [2]: of the current list and of the one being built, by turns
     int *s_ends;                     // [2]: lowered vertices that do not propagate (no out-edges, or within the tolerance): kept from the list's far end
+    int *s_slight;                   // whether an edge of the round lowers its target within the tolerance
     LoneShared *s_lone;
     const FirstEdges *__restrict__ first;  // null where the graph has none
     const int *__restrict__ index;
@@ -836,26 +837,27 @@ struct SmallRounds {
                 }
                 atomicMin(&s_slot_val[slot], order_of(nv[k]));
             };
-            bool slight = false;
 #pragma unroll
             for (int k = 0; k < PER; ++k)
                 if (tid + k * T < m && nv[k] < old[k]) {
                     if (Push::activates(old[k], nv[k])) keep(k, true);
-                    else slight = true;
+                    else *s_slight = 1;
                 }
-            if constexpr (Push::kTolerance) {
+            __syncthreads();  // the next list is complete
+            const int n2 = (int)(s_counters[now ^ 1] >> 32);
+            int ends2 = s_ends[now ^ 1];
+            // (a word of LDS and not __syncthreads_or: that took a 40 x 1,000 grid from 2.31 to 2.74 ms)
+            if (Push::kTolerance && *s_slight) {
                 // Targets that no edge lowers past the tolerance: their value is stored and goes no further.  After the
                 // others, so that a target that one edge lowers a little and another by more is on the list.
-                if (__syncthreads_or(slight)) {
-#pragma unroll
-                    for (int k = 0; k < PER; ++k)
-                        if (tid + k * T < m && nv[k] < old[k] && !Push::activates(old[k], nv[k])) keep(k, false);
-                    __syncthreads();
-                }
-            } else {
                 __syncthreads();
-            }  // the next list is complete
-            const int n2 = (int)(s_counters[now ^ 1] >> 32), ends2 = s_ends[now ^ 1];
+#pragma unroll
+                for (int k = 0; k < PER; ++k)
+                    if (tid + k * T < m && nv[k] < old[k] && !Push::activates(old[k], nv[k])) keep(k, false);
+                if (tid == 0) *s_slight = 0;
+                __syncthreads();
+                ends2 = s_ends[now ^ 1];
+            }
             const auto settle = [&](int i) {  // the vertex's value out of its slot, which is emptied
                 const int slot = s_val[i];
                 s_val[i] = s_slot_val[slot];
@@ -1043,7 +1045,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     extern __shared__ int s_small[];
     __shared__ LoneShared s_lone;
     __shared__ unsigned long long s_counters[2];
-    __shared__ int s_ends[2], s_rounds, s_pending, s_done;
+    __shared__ int s_ends[2], s_rounds, s_pending, s_done, s_slight;
     SmallRounds<Push> sr;
     sr.s_start = s_small;
     sr.s_edge = sr.s_start + kSmallEdges;
@@ -1054,6 +1056,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     sr.s_slot_val = sr.s_slot_vertex + kSmallSlots;
     sr.s_counters = s_counters;
     sr.s_ends = s_ends;
+    sr.s_slight = &s_slight;
     sr.s_lone = &s_lone;
     sr.first = first;
     sr.index = index;
@@ -1081,7 +1084,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
         s_counters[0] = ((unsigned long long)count << 32) + (unsigned long long)edges;
         s_counters[1] = 0ull;
         s_ends[0] = s_ends[1] = 0;
-        s_done = 0;
+        s_done = s_slight = 0;
     }
     __syncthreads();
     int rounds = 0;
