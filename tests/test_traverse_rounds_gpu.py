@@ -175,3 +175,24 @@ def test_cycle_that_falls_within_the_tolerance():
         np.testing.assert_array_equal(w.read(), np.array([-2 ** -21, 1.0, 2.0], np.float32))
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("pairs,more", [((8 << 20) // 2, 32), ((8 << 20) // 2 + 1, 0)])
+def test_memory_of_large_graphs_is_bounded(pairs, more):
+    """What the first call keeps per vertex: its state (three words), four words of lists and, up to 8 Mi vertices, 32 bytes of
+    first edges.  Pairs of vertices, one edge each."""
+    import torch
+    from drone_amd.traverse import CCWorkerCUDA
+    u = np.arange(0, 2 * pairs, 2, dtype=np.int32)
+    w = CCWorkerCUDA(2 * pairs, u, u + 1)
+    try:
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        res = w.peval()
+        kept = before - torch.cuda.mem_get_info()[0]
+        want = 2 * pairs * (12 + 16 + more)
+        assert abs(kept - want) <= 24 << 20, (kept, want)  # allocations come in pieces of at least 2 MB
+        assert res.VisitedSize == pairs
+        np.testing.assert_array_equal(w.read(), np.arange(2 * pairs) // 2 * 2)
+    finally:
+        w.close()
