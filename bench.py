@@ -375,8 +375,8 @@ def bench_spmm_sweep(cpu_baseline=False, widths=(16, 64, 256)):
 
 def bench_traverse(cpu_baseline=True):
     """SSSP_PEVal (unit lengths, directed R-MAT scale 22 ef 16 seed 2) and CC_PEVal (the same graph symmetrised) through
-    the Go worker's boundary: one subgraph to its local fixed point.  TEPS = edges of the subgraph / time of the call.
-    The CPU figure is the oracle's serial restatement of sssp.cu / cc.cu, one thread."""
+    the Go worker's boundary: one subgraph to its local fixed point.  TEPS of SSSP = edges of the subgraph / time of the
+    call; CC is reported in milliseconds only (most of its edges are never looked at).  The CPU figure is the oracle's serial restatement of sssp.cu / cc.cu, one thread."""
     import numpy as np
     from drone_amd import rmat
     from drone_amd.traverse import CCWorkerCUDA, SSSPWorkerCUDA
@@ -389,8 +389,7 @@ def bench_traverse(cpu_baseline=True):
     def run(worker, edges, name):
         worker.peval()
         ms = min(timed_ms(worker.peval) for _ in range(3))
-        out[name] = {"edges": int(edges), "local_vertices": int(worker.n), "peval_ms": ms,
-                     "GTEPS": edges / (ms * 1e-3) / 1e9}
+        out[name] = {"edges": int(edges), "local_vertices": int(worker.n), "peval_ms": ms}
         return worker.read()
 
     def timed_ms(fn):
@@ -400,6 +399,7 @@ def bench_traverse(cpu_baseline=True):
 
     w = SSSPWorkerCUDA(n, u, v, startId=int(u[0]))
     dist = run(w, len(u), "sssp")
+    out["sssp"]["GTEPS"] = len(u) / (out["sssp"]["peval_ms"] * 1e-3) / 1e9
     w.close()
     us, vs = np.concatenate([u, v]).astype(np.int64), np.concatenate([v, u]).astype(np.int64)
     key = np.unique((us << 32) | vs)
@@ -426,8 +426,7 @@ def bench_traverse(cpu_baseline=True):
         nl, g2l, l2g, index, dst = oracle.build_graph(n, us, vs)
         st = oracle.CCState(index, dst)
         ms = timed_ms(st.peval)
-        out["cc"]["cpu_baseline"] = {"value": len(us) / (ms * 1e-3) / 1e9, "unit": "GTEPS", "cores": 1, "kind": "port",
-                                     "ms": ms, "identical": bool(np.array_equal(st.val, lab))}
+        out["cc"]["cpu_baseline"] = {"value": ms, "unit": "ms", "cores": 1, "kind": "port", "identical": bool(np.array_equal(st.val, lab))}
     return out
 
 
