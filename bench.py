@@ -2,7 +2,7 @@
 
 python bench.py [--gpus 1] [--steps K] [--warmup W]
 
-Headline workload (the second benchmark configuration, configs[1]): PageRank on one subgraph at real shape - R-MAT scale 24, edge
+Headline workload: PageRank on one subgraph at real shape - R-MAT scale 24, edge
 factor 16, seed 2, in-edge CSR (int64 row_ptr, int32 col_idx), fp64 ranks, damping 0.85.  One "step" is one
 complete 50-iteration PageRank job through drone_pr_run_f64; inputs are resident in HBM before the timed
 region.  value = directed edges in the CSR x 50 x K / seconds / 1e9 (GTEPS).
@@ -19,7 +19,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# R-MAT candidates drawn for configs[3]: after rejecting ids >= 232,965, self-loops and duplicates this leaves
+# R-MAT candidates drawn for the GCN step's graph: after rejecting ids >= 232,965, self-loops and duplicates this leaves
 # about 114.6 M undirected edges (the figure the configuration names); the exact count is printed and reported.
 C4_CANDIDATES = 221_000_000
 
@@ -65,7 +65,7 @@ def pr_traffic_from_profile(path=PR_TRAFFIC_PROFILE):
 
 def cpu_baselines(x_host, alpha, threads):
     """Oracle timings on the host cores: (a) fp64 pull over the same CSR, a bounded number of iterations;
-    (b) the map-based float delta-push restatement of DRONE's Go 'pr' job on configs[0] (scale 16)."""
+    (b) the map-based float delta-push restatement of DRONE's Go 'pr' job on R-MAT scale 16."""
     import numpy as np
     from oracle import oracle as orc
     from drone_amd import rmat
@@ -92,7 +92,7 @@ def cpu_baselines(x_host, alpha, threads):
     g.close()
     go = dict(value=edges / dt / 1e9, unit="GTEPS", cores=1, kind="port",
               sample=f"map-based float32 delta-push restatement of DRONE's Go pr job, R-MAT scale 16 "
-                     f"(configs[0]), PEval + 20 IncEval at eps=0, {edges} edge traversals in {dt:.2f} s")
+                     f"(R-MAT scale 16), PEval + 20 IncEval at eps=0, {edges} edge traversals in {dt:.2f} s")
     return pull, go
 
 
@@ -158,7 +158,7 @@ def spmm_report(name, n, nnz, K, ms, traffic_label=None):
 
 
 def bench_gcn_step(steps, warmup, cpu_baseline=False):
-    """configs[3]: 2-layer GCN training step on the dense power-law graph (232,965 vertices)."""
+    """2-layer GCN training step on the dense power-law graph (232,965 vertices)."""
     import numpy as np
     import torch
     from drone_amd import gcn, graphs, rmat
@@ -270,7 +270,7 @@ def bench_gcn_step(steps, warmup, cpu_baseline=False):
         log(f"cpu baseline SpMM K=128: {cpu['value']:.0f} ms on {cpu['cores']} threads (GPU {kernels[0]['ms']:.2f} ms)")
     plan.close()
     return {"cpu_baseline_spmm": cpu,
-            "workload": f"2-layer GCN training step (configs[3]): N={N}, nnz={nnz}, 602->128->41, ReLU, dropout 0.5, "
+            "workload": f"2-layer GCN training step: N={N}, nnz={nnz}, 602->128->41, ReLU, dropout 0.5, "
                         "softmax cross-entropy, SGD lr 0.01, fp32",
             "step_ms": step_ms, "steps": steps, "setup_ms_one_off": setup_s * 1e3,
             "step_contains": "SpMM K=128 forward, K=41 forward, K=41 backward, K=128 backward; 5 GEMMs; glue",
@@ -300,7 +300,7 @@ def cpu_spmm_baseline(rp, ci, val, N, K, nnz, seed=7):
 
 
 def bench_gcn_layer(cpu_baseline=False):
-    """one GCN layer forward ReLU(A_hat * (H * W)), R-MAT scale 20."""
+    """One GCN layer forward ReLU(A_hat * (H * W)), R-MAT scale 20."""
     import torch
     from drone_amd import gcn, graphs, rmat
     g = graphs.gcn_graph_torch(20, 16, seed=3)
@@ -328,9 +328,9 @@ def bench_gcn_layer(cpu_baseline=False):
     cpu = cpu_spmm_baseline(g["rp"], g["ci"], val, N, K, nnz) if cpu_baseline else None
     if cpu:
         cpu["gpu_ms"] = ms_spmm
-    log(f"GCN layer (configs[2]): {ms:.2f} ms, SpMM {ms_spmm:.2f} ms, GEMM {ms_gemm:.2f} ms" +
+    log(f"GCN layer: {ms:.2f} ms, SpMM {ms_spmm:.2f} ms, GEMM {ms_gemm:.2f} ms" +
         (f"; CPU SpMM {cpu['value']:.0f} ms on {cpu['cores']} threads" if cpu else ""))
-    return {"workload": f"GCN layer forward (configs[2]): R-MAT scale 20 undirected + self-loops, N={N}, nnz={nnz}, K=128",
+    return {"workload": f"GCN layer forward: R-MAT scale 20 undirected + self-loops, N={N}, nnz={nnz}, K=128",
             "layer_ms": ms, "spmm": spmm_report("spmm (rows + band pieces + bit core) K=128", N, nnz, K, ms_spmm,
                                                 traffic_label="c3_K128"),
             "spmm_plan": plan_info,
@@ -339,7 +339,7 @@ def bench_gcn_layer(cpu_baseline=False):
 
 
 def bench_spmm_sweep(cpu_baseline=False, widths=(16, 64, 256)):
-    """skew-stress SpMM sweep, R-MAT scale 22 ef 32 a/b/c = .70/.12/.12, row-normalised, K in 16/64/256,
+    """Skew-stress SpMM sweep, R-MAT scale 22 ef 32 a/b/c = .70/.12/.12, row-normalised, K in 16/64/256,
     forward (A*H) and transpose (A^T*G)."""
     import torch
     from drone_amd import gcn, rmat
@@ -351,7 +351,7 @@ def bench_spmm_sweep(cpu_baseline=False, widths=(16, 64, 256)):
     val = (1.0 / torch.repeat_interleave(deg.float(), (rp[1:] - rp[:-1]).long())).contiguous()
     rpT, ciT, vT = gcn.csr_transpose(N, N, rp, ci, val)
     inv_deg, ones = (1.0 / deg.float()).contiguous(), torch.ones(N, device="cuda")   # val = inv_deg[row] * 1
-    out = {"workload": f"SpMM sweep (configs[4]): R-MAT scale 22 ef 32 skewed, N={N}, nnz={nnz}, max row "
+    out = {"workload": f"SpMM sweep: R-MAT scale 22 ef 32 skewed, N={N}, nnz={nnz}, max row "
                        f"{int((rp[1:]-rp[:-1]).max())}, max transposed row {int((rpT[1:]-rpT[:-1]).max())}", "kernels": []}
     for K in widths:
         H = torch.rand((N, K), device="cuda") * 2 - 1
@@ -363,7 +363,7 @@ def bench_spmm_sweep(cpu_baseline=False, widths=(16, 64, 256)):
             info = dict(plan.info(), bit_core=plan.bit_core())
             plan.close()
             out["kernels"].append(dict(spmm_report(f"{name} K={K}", N, nnz, K, ms, traffic_label=f"c5_K{K}"), plan=info))
-            log(f"SpMM sweep (configs[4]) {name} K={K}: {ms:.2f} ms = {out['kernels'][-1]['frac_of_hbm_peak']*100:.1f} % of "
+            log(f"SpMM sweep {name} K={K}: {ms:.2f} ms = {out['kernels'][-1]['frac_of_hbm_peak']*100:.1f} % of "
                 f"the HBM roofline")
         del H, C_
     if cpu_baseline and 64 in widths:
@@ -555,8 +555,8 @@ def main():
     ap.add_argument("--widths", default="16,64,256", help="feature widths of --suite sweep (a profiling run takes one)")
     ap.add_argument("--suite", default="default", choices=["pr", "default", "full", "gcn", "layer", "sweep", "traverse", "exchange"],
                     help="pr: PageRank only (fp64 pull plan, then the reference's PR_PEVal / PR_IncEVal on the same "
-                         "graph); default (= full): + the GCN training step (configs[3]), the GCN layer (configs[2]), "
-                         "the SpMM sweep (configs[4]), the SSSP / CC jobs and the replica exchange; gcn, layer, sweep, "
+                         "graph); default (= full): + the GCN training step, the GCN layer, "
+                         "the SpMM sweep, the SSSP / CC jobs and the replica exchange; gcn, layer, sweep, "
                          "traverse, exchange: that part alone")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
@@ -630,7 +630,7 @@ def main():
         "value": gteps, "unit": "GTEPS", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": dt / args.steps * 1e3, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f64", "data": "synthetic",
-        "config": {"workload": f"PageRank pull SpMV, R-MAT scale {args.scale} ef 16 seed 2 (configs[1]), "
+        "config": {"workload": f"PageRank pull SpMV, R-MAT scale {args.scale} ef 16 seed 2, "
                                f"N={n}, E={nnz} directed in-edges, int64 row_ptr / int32 col_idx, fp64, "
                                f"damping 0.85, {args.iters} iterations per step",
                    "iterations_per_step": args.iters, "vertices": n, "edges": nnz},

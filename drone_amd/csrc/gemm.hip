@@ -52,7 +52,7 @@ struct alignas(4) Float4U {
 // those of its own that exist in their place (store(): doing it here would wait for the load).  The last, partial tile of
 // the reduction takes dword loads with a check per element.  The two paths distribute the elements over the lanes
 // differently, so store() must be told which one filled the registers.  With checked dword loads for every tile that
-// reaches past the matrix, 30,011 x 301 x 100 took 41 us (36 now), 602 x 128 over 232,965 rows 384 (336), 1,000 x 3,000 x
+// reaches past the matrix, 30,011 x 301 x 100 took 41 us (36 now), 602 x 128 over 232,965 rows 384 (336; the model pads that operand), 1,000 x 3,000 x
 // 1,001 transposed 350 (208).
 template <int EXT, bool K_CONTIG, bool INSIDE>
 struct TileLoader {

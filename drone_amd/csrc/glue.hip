@@ -342,12 +342,12 @@ __global__ __launch_bounds__(kThreads) void loss_kernel(drone_loss_pass p, int r
 // cuda_gcn.cu:226-246: a labelled row is wrong iff some logit is strictly greater than the true-class logit; rows of
 // mirrors (skip[row] != -1, the reference's Mirror2WorkerHost) are left out of the counts (:234).
 // pred[row] = arg-max with ties to the lowest index (optional).  counts[0] += correct, counts[1] += labelled.
-// kAccGroups groups of 64 / L rows are in flight per wavefront, their logits in registers (see cross_entropy_kernel).
+// kAccGroups groups of 64 / L rows are in flight per wavefront, their logits in registers (see loss_kernel).
 constexpr int kAccGroups = 4;
 // Work-groups of 1024 lanes, at most one per CU: every work-group ends with two atomics on the same two counters, and
 // those cost about 9 ns each (1024 work-groups of 256 lanes: 40 us for 232,965 x 41, 2048: 58 us).
 constexpr int kAccThreads = 1024, kAccBlocks = 256;
-template <int L>  // lanes per row, as in cross_entropy_kernel
+template <int L>  // lanes per row, as in loss_kernel
 __global__ __launch_bounds__(kAccThreads) void accuracy_kernel(int n, int classes, const float *__restrict__ logits, int ld,
                                                             const int *__restrict__ truth, const int *__restrict__ skip,
                                                             int *__restrict__ pred, int *__restrict__ counts)

@@ -94,7 +94,8 @@ constexpr int kSplitRow = 512;          // rows with more non-zeros are cut into
 // matrix the longest one is what the launch waits for.  us with pieces of at most 1,024 / 256 / 128 entries: training step
 // on 30,011 vertices (0.7 M entries) 393 / 292 / 280, forward + transposed product of 20 K vertices and 0.3 M entries at
 // K = 128 163 / 87 / 74, 0.1 M vertices and 1 M entries at K = 64 125 / 85 / 80, 0.2 M vertices and 3 M entries at K = 32
-// 133 / 120 / 126, 1 M vertices and 15 M entries at K = 41 816 / 670 / 664; the 232,965-vertex step 8,818 / 8,721.
+// 133 / 120 / 126, 1 M vertices and 15 M entries at K = 41 816 / 670 / 664; the 232,965-vertex step
+// 8,818 / 8,721, less than its runs differ by.
 // The partial rows of a row are added one after the other, eight at a time: a row of very many entries gets longer pieces, so
 // that neither chain outgrows the other (16 entries against 8 pieces per round trip).
 constexpr int kLeastPiece = 128, kMostPiece = 256, kHubPiece = 1024;
