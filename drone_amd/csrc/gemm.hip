@@ -922,14 +922,23 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
             d.ks = K >= 384 ? 8 : K >= 64 ? 4 : 1;
         }
     }
+    // Deep reductions (384 steps and more) bring the tiled kernel's streams up to speed - 2.8 instead of 2.0 TB/s, and two of
+    // its work-groups on a CU take 0.85 of two rounds -, and the direct kernel, whose row blocks each read all of op(B), reaches
+    // 60 instead of 75 TFLOP/s there.  us direct / tiled: dense rectangles of an SpMM plan, 4,096 x 32,768 x 41 336 / 196 and
+    // 16,384 x 32,768 x 64 834 / 688; layers of 53,965 x 527 x 59 60 / 49, 128,580 x 582 x 63 151 / 118, 11,824 x 619 x 94
+    // 28 / 55.  With one set of rates for all depths an SpMM of 229 M entries and 41 columns under an ordinary plan took
+    // 2.46 ms (2.26).
+    const bool deep = K >= 384;
     // us: matrix instructions at the rate the kernel reaches on padded blocks, or its memory traffic
     const double in = 4.0 * ((double)M * K + (double)K * N), out = 4.0 * M * N;
     const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
-    const double direct_us = std::max(padded / 75e6, in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
+    const double direct_us = std::max(padded / (deep && !ta ? 60e6 : 75e6), in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
     // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.25 for a 128-wide one)
     const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
-    const double tiled_us = std::max(ceil_div((int64_t)tiles * splits, 256) * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.25),
-                                     in / 2.0e6 + out / 2.4e6) + (splits > 1 ? 5 : 0);
+    const int64_t groups = (int64_t)tiles * splits;
+    const double rounds = ceil_div(groups, 256) * (deep && groups > 256 ? 0.85 : 1.0);
+    const double tiled_us = std::max(rounds * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.25),
+                                     in / (deep ? 2.8e6 : 2.0e6) + out / 2.4e6) + (splits > 1 ? 5 : 0);
     if (tiled_us < direct_us) d.ks = 0;
     return d;
 }
