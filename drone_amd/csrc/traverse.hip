@@ -902,7 +902,9 @@ struct SmallRounds {
     // in registers and the L2 warm.  (Four edges per lane, up to 256: a 40 x 1,000 grid took 3.0 ms instead of 2.3.)
     // warm(), run by the other wavefronts beside it, brings the vertices' first edges into this XCD's L2 if they fit: a
     // launch finds it cold.  (Only what nobody writes.)  A branch that is taken costs the lone wavefront a refill of its
-    // instructions, so the common case is the one that falls through (without the hints a hop takes 0.41 us).
+    // instructions, so a path's case is the one that falls through: without the hints a hop of distances takes 0.41 us (grids two
+    // and five wide 1 % less than with them).  Labels are faster without.
+#define DRONE_LONE_EXPECT(condition, value) (Push::kTolerance ? __builtin_expect((condition), (value)) : (condition))
     // Ends with the list in LDS and all values stored.
     __device__ __forceinline__ void run_lone(int max_rounds, int &rounds, bool &pending) const
     {
@@ -942,7 +944,7 @@ struct SmallRounds {
             bool lowers = lane < m && nv < old;
             const int mark = first_mark + rounds++;
             const unsigned long long lowering = __ballot(lowers);
-            if (__builtin_expect(__popcll(lowering) > 1, 0)) {
+            if (DRONE_LONE_EXPECT(__popcll(lowering) > 1, 0)) {
                 int leader = lane;
                 bool open = lowers;
                 int *tag = s_lone->tag + (((unsigned int)t * 0x9E3779B1u) >> 24);
@@ -967,15 +969,18 @@ struct SmallRounds {
                     lanes_meet();
                 }
             }
-            const bool goes = lowers && Push::activates(old, nv);
-            if (lowers) push.store(t, nv);
-            if (goes) active[t] = mark;
-            if (__builtin_expect(__popcll(lowering) == 1 && rounds < max_rounds, 1)) {  // its edges go to the first lanes, out of registers
+            const bool goes = Push::kTolerance ? lowers && Push::activates(old, nv) : lowers;
+            if (lowers) {
+                push.store(t, nv);
+                if (!Push::kTolerance) active[t] = mark;
+            }
+            if (Push::kTolerance && goes) active[t] = mark;
+            if (DRONE_LONE_EXPECT(__popcll(lowering) == 1 && rounds < max_rounds, 1)) {  // its edges go to the first lanes, out of registers
                 const int who = __ffsll(lowering) - 1, degree = __builtin_amdgcn_readlane(goes ? f.degree : 0, who);
-                if (__builtin_expect(degree <= kWave, 1)) {
+                if (DRONE_LONE_EXPECT(degree <= kWave, 1)) {
                     count = degree > 0;
                     m = degree;
-                    if (__builtin_expect(m == 0, 0)) break;
+                    if (DRONE_LONE_EXPECT(m == 0, 0)) break;
                     e = __builtin_amdgcn_readlane(f.begin, who) + lane;
                     from = value_of_order(__builtin_amdgcn_readlane(order_of(nv), who), Value{});
                     t = -1;
@@ -1024,6 +1029,7 @@ struct SmallRounds {
             s_ends[0] = s_ends[1] = 0;
         }
     }
+#undef DRONE_LONE_EXPECT
 
     // Touches the lines of the vertices' first edges, until *stop.
     __device__ __forceinline__ void warm(int n, const int *stop) const
