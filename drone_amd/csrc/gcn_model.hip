@@ -49,7 +49,7 @@ void drone_gcn_mod::GCN::choose_truth(int current_split)
     }
     double *part = static_cast<double *>(truth_scratch);
     set_truth_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), kTruthBlocks), kSpmvBlock, 0, static_cast<hipStream_t>(s)>>>(
-        truth, split, label, current_split, n, counts_rows ? labelled : nullptr, labelled_h, part,
+        truth, split, label, current_split, n, counts_rows ? labelled : nullptr, &ce->pinned->labelled, part,
         reinterpret_cast<unsigned int *>(part + kTruthBlocks));
     DRONE_GCN_HIP(hipGetLastError());
     truth_split = current_split;
@@ -139,7 +139,7 @@ extern "C" int drone_gcn_set_truth(struct drone_gcn *h, int split)
 {
     clear_error();
     DRONE_REQUIRE(h != nullptr, "handle");
-    h->model->set_truth(split);
+    h->model->choose_truth(split);  // the handle shows nothing that set_truth() would wait for
     return DRONE_OK;
 }
 

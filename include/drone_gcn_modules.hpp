@@ -342,7 +342,13 @@ class CrossEntropyLoss : public Module {
     int num_classes;
     drone_stream_t s;
 public:
-    float *d_loss = nullptr;  // pinned scalar that the device writes: GCN::read_metrics() reads it without a copy
+    // Pinned memory that the device writes and GCN::read_metrics() reads without a copy (labelled, report: GCN's).
+    struct Pinned {
+        float loss;
+        int labelled;
+        drone_loss_report report;
+    } *pinned = nullptr;
+    float *d_loss = nullptr;  // = &pinned->loss
     int *d_count = nullptr;   // device scalar
     float grad_scale = 1.0f;  // 1 = the reference's sum-reduced gradient
     const int *mean_over = nullptr;  // device: scale the gradient by 1 / *mean_over instead
@@ -374,11 +380,12 @@ public:
         : logits(logits_), truth(truth_), num_classes(num_classes_), s(stream)
     {
         ModuleName = std::move(name);
-        DRONE_GCN_HIP(hipHostMalloc(&d_loss, sizeof(float)));
-        *d_loss = 0.0f;
+        DRONE_GCN_HIP(hipHostMalloc(&pinned, sizeof(Pinned)));
+        *pinned = Pinned{};
+        d_loss = &pinned->loss;
         DRONE_GCN_HIP(hipMalloc(&d_count, sizeof(int)));
     }
-    ~CrossEntropyLoss() override { (void)hipHostFree(d_loss); (void)hipFree(d_count); }
+    ~CrossEntropyLoss() override { (void)hipHostFree(pinned); (void)hipFree(d_count); }
     void forward(bool training) override
     {
         const drone_loss_pass p = pass(training);
@@ -492,13 +499,11 @@ public:
     float *x_padded = nullptr;   // the model's zero-padded copy of X, when it needs one
     int *truth = nullptr;   // device [N]: label on rows of the current split, -1 elsewhere
     int truth_split = -1, truth_count = 0;  // the split chosen last and, with mean_gradient, its labelled rows
-    // What a forward pass reports besides the loss, for the device and, once the stream has been waited for, for the host:
-    // pinned memory, so read_metrics() copies nothing.
-    drone_loss_report *report = nullptr;
-    float *l2_sum = nullptr;  // = &report->sum_squares: sum of W1^2 (cuda_gcn.cu:254-260)
-    int *counts = nullptr;    // = &report->correct: [2], correct and counted rows
-    int *labelled = nullptr;  // device: the labelled rows as set_truth's kernel counts them
-    int *labelled_h = nullptr;  // pinned: the same
+    // What a forward pass reports besides the loss (in ce->pinned), for the device and, once the stream has been waited for, for
+    // the host.
+    float *l2_sum = nullptr;  // sum of W1^2 (cuda_gcn.cu:254-260)
+    int *counts = nullptr;    // [2]: correct and counted rows
+    int *labelled = nullptr;  // device: the labelled rows as set_truth's kernel counts them, with mean_gradient
     bool truth_pending = false; // counted, but truth_count and ce->grad_scale do not hold it yet
     void *truth_scratch = nullptr;
     const int *label = nullptr, *split = nullptr;  // device, borrowed
@@ -558,13 +563,7 @@ public:
         const int max_dim = p.hidden_dim > p.output_dim ? p.hidden_dim : p.output_dim;
         adj.reset(new Adjacency(N, nnz, rp, ci, in_degree, out_degree, max_dim, s));
         DRONE_GCN_HIP(hipMalloc(&truth, sizeof(int) * (size_t)N));
-        DRONE_GCN_HIP(hipMalloc(&labelled, sizeof(int)));
-        DRONE_GCN_HIP(hipHostMalloc(&labelled_h, sizeof(int)));
-        DRONE_GCN_HIP(hipHostMalloc(&report, sizeof(drone_loss_report)));
-        *report = drone_loss_report{};
-        l2_sum = &report->sum_squares;
-        counts = &report->correct;
-        static_assert(offsetof(drone_loss_report, counted) == offsetof(drone_loss_report, correct) + sizeof(int), "counts[1]");
+        if (p.mean_gradient) DRONE_GCN_HIP(hipMalloc(&labelled, sizeof(int)));
         const Replicas *r = cut ? &replicas : nullptr;
 
         if (p.fold_input_aggregation) {
@@ -601,7 +600,10 @@ public:
         // weights as they are before the optimiser step - comes out of the loss's launch
         ce->skip = mirror2worker;
         ce->l2_weight = layer1_weight;
-        ce->report = report;
+        ce->report = &ce->pinned->report;
+        l2_sum = &ce->report->sum_squares;
+        counts = &ce->report->correct;
+        static_assert(offsetof(drone_loss_report, counted) == offsetof(drone_loss_report, correct) + sizeof(int), "counts[1]");
         if (p.use_adam) {
             AdamParams ap;
             ap.lr = p.learning_rate;
@@ -618,13 +620,15 @@ public:
         (void)hipFree(x_padded);
         (void)hipFree(truth);
         (void)hipFree(labelled);
-        (void)hipHostFree(labelled_h);
         (void)hipFree(truth_scratch);
-        (void)hipHostFree(report);
     }
 
-    // cuda_gcn.cu:211-223.  With mean_gradient a change of the split waits for the stream: truth_count and ce->grad_scale
-    // are the new split's when it returns (on a capturing stream they follow at the next read_metrics()).
+    // Enqueues the truth of a split (cuda_gcn.cu:211-223).  With mean_gradient a change of the split also counts its labelled rows,
+    // and until the next read_metrics() the loss takes that count from the device: no wait.
+    void choose_truth(int current_split);  // defined in gcn_model.hip (needs a kernel)
+    // The same for a program that reads what it chose.  With mean_gradient a change of the split waits for the stream:
+    // truth_count and ce->grad_scale are the new split's when it returns (on a capturing stream they follow at the next
+    // read_metrics()).
     void set_truth(int current_split)
     {
         choose_truth(current_split);
@@ -682,14 +686,11 @@ public:
     }
 
 private:
-    // Enqueues the new truth.  With mean_gradient a change of the split also counts its labelled rows, and until
-    // settle_truth() the loss takes that count from the device: train_epoch() and eval() need no wait before their own.
-    void choose_truth(int current_split);  // defined in gcn_model.hip (needs a kernel)
     void settle_truth()  // behind a wait for the stream
     {
         if (!truth_pending) return;
         truth_pending = false;
-        truth_count = *labelled_h;
+        truth_count = ce->pinned->labelled;
         ce->grad_scale = truth_count > 0 ? 1.0f / (float)truth_count : 1.0f;
         ce->mean_over = nullptr;
     }
