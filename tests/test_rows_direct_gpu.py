@@ -103,3 +103,39 @@ def test_chains_of_masters_take_the_general_path(oracle, compress):
             lib().drone_graph_destroy(w.g)
             w.g = None
         lb.close()
+
+
+def test_workers_that_disagree_about_the_rows_get_an_error():
+    """Different widths, or compressed rows on one side only: every worker gets an error instead of waiting, and the group goes on
+    working."""
+    import torch
+    from drone_amd import gcn, rmat
+    from drone_amd._lib import DroneError, lib
+    from drone_amd.pagerank import Loopback, run_workers
+    from drone_amd.traverse import _WorkerCUDA
+    n, W = 1 << 9, 3
+    u, v = rmat.clean_directed_np(*rmat.rmat_edges(9, 8 << 9, seed=5))
+    parts, _ = vertex_cut(u, v, W, 5)
+    lb = Loopback(W, timeout_ms=20000)
+    ws = [_WorkerCUDA(n, p["u"], p["v"], workerId=i, workerNum=W, routes=p, loopback=lb) for i, p in enumerate(parts)]
+    try:
+        rows = [torch.ones(w.n, 8, device="cuda") for w in ws]
+        torch.cuda.synchronize()
+
+        def sync(i, K, compress):
+            try:
+                return gcn.graphsum_sync_rows(ws[i].g, rows[i][:, :K], i, W, ws[i].comm, compress)
+            except DroneError as e:
+                return str(e)
+
+        for K, compress in (((8, 8, 7), (False,) * 3), ((8, 8, 8), (False, True, False))):
+            got = run_workers([(lambda i=i: sync(i, K[i], compress[i])) for i in range(W)])
+            assert all(isinstance(g, str) and "different exchange steps" in g for g in got)
+            assert all(bool((r == 1.0).all()) for r in rows)
+        got = run_workers([(lambda i=i: sync(i, 8, False)) for i in range(W)])
+        assert [g[1] for g in got] == [len(p["mirror_vertex"]) for p in parts]
+    finally:
+        for w in ws:
+            lib().drone_graph_destroy(w.g)
+            w.g = None
+        lb.close()
