@@ -93,6 +93,7 @@ struct GraphExt {
     RouteLists routes;
     RowSync row_sync;
     FirstEdges *first_edges = nullptr;  // device [n], at most 256 MB, or null: see ensure_first_edges in traverse.hip
+    bool one_way = false;     // labels: an edge without its reverse has been seen
     // SSSP: edge lengths in in-edge order
     int *in_eid = nullptr;    // device [edges]: position in the out-edge CSR (g->dst / g->edgeLen) of each in-edge
     float *in_len = nullptr;  // device [edges]: g->edgeLen in in-edge order, refreshed at every SSSP_PEVal

@@ -81,6 +81,7 @@ struct TraverseState {
 struct Report {
     TraverseState state;
     double visited;  // vertices with active != 0, if the list is empty
+    int again;       // labels: whether edges between trees are left
 };
 // Two lists of vertices, and where each listed vertex's out-edges start in the list's concatenated out-edges.
 struct Lists {
@@ -88,32 +89,6 @@ struct Lists {
 };
 // A list of no vertices that no round may take for its own: all of them still have to propagate.
 __host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
-
-// cc.cu:10-20 and, in place of the first round, labels from further away: a vertex follows its first in-neighbour, that one's
-// first, and so on for as long as the numbers fall and for at most kCcHops hops, and takes the number it arrives at.  It
-// arrives there against the edges' direction, so the label is one that propagation would bring; rows are in ascending order,
-// so the first in-neighbour is the least.  All vertices still have to propagate: the next round looks at every in-edge of
-// every vertex that can fall.  500,009 vertices, 11.5 M edges: 17.5 us instead of 64 for the sweep over all edges that
-// stood here, and the rounds after it start nearer: labels of the graph 241 -> 123 us.
-constexpr int kCcHops = 32;
-__global__ void cc_init_kernel(int n, const int *__restrict__ in_index, const int *__restrict__ in_src, int *__restrict__ active,
-                               int *__restrict__ cc, int *__restrict__ ubm, TraverseState *__restrict__ state)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        int label = i;
-        for (int hop = 0; hop < kCcHops && label > 0; ++hop) {
-            const int e0 = in_index[label], e1 = in_index[label + 1];
-            if (e0 == e1) break;
-            const int u = in_src[e0];
-            if (u >= label) break;
-            label = u;
-        }
-        active[i] = label < i;  // the mark of round 1, cc.cu:16
-        cc[i] = label;
-        ubm[i] = 0;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 2, 1, 0, 0.0};
-}
 
 // sssp.cu:23-38, and the list of the first round: the start vertex if this subgraph holds it (sssp.cu:30) and it has
 // out-edges.
@@ -144,6 +119,215 @@ __device__ __forceinline__ void publish_sum(double mine, double *s_red, double *
     if (!last_block_done(ticket, one)) return;
     const double all = block_sum_of_parts(block_part, (int)gridDim.x, s_red);
     if (threadIdx.x == 0) *out = all;
+}
+
+// ---- labels by joining trees -------------------------------------------------------------------------------
+// Where every edge has its reverse, a vertex's label is the least vertex of its component, and it need not travel there hop by
+// hop: the vertices are kept as trees in cc[] itself (cc[v] = v's parent, at most v; a root is its own), an edge between two
+// trees makes the larger root a child of the smaller, and at the end every vertex takes its root's number.  Along edges whose
+// reverse is missing only rounds of the kernels below can tell; what the trees hold by then is a valid start for them, since
+// trees are only ever joined along edges that lead both ways.  So no property of the graph is assumed: every edge a tree
+// is made of is looked up in the other direction.
+//   cc_begin    parent = least in-neighbour if that is smaller (rows are in ascending order: the first)
+//   cc_flatten  parent = root
+//   cc_link     joins the trees that edges lead between
+//   cc_finish   label = root, flags, and the report
+// Four launches and one wait whatever the graph's diameter: labels of 500,009 vertices and 11.5 M edges 126 -> 55 us against rounds
+// of propagation, of a path of 12,000 vertices 8.5 ms -> 49 us, of a 1,000 x 1,000 grid 18.9 ms -> 194 us, these two numbered at
+// random.  They are bound by their chains of dependent loads (row bounds, neighbour, its row, ...) and the launches.
+constexpr int kCcSamples = kWave;
+constexpr int kCcSteps = 64;  // along one edge, of one cc_link: past them it is left to the next
+struct CcTrees {
+    int directed;            // number of the last call that found an edge without its reverse
+    int again;               // number of the last pass that left an edge undone
+    int sample[kCcSamples];  // roots of vertices from all over the graph
+};
+
+// Whether the edge u -> v, entry i of v's in-row, has its reverse v -> u.  It usually is entry i of v's out-row (edge files that name
+// an edge in both directions are often sorted); short out-rows are looked through, otherwise v is searched in u's in-row.
+struct Rows {
+    const int *__restrict__ in_index;
+    const int *__restrict__ in_src;
+    const int *__restrict__ index;
+    const int *__restrict__ dst;
+
+    __device__ __forceinline__ bool leads_back(int u, int v, unsigned int i) const
+    {
+        const unsigned int d0 = index[v], d1 = index[v + 1];
+        if (d0 + i < d1 && dst[d0 + i] == u) return true;
+        if (d1 - d0 <= 8) {
+            bool found = false;
+            for (unsigned int d = d0; d < d1; d += 4)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) found |= dst[d + k < d1 ? d + k : d1 - 1] == u;
+            return found;
+        }
+        unsigned int lo = in_index[u], hi = in_index[u + 1];
+        const unsigned int end = hi;
+        while (lo < hi) {
+            const unsigned int mid = (lo + hi) >> 1;
+            if (in_src[mid] < v) lo = mid + 1; else hi = mid;
+        }
+        return lo < end && in_src[lo] == v;
+    }
+};
+// Parents only ever move to smaller numbers of the same tree, so an old one still leads to the root.
+__device__ __forceinline__ int parent_of(const int *cc, int v) { return __hip_atomic_load(cc + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+
+// cc.cu:10-20
+__global__ __launch_bounds__(kSpmvBlock) void cc_begin_kernel(int n, Rows rows, int *__restrict__ cc, int *__restrict__ ubm,
+                                                              TraverseState *__restrict__ state, CcTrees *trees, int call)
+{
+    for (int v = blockIdx.x * kSpmvBlock + threadIdx.x; v < n; v += gridDim.x * kSpmvBlock) {
+        const int e0 = rows.in_index[v], e1 = rows.in_index[v + 1];
+        int parent = v;
+        if (e0 < e1) {
+            const int u = rows.in_src[e0];
+            if (u < v) {
+                parent = u;
+                if (!rows.leads_back(u, v, 0)) trees->directed = call;
+            }
+        }
+        cc[v] = parent;
+        ubm[v] = 0;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 2, 1, 0, 0.0};
+}
+
+// The root of v, which hands on how far it has come: walkers below take it from there, so a chain of d parents takes about
+// log2(d) steps.  Where a walk is long, what the other XCDs have stored counts, so loads and stores go past the L2.
+__device__ __forceinline__ int walk_to_root(int *cc, int v)
+{
+    int p = parent_of(cc, v);
+    for (int step = 0;; ++step) {
+        const bool far = step >= 8;
+        const int up = far ? __hip_atomic_load(cc + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : parent_of(cc, p);
+        if (up == p) return p;
+        p = up;
+        if (far) __hip_atomic_store(cc + v, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else __hip_atomic_store(cc + v, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+
+__host__ __device__ __forceinline__ int sample_stride(int n) { return n / kCcSamples > 0 ? n / kCcSamples : 1; }
+
+__global__ __launch_bounds__(kSpmvBlock) void cc_flatten_kernel(int n, int *cc, CcTrees *trees)
+{
+    const int stride = sample_stride(n);
+    for (int v = blockIdx.x * kSpmvBlock + threadIdx.x; v < n; v += gridDim.x * kSpmvBlock) {
+        const int root = walk_to_root(cc, v);
+        if (v % stride == 0 && v / stride < kCcSamples) trees->sample[v / stride] = root;
+    }
+}
+
+// Joins the trees of a and b.  The larger of the two goes up its tree until it is the other one or a root, which becomes a child of
+// the other: each step lowers the larger, so it ends; whether a is still a root is for the compare-and-swap at the memory
+// side to say.
+__device__ __forceinline__ bool join_trees(int *cc, int a, int b)
+{
+    for (int step = 0; step < kCcSteps; ++step) {
+        if (a == b) return true;
+        const int high = a > b ? a : b, low = a > b ? b : a;
+        int up = parent_of(cc, high);
+        if (up == high) {
+            up = atomicCAS(cc + high, high, low);
+            if (up == high) return true;
+        }
+        a = up;
+        b = low;
+    }
+    return false;
+}
+
+// Rows are dealt out by length, as in pull_open_kernel.  Vertices of the tree that most samples lie in - after cc_begin usually
+// most of a component with hubs - are left out: an edge to one of the other trees is looked at from there.
+constexpr int kLinkThreads = 256, kLinkBlocks = 2048;
+constexpr int kLinkLane = 8, kLinkWave = 2048;  // entries up to which a row gets a lane, a wavefront
+__global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows, int *cc, CcTrees *trees, int call, int pass)
+{
+    constexpr int kWaves = kLinkThreads / kWave;
+    __shared__ int s_wave[kLinkThreads], s_block[kLinkThreads];
+    __shared__ int s_waves, s_blocks;
+    if (trees->directed == call) return;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int stride = sample_stride(n), samples = (n - 1) / stride + 1 < kCcSamples ? (n - 1) / stride + 1 : kCcSamples;
+    const int mine = lane < samples ? trees->sample[lane] : -1;
+    int left_out = -1, most = 0;
+    for (int k = 0; k < samples; ++k) {
+        const int root = __builtin_amdgcn_readlane(mine, k), count = __popcll(__ballot(mine == root));
+        if (count > most) {
+            most = count;
+            left_out = root;
+        }
+    }
+    const auto edge = [&](int v, unsigned int i, int a, int u, int b) {  // entry i of v's row; roots a, b
+        if (a == b) return;
+        if (!rows.leads_back(u, v, i)) trees->directed = call;
+        else if (!join_trees(cc, a, b)) trees->again = pass;
+    };
+    const auto walk = [&](int row, int first, int lanes) {
+        const unsigned int e0 = rows.in_index[row], e1 = rows.in_index[row + 1];
+        const int a = parent_of(cc, row);
+        for (unsigned int e = e0 + first; e < e1; e += 2 * lanes) {
+            const bool two = e + lanes < e1;
+            const int u0 = rows.in_src[e], u1 = rows.in_src[two ? e + lanes : e];
+            const int b0 = parent_of(cc, u0), b1 = parent_of(cc, u1);
+            edge(row, e - e0, a, u0, b0);
+            if (two) edge(row, e + lanes - e0, a, u1, b1);
+        }
+    };
+    const int64_t pieces = ((int64_t)n + kWave - 1) / kWave, per_pass = (int64_t)kWaves * gridDim.x;
+    for (int64_t at = 0; at < pieces; at += per_pass) {
+        if (tid == 0) s_waves = s_blocks = 0;
+        __syncthreads();
+        const int64_t r64 = (at + (int64_t)wave * gridDim.x + blockIdx.x) * kWave + lane;
+        if (r64 < n) {
+            const int r = (int)r64;
+            const int a = parent_of(cc, r);
+            if (a != left_out) {
+                const unsigned int e0 = rows.in_index[r], e1 = rows.in_index[r + 1];
+                if (e1 - e0 <= kLinkLane) {
+                    for (unsigned int e = e0; e < e1; e += 4) {
+                        int u[4], b[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) u[k] = rows.in_src[e + k < e1 ? e + k : e1 - 1];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) b[k] = parent_of(cc, u[k]);
+                        for (int k = 0; k < 4; ++k)
+                            if (e + k < e1) edge(r, e + k - e0, a, u[k], b[k]);
+                    }
+                } else if (e1 - e0 <= kLinkWave) {
+                    s_wave[atomicAdd(&s_waves, 1)] = r;
+                } else {
+                    s_block[atomicAdd(&s_blocks, 1)] = r;
+                }
+            }
+        }
+        __syncthreads();
+        const int waves = s_waves, blocks = s_blocks;
+        for (int i = wave; i < waves; i += kWaves) walk(s_wave[i], lane, kWave);
+        for (int i = 0; i < blocks; ++i) walk(s_block[i], tid, kLinkThreads);
+        __syncthreads();  // the lists have been read
+    }
+}
+
+// Labels, cc.cu:16's flags (lowered or not; common.cu:17-31 counts the lowered) and where that leaves the traversal: at its end,
+// or with everything still to propagate.
+__global__ __launch_bounds__(kSpmvBlock) void cc_finish_kernel(int n, int *cc, int *__restrict__ active, const CcTrees *trees, int call, int pass,
+                                                               double *block_part, unsigned int *ticket, Report *report)
+{
+    __shared__ double s_red[kSpmvBlock / kWave];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        report->state = TraverseState{trees->directed == call ? everything() : 0ull, 2, 1, 0, 0.0};
+        report->again = trees->again == pass;
+    }
+    double lowered = 0.0;
+    for (int v = blockIdx.x * kSpmvBlock + threadIdx.x; v < n; v += gridDim.x * kSpmvBlock) {
+        const bool falls = walk_to_root(cc, v) < v;
+        active[v] = falls;
+        lowered += falls;
+    }
+    publish_sum(lowered, s_red, block_part, ticket, &report->visited);
 }
 
 // cc.cu:391-404 / sssp.cu:483-496
@@ -212,6 +396,8 @@ struct TraverseExt {
     unsigned long long *counters = nullptr; // device: vertices << 32 | out-edges of the list being built; zero between launches
     unsigned int *ticket = nullptr;         // device [ticket_words(kListBlocks)]: counters of last_block_done, zero between launches
     TraverseState *state = nullptr;         // device
+    CcTrees *trees = nullptr;               // device
+    int call = 0, pass = 0;                 // of the tree kernels, counted: what *trees names them by
     Report *report = nullptr;               // pinned
 };
 
@@ -244,6 +430,8 @@ TraverseExt *traverse_ext_create(int n)
     DRONE_HIP_OR_DIE(hipMalloc(&t->counters, sizeof(unsigned long long)));
     DRONE_HIP_OR_DIE(hipMemset(t->counters, 0, sizeof(unsigned long long)));
     DRONE_HIP_OR_DIE(hipMalloc(&t->state, sizeof(TraverseState)));
+    DRONE_HIP_OR_DIE(hipMalloc(&t->trees, sizeof(CcTrees)));
+    DRONE_HIP_OR_DIE(hipMemset(t->trees, 0, sizeof(CcTrees)));
     DRONE_HIP_OR_DIE(hipMalloc(&t->ticket, sizeof(unsigned int) * ticket_words(kListBlocks)));
     DRONE_HIP_OR_DIE(hipMemset(t->ticket, 0, sizeof(unsigned int) * ticket_words(kListBlocks)));
     DRONE_HIP_OR_DIE(hipStreamSynchronize(nullptr));  // the kernels that count may run on any stream
@@ -262,6 +450,7 @@ void traverse_ext_destroy(void *ext)
     (void)hipFree(t->counters);
     (void)hipFree(t->ticket);
     (void)hipFree(t->state);
+    (void)hipFree(t->trees);
     (void)hipHostFree(t->report);
     delete t;
 }
@@ -1176,7 +1365,7 @@ void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
 // usually follow each other - a list grows past what one work-group takes, then past what is worth pushing, and shrinks
 // again - and only then waits.  Breadth-first distances over 1 M vertices and 11.5 M edges: 550 us with a wait per round and sweeps
 // over all edges, 269 with the kernels here and a wait per round, 128 with the rounds enqueued together; labels of
-// 500,009 vertices 880, 440, 244 (123 since their first round follows chains, see cc_init_kernel).
+// 500,009 vertices 880, 440, 244 (where every edge has its reverse, labels need no rounds: see cc_begin_kernel).
 template <typename Run>
 int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bool known, hipStream_t s)
 {
@@ -1286,6 +1475,31 @@ struct CcRun {
     void pull() { launch_pull(g, t, CcPull{cc}, s); }
 };
 
+// Trees from the least in-neighbours, joined until no edge leads between two of them, or left to the rounds: returns where that
+// leaves the traversal.  A pass that gives up on an edge has flattened what was in its way, so the next gets further.  A graph that
+// has shown an edge without its reverse is not tried again: it starts from the trees of the least in-neighbours.
+TraverseState join_labels(Graph *g, TraverseExt *t, int *cc, hipStream_t s)
+{
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
+    const int n = x->n, call = ++t->call;
+    const Rows rows{x->in_index, x->in_src, g->index, g->dst};
+    const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), 4096);
+    cc_begin_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, g->updateByMessage, t->state, t->trees, call);
+    for (;;) {
+        const int pass = ++t->pass;
+        cc_flatten_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, cc, t->trees);
+        if (!x->one_way)
+            cc_link_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kLinkThreads), kLinkBlocks), kLinkThreads, 0, s>>>(
+                n, rows, cc, t->trees, call, pass);
+        cc_finish_kernel<<<sum_blocks(n, 1), kSpmvBlock, 0, s>>>(n, cc, g->active, t->trees, call, pass, t->block_part, t->ticket, t->report);
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        if (x->one_way) return TraverseState{everything(), 2, 1, 0, 0.0};
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+        x->one_way = t->report->state.listed != 0;
+        if (x->one_way || !t->report->again) return t->report->state;
+    }
+}
+
 // levels: the rounds start from one vertex, so over unit lengths round k reaches the vertices at distance k.  Whether all
 // lengths are 1.0 (as build_graph leaves them) is counted on the device, at the start of such a call and otherwise when a
 // sweep first needs to know it, as are the lengths in in-edge order, whose random gather costs more than a whole sweep.
@@ -1393,17 +1607,20 @@ extern "C" Response CC_PEVal(Graph *g, CCValues *values, int workerId, int worke
     hipStream_t s = comm ? static_cast<hipStream_t>(comm->s) : nullptr;
     Response res = {};
     const int n = getLocalVertexSize(g);
-    ensure_first_edges(g, s);
     ensure_flags(g);
     if (!values->ext) {  // cc.cu:349-351: the state is allocated by this call
         DRONE_HIP_OR_DIE(hipMalloc(&values->ccValue, sizeof(int) * (size_t)(n > 0 ? n : 1)));
         values->ext = traverse_ext_create(n);
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    const GraphExt *x = static_cast<const GraphExt *>(g->ext);
-    cc_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, x->in_index, x->in_src, g->active, values->ccValue, g->updateByMessage, t->state);
-    CcRun run{g, t, values->ccValue, s};
-    if (n > 0) run_to_fixed_point(g, t, run, TraverseState{everything(), 2, 1, 0, 0.0}, true, s);
+    if (n > 0) {
+        const TraverseState now = join_labels(g, t, values->ccValue, s);
+        CcRun run{g, t, values->ccValue, s};
+        if (now.listed != 0) {
+            ensure_first_edges(g, s);
+            run_to_fixed_point(g, t, run, now, true, s);
+        }
+    }
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1427,6 +1644,7 @@ extern "C" Response CC_IncEVal(Graph *g, CCValues *values, int workerId, int wor
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
     const int n = getLocalVertexSize(g);
+    ensure_first_edges(g, s);
     process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
     launch_collect(g, t, 0, 1, 0, s);  // cc.cu:425: the vertices a message activated propagate
     CcRun run{g, t, values->ccValue, s};

@@ -1,0 +1,107 @@
+"""CC_PEVal where labels come from joining trees: graphs whose edges all have their reverse, with rows on both sides of every
+length at which they are dealt out differently, long chains, many components, and graphs in which one edge has no reverse.
+Labels are whole numbers: exact."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(u, v):
+    return np.concatenate([u, v]), np.concatenate([v, u])
+
+
+def _named(u, v, seed):
+    """Random names, edges in random order."""
+    rng = np.random.default_rng(seed)
+    perm, order = rng.permutation(int(max(u.max(), v.max())) + 1), rng.permutation(len(u))
+    return perm[u][order].astype(np.int32), perm[v][order].astype(np.int32)
+
+
+def _grid(w, h):
+    at = np.arange(w * h).reshape(h, w)
+    return _both(np.concatenate([at[:-1].ravel(), at[:, :-1].ravel()]), np.concatenate([at[1:].ravel(), at[:, 1:].ravel()]))
+
+
+def _path(n):
+    return _both(np.arange(n - 1), np.arange(1, n))
+
+
+def _stars(degrees):
+    """Stars of the given numbers of leaves, the centres chained through their last leaves."""
+    u, v, at = [], [], 0
+    for d in degrees:
+        u += [at] * d
+        v += range(at + 1, at + d + 1)
+        if at + d + 1 < sum(degrees) + len(degrees):
+            u.append(at + d)
+            v.append(at + d + 1)
+        at += d + 1
+    return _both(np.array(u), np.array(v))
+
+
+def _blocks(sizes, seed):
+    """Components of the given sizes: a random tree and as many edges more, some of them twice and from a vertex to itself."""
+    rng = np.random.default_rng(seed)
+    u, v, base = [], [], 0
+    for k in sizes:
+        child = np.arange(1, k)
+        more = rng.integers(0, k, (2, k))
+        u += [base + child, base + more[0], base + more[0][:3]]
+        v += [base + (rng.random(k - 1) * child).astype(np.int64), base + more[1], base + more[1][:3]]
+        base += k
+    return _both(np.concatenate(u), np.concatenate(v))
+
+
+CASES = {
+    "pair": lambda: _both(np.array([0]), np.array([1])),
+    "samples": lambda: _path(65),
+    "path_in_order": lambda: tuple(x.astype(np.int32) for x in _path(70_001)),
+    "path": lambda: _named(*_path(30_011), 1),
+    "grid": lambda: _named(*_grid(211, 97), 2),
+    "rows": lambda: _named(*_stars([1, 7, 8, 9, 63, 64, 65, 255, 257, 511, 2047, 2048, 2049, 9000]), 3),
+    "components": lambda: _named(*_blocks([2] * 300 + [3, 17, 1000, 40_000] * 3, 4), 5),
+    "one_by_one": lambda: _named(*_blocks([2] * 40_000, 6), 7),
+    # falling and rising turns: roots that are joined to one another in a long row
+    "comb": lambda: _both(np.concatenate([np.arange(0, 20_000), np.arange(1, 20_000)]),
+                          np.concatenate([40_000 + np.arange(0, 20_000), 40_000 + np.arange(0, 19_999)])),
+}
+
+
+def _labels(n, index, dst):
+    src = np.repeat(np.arange(n), np.diff(index))
+    cc = np.arange(n)
+    while True:  # least label over in-edges, and the label of that label
+        new = cc.copy()
+        np.minimum.at(new, dst, cc[src])
+        new = np.minimum(new, new[new])
+        if np.array_equal(new, cc):
+            return cc
+        cc = new
+
+
+@pytest.mark.parametrize("without_reverse", [0, 1, 2])
+@pytest.mark.parametrize("name", CASES)
+def test_labels_by_trees(oracle, name, without_reverse):
+    from drone_amd.traverse import CCWorkerCUDA
+    u, v = (np.asarray(x, np.int32) for x in CASES[name]())
+    if without_reverse == 1:  # one edge leads one way
+        u, v = u[:-1], v[:-1]
+    elif without_reverse == 2:  # many do
+        keep = np.random.default_rng(8).random(len(u)) < 0.9
+        keep[0] = True
+        u, v = u[keep], v[keep]
+    nglobal = int(max(u.max(), v.max())) + 1
+    n, _, _, index, dst = oracle.build_graph(nglobal, u, v)
+    want = _labels(n, index, dst)
+    w = CCWorkerCUDA(nglobal, u, v)
+    try:
+        for _ in range(3):
+            res = w.peval()
+            np.testing.assert_array_equal(w.read(), want)
+            flags = w.flags()
+            np.testing.assert_array_equal(flags["active"] > 0, want < np.arange(n))
+            assert not flags["updateByMessage"].any()
+            assert res.VisitedSize == np.count_nonzero(want < np.arange(n))
+    finally:
+        w.close()
