@@ -71,6 +71,18 @@ struct alignas(32) FirstEdges {
     int begin, degree, dst[kFirstEdges], pad[2];
 };
 
+// Shortest paths on graphs that are mostly chains: see traverse_chains.h.
+struct Chains {
+    bool tried = false, ready = false;
+    bool other_lengths = false;    // the last call found lengths other than 1.0
+    int64_t most = 0;              // edges a list can have: those of all ends
+    DeviceArena arena;             // of the arrays below
+    int2 *arc = nullptr;           // device [2 n]
+    int *dst = nullptr;            // device [edges]
+    float *len = nullptr;          // device [edges]
+    FirstEdges *first = nullptr;   // device [n]
+};
+
 struct GraphExt {
     int n = 0;
     int edges = 0;
@@ -93,6 +105,7 @@ struct GraphExt {
     RouteLists routes;
     RowSync row_sync;
     FirstEdges *first_edges = nullptr;  // device [n], at most 256 MB, or null: see ensure_first_edges in traverse.hip
+    Chains chains;
     bool one_way = false;     // labels: an edge without its reverse has been seen
     // SSSP: edge lengths in in-edge order
     int *in_eid = nullptr;    // device [edges]: position in the out-edge CSR (g->dst / g->edgeLen) of each in-edge

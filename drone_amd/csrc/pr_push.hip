@@ -319,6 +319,7 @@ void drone::graph_ext_release(GraphExt *x)
     row_sync_release(&x->row_sync);
     direct_rows_release(&x->row_sync.direct);
     if (x->first_edges) (void)hipFree(x->first_edges);
+    x->chains.arena.release();
     if (x->in_eid) (void)hipFree(x->in_eid);
     if (x->in_len) (void)hipFree(x->in_len);
     *x = GraphExt{};

@@ -330,6 +330,12 @@ __global__ __launch_bounds__(kSpmvBlock) void cc_finish_kernel(int n, int *cc, i
     publish_sum(lowered, s_red, block_part, ticket, &report->visited);
 }
 
+}  // namespace
+
+#include "traverse_chains.h"
+
+namespace {
+
 // cc.cu:391-404 / sssp.cu:483-496
 __global__ __launch_bounds__(kSpmvBlock) void process_messages_kernel(int n, int *__restrict__ active, int *__restrict__ ubm)
 {
@@ -1475,6 +1481,12 @@ struct CcRun {
     void pull() { launch_pull(g, t, CcPull{cc}, s); }
 };
 
+Rows rows_of(const Graph *g)
+{
+    const GraphExt *x = static_cast<const GraphExt *>(g->ext);
+    return Rows{x->in_index, x->in_src, g->index, g->dst};
+}
+
 // Trees from the least in-neighbours, joined until no edge leads between two of them, or left to the rounds: returns where that
 // leaves the traversal.  A pass that gives up on an edge has flattened what was in its way, so the next gets further.  A graph that
 // has shown an edge without its reverse is not tried again: it starts from the trees of the least in-neighbours.
@@ -1482,7 +1494,7 @@ TraverseState join_labels(Graph *g, TraverseExt *t, int *cc, hipStream_t s)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
     const int n = x->n, call = ++t->call;
-    const Rows rows{x->in_index, x->in_src, g->index, g->dst};
+    const Rows rows = rows_of(g);
     const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), 4096);
     cc_begin_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, g->updateByMessage, t->state, t->trees, call);
     for (;;) {
@@ -1534,6 +1546,7 @@ struct SsspRun {
     void sweep(int mark)
     {
         GraphExt *x = static_cast<GraphExt *>(g->ext);
+        ensure_aggregation_ready(g);
         if (unit_lengths()) {
             spmv_merge_launch<MinF32, int, kIpt>(x->mt, x->ms, x->in_index, x->in_src, SsspUnitEpi{{dist, nullptr, g->active, mark}},
                                                  t->stat, s);
@@ -1587,6 +1600,70 @@ void ensure_first_edges(Graph *g, hipStream_t s)
         return;
     }
     first_edges_kernel<<<(unsigned)std::min<int64_t>(ceil_div(x->n, 256), 2048), 256, 0, s>>>(x->n, g->index, g->dst, x->first_edges);
+}
+
+// The chains of a graph, if nearly all its vertices lie in some: distances over them are weighted, and a graph of ends that is not
+// much smaller than the graph takes as many rounds as the graph.  A vertex that is not inner for each kChainsPer that
+// are leaves at most 3 edges per vertex where it has few, which keeps denser graphs from being looked at at all; chains shorter
+// than kChainsLeast hops cost less than looking for them.
+constexpr int kChainsPer = 8, kChainsLeast = 256, kChainsEdgesPer = 3;
+bool ensure_chains(Graph *g, TraverseExt *t, hipStream_t s)
+{
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
+    Chains &c = x->chains;
+    if (c.tried) return c.ready;
+    c.tried = true;
+    const int n = x->n;
+    if (n < kChainsLeast || (int64_t)x->edges > (int64_t)kChainsEdgesPer * n || (int64_t)sizeof(FirstEdges) * n > kFirstEdgesMost) return false;
+    const Rows rows = rows_of(g);
+    count_inner_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, rows, t->block_part, t->ticket, &t->report->visited);
+    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+    const int64_t inner = (int64_t)t->report->visited;
+    if ((n - inner) * kChainsPer > n) return false;
+    c.most = x->edges - 2 * inner;  // (in a ring, which nothing else reaches, lists have up to two vertices)
+    c.arena.want(&c.arc, 2 * (size_t)n);
+    c.arena.want(&c.dst, (size_t)x->edges);
+    c.arena.want(&c.len, (size_t)x->edges);
+    c.arena.want(&c.first, (size_t)n);
+    if (c.arena.commit() != hipSuccess) {
+        (void)hipGetLastError();
+        c.arena.release();
+        return false;
+    }
+    const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(n, kSpmvBlock), 4096);
+    chain_arcs_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, c.arc);
+    for (int64_t reach = 1; reach < n; reach *= kChainJumps + 1) chain_jump_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, c.arc);
+    chain_edges_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, c.arc, c.dst, c.len, c.first);
+    DRONE_HIP_OR_DIE(hipGetLastError());
+    return c.ready = true;
+}
+
+// Rounds over the ends of the chains until nothing changes, and the inner vertices' distances; false if the lengths are not all 1.0,
+// with nothing done.  sssp_init_kernel and count_not_one_kernel have been launched.
+bool run_chains(Graph *g, TraverseExt *t, float *dist, int start_id, hipStream_t s)
+{
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
+    Chains &c = x->chains;
+    const int n = x->n;
+    const Rows rows = rows_of(g);
+    const SsspPush push{dist, c.len};
+    const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div(c.most, kPushThreads), kPushBlocks);
+    const bool long_lists = c.most > kSmallEdges;
+    chain_start_kernel<<<1, kWave, 0, s>>>(rows, g->Global2Local, start_id, c.arc, g->active, dist, t->lists.vertex[0], t->lists.offset[0], t->state);
+    const auto small = [&] { push_rounds_small_kernel<SsspPush><<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, c.dst, c.first, push, g->active, n); };
+    do {
+        small();
+        for (int k = 0; k < 3 && long_lists; ++k)
+            push_round_kernel<SsspPush><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, (unsigned long long)c.most, t->lists, g->index,
+                                                                      c.dst, push, g->active, t->counters, t->ticket);
+        if (long_lists) small();
+        chain_fill_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, rows, g->Global2Local, start_id, c.arc, g->active, dist, t->state, t->block_part,
+                                                              t->ticket, t->report);
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
+        c.other_lengths = t->report->state.not_one != 0.0;
+    } while (!c.other_lengths && t->report->state.listed != 0);
+    return !c.other_lengths;
 }
 
 void ensure_flags(Graph *g)
@@ -1685,19 +1762,27 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
         set_error(DRONE_ERR_INVALID, "SSSP_PEVal: startId %d is outside [0, %d)", startId, nglobal);
         die("SSSP_PEVal");
     }
-    ensure_aggregation_ready(g);
-    ensure_first_edges(g, s);
     ensure_flags(g);
     if (!values->ext) {  // sssp.cu:408-411
         DRONE_HIP_OR_DIE(hipMalloc(&values->distance, sizeof(float) * (size_t)(n > 0 ? n : 1)));
         values->ext = traverse_ext_create(n);
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
-    sssp_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage,
-                                                     g->index, t->lists.vertex[0], t->lists.offset[0], t->state);
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
     SsspRun run{g, t, values->distance, s, true};
-    run.count_lengths();
-    report_rounds(run_to_fixed_point(g, t, run, TraverseState{}, false, s), "SSSP_PEVal");
+    const auto begin = [&] {
+        sssp_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage,
+                                                         g->index, t->lists.vertex[0], t->lists.offset[0], t->state);
+        run.count_lengths();
+    };
+    const bool chains = ensure_chains(g, t, s) && !x->chains.other_lengths;
+    begin();
+    if (!chains || !run_chains(g, t, values->distance, startId, s)) {
+        if (chains) begin();
+        ensure_first_edges(g, s);
+        report_rounds(run_to_fixed_point(g, t, run, TraverseState{}, false, s), "SSSP_PEVal");
+        x->chains.other_lengths = t->report->state.not_one != 0.0;
+    }
     res.LocalVertexSize = n;
     res.CalTime = (float)seconds_since(t0);
     const auto t1 = std::chrono::steady_clock::now();
@@ -1721,6 +1806,7 @@ extern "C" Response SSSP_IncEVal(Graph *g, SSSPValues *values, int workerId, int
     }
     TraverseExt *t = static_cast<TraverseExt *>(values->ext);
     const int n = getLocalVertexSize(g);
+    ensure_first_edges(g, s);
     process_messages_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, g->active, g->updateByMessage);
     launch_collect(g, t, 0, 1, 0, s);
     SsspRun run{g, t, values->distance, s, false};
