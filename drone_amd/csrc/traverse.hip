@@ -67,6 +67,8 @@ struct SsspUnitEpi : SsspEpi {
     __device__ __forceinline__ MinF32 load(int c, int64_t) const { return MinF32{dist[c] + 1.0f}; }
 };
 
+constexpr double kNotWhole = (double)(1ll << 32);
+
 // Where a traversal stands.  Its launches hand it on in device memory, so that several rounds can be enqueued before the host
 // has to know how the first of them went: every kernel that runs rounds looks at `listed` and leaves lists that are not for
 // it alone.
@@ -75,7 +77,9 @@ struct TraverseState {
     int mark;                   // of the next round, cc.cu:37 `active[v] = step + 1`: positive, and different in every round
     int rounds;                 // rounds completed
     int which;                  // which of the two list buffers holds the list
-    double not_one;             // lengths other than 1.0
+    double not_one;             // lengths other than 1.0, and kNotWhole for each that is no whole number
+    // All lengths are whole numbers, some not 1.0: every improvement is past the tolerance.
+    __host__ __device__ bool other_whole() const { return not_one > 0.0 && not_one < kNotWhole; }
 };
 // Pinned memory; `state` is as the last launch before the wait left it.
 struct Report {
@@ -367,20 +371,21 @@ __global__ void iota_kernel(int *out, int n)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = i;
 }
 
-// *out = lengths other than 1.0 (len is 16-byte aligned).
+// *out = lengths other than 1.0, and kNotWhole for each that is no whole number (len is 16-byte aligned).
 __global__ __launch_bounds__(kSpmvBlock) void count_not_one_kernel(int n, const float *__restrict__ len, double *block_part,
                                                                    unsigned int *ticket, double *out)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
     double cnt = 0.0;
+    const auto other = [](float v) { return v == 1.0f ? 0.0 : v == rintf(v) && fabsf(v) < 0x1p24f ? 1.0 : 1.0 + kNotWhole; };
     const float4 *len4 = reinterpret_cast<const float4 *>(len);
     const int quads = n / 4;
 #pragma unroll 4
     for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += gridDim.x * kSpmvBlock) {
         const float4 v = len4[i];
-        cnt += (double)((v.x != 1.0f) + (v.y != 1.0f) + (v.z != 1.0f) + (v.w != 1.0f));
+        if (v.x != 1.0f || v.y != 1.0f || v.z != 1.0f || v.w != 1.0f) cnt += (other(v.x) + other(v.y)) + (other(v.z) + other(v.w));
     }
-    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) cnt += len[4 * quads + threadIdx.x] != 1.0f;
+    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) cnt += other(len[4 * quads + threadIdx.x]);
     publish_sum(cnt, s_red, block_part, ticket, out);
 }
 
@@ -616,7 +621,8 @@ __global__ __launch_bounds__(kSpmvBlock) void collect_frontier_kernel(int n, con
 // a value that is not above the new one there never will be (values only fall), whatever the load's age, so only real
 // improvements pay for atomics, which are carried out at the memory side.  A target lowered in this round is appended to
 // `next` once: its active flag is swapped to this round's mark, and only the lane that changes it appends.
-// Lists of at most `above` edges are push_rounds_small_kernel's, of more than `limit` a sweep's: left alone.
+// Lists of at most `above` edges are push_rounds_small_kernel's, of more than `limit` (over whole lengths other than 1.0
+// limit_whole) a sweep's: left alone.
 // (One wavefront per vertex and 1,024-edge piece, pieces along grid.y, launched 400,000 work-groups for a list of 50,000
 // vertices with one hub of 39,000 edges: 70 us per round on the 11.5 M-edge graph, 9 us this way.)
 constexpr int kPushThreads = 256;
@@ -722,7 +728,7 @@ __device__ __forceinline__ void push_chunks(PushShared<typename Push::Value, PER
 
 template <typename Push>
 __global__ __launch_bounds__(kPushThreads) void push_round_kernel(TraverseState *state, unsigned long long above, unsigned long long limit,
-                                                                  Lists lists, const int *__restrict__ index,
+                                                                  unsigned long long limit_whole, Lists lists, const int *__restrict__ index,
                                                                   const int *__restrict__ dst, Push push, int *__restrict__ active,
                                                                   unsigned long long *counters, unsigned int *ticket)
 {
@@ -733,7 +739,7 @@ __global__ __launch_bounds__(kPushThreads) void push_round_kernel(TraverseState 
     } s_push;
     const TraverseState now = *state;
     const unsigned long long edges = now.listed & 0xFFFFFFFFull;
-    if (edges <= above || edges > limit) return;
+    if (edges <= above || edges > (now.other_whole() ? limit_whole : limit)) return;
     const int count = (int)(now.listed >> 32), w = now.which & 1;
     if (edges >= (unsigned long long)kPushWideEdges)
         push_chunks<Push, 8>(s_push.wide, count, (int)edges, now.mark, lists.vertex[w], lists.offset[w], index, dst, push, active,
@@ -1341,6 +1347,12 @@ void allow_small_lds()
 // the list's out-edges and two atomics per vertex it lowers, a sweep up to all edges but nothing per vertex.
 constexpr unsigned kPullShare = 16;
 unsigned long long push_limit(const GraphExt *x) { return std::max((unsigned long long)x->edges / kPullShare, (unsigned long long)kSmallEdges); }
+// Over whole lengths other than 1.0, where there are no sweeps over the open vertices, a small graph's lists are all pushed: a sweep
+// over all edges is two launches, and a third collects what it lowered.  10,000 vertices, 70,000 edges 200 -> 134 us, a 40 x 1,000
+// grid 16.5 -> 13.2 ms; 100,000 vertices, 1.3 M edges 204 -> 228 us, where a list of most edges costs more in atomics.  (Over other
+// lengths a sweep takes improvements along that a push leaves, so there what was swept stays swept.)
+constexpr unsigned long long kPushAll = 1ull << 19;
+unsigned long long push_limit_whole(const GraphExt *x) { return (unsigned long long)x->edges <= kPushAll ? kPushAll : push_limit(x); }
 
 // List 0 <- the vertices with active == value.
 void launch_collect(Graph *g, TraverseExt *t, int value, int next_mark, int rounds, hipStream_t s)
@@ -1378,24 +1390,26 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bo
     using Push = decltype(run.push);
     GraphExt *x = static_cast<GraphExt *>(g->ext);
     const int n = x->n;
-    const unsigned long long limit = push_limit(x);
+    const unsigned long long limit = push_limit(x), limit_whole = push_limit_whole(x);
+    const auto now_limit = [&] { return now.other_whole() ? limit_whole : limit; };
     const auto small = [&] {
         push_rounds_small_kernel<Push><<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, g->dst, x->first_edges, run.push,
                                                                             g->active, n);
     };
     const auto push = [&](int times) {  // there are such lists at all if limit > kSmallEdges
-        const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div((int64_t)limit, kPushThreads), kPushBlocks);
-        for (int i = 0; i < times && limit > (unsigned long long)kSmallEdges; ++i)
-            push_round_kernel<Push><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, limit, t->lists, g->index, g->dst, run.push,
+        const unsigned long long most = std::min(now_limit(), (unsigned long long)x->edges);
+        const unsigned blocks = (unsigned)std::min<int64_t>(ceil_div((int64_t)most, kPushThreads), kPushBlocks);
+        for (int i = 0; i < times && most > (unsigned long long)kSmallEdges; ++i)
+            push_round_kernel<Push><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, limit, limit_whole, t->lists, g->index, g->dst, run.push,
                                                                   g->active, t->counters, t->ticket);
     };
-    int sweeps = 1;  // per wait: doubles while nothing else is to be done
+    int sweeps = 1, pushes = 3;  // per wait: double while nothing else is to be done
     const auto pull_maybe = [&](int times) {
         for (int i = 0; i < times && run.speculates(now) && (unsigned long long)x->edges > limit; ++i) run.pull();
     };
     for (;;) {
         const unsigned long long edges = now.listed & 0xFFFFFFFFull;
-        int sweeps_next = 1;
+        int sweeps_next = 1, pushes_next = 3;
         const auto can_pull = [&] {
             if constexpr (Run::kSweeps) return run.can_pull(now);
             else return true;
@@ -1406,9 +1420,10 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bo
             pull_maybe(2);
             push(2);
             small();
-        } else if (edges <= limit) {
-            push(3);
+        } else if (edges <= now_limit()) {
+            push(pushes);
             small();
+            pushes_next = std::min(2 * pushes, 24);
         } else if (can_pull()) {
             run.pull();
             pull_maybe(1);
@@ -1422,6 +1437,7 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bo
             sweeps_next = std::min(2 * sweeps, 8);
         }
         sweeps = sweeps_next;
+        pushes = pushes_next;
         launch_report(g, t, false, s);
         DRONE_HIP_OR_DIE(hipGetLastError());
         DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
@@ -1654,7 +1670,7 @@ bool run_chains(Graph *g, TraverseExt *t, float *dist, int start_id, hipStream_t
     do {
         small();
         for (int k = 0; k < 3 && long_lists; ++k)
-            push_round_kernel<SsspPush><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, (unsigned long long)c.most, t->lists, g->index,
+            push_round_kernel<SsspPush><<<blocks, kPushThreads, 0, s>>>(t->state, kSmallEdges, (unsigned long long)c.most, (unsigned long long)c.most, t->lists, g->index,
                                                                       c.dst, push, g->active, t->counters, t->ticket);
         if (long_lists) small();
         chain_fill_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, rows, g->Global2Local, start_id, c.arc, g->active, dist, t->state, t->block_part,
