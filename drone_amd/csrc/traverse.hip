@@ -166,13 +166,21 @@ struct Rows {
                 for (int k = 0; k < 4; ++k) found |= dst[d + k < d1 ? d + k : d1 - 1] == u;
             return found;
         }
-        unsigned int lo = in_index[u], hi = in_index[u + 1];
+        return in_row(v, in_index[u], in_index[u + 1]);
+    }
+    // The same for the edge v -> u, entry i of v's out-row, of a v whose in-row is at [e0, e1).
+    __device__ __forceinline__ bool comes_back(int u, unsigned int i, unsigned int e0, unsigned int e1) const
+    {
+        return (e0 + i < e1 && in_src[e0 + i] == u) || in_row(u, e0, e1);
+    }
+    __device__ __forceinline__ bool in_row(int u, unsigned int lo, unsigned int hi) const
+    {
         const unsigned int end = hi;
         while (lo < hi) {
             const unsigned int mid = (lo + hi) >> 1;
-            if (in_src[mid] < v) lo = mid + 1; else hi = mid;
+            if (in_src[mid] < u) lo = mid + 1; else hi = mid;
         }
-        return lo < end && in_src[lo] == v;
+        return lo < end && in_src[lo] == u;
     }
 };
 // Parents only ever move to smaller numbers of the same tree, so an old one still leads to the root.
@@ -244,16 +252,17 @@ __device__ __forceinline__ bool join_trees(int *cc, int a, int b)
 }
 
 // Rows are dealt out by length, as in pull_open_kernel.  Vertices of the tree that most samples lie in - after cc_begin usually
-// most of a component with hubs - are left out: an edge to one of the other trees is looked at from there.
+// most of a component with hubs - are left out: an edge from it to a vertex of another tree is in that vertex's in-row, an edge from
+// there to it in that vertex's out-row, which is looked through for those that do not come back.
 constexpr int kLinkThreads = 256, kLinkBlocks = 2048;
 constexpr int kLinkLane = 8, kLinkWave = 2048;  // entries up to which a row gets a lane, a wavefront
 __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows, int *cc, CcTrees *trees, int call, int pass)
 {
     constexpr int kWaves = kLinkThreads / kWave;
     __shared__ int s_wave[kLinkThreads], s_block[kLinkThreads];
-    __shared__ int s_waves, s_blocks;
-    if (trees->directed == call) return;
+    __shared__ int s_waves, s_blocks, s_over;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    if (tid == 0) s_over = trees->directed == call;  // read once: other work-groups may set it meanwhile
     const int stride = sample_stride(n), samples = (n - 1) / stride + 1 < kCcSamples ? (n - 1) / stride + 1 : kCcSamples;
     const int mine = lane < samples ? trees->sample[lane] : -1;
     int left_out = -1, most = 0;
@@ -269,6 +278,9 @@ __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows,
         if (!rows.leads_back(u, v, i)) trees->directed = call;
         else if (!join_trees(cc, a, b)) trees->again = pass;
     };
+    const auto leaves = [&](int a, unsigned int i, int u, int b, unsigned int e0, unsigned int e1) {  // entry i of an out-row
+        if ((b == left_out || u == left_out) && b != a && !rows.comes_back(u, i, e0, e1)) trees->directed = call;
+    };
     const auto walk = [&](int row, int first, int lanes) {
         const unsigned int e0 = rows.in_index[row], e1 = rows.in_index[row + 1];
         const int a = parent_of(cc, row);
@@ -279,7 +291,17 @@ __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows,
             edge(row, e - e0, a, u0, b0);
             if (two) edge(row, e + lanes - e0, a, u1, b1);
         }
+        const unsigned int d0 = rows.index[row], d1 = rows.index[row + 1];
+        for (unsigned int d = d0 + first; d < d1; d += 2 * lanes) {
+            const bool two = d + lanes < d1;
+            const int u0 = rows.dst[d], u1 = rows.dst[two ? d + lanes : d];
+            const int b0 = parent_of(cc, u0), b1 = parent_of(cc, u1);
+            leaves(a, d - d0, u0, b0, e0, e1);
+            if (two) leaves(a, d + lanes - d0, u1, b1, e0, e1);
+        }
     };
+    __syncthreads();
+    if (s_over) return;
     const int64_t pieces = ((int64_t)n + kWave - 1) / kWave, per_pass = (int64_t)kWaves * gridDim.x;
     for (int64_t at = 0; at < pieces; at += per_pass) {
         if (tid == 0) s_waves = s_blocks = 0;
@@ -289,18 +311,27 @@ __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows,
             const int r = (int)r64;
             const int a = parent_of(cc, r);
             if (a != left_out) {
-                const unsigned int e0 = rows.in_index[r], e1 = rows.in_index[r + 1];
-                if (e1 - e0 <= kLinkLane) {
-                    for (unsigned int e = e0; e < e1; e += 4) {
-                        int u[4], b[4];
+                const unsigned int e0 = rows.in_index[r], e1 = rows.in_index[r + 1], d0 = rows.index[r], d1 = rows.index[r + 1];
+                const unsigned int longer = max(e1 - e0, d1 - d0);
+                if (longer <= kLinkLane) {
+                    for (unsigned int i = 0; i < longer; i += 4) {
+                        int u[4], b[4], to[4], c[4];
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) u[k] = rows.in_src[e + k < e1 ? e + k : e1 - 1];
+                        for (int k = 0; k < 4; ++k) {
+                            u[k] = e0 + i + k < e1 ? rows.in_src[e0 + i + k] : r;
+                            to[k] = d0 + i + k < d1 ? rows.dst[d0 + i + k] : r;
+                        }
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) b[k] = parent_of(cc, u[k]);
-                        for (int k = 0; k < 4; ++k)
-                            if (e + k < e1) edge(r, e + k - e0, a, u[k], b[k]);
+                        for (int k = 0; k < 4; ++k) {
+                            b[k] = u[k] == r ? a : parent_of(cc, u[k]);
+                            c[k] = to[k] == r || to[k] == u[k] ? a : parent_of(cc, to[k]);  // in the second case it comes back
+                        }
+                        for (int k = 0; k < 4; ++k) {
+                            edge(r, i + k, a, u[k], b[k]);
+                            leaves(a, i + k, to[k], c[k], e0, e1);
+                        }
                     }
-                } else if (e1 - e0 <= kLinkWave) {
+                } else if (longer <= kLinkWave) {
                     s_wave[atomicAdd(&s_waves, 1)] = r;
                 } else {
                     s_block[atomicAdd(&s_blocks, 1)] = r;

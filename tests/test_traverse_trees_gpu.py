@@ -105,3 +105,35 @@ def test_labels_by_trees(oracle, name, without_reverse):
             assert res.VisitedSize == np.count_nonzero(want < np.arange(n))
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("other_is_hub", [False, True])
+@pytest.mark.parametrize("into_the_largest", [True, False])
+@pytest.mark.parametrize("size", [10, 100, 3_000])
+def test_one_edge_without_reverse_between_components(oracle, size, into_the_largest, other_is_hub):
+    """A component of most vertices and a small one, joined by one edge that leads one way and is not the least of its row."""
+    from drone_amd.traverse import CCWorkerCUDA
+    rng = np.random.default_rng(size)
+    small, large = np.arange(0, size, dtype=np.int32), np.arange(size, 40 * size, dtype=np.int32)
+    if not into_the_largest:  # the one way leads from smaller to larger labels
+        small, large = np.arange(39 * size, 40 * size, dtype=np.int32), np.arange(0, 39 * size, dtype=np.int32)
+
+    def connected(names, hub):  # a star, or a random tree
+        k = np.arange(1, len(names))
+        up = np.zeros(len(k), np.int64) if hub else (rng.random(len(k)) * k).astype(np.int64)
+        return _both(names[k], names[up])
+
+    # local numbers go by first appearance
+    us, vs = zip(*sorted([connected(small, other_is_hub), connected(large, False)], key=lambda e: e[0].min()))
+    one = (small[-1], large[-1]) if into_the_largest else (large[-1], small[-1])
+    u, v = np.concatenate([*us, [one[0]]]).astype(np.int32), np.concatenate([*vs, [one[1]]]).astype(np.int32)
+    n, l2g, _, index, dst = oracle.build_graph(40 * size, u, v)
+    want = _labels(n, index, dst)
+    assert want.max() == 0  # the edge joins them, though one way only
+    w = CCWorkerCUDA(40 * size, u, v)
+    try:
+        for _ in range(2):
+            w.peval()
+            np.testing.assert_array_equal(w.read(), want)
+    finally:
+        w.close()
