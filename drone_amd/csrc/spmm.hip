@@ -52,7 +52,7 @@ struct drone_spmm_plan {
     int max_k = 0;
     // short rows in chunks: consecutive rows of at most 64 entries together (or one row of any length up to the split)
     int num_chunks = 0;
-    int *chunk_r0 = nullptr, *chunk_r1 = nullptr;  // device [num_chunks]
+    int4 *chunk = nullptr;  // device [num_chunks]: {first row, last + 1, first entry, last + 1}
     // long rows, cut into band pieces
     int num_long = 0, num_pieces = 0;
     int64_t long_nnz = 0;
@@ -61,7 +61,8 @@ struct drone_spmm_plan {
     int *ci2 = nullptr;                                                      // device [long_nnz]: columns, (band,row)-sorted
     float *val2 = nullptr;                                                   // device [long_nnz]: values in the same order
     unsigned *perm = nullptr;                                                // device [long_nnz]: sorted position -> entry
-    float *partial = nullptr;                                                // device [num_pieces x max_k]
+    float *partial = nullptr;                                                // device [num_pieces x ldp]
+    int ldp = 0;                                                             // max_k rounded up to 16 bytes
     int num_bands = 0, band_cols = 0;
     // dense core (see the file comment); rows and columns below are in rank order
     struct Rect { int row0, rows, width; size_t a_off; };
@@ -126,6 +127,24 @@ constexpr size_t kBandBytes = 3u << 20; // feature rows of one band (three quart
 // With 2 MB bands, 10 / 15 / 24 / 32 hot bands: 5.44 / 4.83 / 4.44 / 4.44 ms (K = 128).
 // With the dense region kept as bits (scaled patterns), 3 MB x 4 / 8 / 12 / 16 / 20 / 28 / 38 / 56 hot bands: 3.45 / 3.00 / 2.85 /
 // 2.75 / 2.80 / 2.95 / 3.07 / 3.05 ms at K = 128 and 1.64 / 1.51 / 1.39 / 1.35 / 1.35 / 1.34 / 1.35 / 1.33 at K = 41.
+// Slices: the feature columns are dealt out over 2^bits work-groups per chunk or piece, each with lane groups that much
+// narrower.  For one thing that halves the serial chain of a row, in a matrix so small that the GPU still holds all the
+// wavefronts; us at K = 128 without / with: 4,001 vertices and 60 K entries 43 / 28, 20,003 hub-heavy ones and 0.3 M entries
+// 57 / 46, epoch on 2,708 vertices 165 / 159.  With more wavefronts than that their fixed costs count: 30,001 vertices 72 / 78.
+constexpr int kResidentWaves = 8192;
+// For another, work-groups go round the eight XCDs in turn, so an XCD always gets the same slice (of a power of two of them):
+// its L2 holds that many times more feature rows, and a band has as many more columns.  Worth it with whole 128-byte lines,
+// slices that are all nearly full, and an operand larger than the L2s together; us without / with: 0.25 M vertices and 6 M
+// entries at K = 128 663 / 541, 1 M vertices and 16 M entries 1,811 / 1,640, the 232,965-vertex step 8,627 / 7,893, 1 M vertices
+// and 32 M entries at K = 256 7,976 / 6,587; but 0.2 M vertices at K = 100 (64 + 36, or 52 + 48 across lines) 312 / 372, and
+// with 32 columns a slice the step took 9,843.
+constexpr int kLineFloats = 32, kSliceCols = 2 * kLineFloats;
+constexpr int64_t kAllL2Bytes = 32 << 20;
+int line_slice_bits(int K, int n_cols)
+{
+    const int bits = K > 2 * kSliceCols ? 2 : 1, free = (kSliceCols << bits) - K;
+    return free >= 0 && free <= kSliceCols / 4 && (int64_t)n_cols * K * (int64_t)sizeof(float) > kAllL2Bytes ? bits : 0;
+}
 constexpr int kBandMaxCols = 8192;      // narrow feature rows: a band is at most this many columns
 constexpr int kRowsPerBlock = 4;        // wavefronts per work-group (2 / 4 / 8: 4.29 / 4.31 / 4.33 ms at K = 128, 2.50 / 2.45 / 2.56 at K = 41)
 constexpr int kDenseChunk = 2048;       // column granularity of the dense rectangles
@@ -172,24 +191,34 @@ constexpr double kFarOperandBytes = 192e6;
 constexpr double kFarGatherFactor = 3.0;
 static_assert(kDenseMaxCols / kDenseChunk <= kBitMaxChunks, "the density histogram keeps at most 128 chunks per wavefront");
 
-template <int VEC> struct VecT;
-template <> struct VecT<4> { using type = float4; };
-template <> struct VecT<2> { using type = float2; };
-template <> struct VecT<1> { using type = float; };
+// 16 bytes at any address that a float may have.  Global memory takes them there; a row that starts off a 16-byte boundary is so
+// read with a quarter of the instructions, and all its columns at once up to K = 256.  us for the forward and the transposed
+// product with four-byte loads / with these: 300,003 vertices and 3 M entries at
+// K = 97 463 / 301, 10,003 vertices and 0.1 M entries at K = 61 69 / 32, 0.1 M vertices and 1.1 M entries at K = 47 110 / 70, K = 10 55 / 53.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// The columns of lane li: VEC of them from `at` on, of which the first `skip` are the lane before's.  (The last lane of a row whose
+// width is not a multiple of VEC moves back to stay inside it.)
+template <int VEC>
+struct LaneColumns {
+    int k, K;
+    __device__ __forceinline__ int at() const { return VEC > 1 && k + VEC > K ? K - VEC : k; }
+    __device__ __forceinline__ int skip() const { return k - at(); }
+    __device__ __forceinline__ bool active() const { return k < K; }
+};
 
 template <int VEC>
 __device__ __forceinline__ void load_vec(const float *p, float (&x)[VEC])
 {
-    if constexpr (VEC == 4) { const float4 v = *reinterpret_cast<const float4 *>(p); x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; }
-    else if constexpr (VEC == 2) { const float2 v = *reinterpret_cast<const float2 *>(p); x[0] = v.x; x[1] = v.y; }
+    if constexpr (VEC == 4) { const f4u v = *reinterpret_cast<const f4u *>(p); x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; }
     else { x[0] = *p; }
 }
 
-// Accumulates sum_e val[e] * B[col[e], kbase .. kbase+VEC) for e in [e0, e1) into acc (per lane), then
+// Accumulates sum_e val[e] * B[col[e], cols.at .. cols.at+VEC) for e in [e0, e1) into acc (per lane), then
 // folds the P lane groups together so that group 0 holds the totals.
 template <int G, int VEC>
 __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restrict__ ci, const float *__restrict__ val,
-                                            const float *__restrict__ B, int ldb, int kbase, bool active,
+                                            const float *__restrict__ B, int ldb, const LaneColumns<VEC> &cols,
                                             float (&acc)[VEC])
 {
     constexpr int P = kWave / G;
@@ -221,7 +250,7 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
                     aa[u] = __shfl(a, q + u * P + sub, kWave);
                 }
             }
-            if (active) {
+            if (cols.active()) {
                 // a slot past the end of the batch loads nothing: its lanes are masked off, so the address unit
                 // spends no cycles on it (padding slots were a quarter of all loads on short pieces)
                 float b[U][VEC];
@@ -229,7 +258,7 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
                 for (int u = 0; u < U; ++u) {
 #pragma unroll
                     for (int v = 0; v < VEC; ++v) b[u][v] = 0.0f;
-                    if (q + u * P + sub < cnt) load_vec<VEC>(B + (size_t)cc[u] * ldb + kbase, b[u]);
+                    if (q + u * P + sub < cnt) load_vec<VEC>(B + (size_t)cc[u] * ldb + cols.at(), b[u]);
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u)
@@ -245,15 +274,20 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
 }
 
 template <int VEC>
-__device__ __forceinline__ void store_row(float *__restrict__ dst, int kbase, int K, const float (&acc)[VEC],
+__device__ __forceinline__ void store_row(float *__restrict__ dst, const LaneColumns<VEC> &cols, const float (&acc)[VEC],
                                           float alpha, float beta)
 {
+    dst += cols.at();
+    if (VEC == 4 && beta == 0.0f) {  // the columns that two lanes have they store the same in
+        *reinterpret_cast<f4u *>(dst) = f4u{alpha * acc[0], alpha * acc[1 % VEC], alpha * acc[2 % VEC], alpha * acc[3 % VEC]};
+        return;
+    }
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
-        if (kbase + v < K) {
+        if (v >= cols.skip()) {
             float r = alpha * acc[v];
-            if (beta != 0.0f) r += beta * dst[kbase + v];
-            dst[kbase + v] = r;
+            if (beta != 0.0f) r += beta * dst[v];
+            dst[v] = r;
         }
 }
 
@@ -273,37 +307,39 @@ struct RowSegments {
     float *__restrict__ C;
     int ldc;
     float alpha, beta;
-    __device__ __forceinline__ int start(int first, int j, int) const { return rp[first + j]; }  // j <= count
+    __device__ __forceinline__ int start(int first, int j) const { return rp[first + j]; }  // j <= count
     __device__ __forceinline__ float *out(int first, int j) const { return C + (size_t)(first + j) * ldc; }
 };
 template <int G, int VEC, typename Segments>
-__device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *__restrict__ chunk_first,
-                                          const int *__restrict__ chunk_last, Segments seg, const int *__restrict__ ci,
-                                          const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
+__device__ __forceinline__ void sum_chunk(int block, int slice, int slices, int num_chunks, const int4 *__restrict__ chunk,
+                                          Segments seg, const int *__restrict__ ci, const float *__restrict__ val,
+                                          const float *__restrict__ B, int ldb, int K)
 {
     constexpr int P = kWave / G;
-    constexpr int U = 8;  // feature-row loads in flight per lane group (4 / 6 / 8 measured the same)
-    const int c = block * kRowsPerBlock + threadIdx.x / kWave;
+    // Feature-row loads in flight per lane group.  With 8 the kernels take 84 registers, 5 or 6 wavefronts a SIMD; with 4 at most
+    // 60 (8 lanes a group: 72), which leaves all 8.  us with 8 / 6 / 4: the 232,965-vertex step 7,831 / 7,713 / 7,684, 30,011
+    // vertices 256 / 254 / 253, 0.1 M vertices and 1 M entries at K = 128 110 / 106 / 100.
+    constexpr int U = 4;
+    const int c = block * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // what it reads stays in scalar registers
     if (c >= num_chunks) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int li = lane % G, sub = lane / G;
-    const int r0 = chunk_first[c], nrows = chunk_last[c] - r0;
+    const int4 mine = chunk[c];
+    const int r0 = mine.x, nrows = mine.y - mine.x, e0 = mine.z, n = mine.w - mine.z;
     const float alpha = seg.alpha, beta = seg.beta;
     if (nrows == 1) {
-        const int e0 = seg.start(r0, 0, 1), e1 = seg.start(r0, 1, 1);
         float *dst = seg.out(r0, 0);
-        for (int k0 = 0; k0 < K; k0 += G * VEC) {
-            const int kbase = k0 + li * VEC;
-            const bool active = kbase < K;
+        for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
+            const LaneColumns<VEC> cols{k0 + li * VEC, K};
             float acc[VEC];
-            row_segment<G, VEC>(e0, e1, ci, val, B, ldb, kbase, active, acc);
-            if (sub == 0 && active) store_row<VEC>(dst, kbase, K, acc, alpha, beta);
+            row_segment<G, VEC>(e0, e0 + n, ci, val, B, ldb, cols, acc);
+            if (sub == 0 && cols.active()) store_row<VEC>(dst, cols, acc, alpha, beta);
         }
         return;
     }
-    // lane j holds where segment r0 + j starts; lanes nrows .. 63 hold where the chunk ends
-    const int start = seg.start(r0, lane < nrows ? lane : nrows, nrows);
-    const int e0 = __shfl(start, 0, kWave), n = __shfl(start, nrows, kWave) - e0;
+    // lane j holds where segment r0 + j starts; lanes nrows .. 63 hold where the chunk ends.  (Its entries are fetched meanwhile:
+    // their bounds come with the chunk's.)
+    const int start = seg.start(r0, lane < nrows ? lane : nrows);
     const int col = lane < n ? ci[e0 + lane] : 0;
     const float a = lane < n ? val[e0 + lane] : 0.0f;
     // the segment of entry `lane`: the last one that starts at or before it
@@ -344,9 +380,8 @@ __device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *
     // segments without entries: out = beta * out, by the first lane group
     const int next_start = __shfl_down(start, 1, kWave);
     const unsigned long long empty = __ballot(lane < nrows && next_start == start);
-    for (int k0 = 0; k0 < K; k0 += G * VEC) {
-        const int kbase = k0 + li * VEC;
-        const bool active = kbase < K;
+    for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
+        const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
@@ -367,13 +402,13 @@ __device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *
             for (int u = 0; u < U; ++u) {
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) b[u][v] = 0.0f;
-                if (active && q0 + u < qb) load_vec<VEC>(B + (size_t)cc[u] * ldb + kbase, b[u]);
+                if (cols.active() && q0 + u < qb) load_vec<VEC>(B + (size_t)cc[u] * ldb + cols.at(), b[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (q0 + u < qb) {
                     if (rr[u] != cur) {
-                        if (cur >= 0 && active) store_row<VEC>(seg.out(r0, cur), kbase, K, acc, alpha, beta);
+                        if (cur >= 0 && cols.active()) store_row<VEC>(seg.out(r0, cur), cols, acc, alpha, beta);
                         cur = rr[u];
 #pragma unroll
                         for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
@@ -383,12 +418,12 @@ __device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *
                 }
             }
         }
-        if (cur >= 0 && active) store_row<VEC>(seg.out(r0, cur), kbase, K, acc, alpha, beta);
+        if (cur >= 0 && cols.active()) store_row<VEC>(seg.out(r0, cur), cols, acc, alpha, beta);
         for (unsigned long long left = empty; left; left &= left - 1) {
             const int j = __ffsll((long long)left) - 1;
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-            if (sub == 0 && active) store_row<VEC>(seg.out(r0, j), kbase, K, acc, alpha, beta);
+            if (sub == 0 && cols.active()) store_row<VEC>(seg.out(r0, j), cols, acc, alpha, beta);
         }
     }
 }
@@ -404,58 +439,58 @@ __device__ __forceinline__ void sum_chunk(int block, int num_chunks, const int *
 // One piece per lane group (two or four pieces side by side in a wavefront, nothing folded across groups) lost too:
 // 4.78 / 3.00 ms for K = 128 / 41 against 4.44 / 2.60 - the wavefront runs as long as its longest piece.
 template <int G, int VEC>
-__device__ __forceinline__ void sum_piece(int block, int num_pieces, const int *__restrict__ piece_begin,
+__device__ __forceinline__ void sum_piece(int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
                                           const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
                                           const int *__restrict__ ci, const float *__restrict__ val,
                                           const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
 {
-    const int s = block * kRowsPerBlock + threadIdx.x / kWave;
+    const int s = block * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (s >= num_pieces) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int li = lane % G, sub = lane / G;
-    for (int k0 = 0; k0 < K; k0 += G * VEC) {
-        const int kbase = k0 + li * VEC;
-        const bool active = kbase < K;
+    for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
+        const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
-        row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, kbase, active, acc);
-        if (sub == 0 && active) store_row<VEC>(partial + (size_t)piece_slot[s] * ldp, kbase, K, acc, 1.0f, 0.0f);
+        row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
+        if (sub == 0 && cols.active()) store_row<VEC>(partial + (size_t)piece_slot[s] * ldp, cols, acc, 1.0f, 0.0f);
     }
 }
 
 template <int G, int VEC>
-__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_pieces_kernel(
+__global__ __launch_bounds__(kWave * kRowsPerBlock, G == 8 ? 6 : 8) void spmm_pieces_kernel(
     int num_pieces, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
     const int *__restrict__ piece_slot, const int *__restrict__ ci, const float *__restrict__ val,
-    const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
+    const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K, int slice_bits)
 {
-    sum_piece<G, VEC>(blockIdx.x, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
+    const int slices = 1 << slice_bits;
+    sum_piece<G, VEC>(blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
 }
 
 template <int G, int VEC, typename Segments>
-__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_chunks_kernel(
-    int num_chunks, const int *__restrict__ chunk_first, const int *__restrict__ chunk_last, Segments seg,
-    const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
+__global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_chunks_kernel(
+    int num_chunks, const int4 *__restrict__ chunk, Segments seg, const int *__restrict__ ci, const float *__restrict__ val,
+    const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
-    sum_chunk<G, VEC>(blockIdx.x, num_chunks, chunk_first, chunk_last, seg, ci, val, B, ldb, K);
+    const int slices = 1 << slice_bits;
+    sum_chunk<G, VEC>(blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_chunks, chunk, seg, ci, val, B, ldb, K);
 }
 
 // Both in one launch, the pieces first: the chunks fill the GPU while the last pieces end, and a launch is saved.  us
 // against one launch each: training step on 30,011 vertices 280 / 263, 20 K vertices and 0.3 M entries at K = 128 74 / 57,
 // 1 M vertices and 15 M entries at K = 41 678 / 619, forward and backward over a vertex cut 757 / 715.  Not beside a bit
-// core: pieces alone take 8 wavefronts per SIMD instead of 6 (76 registers here), and the product of 3 M vertices at
-// K = 64 took 2,369 / 2,442.
+// core, where a launch costs nothing and the product of 3 M vertices at K = 64 took 2,369 / 2,442.
 template <int G, int VEC>
-__global__ __launch_bounds__(kWave * kRowsPerBlock) void spmm_gather_kernel(
+__global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_gather_kernel(
     int num_pieces, int piece_blocks, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
     const int *__restrict__ piece_slot, const int *__restrict__ ci2, const float *__restrict__ val2,
-    float *__restrict__ partial, int ldp, int num_chunks, const int *__restrict__ chunk_first,
-    const int *__restrict__ chunk_last, RowSegments seg, const int *__restrict__ ci, const float *__restrict__ val,
-    const float *__restrict__ B, int ldb, int K)
+    float *__restrict__ partial, int ldp, int num_chunks, const int4 *__restrict__ chunk, RowSegments seg,
+    const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
-    if ((int)blockIdx.x < piece_blocks)
-        sum_piece<G, VEC>(blockIdx.x, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
+    const int slices = 1 << slice_bits, block = blockIdx.x >> slice_bits, slice = blockIdx.x & (slices - 1);
+    if (block < piece_blocks)
+        sum_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
     else
-        sum_chunk<G, VEC>(blockIdx.x - piece_blocks, num_chunks, chunk_first, chunk_last, seg, ci, val, B, ldb, K);
+        sum_chunk<G, VEC>(block - piece_blocks, slice, slices, num_chunks, chunk, seg, ci, val, B, ldb, K);
 }
 
 // C[row,:] = alpha * (sum of the row's partial pieces, in slot = (band, position) order) + beta * C[row,:]
@@ -489,15 +524,14 @@ __global__ void spmm_combine_kernel(int num_long, const int *__restrict__ long_r
 // The same sums with 16-byte accesses: L lanes per long row (L a power of two, 4 L >= K), 64 / L rows per wavefront, eight
 // 16-byte loads in flight per lane, still added in slot order.  One 128-lane work-group per row with a float per lane
 // took 0.155 / 0.070 ms for the 0.34 / 0.11 GB of partial rows of a 128- / 41-wide product on the 232,965-vertex graph
-// (a hundred thousand work-groups of two or three round trips each).  wide_c: C's rows can be written in aligned
-// 16-byte pieces; the piece that holds column K - 1 is written float by float when K is not a multiple of four.
+// (a hundred thousand work-groups of two or three round trips each).  The piece that holds column K - 1 is written float by
+// float when K is not a multiple of four.
 typedef float combine_f4 __attribute__((ext_vector_type(4)));
 template <int L>
 __global__ __launch_bounds__(256) void spmm_combine4_kernel(int num_long, const int *__restrict__ long_row,
                                                             const int *__restrict__ first_slot,
                                                             const float *__restrict__ partial, int ldp,
-                                                            float *__restrict__ C, int ldc, int K, float alpha, float beta,
-                                                            bool wide_c)
+                                                            float *__restrict__ C, int ldc, int K, float alpha, float beta)
 {
     constexpr int R = kWave / L;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -524,10 +558,10 @@ __global__ __launch_bounds__(256) void spmm_combine4_kernel(int num_long, const 
         }
     }
     float *dst = C + (size_t)r * ldc + k;
-    if (wide_c && k + 4 <= K) {
-        combine_f4 out = alpha * sum;
-        if (beta != 0.0f) out += beta * *reinterpret_cast<const combine_f4 *>(dst);
-        *reinterpret_cast<combine_f4 *>(dst) = out;
+    if (k + 4 <= K) {
+        f4u out = alpha * sum;
+        if (beta != 0.0f) out += beta * *reinterpret_cast<const f4u *>(dst);
+        *reinterpret_cast<f4u *>(dst) = out;
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -748,36 +782,32 @@ __global__ void gather_sorted_kernel(int64_t count, const unsigned *__restrict__
 
 template <int G, int VEC>
 void launch_spmm(const drone_spmm_plan *plan, const int *rp, const int *ci, const float *v, const float *B, int ldb,
-                 float *C, int ldc, int K, float alpha, float beta, hipStream_t s)
+                 float *C, int ldc, int K, float alpha, float beta, int slice_bits, hipStream_t s)
 {
     const int piece_blocks = (int)ceil_div(plan->num_pieces, kRowsPerBlock), chunk_blocks = (int)ceil_div(plan->num_chunks, kRowsPerBlock);
     const RowSegments rows{rp, C, ldc, alpha, beta};
     if (piece_blocks > 0 && chunk_blocks > 0 && plan->bits.tiles == 0) {
-        spmm_gather_kernel<G, VEC><<<(unsigned)piece_blocks + (unsigned)chunk_blocks, kWave * kRowsPerBlock, 0, s>>>(
+        spmm_gather_kernel<G, VEC><<<((unsigned)piece_blocks + (unsigned)chunk_blocks) << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
             plan->num_pieces, piece_blocks, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2,
-            plan->partial, plan->max_k, plan->num_chunks, plan->chunk_r0, plan->chunk_r1, rows, ci, v, B, ldb, K);
+            plan->partial, plan->ldp, plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
     } else {
         if (piece_blocks > 0)
-            spmm_pieces_kernel<G, VEC><<<piece_blocks, kWave * kRowsPerBlock, 0, s>>>(
+            spmm_pieces_kernel<G, VEC><<<(unsigned)piece_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
                 plan->num_pieces, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2, B, ldb,
-                plan->partial, plan->max_k, K);
+                plan->partial, plan->ldp, K, slice_bits);
         if (chunk_blocks > 0)
-            spmm_chunks_kernel<G, VEC, RowSegments><<<chunk_blocks, kWave * kRowsPerBlock, 0, s>>>(
-                plan->num_chunks, plan->chunk_r0, plan->chunk_r1, rows, ci, v, B, ldb, K);
+            spmm_chunks_kernel<G, VEC, RowSegments><<<(unsigned)chunk_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
+                plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
     }
     if (plan->num_long > 0) {  // also when every entry of the long rows went to the dense part: C = beta * C there
-        const int ldp = plan->max_k;
-        // the partial rows are read in 16-byte pieces up to column 4 ceil(K / 4): they must hold that many floats
-        const bool pieces16 = ldp % 4 == 0 && K <= 256 && (reinterpret_cast<uintptr_t>(plan->partial) & 15) == 0;
-        const bool wide_c = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
         const auto launch = [&](auto kernel, int lanes) {
             const int rows_per_group = 4 * (kWave / lanes);
             kernel<<<(int)ceil_div(plan->num_long, rows_per_group), 256, 0, s>>>(plan->num_long, plan->long_row, plan->first_slot,
-                                                                               plan->partial, ldp, C, ldc, K, alpha, beta, wide_c);
+                                                                               plan->partial, plan->ldp, C, ldc, K, alpha, beta);
         };
-        if (!pieces16)
+        if (K > 256)
             spmm_combine_kernel<<<plan->num_long, 128, 0, s>>>(plan->num_long, plan->long_row, plan->first_slot,
-                                                              plan->partial, ldp, C, ldc, K, alpha, beta);
+                                                              plan->partial, plan->ldp, C, ldc, K, alpha, beta);
         else if (K <= 16) launch(spmm_combine4_kernel<4>, 4);
         else if (K <= 32) launch(spmm_combine4_kernel<8>, 8);
         else if (K <= 64) launch(spmm_combine4_kernel<16>, 16);
@@ -818,11 +848,12 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
     p->long_nnz = long_nnz;
 
     const int ld = (p->max_k + 3) / 4 * 4;
-    int band_cols = (int)(kBandBytes / (sizeof(float) * (size_t)ld));
+    const int slice_bits = line_slice_bits(p->max_k, p->n_cols), hot_bands = slice_bits > 0 ? kHotBands / 2 : kHotBands;
+    int band_cols = (int)(kBandBytes / (sizeof(float) * (size_t)ld)) << slice_bits;
     if (band_cols < 64) band_cols = 64;
-    if (band_cols > kBandMaxCols) band_cols = kBandMaxCols;
+    if (band_cols > kBandMaxCols << slice_bits) band_cols = kBandMaxCols << slice_bits;
     int num_bands = (int)ceil_div(p->n_cols, band_cols);
-    if (num_bands > kHotBands + 1) num_bands = kHotBands + 1;
+    if (num_bands > hot_bands + 1) num_bands = hot_bands + 1;
     if (num_bands < 1) num_bands = 1;
     if (long_nnz <= kOneBandEntries) num_bands = 1;
     const auto piece_of_row = [&](int i) { return piece_entries(p->nnz, long_offset[i + 1] - long_offset[i]); };
@@ -1002,7 +1033,7 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
         DRONE_HIP_TRY(hipMalloc(&p->piece_begin, sizeof(int) * (size_t)num_pieces));
         DRONE_HIP_TRY(hipMalloc(&p->piece_end, sizeof(int) * (size_t)num_pieces));
         DRONE_HIP_TRY(hipMalloc(&p->piece_slot, sizeof(int) * (size_t)num_pieces));
-        DRONE_HIP_TRY(hipMalloc(&p->partial, sizeof(float) * (size_t)num_pieces * (size_t)p->max_k));
+        DRONE_HIP_TRY(hipMalloc(&p->partial, sizeof(float) * (size_t)num_pieces * (size_t)p->ldp));
         DRONE_HIP_TRY(hipMemcpy(p->first_slot, first_slot.data(), sizeof(int) * first_slot.size(), hipMemcpyHostToDevice));
         DRONE_HIP_TRY(hipMemcpy(p->piece_begin, pb.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
         DRONE_HIP_TRY(hipMemcpy(p->piece_end, pe.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
@@ -1120,15 +1151,12 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
         if (len > kSplitRow) long_row.push_back(r);
     }
     // chunks of the short rows
-    std::vector<int> h_c0, h_c1;
+    std::vector<int4> h_chunk;
     const int most = chunk_entries(n_rows, nnz);
     {
         int first = -1, entries = 0;
         const auto close = [&](int end) {
-            if (first >= 0) {
-                h_c0.push_back(first);
-                h_c1.push_back(end);
-            }
+            if (first >= 0) h_chunk.push_back(make_int4(first, end, h_rp[first], h_rp[end]));
             first = -1;
             entries = 0;
         };
@@ -1138,8 +1166,7 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
                 close(r);
             } else if (len > kWave) {  // more than one load of pairs: a chunk of its own
                 close(r);
-                h_c0.push_back(r);
-                h_c1.push_back(r + 1);
+                h_chunk.push_back(make_int4(r, r + 1, h_rp[r], h_rp[r + 1]));
             } else {
                 if (first >= 0 && (entries + len > most || r - first >= kWave - 1)) close(r);
                 if (first < 0) first = r;
@@ -1170,13 +1197,12 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
         p->nnz = nnz;
         p->max_k = max_k;
         p->scaled = scaled;
-        p->num_chunks = (int)h_c0.size();
+        p->num_chunks = (int)h_chunk.size();
+        p->ldp = (max_k + 3) / 4 * 4;
         if (p->num_chunks > 0) {
             const auto upload = [&]() -> int {
-                DRONE_HIP_TRY(hipMalloc(&p->chunk_r0, sizeof(int) * h_c0.size()));
-                DRONE_HIP_TRY(hipMalloc(&p->chunk_r1, sizeof(int) * h_c1.size()));
-                DRONE_HIP_TRY(hipMemcpy(p->chunk_r0, h_c0.data(), sizeof(int) * h_c0.size(), hipMemcpyHostToDevice));
-                DRONE_HIP_TRY(hipMemcpy(p->chunk_r1, h_c1.data(), sizeof(int) * h_c1.size(), hipMemcpyHostToDevice));
+                DRONE_HIP_TRY(hipMalloc(&p->chunk, sizeof(int4) * h_chunk.size()));
+                DRONE_HIP_TRY(hipMemcpy(p->chunk, h_chunk.data(), sizeof(int4) * h_chunk.size(), hipMemcpyHostToDevice));
                 return DRONE_OK;
             };
             const int urc = upload();
@@ -1246,8 +1272,7 @@ extern "C" int drone_spmm_plan_update_values(drone_spmm_plan *p, const float *v,
 extern "C" int drone_spmm_plan_destroy(drone_spmm_plan *p)
 {
     if (!p) return DRONE_OK;
-    (void)hipFree(p->chunk_r0);
-    (void)hipFree(p->chunk_r1);
+    (void)hipFree(p->chunk);
     (void)hipFree(p->long_row);
     (void)hipFree(p->first_slot);
     (void)hipFree(p->piece_begin);
@@ -1329,23 +1354,27 @@ extern "C" int drone_spmm_csr_f32(const drone_spmm_plan *plan, const int *rp, co
         if (st != DRONE_OK) return st;
         DRONE_HIP_TRY(hipEventRecord(plan->bits.join, plan->bits.side));
     }
-    const auto aligned = [&](int a) {
-        return ldb % a == 0 && ldc % a == 0 && ((uintptr_t)B % (4 * a)) == 0 && ((uintptr_t)C % (4 * a)) == 0;
-    };
-    // widest vector the layout allows, then the smallest lane group that covers K
-    if (aligned(4)) {
-        const int need = (K + 3) / 4;
-        if (need <= 4) launch_spmm<4, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (need <= 8) launch_spmm<8, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (need <= 16) launch_spmm<16, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (need <= 32) launch_spmm<32, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else launch_spmm<64, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
+    if (K < 4) {
+        launch_spmm<4, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
     } else {
-        if (K <= 4) launch_spmm<4, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (K <= 8) launch_spmm<8, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (K <= 16) launch_spmm<16, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else if (K <= 32) launch_spmm<32, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
-        else launch_spmm<64, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, s);
+        // the smallest lane group that covers K, or a slice of it
+        int lanes = 4, slice_bits = line_slice_bits(K, plan->n_cols);
+        while (lanes < kWave && lanes * 4 < K) lanes *= 2;
+        if (slice_bits > 0 && ldb % kLineFloats == 0 && (uintptr_t)B % (4 * kLineFloats) == 0) {
+            lanes = kSliceCols / 4;
+        } else {
+            slice_bits = 0;
+            for (int64_t waves = (int64_t)plan->num_pieces + plan->num_chunks; lanes > 4 && 2 * waves <= kResidentWaves; waves *= 2) {
+                ++slice_bits;
+                lanes /= 2;
+            }
+        }
+        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, slice_bits, s); };
+        if (lanes == 4) launch(std::integral_constant<int, 4>());
+        else if (lanes == 8) launch(std::integral_constant<int, 8>());
+        else if (lanes == 16) launch(std::integral_constant<int, 16>());
+        else if (lanes == 32) launch(std::integral_constant<int, 32>());
+        else launch(std::integral_constant<int, 64>());
     }
     int dense_status = DRONE_OK;
     if (plan->bits.tiles > 0) {

@@ -251,6 +251,7 @@ __global__ __launch_bounds__(512, 1) void bits_mfma_kernel(const int *__restrict
 // (one per group, p and dword) regroup them, against 288 matrix instructions.  A stage is 64 ranked columns (two
 // steps): 8 groups x 3 parts x 16 CT features, fetched and handed over exactly as in bits_mfma_kernel.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));  // global memory takes it at any float's address
 template <int CT>
 __global__ __launch_bounds__(512, 1) void bits_mfma16_kernel(const int *__restrict__ unit_tile,
                                                              const int *__restrict__ unit_c0,
@@ -392,15 +393,14 @@ __global__ __launch_bounds__(256) void bits_combine_kernel(int rows, const int *
     }
 }
 
-// The same with 16-byte accesses: L lanes per ranked row (4 L >= K, K <= 256), 64 / L rows per wavefront.  wide_c: C's rows
-// can be read and written in aligned 16-byte pieces; the piece that holds column K - 1 goes float by float when K is not
-// a multiple of four (the tile sums' own rows are 128 floats long, so reading them past K is harmless).
+// The same with 16-byte accesses: L lanes per ranked row (4 L >= K, K <= 256), 64 / L rows per wavefront.  The piece that holds
+// column K - 1 goes float by float when K is not a multiple of four (the tile sums' own rows are 128 floats long, so reading them past K is harmless).
 template <int L>
 __global__ __launch_bounds__(256) void bits_combine4_kernel(int rows, const int *__restrict__ tile_unit0,
                                                             const float *__restrict__ partial, int num_units,
                                                             const int *__restrict__ dense_row,
                                                             const float *__restrict__ row_scale, float *__restrict__ C,
-                                                            int ldc, int K, float alpha, bool wide_c)
+                                                            int ldc, int K, float alpha)
 {
     constexpr int R = kWave / L;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -412,10 +412,10 @@ __global__ __launch_bounds__(256) void bits_combine4_kernel(int rows, const int 
     const float scale = alpha * row_scale[row];
     const float *src = partial + ((size_t)(k / 128) * num_units * kBitTileRows + rr % kBitTileRows) * kPartialLd + k % 128;
     float *dst = C + (size_t)row * ldc + k;
-    const bool whole = wide_c && k + 4 <= K;
+    const bool whole = k + 4 <= K;
     f32x4 before = {0.0f, 0.0f, 0.0f, 0.0f};
     if (whole) {
-        before = *reinterpret_cast<const f32x4 *>(dst);  // in flight with the tile sums
+        before = *reinterpret_cast<const f32x4_any *>(dst);  // in flight with the tile sums
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256) void bits_combine4_kernel(int rows, const int 
     }
     const f32x4 out = before + scale * sum;
     if (whole) {
-        *reinterpret_cast<f32x4 *>(dst) = out;
+        *reinterpret_cast<f32x4_any *>(dst) = out;
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -595,10 +595,9 @@ int bit_core_add(const BitCore *bc, const int *dense_row, const float *row_scale
     int grid = (int)ceil_div(bc->rows, 4);
     if (grid > 65536) grid = 65536;
     if (K <= 256) {
-        const bool wide_c = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
         const auto launch = [&](auto kernel, int lanes) {
             kernel<<<(int)ceil_div(bc->rows, 4 * (kWave / lanes)), 256, 0, s>>>(bc->rows, bc->tile_unit0, bc->partial, bc->num_units,
-                                                                               dense_row, row_scale, C, ldc, K, alpha, wide_c);
+                                                                               dense_row, row_scale, C, ldc, K, alpha);
         };
         if (K <= 16) launch(bits_combine4_kernel<4>, 4);
         else if (K <= 32) launch(bits_combine4_kernel<8>, 8);

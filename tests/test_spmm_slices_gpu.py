@@ -1,0 +1,90 @@
+"""The aggregation at every width of its lane groups and slices, at any alignment: feature widths around powers of two, operands whose
+rows start off 16-byte and 128-byte boundaries or lie in a wider array, operands below and above the size from which slices go by whole
+lines (32 MB), few and many wavefronts, and plans that keep a part as bits."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+
+#        feature widths, leading dimensions, first column, rows, columns, entries a row
+CASES = {
+    "narrow": ([1, 2, 3, 4, 5, 6, 7, 8, 9], [9, 12, 13], 1, 301, 401, 9),
+    "groups": ([15, 16, 17, 31, 32, 33, 63, 64, 65, 66], [67, 68], 0, 301, 401, 30),
+    "few_wavefronts": ([100, 127, 128, 129, 160, 255, 256, 257, 300], [300, 301], 3, 301, 401, 300),
+    "many_wavefronts": ([10, 61, 97, 128], [128, 131], 0, 12_001, 20_011, 40),
+    "lines": ([97, 111, 112, 113, 125, 128], [128, 160], 0, 4_001, 90_001, 40),
+    "no_lines": ([113, 128], [132, 129], 0, 4_001, 90_001, 40),
+    "four_slices": ([239, 240, 241, 254, 256], [256], 0, 3_001, 40_001, 40),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_every_width_and_alignment(name):
+    import torch
+    from drone_amd import gcn
+    widths, lds, first, n_rows, n_cols, mean = CASES[name]
+    rng = np.random.default_rng(len(name))
+    lengths = rng.poisson(mean, n_rows)
+    lengths[rng.integers(0, n_rows, 9)] = [0, 0, 1, 64, 65, 129, 512, 513, 1300]
+    lengths = np.minimum(lengths, n_cols)
+    indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    # distinct columns of a row: a start, and steps that do not come round
+    cols = np.concatenate([np.sort((int(rng.integers(n_cols)) + np.arange(d) * max(1, n_cols // max(d, 1))) % n_cols) for d in lengths])
+    m = sp.csr_matrix((rng.uniform(-1, 1, indptr[-1]).astype(np.float32), cols.astype(np.int32), indptr), shape=(n_rows, n_cols))
+    m64, mabs = m.astype(np.float64), abs(m).astype(np.float64)
+    rp, ci, v = (torch.from_numpy(a).cuda() for a in (indptr, m.indices, m.data))
+    for ld in lds:
+        room = rng.uniform(-1, 1, n_cols * ld + first).astype(np.float32)
+        C0 = rng.uniform(-1, 1, n_rows * ld + first).astype(np.float32)
+        B = np.lib.stride_tricks.as_strided(room[first:], (n_cols, ld), (4 * ld, 4))
+        Bd = torch.from_numpy(room).cuda()[first:].as_strided((n_cols, ld), (ld, 1))
+        for K in (k for k in widths if k <= ld):
+            plan = gcn.SpmmPlan(rp, ci, v, n_cols, max_k=K)
+            want, scale = m64 @ B[:, :K].astype(np.float64), mabs @ np.abs(B[:, :K].astype(np.float64))
+            for beta in (0.0, -0.5):
+                whole = torch.from_numpy(C0.copy()).cuda()
+                out = whole[first:].as_strided((n_rows, ld), (ld, 1))
+                gcn.spmm(plan, rp, ci, v, Bd, K=K, out=out, alpha=1.5, beta=beta)
+                got = whole.cpu().numpy()
+                before = C0[first:].reshape(n_rows, ld)
+                after = got[first:].reshape(n_rows, ld)
+                np.testing.assert_array_equal(got[:first], C0[:first])
+                np.testing.assert_array_equal(after[:, K:], before[:, K:])
+                # chains of at most 1,300 entries, a rounding of 2^-24 of the sum of magnitudes each, twice over for scaling
+                bound = 1.5 * scale + 0.5 * np.abs(before[:, :K]) + 1e-30
+                assert np.max(np.abs(after[:, :K] - (1.5 * want + beta * before[:, :K])) / bound) <= 1.6e-4, (ld, K, beta)
+            plan.close()
+
+
+@pytest.mark.parametrize("K,ld", [(6, 7), (41, 41), (97, 99), (127, 128), (128, 128), (131, 131), (250, 251)])
+def test_bits_at_any_alignment(monkeypatch, K, ld):
+    """A pattern with a dense corner, kept as bits, whatever the alignment of the rows."""
+    import torch
+    from drone_amd import gcn
+    monkeypatch.setenv("DRONE_SPMM_DENSE_MIN_GAIN_MS", "0")
+    rng = np.random.default_rng(K)
+    n = 5000
+    dense = sp.random(1500, n, 0.25, format="csr", random_state=3)
+    m = sp.vstack([dense, sp.random(n - 1500, n, 0.002, format="csr", random_state=4)]).tocsr()
+    m.sort_indices()
+    rows, colscale = rng.uniform(0.5, 1, n).astype(np.float32), rng.uniform(0.5, 1, n).astype(np.float32)
+    val = (np.repeat(rows, np.diff(m.indptr)) * colscale[m.indices]).astype(np.float32)
+    m = sp.csr_matrix((val, m.indices, m.indptr), shape=m.shape)
+    rp, ci, v, rs, cs = (torch.from_numpy(np.ascontiguousarray(a)).cuda()
+                         for a in (m.indptr.astype(np.int32), m.indices.astype(np.int32), m.data, rows, colscale))
+    B, C0 = (rng.uniform(-1, 1, (n, ld)).astype(np.float32) for _ in range(2))
+    Bd = torch.from_numpy(B).cuda()
+    plan = gcn.SpmmPlan(rp, ci, v, n, max_k=K, row_scale=rs, col_scale=cs)
+    assert plan.bit_core()["cells"] > 0
+    m64 = m.astype(np.float64)
+    want, scale = m64 @ B[:, :K].astype(np.float64), m64 @ np.abs(B[:, :K].astype(np.float64))
+    for beta in (0.0, 2.0):
+        out = torch.from_numpy(C0.copy()).cuda()
+        gcn.spmm(plan, rp, ci, v, Bd, K=K, out=out, alpha=0.75, beta=beta)
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(got[:, K:], C0[:, K:])
+        bound = 0.75 * scale + abs(beta) * np.abs(C0[:, :K])
+        # 1,250 entries a row: as many roundings of 2^-24
+        assert np.max(np.abs(got[:, :K] - (0.75 * want + beta * C0[:, :K])) / bound) <= 1.5e-4, beta
+    plan.close()
