@@ -20,6 +20,10 @@
 // 0.13 ... 1.2 ms instead of 0.3 ... 2.7 ms.  Below 16 K vertices it is a launch (2.3 us) plus one chain of slice
 // descriptor, ids, gathers and the partials' sum out of a cold L2; at 64 K and more the rate of gathers that hit L2.
 // Lanes of 4 or 16 entries (kSellDepth) instead of 8: 10.0 / 9.3 us at 64 K.
+//
+// Larger matrices whose hubs are named often enough keep the first kSellHot sources - rows of many entries are named often, so
+// they come first - in every CU's LDS (sell_iterate_hot_kernel): 131 K 14.2 -> 11.9, 262 K 24.3 -> 18.5, 524 K 41.3 -> 37.8, 0.4 M
+// vertices and 7.0 M entries 35.7 -> 33.1.  What is left is the rate of the other gathers.
 #pragma once
 #include "common.h"
 
@@ -28,10 +32,12 @@ namespace drone {
 constexpr int kSellClasses = 7;      // P = 64, 32, ..., 1
 constexpr int kSellDepth = 8;        // most entries of a lane in a slice with P < 64; gathers in flight per lane
 constexpr int kSellWaveSteps = 16;   // most steps of a slice with P = 64: longer rows are hubs
+constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,008 of 163,840 bytes
 
 struct SellRows {
     int64_t n = 0, nnz = 0;
-    int threads = 256;               // work-group size of the iteration, 256 or 512
+    int threads = 256;               // work-group size of the iteration, 256 or 512; 1,024 with the hot sources in LDS
+    bool hot = false;                // sell_iterate_hot_kernel: ids from kSellHot on are one more, and kSellHot is the padding
     int hubs = 0, slices = 0, blocks = 0;
     int row_begin[kSellClasses + 1] = {};    // first row of the class (row_begin[kSellClasses] = n)
     int slice_begin[kSellClasses + 1] = {};  // first slice of the class

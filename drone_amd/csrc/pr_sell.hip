@@ -9,14 +9,23 @@
 namespace drone {
 namespace {
 
-// Up to here (rows + entries) the layout beats the row blocks: at 8.5 M items 41.3 against 43.8 us per iteration, at 17 M
-// (8 MB of gather source, twice an XCD's L2) the row blocks' sorted gathers take 63.8 and this path has nothing to offer.
+// Up to here (rows + entries) the layout beats the row blocks: at 8.5 M items 37.8 (41.3 without sources in LDS) against 43.8 us
+// per iteration, at 17 M (8 MB of gather source, twice an XCD's L2) 73.7 against the 63.8 of the row blocks' sorted gathers.
 constexpr int64_t kSellMaxItems = 9 << 20;
 // Work-groups of 256 / 512 / 1,024 lanes, us per iteration at 0.012 / 0.057 / 1.02 / 2.07 / 4.2 / 8.5 M items: 4.05 / 4.7 /
 // 9.1 / 14.6 / 24.2 / 51.5, 4.2 / 5.1 / 9.6 / 14.1 / 24.3 / 41.3, 5.3 / 6.3 / 12.2 / 14.5 / 21.1 / 43.4: small ones for small
 // matrices (more CUs at work), 512 once the partials of so many work-groups and the hub rows count.
 constexpr int64_t kSellWideItems = 1200 << 10;
 constexpr int kSellInitThreads = 256, kSellInitBlocks = 512;
+// From kSellWideItems on the hottest sources sit in LDS, if that many of the entries name one of them (of kSellSamples
+// looked at): us per iteration without / with, and the share, 2.0 M items (131,072 vertices) 14.1 / 11.9 at 0.89, 4.2 M 24.2 / 18.5 at
+// 0.79, 8.5 M 41.3 / 37.8 at 0.71, 1 M vertices and 7.8 M entries 45.3 / 40.6 at 0.63; half as many sources in LDS 41.3 / 44.0 at
+// 0.57, 45.3 / 45.8 at 0.50.  Bringing 160 KB into every CU's LDS takes 3 us whatever there is to do: 1.0 M items 9.0 / 9.6.
+constexpr double kSellHotShare = 0.6;
+constexpr int kSellSamples = 1 << 16;
+constexpr int kSellHotThreads = 1024, kSellHotBlocks = 256;
+constexpr size_t kSellHotLds = sizeof(double) * kSellHot;
+static_assert(kSellInitBlocks <= kSellHotThreads && kSellHot % 2 == 0, "a partial per lane; pairs");
 constexpr int kSellMassLoads = 4;  // partials of the dangling mass per lane that are requested ahead
 
 // What a kernel needs of SellRows, by value.
@@ -138,6 +147,106 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
     if (tid == 0) part_out[blockIdx.x] = total;
 }
 
+// Sum of the sources of `steps` consecutive steps of T ids from `ids` on (this lane's), the first kSellDepth of which are there already.
+// Both kinds of load are under the lanes' own condition: a hot lane costs the L1 nothing.
+template <int T>
+__device__ __forceinline__ double sell_hot_sum(int (&id)[kSellDepth], const int32_t *__restrict__ ids, int steps,
+                                               const double *s_hot, const double *__restrict__ c_in)
+{
+    double sum = 0.0;
+    for (int s = 0;;) {
+        double v[kSellDepth];
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) {
+            v[k] = 0.0;
+            if (id[k] > kSellHot) v[k] = c_in[id[k] - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k)
+            if (id[k] < kSellHot) v[k] = s_hot[id[k]];
+        s += kSellDepth;
+        if (s < steps) {
+#pragma unroll
+            for (int k = 0; k < kSellDepth; ++k) id[k] = s + k < steps ? ids[(size_t)(s + k) * T] : kSellHot;
+        }
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) sum += v[k];
+        if (s >= steps) return sum;
+    }
+}
+
+// One iteration with the hottest sources in LDS; one work-group per CU, the slices dealt out to the wavefronts of all.
+__global__ __launch_bounds__(kSellHotThreads) void sell_iterate_hot_kernel(
+    int n, int hubs, int slices, const int32_t *__restrict__ hub_step, const int32_t *__restrict__ hub_col,
+    const int4 *__restrict__ slice, const int32_t *__restrict__ col, const double *__restrict__ c_in,
+    const double *__restrict__ inv, double *__restrict__ c_out, const double *__restrict__ part_in, int parts,
+    double *__restrict__ part_out, double alpha, double inv_n, const int32_t *__restrict__ order, double *__restrict__ r_out)
+{
+    constexpr int T = kSellHotThreads;
+    extern __shared__ double s_hot[];  // [kSellHot]
+    __shared__ double s_dang[T / kWave], s_red[T / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int stride = (int)gridDim.x * (T / kWave);
+    // The first slice's ids, and the dangling mass, travel beside the hot sources.
+    int s = (int)blockIdx.x + (int)gridDim.x * wave;
+    int4 d = s < slices ? slice[s] : make_int4(0, 0, 0, 0);
+    int id[kSellDepth];
+    const auto fetch = [&](int4 what, int (&to)[kSellDepth]) {
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) to[k] = k < what.y ? col[((size_t)what.x + k) * kWave + lane] : kSellHot;
+    };
+    fetch(d, id);
+    const double mass = tid < parts ? part_in[tid] : 0.0;
+    const int hot = n < kSellHot ? n : kSellHot;
+    const double2 *c2 = reinterpret_cast<const double2 *>(c_in);
+    constexpr int kPieces = (kSellHot / 2 + T - 1) / T;
+    const int rot = ((int)blockIdx.x / 8) % kPieces;  // work-groups of an XCD would all ask one L2 channel for the same line: 2 M items 13.3 -> 11.9 us
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k) {
+        const int i = tid + (k + rot < kPieces ? k + rot : k + rot - kPieces) * T;
+        if (2 * i + 1 < hot) reinterpret_cast<double2 *>(s_hot)[i] = c2[i];
+        else if (2 * i < hot) s_hot[2 * i] = c_in[2 * i];
+    }
+    const double dang = block_sum<T>(mass, s_dang);
+    const double base = (1.0 - alpha) * inv_n + alpha * dang * inv_n;
+    double stat = 0.0;
+    const auto finish = [&](int row, double iv, double sum) {
+        const double rn = base + alpha * sum;
+        c_out[row] = rn * iv;
+        if (r_out) r_out[order[row]] = rn;
+        if (iv == 0.0) stat += rn;
+    };
+    for (int h = blockIdx.x; h < hubs; h += gridDim.x) {
+        const int s0 = hub_step[h], s1 = hub_step[h + 1];
+        const double iv = inv[h];
+        const int32_t *ids = hub_col + (size_t)s0 * T + tid;
+        int hub_id[kSellDepth];
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) hub_id[k] = s0 + k < s1 ? ids[(size_t)k * T] : kSellHot;
+        const double sum = block_sum<T>(sell_hot_sum<T>(hub_id, ids, s1 - s0, s_hot, c_in), s_red);
+        if (tid == 0) finish(h, iv, sum);
+        __syncthreads();  // s_red is used again
+    }
+    while (s < slices) {
+        const int next = s + stride;
+        const int4 after = next < slices ? slice[next] : make_int4(0, 0, 0, 0);
+        const int lanes_log = d.w & 7, lanes = 1 << lanes_log, r = lane >> lanes_log;
+        const bool mine = (lane & (lanes - 1)) == 0 && r < (d.w >> 3);
+        const double iv = mine ? inv[d.z + r] : 0.0;
+        int id_after[kSellDepth];
+        fetch(after, id_after);
+        double sum = sell_hot_sum<kWave>(id, col + (size_t)d.x * kWave + lane, d.y, s_hot, c_in);
+        for (int m = lanes >> 1; m > 0; m >>= 1) sum += __shfl_xor(sum, m, kWave);
+        if (mine) finish(d.z + r, iv, sum);
+        d = after;
+        s = next;
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) id[k] = id_after[k];
+    }
+    const double total = block_sum<T>(stat, s_red);
+    if (tid == 0) part_out[blockIdx.x] = total;
+}
+
 // ---- building the layout ---------------------------------------------------------------------------------------------
 __global__ void sell_lengths_kernel(int n, const int64_t *__restrict__ row_ptr, unsigned *__restrict__ len, int32_t *__restrict__ id)
 {
@@ -147,7 +256,7 @@ __global__ void sell_lengths_kernel(int n, const int64_t *__restrict__ row_ptr, 
     }
 }
 
-// new_id of every vertex; bounds[k] = rows (longest first) with more than limit[k] entries, bounds[kSellClasses] = longest
+// new_id of every vertex; bounds[k] = rows (longest first) with more than limit[k] entries
 __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorted, const int32_t *__restrict__ order,
                                    int hub_limit, int32_t *__restrict__ new_id, int *__restrict__ bounds)
 {
@@ -162,8 +271,17 @@ __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorte
         }
         bounds[threadIdx.x] = lo;
     } else if (threadIdx.x == kSellClasses) {
-        bounds[kSellClasses] = n > 0 ? (int)len_sorted[0] : 0;
+        bounds[kSellClasses] = 0;  // for sell_sample_kernel
     }
+}
+
+// *named += entries, of kSellSamples from all over the matrix, whose source is one of the first kSellHot
+__global__ __launch_bounds__(256) void sell_sample_kernel(int64_t nnz, const int32_t *__restrict__ col, const int32_t *__restrict__ new_id,
+                                                          int *__restrict__ named)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const unsigned long long hot = __ballot(new_id[col[(int64_t)((double)i / kSellSamples * (double)nnz)]] < kSellHot);
+    if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(named, __popcll(hot));
 }
 
 __device__ __forceinline__ void sell_slice_rows(const SellShape &sh, int s, int &k, int &first_row, int &last_row)
@@ -199,12 +317,17 @@ __global__ __launch_bounds__(256) void sell_fill_kernel(SellShape sh, int thread
                                                         const int32_t *__restrict__ new_id,
                                                         const int32_t *__restrict__ hub_step,
                                                         const int32_t *__restrict__ slice_step, int4 *__restrict__ slice,
-                                                        int32_t *__restrict__ hub_out, int32_t *__restrict__ out)
+                                                        int32_t *__restrict__ hub_out, int32_t *__restrict__ out, bool hot)
 {
+    const auto source = [&](bool there, int64_t e) {
+        if (!there) return hot ? kSellHot : sh.n;
+        const int id = new_id[col[e]];
+        return id + (hot && id >= kSellHot);
+    };
     if ((int)blockIdx.x < sh.hubs) {
         const int64_t e0 = row_ptr[order[blockIdx.x]], e1 = row_ptr[order[blockIdx.x] + 1];
         const int64_t at = (int64_t)hub_step[blockIdx.x] * threads, count = (int64_t)hub_step[blockIdx.x + 1] * threads - at;
-        for (int64_t i = threadIdx.x; i < count; i += 256) hub_out[at + i] = e0 + i < e1 ? new_id[col[e0 + i]] : sh.n;
+        for (int64_t i = threadIdx.x; i < count; i += 256) hub_out[at + i] = source(e0 + i < e1, e0 + i);
         return;
     }
     const int s = ((int)blockIdx.x - sh.hubs) * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
@@ -220,7 +343,7 @@ __global__ __launch_bounds__(256) void sell_fill_kernel(SellShape sh, int thread
     const int st0 = slice_step[s], st1 = slice_step[s + 1], rows = last_row - first_row < (1 << k) ? last_row - first_row : 1 << k;
     if (lane == 0) slice[s] = make_int4(st0, st1 - st0, first_row, rows << 3 | (6 - k));
     for (int st = st0; st < st1; ++st, e0 += lanes)
-        out[(size_t)st * kWave + lane] = e0 < e1 ? new_id[col[e0]] : sh.n;
+        out[(size_t)st * kWave + lane] = source(e0 < e1, e0);
 }
 
 SellShape shape_of(const SellRows &sr)
@@ -289,8 +412,14 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
         need = temp_bytes;
         DRONE_HIP_TRY(rocprim::radix_sort_pairs_desc(temp, need, len, len_sorted, ids, sr->order, cnt, 0, key_bits, s));
         sell_bounds_kernel<<<grid, 256, 0, s>>>((int)n, len_sorted, sr->order, hub_limit, new_id, bounds);
+        if (n + nnz > kSellWideItems && nnz >= kSellSamples) sell_sample_kernel<<<kSellSamples / 256, 256, 0, s>>>(nnz, col, new_id, bounds + kSellClasses);
         DRONE_HIP_TRY(hipMemcpyAsync(h, bounds, sizeof(int) * (kSellClasses + 1), hipMemcpyDeviceToHost, s));
         DRONE_HIP_TRY(hipStreamSynchronize(s));
+        if (h[kSellClasses] >= kSellHotShare * kSellSamples) {
+            sr->hot = true;
+            sr->threads = kSellHotThreads;
+            DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&sell_iterate_hot_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSellHotLds));
+        }
         sr->hubs = h[0];
         for (int k = 0; k < kSellClasses; ++k) {
             sr->row_begin[k] = h[k];
@@ -300,7 +429,7 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
         sr->row_begin[kSellClasses] = (int)n;
         sr->slices = sr->slice_begin[kSellClasses];
         DRONE_REQUIRE((size_t)sr->slices <= most_slices && (size_t)sr->hubs <= most_hubs, "slice bound");
-        sr->blocks = sr->hubs + (int)ceil_div(sr->slices, sr->threads / kWave);
+        sr->blocks = sr->hot ? kSellHotBlocks : sr->hubs + (int)ceil_div(sr->slices, sr->threads / kWave);
         sr->init_blocks = (int)std::min<int64_t>(ceil_div(n, kSellInitThreads), kSellInitBlocks);
         const SellShape sh = shape_of(*sr);
         sell_steps_kernel<<<(int)ceil_div(std::max(sr->slices, sr->hubs) + 1, 256), 256, 0, s>>>(sh, sr->threads, len_sorted, hub_steps, slice_steps);
@@ -315,7 +444,7 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
         sr->entries.want(&sr->col, (size_t)h[1] * kWave);
         DRONE_HIP_TRY(sr->entries.commit());
         sell_fill_kernel<<<sr->hubs + (int)ceil_div(sr->slices, 256 / kWave), 256, 0, s>>>(
-            sh, sr->threads, sr->order, row_ptr, col, new_id, sr->hub_step, slice_step, sr->slice, sr->hub_col, sr->col);
+            sh, sr->threads, sr->order, row_ptr, col, new_id, sr->hub_step, slice_step, sr->slice, sr->hub_col, sr->col, sr->hot);
         DRONE_HIP_TRY(hipGetLastError());
         DRONE_HIP_TRY(hipStreamSynchronize(s));  // the temporaries go next
         return DRONE_OK;
@@ -345,13 +474,14 @@ int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t s)
 int sell_iterate(const SellRows &sr, int it, double alpha, double *rank_out, hipStream_t s)
 {
     const int parts = it == 0 ? sr.init_blocks : sr.blocks, now = it & 1;
-    const auto launch = [&](auto kernel) {
-        kernel<<<sr.blocks, sr.threads, 0, s>>>((int)sr.n, sr.hubs, sr.slices, sr.hub_step, sr.hub_col, sr.slice, sr.col, sr.c[now], sr.inv,
+    const auto launch = [&](auto kernel, size_t lds) {
+        kernel<<<sr.blocks, sr.threads, lds, s>>>((int)sr.n, sr.hubs, sr.slices, sr.hub_step, sr.hub_col, sr.slice, sr.col, sr.c[now], sr.inv,
                                                 sr.c[now ^ 1], sr.part[now], parts, sr.part[now ^ 1], alpha,
                                                 1.0 / (double)sr.n, sr.order, rank_out);
     };
-    if (sr.threads == 512) launch(sell_iterate_kernel<512>);
-    else launch(sell_iterate_kernel<256>);
+    if (sr.hot) launch(sell_iterate_hot_kernel, kSellHotLds);
+    else if (sr.threads == 512) launch(sell_iterate_kernel<512>, 0);
+    else launch(sell_iterate_kernel<256>, 0);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
