@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "pr_rowblock.h"
+#include "pr_sell.h"
 #include "relabel.h"
 #include "spmv_merge.h"
 
@@ -97,6 +98,11 @@ struct GraphExt {
     RowBlocks rb;             // over the in-edge CSR with its sources renumbered hot-first
     MergeScratch ms_rb;
     int32_t *rb_new_id = nullptr;  // device [n]: local id -> renumbered id (where a vertex's push value is kept)
+    // mid-size subgraphs: sliced rows with the hottest sources in LDS (pr_sell.h, built by loadOutDegree); numbered by rb_new_id as well
+    bool sell_tried = false, sell_ready = false;
+    SellRows sell;
+    double *sell_part = nullptr;       // device [kSellHotBlocks]
+    unsigned int *sell_ticket = nullptr;  // device [ticket_words(kSellHotBlocks)], zero between launches
     // fp64 pull run driven from the Graph
     drone_pr_plan *plan64 = nullptr;
     int64_t *row_ptr64 = nullptr;

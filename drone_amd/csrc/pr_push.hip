@@ -3,6 +3,7 @@
 // a vertex kernel decides what every vertex pushes this superstep (push[u] = delta/outdeg, or 0 when
 // the change is below eps), and the merge-path aggregation pulls diff[v] = sum of push[u] over the
 // in-edges of v together with the number of non-zero pushes, which gives g->active and VisitedSize.
+#include <algorithm>
 #include <chrono>
 #include <cstdlib>
 
@@ -95,25 +96,50 @@ __global__ __launch_bounds__(kSpmvBlock) void pr_increment_vertex_kernel(
     __shared__ double s_red[kSpmvBlock / kWave];
     const float ga = *global_acc + *global_diff;
     double part = 0.0;
-    for (int id = blockIdx.x * kSpmvBlock + threadIdx.x; id < n; id += gridDim.x * kSpmvBlock) {
-        update_by_message[id] = 0;
-        const float a = acc[id] + diff[id];
-        acc[id] = a;
-        const float old = pr[id];
+    // the value vertex id pushes; its rank is updated
+    const auto advance = [&](int id, float a, int od, float &rank) {
+        const float old = rank;
         const float p = kAlpha * (a + ga) + (1 - kAlpha);
         float d = p - old;
         if (d < 0) d = -d;
         float out = 0.0f;
         if (!(d < kEps)) {
-            const int od = outdeg[id];
             if (od == 0) {
                 if (m2w[id] == -1) part += (double)((p - old) / (float)nglobal);
             } else {
                 out = (p - old) / (float)od;
             }
-            pr[id] = p;
+            rank = p;
         }
-        push[push_slot ? push_slot[id] : id] = out;
+        return out;
+    };
+    // Four vertices a lane, their loads in flight together (the arrays start where hipMalloc put them): ten supersteps of 900,001 vertices
+    // 717 -> 705 us, of 2,000 vertices 291 -> 281.
+    const int quads = n / 4;
+    for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += gridDim.x * kSpmvBlock) {
+        float4 a = reinterpret_cast<const float4 *>(acc)[i], rank = reinterpret_cast<const float4 *>(pr)[i];
+        const float4 df = reinterpret_cast<const float4 *>(diff)[i];
+        const int4 od = reinterpret_cast<const int4 *>(outdeg)[i];
+        const int4 slot = push_slot ? reinterpret_cast<const int4 *>(push_slot)[i] : make_int4(4 * i, 4 * i + 1, 4 * i + 2, 4 * i + 3);
+        a = make_float4(a.x + df.x, a.y + df.y, a.z + df.z, a.w + df.w);
+        const float4 out = make_float4(advance(4 * i, a.x, od.x, rank.x), advance(4 * i + 1, a.y, od.y, rank.y),
+                                       advance(4 * i + 2, a.z, od.z, rank.z), advance(4 * i + 3, a.w, od.w, rank.w));
+        reinterpret_cast<int4 *>(update_by_message)[i] = make_int4(0, 0, 0, 0);
+        reinterpret_cast<float4 *>(acc)[i] = a;
+        reinterpret_cast<float4 *>(pr)[i] = rank;
+        push[slot.x] = out.x;
+        push[slot.y] = out.y;
+        push[slot.z] = out.z;
+        push[slot.w] = out.w;
+    }
+    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) {
+        const int id = 4 * quads + threadIdx.x;
+        const float a = acc[id] + diff[id];
+        update_by_message[id] = 0;
+        acc[id] = a;
+        float rank = pr[id];
+        push[push_slot ? push_slot[id] : id] = advance(id, a, outdeg[id], rank);
+        pr[id] = rank;
     }
     const double total = block_sum_256(part, s_red);
     // The last work-group reads block_part[] and nothing else the others wrote: only what went through publish_part is
@@ -214,6 +240,44 @@ __global__ void invert_order_kernel(const int32_t *__restrict__ order, int n, in
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) new_id[order[i]] = i;
 }
 
+void sell_rows_release(GraphExt *x)
+{
+    sell_destroy(&x->sell);
+    (void)hipFree(x->sell_part);
+    (void)hipFree(x->sell_ticket);
+    (void)hipFree(x->rb_new_id);
+    x->sell_part = nullptr;
+    x->sell_ticket = nullptr;
+    x->rb_new_id = nullptr;
+    x->sell_ready = false;
+}
+
+// Sliced rows with the hottest sources in LDS (sell_push_kernel), once per graph, where there are enough edges and enough of them lead
+// from these.  A superstep of 900,001 vertices and 13.5 M edges, merge path / these: 99 / 70 us; 0.4 M vertices and 6 M edges 59 / 46, 2 M
+// and 15 M 125 / 107, 0.3 M and 3.5 M 42 / 42.  Building them takes about 1 ms, which such a job has back after 40 supersteps; it
+// belongs to what is prepared for PageRank, so loadOutDegree does it, not the first superstep (1.37 -> 1.05 ms of ten).  Any failure (memory) leaves the
+// merge path in place.
+void ensure_sell_rows(Graph *g, hipStream_t s)
+{
+    GraphExt *x = static_cast<GraphExt *>(g->ext);
+    if (x->sell_tried || x->edges >= std::min(row_block_min_edges(), kRowBlockMinEdges) || !sell_f32_suits(x->n, x->edges)) return;
+    x->sell_tried = true;
+    int rc = DRONE_OK;
+    const size_t words = ticket_words(kSellHotBlocks);
+    if (hipMalloc(&x->rb_new_id, sizeof(int32_t) * (size_t)x->n) != hipSuccess) rc = DRONE_ERR_HIP;
+    if (rc == DRONE_OK) rc = sell_create_f32(&x->sell, x->n, x->edges, x->in_index, x->in_src, x->rb_new_id, s);
+    if (rc == DRONE_OK && x->sell.hot &&
+        (hipMalloc(&x->sell_part, sizeof(double) * kSellHotBlocks) != hipSuccess || hipMalloc(&x->sell_ticket, sizeof(unsigned int) * words) != hipSuccess ||
+         hipMemsetAsync(x->sell_ticket, 0, sizeof(unsigned int) * words, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess))
+        rc = DRONE_ERR_HIP;
+    if (rc != DRONE_OK || !x->sell.hot) {
+        sell_rows_release(x);
+        clear_error();
+        return;
+    }
+    x->sell_ready = true;
+}
+
 // Builds, once per graph, the row blocks of the in-edge CSR with its sources renumbered hot-first (most gathered
 // first, so the popular push values share few cache lines).  Rows keep their local ids, so diff / active and
 // everything the caller and the exchange see stay in local order; only the push vector is kept in the renumbered
@@ -226,9 +290,12 @@ __global__ void invert_order_kernel(const int32_t *__restrict__ order, int n, in
 void ensure_row_blocks(Graph *g, hipStream_t s)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
-    if (x->rb_tried) return;
+    if (x->rb_tried || x->sell_ready) return;
     x->rb_tried = true;
-    if (x->edges < row_block_min_edges() || x->edges == 0) return;
+    if (x->edges < row_block_min_edges() || x->edges == 0) {
+        ensure_sell_rows(g, s);
+        return;
+    }
     int64_t *row_ptr = nullptr;
     Relabel rl;
     int rc = DRONE_OK;
@@ -269,7 +336,7 @@ void ensure_row_blocks(Graph *g, hipStream_t s)
 const int32_t *push_slot_of(Graph *g)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
-    return x->rb_ready ? x->rb_new_id : nullptr;
+    return x->rb_ready || x->sell_ready ? x->rb_new_id : nullptr;
 }
 
 int aggregate_push(Graph *g, PRValues *values, hipStream_t s)
@@ -291,6 +358,11 @@ int aggregate_push(Graph *g, PRValues *values, hipStream_t s)
         spmv_fixup_kernel<PushF2, PushEpi, StoreStat><<<fb, kSpmvBlock, 0, s>>>(
             rb.num_blocks, rb.block_row, rb.walk_len, carry, x->ms_rb.tile_stat, epi, x->ms_rb.block_stat,
             x->ms_rb.ticket, StoreStat{px->stat, px->stat_host});
+    } else if (x->sell_ready) {
+        if (sell_push(x->sell, px->push, values->diffValue, g->active, x->sell_part, x->sell_ticket, StoreStat{px->stat, px->stat_host}, s) != DRONE_OK) {
+            printf("Failed: %s\n", drone_last_error_string());
+            exit(EXIT_FAILURE);
+        }
     } else {
         spmv_merge_launch<PushF2, int, kPushIpt, PushEpi>(x->mt, x->ms, x->in_index, x->in_src, epi, px->stat, s,
                                                           px->stat_host);
@@ -310,7 +382,7 @@ void drone::graph_ext_release(GraphExt *x)
     merge_scratch_destroy(&x->ms);
     row_blocks_destroy(&x->rb);
     merge_scratch_destroy(&x->ms_rb);
-    (void)hipFree(x->rb_new_id);
+    sell_rows_release(x);
     if (x->plan64) (void)drone_pr_plan_destroy(x->plan64);
     if (x->row_ptr64) (void)hipFree(x->row_ptr64);
     if (x->inv64) (void)hipFree(x->inv64);
@@ -337,6 +409,7 @@ extern "C" void loadOutDegree(Graph *g, PRValues *values, int *globalOutDegree)
     set_out_degree_kernel<<<1024, 256>>>(values->outDegree, d_global, g->Local2Global, n);
     DRONE_HIP_OR_DIE(hipDeviceSynchronize());
     (void)hipFree(d_global);
+    ensure_sell_rows(g, nullptr);
 }
 
 extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm)
@@ -353,8 +426,8 @@ extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int worke
         printf("Failed: PR_PEVal before loadOutDegree\n");
         exit(EXIT_FAILURE);
     }
-    ensure_aggregation_ready(g);
     ensure_row_blocks(g, s);  // before the first vertex kernel: it decides where push values are kept
+    if (!push_slot_of(g)) ensure_aggregation_ready(g);
     // pr.cu:383-389: the state vectors are allocated by this call
     if (!g->active) DRONE_HIP_OR_DIE(hipMalloc(&g->active, sizeof(int) * cnt));
     if (!g->updateByMessage) DRONE_HIP_OR_DIE(hipMalloc(&g->updateByMessage, sizeof(int) * cnt));
@@ -394,7 +467,9 @@ extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int worke
 
 extern "C" int drone_pr_aggregation(const Graph *g)
 {
-    return g && g->ext && static_cast<const GraphExt *>(g->ext)->rb_ready ? 1 : 0;
+    if (!g || !g->ext) return 0;
+    const GraphExt *x = static_cast<const GraphExt *>(g->ext);
+    return x->rb_ready ? 1 : x->sell_ready ? 2 : 0;
 }
 
 extern "C" Response PR_IncEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm)

@@ -22,22 +22,24 @@
 // Lanes of 4 or 16 entries (kSellDepth) instead of 8: 10.0 / 9.3 us at 64 K.
 //
 // Larger matrices whose hubs are named often enough keep the first kSellHot sources - rows of many entries are named often, so
-// they come first - in every CU's LDS (sell_iterate_hot_kernel): 131 K 14.2 -> 11.9, 262 K 24.3 -> 18.5, 524 K 41.3 -> 37.8, 0.4 M
-// vertices and 7.0 M entries 35.7 -> 33.1.  What is left is the rate of the other gathers.
+// they come first - in every CU's LDS (sell_iterate_hot_kernel): 131 K 14.2 -> 11.8, 262 K 24.3 -> 18.1, 524 K 41.3 -> 37.0, 0.4 M
+// vertices and 7.0 M entries 35.7 -> 33.  What is left is the rate of the other gathers, and a round trip or two per slice
+// (deeper lanes, 16 instead of 8 entries: 11.1 / 18.0 / 38.4 with an id array of their own; floats, whose rows are longer, have 16).
 #pragma once
-#include "common.h"
+#include "spmv_merge.h"
 
 namespace drone {
 
 constexpr int kSellClasses = 7;      // P = 64, 32, ..., 1
 constexpr int kSellDepth = 8;        // most entries of a lane in a slice with P < 64; gathers in flight per lane
 constexpr int kSellWaveSteps = 16;   // most steps of a slice with P = 64: longer rows are hubs
-constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,008 of 163,840 bytes
+constexpr int kSellDepthF32 = 16, kSellWaveStepsF32 = 32;  // the same of float rows
+constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,000 of 163,840 bytes
 
 struct SellRows {
     int64_t n = 0, nnz = 0;
     int threads = 256;               // work-group size of the iteration, 256 or 512; 1,024 with the hot sources in LDS
-    bool hot = false;                // sell_iterate_hot_kernel: ids from kSellHot on are one more, and kSellHot is the padding
+    int hot = 0;                     // sources kept in LDS, or 0: ids from there on are one more, and that number is the padding
     int hubs = 0, slices = 0, blocks = 0;
     int row_begin[kSellClasses + 1] = {};    // first row of the class (row_begin[kSellClasses] = n)
     int slice_begin[kSellClasses + 1] = {};  // first slice of the class
@@ -57,6 +59,15 @@ struct SellRows {
 // Whether the layout suits the matrix (n rows, nnz entries).
 bool sell_suits(int64_t n, int64_t nnz);
 int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, const int32_t *col, hipStream_t stream);
+// The rows alone, for float sources of which a work-group keeps kSellHotF32: sr->hot is 0, and nothing built, where the entries name
+// too few of them.  Fills `order` and the entries, and new_id (device [n]): caller's id -> source.
+constexpr int kSellHotF32 = 2 * kSellHot;
+bool sell_f32_suits(int64_t n, int64_t nnz);
+int sell_create_f32(SellRows *sr, int64_t n, int64_t nnz, const int *row_ptr, const int32_t *col, int32_t *new_id, hipStream_t stream);
+constexpr int kSellHotThreads = 1024, kSellHotBlocks = 256;
+// One superstep's aggregation over it.  part, ticket: device [kSellHotBlocks] and [ticket_words(kSellHotBlocks)].
+int sell_push(const SellRows &sr, const float *push, float *diff, int *active, double *part, unsigned int *ticket, const StoreStat &stat,
+              hipStream_t stream);
 void sell_destroy(SellRows *sr);
 // The two kinds of launch of a run: sell_begin reads the caller's inverse out-degrees, makes the first gather source and
 // its dangling mass; sell_iterate is one iteration (it = 0, 1, ...), the last of which passes rank_out.

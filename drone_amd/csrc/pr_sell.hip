@@ -9,7 +9,7 @@
 namespace drone {
 namespace {
 
-// Up to here (rows + entries) the layout beats the row blocks: at 8.5 M items 37.8 (41.3 without sources in LDS) against 43.8 us
+// Up to here (rows + entries) the layout beats the row blocks: at 8.5 M items 37.0 (41.3 without sources in LDS) against 43.8 us
 // per iteration, at 17 M (8 MB of gather source, twice an XCD's L2) 73.7 against the 63.8 of the row blocks' sorted gathers.
 constexpr int64_t kSellMaxItems = 9 << 20;
 // Work-groups of 256 / 512 / 1,024 lanes, us per iteration at 0.012 / 0.057 / 1.02 / 2.07 / 4.2 / 8.5 M items: 4.05 / 4.7 /
@@ -17,15 +17,17 @@ constexpr int64_t kSellMaxItems = 9 << 20;
 // matrices (more CUs at work), 512 once the partials of so many work-groups and the hub rows count.
 constexpr int64_t kSellWideItems = 1200 << 10;
 constexpr int kSellInitThreads = 256, kSellInitBlocks = 512;
-// From kSellWideItems on the hottest sources sit in LDS, if that many of the entries name one of them (of kSellSamples
-// looked at): us per iteration without / with, and the share, 2.0 M items (131,072 vertices) 14.1 / 11.9 at 0.89, 4.2 M 24.2 / 18.5 at
-// 0.79, 8.5 M 41.3 / 37.8 at 0.71, 1 M vertices and 7.8 M entries 45.3 / 40.6 at 0.63; half as many sources in LDS 41.3 / 44.0 at
-// 0.57, 45.3 / 45.8 at 0.50.  Bringing 160 KB into every CU's LDS takes 3 us whatever there is to do: 1.0 M items 9.0 / 9.6.
+// From kSellWideItems on the hottest sources sit in LDS, if that many of the entries name one of them (of kSellSamples looked
+// at): us per iteration without / with, and the share, 2.0 M items (131,072 vertices) 14.1 / 11.8 at 0.89, 4.2 M 24.2 / 18.1 at 0.79,
+// 8.5 M 41.3 / 37.0 at 0.71, 1 M vertices and 7.8 M entries 45.3 / 38.2 at 0.63; half as many sources in LDS 41.3 / 44.0 at 0.57,
+// 45.3 / 45.8 at 0.50.  Bringing 160 KB into every CU's LDS takes 3 us whatever there is to do: 1.0 M items 9.0 / 9.6.
 constexpr double kSellHotShare = 0.6;
+// Float rows from here on: see ensure_sell_rows in pr_push.hip for both sides.
+constexpr int64_t kSellF32Items = 4 << 20;
 constexpr int kSellSamples = 1 << 16;
-constexpr int kSellHotThreads = 1024, kSellHotBlocks = 256;
 constexpr size_t kSellHotLds = sizeof(double) * kSellHot;
-static_assert(kSellInitBlocks <= kSellHotThreads && kSellHot % 2 == 0, "a partial per lane; pairs");
+static_assert(kSellInitBlocks <= kSellHotThreads && kSellHotBlocks <= kSellHotThreads, "a partial per lane");
+static_assert(sizeof(float) * kSellHotF32 == kSellHotLds, "the same LDS");
 constexpr int kSellMassLoads = 4;  // partials of the dangling mass per lane that are requested ahead
 
 // What a kernel needs of SellRows, by value.
@@ -34,10 +36,10 @@ struct SellShape {
     int row_begin[kSellClasses + 1], slice_begin[kSellClasses + 1];
 };
 
-// Class of a row of `len` entries: the smallest P with at most kSellDepth entries per lane; class k has P = 64 >> k.
-__host__ __device__ inline int sell_class_limit(int k, int hub_limit)  // longest row of class k
+// Class of a row of `len` entries: the smallest P with at most kSellDepth (kSellDepthF32) entries per lane; class k has P = 64 >> k.
+__host__ __device__ inline int sell_class_limit(int k, bool f32)  // longest row of class k
 {
-    return k == 0 ? hub_limit : (64 >> k) * kSellDepth;
+    return k == 0 ? kWave * (f32 ? kSellWaveStepsF32 : kSellWaveSteps) : (64 >> k) * (f32 ? kSellDepthF32 : kSellDepth);
 }
 
 template <int T>
@@ -147,31 +149,57 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
     if (tid == 0) part_out[blockIdx.x] = total;
 }
 
-// Sum of the sources of `steps` consecutive steps of T ids from `ids` on (this lane's), the first kSellDepth of which are there already.
-// Both kinds of load are under the lanes' own condition: a hot lane costs the L1 nothing.
-template <int T>
-__device__ __forceinline__ double sell_hot_sum(int (&id)[kSellDepth], const int32_t *__restrict__ ids, int steps,
-                                               const double *s_hot, const double *__restrict__ c_in)
+// v[k] = source of id[k], the padding's 0.  Both kinds of load are under the lanes' own condition: a hot lane costs the L1 nothing.
+template <int HOT, int D, typename V>
+__device__ __forceinline__ void sell_hot_gather(const int (&id)[D], const V *s_hot, const V *__restrict__ c_in, V (&v)[D])
 {
-    double sum = 0.0;
-    for (int s = 0;;) {
-        double v[kSellDepth];
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) {
-            v[k] = 0.0;
-            if (id[k] > kSellHot) v[k] = c_in[id[k] - 1];
-        }
+    for (int k = 0; k < D; ++k) {
+        v[k] = V(0);
+        if (id[k] > HOT) v[k] = c_in[id[k] - 1];
+    }
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k)
-            if (id[k] < kSellHot) v[k] = s_hot[id[k]];
-        s += kSellDepth;
-        if (s < steps) {
+    for (int k = 0; k < D; ++k)
+        if (id[k] < HOT) v[k] = s_hot[id[k]];
+}
+
+// Calls add(value) for the sources of steps [s, steps) of T ids from `ids` on (this lane's).
+template <int T, int HOT, int D, typename V, typename Add>
+__device__ __forceinline__ void sell_hot_each(int s, int steps, const int32_t *__restrict__ ids, const V *s_hot, const V *__restrict__ c_in, Add add)
+{
+    for (; s < steps; s += D) {
+        int id[D];
+        V v[D];
 #pragma unroll
-            for (int k = 0; k < kSellDepth; ++k) id[k] = s + k < steps ? ids[(size_t)(s + k) * T] : kSellHot;
-        }
+        for (int k = 0; k < D; ++k) id[k] = s + k < steps ? ids[(size_t)(s + k) * T] : HOT;
+        sell_hot_gather<HOT>(id, s_hot, c_in, v);
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) sum += v[k];
-        if (s >= steps) return sum;
+        for (int k = 0; k < D; ++k) add(v[k]);
+    }
+}
+
+// The first D steps of a slice.
+template <int HOT, int D>
+__device__ __forceinline__ void sell_hot_fetch(const int4 &slice, const int32_t *__restrict__ col, int lane, int (&id)[D])
+{
+#pragma unroll
+    for (int k = 0; k < D; ++k) id[k] = k < slice.y ? col[((size_t)slice.x + k) * kWave + lane] : HOT;
+}
+
+// s_hot[i] = c_in[i] for the first HOT of n sources, in pieces of 16 bytes.  Every CU of an XCD starts at another piece: otherwise they
+// would all ask one L2 channel for the same line (2 M items 13.3 -> 11.9 us).
+template <int HOT, typename V>
+__device__ __forceinline__ void sell_hot_stage(int n, const V *__restrict__ c_in, V *s_hot)
+{
+    constexpr int W = 16 / sizeof(V), T = kSellHotThreads, kPieces = (HOT / W + T - 1) / T;
+    static_assert(HOT % W == 0, "whole pieces");
+    const int hot = n < HOT ? n : HOT, rot = ((int)blockIdx.x / 8) % kPieces;
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k) {
+        const int i = ((int)threadIdx.x + (k + rot < kPieces ? k + rot : k + rot - kPieces) * T) * W;
+        if (i + W <= hot) *reinterpret_cast<float4 *>(s_hot + i) = *reinterpret_cast<const float4 *>(c_in + i);
+        else
+            for (int j = i; j < hot; ++j) s_hot[j] = c_in[j];
     }
 }
 
@@ -189,24 +217,12 @@ __global__ __launch_bounds__(kSellHotThreads) void sell_iterate_hot_kernel(
     const int stride = (int)gridDim.x * (T / kWave);
     // The first slice's ids, and the dangling mass, travel beside the hot sources.
     int s = (int)blockIdx.x + (int)gridDim.x * wave;
-    int4 d = s < slices ? slice[s] : make_int4(0, 0, 0, 0);
+    const auto descriptor = [&](int at) { return at < slices ? slice[at] : make_int4(0, 0, 0, 0); };
+    int4 d = descriptor(s), after = descriptor(s + stride);
     int id[kSellDepth];
-    const auto fetch = [&](int4 what, int (&to)[kSellDepth]) {
-#pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) to[k] = k < what.y ? col[((size_t)what.x + k) * kWave + lane] : kSellHot;
-    };
-    fetch(d, id);
+    sell_hot_fetch<kSellHot>(d, col, lane, id);
     const double mass = tid < parts ? part_in[tid] : 0.0;
-    const int hot = n < kSellHot ? n : kSellHot;
-    const double2 *c2 = reinterpret_cast<const double2 *>(c_in);
-    constexpr int kPieces = (kSellHot / 2 + T - 1) / T;
-    const int rot = ((int)blockIdx.x / 8) % kPieces;  // work-groups of an XCD would all ask one L2 channel for the same line: 2 M items 13.3 -> 11.9 us
-#pragma unroll
-    for (int k = 0; k < kPieces; ++k) {
-        const int i = tid + (k + rot < kPieces ? k + rot : k + rot - kPieces) * T;
-        if (2 * i + 1 < hot) reinterpret_cast<double2 *>(s_hot)[i] = c2[i];
-        else if (2 * i < hot) s_hot[2 * i] = c_in[2 * i];
-    }
+    sell_hot_stage<kSellHot>(n, c_in, s_hot);
     const double dang = block_sum<T>(mass, s_dang);
     const double base = (1.0 - alpha) * inv_n + alpha * dang * inv_n;
     double stat = 0.0;
@@ -220,35 +236,103 @@ __global__ __launch_bounds__(kSellHotThreads) void sell_iterate_hot_kernel(
         const int s0 = hub_step[h], s1 = hub_step[h + 1];
         const double iv = inv[h];
         const int32_t *ids = hub_col + (size_t)s0 * T + tid;
-        int hub_id[kSellDepth];
-#pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) hub_id[k] = s0 + k < s1 ? ids[(size_t)k * T] : kSellHot;
-        const double sum = block_sum<T>(sell_hot_sum<T>(hub_id, ids, s1 - s0, s_hot, c_in), s_red);
+        double sum = 0.0;
+        sell_hot_each<T, kSellHot, kSellDepth>(0, s1 - s0, ids, s_hot, c_in, [&](double v) { sum += v; });
+        sum = block_sum<T>(sum, s_red);
         if (tid == 0) finish(h, iv, sum);
         __syncthreads();  // s_red is used again
     }
     while (s < slices) {
-        const int next = s + stride;
-        const int4 after = next < slices ? slice[next] : make_int4(0, 0, 0, 0);
+        const int4 later = descriptor(s + 2 * stride);  // it takes a round trip before its ids can be asked for
         const int lanes_log = d.w & 7, lanes = 1 << lanes_log, r = lane >> lanes_log;
         const bool mine = (lane & (lanes - 1)) == 0 && r < (d.w >> 3);
         const double iv = mine ? inv[d.z + r] : 0.0;
-        int id_after[kSellDepth];
-        fetch(after, id_after);
-        double sum = sell_hot_sum<kWave>(id, col + (size_t)d.x * kWave + lane, d.y, s_hot, c_in);
+        double sum = 0.0, v[kSellDepth];
+        sell_hot_gather<kSellHot>(id, s_hot, c_in, v);
+        sell_hot_fetch<kSellHot>(after, col, lane, id);
+#pragma unroll
+        for (int k = 0; k < kSellDepth; ++k) sum += v[k];
+        sell_hot_each<kWave, kSellHot, kSellDepth>(kSellDepth, d.y, col + (size_t)d.x * kWave + lane, s_hot, c_in, [&](double x) { sum += x; });
         for (int m = lanes >> 1; m > 0; m >>= 1) sum += __shfl_xor(sum, m, kWave);
         if (mine) finish(d.z + r, iv, sum);
         d = after;
-        s = next;
-#pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) id[k] = id_after[k];
+        after = later;
+        s += stride;
     }
     const double total = block_sum<T>(stat, s_red);
     if (tid == 0) part_out[blockIdx.x] = total;
 }
 
+// diff[v] = sum of the pushes of v's row, active[v] = whether any is not 0; the number of active rows goes to `stat`.
+__global__ __launch_bounds__(kSellHotThreads) void sell_push_kernel(int n, int hubs, int slices, const int32_t *__restrict__ hub_step,
+                                                                    const int32_t *__restrict__ hub_col,
+                                                                    const int4 *__restrict__ slice, const int32_t *__restrict__ col,
+                                                                    const float *__restrict__ push, const int32_t *__restrict__ order,
+                                                                    float *__restrict__ diff, int *__restrict__ active,
+                                                                    double *part, unsigned int *ticket, StoreStat stat)
+{
+    constexpr int T = kSellHotThreads, H = kSellHotF32, D = kSellDepthF32;
+    extern __shared__ float s_push[];  // [kSellHotF32]
+    __shared__ double s_red[T / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int stride = (int)gridDim.x * (T / kWave);
+    int s = (int)blockIdx.x + (int)gridDim.x * wave;
+    const auto descriptor = [&](int at) { return at < slices ? slice[at] : make_int4(0, 0, 0, 0); };
+    int4 d = descriptor(s), after = descriptor(s + stride);
+    int id[D];
+    sell_hot_fetch<H>(d, col, lane, id);
+    sell_hot_stage<H>(n, push, s_push);
+    __syncthreads();
+    int lowered = 0;
+    const auto finish = [&](int v, float sum, bool any) {
+        diff[v] = sum;
+        active[v] = any;
+        lowered += any;
+    };
+    for (int h = blockIdx.x; h < hubs; h += gridDim.x) {
+        const int s0 = hub_step[h], s1 = hub_step[h + 1];
+        const int32_t *ids = hub_col + (size_t)s0 * T + tid;
+        float sum = 0.0f;
+        bool any = false;
+        sell_hot_each<T, H, D>(0, s1 - s0, ids, s_push, push, [&](float v) { sum += v; any |= v != 0.0f; });
+        const bool some = __syncthreads_or(any);
+        const double total = block_sum<T>((double)sum, s_red);
+        if (tid == 0) finish(order[h], (float)total, some);
+        __syncthreads();  // s_red is used again
+    }
+    while (s < slices) {
+        const int4 later = descriptor(s + 2 * stride);
+        const int lanes_log = d.w & 7, lanes = 1 << lanes_log, r = lane >> lanes_log;
+        const int row = (lane & (lanes - 1)) == 0 && r < (d.w >> 3) ? order[d.z + r] : -1;
+        float sum = 0.0f, v[D];
+        bool any = false;
+        const auto add = [&](float x) {
+            sum += x;
+            any |= x != 0.0f;
+        };
+        sell_hot_gather<H>(id, s_push, push, v);
+        sell_hot_fetch<H>(after, col, lane, id);
+#pragma unroll
+        for (int k = 0; k < D; ++k) add(v[k]);
+        sell_hot_each<kWave, H, D>(D, d.y, col + (size_t)d.x * kWave + lane, s_push, push, add);
+        const unsigned long long some = __ballot(any);
+        for (int m = lanes >> 1; m > 0; m >>= 1) sum += __shfl_xor(sum, m, kWave);
+        if (row >= 0) finish(row, sum, ((some >> lane) & (lanes == kWave ? ~0ull : (1ull << lanes) - 1)) != 0);
+        d = after;
+        after = later;
+        s += stride;
+    }
+    const double total = block_sum<T>((double)lowered, s_red);
+    unsigned int one = 0;
+    if (tid == 0) one = publish_part(part + blockIdx.x, total);
+    if (!last_block_done(ticket, one)) return;
+    const double all = block_sum<T>(tid < (int)gridDim.x ? load_agent(part + tid) : 0.0, s_red);
+    if (tid == 0) stat(all);
+}
+
 // ---- building the layout ---------------------------------------------------------------------------------------------
-__global__ void sell_lengths_kernel(int n, const int64_t *__restrict__ row_ptr, unsigned *__restrict__ len, int32_t *__restrict__ id)
+template <typename Off>
+__global__ void sell_lengths_kernel(int n, const Off *__restrict__ row_ptr, unsigned *__restrict__ len, int32_t *__restrict__ id)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         len[i] = (unsigned)(row_ptr[i + 1] - row_ptr[i]);
@@ -256,14 +340,14 @@ __global__ void sell_lengths_kernel(int n, const int64_t *__restrict__ row_ptr, 
     }
 }
 
-// new_id of every vertex; bounds[k] = rows (longest first) with more than limit[k] entries
+// new_id of every vertex; bounds[k] = rows (longest first) with more entries than class k takes
 __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorted, const int32_t *__restrict__ order,
-                                   int hub_limit, int32_t *__restrict__ new_id, int *__restrict__ bounds)
+                                   bool f32, int32_t *__restrict__ new_id, int *__restrict__ bounds)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) new_id[order[i]] = i;
     if (blockIdx.x != 0) return;
     if (threadIdx.x < kSellClasses) {
-        const unsigned limit = (unsigned)sell_class_limit(threadIdx.x, hub_limit);
+        const unsigned limit = (unsigned)sell_class_limit(threadIdx.x, f32);
         int lo = 0, hi = n;  // first row with at most `limit` entries
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -275,13 +359,13 @@ __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorte
     }
 }
 
-// *named += entries, of kSellSamples from all over the matrix, whose source is one of the first kSellHot
+// *named += entries, of kSellSamples from all over the matrix, whose source is one of the first `hot`
 __global__ __launch_bounds__(256) void sell_sample_kernel(int64_t nnz, const int32_t *__restrict__ col, const int32_t *__restrict__ new_id,
-                                                          int *__restrict__ named)
+                                                          int hot, int *__restrict__ named)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const unsigned long long hot = __ballot(new_id[col[(int64_t)((double)i / kSellSamples * (double)nnz)]] < kSellHot);
-    if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(named, __popcll(hot));
+    const unsigned long long names = __ballot(new_id[col[(int64_t)((double)i / kSellSamples * (double)nnz)]] < hot);
+    if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(named, __popcll(names));
 }
 
 __device__ __forceinline__ void sell_slice_rows(const SellShape &sh, int s, int &k, int &first_row, int &last_row)
@@ -312,17 +396,18 @@ __global__ void sell_steps_kernel(SellShape sh, int threads, const unsigned *__r
 }
 
 // The ids of every hub row and slice, one wavefront per slice and one work-group per hub row.
+template <typename Off>
 __global__ __launch_bounds__(256) void sell_fill_kernel(SellShape sh, int threads, const int32_t *__restrict__ order,
-                                                        const int64_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
+                                                        const Off *__restrict__ row_ptr, const int32_t *__restrict__ col,
                                                         const int32_t *__restrict__ new_id,
                                                         const int32_t *__restrict__ hub_step,
                                                         const int32_t *__restrict__ slice_step, int4 *__restrict__ slice,
-                                                        int32_t *__restrict__ hub_out, int32_t *__restrict__ out, bool hot)
+                                                        int32_t *__restrict__ hub_out, int32_t *__restrict__ out, int hot)
 {
     const auto source = [&](bool there, int64_t e) {
-        if (!there) return hot ? kSellHot : sh.n;
+        if (!there) return hot ? hot : sh.n;
         const int id = new_id[col[e]];
-        return id + (hot && id >= kSellHot);
+        return id + (hot && id >= hot);
     };
     if ((int)blockIdx.x < sh.hubs) {
         const int64_t e0 = row_ptr[order[blockIdx.x]], e1 = row_ptr[order[blockIdx.x] + 1];
@@ -361,14 +446,19 @@ SellShape shape_of(const SellRows &sr)
 
 bool sell_suits(int64_t n, int64_t nnz) { return n + nnz <= kSellMaxItems; }
 
-int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, const int32_t *col, hipStream_t s)
+namespace {
+
+// f32_id: of sell_create_f32, or null.
+template <typename Off>
+int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const int32_t *col, int32_t *f32_id, hipStream_t s)
 {
+    const int hot = f32_id ? kSellHotF32 : kSellHot;
     sr->n = n;
     sr->nnz = nnz;
     sr->threads = n + nnz > kSellWideItems ? 512 : 256;
-    const int hub_limit = kWave * kSellWaveSteps;
+    constexpr int kWords = kSellClasses + 1;
     unsigned *len = nullptr, *len_sorted = nullptr;
-    int32_t *ids = nullptr, *new_id = nullptr, *hub_steps = nullptr, *slice_steps = nullptr, *slice_step = nullptr;
+    int32_t *ids = nullptr, *new_id = f32_id, *hub_steps = nullptr, *slice_steps = nullptr, *slice_step = nullptr;
     int *bounds = nullptr, *h = nullptr;
     char *temp = nullptr;
     DeviceArena temps;
@@ -376,17 +466,21 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
         const size_t cnt = (size_t)n;
         // no more slices than rows of one lane each, plus one partly filled slice per class, plus 1 lane per kSellDepth / 2 entries
         const size_t most_slices = cnt / kWave + (size_t)nnz / (kWave * kSellDepth / 2) + 2 * kSellClasses + 1;
-        const size_t most_hubs = (size_t)nnz / hub_limit + 1;
+        const size_t most_hubs = (size_t)nnz / sell_class_limit(0, f32_id != nullptr) + 1;
         size_t temp_bytes = 0, need = 0;
         sr->arena.want(&sr->order, cnt);
         sr->arena.want(&sr->hub_step, most_hubs + 1);
         sr->arena.want(&sr->slice, most_slices);
-        sr->arena.want(&sr->c[0], cnt + 1);
-        sr->arena.want(&sr->c[1], cnt + 1);
-        sr->arena.want(&sr->inv, cnt);
+        if (!f32_id) {
+            sr->arena.want(&sr->c[0], cnt + 1);
+            sr->arena.want(&sr->c[1], cnt + 1);
+            sr->arena.want(&sr->inv, cnt);
+        }
         const size_t most_blocks = std::max<size_t>(most_hubs + ceil_div((int64_t)most_slices, sr->threads / kWave), kSellInitBlocks);
-        sr->arena.want(&sr->part[0], most_blocks);
-        sr->arena.want(&sr->part[1], most_blocks);
+        if (!f32_id) {
+            sr->arena.want(&sr->part[0], most_blocks);
+            sr->arena.want(&sr->part[1], most_blocks);
+        }
         DRONE_HIP_TRY(sr->arena.commit());
         DRONE_HIP_TRY(rocprim::radix_sort_pairs_desc(nullptr, temp_bytes, reinterpret_cast<unsigned *>(0x1000),
                                                      reinterpret_cast<unsigned *>(0x2000), reinterpret_cast<int32_t *>(0x3000),
@@ -397,29 +491,31 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
         temps.want(&len, cnt);
         temps.want(&len_sorted, cnt);
         temps.want(&ids, cnt);
-        temps.want(&new_id, cnt);
+        if (!f32_id) temps.want(&new_id, cnt);
         temps.want(&hub_steps, most_hubs + 1);
         temps.want(&slice_steps, most_slices + 1);
         temps.want(&slice_step, most_slices + 1);
-        temps.want(&bounds, kSellClasses + 1);
+        temps.want(&bounds, kWords);
         temps.want(&temp, temp_bytes);
         DRONE_HIP_TRY(temps.commit());
-        DRONE_HIP_TRY(hipHostMalloc(&h, sizeof(int) * (kSellClasses + 1)));
+        DRONE_HIP_TRY(hipHostMalloc(&h, sizeof(int) * kWords));
         const int grid = (int)std::min<int64_t>(ceil_div(n, 256), 2048);
         int key_bits = 1;
         while (key_bits < 32 && (1ll << key_bits) <= nnz) ++key_bits;
         sell_lengths_kernel<<<grid, 256, 0, s>>>((int)n, row_ptr, len, ids);
         need = temp_bytes;
         DRONE_HIP_TRY(rocprim::radix_sort_pairs_desc(temp, need, len, len_sorted, ids, sr->order, cnt, 0, key_bits, s));
-        sell_bounds_kernel<<<grid, 256, 0, s>>>((int)n, len_sorted, sr->order, hub_limit, new_id, bounds);
-        if (n + nnz > kSellWideItems && nnz >= kSellSamples) sell_sample_kernel<<<kSellSamples / 256, 256, 0, s>>>(nnz, col, new_id, bounds + kSellClasses);
-        DRONE_HIP_TRY(hipMemcpyAsync(h, bounds, sizeof(int) * (kSellClasses + 1), hipMemcpyDeviceToHost, s));
+        sell_bounds_kernel<<<grid, 256, 0, s>>>((int)n, len_sorted, sr->order, f32_id != nullptr, new_id, bounds);
+        if (n + nnz > kSellWideItems && nnz >= kSellSamples) sell_sample_kernel<<<kSellSamples / 256, 256, 0, s>>>(nnz, col, new_id, hot, bounds + kSellClasses);
+        DRONE_HIP_TRY(hipMemcpyAsync(h, bounds, sizeof(int) * kWords, hipMemcpyDeviceToHost, s));
         DRONE_HIP_TRY(hipStreamSynchronize(s));
         if (h[kSellClasses] >= kSellHotShare * kSellSamples) {
-            sr->hot = true;
+            sr->hot = hot;
             sr->threads = kSellHotThreads;
-            DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&sell_iterate_hot_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSellHotLds));
+            DRONE_HIP_TRY(hipFuncSetAttribute(f32_id ? reinterpret_cast<const void *>(&sell_push_kernel) : reinterpret_cast<const void *>(&sell_iterate_hot_kernel),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSellHotLds));
         }
+        if (f32_id && !sr->hot) return DRONE_OK;
         sr->hubs = h[0];
         for (int k = 0; k < kSellClasses; ++k) {
             sr->row_begin[k] = h[k];
@@ -452,8 +548,22 @@ int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, co
     const int rc = body();
     temps.release();
     if (h) (void)hipHostFree(h);
-    if (rc != DRONE_OK) sell_destroy(sr);
+    if (rc != DRONE_OK || (f32_id && !sr->hot)) sell_destroy(sr);
     return rc;
+}
+
+}  // namespace
+
+int sell_create(SellRows *sr, int64_t n, int64_t nnz, const int64_t *row_ptr, const int32_t *col, hipStream_t s)
+{
+    return sell_build(sr, n, nnz, row_ptr, col, nullptr, s);
+}
+
+bool sell_f32_suits(int64_t n, int64_t nnz) { return n + nnz > kSellF32Items && n < INT32_MAX - 1; }
+
+int sell_create_f32(SellRows *sr, int64_t n, int64_t nnz, const int *row_ptr, const int32_t *col, int32_t *new_id, hipStream_t s)
+{
+    return sell_build(sr, n, nnz, row_ptr, col, new_id, s);
 }
 
 void sell_destroy(SellRows *sr)
@@ -482,6 +592,15 @@ int sell_iterate(const SellRows &sr, int it, double alpha, double *rank_out, hip
     if (sr.hot) launch(sell_iterate_hot_kernel, kSellHotLds);
     else if (sr.threads == 512) launch(sell_iterate_kernel<512>, 0);
     else launch(sell_iterate_kernel<256>, 0);
+    DRONE_HIP_TRY(hipGetLastError());
+    return DRONE_OK;
+}
+
+int sell_push(const SellRows &sr, const float *push, float *diff, int *active, double *part, unsigned int *ticket, const StoreStat &stat,
+              hipStream_t s)
+{
+    sell_push_kernel<<<sr.blocks, sr.threads, kSellHotLds, s>>>((int)sr.n, sr.hubs, sr.slices, sr.hub_step, sr.hub_col, sr.slice, sr.col,
+                                                               push, sr.order, diff, active, part, ticket, stat);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }

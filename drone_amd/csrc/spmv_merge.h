@@ -60,6 +60,18 @@ template <> __device__ __forceinline__ double vzero<double>() { return 0.0; }
 template <> __device__ __forceinline__ float vzero<float>() { return 0.0f; }
 template <> __device__ __forceinline__ PushF2 vzero<PushF2>() { return PushF2{0.0f, 0.0f}; }
 
+// What an entry's value takes in LDS: its count follows from its sum.
+template <typename V> struct Entry {
+    using Stored = V;
+    static __device__ __forceinline__ V pack(V v) { return v; }
+    static __device__ __forceinline__ V value(V v) { return v; }
+};
+template <> struct Entry<PushF2> {
+    using Stored = float;
+    static __device__ __forceinline__ float pack(PushF2 v) { return v.s; }
+    static __device__ __forceinline__ PushF2 value(float s) { return PushF2{s, s != 0.0f ? 1.0f : 0.0f}; }
+};
+
 __device__ __forceinline__ double shfl_up_v(double v, int d) { return __shfl_up(v, d, kWave); }
 __device__ __forceinline__ float shfl_up_v(float v, int d) { return __shfl_up(v, d, kWave); }
 __device__ __forceinline__ PushF2 shfl_up_v(PushF2 v, int d)
@@ -131,8 +143,12 @@ __global__ __launch_bounds__(kSpmvBlock) void spmv_merge_kernel(
     const int32_t *__restrict__ col, Epi epi, V *__restrict__ tile_carry, double *__restrict__ tile_stat)
 {
     constexpr int TILE = kSpmvBlock * IPT;
-    __shared__ V s_val[TILE];  // gathered values, later the row totals
-    __shared__ int s_rowend[TILE + 1];
+    using Stored = typename Entry<V>::Stored;
+    // gathered values and row ends, later the row totals
+    constexpr size_t kMerge = sizeof(Stored) * TILE + sizeof(int) * (TILE + 1), kTotals = sizeof(V) * TILE;
+    __shared__ __attribute__((aligned(16))) char s_mem[kMerge > kTotals ? kMerge : kTotals];
+    Stored *const s_val = reinterpret_cast<Stored *>(s_mem);
+    int *const s_rowend = reinterpret_cast<int *>(s_mem + sizeof(Stored) * TILE);
     __shared__ V s_wave_v[kSpmvBlock / kWave];
     __shared__ int s_wave_f[kSpmvBlock / kWave];
     __shared__ double s_red[kSpmvBlock / kWave];
@@ -160,9 +176,10 @@ __global__ __launch_bounds__(kSpmvBlock) void spmv_merge_kernel(
             const int i = tid + k * kSpmvBlock;
             c[k] = i < ne ? __builtin_nontemporal_load(col + e0 + i) : -1;
         }
-        V x[IPT];
+        Stored x[IPT];
 #pragma unroll
-        for (int k = 0; k < IPT; ++k) x[k] = c[k] >= 0 ? epi.load(c[k], e0 + tid + k * kSpmvBlock) : vzero<V>();
+        for (int k = 0; k < IPT; ++k)
+            x[k] = Entry<V>::pack(c[k] >= 0 ? epi.load(c[k], e0 + tid + k * kSpmvBlock) : vzero<V>());
 #pragma unroll
         for (int k = 0; k < IPT; ++k) {
             const int i = tid + k * kSpmvBlock;
@@ -191,7 +208,7 @@ __global__ __launch_bounds__(kSpmvBlock) void spmv_merge_kernel(
         out[k] = vzero<V>();
         if (d + k < items) {
             if (j < s_rowend[i]) {
-                acc = acc + s_val[j];
+                acc = acc + Entry<V>::value(s_val[j]);
                 ++j;
             } else {
                 out[k] = acc;
@@ -225,7 +242,7 @@ __global__ __launch_bounds__(kSpmvBlock) void spmv_merge_kernel(
     for (int w = 0; w < wave; ++w) cv = s_wave_f[w] ? s_wave_v[w] : cv + s_wave_v[w];
     const V carry_in = ef ? ev : cv + ev;
 
-    V *s_rowsum = s_val;
+    V *const s_rowsum = reinterpret_cast<V *>(s_mem);
     {
         int row = row_first;
         bool first = true;

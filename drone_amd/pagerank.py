@@ -173,8 +173,9 @@ class PRWorkerCUDA:
         return out
 
     def aggregation(self):
-        """'row-blocks' or 'merge-path': the kernels PR_PEVal / PR_IncEVal use for this graph (decided at the first peval)."""
-        return "row-blocks" if lib().drone_pr_aggregation(self.g) else "merge-path"
+        """'row-blocks', 'sliced-rows' or 'merge-path': the kernels PR_PEVal / PR_IncEVal use for this graph (decided by the
+        first peval)."""
+        return ("merge-path", "row-blocks", "sliced-rows")[lib().drone_pr_aggregation(self.g)]
 
     def close(self):
         if self.g:

@@ -126,7 +126,8 @@ Response PR_PEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm 
 Response PR_IncEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm);
 
 /* No counterpart in the reference: which kernels PR_PEVal / PR_IncEVal aggregate this graph with.  0 = merge
- * path (also before the first PR_PEVal has decided), 1 = source-sorted row blocks. */
+ * path (also before the first PR_PEVal has decided), 1 = source-sorted row blocks, 2 = sliced rows with the hottest
+ * sources in LDS. */
 int drone_pr_aggregation(const Graph *g);
 
 /* No counterpart in the reference (it never frees): optional clean-up. */
