@@ -898,12 +898,18 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
     if (K < 1 || (ta && tb) || (ta && M < 2)) return d;
     const auto blocks = [&]() { return ceil_div(M, 16 * d.mt) * ceil_div(N, 16 * d.nt); };
     if (ta) {
+        // One work-group per CU, its wavefronts a group of 16 steps each at least (two work-groups and five groups at most before:
+        // twice the partial sums, or a few CUs at work), and blocks that grow with the product: a block of 4 x 4 tiles reads a third
+        // less per product than one of 2 x 4, and has nothing to hide in a short reduction.  us before / now: outputs of 301 x 100 over
+        // 30,011 rows 41.1 / 35.4, 300 x 128 over 100,000 109 / 85, 1,400 x 128 over 5,000 38.2 / 33.8, 200 x 64 over 60,000 33.6 /
+        // 28.8 (2 x 4: 33.3) and over 9,001 14.5 / 10.9 (2 x 4: 11.5), 100 x 50 over 15,003 15.5 / 11.3, 100 x 23 over 30,011 16.9 /
+        // 11.5, 64 x 30 over 5,000 17.4 / 8.5, 64 x 7 over 2,708 11.1 / 8.3.
+        const double macs = (double)M * N * K;
         if (N <= 16) { d.mt = M <= 16 ? 1 : 2; d.nt = 1; d.ks = 16; }
-        else if (N <= 32) { d.mt = 2; d.nt = 2; d.ks = 16; }
+        else if (N <= 32) { d.mt = M > 64 ? 4 : 2; d.nt = 2; d.ks = M > 64 ? 8 : 16; }
         else if (ceil_div(N, 64) * 64 * 4 > ceil_div(N, 32) * 32 * 5) { d.mt = M >= 64 ? 4 : 2; d.nt = 2; d.ks = 8; }
-        else { d.mt = 2; d.nt = 4; d.ks = 8; }
-        // about 512 work-groups, none of them with less than five groups of 16 steps per wavefront
-        d.splits = (int)std::max<int64_t>(1, std::min<int64_t>({512 / blocks(), K / (80 * d.ks), 128}));
+        else { d.mt = M > 32 && macs >= 5e8 ? 4 : 2; d.nt = macs >= 1.5e8 ? 4 : 2; d.ks = 8; }
+        d.splits = (int)std::max<int64_t>(1, std::min<int64_t>({256 / blocks(), K / (16 * d.ks), 128}));
     } else {
         const int n16 = (int)ceil_div(N, 16);
         d.mt = 1;
@@ -932,7 +938,7 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
     // us: matrix instructions at the rate the kernel reaches on padded blocks, or its memory traffic
     const double in = 4.0 * ((double)M * K + (double)K * N), out = 4.0 * M * N;
     const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
-    const double direct_us = std::max(padded / (deep && !ta ? 60e6 : 75e6), in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
+    const double direct_us = std::max(padded / (deep && !ta ? 60e6 : d.mt * d.nt == 16 ? 90e6 : 75e6), in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
     // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.25 for a 128-wide one)
     const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
     const int64_t groups = (int64_t)tiles * splits;
@@ -997,6 +1003,7 @@ int sgemm_direct(DirectShape d, bool may_allocate, bool ta, bool tb, int M, int 
     DRONE_DIRECT(2, 2, false, false, 8)
     DRONE_DIRECT(4, 2, false, false, 8)
     DRONE_DIRECT(2, 4, false, false, 8)
+    DRONE_DIRECT(4, 4, false, false, 8)
 #undef DRONE_DIRECT_ROWS
 #undef DRONE_DIRECT
     DRONE_REQUIRE(done, "no instance of the direct kernel for this shape");
