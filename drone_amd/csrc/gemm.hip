@@ -3,8 +3,8 @@
 // forward, :72-85 input gradient, :92-105 weight gradient), which are tall-skinny: M or K is the vertex
 // count, the other dimensions are feature widths (41..602).
 //
-// Work-group = 512 lanes: 4 product wavefronts computing a 128 x BN tile of C (BN = 128 or 64) with
-// v_mfma_f32_32x32x2_f32 - every one owns a (128/WM) x (BN/WN) sub-tile as 32x32 accumulators - and 4 loader
+// Work-group = 512 lanes: 4 product wavefronts computing a BM x BN tile of C (128 x 128, 64 x 128 or 128 x 64) with
+// v_mfma_f32_32x32x2_f32 - every one owns a (BM/WM) x (BN/WN) sub-tile as 32x32 accumulators - and 4 loader
 // wavefronts that move the A and B tiles of depth 32 from global memory into LDS.  The split exists because a
 // wavefront that issues a global load into a backed-up memory pipeline stalls at the issue, in order, for
 // thousands of cycles (measured with the cycle counter: issuing one tile's loads took longer than multiplying
@@ -34,7 +34,7 @@ namespace {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 128;
+constexpr int kTileRows = 128;
 constexpr int BK = 32;
 constexpr int PAD = 4;
 
@@ -129,7 +129,7 @@ struct TileLoader {
 
 // op(A) is M x K: TA=false -> A stored M x K (k contiguous); TA=true -> A stored K x M (m contiguous).
 // op(B) is K x N: TB=false -> B stored K x N (n contiguous); TB=true -> B stored N x K (k contiguous).
-template <int BN, bool TA, bool TB>
+template <int BM, int BN, bool TA, bool TB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void sgemm_mfma_kernel(
     int M, int N, int K, float alpha, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
     float beta, float *__restrict__ C, int ldc, int k_chunk, float *__restrict__ partial)
@@ -734,14 +734,14 @@ int workspace(size_t bytes, hipStream_t s, float **out)
     return DRONE_OK;
 }
 
-template <int BN>
+template <int BM, int BN>
 void launch(bool ta, bool tb, dim3 grid, hipStream_t s, int M, int N, int K, float alpha, const float *A, int lda,
             const float *B, int ldb, float beta, float *C, int ldc, int k_chunk, float *partial)
 {
-    if (!ta && !tb) sgemm_mfma_kernel<BN, false, false><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    else if (!ta && tb) sgemm_mfma_kernel<BN, false, true><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    else if (ta && !tb) sgemm_mfma_kernel<BN, true, false><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    else sgemm_mfma_kernel<BN, true, true><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    if (!ta && !tb) sgemm_mfma_kernel<BM, BN, false, false><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    else if (!ta && tb) sgemm_mfma_kernel<BM, BN, false, true><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    else if (ta && !tb) sgemm_mfma_kernel<BM, BN, true, false><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    else sgemm_mfma_kernel<BM, BN, true, true><<<grid, 512, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
 }
 
 }  // namespace
@@ -875,6 +875,13 @@ void sgemm_tall(int transB, int M, int N, int K, float alpha, const float *A, in
 #undef DRONE_TALL
 }
 
+// Whether 128-column tiles have 64 rows instead of 128: two of their work-groups on a CU work while one waits at its barrier
+// (matrix cores busy 53 % of the time with one), and half as many CUs idle at the end.  us 128 / 64 rows: 30,011 x 301 x 100 34.6 /
+// 32.0, 45,000 x 300 x 128 51.3 / 43.7, 5,000 x 1,000 x 1,000 146 / 119, 1,000 x 1,001 x 3,000 82 / 76.  Not where 128-row tiles come
+// two to a CU anyway, 60,000 x 400 x 100 67.6 / 70.6, and not with A transposed, whose tiles are read in shorter runs: 602 x
+// 128 over 232,965 rows 330 / 374.
+bool half_rows(bool transA, int tiles) { return !transA && tiles <= 384; }
+
 // How many ways the tiled kernel splits the reduction: when the output has too few tiles to fill 256 CUs and K is long.
 int tiled_splits(int tiles, int K)
 {
@@ -940,9 +947,9 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
     const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
     const double direct_us = std::max(padded / (deep && !ta ? 60e6 : d.mt * d.nt == 16 ? 90e6 : 75e6), in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
     // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.25 for a 128-wide one)
-    const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
+    const int tiles = (int)(ceil_div(M, kTileRows) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
     const int64_t groups = (int64_t)tiles * splits;
-    const double rounds = ceil_div(groups, 256) * (deep && groups > 256 ? 0.85 : 1.0);
+    const double rounds = ceil_div(groups, 256) * (deep && groups > 256 ? 0.85 : N > 64 && half_rows(ta, tiles) ? 0.9 : 1.0);
     const double tiled_us = std::max(rounds * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.25),
                                      in / (deep ? 2.8e6 : 2.0e6) + out / 2.4e6) + (splits > 1 ? 5 : 0);
     if (tiled_us < direct_us) d.ks = 0;
@@ -1037,7 +1044,8 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
         return sgemm_direct(direct, may_allocate, transA != 0, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
     const bool narrow = N <= 64;
     const int bn = narrow ? 64 : 128;
-    const int tiles = (int)(ceil_div(M, BM) * ceil_div(N, bn));
+    const int tiles = (int)(ceil_div(M, kTileRows) * ceil_div(N, bn));
+    const int bm = !narrow && half_rows(transA != 0, tiles) ? kTileRows / 2 : kTileRows;
     int splits = tiled_splits(tiles, K);
     int k_chunk = (int)ceil_div(ceil_div(K > 0 ? K : 1, splits), BK) * BK;
     splits = (int)ceil_div(K > 0 ? K : 1, k_chunk);
@@ -1048,10 +1056,11 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
         const int rc = split_scratch(may_allocate, floats, s, M, N, K, splits, &partial);
         if (rc != DRONE_OK) return rc;
     }
-    dim3 grid((unsigned)ceil_div(N, bn), (unsigned)ceil_div(M, BM), (unsigned)splits);
+    dim3 grid((unsigned)ceil_div(N, bn), (unsigned)ceil_div(M, bm), (unsigned)splits);
     DRONE_REQUIRE(grid.y <= 65535u * 32u, "M too large for the launch grid");
-    if (narrow) launch<64>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    else launch<128>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    if (narrow) launch<kTileRows, 64>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    else if (bm < kTileRows) launch<kTileRows / 2, 128>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    else launch<kTileRows, 128>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
     if (splits > 1) launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;

@@ -14,3 +14,10 @@ pytestmark = pytest.mark.gpu
     (1400, 100, 3_572), (1400, 128, 127), (16, 16, 257), (17, 16, 255)])
 def test_weight_gradients(M, N, K):
     _edges(1, 0, M, N, K)
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(49_152, 128, 300), (49_153, 127, 300), (24_513, 129, 65), (4_097, 900, 97), (65, 3_001, 1_001), (63, 3_001, 1_000),
+                                   (12_345, 70, 1_100), (700, 40, 1_471), (700, 57, 384 + 16 * 8 + 5)])
+def test_rows_of_half_tiles_and_deep_reductions(M, N, K, tb):
+    _edges(0, tb, M, N, K)
