@@ -94,26 +94,6 @@ struct Lists {
 // A list of no vertices that no round may take for its own: all of them still have to propagate.
 __host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
 
-// sssp.cu:23-38, and the list of the first round: the start vertex if this subgraph holds it (sssp.cu:30) and it has
-// out-edges.
-__global__ void sssp_init_kernel(int n, const int *__restrict__ global_to_local, int start_id, int *__restrict__ active,
-                                 float *__restrict__ dist, int *__restrict__ ubm, const int *__restrict__ index,
-                                 int *__restrict__ list, int *__restrict__ offset, TraverseState *__restrict__ state)
-{
-    const int start = global_to_local[start_id];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        active[i] = i == start ? 0 : -1;
-        dist[i] = i == start ? 0.0f : kUnreached;
-        ubm[i] = 0;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const int degree = start >= 0 ? index[start + 1] - index[start] : 0;
-        list[0] = start;
-        offset[0] = 0;
-        *state = TraverseState{degree > 0 ? (1ull << 32) + (unsigned long long)degree : 0ull, 1, 0, 0, 0.0};
-    }
-}
-
 // Ends a counting kernel: the last work-group adds the work-groups' counts and leaves the sum in *out.
 __device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
 {
@@ -402,22 +382,57 @@ __global__ void iota_kernel(int *out, int n)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = i;
 }
 
-// *out = lengths other than 1.0, and kNotWhole for each that is no whole number (len is 16-byte aligned).
+// Lengths other than 1.0, and kNotWhole for each that is no whole number: this lane's share (len is 16-byte aligned).
+__device__ __forceinline__ double count_other_lengths(int n, const float *__restrict__ len)
+{
+    constexpr int kInFlight = 2;  // more, or more work-groups: the same within 2 %
+    double cnt = 0.0;
+    const auto other = [](float v) { return v == 1.0f ? 0.0 : v == rintf(v) && fabsf(v) < 0x1p24f ? 1.0 : 1.0 + kNotWhole; };
+    const float4 *len4 = reinterpret_cast<const float4 *>(len);
+    const int quads = n / 4, stride = gridDim.x * kSpmvBlock;
+    for (int64_t i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += (int64_t)kInFlight * stride) {
+        float4 v[kInFlight];
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k) v[k] = i + (int64_t)k * stride < quads ? len4[i + (int64_t)k * stride] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k)
+            if (v[k].x != 1.0f || v[k].y != 1.0f || v[k].z != 1.0f || v[k].w != 1.0f) cnt += (other(v[k].x) + other(v[k].y)) + (other(v[k].z) + other(v[k].w));
+    }
+    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) cnt += other(len[4 * quads + threadIdx.x]);
+    return cnt;
+}
 __global__ __launch_bounds__(kSpmvBlock) void count_not_one_kernel(int n, const float *__restrict__ len, double *block_part,
                                                                    unsigned int *ticket, double *out)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
-    double cnt = 0.0;
-    const auto other = [](float v) { return v == 1.0f ? 0.0 : v == rintf(v) && fabsf(v) < 0x1p24f ? 1.0 : 1.0 + kNotWhole; };
-    const float4 *len4 = reinterpret_cast<const float4 *>(len);
-    const int quads = n / 4;
-#pragma unroll 4
-    for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += gridDim.x * kSpmvBlock) {
-        const float4 v = len4[i];
-        if (v.x != 1.0f || v.y != 1.0f || v.z != 1.0f || v.w != 1.0f) cnt += (other(v.x) + other(v.y)) + (other(v.z) + other(v.w));
+    publish_sum(count_other_lengths(n, len), s_red, block_part, ticket, out);
+}
+
+// sssp.cu:23-38, the list of the first round - the start vertex if this subgraph holds it (sssp.cu:30) and it has out-edges -, and the
+// count of the lengths, which the stores do not wait for.  Distances of 1 M vertices and
+// 13 M edges 129 us with two launches, 121 with one; 20,000 vertices 77 and 69.
+__global__ __launch_bounds__(kSpmvBlock) void sssp_begin_kernel(int n, const int *__restrict__ global_to_local, int start_id, int *__restrict__ active,
+                                                                float *__restrict__ dist, int *__restrict__ ubm, const int *__restrict__ index,
+                                                                int *__restrict__ list, int *__restrict__ offset, int edges,
+                                                                const float *__restrict__ len, double *block_part, unsigned int *ticket,
+                                                                TraverseState *state)
+{
+    __shared__ double s_red[kSpmvBlock / kWave];
+    const int start = global_to_local[start_id];
+    for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < n; i += gridDim.x * kSpmvBlock) {
+        active[i] = i == start ? 0 : -1;
+        dist[i] = i == start ? 0.0f : kUnreached;
+        ubm[i] = 0;
     }
-    if (blockIdx.x == 0 && (int)threadIdx.x < n - 4 * quads) cnt += other(len[4 * quads + threadIdx.x]);
-    publish_sum(cnt, s_red, block_part, ticket, out);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const int degree = start >= 0 ? index[start + 1] - index[start] : 0;
+        list[0] = start;
+        offset[0] = 0;
+        state->listed = degree > 0 ? (1ull << 32) + (unsigned long long)degree : 0ull;
+        state->mark = 1;
+        state->rounds = state->which = 0;
+    }
+    publish_sum(count_other_lengths(edges, len), s_red, block_part, ticket, &state->not_one);
 }
 
 __global__ void gather_len_kernel(int n, const int *__restrict__ eid, const float *__restrict__ len,
@@ -821,6 +836,13 @@ constexpr int kPullThreads = 1024, kPullBlocks = 512;  // all resident at once: 
 constexpr int kPullList = 2048;
 constexpr int kPullLane = 8, kPullGroup = 256, kPullWave = 4096;
 
+// A row that waits for more lanes than one, and what is known of it.
+struct OpenRow {
+    int vertex;
+    unsigned int e0, e1;
+    int was;  // order_of
+};
+
 template <typename Pull>
 __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *state, unsigned long long limit, int n,
                                                                  const int *__restrict__ in_index,
@@ -831,7 +853,7 @@ __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *
     using Value = typename Pull::Value;
     constexpr int kWaves = kPullThreads / kWave;
     __shared__ ListBuffer<kPullList> s_buf;
-    __shared__ int s_group[kPullThreads], s_wave[kPullThreads], s_block[kPullThreads];
+    __shared__ OpenRow s_group[kPullThreads], s_wave[kPullThreads], s_block[kPullThreads];
     __shared__ int s_groups, s_waves, s_blocks, s_best;
     const TraverseState now = *state;
     if ((now.listed & 0xFFFFFFFFull) <= limit || !pull.begin(now)) return;
@@ -845,13 +867,13 @@ __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *
         if (degree > 0) s_buf.add(r, degree);
     };
     // G lanes a row
-    const auto walk = [&](auto lanes, const int *rows, int count) {
+    const auto walk = [&](auto lanes, const OpenRow *rows, int count) {
         constexpr int G = decltype(lanes)::value;
         const int l = tid & (G - 1);
         for (int i = tid / G; i < count; i += kPullThreads / G) {
-            const int row = rows[i];
-            const unsigned int e0 = in_index[row], e1 = in_index[row + 1];
-            const Value was = pull.at(row);
+            const int row = rows[i].vertex;
+            const unsigned int e0 = rows[i].e0, e1 = rows[i].e1;
+            const Value was = value_of_order(rows[i].was, Value{});
             Value best = was;
             for (unsigned int base = e0; base < e1; base += 2 * G) {
                 int u[2];
@@ -900,11 +922,11 @@ __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *
                     }
                     lower(r, was, best);
                 } else if (e1 - e0 <= kPullGroup) {
-                    s_group[atomicAdd(&s_groups, 1)] = r;
+                    s_group[atomicAdd(&s_groups, 1)] = OpenRow{r, e0, e1, order_of(was)};
                 } else if (e1 - e0 <= kPullWave) {
-                    s_wave[atomicAdd(&s_waves, 1)] = r;
+                    s_wave[atomicAdd(&s_waves, 1)] = OpenRow{r, e0, e1, order_of(was)};
                 } else {
-                    s_block[atomicAdd(&s_blocks, 1)] = r;
+                    s_block[atomicAdd(&s_blocks, 1)] = OpenRow{r, e0, e1, order_of(was)};
                 }
             }
         }
@@ -912,9 +934,9 @@ __global__ __launch_bounds__(kPullThreads) void pull_open_kernel(TraverseState *
         walk(std::integral_constant<int, kWave>{}, s_wave, s_waves);
         walk(std::integral_constant<int, 16>{}, s_group, s_groups);
         for (int i = 0; i < s_blocks; ++i) {  // the same count for all: s_blocks is settled
-            const int row = s_block[i];
-            const unsigned int e0 = in_index[row], e1 = in_index[row + 1];
-            const Value was = pull.at(row);
+            const int row = s_block[i].vertex;
+            const unsigned int e0 = s_block[i].e0, e1 = s_block[i].e1;
+            const Value was = value_of_order(s_block[i].was, Value{});
             if (tid == 0) s_best = order_of(was);
             __syncthreads();
             Value best = was;
@@ -1686,7 +1708,7 @@ bool ensure_chains(Graph *g, TraverseExt *t, hipStream_t s)
 }
 
 // Rounds over the ends of the chains until nothing changes, and the inner vertices' distances; false if the lengths are not all 1.0,
-// with nothing done.  sssp_init_kernel and count_not_one_kernel have been launched.
+// with nothing done.  sssp_begin_kernel has been launched.
 bool run_chains(Graph *g, TraverseExt *t, float *dist, int start_id, hipStream_t s)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
@@ -1818,9 +1840,10 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
     GraphExt *x = static_cast<GraphExt *>(g->ext);
     SsspRun run{g, t, values->distance, s, true};
     const auto begin = [&] {
-        sssp_init_kernel<<<t->blocks, kSpmvBlock, 0, s>>>(n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage,
-                                                         g->index, t->lists.vertex[0], t->lists.offset[0], t->state);
-        run.count_lengths();
+        sssp_begin_kernel<<<std::max(sum_blocks(n), sum_blocks(x->edges, 16)), kSpmvBlock, 0, s>>>(
+            n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage, g->index, t->lists.vertex[0], t->lists.offset[0], x->edges,
+            g->edgeLen, t->block_part, t->ticket, t->state);
+        run.counted = true;
     };
     const bool chains = ensure_chains(g, t, s) && !x->chains.other_lengths;
     begin();

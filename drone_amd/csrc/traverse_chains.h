@@ -115,7 +115,7 @@ struct ChainEnd {
 };
 __device__ __forceinline__ ChainEnd chain_end(int2 at, const Rows &rows) { return ChainEnd{rows.dst[rows.index[at.x >> 1] + (at.x & 1)], at.y + 1}; }
 
-// After sssp_init_kernel and the count of the lengths: an inner start vertex has reached its chain's ends.  Over lengths other than
+// After sssp_begin_kernel: an inner start vertex has reached its chain's ends.  Over lengths other than
 // 1.0 there is nothing to do here.
 __global__ void chain_start_kernel(Rows rows, const int *__restrict__ global_to_local, int start_id, const int2 *__restrict__ arc,
                                    int *__restrict__ active, float *__restrict__ dist, int *__restrict__ list, int *__restrict__ offset,
