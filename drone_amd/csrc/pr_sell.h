@@ -15,8 +15,8 @@
 // sort are about as long - with the id of a source that is always 0.  Rows of more than 64 * kSellWaveSteps entries are
 // hubs: a work-group each, T consecutive ids per step.  Every sum has a fixed order, so the results are bitwise repeatable.
 //
-// Measured, R-MAT edge factor 16, us per iteration (row blocks before, this): 1 K vertices 11.6 -> 4.05, 4 K 17.1 -> 4.7,
-// 16 K 18.3 -> 4.9, 64 K 19.4 -> 9.1, 131 K 24.0 -> 14.2, 262 K 32.1 -> 24.3, 524 K 43.8 -> 41.3; the plan takes
+// Measured, R-MAT edge factor 16, us per iteration (row blocks before, this): 1 K vertices 11.6 -> 4.05, 4 K 17.1 -> 4.3,
+// 16 K 18.3 -> 4.7, 64 K 19.4 -> 8.0, 131 K 24.0 -> 14.2, 262 K 32.1 -> 24.3, 524 K 43.8 -> 41.3; the plan takes
 // 0.13 ... 1.2 ms instead of 0.3 ... 2.7 ms.  Below 16 K vertices it is a launch (2.3 us) plus one chain of slice
 // descriptor, ids, gathers and the partials' sum out of a cold L2; at 64 K and more the rate of gathers that hit L2.
 // Lanes of 4 or 16 entries (kSellDepth) instead of 8: 10.0 / 9.3 us at 64 K.
@@ -32,7 +32,10 @@ namespace drone {
 
 constexpr int kSellClasses = 7;      // P = 64, 32, ..., 1
 constexpr int kSellDepth = 8;        // most entries of a lane in a slice with P < 64; gathers in flight per lane
-constexpr int kSellWaveSteps = 16;   // most steps of a slice with P = 64: longer rows are hubs
+// Gathers in flight per lane of a hub row's work-group, and most steps of a slice with P = 64 (longer rows are hubs) without / with
+// the hottest sources in LDS.  In a small matrix the longest rows are what a launch waits for; us per run of 20 iterations at 4 K /
+// 64 K vertices with 8 in flight and 16 steps 93 / 179, 16 and 16 94 / 165, 16 and 12 86 / 158, 16 and 8 86 / 161, 16 and 4 85 / 175.
+constexpr int kSellHubDepth = 16, kSellWaveSteps = 12, kSellWaveStepsWide = 16;
 constexpr int kSellDepthF32 = 16, kSellWaveStepsF32 = 32;  // the same of float rows
 constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,000 of 163,840 bytes
 

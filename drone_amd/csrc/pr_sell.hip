@@ -37,16 +37,22 @@ struct SellShape {
 };
 
 // Class of a row of `len` entries: the smallest P with at most kSellDepth (kSellDepthF32) entries per lane; class k has P = 64 >> k.
-__host__ __device__ inline int sell_class_limit(int k, bool f32)  // longest row of class k
+__host__ __device__ inline int sell_class_limit(int k, bool f32, int hub_limit)  // longest row of class k
 {
-    return k == 0 ? kWave * (f32 ? kSellWaveStepsF32 : kSellWaveSteps) : (64 >> k) * (f32 ? kSellDepthF32 : kSellDepth);
+    return k == 0 ? hub_limit : (64 >> k) * (f32 ? kSellDepthF32 : kSellDepth);
+}
+
+__device__ __forceinline__ double wave_sum(double v)  // valid in every lane
+{
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
+    return v;
 }
 
 template <int T>
 __device__ __forceinline__ double block_sum(double v, double *s_red)  // valid in every thread
 {
-#pragma unroll
-    for (int m = kWave / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
+    v = wave_sum(v);
     if ((threadIdx.x & (kWave - 1)) == 0) s_red[threadIdx.x / kWave] = v;
     __syncthreads();
     double t = 0.0;
@@ -74,20 +80,20 @@ __global__ __launch_bounds__(kSellInitThreads) void sell_begin_kernel(int n, con
     if (threadIdx.x == 0) part[blockIdx.x] = total;
 }
 
-// Sum of c_in over `steps` consecutive steps of T ids starting at `ids` (this lane's), kSellDepth gathers in flight.
-template <int T>
+// Sum of c_in over `steps` consecutive steps of T ids starting at `ids` (this lane's), D gathers in flight.
+template <int T, int D>
 __device__ __forceinline__ double sell_sum(const int32_t *__restrict__ ids, int steps, const double *__restrict__ c_in, int pad)
 {
     double sum = 0.0;
-    for (int s = 0; s < steps; s += kSellDepth) {
-        int id[kSellDepth];
-        double v[kSellDepth];
+    for (int s = 0; s < steps; s += D) {
+        int id[D];
+        double v[D];
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) id[k] = s + k < steps ? ids[(size_t)(s + k) * T] : pad;  // uniform condition
+        for (int k = 0; k < D; ++k) id[k] = s + k < steps ? ids[(size_t)(s + k) * T] : pad;  // uniform condition
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) v[k] = s + k < steps ? c_in[id[k]] : 0.0;
+        for (int k = 0; k < D; ++k) v[k] = s + k < steps ? c_in[id[k]] : 0.0;
 #pragma unroll
-        for (int k = 0; k < kSellDepth; ++k) sum += v[k];
+        for (int k = 0; k < D; ++k) sum += v[k];
     }
     return sum;
 }
@@ -103,7 +109,7 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
                                                          double *__restrict__ part_out, double alpha, double inv_n,
                                                          const int32_t *__restrict__ order, double *__restrict__ r_out)
 {
-    __shared__ double s_dang[T / kWave], s_red[T / kWave];
+    __shared__ double s_dang[T / kWave], s_hub[T / kWave], s_red[T / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     // The partials are requested first and added up last: they travel beside the entries.
     double mass[kSellMassLoads];
@@ -117,9 +123,9 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
             row = blockIdx.x;
             iv = inv[row];
         }
-        sum = sell_sum<T>(hub_col + (size_t)s0 * T + tid, s1 - s0, c_in, n);
-        sum = block_sum<T>(sum, s_red);
-        __syncthreads();  // s_red is used again below
+        sum = sell_sum<T, kSellHubDepth>(hub_col + (size_t)s0 * T + tid, s1 - s0, c_in, n);
+        sum = wave_sum(sum);
+        if (lane == 0) s_hub[wave] = sum;
     } else {
         const int s = __builtin_amdgcn_readfirstlane(((int)blockIdx.x - hubs) * (T / kWave) + wave);
         if (s < slices) {  // the same for the whole wavefront
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
                 row = d.z + r;
                 iv = inv[row];
             }
-            sum = sell_sum<kWave>(col + (size_t)d.x * kWave + lane, d.y, c_in, n);
+            sum = sell_sum<kWave, kSellDepth>(col + (size_t)d.x * kWave + lane, d.y, c_in, n);
             for (int m = lanes >> 1; m > 0; m >>= 1) sum += __shfl_xor(sum, m, kWave);
         }
     }
@@ -137,7 +143,12 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
 #pragma unroll
     for (int k = 0; k < kSellMassLoads; ++k) all += tid + k * T < parts ? mass[k] : 0.0;
     for (int i = tid + kSellMassLoads * T; i < parts; i += T) all += part_in[i];
-    const double dang = block_sum<T>(all, s_dang);
+    const double dang = block_sum<T>(all, s_dang);  // its barrier is s_hub's too
+    if ((int)blockIdx.x < hubs) {
+        sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < T / kWave; ++w) sum += s_hub[w];
+    }
     double stat = 0.0;
     if (row >= 0) {
         const double rn = (1.0 - alpha) * inv_n + alpha * dang * inv_n + alpha * sum;
@@ -342,12 +353,12 @@ __global__ void sell_lengths_kernel(int n, const Off *__restrict__ row_ptr, unsi
 
 // new_id of every vertex; bounds[k] = rows (longest first) with more entries than class k takes
 __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorted, const int32_t *__restrict__ order,
-                                   bool f32, int32_t *__restrict__ new_id, int *__restrict__ bounds)
+                                   bool f32, int hub_limit, int32_t *__restrict__ new_id, int *__restrict__ bounds)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) new_id[order[i]] = i;
     if (blockIdx.x != 0) return;
     if (threadIdx.x < kSellClasses) {
-        const unsigned limit = (unsigned)sell_class_limit(threadIdx.x, f32);
+        const unsigned limit = (unsigned)sell_class_limit(threadIdx.x, f32, hub_limit);
         int lo = 0, hi = n;  // first row with at most `limit` entries
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -457,6 +468,7 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
     sr->nnz = nnz;
     sr->threads = n + nnz > kSellWideItems ? 512 : 256;
     constexpr int kWords = kSellClasses + 1;
+    const int hub_limit = kWave * (f32_id ? kSellWaveStepsF32 : n + nnz > kSellWideItems ? kSellWaveStepsWide : kSellWaveSteps);
     unsigned *len = nullptr, *len_sorted = nullptr;
     int32_t *ids = nullptr, *new_id = f32_id, *hub_steps = nullptr, *slice_steps = nullptr, *slice_step = nullptr;
     int *bounds = nullptr, *h = nullptr;
@@ -466,7 +478,7 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         const size_t cnt = (size_t)n;
         // no more slices than rows of one lane each, plus one partly filled slice per class, plus 1 lane per kSellDepth / 2 entries
         const size_t most_slices = cnt / kWave + (size_t)nnz / (kWave * kSellDepth / 2) + 2 * kSellClasses + 1;
-        const size_t most_hubs = (size_t)nnz / sell_class_limit(0, f32_id != nullptr) + 1;
+        const size_t most_hubs = (size_t)nnz / hub_limit + 1;
         size_t temp_bytes = 0, need = 0;
         sr->arena.want(&sr->order, cnt);
         sr->arena.want(&sr->hub_step, most_hubs + 1);
@@ -505,7 +517,7 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         sell_lengths_kernel<<<grid, 256, 0, s>>>((int)n, row_ptr, len, ids);
         need = temp_bytes;
         DRONE_HIP_TRY(rocprim::radix_sort_pairs_desc(temp, need, len, len_sorted, ids, sr->order, cnt, 0, key_bits, s));
-        sell_bounds_kernel<<<grid, 256, 0, s>>>((int)n, len_sorted, sr->order, f32_id != nullptr, new_id, bounds);
+        sell_bounds_kernel<<<grid, 256, 0, s>>>((int)n, len_sorted, sr->order, f32_id != nullptr, hub_limit, new_id, bounds);
         if (n + nnz > kSellWideItems && nnz >= kSellSamples) sell_sample_kernel<<<kSellSamples / 256, 256, 0, s>>>(nnz, col, new_id, hot, bounds + kSellClasses);
         DRONE_HIP_TRY(hipMemcpyAsync(h, bounds, sizeof(int) * kWords, hipMemcpyDeviceToHost, s));
         DRONE_HIP_TRY(hipStreamSynchronize(s));

@@ -43,3 +43,25 @@ def test_hot_sources(oracle, n, filler, hot_share, more):
         assert np.max(np.abs(got - ref) / ref) <= 2 * iters * max(length.max(), n // 256) * 2.0 ** -53
         assert np.array_equal(got, plan.run(0.85, iters).cpu().numpy())
     plan.close()
+
+
+@pytest.mark.parametrize("n,more", [(9_001, []), (9_002, [4095, 4096, 4097, 8999]), (700, [699])])
+def test_hub_rows_of_small_matrices(oracle, n, more):
+    """Rows around the length from which a work-group takes them, and around one and two rounds of its gathers."""
+    import torch
+    from drone_amd.pagerank import PullPlanF64
+    rng = np.random.default_rng(n)
+    length = rng.integers(0, 12, n)
+    at = [767, 768, 769] * (n > 1000) + more
+    length[rng.choice(n, len(at), replace=False)] = at
+    rp = np.concatenate([[0], np.cumsum(length)]).astype(np.int64)
+    ci = np.concatenate([rng.permutation(n)[:d] for d in length]).astype(np.int32)
+    outdeg = np.bincount(ci, minlength=n)
+    inv = np.where(outdeg > 0, 1.0 / np.maximum(outdeg, 1), 0.0)
+    plan = PullPlanF64(torch.from_numpy(rp).cuda(), torch.from_numpy(ci).cuda(), torch.from_numpy(inv).cuda())
+    for iters in (1, 2, 5):
+        got = plan.run(0.85, iters).cpu().numpy()
+        ref = oracle.pr_pull_f64(rp, ci, inv, 0.85, iters)
+        # as above
+        assert np.max(np.abs(got - ref) / ref) <= 2 * iters * max(length.max(), 64) * 2.0 ** -53
+    plan.close()
