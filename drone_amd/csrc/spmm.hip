@@ -62,6 +62,8 @@ struct drone_spmm_plan {
     float *val2 = nullptr;                                                   // device [long_nnz]: values in the same order
     unsigned *perm = nullptr;                                                // device [long_nnz]: sorted position -> entry
     float *partial = nullptr;                                                // device [num_pieces x ldp]
+    int *piece_long = nullptr;        // device [num_pieces]: which long row a piece is of, where pieces join their rows themselves
+    unsigned *ticket = nullptr;       // device [num_long x kMostSlices], zero between launches: pieces of a row that are done
     int ldp = 0;                                                             // max_k rounded up to 16 bytes
     int num_bands = 0, band_cols = 0;
     // dense core (see the file comment); rows and columns below are in rank order
@@ -132,6 +134,8 @@ constexpr size_t kBandBytes = 3u << 20; // feature rows of one band (three quart
 // wavefronts; us at K = 128 without / with: 4,001 vertices and 60 K entries 43 / 28, 20,003 hub-heavy ones and 0.3 M entries
 // 57 / 46, epoch on 2,708 vertices 165 / 159.  With more wavefronts than that their fixed costs count: 30,001 vertices 72 / 78.
 constexpr int kResidentWaves = 8192;
+constexpr int kMostSlices = 16;  // of a 64-lane row, down to 4 lanes
+constexpr int kJoinPieces = 4096;  // up to here pieces join their rows themselves, see JoinRows
 // For another, work-groups go round the eight XCDs in turn, so an XCD always gets the same slice (of a power of two of them):
 // its L2 holds that many times more feature rows, and a band has as many more columns.  Worth it with whole 128-byte lines,
 // slices that are all nearly full, and an operand larger than the L2s together; us without / with: 0.25 M vertices and 6 M
@@ -456,6 +460,75 @@ __device__ __forceinline__ void sum_piece(int block, int slice, int slices, int 
     }
 }
 
+// Where the pieces are few, the wavefront that ends a row's last piece adds its partial sums, in slot order as spmm_combine4_kernel does, and
+// that launch is saved.  What another XCD is to read travels as in publish_part (spmv_merge.h): through returning exchanges at
+// agent scope, waited for before the row's ticket is drawn, and read by agent-scope loads.  An exchange per float is carried
+// out at the memory side, which many pieces would wait for (574,000 in the 232,965-vertex step); a few thousand end long before
+// the chunks behind them.  us without / with: 30,011-vertex step 234 / 219, 9,001 vertices 90 / 82, 20,003 hub-heavy vertices and 0.3 M entries
+// at K = 128 38 / 32, 10,003 at K = 61 22 / 17, 0.1 M vertices and 1 M entries at K = 128 97 / 91; from some 10,000 pieces on nothing.
+struct JoinRows {
+    const int *__restrict__ piece_long;
+    const int *__restrict__ long_row;
+    const int *__restrict__ first_slot;
+    unsigned *ticket;
+};
+template <int G, int VEC>
+__device__ __forceinline__ void join_piece(int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
+                                           const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
+                                           const int *__restrict__ ci, const float *__restrict__ val,
+                                           const float *__restrict__ B, int ldb, float *partial, int ldp, int K, const JoinRows &rows,
+                                           const RowSegments &to)
+{
+    const int s = block * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (s >= num_pieces) return;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int li = lane % G, sub = lane / G;
+    const int i = rows.piece_long[s], s0 = rows.first_slot[i], s1 = rows.first_slot[i + 1];
+    unsigned one = 1u;
+    for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
+        const LaneColumns<VEC> cols{k0 + li * VEC, K};
+        float acc[VEC];
+        row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
+        if (sub == 0 && cols.active()) {
+            float *mine = partial + (size_t)piece_slot[s] * ldp + cols.at();
+            unsigned before[VEC];
+#pragma unroll
+            for (int v = 0; v < VEC; ++v)
+                before[v] = __hip_atomic_exchange(reinterpret_cast<unsigned *>(mine + v), __float_as_uint(acc[v]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) asm volatile("" : "+v"(one) : "v"(before[v]));  // the ticket is drawn once they have returned
+        }
+    }
+    // (lane 0's increment hangs on its own exchanges; the wait for them is the whole wavefront's)
+    unsigned drawn = 0;
+    if (lane == 0) drawn = atomicAdd(rows.ticket + (size_t)i * kMostSlices + slice, one);
+    if (__builtin_amdgcn_readfirstlane(drawn) != (unsigned)(s1 - s0) - 1u) return;
+    if (lane == 0) atomicExch(rows.ticket + (size_t)i * kMostSlices + slice, 0u);
+    float *dst = to.C + (size_t)rows.long_row[i] * to.ldc;
+    if (sub != 0) return;
+    for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
+        const LaneColumns<VEC> cols{k0 + li * VEC, K};
+        if (!cols.active()) continue;
+        float sum[VEC];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) sum[v] = 0.0f;
+        for (int slot = s0; slot < s1; slot += 8) {
+            float p[8][VEC];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float *src = partial + (size_t)(slot + u < s1 ? slot + u : s1 - 1) * ldp + cols.at();
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) p[u][v] = __hip_atomic_load(src + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) sum[v] += slot + u < s1 ? p[u][v] : 0.0f;
+        }
+        store_row<VEC>(dst, cols, sum, to.alpha, to.beta);
+    }
+}
+
 template <int G, int VEC>
 __global__ __launch_bounds__(kWave * kRowsPerBlock, G == 8 ? 6 : 8) void spmm_pieces_kernel(
     int num_pieces, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
@@ -479,18 +552,22 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_chunks_kernel(
 // against one launch each: training step on 30,011 vertices 280 / 263, 20 K vertices and 0.3 M entries at K = 128 74 / 57,
 // 1 M vertices and 15 M entries at K = 41 678 / 619, forward and backward over a vertex cut 757 / 715.  Not beside a bit
 // core, where a launch costs nothing and the product of 3 M vertices at K = 64 took 2,369 / 2,442.
-template <int G, int VEC>
+template <int G, int VEC, bool JOIN>
 __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_gather_kernel(
     int num_pieces, int piece_blocks, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
     const int *__restrict__ piece_slot, const int *__restrict__ ci2, const float *__restrict__ val2,
-    float *__restrict__ partial, int ldp, int num_chunks, const int4 *__restrict__ chunk, RowSegments seg,
+    float *partial, int ldp, JoinRows join, int num_chunks, const int4 *__restrict__ chunk, RowSegments seg,
     const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
     const int slices = 1 << slice_bits, block = blockIdx.x >> slice_bits, slice = blockIdx.x & (slices - 1);
-    if (block < piece_blocks)
-        sum_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
-    else
+    if (block < piece_blocks) {
+        if constexpr (JOIN)
+            join_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K, join, seg);
+        else
+            sum_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
+    } else {
         sum_chunk<G, VEC>(block - piece_blocks, slice, slices, num_chunks, chunk, seg, ci, val, B, ldb, K);
+    }
 }
 
 // C[row,:] = alpha * (sum of the row's partial pieces, in slot = (band, position) order) + beta * C[row,:]
@@ -787,9 +864,17 @@ void launch_spmm(const drone_spmm_plan *plan, const int *rp, const int *ci, cons
     const int piece_blocks = (int)ceil_div(plan->num_pieces, kRowsPerBlock), chunk_blocks = (int)ceil_div(plan->num_chunks, kRowsPerBlock);
     const RowSegments rows{rp, C, ldc, alpha, beta};
     if (piece_blocks > 0 && chunk_blocks > 0 && plan->bits.tiles == 0) {
-        spmm_gather_kernel<G, VEC><<<((unsigned)piece_blocks + (unsigned)chunk_blocks) << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
-            plan->num_pieces, piece_blocks, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2,
-            plan->partial, plan->ldp, plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
+        const JoinRows join{plan->piece_long, plan->long_row, plan->first_slot, plan->ticket};
+        const auto launch = [&](auto kernel) {
+            kernel<<<((unsigned)piece_blocks + (unsigned)chunk_blocks) << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
+                plan->num_pieces, piece_blocks, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2,
+                plan->partial, plan->ldp, join, plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
+        };
+        if (plan->ticket) {
+            launch(spmm_gather_kernel<G, VEC, true>);
+            return;
+        }
+        launch(spmm_gather_kernel<G, VEC, false>);
     } else {
         if (piece_blocks > 0)
             spmm_pieces_kernel<G, VEC><<<(unsigned)piece_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
@@ -1003,8 +1088,8 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
         std::vector<int> first_slot((size_t)num_long + 1, 0);
         for (int i = 0; i < num_long; ++i) first_slot[i + 1] = first_slot[i] + pieces_of_row[i];
         const int num_pieces = first_slot[num_long];
-        std::vector<int> cursor(first_slot.begin(), first_slot.end() - 1), pb, pe, ps;
-        pb.reserve(num_pieces); pe.reserve(num_pieces); ps.reserve(num_pieces);
+        std::vector<int> cursor(first_slot.begin(), first_slot.end() - 1), pb, pe, ps, pl;
+        pb.reserve(num_pieces); pe.reserve(num_pieces); ps.reserve(num_pieces); pl.reserve(num_pieces);
         int dense_rows = 0;
         while (dense_rows < num_long && dense_width_of_long[by_rank[dense_rows]] > 0) ++dense_rows;
         std::vector<int> seg_begin((size_t)dense_rows, 0), seg_end((size_t)dense_rows, 0);
@@ -1024,6 +1109,7 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
                 pb.push_back((int)b);
                 pe.push_back((int)(b + piece < end ? b + piece : end));
                 ps.push_back(cursor[i]++);
+                pl.push_back(i);
             }
             pos = end;
         }
@@ -1038,6 +1124,13 @@ int build_band_pieces(drone_spmm_plan *p, const std::vector<int> &h_rp, const st
         DRONE_HIP_TRY(hipMemcpy(p->piece_begin, pb.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
         DRONE_HIP_TRY(hipMemcpy(p->piece_end, pe.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
         DRONE_HIP_TRY(hipMemcpy(p->piece_slot, ps.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
+        if (dense_rows == 0 && p->num_chunks > 0 && num_pieces <= kJoinPieces) {
+            const std::vector<unsigned> zero((size_t)num_long * kMostSlices, 0u);
+            DRONE_HIP_TRY(hipMalloc(&p->piece_long, sizeof(int) * (size_t)num_pieces));
+            DRONE_HIP_TRY(hipMalloc(&p->ticket, sizeof(unsigned) * zero.size()));
+            DRONE_HIP_TRY(hipMemcpy(p->piece_long, pl.data(), sizeof(int) * (size_t)num_pieces, hipMemcpyHostToDevice));
+            DRONE_HIP_TRY(hipMemcpy(p->ticket, zero.data(), sizeof(unsigned) * zero.size(), hipMemcpyHostToDevice));
+        }
         // 5. the dense part: bits for a scaled pattern, fp32 rectangles otherwise
         if (dense_rows > 0 && p->scaled) {
             std::vector<int> h_row((size_t)dense_rows), h_width((size_t)dense_rows);
@@ -1282,6 +1375,8 @@ extern "C" int drone_spmm_plan_destroy(drone_spmm_plan *p)
     (void)hipFree(p->val2);
     (void)hipFree(p->perm);
     (void)hipFree(p->partial);
+    (void)hipFree(p->piece_long);
+    (void)hipFree(p->ticket);
     (void)hipFree(p->dense_row);
     (void)hipFree(p->dense_seg_begin);
     (void)hipFree(p->dense_seg_end);

@@ -88,3 +88,33 @@ def test_bits_at_any_alignment(monkeypatch, K, ld):
         # 1,250 entries a row: as many roundings of 2^-24
         assert np.max(np.abs(got[:, :K] - (0.75 * want + beta * C0[:, :K])) / bound) <= 1.5e-4, beta
     plan.close()
+
+
+def test_pieces_join_their_rows_again_and_again():
+    """One plan, products of several widths in turn, with and without what was there before: the rows' tickets start over each time."""
+    import torch
+    from drone_amd import gcn
+    rng = np.random.default_rng(12)
+    n_cols = 6000
+    lengths = np.concatenate([rng.integers(0, 40, 500), [513, 640, 641, 1025, 5999, 6000, 700, 2049]])
+    indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.permutation(n_cols)[:d]) for d in lengths]).astype(np.int32)
+    m = sp.csr_matrix((rng.uniform(-1, 1, indptr[-1]).astype(np.float32), cols, indptr), shape=(len(lengths), n_cols))
+    rp, ci, v = (torch.from_numpy(a).cuda() for a in (indptr, m.indices, m.data))
+    B = rng.uniform(-1, 1, (n_cols, 260)).astype(np.float32)
+    Bd, C0 = torch.from_numpy(B).cuda(), torch.from_numpy(rng.uniform(-1, 1, (len(lengths), 260)).astype(np.float32)).cuda()
+    plan = gcn.SpmmPlan(rp, ci, v, n_cols, max_k=260)
+    want, scale = m.astype(np.float64) @ B.astype(np.float64), abs(m).astype(np.float64) @ np.abs(B.astype(np.float64))
+    first = {}
+    for turn in range(12):
+        for K, beta in ((3, 0.0), (61, 1.0), (128, 0.0), (7, 1.0), (260, 0.0), (64, 1.0)):
+            out = C0.clone()
+            gcn.spmm(plan, rp, ci, v, Bd, K=K, out=out, beta=beta)
+            if turn == 0:
+                first[K] = out
+                got, before = out.cpu().numpy(), C0.cpu().numpy()
+                # 6,000 entries a row: chains of 750 and 47 partial sums, far below as many roundings of 2^-24
+                assert np.max(np.abs(got[:, :K] - (want + beta * before)[:, :K]) / (scale + np.abs(before))[:, :K]) <= 6000 * 2.0 ** -24
+                assert np.array_equal(got[:, K:], before[:, K:])
+            assert torch.equal(out, first[K])
+    plan.close()
