@@ -177,7 +177,7 @@ struct LossScratch {
 
 // A work-group's part of sum x[i]^2, in double: every lane four independent chains (one chain of dependent loads and fp64 adds
 // in a single work-group took 117 us for the 77,056 weights of a 602 x 128 layer).  Valid in thread 0.
-__device__ __forceinline__ double squares_part(const float *__restrict__ x, int64_t n, int block, int blocks, double *s_red)
+__device__ __forceinline__ double squares_part(const float *__restrict__ x, int64_t n, int block, int blocks)  // this lane's
 {
     const int64_t step = (int64_t)blocks * kThreads;
     double t[4] = {0.0, 0.0, 0.0, 0.0};
@@ -190,19 +190,28 @@ __device__ __forceinline__ double squares_part(const float *__restrict__ x, int6
         t[3] += (double)d * (double)d;
     }
     for (; i < n; i += step) t[0] += (double)x[i] * (double)x[i];
-    return block_sum_256((t[0] + t[1]) + (t[2] + t[3]), s_red);
+    return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
+template <typename V>
+__device__ __forceinline__ V sum_of_lanes(V v)
+{
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
+    return v;
 }
 
 // The loss, the gradient, and what is reported with them, in one launch: the last work-group adds the parts of all.
 // Work-groups past row_blocks add up the squares of the weights meanwhile.  A training step and the report of its loss
 // spent five launches and three copies on this (cross-entropy and its finish, accuracy and the clearing of its counts,
 // sum of squares; ~5 us each where the graph is small): an epoch with its evaluation on 2,708
-// vertices 310 -> 190 us.
+// vertices 310 -> 190 us.  (The five sums share a barrier on either side of the hand-over: 8.2 -> 6.3 us there.)
 template <int L>
 __global__ __launch_bounds__(kThreads) void loss_kernel(drone_loss_pass p, int row_blocks, LossScratch scratch)
 {
     constexpr int R = kWave / L, kWaves = kThreads / kWave, U = kCeGroups;
-    __shared__ double s_red[5][kWaves], s_part[5];
+    __shared__ double s_red[5][kWaves];
+    static_assert(kWaves == 4, "the sums of four wavefronts");
     const int n = p.n, classes = p.classes, ld = p.ld, ldg = p.ldg;
     const float *__restrict__ logits = p.logits;
     const int *__restrict__ truth = p.truth;
@@ -214,7 +223,7 @@ __global__ __launch_bounds__(kThreads) void loss_kernel(drone_loss_pass p, int r
     int cnt = 0, correct = 0, counted = 0;
     double squares = 0.0;
     if ((int)blockIdx.x >= row_blocks)
-        squares = squares_part(p.weights, p.weight_count, (int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks, s_red[4]);
+        squares = squares_part(p.weights, p.weight_count, (int)blockIdx.x - row_blocks, (int)gridDim.x - row_blocks);
     const int mean_over = p.mean_over && grad ? *p.mean_over : 0;
     const float grad_scale = p.mean_over ? (mean_over > 0 ? 1.0f / (float)mean_over : 1.0f) : p.grad_scale;
     for (int64_t base = ((int64_t)blockIdx.x * kWaves + wave) * R * U; base < n && (int)blockIdx.x < row_blocks;
@@ -315,24 +324,29 @@ __global__ __launch_bounds__(kThreads) void loss_kernel(drone_loss_pass p, int r
         }
     }
     // (whole numbers below 2^53: exact)
-    const double parts[5] = {block_sum_256(loss, s_red[0]), block_sum_256((double)cnt, s_red[1]),
-                             block_sum_256((double)correct, s_red[2]), block_sum_256((double)counted, s_red[3]), squares};
-    if (threadIdx.x == 0) {
+    const auto to_lds = [&](const double (&v)[5]) {
+        if (lane == 0) {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) s_part[k] = parts[k];
-    }
-    __syncthreads();
+            for (int k = 0; k < 5; ++k) s_red[k][wave] = v[k];
+        }
+        __syncthreads();
+    };
+    const auto of_block = [&](int k) { return (s_red[k][0] + s_red[k][1]) + (s_red[k][2] + s_red[k][3]); };
+    to_lds({sum_of_lanes(loss), (double)sum_of_lanes(cnt), (double)sum_of_lanes(correct), (double)sum_of_lanes(counted), sum_of_lanes(squares)});
     unsigned int one = 0;
     // five lanes, one instruction: it has returned for all of them when it has for thread 0
-    if (threadIdx.x < 5) one = publish_part(scratch.part + threadIdx.x * kLossBlocks + blockIdx.x, s_part[threadIdx.x]);
+    if (threadIdx.x < 5) one = publish_part(scratch.part + threadIdx.x * kLossBlocks + blockIdx.x, of_block(threadIdx.x));
     if (!last_block_done(scratch.ticket, one)) return;
     double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (int i = threadIdx.x; i < (int)gridDim.x; i += kThreads)
 #pragma unroll
         for (int k = 0; k < 5; ++k) sum[k] += load_agent(scratch.part + k * kLossBlocks + i);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) sum[k] = block_sum_256(sum[k], s_red[k]);
+    for (int k = 0; k < 5; ++k) sum[k] = sum_of_lanes(sum[k]);
+    to_lds(sum);
     if (threadIdx.x != 0) return;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) sum[k] = of_block(k);
     const float mean = (float)(sum[0] / sum[1]);  // over the labelled rows
     if (p.loss) *p.loss = mean;
     if (p.labelled) *p.labelled = (int)sum[1];

@@ -306,6 +306,7 @@ __device__ __forceinline__ unsigned int publish_part(double *slot, double v)
 // ticket_words(work-groups of the launch) device words, zero before the launch; the last drawers set them back, so
 // consecutive launches on one stream can share them.  `one`: what publish_part returned to thread 0.
 constexpr int kTicketGroup = 64;   // work-groups per first-level counter
+constexpr int kTicketDirect = 128; // up to so many work-groups draw from the launch's counter at once: a second round trip takes as long
 constexpr int kTicketStride = 32;  // words between counters: a cache line each
 inline size_t ticket_words(int64_t max_blocks)
 {
@@ -322,13 +323,19 @@ __device__ __forceinline__ bool last_block_done(unsigned int *ticket, unsigned i
         unsigned int *mine = ticket + (size_t)(group + 1) * kTicketStride;
         bool last = false;
 #if DRONE_HANDOVER_FENCED
-        if (__hip_atomic_fetch_add(mine, one, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1) {
+        if (blocks <= kTicketDirect) {
+            last = __hip_atomic_fetch_add(ticket, one, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == blocks - 1;
+            if (last) atomicExch(ticket, 0u);
+        } else if (__hip_atomic_fetch_add(mine, one, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1) {
             atomicExch(mine, 0u);
             last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
             if (last) atomicExch(ticket, 0u);
         }
 #else
-        if (atomicAdd(mine, one) == in_group - 1) {  // returns before the next draw is issued
+        if (blocks <= kTicketDirect) {
+            last = atomicAdd(ticket, one) == blocks - 1;
+            if (last) atomicExch(ticket, 0u);
+        } else if (atomicAdd(mine, one) == in_group - 1) {  // returns before the next draw is issued
             atomicExch(mine, 0u);
             last = atomicAdd(ticket, 1u) == groups - 1;
             if (last) atomicExch(ticket, 0u);
