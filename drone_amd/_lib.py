@@ -132,6 +132,7 @@ SIGNATURES = {
     "drone_sgd_step_f32": (_I, [_P, _P, _I64, _F, _P]),
     "drone_adam_step_f32": (_I, [_P, _P, _P, _P, _I64, _I, _F, _F, _F, _F, _F, _I, _P]),
     "drone_loss_pass_f32": (_I, [_P, _P]),
+    "drone_loss_pass_split_f32": (_I, [_P, _P, _P, _I, _P, _P]),
     "drone_sgd_steps_f32": (_I, [_P, _I, _F, _P]),
     "drone_adam_steps_f32": (_I, [_P, _I, _F, _F, _F, _F, _F, _I, _P]),
     "drone_fill_f32": (_I, [_P, _I64, _F, _P]),

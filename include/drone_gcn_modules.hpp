@@ -391,6 +391,12 @@ public:
         const drone_loss_pass p = pass(training);
         DRONE_GCN_CHECK(drone_loss_pass_f32(&p, s));
     }
+    // forward() with the truth of a split, which it writes to truth_out
+    void forward_on(bool training, const int *split, const int *label, int which, int *truth_out)
+    {
+        const drone_loss_pass p = pass(training);
+        DRONE_GCN_CHECK(drone_loss_pass_split_f32(&p, split, label, which, truth_out, s));
+    }
     void backward() override {}
 };
 
@@ -595,6 +601,7 @@ public:
         modules.emplace_back(graphsum2);
         ce = new CrossEntropyLoss(output, truth, p.output_dim, "CrossEntropy", s);
         modules.emplace_back(ce);
+        built_modules = modules.size();
         // cuda_gcn.cu:298-299, 314-315: what train_epoch / eval report besides the loss - the accuracy over the labelled
         // rows that are not mirrors (:226-246) and the L2 penalty weight_decay * sum(W1^2) / 2 (:254-260), from the
         // weights as they are before the optimiser step - comes out of the loss's launch
@@ -674,18 +681,33 @@ public:
     }
     std::pair<float, float> train_epoch()
     {
-        choose_truth(1);
-        train_step_async();
+        forward_on_split(true, 1);
+        backward();
+        optimizer->step();
         return read_metrics();
     }
     std::pair<float, float> eval(int current_split)  // cuda_gcn.cu:308-318
     {
-        choose_truth(current_split);
-        forward(false);
+        forward_on_split(false, current_split);
         return read_metrics();
     }
 
 private:
+    // choose_truth() and forward().  Only the loss, the last module, looks at the truth, so its launch chooses it - unless the
+    // labelled rows have to be counted first, or the program has changed the modules.
+    void forward_on_split(bool training, int current_split)
+    {
+        const bool counts_rows = params.mean_gradient && current_split != truth_split;
+        if (counts_rows || modules.size() != built_modules || modules.back().get() != ce) {
+            choose_truth(current_split);
+            forward(training);
+            return;
+        }
+        for (size_t i = 0; i + 1 < built_modules; ++i) modules[i]->forward(training);
+        ce->forward_on(training, split, label, current_split, truth);
+        truth_split = current_split;
+    }
+    size_t built_modules = 0;
     void settle_truth()  // behind a wait for the stream
     {
         if (!truth_pending) return;

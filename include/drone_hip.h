@@ -343,6 +343,10 @@ typedef struct drone_loss_pass {
     drone_loss_report *report; /* optional; device or pinned host memory */
 } drone_loss_pass;
 int drone_loss_pass_f32(const drone_loss_pass *pass, drone_stream_t stream);
+/* CUDAGCN::set_truth (cuda_gcn.cu:211-223) and the pass behind it in one launch: truth[i] = split[i] == which ? label[i] : -1 for
+ * the pass's n rows (device arrays), which the pass uses instead of pass->truth. */
+int drone_loss_pass_split_f32(const drone_loss_pass *pass, const int *split, const int *label, int which, int *truth,
+                              drone_stream_t stream);
 /* cuda_gcn.cu:226-246: a labelled row is correct unless some logit is strictly greater than the true-class
  * logit; rows with skip[row] != -1 are not counted (:234 passes Mirror2Worker, so a replicated vertex is counted
  * on its master's worker only; skip may be NULL).  counts[0] += correct, counts[1] += counted (device ints,
