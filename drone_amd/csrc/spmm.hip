@@ -5,9 +5,9 @@
 // numeric CSR transpose (cusparseCsr2cscEx2, cuda_module.cu:175-186).
 //
 // Wave shape: the 64 lanes are split into P = 64/G groups of G lanes; a group owns one non-zero at a time and
-// its lanes read VEC consecutive floats each of the K-wide feature row B[col,:] (one coalesced G*VEC*4-byte
-// read), U rows deep, so P*U feature-row loads are in flight per wave.  (col,val) pairs are read 64 at a time,
-// one per lane, and handed to the groups by cross-lane reads.
+// its lanes read VEC consecutive floats each of the K-wide feature row B[col,:], or of a slice of its columns that the
+// work-group takes (one coalesced G*VEC*4-byte read), U rows deep, so P*U feature-row loads are in flight per wave.  (col,val)
+// pairs are read 64 at a time, one per lane, and handed to the groups by cross-lane reads.
 //
 // Schedule: rows of at most kSplitRow non-zeros are taken in row order, a wavefront per chunk of consecutive rows
 // that hold at most 64 entries together (sum_chunk; fewer in small matrices).  Longer rows carry
@@ -18,7 +18,8 @@
 // long rows' entries stably sorted by (band, row) and the resulting pieces (<= piece_entries()) as a work
 // list in that order.  Work-groups are dispatched in list order, so at any moment the resident wavefronts
 // work inside one band whose feature rows stay in L2.  A piece writes its partial row to plan-owned scratch;
-// a second kernel adds each long row's partials in (band, position) order - no atomics, bitwise repeatable.
+// a second kernel adds each long row's partials in (band, position) order - no float atomics, bitwise repeatable (where the
+// pieces are few, the wavefront that ends a row's last piece does it in the same order: JoinRows).
 //
 // Dense core: power-law graphs with a high edge factor have a core (most frequent columns x longest rows) that is
 // tens of percent dense.  There a gather per non-zero moves K*4 bytes through L2 for every entry, while a dense
