@@ -233,7 +233,9 @@ __device__ __forceinline__ bool join_trees(int *cc, int a, int b)
 
 // Rows are dealt out by length, as in pull_open_kernel.  Vertices of the tree that most samples lie in - after cc_begin usually
 // most of a component with hubs - are left out: an edge from it to a vertex of another tree is in that vertex's in-row, an edge from
-// there to it in that vertex's out-row, which is looked through for those that do not come back.
+// there to it in that vertex's out-row, which is looked through for those that do not come back.  A root that has been made a
+// child of that tree meanwhile is left out too, so this holds for edges between any two trees: whichever of an edge's ends is looked
+// at sees it, and if neither is, both are in that tree.
 constexpr int kLinkThreads = 256, kLinkBlocks = 2048;
 constexpr int kLinkLane = 8, kLinkWave = 2048;  // entries up to which a row gets a lane, a wavefront
 __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows, int *cc, CcTrees *trees, int call, int pass)
@@ -259,7 +261,7 @@ __global__ __launch_bounds__(kLinkThreads) void cc_link_kernel(int n, Rows rows,
         else if (!join_trees(cc, a, b)) trees->again = pass;
     };
     const auto leaves = [&](int a, unsigned int i, int u, int b, unsigned int e0, unsigned int e1) {  // entry i of an out-row
-        if ((b == left_out || u == left_out) && b != a && !rows.comes_back(u, i, e0, e1)) trees->directed = call;
+        if (b != a && !rows.comes_back(u, i, e0, e1)) trees->directed = call;
     };
     const auto walk = [&](int row, int first, int lanes) {
         const unsigned int e0 = rows.in_index[row], e1 = rows.in_index[row + 1];
