@@ -116,9 +116,11 @@ __device__ __forceinline__ void publish_sum(double mine, double *s_red, double *
 //   cc_flatten  parent = root
 //   cc_link     joins the trees that edges lead between
 //   cc_finish   label = root, flags, and the report
-// Four launches and one wait whatever the graph's diameter: labels of 500,009 vertices and 11.5 M edges 126 -> 55 us against rounds
-// of propagation, of a path of 12,000 vertices 8.5 ms -> 49 us, of a 1,000 x 1,000 grid 18.9 ms -> 194 us, these two numbered at
-// random.  They are bound by their chains of dependent loads (row bounds, neighbour, its row, ...) and the launches.
+// Four launches and one wait whatever the graph's diameter: labels of 500,009 vertices and 11.5 M edges 126 -> 57 us against rounds
+// of propagation, of 2.4 M vertices and 30 edges each 214 -> 128, of a path of 12,000 vertices 8.5 ms -> 49 us, of a 1,000 x 1,000
+// grid 18.9 ms -> 194 us, these numbered at random; of R-MAT numbered as generated, 2.4 M vertices and 128 M edges, 85 -> 101 us,
+// half of it cc_begin's two lines of memory per vertex (looking for the way back of a parent's edge only where trees join: 78 us
+// there, but a chain of look-ups elsewhere, 500,009 vertices 92, 2.4 M 260).  They are bound by their chains of dependent loads (row bounds, neighbour, its row, ...) and the launches.
 constexpr int kCcSamples = kWave;
 constexpr int kCcSteps = 64;  // along one edge, of one cc_link: past them it is left to the next
 struct CcTrees {
