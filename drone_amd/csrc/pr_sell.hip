@@ -222,7 +222,7 @@ __global__ __launch_bounds__(kSellHotThreads) void sell_iterate_hot_kernel(
     double *__restrict__ part_out, double alpha, double inv_n, const int32_t *__restrict__ order, double *__restrict__ r_out)
 {
     constexpr int T = kSellHotThreads;
-    extern __shared__ double s_hot[];  // [kSellHot]
+    extern __shared__ __attribute__((aligned(16))) double s_hot[];  // [kSellHot], filled in pieces of 16 bytes
     __shared__ double s_dang[T / kWave], s_red[T / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int stride = (int)gridDim.x * (T / kWave);
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(kSellHotThreads) void sell_push_kernel(int n, int h
                                                                     double *part, unsigned int *ticket, StoreStat stat)
 {
     constexpr int T = kSellHotThreads, H = kSellHotF32, D = kSellDepthF32;
-    extern __shared__ float s_push[];  // [kSellHotF32]
+    extern __shared__ __attribute__((aligned(16))) float s_push[];  // [kSellHotF32], filled in pieces of 16 bytes
     __shared__ double s_red[T / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int stride = (int)gridDim.x * (T / kWave);
