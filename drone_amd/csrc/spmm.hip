@@ -46,6 +46,7 @@
 
 #include "common.h"
 #include "spmm_bits.h"
+#include "spmm_slices.h"
 
 struct drone_spmm_plan {
     int n_rows = 0, n_cols = 0;
@@ -130,26 +131,7 @@ constexpr size_t kBandBytes = 3u << 20; // feature rows of one band (three quart
 // With 2 MB bands, 10 / 15 / 24 / 32 hot bands: 5.44 / 4.83 / 4.44 / 4.44 ms (K = 128).
 // With the dense region kept as bits (scaled patterns), 3 MB x 4 / 8 / 12 / 16 / 20 / 28 / 38 / 56 hot bands: 3.45 / 3.00 / 2.85 /
 // 2.75 / 2.80 / 2.95 / 3.07 / 3.05 ms at K = 128 and 1.64 / 1.51 / 1.39 / 1.35 / 1.35 / 1.34 / 1.35 / 1.33 at K = 41.
-// Slices: the feature columns are dealt out over 2^bits work-groups per chunk or piece, each with lane groups that much
-// narrower.  For one thing that halves the serial chain of a row, in a matrix so small that the GPU still holds all the
-// wavefronts; us at K = 128 without / with: 4,001 vertices and 60 K entries 43 / 28, 20,003 hub-heavy ones and 0.3 M entries
-// 57 / 46, epoch on 2,708 vertices 165 / 159.  With more wavefronts than that their fixed costs count: 30,001 vertices 72 / 78.
-constexpr int kResidentWaves = 8192;
-constexpr int kMostSlices = 16;  // of a 64-lane row, down to 4 lanes
 constexpr int kJoinPieces = 4096;  // up to here pieces join their rows themselves, see JoinRows
-// For another, work-groups go round the eight XCDs in turn, so an XCD always gets the same slice (of a power of two of them):
-// its L2 holds that many times more feature rows, and a band has as many more columns.  Worth it with whole 128-byte lines,
-// slices that are all nearly full, and an operand larger than the L2s together; us without / with: 0.25 M vertices and 6 M
-// entries at K = 128 663 / 541, 1 M vertices and 16 M entries 1,811 / 1,640, the 232,965-vertex step 8,627 / 7,893, 1 M vertices
-// and 32 M entries at K = 256 7,976 / 6,587; but 0.2 M vertices at K = 100 (64 + 36, or 52 + 48 across lines) 312 / 372, and
-// with 32 columns a slice the step took 9,843.
-constexpr int kLineFloats = 32, kSliceCols = 2 * kLineFloats;
-constexpr int64_t kAllL2Bytes = 32 << 20;
-int line_slice_bits(int K, int n_cols)
-{
-    const int bits = K > 2 * kSliceCols ? 2 : 1, free = (kSliceCols << bits) - K;
-    return free >= 0 && free <= kSliceCols / 4 && (int64_t)n_cols * K * (int64_t)sizeof(float) > kAllL2Bytes ? bits : 0;
-}
 constexpr int kBandMaxCols = 8192;      // narrow feature rows: a band is at most this many columns
 constexpr int kRowsPerBlock = 4;        // wavefronts per work-group (2 / 4 / 8: 4.29 / 4.31 / 4.33 ms at K = 128, 2.50 / 2.45 / 2.56 at K = 41)
 constexpr int kDenseChunk = 2048;       // column granularity of the dense rectangles
@@ -1453,23 +1435,14 @@ extern "C" int drone_spmm_csr_f32(const drone_spmm_plan *plan, const int *rp, co
     if (K < 4) {
         launch_spmm<4, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
     } else {
-        // the smallest lane group that covers K, or a slice of it
-        int lanes = 4, slice_bits = line_slice_bits(K, plan->n_cols);
-        while (lanes < kWave && lanes * 4 < K) lanes *= 2;
-        if (slice_bits > 0 && ldb % kLineFloats == 0 && (uintptr_t)B % (4 * kLineFloats) == 0) {
-            lanes = kSliceCols / 4;
-        } else {
-            slice_bits = 0;
-            for (int64_t waves = (int64_t)plan->num_pieces + plan->num_chunks; lanes > 4 && 2 * waves <= kResidentWaves; waves *= 2) {
-                ++slice_bits;
-                lanes /= 2;
-            }
-        }
-        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, slice_bits, s); };
-        if (lanes == 4) launch(std::integral_constant<int, 4>());
-        else if (lanes == 8) launch(std::integral_constant<int, 8>());
-        else if (lanes == 16) launch(std::integral_constant<int, 16>());
-        else if (lanes == 32) launch(std::integral_constant<int, 32>());
+        const bool whole_lines = ldb % kLineFloats == 0 && (uintptr_t)B % (4 * kLineFloats) == 0;
+        const Slicing by = slicing(K, plan->n_cols, whole_lines, (int64_t)plan->num_pieces + plan->num_chunks,
+                                   ceil_div(plan->num_pieces, kRowsPerBlock) + ceil_div(plan->num_chunks, kRowsPerBlock), kWave * kRowsPerBlock);
+        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s); };
+        if (by.lanes == 4) launch(std::integral_constant<int, 4>());
+        else if (by.lanes == 8) launch(std::integral_constant<int, 8>());
+        else if (by.lanes == 16) launch(std::integral_constant<int, 16>());
+        else if (by.lanes == 32) launch(std::integral_constant<int, 32>());
         else launch(std::integral_constant<int, 64>());
     }
     int dense_status = DRONE_OK;
