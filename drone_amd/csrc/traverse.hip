@@ -108,19 +108,21 @@ __device__ __forceinline__ void publish_sum(double mine, double *s_red, double *
 // ---- labels by joining trees -------------------------------------------------------------------------------
 // Where every edge has its reverse, a vertex's label is the least vertex of its component, and it need not travel there hop by
 // hop: the vertices are kept as trees in cc[] itself (cc[v] = v's parent, at most v; a root is its own), an edge between two
-// trees makes the larger root a child of the smaller, and at the end every vertex takes its root's number.  Along edges whose
-// reverse is missing only rounds of the kernels below can tell; what the trees hold by then is a valid start for them, since
-// trees are only ever joined along edges that lead both ways.  So no property of the graph is assumed: every edge a tree
-// is made of is looked up in the other direction.
+// trees makes the larger root a child of the smaller, and at the end every vertex takes its root's number.  (Joining by
+// compare-and-swap on the roots, rows dealt out by length, and leaving out the tree that a sample finds largest are known from ECL-CC -
+// Jaiganesh and Burtscher, 2018 - and Afforest - Sutton, Ben-Nun and Barak, 2018.)  Along edges whose reverse is missing only
+// rounds of the kernels below can tell, so no property of the graph is assumed: a tree is joined along edges that lead both ways,
+// and every edge inside it is looked up in the other direction, which is how the label of the tree above comes to all of it.
+// The tree of vertex 0 is the exception: it is never joined to another, its label is the least there is, and the edges it is made of
+// bring that label down.  By then it holds most of the graph where there are hubs, and its vertices are spared a line of memory each.
 //   cc_begin    parent = least in-neighbour if that is smaller (rows are in ascending order: the first)
-//   cc_flatten  parent = root
+//   cc_flatten  parent = root, the edges to the parents looked up
 //   cc_link     joins the trees that edges lead between
 //   cc_finish   label = root, flags, and the report
-// Four launches and one wait whatever the graph's diameter: labels of 500,009 vertices and 11.5 M edges 126 -> 57 us against rounds
-// of propagation, of 2.4 M vertices and 30 edges each 214 -> 128, of a path of 12,000 vertices 8.5 ms -> 49 us, of a 1,000 x 1,000
-// grid 18.9 ms -> 194 us, these numbered at random; of R-MAT numbered as generated, 2.4 M vertices and 128 M edges, 85 -> 101 us,
-// half of it cc_begin's two lines of memory per vertex (looking for the way back of a parent's edge only where trees join: 78 us
-// there, but a chain of look-ups elsewhere, 500,009 vertices 92, 2.4 M 260).  They are bound by their chains of dependent loads (row bounds, neighbour, its row, ...) and the launches.
+// Four launches and one wait whatever the graph's diameter; us of a call, by rounds / with every parent looked up / this: 500,009
+// vertices and 11.6 M edges 124 / 57 / 51, 1.2 M and 33 M 175 / 89 / 81, 2.4 M and 107 M 215 / 128 / 107, R-MAT numbered as generated, 2.4 M
+// and 128 M 85 / 100 / 71, a path of 12,000 7,630 / 51 / 51, a 1,000 x 1,000 grid 17,200 / 220 / 218.  They are bound by a line of memory per
+// vertex, their chains of dependent loads (row bounds, neighbour, its row, ...) and the launches.
 constexpr int kCcSamples = kWave;
 constexpr int kCcSteps = 64;  // along one edge, of one cc_link: past them it is left to the next
 struct CcTrees {
@@ -170,19 +172,11 @@ __device__ __forceinline__ int parent_of(const int *cc, int v) { return __hip_at
 
 // cc.cu:10-20
 __global__ __launch_bounds__(kSpmvBlock) void cc_begin_kernel(int n, Rows rows, int *__restrict__ cc, int *__restrict__ ubm,
-                                                              TraverseState *__restrict__ state, CcTrees *trees, int call)
+                                                              TraverseState *__restrict__ state)
 {
     for (int v = blockIdx.x * kSpmvBlock + threadIdx.x; v < n; v += gridDim.x * kSpmvBlock) {
         const int e0 = rows.in_index[v], e1 = rows.in_index[v + 1];
-        int parent = v;
-        if (e0 < e1) {
-            const int u = rows.in_src[e0];
-            if (u < v) {
-                parent = u;
-                if (!rows.leads_back(u, v, 0)) trees->directed = call;
-            }
-        }
-        cc[v] = parent;
+        cc[v] = e0 < e1 ? min(rows.in_src[e0], v) : v;
         ubm[v] = 0;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) *state = TraverseState{everything(), 2, 1, 0, 0.0};
@@ -233,12 +227,15 @@ __device__ __forceinline__ int walk_to_root(int *cc, int v)
 
 __host__ __device__ __forceinline__ int sample_stride(int n) { return n / kCcSamples > 0 ? n / kCcSamples : 1; }
 
-__global__ __launch_bounds__(kSpmvBlock) void cc_flatten_kernel(int n, int *cc, CcTrees *trees)
+// look_up: cc_begin has just made the parents, so that they are the first entries of the in-rows.
+__global__ __launch_bounds__(kSpmvBlock) void cc_flatten_kernel(int n, Rows rows, int *cc, CcTrees *trees, int call, bool look_up)
 {
     const int stride = sample_stride(n);
     for (int v = blockIdx.x * kSpmvBlock + threadIdx.x; v < n; v += gridDim.x * kSpmvBlock) {
-        const int root = walk_to_root(cc, v);
+        const int parent = parent_of(cc, v), root = walk_to_root(cc, v);  // nobody else writes cc[v]
         if (v % stride == 0 && v / stride < kCcSamples) trees->sample[v / stride] = root;
+        if (look_up && root != 0 && parent != v && parent_of(&trees->directed, 0) != call && !rows.leads_back(parent, v, 0))
+            trees->directed = call;
     }
 }
 
@@ -1603,10 +1600,10 @@ TraverseState join_labels(Graph *g, TraverseExt *t, int *cc, hipStream_t s)
     }
     const int call = ++t->call;
     const Rows rows = rows_of(g);
-    cc_begin_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, g->updateByMessage, t->state, t->trees, call);
-    for (;;) {
+    cc_begin_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, g->updateByMessage, t->state);
+    for (bool first = true;; first = false) {
         const int pass = ++t->pass;
-        cc_flatten_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, cc, t->trees);
+        cc_flatten_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, t->trees, call, first);
         cc_link_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kLinkThreads), kLinkBlocks), kLinkThreads, 0, s>>>(n, rows, cc, t->trees, call, pass);
         cc_finish_kernel<<<sum_blocks(n, 1), kSpmvBlock, 0, s>>>(n, cc, g->active, t->trees, call, pass, t->block_part, t->ticket, t->report);
         DRONE_HIP_OR_DIE(hipGetLastError());

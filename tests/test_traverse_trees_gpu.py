@@ -137,3 +137,32 @@ def test_one_edge_without_reverse_between_components(oracle, size, into_the_larg
             np.testing.assert_array_equal(w.read(), want)
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("one_way", [0.0, 0.02, 0.3])
+@pytest.mark.parametrize("first_tree", ["few", "half", "most"])
+def test_edges_of_the_first_tree_need_not_lead_back(oracle, first_tree, one_way):
+    """Random graphs whose vertex 0 is in the tree of few, half or most of the vertices, by edges of which some lead one way, and
+    whose other edges have their reverse, all but some: what the tree of vertex 0 is made of is not looked up in the other direction."""
+    from drone_amd.traverse import CCWorkerCUDA
+    rng = np.random.default_rng([len(first_tree), int(100 * one_way)])
+    for n in (2, 3, 65, 700, 5_000, 70_003):
+        first = rng.permutation(np.arange(1, n))[:int(n * {"few": 0.05, "half": 0.5, "most": 0.95}[first_tree])]
+        down_u, down_v = np.zeros(len(first), np.int64), first           # 0 -> its tree
+        back = rng.random(len(first)) >= max(one_way, 0.3)               # some of them lead back
+        a, b = rng.integers(0, n, (2, n // 3 + 1))                       # any two vertices, this edge
+        there = rng.random(len(a)) >= one_way                            # and its reverse
+        own = np.arange(n)                                               # (numbers go by first appearance)
+        u = np.concatenate([own, down_u, down_v[back], a, b[there]]).astype(np.int32)
+        v = np.concatenate([own, down_v, down_u[back], b, a[there]]).astype(np.int32)
+        _, l2g, _, index, dst = oracle.build_graph(n, u, v)
+        assert np.array_equal(l2g, own)
+        want = _labels(n, index, dst)
+        w = CCWorkerCUDA(n, u, v)
+        try:
+            for _ in range(2):
+                w.peval()
+                np.testing.assert_array_equal(w.read(), want)
+                np.testing.assert_array_equal(w.flags()["active"] > 0, want < own)
+        finally:
+            w.close()
