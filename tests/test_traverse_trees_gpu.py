@@ -166,3 +166,33 @@ def test_edges_of_the_first_tree_need_not_lead_back(oracle, first_tree, one_way)
                 np.testing.assert_array_equal(w.flags()["active"] > 0, want < own)
         finally:
             w.close()
+
+
+def test_one_way_edge_into_a_root_that_is_joined_before_its_row_is_due(oracle):
+    """Rows come to cc_link's work-groups 64 at a time, piece i to work-group i mod 2,048, and past 524,288 vertices a work-group has a second
+    round of them.  Here work-group 0 has a row of half a million entries in its first round and vertex r in its second; by then
+    work-group 1 has looked at the vertex that an edge leads from to r, one way, and, in its second round, joined r to the tree that most
+    samples lie in, whose vertices are left out.  The edge carries the least label into all of that tree."""
+    from drone_amd.traverse import CCWorkerCUDA
+    work_groups, piece, samples = 2048, 64, 64
+    second = 4 * work_groups * piece
+    n = second + 16 * piece
+    largest, hub, r, y, q, z = 2, 3, second, second + piece, second + piece + 1, second + 5 * piece
+    own = np.arange(n)
+    sampled = own[::n // samples][1:samples]
+    sampled = sampled[sampled < second]
+    many = np.setdiff1d(np.arange(2 * piece, second), sampled)
+    pairs = [(0, q), (r, y), (y, z), (largest, z)] + [(largest, int(v)) for v in sampled]
+    a, b = np.concatenate([np.array(pairs).T, np.stack([np.full_like(many, hub), many])], 1)
+    u, v = np.concatenate([own, a, b, [q]]).astype(np.int32), np.concatenate([own, b, a, [r]]).astype(np.int32)
+    _, l2g, _, index, dst = oracle.build_graph(n, u, v)
+    assert np.array_equal(l2g, own)
+    want = _labels(n, index, dst)
+    assert want[r] == want[y] == want[z] == want[largest] == 0 and np.all(want[sampled] == 0) and np.all(want[many] == hub)
+    for _ in range(3):  # (a graph that has shown an edge without its reverse is not tried again)
+        w = CCWorkerCUDA(n, u, v)
+        try:
+            w.peval()
+            np.testing.assert_array_equal(w.read(), want)
+        finally:
+            w.close()
