@@ -98,8 +98,9 @@ struct GraphExt {
     RowBlocks rb;             // over the in-edge CSR with its sources renumbered hot-first
     MergeScratch ms_rb;
     int32_t *rb_new_id = nullptr;  // device [n]: local id -> renumbered id (where a vertex's push value is kept)
-    // mid-size subgraphs: sliced rows with the hottest sources in LDS (pr_sell.h, built by loadOutDegree); numbered by rb_new_id as well
+    // mid-size subgraphs: sliced rows with the hottest sources in LDS (pr_sell.h), after some supersteps without; numbered by rb_new_id as well
     bool sell_tried = false, sell_ready = false;
+    int64_t merge_supersteps = 0;
     SellRows sell;
     double *sell_part = nullptr;       // device [kSellHotBlocks]
     unsigned int *sell_ticket = nullptr;  // device [ticket_words(kSellHotBlocks)], zero between launches

@@ -219,16 +219,18 @@ void exchange_push(Graph *g, PRValues *values, int workerId, int workerNum, Comm
 // DRONE_PR_ROWBLOCK_MIN_EDGES in the environment moves the limit for jobs that run longer or shorter.
 constexpr int64_t kRowBlockMinEdges = 24ll << 20;
 
-int64_t row_block_min_edges()
+int64_t from_environment(const char *name, int64_t otherwise)
 {
-    const char *env = getenv("DRONE_PR_ROWBLOCK_MIN_EDGES");
+    const char *env = getenv(name);
     if (env && *env) {
         char *end = nullptr;
         const long long v = strtoll(env, &end, 10);
         if (end != env && *end == '\0' && v >= 0) return v;
     }
-    return kRowBlockMinEdges;
+    return otherwise;
 }
+
+int64_t row_block_min_edges() { return from_environment("DRONE_PR_ROWBLOCK_MIN_EDGES", kRowBlockMinEdges); }
 
 __global__ void widen_offsets_kernel(const int *in, int64_t *out, int count)
 {
@@ -253,14 +255,22 @@ void sell_rows_release(GraphExt *x)
 }
 
 // Sliced rows with the hottest sources in LDS (sell_push_kernel), once per graph, where there are enough edges and enough of them lead
-// from these.  A superstep of 900,001 vertices and 13.5 M edges, merge path / these: 99 / 70 us; 0.4 M vertices and 6 M edges 59 / 46, 2 M
-// and 15 M 125 / 107, 0.3 M and 3.5 M 42 / 42.  Building them takes about 1 ms, which such a job has back after 40 supersteps; it
-// belongs to what is prepared for PageRank, so loadOutDegree does it, not the first superstep (1.37 -> 1.05 ms of ten).  Any failure (memory) leaves the
-// merge path in place.
+// from these.  A superstep of 900,001 vertices and 13.5 M edges, merge path / these: 100 / 68 us; 0.4 M vertices and 6 M edges 59 / 46, 2 M
+// and 15 M 125 / 107, 0.3 M and 3.5 M 42 / 42.  Building them takes 0.9 ms (0.4 M vertices 0.5), which 20 to 40 supersteps give
+// back, and 12 ms more in a process that has not run these kernels yet, which takes 400.  So a graph gets them once it has had
+// kSlicedRowsAfter supersteps on the merge path: a job to eps, some 85 supersteps, costs what it did without them, a graph that
+// serves more than that has them before long, and the superstep that builds them shows it in its CalTime.  (Built in loadOutDegree
+// it and a first job of ten supersteps took 2.2 ms instead of 1.6, in a new process 14.5 instead of 2.4.)  Sums before and after
+// are added in another order.  DRONE_PR_SLICED_ROWS_AFTER in the environment moves the number.  Any failure (memory) leaves the merge
+// path in place.
+constexpr int64_t kSlicedRowsAfter = 128;
+
+// At the start of a superstep, before its vertex kernel: that decides where push values are kept.
 void ensure_sell_rows(Graph *g, hipStream_t s)
 {
     GraphExt *x = static_cast<GraphExt *>(g->ext);
-    if (x->sell_tried || x->edges >= std::min(row_block_min_edges(), kRowBlockMinEdges) || !sell_f32_suits(x->n, x->edges)) return;
+    if (x->sell_tried || x->rb_ready || x->edges >= std::min(row_block_min_edges(), kRowBlockMinEdges) || !sell_f32_suits(x->n, x->edges)) return;
+    if (x->merge_supersteps++ < from_environment("DRONE_PR_SLICED_ROWS_AFTER", kSlicedRowsAfter)) return;
     x->sell_tried = true;
     int rc = DRONE_OK;
     const size_t words = ticket_words(kSellHotBlocks);
@@ -292,10 +302,7 @@ void ensure_row_blocks(Graph *g, hipStream_t s)
     GraphExt *x = static_cast<GraphExt *>(g->ext);
     if (x->rb_tried || x->sell_ready) return;
     x->rb_tried = true;
-    if (x->edges < row_block_min_edges() || x->edges == 0) {
-        ensure_sell_rows(g, s);
-        return;
-    }
+    if (x->edges < row_block_min_edges() || x->edges == 0) return;
     int64_t *row_ptr = nullptr;
     Relabel rl;
     int rc = DRONE_OK;
@@ -409,7 +416,6 @@ extern "C" void loadOutDegree(Graph *g, PRValues *values, int *globalOutDegree)
     set_out_degree_kernel<<<1024, 256>>>(values->outDegree, d_global, g->Local2Global, n);
     DRONE_HIP_OR_DIE(hipDeviceSynchronize());
     (void)hipFree(d_global);
-    ensure_sell_rows(g, nullptr);
 }
 
 extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm)
@@ -426,7 +432,8 @@ extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int worke
         printf("Failed: PR_PEVal before loadOutDegree\n");
         exit(EXIT_FAILURE);
     }
-    ensure_row_blocks(g, s);  // before the first vertex kernel: it decides where push values are kept
+    ensure_row_blocks(g, s);
+    ensure_sell_rows(g, s);
     if (!push_slot_of(g)) ensure_aggregation_ready(g);
     // pr.cu:383-389: the state vectors are allocated by this call
     if (!g->active) DRONE_HIP_OR_DIE(hipMalloc(&g->active, sizeof(int) * cnt));
@@ -486,6 +493,7 @@ extern "C" Response PR_IncEVal(Graph *g, PRValues *values, int workerId, int wor
     }
     PRExt *px = static_cast<PRExt *>(values->ext);
     const int n = getLocalVertexSize(g), nglobal = getGlobalVertexSize(g);
+    ensure_sell_rows(g, s);
     pr_increment_vertex_kernel<<<px->vertex_blocks, kSpmvBlock, 0, s>>>(
         n, nglobal, values->outDegree, g->Mirror2Worker, values->prValue, values->accValue, values->diffValue,
         values->globalAcc, values->globalDiff, px->push, push_slot_of(g), g->updateByMessage, px->block_part,

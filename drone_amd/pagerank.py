@@ -173,8 +173,7 @@ class PRWorkerCUDA:
         return out
 
     def aggregation(self):
-        """'row-blocks', 'sliced-rows' or 'merge-path': the kernels PR_PEVal / PR_IncEVal use for this graph (decided by the
-        first peval)."""
+        """'row-blocks', 'sliced-rows' or 'merge-path': the kernels that the last PR_PEVal / PR_IncEVal of this graph used."""
         return ("merge-path", "row-blocks", "sliced-rows")[lib().drone_pr_aggregation(self.g)]
 
     def close(self):

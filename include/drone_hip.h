@@ -121,13 +121,16 @@ void loadOutDegree(Graph *g, PRValues *values, int *globalOutDegree);
  * A subgraph of 24 Mi edges or more gets a second, source-sorted copy of its in-edges at the first PR_PEVal
  * (about 10 bytes per edge and 4 ... 16 ms for 32 ... 263 M edges), which takes a third to a half off every superstep
  * after it; the environment variable DRONE_PR_ROWBLOCK_MIN_EDGES (an edge count, read at the first PR_PEVal of
- * each graph) moves that limit, e.g. 0 for jobs that run many supersteps on smaller subgraphs. */
+ * each graph) moves that limit, e.g. 0 for jobs that run many supersteps on smaller subgraphs.
+ * A smaller subgraph of 4 Mi vertices and edges or more, whose edges mostly lead from few vertices, gets its in-edges in
+ * slices once it has had 128 supersteps (DRONE_PR_SLICED_ROWS_AFTER supersteps, read at every superstep until then): about
+ * 1 ms in the CalTime of that one, a quarter to a third off those after it. */
 Response PR_PEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm);
 Response PR_IncEVal(Graph *g, PRValues *values, int workerId, int workerNum, Comm *comm);
 
 /* No counterpart in the reference: which kernels PR_PEVal / PR_IncEVal aggregate this graph with.  0 = merge
- * path (also before the first PR_PEVal has decided), 1 = source-sorted row blocks, 2 = sliced rows with the hottest
- * sources in LDS. */
+ * path (also before the first PR_PEVal has decided, or enough supersteps for slices have passed), 1 = source-sorted row
+ * blocks, 2 = sliced rows with the hottest sources in LDS. */
 int drone_pr_aggregation(const Graph *g);
 
 /* No counterpart in the reference (it never frees): optional clean-up. */
