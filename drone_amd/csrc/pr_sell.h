@@ -33,8 +33,11 @@ namespace drone {
 constexpr int kSellClasses = 7;      // P = 64, 32, ..., 1
 constexpr int kSellDepth = 8;        // most entries of a lane in a slice with P < 64; gathers in flight per lane
 // Gathers in flight per lane of a hub row's work-group, and most steps of a slice with P = 64 (longer rows are hubs) without / with
-// the hottest sources in LDS.  In a small matrix the longest rows are what a launch waits for; us per run of 20 iterations at 4 K /
-// 64 K vertices with 8 in flight and 16 steps 93 / 179, 16 and 16 94 / 165, 16 and 12 86 / 158, 16 and 8 86 / 161, 16 and 4 85 / 175.
+// the hottest sources in LDS.  In a small matrix the longest rows are what a launch waits for.  Runs of 20 iterations at 18 sizes, 700
+// to 100,003 vertices and 4 to 30 entries a row, against 8 in flight and 16 steps, geometric mean and the two ends: 16 and 12 1.038 times as
+// fast (40,009 vertices with 8 entries 119 -> 100 us, with 20 entries 130 -> 138), 12 and 10 1.041 (119 -> 100; 100,003 with 9 163 -> 170),
+// 16 and 8 1.035 (119 -> 100; 130 -> 137), 12 and 12 1.034 (119 -> 100; 130 -> 135), 8 and 8 1.029, 8 and 12 1.020, 16 and 14 1.014: as good
+// as any, and the best at R-MAT scale 16 with 16 entries (178 -> 162; 12 and 10 168, 12 and 12 169).
 constexpr int kSellHubDepth = 16, kSellWaveSteps = 12, kSellWaveStepsWide = 16;
 constexpr int kSellDepthF32 = 16, kSellWaveStepsF32 = 32;  // the same of float rows
 constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,000 of 163,840 bytes
