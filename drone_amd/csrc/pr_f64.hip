@@ -241,6 +241,14 @@ extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
     return DRONE_OK;
 }
 
+extern "C" int drone_pr_plan_patience(drone_pr_plan *p, int looks)
+{
+    clear_error();
+    DRONE_REQUIRE(p != nullptr && looks >= 0, "number of looks");
+    p->sr.patience = looks;
+    return DRONE_OK;
+}
+
 extern "C" int drone_pr_profile_enable(drone_pr_plan *p, int max_launches)
 {
     clear_error();
@@ -302,6 +310,7 @@ extern "C" int drone_pr_run_f64(drone_pr_plan *p, double alpha, int iters, doubl
     }
     // the caller may have refreshed inv_outdeg since the plan was made: re-read it every run (8N bytes)
     if (p->sell) {
+        if (p->sr.resident && iters >= kSellResidentIters && p->prof_n >= p->prof_cap) return sell_run(p->sr, p->inv_user, iters, alpha, rank_out, s);
         int rc = sell_begin(p->sr, p->inv_user, s);
         for (int it = 0; it < iters && rc == DRONE_OK; ++it) {
             const bool prof = p->prof_n < p->prof_cap;

@@ -58,6 +58,13 @@ struct SellRows {
     double *inv = nullptr;           // device [n]: inverse out-degrees in row order, refreshed by every run
     double *part[2] = {nullptr, nullptr};  // device: dangling mass per work-group, of this iteration and the one before
     int init_blocks = 0;
+    int patience = 64;               // looks at the gate before a work-group of it does the run alone
+    int resident = 0;                // work-groups of sell_resident_kernel, or 0: a launch per iteration
+    int staged = 0;                  // slots that a lane of it brings into LDS
+    size_t lds = 0;                  // bytes of its sources in LDS
+    int live = 0, live_slices = 0;   // rows with entries, and the slices that have one of them
+    unsigned long long *exchange = nullptr;  // device [4 n]: its sources on their way, kSellNone between runs
+    unsigned *gate = nullptr;        // device [2 * kTicketStride]: who has come and who has left, 0 between runs
     DeviceArena arena;               // everything above
     DeviceArena entries;             // hub_col and col, whose sizes are known last
 };
@@ -79,5 +86,9 @@ void sell_destroy(SellRows *sr);
 // its dangling mass; sell_iterate is one iteration (it = 0, 1, ...), the last of which passes rank_out.
 int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t stream);
 int sell_iterate(const SellRows &sr, int it, double alpha, double *rank_out, hipStream_t stream);
+// A whole run of iters >= 1 in one launch, where sr.resident is not 0.  Worth it from kSellResidentIters on: entering costs what two launches
+// do (4 K vertices and 53 K entries, us for 1, 2, 3 and 20 iterations: 9.3, 11.9, 13.7, 48 instead of 7.2, 11.8, 16.6, 86).
+constexpr int kSellResidentIters = 3;
+int sell_run(const SellRows &sr, const double *inv_user, int iters, double alpha, double *rank_out, hipStream_t stream);
 
 }  // namespace drone

@@ -28,6 +28,11 @@ constexpr int kSellSamples = 1 << 16;
 constexpr size_t kSellHotLds = sizeof(double) * kSellHot;
 static_assert(kSellInitBlocks <= kSellHotThreads && kSellHotBlocks <= kSellHotThreads, "a partial per lane");
 static_assert(sizeof(float) * kSellHotF32 == kSellHotLds, "the same LDS");
+// Whole runs in one launch of up to kSellResidentBlocks work-groups, kSellResidentSlices slices to each as long as there are no more: a
+// wavefront per SIMD gathers, and the fewer work-groups read every source the better (1 K vertices, 12 K entries, us per iteration with 1, 2, 4
+// and 8 slices a work-group 1.45, 1.31, 1.26, 1.33; up to 128 work-groups at 8 K vertices 2.6 instead of 2.4).
+constexpr int kSellResidentBlocks = 64, kSellResidentSlices = 4, kSellStaged = 12;
+constexpr size_t kSellResidentLds = 152 << 10;  // of 160; the kernel's own arrays are 1
 constexpr int kSellMassLoads = 4;  // partials of the dangling mass per lane that are requested ahead
 
 // What a kernel needs of SellRows, by value.
@@ -158,6 +163,355 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
     }
     const double total = block_sum<T>(stat, s_red);
     if (tid == 0) part_out[blockIdx.x] = total;
+}
+
+// ---- whole runs in one launch -----------------------------------------------------------------------------------------
+// Runs of a launch per iteration wait for launches: 2.3 us each, and then a chain of descriptor, ids and gathers out of a cold cache (4.1 us
+// per iteration at 500 vertices as at 4 K).  What is left here is one trip of a value to memory and back (1.2 us for 1 K values between
+// any number of work-groups, 1.4 for 4 K), bringing the sources into LDS at 30 bytes a cycle, and the chains of gathers and lane
+// sums in between.  20 iterations, us, a launch per iteration / this: 500 vertices and 2 K entries 69 / 32, 4 K and 53 K 86 / 48, 6 K and
+// 43 K 86 / 50, 12 K and 115 K 98 / 69, 12 K and 343 K 102 / 80.  More slices than wavefronts lose: 8 K and 595 K 102 / 139, 12 K and 622 K
+// 119 / 170; so do more hub rows than work-groups (4 K and 464 K, 3 iterations 16.9 / 19.8, 20 96.7 / 93.5).  All 1,024 lanes bring sources
+// in, the slots' loads and the LDS writes without a bounds check (with one 2.05 -> 2.4 us per iteration); work-groups of 256 or 512
+// lanes take longer from 2 K vertices on (4 K 2.9 and 2.3 instead of 2.0).
+//
+// Small matrices: the work-groups stay for the whole run, with the entries of their rows in registers and all sources in LDS, and
+// hand each other the new sources through memory.  A source is its own flag: a slot that holds kSellNone (a NaN that no sum makes)
+// is not written yet, so a value that is there is the value, and no order between different slots is needed to read it.  Slots are
+// 8-byte relaxed atomics at agent scope, which every XCD reads and writes at the same place.
+//
+// Four sets of slots.  Iteration `it` reads set it, writes set it + 1, and its owners clear set it - 1 (indexes modulo 4): whoever
+// holds all of set it knows that every work-group, each of which owns a row, has finished reading set it - 1.  Set it - 1 is written
+// again two iterations on and looked at three on; the owner waits for its clearing store (which writes through) before it publishes
+// again, and who looks at the set has read what it published then.  The last work-group to leave clears the last set, and the counters.
+//
+// The work-groups wait for each other, so all must have a place on the chip before any starts.  Each reports at a gate; one that
+// has looked `patience` times in vain closes it and does the whole run alone, and the others go.  (Behind a gate that has opened
+// all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long goes on with the NaN.)
+constexpr int kSellResidentThreads = 1024;
+constexpr unsigned long long kSellNone = 0x7ffc5e1100a1b2c3ull, kSellNan = 0x7ff8000000000000ull;
+constexpr unsigned kSellClosed = 1u << 31;
+constexpr int kSellPolls = 1 << 22;
+constexpr int kSellWaitStores = 0x0f70;  // s_waitcnt vmcnt(0)
+
+__device__ __forceinline__ void slot_store(unsigned long long *p, unsigned long long v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ unsigned long long slot_load(const unsigned long long *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+__device__ __forceinline__ bool slot_is_none(unsigned long long v) { return (unsigned)(v >> 32) == (unsigned)(kSellNone >> 32); }
+
+// Four sets of `slots` slots of which `used` are.
+__global__ void sell_slots_kernel(int slots, int used, unsigned long long *__restrict__ exchange, unsigned *__restrict__ gate)
+{
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 4 * slots; i += gridDim.x * blockDim.x)
+        exchange[i] = i % slots < used ? kSellNone : 0;
+    if (blockIdx.x == 0 && threadIdx.x < 2 * kTicketStride) gate[threadIdx.x] = 0;
+}
+
+// Through the gate: this work-group's number among `groups`, or -1 to leave.  ticket: how many came before.
+__device__ __forceinline__ int sell_enter(unsigned *gate, unsigned ticket, int &groups, int patience)
+{
+    const unsigned all = gridDim.x;
+    unsigned seen = ticket + 1;
+    for (int looks = 0;; ++looks) {
+        if (seen & kSellClosed) return -1;
+        if (seen == all && patience > 0) return (int)ticket;
+        if (looks >= patience) {
+            unsigned expected = seen;
+            if (__hip_atomic_compare_exchange_strong(gate, &expected, seen | kSellClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                groups = 1;
+                return 0;
+            }
+        }
+        seen = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+template <int Ctrl>
+__device__ __forceinline__ double dpp_add(double v)
+{
+    const long long bits = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)bits, Ctrl, 0xf, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(bits >> 32), Ctrl, 0xf, 0xf, true);
+    return v + __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+template <int Lanes>
+__device__ __forceinline__ double swap_add(double v)
+{
+    const long long bits = __double_as_longlong(v);
+    const unsigned lo = (unsigned)bits, hi = (unsigned)(bits >> 32);
+    const auto l = Lanes == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false) : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = Lanes == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false) : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    const auto value = [](unsigned a, unsigned b) { return __longlong_as_double((long long)((unsigned long long)b << 32 | a)); };
+    return value(l[0], h[0]) + value(l[1], h[1]);
+}
+
+// Sum over neighbouring `lanes` lanes (a power of two, the same for the whole wavefront), valid in each of them.  Without the LDS
+// crossbar, whose six round trips would be a third of an iteration's work.
+__device__ __forceinline__ double lanes_sum(double v, int lanes)
+{
+    if (lanes > 1) v = dpp_add<0xb1>(v);    // quad_perm 1 0 3 2
+    if (lanes > 2) v = dpp_add<0x4e>(v);    // quad_perm 2 3 0 1
+    if (lanes > 4) v = dpp_add<0x141>(v);   // row_half_mirror: the quads are even by now
+    if (lanes > 8) v = dpp_add<0x140>(v);   // row_mirror
+    if (lanes > 16) v = swap_add<16>(v);
+    if (lanes > 32) v = swap_add<32>(v);
+    return v;
+}
+
+// Rows [0, live) have entries.  The others' rank is the iteration's constant term, so nobody has to be told: every work-group makes
+// their sources for itself.  A set has a slot per live row and is zeros up to S = K * T, of which a lane brings K into LDS.
+template <int K>
+__global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
+    int n, int live, int hubs, int slices, int hub_width, const int32_t *__restrict__ hub_step, const int32_t *__restrict__ hub_col,
+    const int4 *__restrict__ slice, const int32_t *__restrict__ col, const int32_t *__restrict__ order,
+    const double *__restrict__ inv_user, double *inv, unsigned long long *exchange, unsigned *gate, int patience, int iters,
+    double alpha, double inv_n, double *__restrict__ r_out)
+{
+    constexpr int T = kSellResidentThreads, S = K * T, D = kSellWaveSteps, kHubAhead = 4, kRest = 4;
+    extern __shared__ __attribute__((aligned(16))) double s_c[];  // sources [S], of the rows without entries [n - live], 0; those rows' inverse out-degrees [n - live]
+    __shared__ double s_mass[T / kWave], s_hub[T / kWave];
+    __shared__ int s_group, s_groups, s_last, s_dangling;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int rest = n - live;
+    unsigned *left = gate + kTicketStride;
+    double *s_rest = s_c + S + rest + 1;
+    unsigned ticket = 0;
+    if (tid == 0) {
+        ticket = __hip_atomic_fetch_add(gate, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_dangling = 0;
+    }
+    __syncthreads();
+    // The uniform ranks' sources, which every work-group makes for itself, and the inverse out-degrees that go with this lane's slots.
+    int dangling = 0;
+    unsigned dangles = 0;
+    double ivs[K];
+    {
+        int vertex[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) vertex[k] = order[min(tid + k * T, n - 1)];
+#pragma unroll
+        for (int k = 0; k < K; ++k) ivs[k] = inv_user[vertex[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const bool there = tid + k * T < live;
+        s_c[tid + k * T] = ivs[k] * inv_n;
+        dangles |= (there && ivs[k] == 0.0) << k;
+        if (!there) ivs[k] = 0.0;
+    }
+    dangling = __builtin_popcount(dangles);
+    for (int i = tid; i < rest; i += kRest * T) {
+        int vertex[kRest];
+        double iv[kRest];
+#pragma unroll
+        for (int k = 0; k < kRest; ++k) vertex[k] = order[min(live + i + k * T, n - 1)];
+#pragma unroll
+        for (int k = 0; k < kRest; ++k) iv[k] = inv_user[vertex[k]];
+#pragma unroll
+        for (int k = 0; k < kRest; ++k)
+            if (i + k * T < rest) {
+                s_c[S + i + k * T] = iv[k] * inv_n;
+                s_rest[i + k * T] = iv[k];
+                dangling += iv[k] == 0.0;
+            }
+    }
+    if (tid == 0) {
+        s_c[S + rest] = 0.0;  // what the padding gathers
+        int all = gridDim.x;
+        s_group = sell_enter(gate, ticket, all, patience);
+        s_groups = all;
+        s_last = 0;
+    }
+    if (dangling) atomicAdd(&s_dangling, dangling);
+    __syncthreads();
+    const int group = __builtin_amdgcn_readfirstlane(s_group), groups = __builtin_amdgcn_readfirstlane(s_groups);
+    const auto leave = [&] {  // thread 0, when the work-group reads no slots any more
+        s_last = __hip_atomic_fetch_add(left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    };
+    const auto close = [&] {
+        if (!s_last) return;
+        if (iters > 1)
+            for (int i = tid; i < live; i += T) slot_store(exchange + (size_t)((iters - 1) & 3) * S + i, kSellNone);
+        if (tid == 0) {
+            __hip_atomic_store(gate, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(left, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
+    if (group < 0) {
+        if (tid == 0) leave();
+        __syncthreads();
+        close();
+        return;
+    }
+    const int stride = groups * (T / kWave), first = group + groups * wave;
+    const bool more = slices > stride || hubs > groups, hub = group < hubs;
+    const auto place = [&](bool there, int row) { return !there ? S + rest : row < live ? row : row + (S - live); };  // in LDS
+    const auto row_of = [&](const int4 &d) {
+        const int lanes_log = d.w & 7, r = lane >> lanes_log;
+        return (lane & ((1 << lanes_log) - 1)) == 0 && r < (d.w >> 3) && d.z + r < live ? d.z + r : -1;
+    };
+    // The first slice of the wavefront and the first hub of the work-group stay in registers.
+    const int4 d0 = first < slices ? slice[first] : make_int4(0, 0, 0, 0);
+    int id[D], hub_id[kHubAhead];
+#pragma unroll
+    for (int k = 0; k < D; ++k) id[k] = col[((size_t)d0.x + k) * kWave + lane];  // (the array goes on for D steps)
+#pragma unroll
+    for (int k = 0; k < D; ++k) id[k] = place(k < d0.y, id[k]);
+    const int row0 = row_of(d0);
+    const double iv0 = row0 >= 0 ? inv_user[order[row0]] : 1.0;
+    // Steps of a hub taken at once, this lane's share of them.
+    const int hub_lanes = T / hub_width, hub_sub = __builtin_amdgcn_readfirstlane(tid / hub_width), hub_lane = tid % hub_width;
+    const auto hub_fetch = [&](int from, int to, int (&ids)[kHubAhead]) {
+#pragma unroll
+        for (int k = 0; k < kHubAhead; ++k) ids[k] = hub_col[(size_t)min(from + hub_sub + k * hub_lanes, to - 1) * hub_width + hub_lane];
+#pragma unroll
+        for (int k = 0; k < kHubAhead; ++k) ids[k] = place(from + hub_sub + k * hub_lanes < to, ids[k]);
+    };
+    int hub_from = 0, hub_to = 0;
+    double hub_iv = 0.0;
+    if (hub) {
+        hub_from = hub_step[group];
+        hub_to = hub_step[group + 1];
+        hub_iv = inv_user[order[group]];
+        hub_fetch(hub_from, hub_to, hub_id);
+    }
+    const double dangling_rows = s_dangling;
+    for (int s = first + stride; s < slices; s += stride) {
+        const int row = row_of(slice[s]);
+        if (row >= 0) inv[row] = inv_user[order[row]];  // read again by this lane only
+    }
+    // A rank is base + alpha * sum, and base is the same everywhere: a slot holds alpha * sum, times the
+    // inverse out-degree where that is not 0, and base, which takes a reduction, is added by the readers and not waited for.
+    bool given_up = false;
+    double base = inv_n, mass = 0.0;  // of the ranks that the iteration starts from: base, and the dangling mass beyond base
+    for (int it = 0; it < iters; ++it) {
+        unsigned long long *out = exchange + (size_t)((it + 1) & 3) * S, *done = exchange + (size_t)((it + 3) & 3) * S;
+        const bool last = it == iters - 1;
+        if (it > 0) {
+            const unsigned long long *in = exchange + (size_t)(it & 3) * S + tid;
+            unsigned long long v[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) v[k] = slot_load(in + k * T);
+            for (int i = tid; i < rest; i += T) s_c[S + i] = base * s_rest[i];
+            for (int polls = 0; !given_up; ++polls) {
+                bool missing = false;
+#pragma unroll
+                for (int k = 0; k < K; ++k) missing |= slot_is_none(v[k]);
+                if (!missing) break;
+                given_up = polls >= kSellPolls;
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (slot_is_none(v[k])) v[k] = slot_load(in + k * T);
+            }
+            mass = 0.0;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                double x = __longlong_as_double((long long)v[k]);
+                if (dangles >> k & 1) {
+                    mass += x;
+                    x *= 0.0;
+                }
+                s_c[tid + k * T] = x + base * ivs[k];
+            }
+            __builtin_amdgcn_s_waitcnt(kSellWaitStores);  // for the clearing stores of the iteration before
+        }
+        __syncthreads();
+        if (last && tid == 0) leave();
+        double sum = 0.0, part = 0.0;
+        const auto gather = [&](auto steps) {
+            double v[decltype(steps)::value];
+#pragma unroll
+            for (int k = 0; k < decltype(steps)::value; ++k) v[k] = s_c[id[k]];
+#pragma unroll
+            for (int k = 0; k < decltype(steps)::value; ++k) sum += v[k];
+        };
+        const auto hub_sum = [&](int from, int to, const int (&ahead)[kHubAhead]) {
+            int ids[kHubAhead];
+            double total = 0.0;
+#pragma unroll
+            for (int k = 0; k < kHubAhead; ++k) ids[k] = ahead[k];
+            for (;;) {
+#pragma unroll
+                for (int k = 0; k < kHubAhead; ++k)
+                    total += s_c[ids[k]];
+                from += kHubAhead * hub_lanes;
+                if (from >= to) return total;
+                hub_fetch(from, to, ids);
+            }
+        };
+        // A row's slots: filled for the next iteration, cleared of the one before.
+        const auto hand_on = [&](int row, double iv, double total) {
+            if (!last) {
+                const unsigned long long bits = (unsigned long long)__double_as_longlong(iv == 0.0 ? alpha * total : alpha * total * iv);
+                slot_store(out + row, slot_is_none(bits) ? kSellNan : bits);
+            }
+            if (it > 0) slot_store(done + row, kSellNone);
+        };
+        if (hub) {
+            part = lanes_sum(hub_sum(hub_from, hub_to, hub_id), kWave);
+            if (lane == 0) s_hub[wave] = part;
+        }
+        if (d0.y > 8) gather(std::integral_constant<int, D>());
+        else if (d0.y > 4) gather(std::integral_constant<int, 8>());
+        else if (d0.y > 0) gather(std::integral_constant<int, 4>());
+        if (first < slices) {
+            sum = lanes_sum(sum, 1 << (d0.w & 7));
+            if (row0 >= 0) hand_on(row0, iv0, sum);
+        }
+        if (hub) {
+            __syncthreads();
+            if (wave == 0) {
+                part = lanes_sum(s_hub[lane & (T / kWave - 1)], T / kWave);
+                if (lane == 0) hand_on(group, hub_iv, part);
+            }
+        }
+        // The constant term of this iteration's ranks.  Behind the barrier the sources in LDS may be replaced.
+        mass = lanes_sum(mass, kWave);
+        if (lane == 0) s_mass[wave] = mass;
+        __syncthreads();
+        const double dang = dangling_rows * base + lanes_sum(s_mass[lane & (T / kWave - 1)], T / kWave);
+        base = (1.0 - alpha) * inv_n + alpha * dang * inv_n;
+        const auto store = [&](int row, double total) {
+            if (last) r_out[order[row]] = base + alpha * total;
+        };
+        if (row0 >= 0) store(row0, sum);
+        if (hub && tid == 0) store(group, part);
+        if (more) {
+            for (int h = group + groups; h < hubs; h += groups) {
+                int ids[kHubAhead];
+                hub_fetch(hub_step[h], hub_step[h + 1], ids);
+                const double total = block_sum<T>(hub_sum(hub_step[h], hub_step[h + 1], ids), s_hub);
+                if (tid == 0) {
+                    hand_on(h, inv_user[order[h]], total);
+                    store(h, total);
+                }
+                __syncthreads();  // s_hub is used again
+            }
+            for (int s = first + stride; s < slices; s += stride) {
+                const int4 d = slice[s];
+                const int row = row_of(d);
+                const double iv = row >= 0 ? inv[row] : 1.0;
+                double total = 0.0;
+                for (int step = 0; step < d.y; step += kSellDepth) {
+                    int ids[kSellDepth];
+#pragma unroll
+                    for (int k = 0; k < kSellDepth; ++k) ids[k] = step + k < d.y ? place(true, col[((size_t)d.x + step + k) * kWave + lane]) : S + rest;
+#pragma unroll
+                    for (int k = 0; k < kSellDepth; ++k) total += s_c[ids[k]];
+                }
+                total = lanes_sum(total, 1 << (d.w & 7));
+                if (row >= 0) {
+                    hand_on(row, iv, total);
+                    store(row, total);
+                }
+            }
+            __syncthreads();  // the sources in LDS and s_hub are replaced next
+        }
+    }
+    for (int i = live + group * T + tid; i < n; i += groups * T) r_out[order[i]] = base;
+    __syncthreads();
+    close();
 }
 
 // v[k] = source of id[k], the padding's 0.  Both kinds of load are under the lanes' own condition: a hot lane costs the L1 nothing.
@@ -351,14 +705,14 @@ __global__ void sell_lengths_kernel(int n, const Off *__restrict__ row_ptr, unsi
     }
 }
 
-// new_id of every vertex; bounds[k] = rows (longest first) with more entries than class k takes
+// new_id of every vertex; bounds[k] = rows (longest first) with more entries than class k takes, bounds[kSellClasses + 1] = rows with any
 __global__ void sell_bounds_kernel(int n, const unsigned *__restrict__ len_sorted, const int32_t *__restrict__ order,
                                    bool f32, int hub_limit, int32_t *__restrict__ new_id, int *__restrict__ bounds)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) new_id[order[i]] = i;
     if (blockIdx.x != 0) return;
-    if (threadIdx.x < kSellClasses) {
-        const unsigned limit = (unsigned)sell_class_limit(threadIdx.x, f32, hub_limit);
+    if (threadIdx.x < kSellClasses || threadIdx.x == kSellClasses + 1) {
+        const unsigned limit = threadIdx.x < kSellClasses ? (unsigned)sell_class_limit(threadIdx.x, f32, hub_limit) : 0;
         int lo = 0, hi = n;  // first row with at most `limit` entries
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -442,6 +796,37 @@ __global__ __launch_bounds__(256) void sell_fill_kernel(SellShape sh, int thread
         out[(size_t)st * kWave + lane] = source(e0 < e1, e0);
 }
 
+using SellResident = decltype(&sell_resident_kernel<1>);
+
+SellResident sell_resident_of(const SellRows &sr)
+{
+    switch (sr.staged) {
+    case 1: return &sell_resident_kernel<1>;
+    case 2: return &sell_resident_kernel<2>;
+    case 3: return &sell_resident_kernel<3>;
+    case 4: return &sell_resident_kernel<4>;
+    case 5: return &sell_resident_kernel<5>;
+    case 6: return &sell_resident_kernel<6>;
+    case 8: return &sell_resident_kernel<8>;
+    case 10: return &sell_resident_kernel<10>;
+    default: return &sell_resident_kernel<kSellStaged>;
+    }
+}
+
+// Whether runs are one launch, and of how many work-groups.
+void choose_resident(SellRows *sr, int live)
+{
+    sr->live = live;
+    sr->live_slices = sr->slice_begin[kSellClasses - 1] + (int)ceil_div(live - sr->row_begin[kSellClasses - 1], kWave);
+    sr->staged = 0;
+    for (const int staged : {kSellStaged, 10, 8, 6, 5, 4, 3, 2, 1})
+        if (staged * kSellResidentThreads >= live) sr->staged = staged;
+    sr->lds = sizeof(double) * ((size_t)sr->staged * kSellResidentThreads + 2 * (size_t)(sr->n - live) + 1);
+    if (!sr->staged || sr->lds > kSellResidentLds || sr->hubs > kSellResidentBlocks || sr->live_slices > kSellResidentBlocks * (kSellResidentThreads / kWave)) return;
+    const int wanted = std::max((int)ceil_div(sr->live_slices, kSellResidentSlices), sr->hubs);
+    sr->resident = std::max(1, std::min({wanted, kSellResidentBlocks, sr->live_slices}));  // each of several owns a row
+}
+
 SellShape shape_of(const SellRows &sr)
 {
     SellShape sh;
@@ -467,7 +852,7 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
     sr->n = n;
     sr->nnz = nnz;
     sr->threads = n + nnz > kSellWideItems ? 512 : 256;
-    constexpr int kWords = kSellClasses + 1;
+    constexpr int kWords = kSellClasses + 2;
     const int hub_limit = kWave * (f32_id ? kSellWaveStepsF32 : n + nnz > kSellWideItems ? kSellWaveStepsWide : kSellWaveSteps);
     unsigned *len = nullptr, *len_sorted = nullptr;
     int32_t *ids = nullptr, *new_id = f32_id, *hub_steps = nullptr, *slice_steps = nullptr, *slice_step = nullptr;
@@ -539,6 +924,7 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         DRONE_REQUIRE((size_t)sr->slices <= most_slices && (size_t)sr->hubs <= most_hubs, "slice bound");
         sr->blocks = sr->hot ? kSellHotBlocks : sr->hubs + (int)ceil_div(sr->slices, sr->threads / kWave);
         sr->init_blocks = (int)std::min<int64_t>(ceil_div(n, kSellInitThreads), kSellInitBlocks);
+        if (!f32_id && !sr->hot) choose_resident(sr, h[kSellClasses + 1]);
         const SellShape sh = shape_of(*sr);
         sell_steps_kernel<<<(int)ceil_div(std::max(sr->slices, sr->hubs) + 1, 256), 256, 0, s>>>(sh, sr->threads, len_sorted, hub_steps, slice_steps);
         need = temp_bytes;
@@ -549,8 +935,17 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         DRONE_HIP_TRY(hipMemcpyAsync(h + 1, slice_step + sr->slices, sizeof(int), hipMemcpyDeviceToHost, s));
         DRONE_HIP_TRY(hipStreamSynchronize(s));
         sr->entries.want(&sr->hub_col, (size_t)h[0] * sr->threads);
-        sr->entries.want(&sr->col, (size_t)h[1] * kWave);
+        sr->entries.want(&sr->col, ((size_t)h[1] + kSellWaveSteps) * kWave);  // sell_resident_kernel reads so far beyond its slice
+        const int slots = sr->staged * kSellResidentThreads;
+        if (sr->resident) {
+            sr->entries.want(&sr->exchange, 4 * (size_t)slots);
+            sr->entries.want(&sr->gate, 2 * kTicketStride);
+        }
         DRONE_HIP_TRY(sr->entries.commit());
+        if (sr->resident) {
+            sell_slots_kernel<<<64, 256, 0, s>>>(slots, sr->live, sr->exchange, sr->gate);
+            DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sell_resident_of(*sr)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sr->lds));
+        }
         sell_fill_kernel<<<sr->hubs + (int)ceil_div(sr->slices, 256 / kWave), 256, 0, s>>>(
             sh, sr->threads, sr->order, row_ptr, col, new_id, sr->hub_step, slice_step, sr->slice, sr->hub_col, sr->col, sr->hot);
         DRONE_HIP_TRY(hipGetLastError());
@@ -589,6 +984,15 @@ int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t s)
 {
     sell_begin_kernel<<<sr.init_blocks, kSellInitThreads, 0, s>>>((int)sr.n, sr.order, inv_user, 1.0 / (double)sr.n, sr.inv,
                                                                  sr.c[0], sr.c[1], sr.part[0]);
+    DRONE_HIP_TRY(hipGetLastError());
+    return DRONE_OK;
+}
+
+int sell_run(const SellRows &sr, const double *inv_user, int iters, double alpha, double *rank_out, hipStream_t s)
+{
+    sell_resident_of(sr)<<<sr.resident, kSellResidentThreads, sr.lds, s>>>(
+        (int)sr.n, sr.live, sr.hubs, sr.live_slices, sr.threads, sr.hub_step, sr.hub_col, sr.slice, sr.col, sr.order, inv_user, sr.inv,
+        sr.exchange, sr.gate, sr.patience, iters, alpha, 1.0 / (double)sr.n, rank_out);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }

@@ -173,7 +173,8 @@ int drone_pr_plan_create_ex(drone_pr_plan **plan, int64_t n, int64_t nnz, const 
 int drone_pr_plan_destroy(drone_pr_plan *plan);
 /* Runs `iters` iterations from r_0 = 1/N and writes r_iters to rank_out [n] (device).
  * Asynchronous on `stream`; allocates nothing and launches kernels only (no copies, clears or waits), so a run can be
- * recorded into a HIP graph and replayed while profiling (drone_pr_profile_enable) is off. */
+ * recorded into a HIP graph and replayed while profiling (drone_pr_profile_enable) is off.  A plan is for one run at
+ * a time. */
 int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_out,
                      drone_stream_t stream);
 /* Per-iteration timing with HIP events on the launch stream.  When enabled, every iteration inside
@@ -183,6 +184,10 @@ int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_
 int drone_pr_profile_enable(drone_pr_plan *plan, int max_launches);
 int drone_pr_profile_read(drone_pr_plan *plan, int *launches, double *mean_ms, double *min_ms,
                           double *max_ms);
+/* Runs of a small matrix are one launch whose work-groups wait for each other.  `looks`: how often each looks whether all
+ * have found a place on the chip, before one of them does the run alone (64 by default; the results are the same to
+ * rounding). */
+int drone_pr_plan_patience(drone_pr_plan *plan, int looks);
 /* Algorithmic bytes of one iteration: 4*nnz + 32*n + 8. */
 int64_t drone_pr_bytes_per_iteration(int64_t n, int64_t nnz);
 

@@ -1,0 +1,123 @@
+"""Runs of small fp64 PageRank plans, whose work-groups stay for the whole run: at the edges of what a lane stages, with more slices
+and hub rows than work-groups, recorded into a graph, and by the one work-group that does the run alone behind a closed gate."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(n, lengths, filler):
+    """Row lengths `lengths` at random places among rows of `filler` entries; the last fifth of the vertices dangles."""
+    rng = np.random.default_rng(n + filler)
+    length = np.full(n, filler, np.int64)
+    length[rng.choice(n, len(lengths), replace=False)] = lengths
+    rp = np.zeros(n + 1, np.int64)
+    rp[1:] = np.cumsum(length)
+    ci = rng.integers(0, max(1, n - n // 5), rp[-1]).astype(np.int32)
+    outdeg = np.bincount(ci, minlength=n)
+    return rp, ci, np.where(outdeg > 0, 1.0 / np.maximum(outdeg, 1), 0.0)
+
+
+def _plan(rp, ci, inv):
+    import torch
+    from drone_amd.pagerank import PullPlanF64
+    return PullPlanF64(torch.from_numpy(rp).cuda(), torch.from_numpy(ci).cuda(), torch.from_numpy(inv).cuda())
+
+
+def _close(got, ref, rp, iters):
+    # positive terms: a sum of L of them is within L * 2^-53 of exact in any order, twice that between two orders
+    n = len(ref)
+    assert np.max(np.abs(got - ref) / ref) <= 2 * iters * max(np.diff(rp).max(), n) * 2.0 ** -53
+
+
+@pytest.mark.parametrize("n,lengths,filler", [
+    (1, [], 0), (1, [], 3), (2, [1], 0), (65, [64, 768, 769], 2),
+    (1023, [2048, 2049, 1, 0], 5), (1024, [], 0), (1025, [12, 13, 96], 9),
+    (4096, [800] * 64, 3), (4097, [800] * 65, 11),           # as many hub rows as work-groups, and one more
+    (6000, [30_000, 5000, 4096, 4097], 1),                   # hub rows of several rounds
+    (8192, [], 60), (8200, [], 60),                          # as many slices as wavefronts, and one more
+    (12288, [768] * 5, 11), (12289, [768] * 5, 11),          # as many rows as fit
+    (19455, [9] * 1024, 0), (14000, [12] * 6000, 0),         # most rows without entries: too many of them to fit, and not
+])
+def test_runs_in_one_launch(oracle, n, lengths, filler):
+    rp, ci, inv = _matrix(n, lengths, filler)
+    plan = _plan(rp, ci, inv)
+    for iters in (1, 2, 3, 4, 5, 9):
+        got = plan.run(0.85, iters).cpu().numpy()
+        _close(got, oracle.pr_pull_f64(rp, ci, inv, 0.85, iters), rp, iters)
+        assert np.array_equal(got, plan.run(0.85, iters).cpu().numpy())
+    plan.close()
+
+
+@pytest.mark.parametrize("n,lengths,filler", [(700, [900, 2100], 4), (6000, [800] * 64, 12)])
+def test_one_work_group_alone(oracle, n, lengths, filler):
+    from drone_amd._lib import check, lib
+    rp, ci, inv = _matrix(n, lengths, filler)
+    plan = _plan(rp, ci, inv)
+    for iters in (1, 2, 5, 6):
+        for looks in (0, 64):  # runs behind a closed gate and open ones follow each other
+            check(lib().drone_pr_plan_patience(plan.h, looks))
+            _close(plan.run(0.85, iters).cpu().numpy(), oracle.pr_pull_f64(rp, ci, inv, 0.85, iters), rp, iters)
+    plan.close()
+
+
+def test_infinite_degrees_stay_in_the_ranks():
+    """A NaN and an infinity among the inverse out-degrees reach the ranks that they reach in a launch per iteration."""
+    rp, ci, inv = _matrix(500, [], 2)
+    inv[3], inv[4] = np.nan, np.inf
+    plan = _plan(rp, ci, inv)
+    for iters in (1, 3):
+        got = plan.run(0.85, iters).cpu().numpy()
+        plan.profile_enable(16)
+        want = plan.run(0.85, iters).cpu().numpy()
+        plan.profile_enable(0)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        there = np.isfinite(want)
+        assert (iters > 1 or there.any()) and np.allclose(got[there], want[there], rtol=1e-13, atol=0)
+    plan.close()
+
+
+def test_replays_of_a_recorded_run():
+    import torch
+    from drone_amd.pagerank import PullPlanF64
+    rp, ci, inv = (torch.from_numpy(a).cuda() for a in _matrix(5000, [900, 1500], 9))
+    side = torch.cuda.Stream()
+    plan = PullPlanF64(rp, ci, inv)
+    eager = plan.run(0.85, 7)
+    torch.cuda.synchronize()
+    plan.stream = side.cuda_stream
+    out, graph = torch.zeros_like(eager), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        plan.run(0.85, 7, out=out)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            plan.run(0.85, 7, out=out)
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    plan.close()
+
+
+def test_runs_beside_each_other():
+    """Four plans on four streams, whose work-groups ask for places at the same time."""
+    import torch
+    from drone_amd.pagerank import PullPlanF64
+    mats = [[torch.from_numpy(a).cuda() for a in _matrix(n, [900], 9)] for n in (3000, 5000, 7000, 9000)]
+    plans = [PullPlanF64(*m) for m in mats]
+    want = [p.run(0.85, 20) for p in plans]
+    torch.cuda.synchronize()
+    outs = [torch.zeros_like(w) for w in want]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in plans]
+    for p, s in zip(plans, streams):
+        p.stream = s.cuda_stream
+    for _ in range(50):
+        for p, o in zip(plans, outs):
+            p.run(0.85, 20, out=o)
+    torch.cuda.synchronize()
+    for p, o, w in zip(plans, outs, want):
+        assert float(((o - w).abs() / w).max()) <= 1e-12  # one run may be a work-group's alone, in another order
+        p.close()
