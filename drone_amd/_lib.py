@@ -135,6 +135,10 @@ SIGNATURES = {
     "drone_loss_pass_f32": (_I, [_P, _P]),
     "drone_loss_pass_split_f32": (_I, [_P, _P, _P, _I, _P, _P]),
     "drone_sgd_steps_f32": (_I, [_P, _I, _F, _P]),
+    "drone_sgd_steps_sums_f32": (_I, [_P, _P, _I, _F, _P]),
+    "drone_adam_steps_sums_f32": (_I, [_P, _P, _I, _F, _F, _F, _F, _F, _I, _P]),
+    "drone_sgemm_tn_sums_floats": (C.c_int64, [_I, _I, _I, _I, _I]),
+    "drone_sgemm_tn_sums_f32": (_I, [_I, _I, _I, _P, _I, _P, _I, _P, _I, _P, C.c_int64, C.POINTER(_I), _P]),
     "drone_adam_steps_f32": (_I, [_P, _I, _F, _F, _F, _F, _F, _I, _P]),
     "drone_fill_f32": (_I, [_P, _I64, _F, _P]),
     "drone_gcn_create": (_I, [C.POINTER(_P), C.POINTER(GcnConfig), _I64, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P]),

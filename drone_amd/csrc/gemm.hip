@@ -784,10 +784,22 @@ void launch_reduce(int M, int N, int splits, const float *partial, float alpha, 
     sgemm_reduce_kernel<<<blocks, kReduceOutputs * kReduceGroups, 0, s>>>(M, N, splits, partial, alpha, beta, C, ldc);
 }
 
-// Scratch for `floats` partial sums: the stream's grow-only buffer, or the fixed array of the entry point that may not
+// Where a caller that adds the sums of a split reduction up by itself wants them.  splits: 0 until they are left there.
+struct KeptSums {
+    float *sums;
+    int64_t floats;
+    int splits = 0;
+};
+
+// Scratch for `floats` partial sums: the caller's, the stream's grow-only buffer, or the fixed array of the entry point that may not
 // allocate.
-int split_scratch(bool may_allocate, size_t floats, hipStream_t s, int M, int N, int K, int splits, float **partial)
+int split_scratch(bool may_allocate, KeptSums *kept, size_t floats, hipStream_t s, int M, int N, int K, int splits, float **partial)
 {
+    if (kept && kept->sums && (int64_t)floats <= kept->floats) {
+        kept->splits = splits;
+        *partial = kept->sums;
+        return DRONE_OK;
+    }
     if (may_allocate) return workspace(sizeof(float) * floats, s, partial);
     if (floats > kStaticScratchFloats) {
         set_error(DRONE_ERR_INVALID,
@@ -801,11 +813,14 @@ int split_scratch(bool may_allocate, size_t floats, hipStream_t s, int M, int N,
 
 // C = alpha * A^T * B + beta * C for a small output and a long reduction (see sgemm_tn_skinny_kernel and
 // sgemm_tn_small_kernel, which takes the outputs whose rows of B can be read in whole pieces).
-int sgemm_tn_skinny(bool may_allocate, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-                    float beta, float *C, int ldc, hipStream_t s)
+bool skinny_is_small(int N, int ldb)
 {
     const int nt = (N + 15) / 16;
-    const bool small = ldb >= (N + nt - 1) / nt * nt;  // a lane reads nt consecutive floats of B's row, also past N
+    return ldb >= (N + nt - 1) / nt * nt;  // a lane reads nt consecutive floats of B's row, also past N
+}
+int skinny_splits(int N, int K, int ldb, int *k_chunk)
+{
+    const bool small = skinny_is_small(N, ldb);
     // two work-groups of four wavefronts per CU, each wavefront at least 16 steps of the reduction deep
     const int rows_per_step = small ? 4 * kSmallWaves * kSmallDepth : 2 * kSkinnyWaves * kSkinnyDepth;
     const int align = small ? 4 * kSmallWaves : 2 * kSkinnyWaves;
@@ -813,17 +828,24 @@ int sgemm_tn_skinny(bool may_allocate, int M, int N, int K, float alpha, const f
     const int deepest = (int)ceil_div(K, rows_per_step * 16);
     if (splits > deepest) splits = deepest;
     if (splits < 1) splits = 1;
-    int k_chunk = (int)ceil_div(ceil_div(K, splits), align) * align;
-    splits = (int)ceil_div(K, k_chunk);
+    *k_chunk = (int)ceil_div(ceil_div(K, splits), align) * align;
+    return (int)ceil_div(K, *k_chunk);
+}
+int sgemm_tn_skinny(bool may_allocate, KeptSums *kept, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+                    float beta, float *C, int ldc, hipStream_t s)
+{
+    int k_chunk = 0;
+    const int nt = (N + 15) / 16, splits = skinny_splits(N, K, ldb, &k_chunk);
+    const bool small = skinny_is_small(N, ldb);
     float *partial = nullptr;
-    const int rc = split_scratch(may_allocate, (size_t)splits * M * N, s, M, N, K, splits, &partial);
+    const int rc = split_scratch(may_allocate, kept, (size_t)splits * M * N, s, M, N, K, splits, &partial);
     if (rc != DRONE_OK) return rc;
     if (!small) sgemm_tn_skinny_kernel<<<splits, kSkinnyWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
     else if (nt == 1) sgemm_tn_small_kernel<1><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
     else if (nt == 2) sgemm_tn_small_kernel<2><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
     else if (nt == 3) sgemm_tn_small_kernel<3><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
     else sgemm_tn_small_kernel<4><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
+    if (!(kept && kept->splits > 0)) launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
@@ -966,14 +988,20 @@ void launch_direct(const DirectShape &d, int M, int N, int K, float alpha, const
     sgemm_direct_kernel<MT, NT, AK, BK, KS><<<grid, kWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
 }
 
-int sgemm_direct(DirectShape d, bool may_allocate, bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
+int direct_splits(const DirectShape &d, int K, int *k_chunk)
+{
+    *k_chunk = (int)ceil_div(ceil_div(K, d.splits), 16) * 16;
+    return (int)ceil_div(K, *k_chunk);
+}
+
+int sgemm_direct(DirectShape d, bool may_allocate, KeptSums *kept, bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
                  int lda, const float *B, int ldb, float beta, float *C, int ldc, hipStream_t s)
 {
-    const int k_chunk = (int)ceil_div(ceil_div(K, d.splits), 16) * 16;
-    d.splits = (int)ceil_div(K, k_chunk);
+    int k_chunk = 0;
+    d.splits = direct_splits(d, K, &k_chunk);
     float *partial = nullptr;
     if (d.splits > 1) {
-        const int rc = split_scratch(may_allocate, (size_t)d.splits * M * N, s, M, N, K, d.splits, &partial);
+        const int rc = split_scratch(may_allocate, kept, (size_t)d.splits * M * N, s, M, N, K, d.splits, &partial);
         if (rc != DRONE_OK) return rc;
     }
     bool done = false;
@@ -1014,12 +1042,27 @@ int sgemm_direct(DirectShape d, bool may_allocate, bool ta, bool tb, int M, int 
 #undef DRONE_DIRECT_ROWS
 #undef DRONE_DIRECT
     DRONE_REQUIRE(done, "no instance of the direct kernel for this shape");
-    if (d.splits > 1) launch_reduce(M, N, d.splits, partial, alpha, beta, C, ldc, s);
+    if (d.splits > 1 && !(kept && kept->splits > 0)) launch_reduce(M, N, d.splits, partial, alpha, beta, C, ldc, s);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
 
-int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,
+// (the skinny kernel's lanes read four floats of A's row and two of B's at once, also the lanes past M and N.  128 x 41
+// outputs: 24.6 us (17.9 by sgemm_direct_kernel) over 30,000 rows, 24.0 (24.5) over 50,000, 31 (39) over 100,000; outputs
+// of 32 rows and fewer are better off with the direct kernel at any length, 43 x 22 and 43 x 41 are not)
+bool skinny_covers(int transA, int transB, int M, int N, int K, int lda, int ldb)
+{
+    return transA && !transB && M > 32 && M <= 128 && N <= 64 && K >= 40000 && lda >= (M + 3) / 4 * 4 && ldb >= (N + 1) / 2 * 2;
+}
+
+int tiled_chunk(int tiles, int K, int *k_chunk)
+{
+    *k_chunk = (int)ceil_div(ceil_div(K > 0 ? K : 1, tiled_splits(tiles, K)), BK) * BK;
+    return (int)ceil_div(K > 0 ? K : 1, *k_chunk);
+}
+int tiles_of(int M, int N) { return (int)(ceil_div(M, kTileRows) * ceil_div(N, N <= 64 ? 64 : 128)); }
+
+int sgemm_entry(bool may_allocate, KeptSums *kept, int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,
                 const float *B, int ldb, float beta, float *C, int ldc, drone_stream_t stream)
 {
     clear_error();
@@ -1034,26 +1077,22 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
         DRONE_HIP_TRY(hipGetLastError());
         return DRONE_OK;
     }
-    // (the skinny kernel's lanes read four floats of A's row and two of B's at once, also the lanes past M and N.  128 x 41
-    // outputs: 24.6 us (17.9 by sgemm_direct_kernel) over 30,000 rows, 24.0 (24.5) over 50,000, 31 (39) over 100,000; outputs
-    // of 32 rows and fewer are better off with the direct kernel at any length, 43 x 22 and 43 x 41 are not)
-    if (transA && !transB && M > 32 && M <= 128 && N <= 64 && K >= 40000 && lda >= (M + 3) / 4 * 4 && ldb >= (N + 1) / 2 * 2)
-        return sgemm_tn_skinny(may_allocate, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+    if (skinny_covers(transA, transB, M, N, K, lda, ldb))
+        return sgemm_tn_skinny(may_allocate, kept, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
     const DirectShape direct = direct_shape(transA != 0, transB != 0, M, N, K);
     if (direct.ks > 0)
-        return sgemm_direct(direct, may_allocate, transA != 0, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+        return sgemm_direct(direct, may_allocate, kept, transA != 0, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
     const bool narrow = N <= 64;
     const int bn = narrow ? 64 : 128;
-    const int tiles = (int)(ceil_div(M, kTileRows) * ceil_div(N, bn));
+    const int tiles = tiles_of(M, N);
     const int bm = !narrow && half_rows(transA != 0, tiles) ? kTileRows / 2 : kTileRows;
-    int splits = tiled_splits(tiles, K);
-    int k_chunk = (int)ceil_div(ceil_div(K > 0 ? K : 1, splits), BK) * BK;
-    splits = (int)ceil_div(K > 0 ? K : 1, k_chunk);
+    int k_chunk = 0;
+    const int splits = tiled_chunk(tiles, K, &k_chunk);
     float *partial = nullptr;
     if (splits > 1) {
         // every (tile, split) work-group stores its whole tile, so the partials need no clearing
         const size_t floats = (size_t)splits * M * N;
-        const int rc = split_scratch(may_allocate, floats, s, M, N, K, splits, &partial);
+        const int rc = split_scratch(may_allocate, kept, floats, s, M, N, K, splits, &partial);
         if (rc != DRONE_OK) return rc;
     }
     dim3 grid((unsigned)ceil_div(N, bn), (unsigned)ceil_div(M, bm), (unsigned)splits);
@@ -1061,7 +1100,7 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
     if (narrow) launch<kTileRows, 64>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
     else if (bm < kTileRows) launch<kTileRows / 2, 128>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
     else launch<kTileRows, 128>(transA != 0, transB != 0, grid, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    if (splits > 1) launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
+    if (splits > 1 && !(kept && kept->splits > 0)) launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
@@ -1070,14 +1109,34 @@ int sgemm_entry(bool may_allocate, int transA, int transB, int M, int N, int K, 
 extern "C" int drone_sgemm_rm_f32(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,
                                   const float *B, int ldb, float beta, float *C, int ldc, drone_stream_t stream)
 {
-    return sgemm_entry(true, transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, stream);
+    return sgemm_entry(true, nullptr, transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, stream);
 }
 
 extern "C" int drone_sgemm_rm_f32_noalloc(int transA, int transB, int M, int N, int K, float alpha, const float *A,
                                           int lda, const float *B, int ldb, float beta, float *C, int ldc,
                                           drone_stream_t stream)
 {
-    return sgemm_entry(false, transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, stream);
+    return sgemm_entry(false, nullptr, transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, stream);
+}
+
+extern "C" int64_t drone_sgemm_tn_sums_floats(int M, int N, int K, int lda, int ldb)
+{
+    if (M < 1 || N < 1 || K < 1) return 0;
+    int k_chunk = 0, splits;
+    const DirectShape direct = direct_shape(true, false, M, N, K);
+    if (skinny_covers(1, 0, M, N, K, lda, ldb)) splits = skinny_splits(N, K, ldb, &k_chunk);
+    else if (direct.ks > 0) splits = direct_splits(direct, K, &k_chunk);
+    else splits = tiled_chunk(tiles_of(M, N), K, &k_chunk);
+    return splits > 1 ? (int64_t)splits * M * N : 0;
+}
+
+extern "C" int drone_sgemm_tn_sums_f32(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc,
+                                       float *sums, int64_t floats, int *splits, drone_stream_t stream)
+{
+    KeptSums kept{sums, floats};
+    const int rc = sgemm_entry(true, &kept, 1, 0, M, N, K, 1.0f, A, lda, B, ldb, 0.0f, C, ldc, stream);
+    if (splits) *splits = rc == DRONE_OK ? kept.splits : 0;
+    return rc;
 }
 
 // Also resolves (and caches) the current device's address of the array, so that a caller who asks for the size before

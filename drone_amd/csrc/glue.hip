@@ -486,30 +486,66 @@ __global__ __launch_bounds__(1024) void sum_squares_kernel(const float *__restri
 constexpr int kStepTensors = 4;
 struct StepTensors {
     drone_step_tensor t[kStepTensors];
+    drone_step_sums sums[kStepTensors];
 };
-__global__ void sgd_kernel(StepTensors tensors, float lr)
-{
-    const drone_step_tensor t = tensors.t[blockIdx.y];
-    float *__restrict__ w = t.w;
-    const float *__restrict__ g = t.grad;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < t.n; i += (int64_t)gridDim.x * blockDim.x)
-        w[i] -= lr * g[i];
-}
+struct SgdStep {
+    float lr;
+    __device__ __forceinline__ void operator()(const drone_step_tensor &t, int64_t i, float g) const { t.w[i] -= lr * g; }
+};
 
 // cuda_kernel.cu:450-460
-__global__ void adam_kernel(StepTensors tensors, float weight_decay, float beta1, float beta2, float eps, float step_size)
+struct AdamStep {
+    float weight_decay, beta1, beta2, eps, step_size;
+    __device__ __forceinline__ void operator()(const drone_step_tensor &t, int64_t i, float g) const
+    {
+        const float w = t.w[i];
+        if (t.decay) g += weight_decay * w;
+        const float mi = (float)(beta1 * t.m[i] + (1.0 - beta1) * g);
+        const float vi = (float)(beta2 * t.v[i] + (1.0 - beta2) * g * g);
+        t.m[i] = mi;
+        t.v[i] = vi;
+        t.w[i] = w - step_size * mi / (sqrtf(vi) + eps);
+    }
+};
+
+// A tensor's gradient is there, or still the partial sums of a split reduction, which are then added up as sgemm_reduce_kernel does
+// it: 32 outputs to 256 lanes, eight sums of an output in flight, a fixed order.  Bound by launches: a reduction of its own for each of two
+// weights, and the step, were 3.4 to 4.7 us each (epoch on 2,708 vertices 135 -> 127 us, 30,011-vertex step, whose layer 1 keeps its reduction, 226 -> 224).
+template <typename Step>
+__global__ __launch_bounds__(kThreads) void step_kernel(StepTensors tensors, Step step)
 {
+    constexpr int G = 8, O = kThreads / G;
+    __shared__ float s_sum[G][O];
     const drone_step_tensor t = tensors.t[blockIdx.y];
-    float *__restrict__ w = t.w, *__restrict__ m = t.m, *__restrict__ v = t.v;
-    const float *__restrict__ grad = t.grad;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < t.n; i += (int64_t)gridDim.x * blockDim.x) {
-        float g = grad[i];
-        if (t.decay) g += weight_decay * w[i];
-        const float mi = (float)(beta1 * m[i] + (1.0 - beta1) * g);
-        const float vi = (float)(beta2 * v[i] + (1.0 - beta2) * g * g);
-        m[i] = mi;
-        v[i] = vi;
-        w[i] -= step_size * mi / (sqrtf(vi) + eps);
+    const drone_step_sums from = tensors.sums[blockIdx.y];
+    if (from.splits <= 0) {
+        for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < t.n; i += (int64_t)gridDim.x * kThreads) step(t, i, t.grad[i]);
+        return;
+    }
+    const int o = threadIdx.x % O, g = threadIdx.x / O;
+    for (int64_t base = (int64_t)blockIdx.x * O; base < t.n; base += (int64_t)gridDim.x * O) {
+        const int64_t i = base + o;
+        float sum = 0.0f;
+        if (i < t.n) {
+            int z = g;
+            for (; z + 7 * G < from.splits; z += 8 * G) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = from.sums[(size_t)(z + u * G) * t.n + i];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum += v[u];
+            }
+            for (; z < from.splits; z += G) sum += from.sums[(size_t)z * t.n + i];
+        }
+        s_sum[g][o] = sum;
+        __syncthreads();
+        if (g == 0 && i < t.n) {
+#pragma unroll
+            for (int k = 1; k < G; ++k) sum += s_sum[k][o];
+            const_cast<float *>(t.grad)[i] = sum;
+            step(t, i, sum);
+        }
+        __syncthreads();
     }
 }
 
@@ -742,27 +778,40 @@ extern "C" int drone_accuracy_f32(int n, int classes, const float *logits, int l
 }
 
 namespace {
-int steps_grid(const drone_step_tensor *t, int tensors, StepTensors *out)
+template <typename Step>
+int launch_steps(const drone_step_tensor *t, const drone_step_sums *sums, int tensors, const Step &step, hipStream_t s)
 {
-    int64_t most = 0;
+    StepTensors all{};
+    int grid = 1;
     for (int i = 0; i < tensors; ++i) {
-        out->t[i] = t[i];
-        most = std::max(most, t[i].n);
+        all.t[i] = t[i];
+        if (sums) all.sums[i] = sums[i];
+        grid = std::max(grid, all.sums[i].splits > 0 ? grid_for(8 * t[i].n, 1) : grid_for(t[i].n));
     }
-    return grid_for(most);
+    step_kernel<<<dim3(grid, tensors), kThreads, 0, s>>>(all, step);
+    DRONE_HIP_TRY(hipGetLastError());
+    return DRONE_OK;
+}
+bool sums_fit(const drone_step_tensor *t, const drone_step_sums *sums, int tensors)
+{
+    for (int i = 0; sums && i < tensors; ++i)
+        if (sums[i].splits > 0 && t[i].n > 0 && !sums[i].sums) return false;
+    return true;
 }
 }  // namespace
 
 extern "C" int drone_sgd_steps_f32(const drone_step_tensor *t, int tensors, float lr, drone_stream_t stream)
 {
+    return drone_sgd_steps_sums_f32(t, nullptr, tensors, lr, stream);
+}
+
+extern "C" int drone_sgd_steps_sums_f32(const drone_step_tensor *t, const drone_step_sums *sums, int tensors, float lr, drone_stream_t stream)
+{
     clear_error();
     DRONE_REQUIRE(t && tensors >= 1 && tensors <= kStepTensors, "tensors");
     for (int i = 0; i < tensors; ++i) DRONE_REQUIRE(t[i].n >= 0 && (t[i].n == 0 || (t[i].w && t[i].grad)), "null operand");
-    StepTensors all{};
-    const int grid = steps_grid(t, tensors, &all);
-    sgd_kernel<<<dim3(grid, tensors), kThreads, 0, as_stream(stream)>>>(all, lr);
-    DRONE_HIP_TRY(hipGetLastError());
-    return DRONE_OK;
+    DRONE_REQUIRE(sums_fit(t, sums, tensors), "null sums");
+    return launch_steps(t, sums, tensors, SgdStep{lr}, as_stream(stream));
 }
 
 extern "C" int drone_sgd_step_f32(float *w, const float *g, int64_t n, float lr, drone_stream_t stream)
@@ -775,16 +824,19 @@ extern "C" int drone_sgd_step_f32(float *w, const float *g, int64_t n, float lr,
 extern "C" int drone_adam_steps_f32(const drone_step_tensor *t, int tensors, float weight_decay, float lr, float beta1,
                                     float beta2, float eps, int step_count, drone_stream_t stream)
 {
+    return drone_adam_steps_sums_f32(t, nullptr, tensors, weight_decay, lr, beta1, beta2, eps, step_count, stream);
+}
+
+extern "C" int drone_adam_steps_sums_f32(const drone_step_tensor *t, const drone_step_sums *sums, int tensors, float weight_decay, float lr,
+                                         float beta1, float beta2, float eps, int step_count, drone_stream_t stream)
+{
     clear_error();
     DRONE_REQUIRE(t && tensors >= 1 && tensors <= kStepTensors && step_count >= 1, "tensors / step_count");
     for (int i = 0; i < tensors; ++i)
         DRONE_REQUIRE(t[i].n >= 0 && (t[i].n == 0 || (t[i].w && t[i].grad && t[i].m && t[i].v)), "operands");
     const float step_size = lr * sqrtf(1 - powf(beta2, (float)step_count)) / (1 - powf(beta1, (float)step_count));
-    StepTensors all{};
-    const int grid = steps_grid(t, tensors, &all);
-    adam_kernel<<<dim3(grid, tensors), kThreads, 0, as_stream(stream)>>>(all, weight_decay, beta1, beta2, eps, step_size);
-    DRONE_HIP_TRY(hipGetLastError());
-    return DRONE_OK;
+    DRONE_REQUIRE(sums_fit(t, sums, tensors), "null sums");
+    return launch_steps(t, sums, tensors, AdamStep{weight_decay, beta1, beta2, eps, step_size}, as_stream(stream));
 }
 
 extern "C" int drone_adam_step_f32(float *w, const float *g, float *m, float *v, int64_t n, int decay,

@@ -52,6 +52,12 @@ struct Variable {
     bool requires_grad, is_weight;
     int rows, cols, ld, size;
     bool owns_data = true;
+    // A weight's gradient between a backward pass and an optimiser step that follow each other inside one call: the partial sums of a
+    // split reduction, which the step adds up (drone_sgemm_tn_sums_f32).  keep_sums: leave it so; splits: whether it is.
+    float *sums = nullptr;  // the model's
+    int64_t sums_floats = 0;
+    bool keep_sums = false;
+    int splits = 0;
 
     Variable(int rows_, int cols_, bool requires_grad_ = true, bool is_weight_ = false, float *external = nullptr,
              int external_ld = 0)
@@ -127,9 +133,15 @@ public:
         if (b->requires_grad) {
             if (mirror2worker)  // cuda_module.cu:89-90: zero the mirrors' rows of c->grad in place, after a->grad used them
                 DRONE_GCN_CHECK(drone_clear_mirror_rows_f32(c->grad, c->ld, m, p, mirror2worker, s));
-            DRONE_GCN_CHECK(drone_sgemm_rm_f32(1, 0, n, p, m, 1.0f, a->data, a->ld, c->grad, c->ld, 0.0f, b->grad, b->ld, s));
+            if (b->keep_sums)
+                DRONE_GCN_CHECK(drone_sgemm_tn_sums_f32(n, p, m, a->data, a->ld, c->grad, c->ld, b->grad, b->ld, b->sums, b->sums_floats,
+                                                        &b->splits, s));
+            else
+                DRONE_GCN_CHECK(drone_sgemm_rm_f32(1, 0, n, p, m, 1.0f, a->data, a->ld, c->grad, c->ld, 0.0f, b->grad, b->ld, s));
         }
     }
+    // The floats of the weight gradient's partial sums.
+    int64_t sums_floats() const { return b->ld == p ? drone_sgemm_tn_sums_floats(n, p, m, a->ld, c->ld) : 0; }
 };
 
 // The weighted adjacency shared by the GraphSum modules of one model: edge values, the transposed CSR and
@@ -437,10 +449,15 @@ public:
     {
         step_count++;
         std::vector<drone_step_tensor> t;
-        for (auto &sl : vars) t.push_back({sl.var->data, sl.var->grad, sl.m, sl.v, (int64_t)sl.var->rows * sl.var->ld, sl.decay});
+        std::vector<drone_step_sums> sums;
+        for (auto &sl : vars) {
+            t.push_back({sl.var->data, sl.var->grad, sl.m, sl.v, (int64_t)sl.var->rows * sl.var->ld, sl.decay});
+            sums.push_back({sl.var->sums, sl.var->splits});
+            sl.var->splits = 0;
+        }
         for (size_t i = 0; i < t.size(); i += 4)
-            DRONE_GCN_CHECK(drone_adam_steps_f32(&t[i], (int)(t.size() - i < 4 ? t.size() - i : 4), params.weight_decay, params.lr,
-                                                 params.beta1, params.beta2, params.eps, step_count, s));
+            DRONE_GCN_CHECK(drone_adam_steps_sums_f32(&t[i], &sums[i], (int)(t.size() - i < 4 ? t.size() - i : 4), params.weight_decay,
+                                                      params.lr, params.beta1, params.beta2, params.eps, step_count, s));
     }
 };
 
@@ -454,9 +471,14 @@ public:
     void step() override
     {
         std::vector<drone_step_tensor> t;
-        for (auto *v : vars) t.push_back({v->data, v->grad, nullptr, nullptr, (int64_t)v->rows * v->ld, 0});
+        std::vector<drone_step_sums> sums;
+        for (auto *v : vars) {
+            t.push_back({v->data, v->grad, nullptr, nullptr, (int64_t)v->rows * v->ld, 0});
+            sums.push_back({v->sums, v->splits});
+            v->splits = 0;
+        }
         for (size_t i = 0; i < t.size(); i += 4)
-            DRONE_GCN_CHECK(drone_sgd_steps_f32(&t[i], (int)(t.size() - i < 4 ? t.size() - i : 4), lr, s));
+            DRONE_GCN_CHECK(drone_sgd_steps_sums_f32(&t[i], &sums[i], (int)(t.size() - i < 4 ? t.size() - i : 4), lr, s));
     }
 };
 
@@ -502,6 +524,8 @@ public:
     Replicas replicas;
     const int *mirror2worker = nullptr;    // device [N] (Graph::Mirror2Worker) with replicas, else null
     CrossEntropyLoss *ce = nullptr;
+    Matmul *matmul1 = nullptr, *matmul2 = nullptr;
+    float *weight_sums = nullptr;      // Variable::sums of both weights
     ReLU *relu = nullptr;              // layer 1 without dropout
     ReLUDropout *relu_drop = nullptr;  // layer 1 with dropout
     int input_cols = 0;          // inner dimension of layer 1's products: input_dim rounded up (padded_inner_dim)
@@ -583,10 +607,10 @@ public:
                 DRONE_GCN_CHECK(drone_spmm_csr_f32(adj->planT, adj->rpT, adj->ciT, adj->valT, input->data + c0, input->ld,
                                                    aggregated_input->data + c0, aggregated_input->ld, k, 1.0f, 0.0f, s));
             }
-            modules.emplace_back(new Matmul(aggregated_input, layer1_weight, layer1_var2, N, input_cols, p.hidden_dim,
+            modules.emplace_back(matmul1 = new Matmul(aggregated_input, layer1_weight, layer1_var2, N, input_cols, p.hidden_dim,
                                             "matmul_layer1_folded", s, nullptr, forward_cols));
         } else {
-            modules.emplace_back(new Matmul(input, layer1_weight, layer1_var1, N, input_cols, p.hidden_dim, "matmul_layer1", s,
+            modules.emplace_back(matmul1 = new Matmul(input, layer1_weight, layer1_var1, N, input_cols, p.hidden_dim, "matmul_layer1", s,
                                             mirror2worker, forward_cols));
             graphsum1 = new GraphSum(layer1_var1, layer1_var2, adj.get(), p.hidden_dim, "graphSum_layer1", s, r);
             modules.emplace_back(graphsum1);
@@ -598,13 +622,27 @@ public:
             relu = new ReLU(layer1_var2, "Relu", s);
             modules.emplace_back(relu);
         }
-        modules.emplace_back(new Matmul(layer1_var2, layer2_weight, layer2_var1, N, p.hidden_dim, p.output_dim, "matmul_layer2", s,
+        modules.emplace_back(matmul2 = new Matmul(layer1_var2, layer2_weight, layer2_var1, N, p.hidden_dim, p.output_dim, "matmul_layer2", s,
                                         mirror2worker));
         graphsum2 = new GraphSum(layer2_var1, output, adj.get(), p.output_dim, "graphSum_layer2", s, r);
         modules.emplace_back(graphsum2);
         ce = new CrossEntropyLoss(output, truth, p.output_dim, "CrossEntropy", s);
         modules.emplace_back(ce);
-        built_modules = modules.size();
+        for (auto &m : modules) built.push_back(m.get());
+        // Sums that wait for the step, up to 2 MB of them: more take a millisecond to allocate and no step gains more than 6 us by it
+        // (or loses, 44 MB of them, which come back from memory: 232,965-vertex step 7,588 -> 7,628 us).
+        constexpr int64_t kMostSums = 1 << 19;
+        int64_t taken = 0;
+        for (Matmul *m : {matmul2, matmul1}) {
+            Variable *w = m == matmul1 ? layer1_weight : layer2_weight;
+            const int64_t wanted = (m->sums_floats() + 63) / 64 * 64;
+            if (taken + wanted > kMostSums) continue;
+            w->sums_floats = wanted;
+            taken += wanted;
+        }
+        if (taken > 0) DRONE_GCN_HIP(hipMalloc(&weight_sums, sizeof(float) * (size_t)taken));
+        layer2_weight->sums = weight_sums;
+        layer1_weight->sums = weight_sums + layer2_weight->sums_floats;
         // cuda_gcn.cu:298-299, 314-315: what train_epoch / eval report besides the loss - the accuracy over the labelled
         // rows that are not mirrors (:226-246) and the L2 penalty weight_decay * sum(W1^2) / 2 (:254-260), from the
         // weights as they are before the optimiser step - comes out of the loss's launch
@@ -622,12 +660,14 @@ public:
         } else {
             optimizer.reset(new SGD({layer1_weight, layer2_weight}, p.learning_rate, s));
         }
+        built_optimizer = optimizer.get();
         DRONE_GCN_HIP(hipDeviceSynchronize());
     }
     GCN(const GCN &) = delete;
     ~GCN()
     {
         (void)hipFree(x_padded);
+        (void)hipFree(weight_sums);
         (void)hipFree(truth);
         (void)hipFree(labelled);
         (void)hipFree(truth_scratch);
@@ -669,8 +709,7 @@ public:
     void train_step_async()
     {
         forward(true);
-        backward();
-        optimizer->step();
+        backward_and_step();
     }
     // {loss + L2 penalty, accuracy} of the last forward pass, as CUDAGCN::train_epoch / eval return them.
     // cross_entropy (optional): the mean cross-entropy alone.
@@ -685,8 +724,7 @@ public:
     std::pair<float, float> train_epoch()
     {
         forward_on_split(true, 1);
-        backward();
-        optimizer->step();
+        backward_and_step();
         return read_metrics();
     }
     std::pair<float, float> eval(int current_split)  // cuda_gcn.cu:308-318
@@ -701,16 +739,33 @@ private:
     void forward_on_split(bool training, int current_split)
     {
         const bool counts_rows = params.mean_gradient && current_split != truth_split;
-        if (counts_rows || modules.size() != built_modules || modules.back().get() != ce) {
+        if (counts_rows || !as_built()) {
             choose_truth(current_split);
             forward(training);
             return;
         }
-        for (size_t i = 0; i + 1 < built_modules; ++i) modules[i]->forward(training);
+        for (size_t i = 0; i + 1 < built.size(); ++i) modules[i]->forward(training);
         ce->forward_on(training, split, label, current_split, truth);
         truth_split = current_split;
     }
-    size_t built_modules = 0;
+    // backward() and the step.  Nobody looks at the weight gradients in between - unless the program has changed what runs.
+    void backward_and_step()
+    {
+        const bool keep = as_built() && optimizer.get() == built_optimizer;
+        for (Variable *w : {layer1_weight, layer2_weight}) w->keep_sums = keep && w->sums_floats > 0;
+        backward();
+        for (Variable *w : {layer1_weight, layer2_weight}) w->keep_sums = false;
+        optimizer->step();
+    }
+    bool as_built() const
+    {
+        if (modules.size() != built.size()) return false;
+        for (size_t i = 0; i < built.size(); ++i)
+            if (modules[i].get() != built[i]) return false;
+        return true;
+    }
+    std::vector<const Module *> built;
+    const Optimizer *built_optimizer = nullptr;
     void settle_truth()  // behind a wait for the stream
     {
         if (!truth_pending) return;

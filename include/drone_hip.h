@@ -378,6 +378,21 @@ typedef struct drone_step_tensor {
     int64_t n;
     int decay;
 } drone_step_tensor;
+/* A weight gradient C = A^T B whose reduction is split: leaves the `*splits` partial sums, M x N each, in `sums` for
+ * drone_*_steps_sums_f32 to add up, or, where it is not split or `floats` are too few, writes C with *splits = 0.
+ * drone_sgemm_tn_sums_floats: how many floats it wants. */
+int64_t drone_sgemm_tn_sums_floats(int M, int N, int K, int lda, int ldb);
+int drone_sgemm_tn_sums_f32(int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc,
+                            float *sums, int64_t floats, int *splits, drone_stream_t stream);
+/* The steps below with gradients that are still such sums: where sums[i].splits > 0, t[i].grad is written (t[i].n floats) and then
+ * used. */
+typedef struct drone_step_sums {
+    const float *sums;
+    int splits;
+} drone_step_sums;
+int drone_sgd_steps_sums_f32(const drone_step_tensor *t, const drone_step_sums *sums, int tensors, float lr, drone_stream_t stream);
+int drone_adam_steps_sums_f32(const drone_step_tensor *t, const drone_step_sums *sums, int tensors, float weight_decay, float lr,
+                              float beta1, float beta2, float eps, int step_count, drone_stream_t stream);
 int drone_sgd_steps_f32(const drone_step_tensor *t, int tensors, float lr, drone_stream_t stream);
 int drone_adam_steps_f32(const drone_step_tensor *t, int tensors, float weight_decay, float lr, float beta1, float beta2,
                          float eps, int step_count, drone_stream_t stream);
