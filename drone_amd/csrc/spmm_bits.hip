@@ -55,15 +55,23 @@ __device__ __forceinline__ unsigned bf16_bits_rne(float x)
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
-// Thread (group of 8 ranked columns, feature column n of the pass): scales, splits and packs 8 values of B.
+// Feature columns that the product of `width` of a pass's 128 reads.
+int split_columns(int width) { return width <= 16 ? 16 : width <= 32 ? 32 : width <= 48 ? 48 : width <= 64 ? 64 : width <= 96 ? 96 : 128; }
+
+// Thread (group of 8 ranked columns, feature column n of the pass): scales, splits and packs 8 values of B.  N: columns that the
+// product reads; the places of the others in `split` stay as they are.  Bound by what it writes, six bytes a value, beside the gathers (with all
+// 128 columns, most of them zeros, forward and transposed product of 2.4 M vertices and 34 M entries at K = 32 926 instead of 894 us, of 3 M
+// at K = 64 2,190 instead of 2,180, and the 232,965-vertex step, whose second layer has 41, 7,697 instead of 7,662).
+template <int N>
 __global__ __launch_bounds__(256) void bits_split_kernel(int groups, const unsigned *__restrict__ col_order,
                                                          const float *__restrict__ col_scale,
-                                                         const float *__restrict__ B, int ldb, int K,
+                                                         const float *__restrict__ B, int ldb, int K, int first_pass,
                                                          uint4 *__restrict__ split)
 {
-    const int kg = blockIdx.x * 2 + threadIdx.x / 128, pass = blockIdx.y;
-    if (kg >= groups) return;
-    const int n = threadIdx.x % 128, k = pass * 128 + n;
+    constexpr int kGroups = 256 / N;
+    const int kg = blockIdx.x * kGroups + threadIdx.x / N, pass = first_pass + blockIdx.y;
+    if ((int)threadIdx.x >= kGroups * N || kg >= groups) return;
+    const int n = threadIdx.x % N, k = pass * 128 + n;
     unsigned part[3][8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -555,9 +563,24 @@ int bit_core_split(const BitCore *bc, const unsigned *col_order, const float *co
 {
     if (bc->tiles == 0) return DRONE_OK;
     DRONE_REQUIRE(K > 0 && K <= bc->max_k, "K exceeds the plan's feature width");
-    const int groups = bc->wmax / 8, passes = (int)ceil_div(K, 128);
-    bits_split_kernel<<<dim3((unsigned)ceil_div(groups, 2), (unsigned)passes), 256, 0, s>>>(groups, col_order, col_scale, B,
-                                                                                           ldb, K, bc->split);
+    const int groups = bc->wmax / 8, whole = K / 128;
+    const auto launch = [&](auto columns, int first, int passes) {
+        constexpr int N = decltype(columns)::value;
+        if (passes > 0)
+            bits_split_kernel<N><<<dim3((unsigned)ceil_div(groups, 256 / N), (unsigned)passes), 256, 0, s>>>(groups, col_order, col_scale, B, ldb, K,
+                                                                                                           first, bc->split);
+    };
+    launch(std::integral_constant<int, 128>(), 0, whole);
+    if (const int rest = K - 128 * whole) {
+        switch (split_columns(rest)) {
+        case 16: launch(std::integral_constant<int, 16>(), whole, 1); break;
+        case 32: launch(std::integral_constant<int, 32>(), whole, 1); break;
+        case 48: launch(std::integral_constant<int, 48>(), whole, 1); break;
+        case 64: launch(std::integral_constant<int, 64>(), whole, 1); break;
+        case 96: launch(std::integral_constant<int, 96>(), whole, 1); break;
+        default: launch(std::integral_constant<int, 128>(), whole, 1);
+        }
+    }
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
@@ -576,12 +599,14 @@ int bit_core_products(const BitCore *bc, int K, hipStream_t s)
             kernel<<<bc->num_units, 512, 0, s>>>(bc->unit_tile, bc->unit_c0, bc->unit_c1, bc->unit_slot, bc->tile_blocks,
                                                  bc->tile_off, bc->bits, split, partial);
         };
-        if (width <= 16) launch(bits_mfma16_kernel<1>);
-        else if (width <= 32) launch(bits_mfma_kernel<1>);
-        else if (width <= 48) launch(bits_mfma16_kernel<3>);
-        else if (width <= 64) launch(bits_mfma_kernel<2>);
-        else if (width <= 96) launch(bits_mfma_kernel<3>);
-        else launch(bits_mfma_kernel<4>);
+        switch (split_columns(width)) {
+        case 16: launch(bits_mfma16_kernel<1>); break;
+        case 32: launch(bits_mfma_kernel<1>); break;
+        case 48: launch(bits_mfma16_kernel<3>); break;
+        case 64: launch(bits_mfma_kernel<2>); break;
+        case 96: launch(bits_mfma_kernel<3>); break;
+        default: launch(bits_mfma_kernel<4>);
+        }
     }
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
