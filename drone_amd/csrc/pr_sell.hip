@@ -186,7 +186,7 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
 // again, and who looks at the set has read what it published then.  The last work-group to leave clears the last set, and the counters.
 //
 // The work-groups wait for each other, so all must have a place on the chip before any starts.  Each reports at a gate; one that
-// has looked `patience` times in vain closes it and does the whole run alone, and the others go.  (Behind a gate that has opened
+// has looked `patience` times in vain closes it and does the whole run alone, and the others go; every sum has the same order then.  (Behind a gate that has opened
 // all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long goes on with the NaN.)
 constexpr int kSellResidentThreads = 1024;
 constexpr unsigned long long kSellNone = 0x7ffc5e1100a1b2c3ull, kSellNan = 0x7ff8000000000000ull;
@@ -481,7 +481,10 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
             for (int h = group + groups; h < hubs; h += groups) {
                 int ids[kHubAhead];
                 hub_fetch(hub_step[h], hub_step[h + 1], ids);
-                const double total = block_sum<T>(hub_sum(hub_step[h], hub_step[h + 1], ids), s_hub);
+                const double wave_part = lanes_sum(hub_sum(hub_step[h], hub_step[h + 1], ids), kWave);
+                if (lane == 0) s_hub[wave] = wave_part;
+                __syncthreads();
+                const double total = lanes_sum(s_hub[lane & (T / kWave - 1)], T / kWave);
                 if (tid == 0) {
                     hand_on(h, inv_user[order[h]], total);
                     store(h, total);
