@@ -31,7 +31,6 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "exchange.h"
-#include "flag.h"
 
 using namespace drone;
 
@@ -87,7 +86,6 @@ struct Report {
     TraverseState state;
     double visited;  // vertices with active != 0, if the list is empty
     int again;       // labels: whether edges between trees are left
-    unsigned raised; // TraverseExt::flag
 };
 // Two lists of vertices, and where each listed vertex's out-edges start in the list's concatenated out-edges.
 struct Lists {
@@ -96,16 +94,15 @@ struct Lists {
 // A list of no vertices that no round may take for its own: all of them still have to propagate.
 __host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
 
-// Ends a counting kernel: the last work-group adds the work-groups' counts and leaves the sum in *out.  True in the thread that does.
-__device__ __forceinline__ bool publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
+// Ends a counting kernel: the last work-group adds the work-groups' counts and leaves the sum in *out.
+__device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
 {
     const double total = block_sum_256(mine, s_red);
     unsigned int one = 0;
     if (threadIdx.x == 0) one = publish_part(block_part + blockIdx.x, total);
-    if (!last_block_done(ticket, one)) return false;
+    if (!last_block_done(ticket, one)) return;
     const double all = block_sum_of_parts(block_part, (int)gridDim.x, s_red);
     if (threadIdx.x == 0) *out = all;
-    return threadIdx.x == 0;
 }
 
 // ---- labels by joining trees -------------------------------------------------------------------------------
@@ -409,20 +406,14 @@ __global__ __launch_bounds__(kSpmvBlock) void process_messages_kernel(int n, int
 // Ends what the host enqueues before it waits: tells it where the traversal stands and, if nothing is left to propagate or
 // `always`, counts the vertices with active != 0 (common.cu:17-31, without atomics on one address).
 __global__ __launch_bounds__(kSpmvBlock) void report_kernel(int n, bool always, const int *__restrict__ active, const TraverseState *state,
-                                                            double *block_part, unsigned int *ticket, Report *report, unsigned *word, unsigned value)
+                                                            double *block_part, unsigned int *ticket, Report *report)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
-    const auto tell = [&] {
-        report->state = *state;
-        raise_flag(word, value);
-    };
-    if (!always && state->listed != 0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) tell();
-        return;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) report->state = *state;
+    if (!always && state->listed != 0) return;
     double cnt = 0.0;
     for (int i = blockIdx.x * kSpmvBlock + threadIdx.x; i < n; i += gridDim.x * kSpmvBlock) cnt += active[i] != 0;
-    if (publish_sum(cnt, s_red, block_part, ticket, &report->visited)) tell();
+    publish_sum(cnt, s_red, block_part, ticket, &report->visited);
 }
 
 __global__ void iota_kernel(int *out, int n)
@@ -504,7 +495,6 @@ struct TraverseExt {
     CcTrees *trees = nullptr;               // device
     int call = 0, pass = 0;                 // of the tree kernels, counted: what *trees names them by
     Report *report = nullptr;               // pinned
-    drone_flag flag{};                      // the waits for it
 };
 
 double seconds_since(std::chrono::steady_clock::time_point t0)
@@ -532,7 +522,6 @@ TraverseExt *traverse_ext_create(int n, const Rows *sampled = nullptr)
     if (t->blocks > 4096) t->blocks = 4096;
     DRONE_HIP_OR_DIE(hipHostMalloc(&t->report, sizeof(Report)));
     *t->report = Report{};
-    t->flag.word = &t->report->raised;
     if (sampled && n > 0) cc_sample_kernel<<<1, kCcSampled>>>(n, *sampled, &t->report->again);
     DRONE_HIP_OR_DIE(hipMalloc(&t->stat, sizeof(double)));
     DRONE_HIP_OR_DIE(hipMalloc(&t->block_part, sizeof(double) * (size_t)kSumBlocks));
@@ -572,13 +561,13 @@ int sum_blocks(int64_t n, int per_lane = 4) { return (int)std::min<int64_t>(std:
 void launch_report(Graph *g, TraverseExt *t, bool always, hipStream_t s)
 {
     const int n = getLocalVertexSize(g);
-    report_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, always, g->active, t->state, t->block_part, t->ticket, t->report, t->flag.word, ++t->flag.raised);
+    report_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, always, g->active, t->state, t->block_part, t->ticket, t->report);
 }
 
 int count_active(Graph *g, TraverseExt *t, hipStream_t s)
 {
     launch_report(g, t, true, s);
-    DRONE_HIP_OR_DIE(flag_seen(&t->flag, s));
+    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
     return (int)t->report->visited;
 }
 
@@ -1547,7 +1536,8 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bo
         sweeps = sweeps_next;
         pushes = pushes_next;
         launch_report(g, t, false, s);
-        DRONE_HIP_OR_DIE(flag_seen(&t->flag, s));
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
         now = t->report->state;
         known = true;
         if (now.listed == 0) return now.rounds;
@@ -1631,7 +1621,8 @@ TraverseState join_labels(Graph *g, TraverseExt *t, int *cc, hipStream_t s)
         cc_flatten_kernel<<<blocks, kSpmvBlock, 0, s>>>(n, rows, cc, t->trees, call, first);
         cc_link_kernel<<<(unsigned)std::min<int64_t>(ceil_div(n, kLinkThreads), kLinkBlocks), kLinkThreads, 0, s>>>(n, rows, cc, t->trees, call, pass);
         cc_finish_kernel<<<sum_blocks(n, 1), kSpmvBlock, 0, s>>>(n, cc, g->active, t->trees, call, pass, t->block_part, t->ticket, t->report);
-        DRONE_HIP_OR_DIE(flag_wait(&t->flag, s));
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
         x->one_way = t->report->state.listed != 0;
         if (x->one_way || !t->report->again) return t->report->state;
     }
@@ -1661,7 +1652,7 @@ struct SsspRun {
         if (!counted) {
             count_lengths();
             launch_report(g, t, false, s);
-            DRONE_HIP_OR_DIE(flag_seen(&t->flag, s));
+            DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
         }
         return t->report->state.not_one == 0.0;
     }
@@ -1784,7 +1775,8 @@ bool run_chains(Graph *g, TraverseExt *t, float *dist, int start_id, hipStream_t
         if (long_lists) small();
         chain_fill_kernel<<<sum_blocks(n), kSpmvBlock, 0, s>>>(n, rows, g->Global2Local, start_id, c.arc, g->active, dist, t->state, t->block_part,
                                                               t->ticket, t->report);
-        DRONE_HIP_OR_DIE(flag_wait(&t->flag, s));
+        DRONE_HIP_OR_DIE(hipGetLastError());
+        DRONE_HIP_OR_DIE(hipStreamSynchronize(s));
         c.other_lengths = t->report->state.not_one != 0.0;
     } while (!c.other_lengths && t->report->state.listed != 0);
     return !c.other_lengths;

@@ -29,12 +29,13 @@ void clear_error()
 }
 
 namespace {
-__global__ void raise_flag_kernel(unsigned *word, unsigned value) { raise_flag(word, value); }
+__global__ void raise_flag_kernel(unsigned *word, unsigned value) { __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
 constexpr int kFlagMicroseconds = 200;  // looked for so long: less than the gain is lost then
 }  // namespace
 
-hipError_t flag_seen(drone_flag *f, hipStream_t s)
+hipError_t flag_wait(drone_flag *f, hipStream_t s)
 {
+    raise_flag_kernel<<<1, 1, 0, s>>>(f->word, ++f->raised);
     const hipError_t launched = hipGetLastError();
     if (launched != hipSuccess) return launched;
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kFlagMicroseconds);
@@ -45,12 +46,6 @@ hipError_t flag_seen(drone_flag *f, hipStream_t s)
         }
     } while (std::chrono::steady_clock::now() < until);
     return hipStreamSynchronize(s);
-}
-
-hipError_t flag_wait(drone_flag *f, hipStream_t s)
-{
-    raise_flag_kernel<<<1, 1, 0, s>>>(f->word, ++f->raised);
-    return flag_seen(f, s);
 }
 
 static inline uint64_t splitmix64(uint64_t x)
