@@ -125,18 +125,13 @@ void graph_ext_release(GraphExt *x);  // frees everything but the struct itself
 // aggregations (their value types are at most 8 bytes).  Built on first use; exits on failure.
 void ensure_aggregation_ready(Graph *g);
 
-struct PushReport {
-    double active;
-    unsigned raised;  // PRExt::flag
-};
 struct PRExt {
     float *push = nullptr;        // device [n]: value each vertex pushes along its out-edges this step
     double *stat = nullptr;       // device scalar: statistic of the last launch
-    PushReport *stat_host = nullptr;  // pinned: the aggregation's last work-group writes the same value to it
+    double *stat_host = nullptr;  // pinned host word that the aggregation's last work-group writes the same value to
     unsigned int *ticket = nullptr;  // device counter of the vertex kernel's last_block_done
     double *block_part = nullptr; // device [vertex_blocks]
     int vertex_blocks = 0;
-    drone_flag flag{};            // a superstep's wait
 };
 
 }  // namespace drone

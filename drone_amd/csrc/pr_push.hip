@@ -8,7 +8,6 @@
 #include <cstdlib>
 
 #include "exchange.h"
-#include "flag.h"
 
 using namespace drone;
 
@@ -365,19 +364,19 @@ int aggregate_push(Graph *g, PRValues *values, hipStream_t s)
         const int fb = fixup_blocks(rb.num_blocks);
         spmv_fixup_kernel<PushF2, PushEpi, StoreStat><<<fb, kSpmvBlock, 0, s>>>(
             rb.num_blocks, rb.block_row, rb.walk_len, carry, x->ms_rb.tile_stat, epi, x->ms_rb.block_stat,
-            x->ms_rb.ticket, StoreStat{px->stat, &px->stat_host->active});
+            x->ms_rb.ticket, StoreStat{px->stat, px->stat_host});
     } else if (x->sell_ready) {
-        if (sell_push(x->sell, px->push, values->diffValue, g->active, x->sell_part, x->sell_ticket, StoreStat{px->stat, &px->stat_host->active}, s) != DRONE_OK) {
+        if (sell_push(x->sell, px->push, values->diffValue, g->active, x->sell_part, x->sell_ticket, StoreStat{px->stat, px->stat_host}, s) != DRONE_OK) {
             printf("Failed: %s\n", drone_last_error_string());
             exit(EXIT_FAILURE);
         }
     } else {
         spmv_merge_launch<PushF2, int, kPushIpt, PushEpi>(x->mt, x->ms, x->in_index, x->in_src, epi, px->stat, s,
-                                                          &px->stat_host->active);
+                                                          px->stat_host);
     }
     DRONE_HIP_OR_DIE(hipGetLastError());
-    DRONE_HIP_OR_DIE(flag_wait(&px->flag, s));  // the aggregation's last work-group has written the count to the host
-    return (int)px->stat_host->active;
+    DRONE_HIP_OR_DIE(hipStreamSynchronize(s));  // the fix-up's last work-group has written the count to the host
+    return (int)*px->stat_host;
 }
 
 }  // namespace
@@ -448,9 +447,7 @@ extern "C" Response PR_PEVal(Graph *g, PRValues *values, int workerId, int worke
         PRExt *px = new PRExt();
         DRONE_HIP_OR_DIE(hipMalloc(&px->push, sizeof(float) * cnt));
         DRONE_HIP_OR_DIE(hipMalloc(&px->stat, sizeof(double)));
-        DRONE_HIP_OR_DIE(hipHostMalloc(&px->stat_host, sizeof(PushReport)));
-        *px->stat_host = PushReport{};
-        px->flag.word = &px->stat_host->raised;
+        DRONE_HIP_OR_DIE(hipHostMalloc(&px->stat_host, sizeof(double)));
         px->vertex_blocks = (int)ceil_div(cnt, kSpmvBlock * 4);
         if (px->vertex_blocks > 4096) px->vertex_blocks = 4096;
         DRONE_HIP_OR_DIE(hipMalloc(&px->block_part, sizeof(double) * (size_t)px->vertex_blocks));

@@ -1,10 +1,9 @@
 // Error channel, seeded generators (host code) and the HIP-event stopwatch.
-#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
 
-#include "flag.h"
+#include "common.h"
 
 namespace drone {
 
@@ -26,26 +25,6 @@ void clear_error()
 {
     g_err_code = 0;
     g_err_msg[0] = '\0';
-}
-
-namespace {
-__global__ void raise_flag_kernel(unsigned *word, unsigned value) { __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
-constexpr int kFlagMicroseconds = 200;  // looked for so long: less than the gain is lost then
-}  // namespace
-
-hipError_t flag_wait(drone_flag *f, hipStream_t s)
-{
-    raise_flag_kernel<<<1, 1, 0, s>>>(f->word, ++f->raised);
-    const hipError_t launched = hipGetLastError();
-    if (launched != hipSuccess) return launched;
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(kFlagMicroseconds);
-    do {
-        for (int i = 0; i < 64; ++i) {
-            if (__atomic_load_n(f->word, __ATOMIC_ACQUIRE) == f->raised) return hipSuccess;
-            __builtin_ia32_pause();
-        }
-    } while (std::chrono::steady_clock::now() < until);
-    return hipStreamSynchronize(s);
 }
 
 static inline uint64_t splitmix64(uint64_t x)
@@ -218,13 +197,5 @@ extern "C" int drone_timer_destroy(drone_timer *t)
 extern "C" int drone_device_synchronize(void)
 {
     DRONE_HIP_TRY(hipDeviceSynchronize());
-    return DRONE_OK;
-}
-
-extern "C" int drone_flag_wait(drone_flag *f, drone_stream_t s)
-{
-    clear_error();
-    DRONE_REQUIRE(f != nullptr && f->word != nullptr, "flag");
-    DRONE_HIP_TRY(flag_wait(f, as_stream(s)));
     return DRONE_OK;
 }

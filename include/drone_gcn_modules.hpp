@@ -359,7 +359,6 @@ public:
         float loss;
         int labelled;
         drone_loss_report report;
-        unsigned raised;
     } *pinned = nullptr;
     float *d_loss = nullptr;  // = &pinned->loss
     int *d_count = nullptr;   // device scalar
@@ -389,7 +388,6 @@ public:
         p.report = report;
         return p;
     }
-    drone_flag flag = {};  // GCN::read_metrics() waits by it
     CrossEntropyLoss(Variable *logits_, const int *truth_, int num_classes_, std::string name, drone_stream_t stream)
         : logits(logits_), truth(truth_), num_classes(num_classes_), s(stream)
     {
@@ -397,7 +395,6 @@ public:
         DRONE_GCN_HIP(hipHostMalloc(&pinned, sizeof(Pinned)));
         *pinned = Pinned{};
         d_loss = &pinned->loss;
-        flag.word = &pinned->raised;
         DRONE_GCN_HIP(hipMalloc(&d_count, sizeof(int)));
     }
     ~CrossEntropyLoss() override { (void)hipHostFree(pinned); (void)hipFree(d_count); }
@@ -715,7 +712,7 @@ public:
     // cross_entropy (optional): the mean cross-entropy alone.
     std::pair<float, float> read_metrics(float *cross_entropy = nullptr)
     {
-        DRONE_GCN_CHECK(drone_flag_wait(&ce->flag, s));
+        DRONE_GCN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(s)));
         settle_truth();
         const float loss = *ce->d_loss;
         if (cross_entropy) *cross_entropy = loss;

@@ -496,13 +496,6 @@ int drone_timer_stop(drone_timer *t, drone_stream_t stream);
 int drone_timer_elapsed_ms(drone_timer *t, float *ms); /* synchronises on the stop event */
 int drone_timer_destroy(drone_timer *t);
 int drone_device_synchronize(void);
-/* Waits for everything enqueued on a stream, as hipStreamSynchronize does, some microseconds faster: through a word of
- * pinned memory.  A flag is for one thread at a time; a stream that takes long is waited for in the usual way. */
-typedef struct drone_flag {
-    unsigned *word;  /* the caller's, pinned, 0 to begin with */
-    unsigned raised; /* the last value asked for, 0 to begin with */
-} drone_flag;
-int drone_flag_wait(drone_flag *flag, drone_stream_t stream);
 
 /* ====================================================================================== */
 /* E. Partition files and the pr_cuda worker's compute side (host code)                   */
