@@ -947,7 +947,8 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         DRONE_HIP_TRY(sr->entries.commit());
         if (sr->resident) {
             sell_slots_kernel<<<64, 256, 0, s>>>(slots, sr->live, sr->exchange, sr->gate);
-            DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sell_resident_of(*sr)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sr->lds));
+            // the limit belongs to the kernel, which plans of other sizes share
+            DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sell_resident_of(*sr)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSellResidentLds));
         }
         sell_fill_kernel<<<sr->hubs + (int)ceil_div(sr->slices, 256 / kWave), 256, 0, s>>>(
             sh, sr->threads, sr->order, row_ptr, col, new_id, sr->hub_step, slice_step, sr->slice, sr->hub_col, sr->col, sr->hot);

@@ -1,5 +1,8 @@
 """Where the arrays of LDS start that kernels fill 16 bytes at a time: dynamic LDS follows a kernel's static LDS, whose size the compiler
-rounds up to the alignment that the dynamic array is declared with and writes into the code object."""
+rounds up to the alignment that the dynamic array is declared with and writes into the code object.  And how much of it a kernel may ask for."""
+import glob
+import os
+import re
 import struct
 
 import pytest
@@ -37,3 +40,13 @@ def test_hot_sources_start_at_16_bytes():
     assert len(hot) == 2
     assert all(size % 16 == 0 for size in hot.values()), hot
     assert all(size + 160_000 <= 163_840 for size in hot.values()), hot
+
+
+def test_limits_of_dynamic_lds_are_constants():
+    """The limit that hipFuncSetAttribute sets belongs to the kernel, not to the handle that sets it: were it a handle's own size, a handle
+    made later with a smaller one would leave too low a limit behind for those made before."""
+    limits = []
+    for path in glob.glob(os.path.join(os.path.dirname(_lib.library_path()), "*.hip")):
+        limits += re.findall(r"hipFuncAttributeMaxDynamicSharedMemorySize,\s*(?:\(int\))?([^()\s]+)\)", open(path).read())
+    assert len(limits) >= 6
+    assert all(re.fullmatch(r"k[A-Z]\w*", limit) for limit in limits), limits

@@ -124,3 +124,15 @@ def test_runs_beside_each_other():
     for p, o, w in zip(plans, outs, want):
         assert torch.equal(o, w)  # also where one run was a work-group's alone
         p.close()
+
+
+def test_plans_that_share_a_kernel(oracle):
+    """Plans of 1,024 rows with entries each: their runs are one kernel, which asks for 152, 8 and 40 KB of LDS in turn."""
+    plans = []
+    for rest in (9000, 0, 2000):
+        rp, ci, inv = _matrix(1024 + rest, [5] * 1024, 0)
+        plans.append((_plan(rp, ci, inv), oracle.pr_pull_f64(rp, ci, inv, 0.85, 6), rp))
+    for plan, want, rp in plans:
+        _close(plan.run(0.85, 6).cpu().numpy(), want, rp, 6)
+    for plan, _, _ in plans:
+        plan.close()
