@@ -101,7 +101,6 @@ SIGNATURES = {
     "drone_pr_plan_destroy": (_I, [_P]),
     "drone_pr_run_f64": (_I, [_P, _D, _I, _P, _P]),
     "drone_pr_profile_enable": (_I, [_P, _I]),
-    "drone_pr_plan_patience": (_I, [_P, _I]),
     "drone_pr_profile_read": (_I, [_P, C.POINTER(_I), C.POINTER(_D), C.POINTER(_D), C.POINTER(_D)]),
     "drone_pr_bytes_per_iteration": (_I64, [_I64, _I64]),
     "drone_pr_run_graph_f64": (_I, [C.POINTER(Graph), C.POINTER(PRValues), _D, _I, _P]),

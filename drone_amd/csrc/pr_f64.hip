@@ -241,6 +241,7 @@ extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
     return DRONE_OK;
 }
 
+// For the tests, which have no busy chip at hand, and not in the public header: SellRows::patience.
 extern "C" int drone_pr_plan_patience(drone_pr_plan *p, int looks)
 {
     clear_error();

@@ -184,9 +184,6 @@ int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_
 int drone_pr_profile_enable(drone_pr_plan *plan, int max_launches);
 int drone_pr_profile_read(drone_pr_plan *plan, int *launches, double *mean_ms, double *min_ms,
                           double *max_ms);
-/* Runs of a small matrix are one launch whose work-groups wait for each other.  `looks`: how often each looks whether all
- * have found a place on the chip, before one of them does the run alone (64 by default; the results are the same). */
-int drone_pr_plan_patience(drone_pr_plan *plan, int looks);
 /* Algorithmic bytes of one iteration: 4*nnz + 32*n + 8. */
 int64_t drone_pr_bytes_per_iteration(int64_t n, int64_t nnz);
 
