@@ -241,12 +241,13 @@ extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
     return DRONE_OK;
 }
 
-// For the tests, which have no busy chip at hand, and not in the public header: SellRows::patience.
-extern "C" int drone_pr_plan_patience(drone_pr_plan *p, int looks)
+// For the tests, which have no busy chip at hand, and not in the public header: SellRows::rule.
+extern "C" int drone_pr_plan_gate(drone_pr_plan *p, int patience, int places)
 {
     clear_error();
-    DRONE_REQUIRE(p != nullptr && looks >= 0, "number of looks");
-    p->sr.patience = looks;
+    DRONE_REQUIRE(p != nullptr && patience >= 0 && places >= 1, "gate");
+    p->sr.rule.patience = patience;
+    p->sr.rule.places = places;
     return DRONE_OK;
 }
 

@@ -42,6 +42,12 @@ constexpr int kSellHubDepth = 16, kSellWaveSteps = 12, kSellWaveStepsWide = 16;
 constexpr int kSellDepthF32 = 16, kSellWaveStepsF32 = 32;  // the same of float rows
 constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,000 of 163,840 bytes
 
+// When the work-groups of a run in one launch stop waiting for the others (sell_enter): not before `patience` looks, and when `places` have come.
+struct SellGate {
+    int patience = 64, places = INT_MAX;
+    int enough = 1, price = 0;  // work-groups as good as all, and looks that the run is worth to one: of the run
+};
+
 struct SellRows {
     int64_t n = 0, nnz = 0;
     int threads = 256;               // work-group size of the iteration, 256 or 512; 1,024 with the hot sources in LDS
@@ -58,7 +64,7 @@ struct SellRows {
     double *inv = nullptr;           // device [n]: inverse out-degrees in row order, refreshed by every run
     double *part[2] = {nullptr, nullptr};  // device: dangling mass per work-group, of this iteration and the one before
     int init_blocks = 0;
-    int patience = 64;               // looks at the gate before a work-group of it does the run alone
+    SellGate rule;                   // of sell_resident_kernel
     int resident = 0;                // work-groups of sell_resident_kernel, or 0: a launch per iteration
     int staged = 0;                  // slots that a lane of it brings into LDS
     size_t lds = 0;                  // bytes of its sources in LDS

@@ -185,12 +185,22 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
 // again two iterations on and looked at three on; the owner waits for its clearing store (which writes through) before it publishes
 // again, and who looks at the set has read what it published then.  The last work-group to leave clears the last set, and the counters.
 //
-// The work-groups wait for each other, so all must have a place on the chip before any starts.  Each reports at a gate; one that
-// has looked `patience` times in vain closes it and does the whole run alone, and the others go; every sum has the same order then.  (Behind a gate that has opened
-// all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long goes on with the NaN.)
+// The work-groups wait for each other, so all that take part must have a place on the chip before any starts.  Each reports at a gate; one
+// that has looked in vain for long enough closes it, those who have come by then do the run, and later ones go; every sum has the same order
+// then.  (Behind the gate all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long goes on with the
+// NaN.)  Long enough: `patience` looks where who is there takes no more rounds of slices and hub rows than all would; else also as many as
+// the run would take with them, at kSellLooksPerRound a round (1.2 us on an idle chip, four times that beside a stream of memory-bound
+// kernels), so that the wait at most doubles it.  20 / 3 iterations beside a stream that adds to 1 GiB of floats, us, a launch per iteration
+// / one work-group behind every closed gate / this: 4 K vertices and 53 K entries 289 / 111 / 112 and 67 / 45 / 47, 12 K and 108 K 313 / 3,300 / 250
+// and 70 / 557 / 175-260, 12 K and 419 K 381 / 12,700 / 250-315 and 82 / 1,930 / 250; beside bf16 products of 8,192 rows, whose work-groups fill
+// the chip for 0.7 ms each, 16,000 / 80-5,300 / 780.  What the short runs of more than 10 K rows lose are the places: 123 registers a lane ask for an
+// empty CU (with 96, at the price of 27 spilled, 71 / 80, but 20 iterations of an idle chip 78 -> 104 and 91 -> 132).
 constexpr int kSellResidentThreads = 1024;
 constexpr unsigned long long kSellNone = 0x7ffc5e1100a1b2c3ull, kSellNan = 0x7ff8000000000000ull;
-constexpr unsigned kSellClosed = 1u << 31;
+// The gate: who has come, and once it is closed how many of them do the run.
+constexpr unsigned kSellClosed = 1u << 31, kSellCame = 0xff;
+constexpr int kSellRunShift = 8, kSellLooksPerRound = 2, kSellMostLooks = 1 << 22;
+static_assert(kSellResidentBlocks <= (int)kSellCame, "a byte each");
 constexpr int kSellPolls = 1 << 22;
 constexpr int kSellWaitStores = 0x0f70;  // s_waitcnt vmcnt(0)
 
@@ -207,22 +217,23 @@ __global__ void sell_slots_kernel(int slots, int used, unsigned long long *__res
     if (blockIdx.x == 0 && threadIdx.x < 2 * kTicketStride) gate[threadIdx.x] = 0;
 }
 
-// Through the gate: this work-group's number among `groups`, or -1 to leave.  ticket: how many came before.
-__device__ __forceinline__ int sell_enter(unsigned *gate, unsigned ticket, int &groups, int patience)
+// Through the gate: this work-group's number in the run and, from kSellRunShift on, how many do it, or -1 to leave.  ticket: the gate when
+// it came.
+__device__ __forceinline__ int sell_enter(unsigned *gate, unsigned ticket, const SellGate &rule)
 {
-    const unsigned all = gridDim.x;
+    const int mine = (int)(ticket & kSellCame);
     unsigned seen = ticket + 1;
-    for (int looks = 0;; ++looks) {
-        if (seen & kSellClosed) return -1;
-        if (seen == all && patience > 0) return (int)ticket;
-        if (looks >= patience) {
-            unsigned expected = seen;
-            if (__hip_atomic_compare_exchange_strong(gate, &expected, seen | kSellClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                groups = 1;
-                return 0;
-            }
+    for (int looks = -rule.patience;; ++looks) {
+        if (seen & kSellClosed) {
+            const int groups = (int)(seen >> kSellRunShift & kSellCame);
+            return mine < groups ? mine | groups << kSellRunShift : -1;
         }
-        seen = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int came = (int)seen;
+        if (came >= (int)gridDim.x && rule.places >= came) return mine | came << kSellRunShift;
+        if (came >= rule.places || (looks >= 0 && (came >= rule.enough || looks * came >= rule.price))) {
+            const unsigned closed = seen | kSellClosed | (unsigned)min(came, rule.places) << kSellRunShift;
+            if (__hip_atomic_compare_exchange_strong(gate, &seen, closed, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) seen = closed;
+        } else seen = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -265,13 +276,13 @@ template <int K>
 __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
     int n, int live, int hubs, int slices, int hub_width, const int32_t *__restrict__ hub_step, const int32_t *__restrict__ hub_col,
     const int4 *__restrict__ slice, const int32_t *__restrict__ col, const int32_t *__restrict__ order,
-    const double *__restrict__ inv_user, double *inv, unsigned long long *exchange, unsigned *gate, int patience, int iters,
+    const double *__restrict__ inv_user, double *inv, unsigned long long *exchange, unsigned *gate, SellGate rule, int iters,
     double alpha, double inv_n, double *__restrict__ r_out)
 {
     constexpr int T = kSellResidentThreads, S = K * T, D = kSellWaveSteps, kHubAhead = 4, kRest = 4;
     extern __shared__ __attribute__((aligned(16))) double s_c[];  // sources [S], of the rows without entries [n - live], 0; those rows' inverse out-degrees [n - live]
     __shared__ double s_mass[T / kWave], s_hub[T / kWave];
-    __shared__ int s_group, s_groups, s_last, s_dangling;
+    __shared__ int s_group, s_last, s_dangling;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int rest = n - live;
     unsigned *left = gate + kTicketStride;
@@ -318,14 +329,13 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
     }
     if (tid == 0) {
         s_c[S + rest] = 0.0;  // what the padding gathers
-        int all = gridDim.x;
-        s_group = sell_enter(gate, ticket, all, patience);
-        s_groups = all;
+        s_group = sell_enter(gate, ticket, rule);
         s_last = 0;
     }
     if (dangling) atomicAdd(&s_dangling, dangling);
     __syncthreads();
-    const int group = __builtin_amdgcn_readfirstlane(s_group), groups = __builtin_amdgcn_readfirstlane(s_groups);
+    const int group = __builtin_amdgcn_readfirstlane(s_group < 0 ? -1 : s_group & (int)kSellCame);
+    const int groups = __builtin_amdgcn_readfirstlane(s_group >> kSellRunShift);
     const auto leave = [&] {  // thread 0, when the work-group reads no slots any more
         s_last = __hip_atomic_fetch_add(left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     };
@@ -828,6 +838,8 @@ void choose_resident(SellRows *sr, int live)
     if (!sr->staged || sr->lds > kSellResidentLds || sr->hubs > kSellResidentBlocks || sr->live_slices > kSellResidentBlocks * (kSellResidentThreads / kWave)) return;
     const int wanted = std::max((int)ceil_div(sr->live_slices, kSellResidentSlices), sr->hubs);
     sr->resident = std::max(1, std::min({wanted, kSellResidentBlocks, sr->live_slices}));  // each of several owns a row
+    const auto rounds = [&](int groups) { return ceil_div(sr->live_slices, groups * (kSellResidentThreads / kWave)) + ceil_div(sr->hubs, groups); };
+    while (sr->rule.enough < sr->resident && rounds(sr->rule.enough) > rounds(sr->resident)) ++sr->rule.enough;
 }
 
 SellShape shape_of(const SellRows &sr)
@@ -994,9 +1006,11 @@ int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t s)
 
 int sell_run(const SellRows &sr, const double *inv_user, int iters, double alpha, double *rank_out, hipStream_t s)
 {
+    SellGate rule = sr.rule;
+    rule.price = (int)std::min<int64_t>((int64_t)iters * kSellLooksPerRound * (ceil_div(sr.live_slices, kSellResidentThreads / kWave) + sr.hubs), kSellMostLooks);
     sell_resident_of(sr)<<<sr.resident, kSellResidentThreads, sr.lds, s>>>(
         (int)sr.n, sr.live, sr.hubs, sr.live_slices, sr.threads, sr.hub_step, sr.hub_col, sr.slice, sr.col, sr.order, inv_user, sr.inv,
-        sr.exchange, sr.gate, sr.patience, iters, alpha, 1.0 / (double)sr.n, rank_out);
+        sr.exchange, sr.gate, rule, iters, alpha, 1.0 / (double)sr.n, rank_out);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
 }
