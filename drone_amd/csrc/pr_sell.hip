@@ -829,6 +829,7 @@ SellResident sell_resident_of(const SellRows &sr)
 // Whether runs are one launch, and of how many work-groups.
 void choose_resident(SellRows *sr, int live)
 {
+    if (sr->n + sr->nnz > kSellWideItems) return;  // sell_resident_kernel keeps kSellWaveSteps steps of a slice; wide plans have longer ones
     sr->live = live;
     sr->live_slices = sr->slice_begin[kSellClasses - 1] + (int)ceil_div(live - sr->row_begin[kSellClasses - 1], kWave);
     sr->staged = 0;

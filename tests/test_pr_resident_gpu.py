@@ -38,6 +38,7 @@ def _close(got, ref, rp, iters):
     (8192, [], 60), (8200, [], 60),                          # as many slices as wavefronts, and one more
     (12288, [768] * 5, 11), (12289, [768] * 5, 11),          # as many rows as fit
     (19455, [9] * 1024, 0), (14000, [12] * 6000, 0),         # most rows without entries: too many of them to fit, and not
+    (1000, [], 768), (1650, [], 768), (1400, [], 900),       # slices as long as the kernel keeps, and matrices that have longer ones
 ])
 def test_runs_in_one_launch(oracle, n, lengths, filler):
     rp, ci, inv = _matrix(n, lengths, filler)
