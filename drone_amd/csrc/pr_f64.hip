@@ -245,7 +245,7 @@ extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
 extern "C" int drone_pr_plan_gate(drone_pr_plan *p, int patience, int places)
 {
     clear_error();
-    DRONE_REQUIRE(p != nullptr && patience >= 0 && places >= 1, "gate");
+    DRONE_REQUIRE(p != nullptr && patience >= -1 && places >= 1, "gate");
     p->sr.rule.patience = patience;
     p->sr.rule.places = places;
     return DRONE_OK;

@@ -42,7 +42,8 @@ constexpr int kSellHubDepth = 16, kSellWaveSteps = 12, kSellWaveStepsWide = 16;
 constexpr int kSellDepthF32 = 16, kSellWaveStepsF32 = 32;  // the same of float rows
 constexpr int kSellHot = 20000;      // sources that a work-group of sell_iterate_hot_kernel keeps in LDS: 160,000 of 163,840 bytes
 
-// When the work-groups of a run in one launch stop waiting for the others (sell_enter): not before `patience` looks, and when `places` have come.
+// When the work-groups of a run in one launch stop waiting for the others (sell_enter): not before `patience` looks, and when `places` have
+// come.  A negative patience is that of a test: none for the others' sources either.
 struct SellGate {
     int patience = 64, places = INT_MAX;
     int enough = 1, price = 0;  // work-groups as good as all, and looks that the run is worth to one: of the run
@@ -70,7 +71,8 @@ struct SellRows {
     size_t lds = 0;                  // bytes of its sources in LDS
     int live = 0, live_slices = 0;   // rows with entries, and the slices that have one of them
     unsigned long long *exchange = nullptr;  // device [4 n]: its sources on their way, kSellNone between runs
-    unsigned *gate = nullptr;        // device [2 * kTicketStride]: who has come and who has left, 0 between runs
+    unsigned *gate = nullptr;        // device [3 * kTicketStride]: who has come and who has left, 0 between runs; `failed`
+    int *failed = nullptr;           // pinned: a work-group of a run has given up waiting for another, and no call has reported it yet
     DeviceArena arena;               // everything above
     DeviceArena entries;             // hub_col and col, whose sizes are known last
 };

@@ -187,13 +187,14 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
 //
 // The work-groups wait for each other, so all that take part must have a place on the chip before any starts.  Each reports at a gate; one
 // that has looked in vain for long enough closes it, those who have come by then do the run, and later ones go; every sum has the same order
-// then.  (Behind the gate all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long goes on with the
-// NaN.)  Long enough: `patience` looks where who is there takes no more rounds of slices and hub rows than all would; else also as many as
-// the run would take with them, at kSellLooksPerRound a round (1.2 us on an idle chip, four times that beside a stream of memory-bound
-// kernels), so that the wait at most doubles it.  20 / 3 iterations beside a stream that adds to 1 GiB of floats, us, a launch per iteration
-// / one work-group behind every closed gate / this: 4 K vertices and 53 K entries 289 / 111 / 112 and 67 / 45 / 47, 12 K and 108 K 313 / 3,300 / 250
-// and 70 / 557 / 175-260, 12 K and 419 K 381 / 12,700 / 250-315 and 82 / 1,930 / 250; beside bf16 products of 8,192 rows, whose work-groups fill
-// the chip for 0.7 ms each, 16,000 / 80-5,300 / 780.  What the short runs of more than 10 K rows lose are the places: 123 registers a lane ask for an
+// then.  (Behind the gate all are on the chip, and every wait ends.  kSellPolls is seconds; a lane that has waited for so long says so and goes
+// on with the NaN.  The last work-group to leave then clears every set, and the plan's next run reports it instead of running.)
+// Long enough: `patience` looks where who is there takes no more rounds of slices and hub rows than all would; else also as many as the run
+// would take with them, at kSellLooksPerRound a round (1.2 us on an idle chip, four times that beside a stream of memory-bound kernels), so
+// that the wait at most doubles it.  20 / 3 iterations beside a stream that adds to 1 GiB of floats, us, a launch per iteration / one
+// work-group behind every closed gate / this: 4 K vertices and 53 K entries 289 / 111 / 112 and 67 / 45 / 47, 12 K and 108 K 313 / 3,300 / 250 and 70 /
+// 557 / 130-260, 12 K and 419 K 381 / 12,700 / 250-315 and 82 / 1,930 / 130-280; beside bf16 products of 8,192 rows, whose work-groups fill the
+// chip for 0.7 ms each, 16,000 / 80-5,300 / 780.  What the short runs of more than 10 K rows lose are the places: 124 registers a lane ask for an
 // empty CU (with 96, at the price of 27 spilled, 71 / 80, but 20 iterations of an idle chip 78 -> 104 and 91 -> 132).
 constexpr int kSellResidentThreads = 1024;
 constexpr unsigned long long kSellNone = 0x7ffc5e1100a1b2c3ull, kSellNan = 0x7ff8000000000000ull;
@@ -202,6 +203,7 @@ constexpr unsigned kSellClosed = 1u << 31, kSellCame = 0xff;
 constexpr int kSellRunShift = 8, kSellLooksPerRound = 2, kSellMostLooks = 1 << 22;
 static_assert(kSellResidentBlocks <= (int)kSellCame, "a byte each");
 constexpr int kSellPolls = 1 << 22;
+constexpr unsigned kSellGaveUp = 1u << 16;  // times those who gave up, beside the count of those who have left
 constexpr int kSellWaitStores = 0x0f70;  // s_waitcnt vmcnt(0)
 
 __device__ __forceinline__ void slot_store(unsigned long long *p, unsigned long long v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -209,12 +211,13 @@ __device__ __forceinline__ unsigned long long slot_load(const unsigned long long
 
 __device__ __forceinline__ bool slot_is_none(unsigned long long v) { return (unsigned)(v >> 32) == (unsigned)(kSellNone >> 32); }
 
-// Four sets of `slots` slots of which `used` are.
-__global__ void sell_slots_kernel(int slots, int used, unsigned long long *__restrict__ exchange, unsigned *__restrict__ gate)
+// Four sets of `slots` slots of which `used` are, the gate, and behind its counters where the last work-group reports.
+__global__ void sell_slots_kernel(int slots, int used, unsigned long long *__restrict__ exchange, unsigned *__restrict__ gate, int *failed)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 4 * slots; i += gridDim.x * blockDim.x)
         exchange[i] = i % slots < used ? kSellNone : 0;
     if (blockIdx.x == 0 && threadIdx.x < 2 * kTicketStride) gate[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *reinterpret_cast<int **>(gate + 2 * kTicketStride) = failed;
 }
 
 // Through the gate: this work-group's number in the run and, from kSellRunShift on, how many do it, or -1 to leave.  ticket: the gate when
@@ -283,6 +286,7 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
     extern __shared__ __attribute__((aligned(16))) double s_c[];  // sources [S], of the rows without entries [n - live], 0; those rows' inverse out-degrees [n - live]
     __shared__ double s_mass[T / kWave], s_hub[T / kWave];
     __shared__ int s_group, s_last, s_dangling;
+    __shared__ unsigned s_gave_up;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int rest = n - live;
     unsigned *left = gate + kTicketStride;
@@ -331,19 +335,23 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
         s_c[S + rest] = 0.0;  // what the padding gathers
         s_group = sell_enter(gate, ticket, rule);
         s_last = 0;
+        s_gave_up = 0;
     }
     if (dangling) atomicAdd(&s_dangling, dangling);
     __syncthreads();
     const int group = __builtin_amdgcn_readfirstlane(s_group < 0 ? -1 : s_group & (int)kSellCame);
     const int groups = __builtin_amdgcn_readfirstlane(s_group >> kSellRunShift);
     const auto leave = [&] {  // thread 0, when the work-group reads no slots any more
-        s_last = __hip_atomic_fetch_add(left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        const unsigned mine = 1 + s_gave_up, before = __hip_atomic_fetch_add(left, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), all = before + mine;
+        s_last = (all & (kSellGaveUp - 1)) != gridDim.x ? 0 : all < kSellGaveUp ? 1 : 4;  // sets to clear
     };
     const auto close = [&] {
         if (!s_last) return;
         if (iters > 1)
-            for (int i = tid; i < live; i += T) slot_store(exchange + (size_t)((iters - 1) & 3) * S + i, kSellNone);
+            for (int set = 0; set < s_last; ++set)
+                for (int i = tid; i < live; i += T) slot_store(exchange + (size_t)((iters - 1 + set) & 3) * S + i, kSellNone);
         if (tid == 0) {
+            if (s_last > 1) __hip_atomic_store(*reinterpret_cast<int **>(gate + 2 * kTicketStride), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(gate, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(left, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -393,7 +401,8 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
     }
     // A rank is base + alpha * sum, and base is the same everywhere: a slot holds alpha * sum, times the
     // inverse out-degree where that is not 0, and base, which takes a reduction, is added by the readers and not waited for.
-    bool given_up = false;
+    bool given_up = rule.patience < 0;
+    if (given_up) s_gave_up = kSellGaveUp;
     double base = inv_n, mass = 0.0;  // of the ranks that the iteration starts from: base, and the dangling mass beyond base
     for (int it = 0; it < iters; ++it) {
         unsigned long long *out = exchange + (size_t)((it + 1) & 3) * S, *done = exchange + (size_t)((it + 3) & 3) * S;
@@ -410,6 +419,7 @@ __global__ __launch_bounds__(kSellResidentThreads) void sell_resident_kernel(
                 for (int k = 0; k < K; ++k) missing |= slot_is_none(v[k]);
                 if (!missing) break;
                 given_up = polls >= kSellPolls;
+                if (given_up) s_gave_up = kSellGaveUp;
 #pragma unroll
                 for (int k = 0; k < K; ++k)
                     if (slot_is_none(v[k])) v[k] = slot_load(in + k * T);
@@ -955,11 +965,11 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
         const int slots = sr->staged * kSellResidentThreads;
         if (sr->resident) {
             sr->entries.want(&sr->exchange, 4 * (size_t)slots);
-            sr->entries.want(&sr->gate, 2 * kTicketStride);
+            sr->entries.want(&sr->gate, 3 * kTicketStride);
         }
         DRONE_HIP_TRY(sr->entries.commit());
         if (sr->resident) {
-            sell_slots_kernel<<<64, 256, 0, s>>>(slots, sr->live, sr->exchange, sr->gate);
+            sell_slots_kernel<<<64, 256, 0, s>>>(slots, sr->live, sr->exchange, sr->gate, h);
             // the limit belongs to the kernel, which plans of other sizes share
             DRONE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sell_resident_of(*sr)), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSellResidentLds));
         }
@@ -967,6 +977,11 @@ int sell_build(SellRows *sr, int64_t n, int64_t nnz, const Off *row_ptr, const i
             sh, sr->threads, sr->order, row_ptr, col, new_id, sr->hub_step, slice_step, sr->slice, sr->hub_col, sr->col, sr->hot);
         DRONE_HIP_TRY(hipGetLastError());
         DRONE_HIP_TRY(hipStreamSynchronize(s));  // the temporaries go next
+        if (sr->resident) {
+            sr->failed = h;
+            *sr->failed = 0;
+            h = nullptr;
+        }
         return DRONE_OK;
     };
     const int rc = body();
@@ -994,6 +1009,7 @@ void sell_destroy(SellRows *sr)
 {
     sr->arena.release();
     sr->entries.release();
+    if (sr->failed) (void)hipHostFree(sr->failed);
     *sr = SellRows{};
 }
 
@@ -1007,6 +1023,11 @@ int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t s)
 
 int sell_run(const SellRows &sr, const double *inv_user, int iters, double alpha, double *rank_out, hipStream_t s)
 {
+    if (__atomic_load_n(sr.failed, __ATOMIC_RELAXED)) {
+        *sr.failed = 0;
+        set_error(DRONE_ERR_HIP, "an earlier run of this plan waited in vain for one of its work-groups: its ranks are not valid");
+        return DRONE_ERR_HIP;
+    }
     SellGate rule = sr.rule;
     rule.price = (int)std::min<int64_t>((int64_t)iters * kSellLooksPerRound * (ceil_div(sr.live_slices, kSellResidentThreads / kWave) + sr.hubs), kSellMostLooks);
     sell_resident_of(sr)<<<sr.resident, kSellResidentThreads, sr.lds, s>>>(

@@ -174,7 +174,8 @@ int drone_pr_plan_destroy(drone_pr_plan *plan);
 /* Runs `iters` iterations from r_0 = 1/N and writes r_iters to rank_out [n] (device).
  * Asynchronous on `stream`; allocates nothing and launches kernels only (no copies, clears or waits), so a run can be
  * recorded into a HIP graph and replayed while profiling (drone_pr_profile_enable) is off.  A plan is for one run at
- * a time. */
+ * a time.  (A run of a small matrix whose work-groups lost each other for seconds, which nothing known can cause, is reported by the
+ * plan's next run, in its place.) */
 int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_out,
                      drone_stream_t stream);
 /* Per-iteration timing with HIP events on the launch stream.  When enabled, every iteration inside

@@ -66,6 +66,25 @@ def test_as_many_work_groups_as_found_a_place(oracle, n, lengths, filler):
     plan.close()
 
 
+@pytest.mark.parametrize("iters", [3, 4, 5, 6, 9])
+def test_a_wait_in_vain_is_reported_and_leaves_the_plan_clean(iters):
+    """Work-groups that wait for nothing: the next run says so, and those after it find no value of that run."""
+    import torch
+    from drone_amd._lib import check, lib
+    plan = _plan(*_matrix(6000, [800] * 64, 12))
+    want = plan.run(0.85, iters)
+    for _ in range(3):
+        check(lib().drone_pr_plan_gate(plan.h, -1, 64))  # the 64 of its hub rows
+        plan.run(0.85, iters)
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="waited in vain"):
+            plan.run(0.85, iters)
+        check(lib().drone_pr_plan_gate(plan.h, 64, 64))
+        for _ in range(3):
+            assert torch.equal(plan.run(0.85, iters), want)
+    plan.close()
+
+
 def test_a_busy_chip_costs_places_and_not_the_run():
     """Beside a stream that keeps every CU busy some work-groups are late, and the others do not leave the run to one of them: it takes
     less than a third of what it takes one (0.3 of 8.6 ms where measured)."""
