@@ -6,6 +6,8 @@
 // The aggregation kernel gathers c_{k-1}, and its row epilogue writes c_k (and r_k on the last
 // iteration) and accumulates d_k, so one iteration touches: row_ptr 8N, col_idx 4E, gather source 8N,
 // inv_outdeg 8N, c_k 8N  =  4E + 32N bytes.
+#include <algorithm>
+
 #include "pr_rowblock.h"
 #include "pr_sell.h"
 #include "relabel.h"
@@ -135,6 +137,7 @@ struct drone_pr_plan {
     // profiling
     int prof_cap = 0, prof_n = 0;
     hipEvent_t *ev0 = nullptr, *ev1 = nullptr;
+    int *prof_iters = nullptr;  // iterations between the two
 };
 
 extern "C" int64_t drone_pr_bytes_per_iteration(int64_t n, int64_t nnz) { return 4 * nnz + 32 * n + 8; }
@@ -237,6 +240,7 @@ extern "C" int drone_pr_plan_destroy(drone_pr_plan *p)
     }
     delete[] p->ev0;
     delete[] p->ev1;
+    delete[] p->prof_iters;
     delete p;
     return DRONE_OK;
 }
@@ -261,11 +265,15 @@ extern "C" int drone_pr_profile_enable(drone_pr_plan *p, int max_launches)
     }
     delete[] p->ev0;
     delete[] p->ev1;
+    delete[] p->prof_iters;
     p->ev0 = p->ev1 = nullptr;
+    p->prof_iters = nullptr;
     p->prof_cap = p->prof_n = 0;
     if (max_launches == 0) return DRONE_OK;
     p->ev0 = new hipEvent_t[max_launches];
     p->ev1 = new hipEvent_t[max_launches];
+    p->prof_iters = new int[max_launches];
+    std::fill_n(p->prof_iters, max_launches, 1);
     for (int i = 0; i < max_launches; ++i) {
         DRONE_HIP_TRY(hipEventCreate(&p->ev0[i]));
         DRONE_HIP_TRY(hipEventCreate(&p->ev1[i]));
@@ -280,16 +288,19 @@ extern "C" int drone_pr_profile_read(drone_pr_plan *p, int *launches, double *me
     clear_error();
     DRONE_REQUIRE(p != nullptr, "plan");
     double sum = 0.0, mn = 1e300, mx = 0.0;
+    int iters = 0;
     for (int i = 0; i < p->prof_n; ++i) {
         float ms = 0.0f;
         DRONE_HIP_TRY(hipEventSynchronize(p->ev1[i]));
         DRONE_HIP_TRY(hipEventElapsedTime(&ms, p->ev0[i], p->ev1[i]));
         sum += ms;
-        if (ms < mn) mn = ms;
-        if (ms > mx) mx = ms;
+        iters += p->prof_iters[i];
+        mn = std::min(mn, (double)ms / p->prof_iters[i]);
+        mx = std::max(mx, (double)ms / p->prof_iters[i]);
+        p->prof_iters[i] = 1;
     }
-    if (launches) *launches = p->prof_n;
-    if (mean_ms) *mean_ms = p->prof_n ? sum / p->prof_n : 0.0;
+    if (launches) *launches = iters;
+    if (mean_ms) *mean_ms = iters ? sum / iters : 0.0;
     if (min_ms) *min_ms = p->prof_n ? mn : 0.0;
     if (max_ms) *max_ms = mx;
     p->prof_n = 0;
@@ -312,7 +323,16 @@ extern "C" int drone_pr_run_f64(drone_pr_plan *p, double alpha, int iters, doubl
     }
     // the caller may have refreshed inv_outdeg since the plan was made: re-read it every run (8N bytes)
     if (p->sell) {
-        if (p->sr.resident && iters >= kSellResidentIters && p->prof_n >= p->prof_cap) return sell_run(p->sr, p->inv_user, iters, alpha, rank_out, s);
+        if (p->sr.resident && iters >= kSellResidentIters) {  // one launch, one pair of events
+            const bool prof = p->prof_n < p->prof_cap;
+            if (prof) DRONE_HIP_TRY(hipEventRecord(p->ev0[p->prof_n], s));
+            const int rc = sell_run(p->sr, p->inv_user, iters, alpha, rank_out, s);
+            if (prof && rc == DRONE_OK) {
+                DRONE_HIP_TRY(hipEventRecord(p->ev1[p->prof_n], s));
+                p->prof_iters[p->prof_n++] = iters;
+            }
+            return rc;
+        }
         int rc = sell_begin(p->sr, p->inv_user, s);
         for (int it = 0; it < iters && rc == DRONE_OK; ++it) {
             const bool prof = p->prof_n < p->prof_cap;

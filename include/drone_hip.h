@@ -158,7 +158,7 @@ int drone_pr_plan_create(drone_pr_plan **plan, int64_t n, int64_t nnz, const int
  * (fastest; row sums are added in LDS in no fixed order, so the last bits may differ between runs, as
  * with the reference's float atomics).  DRONE_PR_DETERMINISTIC selects the merge-path kernel, whose
  * results are bitwise reproducible.  Small matrices (rows + entries up to 9 Mi) get a layout of their own in
- * either mode, one launch per iteration and bitwise reproducible. */
+ * either mode, bitwise reproducible, with one launch per iteration or, of up to about 12,000 rows with entries, per run. */
 #define DRONE_PR_DETERMINISTIC 1
 /* Tuning overrides of the default mode.  Row blocks of a large matrix (about 50 M entries and more) are shared by up
  * to four work-groups, which then find more entries per cache line of the gather source; small matrices keep one
@@ -181,7 +181,9 @@ int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_
 /* Per-iteration timing with HIP events on the launch stream.  When enabled, every iteration inside
  * drone_pr_run_f64 - the aggregation kernel, the merge of shared blocks, the row fix-up and the dangling-mass
  * reduction, i.e. everything the algorithmic bytes of one iteration pay for - is bracketed by an event pair (at
- * most `max_launches` are kept).  drone_pr_profile_read synchronises the events and returns the mean duration. */
+ * most `max_launches` are kept); a run that is one launch (three iterations or more of a small matrix) by one pair, an
+ * iteration's duration being its share.  drone_pr_profile_read synchronises the events and returns the number of
+ * iterations and their mean duration. */
 int drone_pr_profile_enable(drone_pr_plan *plan, int max_launches);
 int drone_pr_profile_read(drone_pr_plan *plan, int *launches, double *mean_ms, double *min_ms,
                           double *max_ms);

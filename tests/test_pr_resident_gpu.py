@@ -120,19 +120,21 @@ def test_a_busy_chip_costs_places_and_not_the_run():
 
 
 def test_infinite_degrees_stay_in_the_ranks():
-    """A NaN and an infinity among the inverse out-degrees reach the ranks that they reach in a launch per iteration."""
+    """A NaN and an infinity among the inverse out-degrees reach the ranks that they reach by way of row blocks."""
+    import torch
+    from drone_amd.pagerank import PullPlanF64
     rp, ci, inv = _matrix(500, [], 2)
     inv[3], inv[4] = np.nan, np.inf
     plan = _plan(rp, ci, inv)
+    blocks = PullPlanF64(*(torch.from_numpy(a).cuda() for a in (rp, ci, inv)), shared_blocks=False)
     for iters in (1, 3):
         got = plan.run(0.85, iters).cpu().numpy()
-        plan.profile_enable(16)
-        want = plan.run(0.85, iters).cpu().numpy()
-        plan.profile_enable(0)
+        want = blocks.run(0.85, iters).cpu().numpy()
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
         there = np.isfinite(want)
         assert (iters > 1 or there.any()) and np.allclose(got[there], want[there], rtol=1e-13, atol=0)
     plan.close()
+    blocks.close()
 
 
 def test_replays_of_a_recorded_run():
@@ -191,3 +193,27 @@ def test_plans_that_share_a_kernel(oracle):
         _close(plan.run(0.85, 6).cpu().numpy(), want, rp, 6)
     for plan, _, _ in plans:
         plan.close()
+
+
+@pytest.mark.parametrize("iters", [2, 3, 20])
+def test_profiled_runs_are_the_same_runs(iters):
+    import torch
+    plan = _plan(*_matrix(4097, [800] * 30, 11))
+    want = plan.run(0.85, iters)
+    plan.profile_enable(64)
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    begin.record()
+    for _ in range(3):
+        assert torch.equal(plan.run(0.85, iters), want)
+    end.record()
+    torch.cuda.synchronize()
+    prof = plan.profile_read()
+    assert prof["launches"] == 3 * iters and 0 < prof["min_ms"] <= prof["mean_ms"] <= prof["max_ms"]
+    assert prof["mean_ms"] * 3 * iters <= begin.elapsed_time(end)
+    assert plan.profile_read()["launches"] == 0
+    plan.profile_enable(1)                               # fewer pairs of events than launches
+    for _ in range(2):
+        assert torch.equal(plan.run(0.85, iters), want)
+    assert plan.profile_read()["launches"] == (iters if iters >= 3 else 1)
+    plan.profile_enable(0)
+    plan.close()
