@@ -12,6 +12,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
@@ -97,9 +98,25 @@ struct Variable {
     }
 };
 
+// Which object it is: one made later has another number, also where it lives at the address of one that is gone.
+class Serial {
+    uint64_t number;
+    static uint64_t next()
+    {
+        static std::atomic<uint64_t> last{0};
+        return ++last;
+    }
+public:
+    Serial() : number(next()) {}
+    Serial(const Serial &) : number(next()) {}
+    Serial &operator=(const Serial &) { return *this; }
+    operator uint64_t() const { return number; }
+};
+
 // cuda_module.cuh:31-37
 class Module {
 public:
+    Serial serial;
     virtual void forward(bool training) = 0;
     virtual void backward() = 0;
     virtual ~Module() {}
@@ -419,6 +436,7 @@ struct AdamParams {
 
 class Optimizer {
 public:
+    Serial serial;
     virtual void step() = 0;
     virtual ~Optimizer() {}
 };
@@ -625,7 +643,7 @@ public:
         modules.emplace_back(graphsum2);
         ce = new CrossEntropyLoss(output, truth, p.output_dim, "CrossEntropy", s);
         modules.emplace_back(ce);
-        for (auto &m : modules) built.push_back(m.get());
+        for (auto &m : modules) built.push_back(m->serial);
         // Sums that wait for the step, up to 2 MB of them: more take a millisecond to allocate and no step gains more than 6 us by it
         // (or loses, 44 MB of them, which come back from memory: 232,965-vertex step 7,588 -> 7,628 us).
         constexpr int64_t kMostSums = 1 << 19;
@@ -657,7 +675,7 @@ public:
         } else {
             optimizer.reset(new SGD({layer1_weight, layer2_weight}, p.learning_rate, s));
         }
-        built_optimizer = optimizer.get();
+        built_optimizer = optimizer->serial;
         DRONE_GCN_HIP(hipDeviceSynchronize());
     }
     GCN(const GCN &) = delete;
@@ -748,7 +766,7 @@ private:
     // backward() and the step.  Nobody looks at the weight gradients in between - unless the program has changed what runs.
     void backward_and_step()
     {
-        const bool keep = as_built() && optimizer.get() == built_optimizer;
+        const bool keep = as_built() && optimizer->serial == built_optimizer;
         for (Variable *w : {layer1_weight, layer2_weight}) w->keep_sums = keep && w->sums_floats > 0;
         backward();
         for (Variable *w : {layer1_weight, layer2_weight}) w->keep_sums = false;
@@ -758,11 +776,11 @@ private:
     {
         if (modules.size() != built.size()) return false;
         for (size_t i = 0; i < built.size(); ++i)
-            if (modules[i].get() != built[i]) return false;
+            if (modules[i]->serial != built[i]) return false;
         return true;
     }
-    std::vector<const Module *> built;
-    const Optimizer *built_optimizer = nullptr;
+    std::vector<uint64_t> built;   // serial numbers
+    uint64_t built_optimizer = 0;
     void settle_truth()  // behind a wait for the stream
     {
         if (!truth_pending) return;

@@ -157,11 +157,115 @@ int main()
 """
 
 
-def _compile(tmp_path, *extra):
+# Programs that put their own modules and optimisers into a model, also at the addresses of the model's own.
+REPLACED = r"""
+#include <cmath>
+#include <new>
+
+#include "drone_gcn_modules.hpp"
+
+using namespace drone_gcn_mod;
+
+template <typename T> T *up(const std::vector<T> &h)
+{
+    T *d = nullptr;
+    DRONE_GCN_HIP(hipMalloc(&d, sizeof(T) * h.size()));
+    DRONE_GCN_HIP(hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
+    return d;
+}
+std::vector<float> down(const Variable *v, const float *d)
+{
+    std::vector<float> h((size_t)v->rows * v->ld);
+    DRONE_GCN_HIP(hipDeviceSynchronize());
+    DRONE_GCN_HIP(hipMemcpy(h.data(), d, sizeof(float) * h.size(), hipMemcpyDeviceToHost));
+    return h;
+}
+int failed = 0;
+#define CHECK(cond) do { if (!(cond)) { printf("line %d: %s\n", __LINE__, #cond); failed = 1; } } while (0)
+
+// Reads both weights' gradients, and steps by a rate of 0.
+std::vector<float> seen1, seen2;
+struct Reader : Optimizer {
+    Variable *w1, *w2;
+    char as_large_as_the_models_own[sizeof(SGD) - sizeof(Optimizer) - 2 * sizeof(Variable *)];
+    Reader(Variable *a, Variable *b) : w1(a), w2(b) {}
+    void step() override { seen1 = down(w1, w1->grad); seen2 = down(w2, w2->grad); }
+};
+static_assert(sizeof(Reader) == sizeof(SGD), "finds a place where one was");
+// The same in the backward pass, in front of layer 1.
+struct Last : Module {
+    Variable *w2;
+    explicit Last(Variable *w) : w2(w) {}
+    void forward(bool) override {}
+    void backward() override { seen2 = down(w2, w2->grad); }
+};
+
+int main()
+{
+    const int N = 3000, fin = 64, hid = 32, cls = 7;
+    std::vector<int> rp(N + 1), ci, deg(N, 3), label(N), split(N);
+    for (int v = 0; v < N; ++v) {
+        rp[v] = (int)ci.size();
+        for (int d : {0, 1, 7}) ci.push_back((v + d) % N);
+        label[v] = v * 5 % cls;
+        split[v] = v % 3 ? 1 : 2;
+    }
+    rp[N] = (int)ci.size();
+    std::vector<float> X(N * fin), W1(fin * hid), W2(hid * cls);
+    for (size_t i = 0; i < X.size(); ++i) X[i] = std::sin(0.37f * i);
+    for (size_t i = 0; i < W1.size(); ++i) W1[i] = 0.3f * std::cos(0.91f * i);
+    for (size_t i = 0; i < W2.size(); ++i) W2[i] = 0.3f * std::sin(1.7f * i);
+    GCNParams p;
+    p.localVertexSize = N; p.input_dim = fin; p.hidden_dim = hid; p.output_dim = cls;
+    p.use_adam = false; p.learning_rate = 0.0f;
+    GCN m(p, (int64_t)ci.size(), up(rp), up(ci), up(deg), up(deg), up(X), fin, up(label), up(split), up(W1), up(W2), nullptr);
+    Variable *const w1 = m.layer1_weight, *const w2 = m.layer2_weight;
+    CHECK(w1->sums_floats > 0 && w2->sums_floats > 0);  // or nothing here is to be seen
+
+    m.set_truth(1);
+    m.forward(true);
+    m.backward();
+    const std::vector<float> g1 = down(w1, w1->grad), g2 = down(w2, w2->grad);
+    const auto forget = [&] {
+        for (Variable *w : {w1, w2}) DRONE_GCN_HIP(hipMemset(w->grad, 0, sizeof(float) * (size_t)w->rows * w->ld));
+        seen1.clear();
+        seen2.clear();
+    };
+    // as built: the step leaves the gradients that backward() alone leaves
+    for (int way = 0; way < 2; ++way) {
+        forget();
+        if (way) m.train_epoch(); else m.train_step_async();
+        CHECK(down(w1, w1->grad) == g1 && down(w2, w2->grad) == g2);
+    }
+    // a module of the program's that reads a gradient during the backward pass
+    forget();
+    m.modules.insert(m.modules.begin(), std::unique_ptr<Module>(new Last(w2)));
+    m.train_epoch();
+    CHECK(seen2 == g2 && down(w1, w1->grad) == g1);
+    m.modules.erase(m.modules.begin());
+    // optimisers of the program's, one after the other, until one has the place of the model's own
+    const void *const place = m.optimizer.get();
+    bool taken = false;
+    for (int i = 0; i < 100 && !taken; ++i) {
+        m.optimizer.reset(new Reader(w1, w2));
+        taken = m.optimizer.get() == place;
+        forget();
+        m.train_step_async();
+        CHECK(seen1 == g1 && seen2 == g2);
+    }
+    CHECK(taken);
+    if (!failed) printf("all as expected\n");
+    fflush(stdout);
+    return failed;
+}
+"""
+
+
+def _compile(tmp_path, *extra, program=PROGRAM):
     cxx = shutil.which("g++") or shutil.which("c++")
     assert cxx, "no C++ compiler"
     src = tmp_path / "modules.cpp"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     subprocess.check_call([cxx, "-std=c++17", "-O1", "-Wall", "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROOT, "include"),
                            "-isystem", os.path.join(ROCM, "include"), str(src), *extra])
 
@@ -170,10 +274,24 @@ def test_module_header_keeps_what_programs_use(tmp_path):
     _compile(tmp_path, "-fsyntax-only")
 
 
-@pytest.mark.gpu
-def test_state_behind_the_model(tmp_path):
+def _run(tmp_path, program):
     exe, lib = str(tmp_path / "modules"), _lib.library_path()
     _compile(tmp_path, "-o", exe, lib, "-Wl,-rpath," + os.path.dirname(lib), "-L" + os.path.join(ROCM, "lib"),
-             "-Wl,-rpath," + os.path.join(ROCM, "lib"), "-lamdhip64")
+             "-Wl,-rpath," + os.path.join(ROCM, "lib"), "-lamdhip64", program=program)
     done = subprocess.run([exe], capture_output=True, text=True, timeout=100)
     assert done.returncode == 0 and "all as expected" in done.stdout, done.stdout + done.stderr
+
+
+@pytest.mark.gpu
+def test_state_behind_the_model(tmp_path):
+    _run(tmp_path, PROGRAM)
+
+
+def test_programs_may_replace_what_a_model_has_built_compile(tmp_path):
+    _compile(tmp_path, "-fsyntax-only", program=REPLACED)
+
+
+@pytest.mark.gpu
+def test_programs_may_replace_what_a_model_has_built(tmp_path):
+    """The gradients are there for a module or an optimiser that is not the model's own, also where it lives at its address."""
+    _run(tmp_path, REPLACED)
