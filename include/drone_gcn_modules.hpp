@@ -98,7 +98,8 @@ struct Variable {
     }
 };
 
-// Which object it is: one made later has another number, also where it lives at the address of one that is gone.
+// Which object it is: one made later has another number, also where it lives at the address of one that is gone, and so has one that
+// was assigned to: an optimiser that took over another's variables no longer steps the model's.
 class Serial {
     uint64_t number;
     static uint64_t next()
@@ -109,7 +110,11 @@ class Serial {
 public:
     Serial() : number(next()) {}
     Serial(const Serial &) : number(next()) {}
-    Serial &operator=(const Serial &) { return *this; }
+    Serial &operator=(const Serial &)
+    {
+        number = next();
+        return *this;
+    }
     operator uint64_t() const { return number; }
 };
 

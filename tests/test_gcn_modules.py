@@ -243,6 +243,11 @@ int main()
     m.train_epoch();
     CHECK(seen2 == g2 && down(w1, w1->grad) == g1);
     m.modules.erase(m.modules.begin());
+    // another optimiser's variables in the model's own: it steps layer 1 alone, and the gradient of layer 2 is there for the program
+    forget();
+    static_cast<SGD &>(*m.optimizer) = SGD({w1}, 0.0f, nullptr);
+    m.train_epoch();
+    CHECK(down(w1, w1->grad) == g1 && down(w2, w2->grad) == g2);
     // optimisers of the program's, one after the other, until one has the place of the model's own
     const void *const place = m.optimizer.get();
     bool taken = false;
