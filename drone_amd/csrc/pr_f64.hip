@@ -323,7 +323,7 @@ extern "C" int drone_pr_run_f64(drone_pr_plan *p, double alpha, int iters, doubl
     }
     // the caller may have refreshed inv_outdeg since the plan was made: re-read it every run (8N bytes)
     if (p->sell) {
-        if (p->sr.resident && iters >= kSellResidentIters) {  // one launch, one pair of events
+        if (p->sr.resident && iters >= p->sr.resident_iters) {  // one launch, one pair of events
             const bool prof = p->prof_n < p->prof_cap;
             if (prof) DRONE_HIP_TRY(hipEventRecord(p->ev0[p->prof_n], s));
             const int rc = sell_run(p->sr, p->inv_user, iters, alpha, rank_out, s);

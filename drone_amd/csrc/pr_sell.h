@@ -67,6 +67,7 @@ struct SellRows {
     int init_blocks = 0;
     SellGate rule;                   // of sell_resident_kernel
     int resident = 0;                // work-groups of sell_resident_kernel, or 0: a launch per iteration
+    int resident_iters = 0;          // iterations of the shortest run that it does
     int staged = 0;                  // slots that a lane of it brings into LDS
     size_t lds = 0;                  // bytes of its sources in LDS
     int live = 0, live_slices = 0;   // rows with entries, and the slices that have one of them
@@ -94,9 +95,13 @@ void sell_destroy(SellRows *sr);
 // its dangling mass; sell_iterate is one iteration (it = 0, 1, ...), the last of which passes rank_out.
 int sell_begin(const SellRows &sr, const double *inv_user, hipStream_t stream);
 int sell_iterate(const SellRows &sr, int it, double alpha, double *rank_out, hipStream_t stream);
-// A whole run of iters >= 1 in one launch, where sr.resident is not 0.  Worth it from kSellResidentIters on: entering costs what two launches
-// do (4 K vertices and 53 K entries, us for 1, 2, 3 and 20 iterations: 9.3, 11.9, 13.7, 48 instead of 7.2, 11.8, 16.6, 86).
-constexpr int kSellResidentIters = 3;
+// A whole run of iters >= 1 in one launch, where sr.resident is not 0.  Worth it from sr.resident_iters on: entering costs what two launches
+// do (4 K vertices and 53 K entries, us for 1, 2, 3 and 20 iterations: 9.3, 11.9, 13.7, 48 instead of 7.2, 11.8, 16.6, 86).  Plans of more than
+// 10 K rows stage 12 slots a lane, whose registers ask for an empty CU, and such a CU comes late on a busy chip: 12,000 vertices and 108 K entries alone
+// 27, 33, 42, 48, 53 us for 3, 5, 8, 10, 12 iterations instead of 27, 35, 49-68, 56-72, 64-75, beside a stream that adds to 1 GiB of floats 178 for any
+// of them instead of 75, 106, 150, 175, 193: from 8 on an idle chip gains more than a busy one loses (10,000 vertices and 200 K entries, which find
+// their places, 62, 73, 88 for 3, 5, 8 instead of 81, 109, 155).
+constexpr int kSellResidentIters = 3, kSellResidentItersEmptyCu = 8;
 int sell_run(const SellRows &sr, const double *inv_user, int iters, double alpha, double *rank_out, hipStream_t stream);
 
 }  // namespace drone

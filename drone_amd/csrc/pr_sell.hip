@@ -191,11 +191,12 @@ __global__ __launch_bounds__(T) void sell_iterate_kernel(int n, int hubs, int sl
 // on with the NaN.  The last work-group to leave then clears every set, and the plan's next run reports it instead of running.)
 // Long enough: `patience` looks where who is there takes no more rounds of slices and hub rows than all would; else also as many as the run
 // would take with them, at kSellLooksPerRound a round (1.2 us on an idle chip, four times that beside a stream of memory-bound kernels), so
-// that the wait at most doubles it.  20 / 3 iterations beside a stream that adds to 1 GiB of floats, us, a launch per iteration / one
-// work-group behind every closed gate / this: 4 K vertices and 53 K entries 289 / 111 / 112 and 67 / 45 / 47, 12 K and 108 K 313 / 3,300 / 250 and 70 /
-// 557 / 130-260, 12 K and 419 K 381 / 12,700 / 250-315 and 82 / 1,930 / 130-280; beside bf16 products of 8,192 rows, whose work-groups fill the
-// chip for 0.7 ms each, 16,000 / 80-5,300 / 780.  What the short runs of more than 10 K rows lose are the places: 124 registers a lane ask for an
-// empty CU (with 96, at the price of 27 spilled, 71 / 80, but 20 iterations of an idle chip 78 -> 104 and 91 -> 132).
+// that the wait at most doubles it.  20 iterations beside a stream that adds to 1 GiB of floats, us, a launch per iteration / one
+// work-group behind every closed gate / this: 4 K vertices and 53 K entries 289 / 111 / 119 (three 67 / 45 / 51), 12 K and 108 K 313 / 3,300 / 177, 12 K and
+// 240 K 323 / - / 220-237, 12 K and 344 K 363 / - / 270, 12 K and 419 K 381 / 12,700 / 250-315; beside bf16 products of 8,192 rows, whose work-groups fill the
+// chip for 0.7 ms each, 16,000 / 80-5,300 / 780.  What the runs of more than 10 K rows wait for are the places: 124 registers a lane ask for an
+// empty CU (with 96, at the price of 27 spilled, 71 / 80 for three iterations, but 20 of an idle chip 78 -> 104 and 91 -> 132), so their short runs
+// are a launch per iteration (kSellResidentItersEmptyCu).
 constexpr int kSellResidentThreads = 1024;
 constexpr unsigned long long kSellNone = 0x7ffc5e1100a1b2c3ull, kSellNan = 0x7ff8000000000000ull;
 // The gate: who has come, and once it is closed how many of them do the run.
@@ -849,6 +850,7 @@ void choose_resident(SellRows *sr, int live)
     if (!sr->staged || sr->lds > kSellResidentLds || sr->hubs > kSellResidentBlocks || sr->live_slices > kSellResidentBlocks * (kSellResidentThreads / kWave)) return;
     const int wanted = std::max((int)ceil_div(sr->live_slices, kSellResidentSlices), sr->hubs);
     sr->resident = std::max(1, std::min({wanted, kSellResidentBlocks, sr->live_slices}));  // each of several owns a row
+    sr->resident_iters = sr->staged < kSellStaged ? kSellResidentIters : kSellResidentItersEmptyCu;
     const auto rounds = [&](int groups) { return ceil_div(sr->live_slices, groups * (kSellResidentThreads / kWave)) + ceil_div(sr->hubs, groups); };
     while (sr->rule.enough < sr->resident && rounds(sr->rule.enough) > rounds(sr->resident)) ++sr->rule.enough;
 }

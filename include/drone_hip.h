@@ -181,7 +181,7 @@ int drone_pr_run_f64(drone_pr_plan *plan, double alpha, int iters, double *rank_
 /* Per-iteration timing with HIP events on the launch stream.  When enabled, every iteration inside
  * drone_pr_run_f64 - the aggregation kernel, the merge of shared blocks, the row fix-up and the dangling-mass
  * reduction, i.e. everything the algorithmic bytes of one iteration pay for - is bracketed by an event pair (at
- * most `max_launches` are kept); a run that is one launch (three iterations or more of a small matrix) by one pair, an
+ * most `max_launches` are kept); a run that is one launch (three iterations or more of a small matrix, eight or more above 10,240 rows with entries) by one pair, an
  * iteration's duration being its share.  drone_pr_profile_read synchronises the events and returns the number of
  * iterations and their mean duration. */
 int drone_pr_profile_enable(drone_pr_plan *plan, int max_launches);

@@ -43,7 +43,7 @@ def _close(got, ref, rp, iters):
 def test_runs_in_one_launch(oracle, n, lengths, filler):
     rp, ci, inv = _matrix(n, lengths, filler)
     plan = _plan(rp, ci, inv)
-    for iters in (1, 2, 3, 4, 5, 9):
+    for iters in (1, 2, 3, 4, 5, 8, 9, 10):
         got = plan.run(0.85, iters).cpu().numpy()
         _close(got, oracle.pr_pull_f64(rp, ci, inv, 0.85, iters), rp, iters)
         assert np.array_equal(got, plan.run(0.85, iters).cpu().numpy())
@@ -216,4 +216,15 @@ def test_profiled_runs_are_the_same_runs(iters):
         assert torch.equal(plan.run(0.85, iters), want)
     assert plan.profile_read()["launches"] == (iters if iters >= 3 else 1)
     plan.profile_enable(0)
+    plan.close()
+
+
+@pytest.mark.parametrize("n,shortest", [(10240, 3), (10241, 8), (12288, 8)])
+def test_short_runs_that_would_wait_for_empty_cus_are_a_launch_per_iteration(n, shortest):
+    """With one pair of events a run in one launch counts all its iterations, and a launch per iteration the first."""
+    plan = _plan(*_matrix(n, [], 9))
+    for iters in (shortest - 1, shortest):
+        plan.profile_enable(1)
+        plan.run(0.85, iters)
+        assert plan.profile_read()["launches"] == (iters if iters == shortest else 1)
     plan.close()
