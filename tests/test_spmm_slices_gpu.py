@@ -97,6 +97,36 @@ def test_bits_at_any_alignment(monkeypatch, K, ld):
     plan.close()
 
 
+def test_bits_of_fewer_columns_after_nan(monkeypatch):
+    """Products of every width of the bit core's tiles behind one that left a NaN in every place of the plan's operand and partial sums:
+    what a narrower product does not write it does not read."""
+    import torch
+    from drone_amd import gcn
+    monkeypatch.setenv("DRONE_SPMM_DENSE_MIN_GAIN_MS", "0")
+    rng = np.random.default_rng(8)
+    n, most = 5000, 256
+    m = sp.vstack([sp.random(1500, n, 0.25, format="csr", random_state=3), sp.random(n - 1500, n, 0.002, format="csr", random_state=4)]).tocsr()
+    m.sort_indices()
+    m.data[:] = 1.0
+    m = m.astype(np.float32)
+    ones = torch.ones(n, device="cuda")
+    rp, ci, v = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (m.indptr.astype(np.int32), m.indices.astype(np.int32), m.data))
+    B = rng.uniform(-1, 1, (n, most)).astype(np.float32)
+    Bd, none = torch.from_numpy(B).cuda(), torch.full((n, most), np.nan, device="cuda")
+    plan = gcn.SpmmPlan(rp, ci, v, n, max_k=most, row_scale=ones, col_scale=ones)
+    assert plan.bit_core()["cells"] > 0
+    m64 = m.astype(np.float64)
+    want, scale = m64 @ B.astype(np.float64), m64 @ np.abs(B).astype(np.float64)
+    out = torch.empty(n, most, device="cuda")
+    for K in (1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129, 144, 145, 176, 192, 224, 225, 256):
+        gcn.spmm(plan, rp, ci, v, none, K=most, out=out)
+        torch.cuda.synchronize()
+        assert bool(out[torch.from_numpy(np.diff(m.indptr) > 0).cuda()].isnan().all())
+        gcn.spmm(plan, rp, ci, v, Bd, K=K, out=out)
+        _check_sums(out.cpu().numpy()[:, :K], want[:, :K], scale[:, :K], np.diff(m.indptr), K)
+    plan.close()
+
+
 def test_pieces_join_their_rows_again_and_again():
     """One plan, products of several widths in turn, with and without what was there before: the rows' tickets start over each time."""
     import torch
