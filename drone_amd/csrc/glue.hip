@@ -510,7 +510,7 @@ struct AdamStep {
 
 // A tensor's gradient is there, or still the partial sums of a split reduction, which are then added up as sgemm_reduce_kernel does
 // it: 32 outputs to 256 lanes, eight sums of an output in flight, a fixed order.  Bound by launches: a reduction of its own for each of two
-// weights, and the step, were 3.4 to 4.7 us each (epoch on 2,708 vertices 135 -> 127 us, 30,011-vertex step, whose layer 1 keeps its reduction, 226 -> 224).
+// weights, and the step, were 3.4 to 4.7 us each (epoch on 2,708 vertices and its evaluation 145 -> 138 us, 30,011-vertex step, whose layer 1 keeps its reduction, 226 -> 224).
 template <typename Step>
 __global__ __launch_bounds__(kThreads) void step_kernel(StepTensors tensors, Step step)
 {

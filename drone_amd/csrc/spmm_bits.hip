@@ -60,8 +60,8 @@ int split_columns(int width) { return width <= 16 ? 16 : width <= 32 ? 32 : widt
 
 // Thread (group of 8 ranked columns, feature column n of the pass): scales, splits and packs 8 values of B.  N: columns that the
 // product reads; the places of the others in `split` stay as they are.  Bound by what it writes, six bytes a value, beside the gathers (with all
-// 128 columns, most of them zeros, forward and transposed product of 2.4 M vertices and 34 M entries at K = 32 926 instead of 894 us, of 3 M
-// at K = 64 2,190 instead of 2,180, and the 232,965-vertex step, whose second layer has 41, 7,697 instead of 7,662).
+// 128 columns, most of them zeros, forward and transposed product of 2.4 M vertices and 34 M entries at K = 32 926 instead of 894 us; a launch for 41
+// columns of 232,965 vertices 88 instead of 50, which is less than two runs of that graph's step of 7,700 differ by, and no call at K = 64 shows it).
 template <int N>
 __global__ __launch_bounds__(256) void bits_split_kernel(int groups, const unsigned *__restrict__ col_order,
                                                          const float *__restrict__ col_scale,
