@@ -18,8 +18,8 @@
 // bounds check per element, so M, N, K and the leading dimensions are arbitrary.
 // Measured on one MI355X: 232,965 x 602 x 128 100 TFLOP/s (640-wide aligned rows 110), 65,536 x 32,768 x 128 (the
 // dense-core shape of the SpMM) 133 TFLOP/s = 84 % of the 157 TFLOP/s fp32 MFMA peak.
-// A long reduction with a small output (the weight gradient: K = vertex count) is split over grid.z; the
-// partial tiles go to a scratch buffer and are summed in split order by a second kernel.
+// A long reduction with few tiles is split over grid.z; the partial tiles go to a scratch buffer and are summed in split order by a
+// second kernel.  Weight gradients (A transposed, K = vertex count) have a kernel of their own, gemm_grad.h.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -27,6 +27,7 @@
 
 #include "common.h"
 #include "gemm_direct.h"
+#include "gemm_grad.h"
 
 namespace drone {
 namespace {
@@ -248,276 +249,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                     }
                 }
             }
-}
-
-// Weight gradients with a small output: C(M x N) = A^T * B with M <= 128, N <= 64 and a reduction over hundreds of
-// thousands of rows (H1^T * dT2 of the 2-layer model: 128 x 41 over 232,965 vertices).  The whole output is eight
-// 32 x 32 accumulators, so ONE wavefront holds it, and with A stored K x M and B stored K x N both operands of
-// v_mfma_f32_32x32x2_f32 come straight from rows of the inputs: no LDS staging, no loader wavefronts, every wavefront
-// streams its own share of the reduction into registers, kSkinnyDepth k-pairs ahead.  A lane reads FOUR consecutive
-// floats of A's row and TWO of B's with one load each (lane r of a half-wavefront: columns 4r .. 4r + 3 and 2r, 2r + 1),
-// and its four / two values go to the four / two tiles: tile i holds the output rows 4r + i, tile j the output columns
-// 2r + j - a renumbering that only the epilogue sees.  (With one dword per lane and tile, six loads per k-pair instead
-// of two, the address unit spends 16 clocks per 256 bytes and the same product took 57 us instead of the figure below;
-// splitting the output rows over the wavefronts instead of the reduction - 32 registers of accumulators, 16 k-pairs in
-// flight - reads B four times and took 70 us.)  The four wavefronts of a work-group add their tiles in wavefront order
-// through LDS; the work-groups' tiles go to the split scratch and are summed in a fixed order by sgemm_reduce_kernel
-// (bitwise repeatable).  Through the tiled kernel the same product ran at 23 TFLOP/s: 227 work-groups with one
-// 128 x 64 tile each, every one paying the LDS pipeline's fill and drain for 1,024 reduction steps.
-#ifndef DRONE_SKINNY_DEPTH
-#define DRONE_SKINNY_DEPTH 4
-#endif
-#ifndef DRONE_SKINNY_SPLITS
-#define DRONE_SKINNY_SPLITS 512
-#endif
-constexpr int kSkinnyDepth = DRONE_SKINNY_DEPTH;   // k-pairs fetched per step and wavefront
-constexpr int kSkinnyWaves = 4;
-struct alignas(4) Float2U {
-    float v[2];
-};
-__global__ __launch_bounds__(kSkinnyWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void sgemm_tn_skinny_kernel(
-    int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb, int k_chunk,
-    float *__restrict__ partial)
-{
-    constexpr int TM = 4, TN = 2;
-    __shared__ float s_tile[128 * 64];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int lr = lane & 31, lk = lane >> 5;
-    const int kb = blockIdx.x * k_chunk;
-    const int ke = kb + k_chunk < K ? kb + k_chunk : K;
-    floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-    // Every load is unconditional: a lane outside the output reads a valid place of the row (the caller guarantees
-    // lda >= M rounded up to 4 and ldb >= N rounded up to 2) and the bits it gets are masked to zero.  (A load whose
-    // value is only selected under a per-lane condition is sunk into a branch of its own by the compiler; the mask keeps
-    // it needed on every path and cannot turn a stray NaN into one.)  Rows are addressed as a wavefront-uniform base plus
-    // a 32-bit lane offset in bytes, the form that costs one register per load.
-    unsigned keep_m[TM], keep_n[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) keep_m[i] = 4 * lr + i < M ? 0xFFFFFFFFu : 0u;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) keep_n[j] = 2 * lr + j < N ? 0xFFFFFFFFu : 0u;
-    const unsigned lane_a = 4u * (unsigned)(lk * lda + (4 * lr < M ? 4 * lr : 0));
-    const unsigned lane_b = 4u * (unsigned)(lk * ldb + (2 * lr < N ? 2 * lr : 0));
-    const int step = 2 * kSkinnyWaves * kSkinnyDepth;
-    const int ke_pairs = kb + ((ke - kb) & ~1);  // whole k-pairs end here; an odd last row is added after the loop
-    // Two register sets with fixed names take turns (a set chosen by a run-time index would live in scratch memory).
-    float a0[kSkinnyDepth][TM], b0[kSkinnyDepth][TN], a1[kSkinnyDepth][TM], b1[kSkinnyDepth][TN];
-    const auto fetch = [&](float (&a)[kSkinnyDepth][TM], float (&b)[kSkinnyDepth][TN], int k_first) {
-        const int k0 = __builtin_amdgcn_readfirstlane(k_first);
-#pragma unroll
-        for (int u = 0; u < kSkinnyDepth; ++u) {
-            const int k = k0 + 2 * kSkinnyWaves * u;               // the pair's first row: uniform
-            const bool live = k < ke_pairs;
-            const unsigned keep_k = live ? 0xFFFFFFFFu : 0u;       // a pair past the end reads rows kb, kb + 1: zeros
-            const char *ra = reinterpret_cast<const char *>(A + (size_t)(live ? k : kb) * lda);
-            const char *rb = reinterpret_cast<const char *>(B + (size_t)(live ? k : kb) * ldb);
-            const Float4U qa = *reinterpret_cast<const Float4U *>(ra + lane_a);
-            const Float2U qb = *reinterpret_cast<const Float2U *>(rb + lane_b);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) a[u][i] = __uint_as_float(__float_as_uint(qa.v[i]) & keep_m[i] & keep_k);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) b[u][j] = __uint_as_float(__float_as_uint(qb.v[j]) & keep_n[j] & keep_k);
-        }
-    };
-    const auto multiply = [&](const float (&a)[kSkinnyDepth][TM], const float (&b)[kSkinnyDepth][TN]) {
-#pragma unroll
-        for (int u = 0; u < kSkinnyDepth; ++u)
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][i], b[u][j], acc[i][j], 0, 0, 0);
-    };
-    int k0 = kb + 2 * wave;
-    if (k0 < ke_pairs) {  // the same for the whole wavefront
-        fetch(a0, b0, k0);
-        for (;;) {
-            fetch(a1, b1, k0 + step);
-            multiply(a0, b0);
-            k0 += step;
-            if (k0 >= ke_pairs) break;
-            fetch(a0, b0, k0 + step);
-            multiply(a1, b1);
-            k0 += step;
-            if (k0 >= ke_pairs) break;
-        }
-    }
-    if (wave == 0 && ke_pairs < ke) {  // the odd last row of the range: a pair whose second row is zero
-        const unsigned keep_k = lk == 0 ? 0xFFFFFFFFu : 0u;
-        const Float4U qa = *reinterpret_cast<const Float4U *>(A + (size_t)ke_pairs * lda + (4 * lr < M ? 4 * lr : 0));
-        const Float2U qb = *reinterpret_cast<const Float2U *>(B + (size_t)ke_pairs * ldb + (2 * lr < N ? 2 * lr : 0));
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(__float_as_uint(qa.v[i]) & keep_m[i] & keep_k),
-                                                                 __uint_as_float(__float_as_uint(qb.v[j]) & keep_n[j] & keep_k),
-                                                                 acc[i][j], 0, 0, 0);
-    }
-    // The wavefronts' tiles, added in wavefront order.  Register v of lane l of tile (i, j) is row 8*(v/4) + 4*(l/32) +
-    // v%4 and column l%32 of the tile, i.e. output row 4 * that row + i and output column 2 * (l%32) + j.
-    for (int w = 0; w < kSkinnyWaves; ++w) {
-        if (wave == w) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int row = 4 * (8 * (v / 4) + 4 * lk + (v % 4)) + i, col = 2 * lr + j;
-                        float *cell = s_tile + row * 64 + col;
-                        *cell = w == 0 ? acc[i][j][v] : *cell + acc[i][j][v];
-                    }
-        }
-        __syncthreads();
-    }
-    float *out = partial + (size_t)blockIdx.x * M * N;
-    for (int idx = threadIdx.x; idx < M * N; idx += kSkinnyWaves * kWave) {
-        const int row = idx / N, col = idx - row * N;
-        out[idx] = s_tile[row * 64 + col];
-    }
-}
-
-// The same product on 16 x 16 tiles (v_mfma_f32_16x16x4_f32) for outputs of at most 128 x 16 NT: 41 columns fill three
-// 16-wide tiles where the 32-wide tiles above multiply 64.  Lane m + 16 q of a wavefront reads, from row k + q of a
-// group of four rows, four consecutive floats of A at columns 4 m and 64 + 4 m (the eight tiles along M: tile (h, i)
-// holds the output rows 64 h + 4 m + i) and NT consecutive floats of B at column NT m (tile j: output columns
-// NT m + j) - three loads per four rows and 8 NT matrix instructions.  Loads are unconditional and masked, rows are
-// addressed as a wavefront-uniform base plus a 32-bit lane offset, two register sets of kSmallDepth groups take turns,
-// and the four wavefronts add their tiles in wavefront order through LDS, all as in sgemm_tn_skinny_kernel.
-template <int W> struct alignas(4) FloatNU {
-    float v[W];
-};
-// One group of four rows per fetch: deeper steps (2 / 3 / 4 groups) measured 50 / 68 / 66 us against 47 for the 128 x 41
-// gradient over 232,965 rows (a wavefront's share of a work-group's 455 rows is then cut into coarser steps, and the
-// matrix instructions of a long step leave the next step's loads less time to land).
-constexpr int kSmallDepth = 1, kSmallWaves = 4;
-template <int NT>
-__global__ __launch_bounds__(kSmallWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void sgemm_tn_small_kernel(
-    int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb, int k_chunk,
-    float *__restrict__ partial)
-{
-    constexpr int CP = 16 * NT;
-    __shared__ float s_tile[2 * 128 * CP];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int lm = lane & 15, lk = lane >> 4;
-    const int kb = blockIdx.x * k_chunk;
-    const int ke = kb + k_chunk < K ? kb + k_chunk : K;
-    floatx4 acc[2][4][NT];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[h][i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    unsigned keep_m[2][4], keep_n[NT];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) keep_m[h][i] = 64 * h + 4 * lm + i < M ? 0xFFFFFFFFu : 0u;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) keep_n[j] = NT * lm + j < N ? 0xFFFFFFFFu : 0u;
-    unsigned lane_a[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) lane_a[h] = 4u * (unsigned)(lk * lda + (64 * h + 4 * lm < M ? 64 * h + 4 * lm : 0));
-    const unsigned lane_b = 4u * (unsigned)(lk * ldb + (NT * lm < N ? NT * lm : 0));
-    const int step = 4 * kSmallWaves * kSmallDepth;
-    const int ke_groups = kb + ((ke - kb) & ~3);  // whole groups of four rows end here; the last 1 - 3 rows follow the loop
-    float a0[kSmallDepth][2][4], b0[kSmallDepth][NT], a1[kSmallDepth][2][4], b1[kSmallDepth][NT];
-    const auto fetch = [&](float (&a)[kSmallDepth][2][4], float (&b)[kSmallDepth][NT], int k_first) {
-        const int k0 = __builtin_amdgcn_readfirstlane(k_first);
-#pragma unroll
-        for (int u = 0; u < kSmallDepth; ++u) {
-            const int k = k0 + 4 * kSmallWaves * u;                // the group's first row: uniform
-            const bool live = k < ke_groups;
-            const unsigned keep_k = live ? 0xFFFFFFFFu : 0u;       // a group past the end reads rows kb .. kb + 3: zeros
-            const char *ra = reinterpret_cast<const char *>(A + (size_t)(live ? k : kb) * lda);
-            const char *rb = reinterpret_cast<const char *>(B + (size_t)(live ? k : kb) * ldb);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const Float4U qa = *reinterpret_cast<const Float4U *>(ra + lane_a[h]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[u][h][i] = __uint_as_float(__float_as_uint(qa.v[i]) & keep_m[h][i] & keep_k);
-            }
-            const FloatNU<NT> qb = *reinterpret_cast<const FloatNU<NT> *>(rb + lane_b);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) b[u][j] = __uint_as_float(__float_as_uint(qb.v[j]) & keep_n[j] & keep_k);
-        }
-    };
-    const auto multiply = [&](const float (&a)[kSmallDepth][2][4], const float (&b)[kSmallDepth][NT]) {
-#pragma unroll
-        for (int u = 0; u < kSmallDepth; ++u)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j)
-                        acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][h][i], b[u][j], acc[h][i][j], 0, 0, 0);
-    };
-    int k0 = kb + 4 * wave;
-    if (k0 < ke_groups) {  // the same for the whole wavefront
-        fetch(a0, b0, k0);
-        for (;;) {
-            fetch(a1, b1, k0 + step);
-            multiply(a0, b0);
-            k0 += step;
-            if (k0 >= ke_groups) break;
-            fetch(a0, b0, k0 + step);
-            multiply(a1, b1);
-            k0 += step;
-            if (k0 >= ke_groups) break;
-        }
-    }
-    if (wave == 0 && ke_groups < ke) {  // the last 1 - 3 rows of the range: a group whose other rows are zero
-        const bool live = ke_groups + lk < ke;
-        const unsigned keep_k = live ? 0xFFFFFFFFu : 0u;
-        const size_t row = (size_t)(live ? ke_groups + lk : ke_groups);
-        const FloatNU<NT> qb = *reinterpret_cast<const FloatNU<NT> *>(B + row * ldb + (NT * lm < N ? NT * lm : 0));
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const Float4U qa = *reinterpret_cast<const Float4U *>(A + row * lda + (64 * h + 4 * lm < M ? 64 * h + 4 * lm : 0));
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        __uint_as_float(__float_as_uint(qa.v[i]) & keep_m[h][i] & keep_k),
-                        __uint_as_float(__float_as_uint(qb.v[j]) & keep_n[j] & keep_k), acc[h][i][j], 0, 0, 0);
-        }
-    }
-    // The wavefronts' tiles, added in a fixed order: wavefronts 0 and 1 store theirs side by side, 2 and 3 add theirs on
-    // top, and the two sums are added on the way out.  Register v of lane l of tile (h, i, j) is row 4 (l / 16) + v and
-    // column l % 16 of the tile, i.e. output row 64 h + 4 * that row + i and output column NT * (l % 16) + j.
-    static_assert(kSmallWaves == 4, "two rounds of two wavefronts");
-    for (int round = 0; round < 2; ++round) {
-        if (wave / 2 == round) {
-            float *mine = s_tile + (wave & 1) * 128 * CP;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            float *cell = mine + (64 * h + 4 * (4 * lk + v) + i) * CP + NT * lm + j;
-                            *cell = round == 0 ? acc[h][i][j][v] : *cell + acc[h][i][j][v];
-                        }
-        }
-        __syncthreads();
-    }
-    float *out = partial + (size_t)blockIdx.x * M * N;
-    for (int idx = threadIdx.x; idx < M * N; idx += kSmallWaves * kWave) {
-        const int row = idx / N, col = idx - row * N;
-        out[idx] = s_tile[row * CP + col] + s_tile[128 * CP + row * CP + col];
-    }
 }
 
 // C = alpha * sum_z partial[z] + beta * C.  A work-group of 256 lanes owns 32 consecutive outputs; lane (o, g) adds the
@@ -811,45 +542,6 @@ int split_scratch(bool may_allocate, KeptSums *kept, size_t floats, hipStream_t 
     return static_scratch(partial);
 }
 
-// C = alpha * A^T * B + beta * C for a small output and a long reduction (see sgemm_tn_skinny_kernel and
-// sgemm_tn_small_kernel, which takes the outputs whose rows of B can be read in whole pieces).
-bool skinny_is_small(int N, int ldb)
-{
-    const int nt = (N + 15) / 16;
-    return ldb >= (N + nt - 1) / nt * nt;  // a lane reads nt consecutive floats of B's row, also past N
-}
-int skinny_splits(int N, int K, int ldb, int *k_chunk)
-{
-    const bool small = skinny_is_small(N, ldb);
-    // two work-groups of four wavefronts per CU, each wavefront at least 16 steps of the reduction deep
-    const int rows_per_step = small ? 4 * kSmallWaves * kSmallDepth : 2 * kSkinnyWaves * kSkinnyDepth;
-    const int align = small ? 4 * kSmallWaves : 2 * kSkinnyWaves;
-    int splits = DRONE_SKINNY_SPLITS;
-    const int deepest = (int)ceil_div(K, rows_per_step * 16);
-    if (splits > deepest) splits = deepest;
-    if (splits < 1) splits = 1;
-    *k_chunk = (int)ceil_div(ceil_div(K, splits), align) * align;
-    return (int)ceil_div(K, *k_chunk);
-}
-int sgemm_tn_skinny(bool may_allocate, KeptSums *kept, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-                    float beta, float *C, int ldc, hipStream_t s)
-{
-    int k_chunk = 0;
-    const int nt = (N + 15) / 16, splits = skinny_splits(N, K, ldb, &k_chunk);
-    const bool small = skinny_is_small(N, ldb);
-    float *partial = nullptr;
-    const int rc = split_scratch(may_allocate, kept, (size_t)splits * M * N, s, M, N, K, splits, &partial);
-    if (rc != DRONE_OK) return rc;
-    if (!small) sgemm_tn_skinny_kernel<<<splits, kSkinnyWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    else if (nt == 1) sgemm_tn_small_kernel<1><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    else if (nt == 2) sgemm_tn_small_kernel<2><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    else if (nt == 3) sgemm_tn_small_kernel<3><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    else sgemm_tn_small_kernel<4><<<splits, kSmallWaves * kWave, 0, s>>>(M, N, K, A, lda, B, ldb, k_chunk, partial);
-    if (!(kept && kept->splits > 0)) launch_reduce(M, N, splits, partial, alpha, beta, C, ldc, s);
-    DRONE_HIP_TRY(hipGetLastError());
-    return DRONE_OK;
-}
-
 // C = alpha * A * op(B) + beta * C for a tall A with rows of at most 128 values (see sgemm_tall_kernel); false when no
 // instance of the kernel covers the shape.
 template <int KQ, int NT, bool TB>
@@ -900,62 +592,45 @@ void sgemm_tall(int transB, int M, int N, int K, float alpha, const float *A, in
 // Whether 128-column tiles have 64 rows instead of 128: two of their work-groups on a CU work while one waits at its barrier
 // (matrix cores busy 53 % of the time with one), and half as many CUs idle at the end.  us 128 / 64 rows: 30,011 x 301 x 100 34.6 /
 // 32.0, 45,000 x 300 x 128 51.3 / 43.7, 5,000 x 1,000 x 1,000 146 / 119, 1,000 x 1,001 x 3,000 82 / 76.  Not where 128-row tiles come
-// two to a CU anyway, 60,000 x 400 x 100 67.6 / 70.6, and not with A transposed, whose tiles are read in shorter runs: 602 x
-// 128 over 232,965 rows 330 / 374.
+// two to a CU anyway, 60,000 x 400 x 100 67.6 / 70.6, and not with A transposed, whose tiles are read in shorter runs.
 bool half_rows(bool transA, int tiles) { return !transA && tiles <= 384; }
 
 // How many ways the tiled kernel splits the reduction: when the output has too few tiles to fill 256 CUs and K is long.
 int tiled_splits(int tiles, int K)
 {
     if (tiles >= 256 || K < 4096) return 1;
-    // two work-groups per CU in one round, and at least 1024 reduction steps per work-group.  Measured on the
-    // weight gradients of the 232,965-vertex model (ms for 128 x 41 / 602 x 128 outputs): 1024 work-groups of at
-    // least 512 steps 0.153 / 0.443; 512 and 512: 0.153 / 0.414; 256 and 1024: 0.106 / 0.516; 512 and 1024:
-    // 0.106 / 0.411; 512 and 2048: 0.123 / 0.414.
+    // two work-groups per CU in one round, and at least 1024 reduction steps per work-group (ms for outputs of 128 x 41 / 602 x 128
+    // over 232,965 steps: 1024 work-groups of at least 512 steps 0.153 / 0.443; 512 and 512: 0.153 / 0.414; 256 and 1024:
+    // 0.106 / 0.516; 512 and 1024: 0.106 / 0.411; 512 and 2048: 0.123 / 0.414)
     return std::max(1, std::min(512 / tiles, (int)ceil_div(K, 1024)));
 }
 
 // Which products sgemm_direct_kernel takes, and in which shape (ks = 0: the tiled kernel).  The shapes were chosen by
-// timing all instances on some 150 layer products (2 ... 128 columns, inner dimensions 2 ... 700, 1,000 ... 233,000 rows)
-// and their weight gradients; the choice between the kernels compares two estimates that were fitted to the same runs.
+// timing all instances on some 150 layer products (2 ... 128 columns, inner dimensions 2 ... 700, 1,000 ... 233,000 rows);
+// the choice between the kernels compares two estimates that were fitted to the same runs.
 struct DirectShape {
-    int mt = 0, nt = 0, ks = 0, splits = 1;
+    int mt = 0, nt = 0, ks = 0;
 };
-DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
+DirectShape direct_shape(int M, int N, int K)
 {
     DirectShape d;
-    if (K < 1 || (ta && tb) || (ta && M < 2)) return d;
+    if (K < 1) return d;
     const auto blocks = [&]() { return ceil_div(M, 16 * d.mt) * ceil_div(N, 16 * d.nt); };
-    if (ta) {
-        // One work-group per CU, its wavefronts a group of 16 steps each at least (two work-groups and five groups at most before:
-        // twice the partial sums, or a few CUs at work), and blocks that grow with the product: a block of 4 x 4 tiles reads a third
-        // less per product than one of 2 x 4, and has nothing to hide in a short reduction.  us before / now: outputs of 301 x 100 over
-        // 30,011 rows 41.1 / 35.4, 300 x 128 over 100,000 109 / 85, 1,400 x 128 over 5,000 38.2 / 33.8, 200 x 64 over 60,000 33.6 /
-        // 28.8 (2 x 4: 33.3) and over 9,001 14.5 / 10.9 (2 x 4: 11.5), 100 x 50 over 15,003 15.5 / 11.3, 100 x 23 over 30,011 16.9 /
-        // 11.5, 64 x 30 over 5,000 17.4 / 8.5, 64 x 7 over 2,708 11.1 / 8.3.
-        const double macs = (double)M * N * K;
-        if (N <= 16) { d.mt = M <= 16 ? 1 : 2; d.nt = 1; d.ks = 16; }
-        else if (N <= 32) { d.mt = M > 64 ? 4 : 2; d.nt = 2; d.ks = M > 64 ? 8 : 16; }
-        else if (ceil_div(N, 64) * 64 * 4 > ceil_div(N, 32) * 32 * 5) { d.mt = M >= 64 ? 4 : 2; d.nt = 2; d.ks = 8; }
-        else { d.mt = M > 32 && macs >= 5e8 ? 4 : 2; d.nt = macs >= 1.5e8 ? 4 : 2; d.ks = 8; }
-        d.splits = (int)std::max<int64_t>(1, std::min<int64_t>({256 / blocks(), K / (16 * d.ks), 128}));
+    const int n16 = (int)ceil_div(N, 16);
+    d.mt = 1;
+    d.nt = n16 <= 4 ? n16 : n16 <= 6 ? 3 : n16 == 7 ? 7 : 4;
+    const int64_t waves = blocks();
+    if (K >= 384 && d.nt != 7) {
+        // the wavefronts of a work-group share a row block: less of op(B) is read per product
+        d.ks = 8;
+        if (waves >= 1024 && d.nt != 3) d.mt = 2;
+    } else if (waves >= 1024) {
+        d.ks = 1;
+        if (waves >= 4096) d.mt = 2;
     } else {
-        const int n16 = (int)ceil_div(N, 16);
-        d.mt = 1;
-        d.nt = n16 <= 4 ? n16 : n16 <= 6 ? 3 : n16 == 7 ? 7 : 4;
-        const int64_t waves = blocks();
-        if (K >= 384 && d.nt != 7) {
-            // the wavefronts of a work-group share a row block: less of op(B) is read per product
-            d.ks = 8;
-            if (waves >= 1024 && d.nt != 3) d.mt = 2;
-        } else if (waves >= 1024) {
-            d.ks = 1;
-            if (waves >= 4096) d.mt = 2;
-        } else {
-            if (d.nt == 7) d.nt = 4;
-            if (K < 256 && d.nt > 2 && waves < 512) d.nt = 2;
-            d.ks = K >= 384 ? 8 : K >= 64 ? 4 : 1;
-        }
+        if (d.nt == 7) d.nt = 4;
+        if (K < 256 && d.nt > 2 && waves < 512) d.nt = 2;
+        d.ks = K >= 384 ? 8 : K >= 64 ? 4 : 1;
     }
     // Deep reductions (384 steps and more) bring the tiled kernel's streams up to speed - 2.8 instead of 2.0 TB/s, and two of
     // its work-groups on a CU take 0.85 of two rounds -, and the direct kernel, whose row blocks each read all of op(B), reaches
@@ -967,92 +642,61 @@ DirectShape direct_shape(bool ta, bool tb, int M, int N, int K)
     // us: matrix instructions at the rate the kernel reaches on padded blocks, or its memory traffic
     const double in = 4.0 * ((double)M * K + (double)K * N), out = 4.0 * M * N;
     const double padded = 2.0 * blocks() * (16 * d.mt) * (16 * d.nt) * K;
-    const double direct_us = std::max(padded / (deep && !ta ? 60e6 : d.mt * d.nt == 16 ? 90e6 : 75e6), in / 4.5e6 + out / 1.9e6) + (d.splits > 1 ? 4 : 0);
+    const double direct_us = std::max(padded / (deep ? 60e6 : 75e6), in / 4.5e6 + out / 1.9e6);
     // us: rounds of work-groups over the CUs times depth-32 tiles (1.6 us for a 64-wide tile, 2.25 for a 128-wide one)
     const int tiles = (int)(ceil_div(M, kTileRows) * ceil_div(N, N <= 64 ? 64 : 128)), splits = tiled_splits(tiles, K);
     const int64_t groups = (int64_t)tiles * splits;
-    const double rounds = ceil_div(groups, 256) * (deep && groups > 256 ? 0.85 : N > 64 && half_rows(ta, tiles) ? 0.9 : 1.0);
+    const double rounds = ceil_div(groups, 256) * (deep && groups > 256 ? 0.85 : N > 64 && half_rows(false, tiles) ? 0.9 : 1.0);
     const double tiled_us = std::max(rounds * ceil_div(ceil_div(K, splits), BK) * (N <= 64 ? 1.6 : 2.25),
                                      in / (deep ? 2.8e6 : 2.0e6) + out / 2.4e6) + (splits > 1 ? 5 : 0);
     if (tiled_us < direct_us) d.ks = 0;
     return d;
 }
 
-template <int MT, int NT, bool AK, bool BK, int KS>
-void launch_direct(const DirectShape &d, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
-                   float beta, float *C, int ldc, int k_chunk, float *partial, hipStream_t s)
+template <int MT, int NT, bool BK, int KS>
+void launch_direct(int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta, float *C, int ldc, hipStream_t s)
 {
     constexpr int kWaves = KS > 4 ? KS : 4;
-    const dim3 grid((unsigned)(ceil_div(N, 16 * NT) * ceil_div(M, 16 * MT * (kWaves / KS))), 1, (unsigned)d.splits);
+    const unsigned grid = (unsigned)(ceil_div(N, 16 * NT) * ceil_div(M, 16 * MT * (kWaves / KS)));
     const size_t lds = KS > 1 ? sizeof(float) * kWaves * MT * NT * 4 * kWave : 0;
-    sgemm_direct_kernel<MT, NT, AK, BK, KS><<<grid, kWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
+    sgemm_direct_kernel<MT, NT, BK, KS><<<grid, kWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 
-int direct_splits(const DirectShape &d, int K, int *k_chunk)
+int sgemm_direct(const DirectShape &d, bool tb, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
+                 float *C, int ldc, hipStream_t s)
 {
-    *k_chunk = (int)ceil_div(ceil_div(K, d.splits), 16) * 16;
-    return (int)ceil_div(K, *k_chunk);
-}
-
-int sgemm_direct(DirectShape d, bool may_allocate, KeptSums *kept, bool ta, bool tb, int M, int N, int K, float alpha, const float *A,
-                 int lda, const float *B, int ldb, float beta, float *C, int ldc, hipStream_t s)
-{
-    int k_chunk = 0;
-    d.splits = direct_splits(d, K, &k_chunk);
-    float *partial = nullptr;
-    if (d.splits > 1) {
-        const int rc = split_scratch(may_allocate, kept, (size_t)d.splits * M * N, s, M, N, K, d.splits, &partial);
-        if (rc != DRONE_OK) return rc;
-    }
     bool done = false;
-#define DRONE_DIRECT(MT_, NT_, AK_, BK_, KS_)                                                              \
-    if (d.mt == MT_ && d.nt == NT_ && d.ks == KS_ && ta != AK_ && tb == BK_) {                              \
-        launch_direct<MT_, NT_, AK_, BK_, KS_>(d, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial, s); \
-        done = true;                                                                                      \
+#define DRONE_DIRECT(MT_, NT_, KS_)                                                                   \
+    if (d.mt == MT_ && d.nt == NT_ && d.ks == KS_) {                                                  \
+        if (tb) launch_direct<MT_, NT_, true, KS_>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);  \
+        else launch_direct<MT_, NT_, false, KS_>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);    \
+        done = true;                                                                                  \
     }
-#define DRONE_DIRECT_ROWS(MT_, NT_, KS_) DRONE_DIRECT(MT_, NT_, true, false, KS_) DRONE_DIRECT(MT_, NT_, true, true, KS_)
-    DRONE_DIRECT_ROWS(1, 1, 1)
-    DRONE_DIRECT_ROWS(1, 2, 1)
-    DRONE_DIRECT_ROWS(1, 3, 1)
-    DRONE_DIRECT_ROWS(1, 4, 1)
-    DRONE_DIRECT_ROWS(1, 7, 1)
-    DRONE_DIRECT_ROWS(2, 1, 1)
-    DRONE_DIRECT_ROWS(2, 2, 1)
-    DRONE_DIRECT_ROWS(2, 3, 1)
-    DRONE_DIRECT_ROWS(2, 4, 1)
-    DRONE_DIRECT_ROWS(2, 7, 1)
-    DRONE_DIRECT_ROWS(1, 1, 4)
-    DRONE_DIRECT_ROWS(1, 2, 4)
-    DRONE_DIRECT_ROWS(1, 3, 4)
-    DRONE_DIRECT_ROWS(1, 4, 4)
-    DRONE_DIRECT_ROWS(1, 1, 8)
-    DRONE_DIRECT_ROWS(1, 2, 8)
-    DRONE_DIRECT_ROWS(1, 3, 8)
-    DRONE_DIRECT_ROWS(1, 4, 8)
-    DRONE_DIRECT_ROWS(2, 1, 8)
-    DRONE_DIRECT_ROWS(2, 2, 8)
-    DRONE_DIRECT_ROWS(2, 4, 8)
-    DRONE_DIRECT(1, 1, false, false, 16)
-    DRONE_DIRECT(2, 1, false, false, 16)
-    DRONE_DIRECT(2, 2, false, false, 16)
-    DRONE_DIRECT(2, 2, false, false, 8)
-    DRONE_DIRECT(4, 2, false, false, 8)
-    DRONE_DIRECT(2, 4, false, false, 8)
-    DRONE_DIRECT(4, 4, false, false, 8)
-#undef DRONE_DIRECT_ROWS
+    DRONE_DIRECT(1, 1, 1)
+    DRONE_DIRECT(1, 2, 1)
+    DRONE_DIRECT(1, 3, 1)
+    DRONE_DIRECT(1, 4, 1)
+    DRONE_DIRECT(1, 7, 1)
+    DRONE_DIRECT(2, 1, 1)
+    DRONE_DIRECT(2, 2, 1)
+    DRONE_DIRECT(2, 3, 1)
+    DRONE_DIRECT(2, 4, 1)
+    DRONE_DIRECT(2, 7, 1)
+    DRONE_DIRECT(1, 1, 4)
+    DRONE_DIRECT(1, 2, 4)
+    DRONE_DIRECT(1, 3, 4)
+    DRONE_DIRECT(1, 4, 4)
+    DRONE_DIRECT(1, 1, 8)
+    DRONE_DIRECT(1, 2, 8)
+    DRONE_DIRECT(1, 3, 8)
+    DRONE_DIRECT(1, 4, 8)
+    DRONE_DIRECT(2, 1, 8)
+    DRONE_DIRECT(2, 2, 8)
+    DRONE_DIRECT(2, 4, 8)
 #undef DRONE_DIRECT
     DRONE_REQUIRE(done, "no instance of the direct kernel for this shape");
-    if (d.splits > 1 && !(kept && kept->splits > 0)) launch_reduce(M, N, d.splits, partial, alpha, beta, C, ldc, s);
     DRONE_HIP_TRY(hipGetLastError());
     return DRONE_OK;
-}
-
-// (the skinny kernel's lanes read four floats of A's row and two of B's at once, also the lanes past M and N.  128 x 41
-// outputs: 24.6 us (17.9 by sgemm_direct_kernel) over 30,000 rows, 24.0 (24.5) over 50,000, 31 (39) over 100,000; outputs
-// of 32 rows and fewer are better off with the direct kernel at any length, 43 x 22 and 43 x 41 are not)
-bool skinny_covers(int transA, int transB, int M, int N, int K, int lda, int ldb)
-{
-    return transA && !transB && M > 32 && M <= 128 && N <= 64 && K >= 40000 && lda >= (M + 3) / 4 * 4 && ldb >= (N + 1) / 2 * 2;
 }
 
 int tiled_chunk(int tiles, int K, int *k_chunk)
@@ -1061,6 +705,11 @@ int tiled_chunk(int tiles, int K, int *k_chunk)
     return (int)ceil_div(K > 0 ? K : 1, *k_chunk);
 }
 int tiles_of(int M, int N) { return (int)(ceil_div(M, kTileRows) * ceil_div(N, N <= 64 ? 64 : 128)); }
+
+// Outputs of 128 tiles and more keep the tiled kernel busy without a split, and its tiles are read once per 128 rows (us tiled /
+// sgemm_grad_kernel: 4,096 x 4,096 over 1,024 rows 271 / 352, 1,000 x 3,000 over 1,001 86 / 84, 4,096 x 512 over 65,536 2,064 / 2,105, 1,000 x
+// 1,000, 64 tiles, over 5,000 104 / 94).
+bool grad_covers(int M, int N, int K) { return K > 0 && tiles_of(M, N) < 128; }
 
 int sgemm_entry(bool may_allocate, KeptSums *kept, int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,
                 const float *B, int ldb, float beta, float *C, int ldc, drone_stream_t stream)
@@ -1077,11 +726,22 @@ int sgemm_entry(bool may_allocate, KeptSums *kept, int transA, int transB, int M
         DRONE_HIP_TRY(hipGetLastError());
         return DRONE_OK;
     }
-    if (skinny_covers(transA, transB, M, N, K, lda, ldb))
-        return sgemm_tn_skinny(may_allocate, kept, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
-    const DirectShape direct = direct_shape(transA != 0, transB != 0, M, N, K);
-    if (direct.ks > 0)
-        return sgemm_direct(direct, may_allocate, kept, transA != 0, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+    if (transA && !transB && grad_covers(M, N, K)) {
+        const GradShape grad = grad_shape(M, N, K);
+        float *partial = nullptr;
+        if (grad.splits > 1) {
+            const int rc = split_scratch(may_allocate, kept, (size_t)grad.splits * M * N, s, M, N, K, grad.splits, &partial);
+            if (rc != DRONE_OK) return rc;
+        }
+        sgemm_grad(grad, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, partial, s);
+        if (partial && !(kept && kept->splits > 0)) launch_reduce(M, N, grad.splits, partial, alpha, beta, C, ldc, s);
+        DRONE_HIP_TRY(hipGetLastError());
+        return DRONE_OK;
+    }
+    if (!transA) {
+        const DirectShape direct = direct_shape(M, N, K);
+        if (direct.ks > 0) return sgemm_direct(direct, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+    }
     const bool narrow = N <= 64;
     const int bn = narrow ? 64 : 128;
     const int tiles = tiles_of(M, N);
@@ -1122,11 +782,8 @@ extern "C" int drone_sgemm_rm_f32_noalloc(int transA, int transB, int M, int N, 
 extern "C" int64_t drone_sgemm_tn_sums_floats(int M, int N, int K, int lda, int ldb)
 {
     if (M < 1 || N < 1 || K < 1) return 0;
-    int k_chunk = 0, splits;
-    const DirectShape direct = direct_shape(true, false, M, N, K);
-    if (skinny_covers(1, 0, M, N, K, lda, ldb)) splits = skinny_splits(N, K, ldb, &k_chunk);
-    else if (direct.ks > 0) splits = direct_splits(direct, K, &k_chunk);
-    else splits = tiled_chunk(tiles_of(M, N), K, &k_chunk);
+    int k_chunk = 0;
+    const int splits = grad_covers(M, N, K) ? grad_shape(M, N, K).splits : tiled_chunk(tiles_of(M, N), K, &k_chunk);
     return splits > 1 ? (int64_t)splits * M * N : 0;
 }
 

@@ -5,7 +5,7 @@
 // 128-row tiles out.  What that buys is parallelism: a wavefront owns 16 (32) rows instead of a work-group 128, and the
 // KS wavefronts of a work-group share one output block by splitting the reduction, adding their blocks in wavefront order
 // through LDS.  A 2,708 x 1,433 x 64 layer product ran as 22 tiles of the tiled kernel on 22 of 256 CUs (66 us; here 12.5),
-// its weight gradient as 12 (102 -> 13); 320 x 100 outputs over 30,011 rows 133 -> 45, 1,000 x 608 x 128 56 -> 7.  Small
+// 1,000 x 608 x 128 56 -> 7.  (Weight gradients: gemm_grad.h.)  Small
 // products are bound by their chain of loads, mid-size ones by the L2 -> L1 traffic above (70 - 80 TFLOP/s), which is why
 // large ones stay with the tiled kernel (100 - 130).
 //
@@ -149,15 +149,13 @@ struct DirectOperand {
     }
 };
 
-// C (M x N) = alpha op(A) op(B) + beta C, or, with `partial`, the raw sums of the reduction range blockIdx.z into
-// partial[blockIdx.z][M][N].  A work-group owns MT x NT tiles of 16 x 16 per output block, its KS wavefronts a share of the
-// reduction each (KS = 1: four wavefronts, an output block each).
-template <int MT, int NT, bool A_K_CONTIG, bool B_K_CONTIG, int KS>
+// C (M x N) = alpha A op(B) + beta C.  A work-group owns MT x NT tiles of 16 x 16 per output block, its KS wavefronts a share of
+// the reduction each (KS = 1: four wavefronts, an output block each).
+template <int MT, int NT, bool B_K_CONTIG, int KS>
 __global__ __launch_bounds__((KS > 4 ? KS : 4) * kWave) void sgemm_direct_kernel(int M, int N, int K, float alpha,
                                                                              const float *__restrict__ A, int lda,
                                                                              const float *__restrict__ B, int ldb,
-                                                                             float beta, float *__restrict__ C, int ldc,
-                                                                             int k_chunk, float *__restrict__ partial)
+                                                                             float beta, float *__restrict__ C, int ldc)
 {
     constexpr int kWaves = KS > 4 ? KS : 4, kBlocks = kWaves / KS;
     constexpr int RP = 16 * MT, CP = 16 * NT;
@@ -167,19 +165,18 @@ __global__ __launch_bounds__((KS > 4 ? KS : 4) * kWave) void sgemm_direct_kernel
     // column blocks of the same rows are neighbours in launch order: they read the same part of A
     const int col_blocks = (N + CP - 1) / CP, row_group = blockIdx.x / col_blocks;
     const int m0 = (row_group * kBlocks + block) * RP, n0 = (blockIdx.x - row_group * col_blocks) * CP;
-    const int kb = blockIdx.z * k_chunk, ke = kb + k_chunk < K ? kb + k_chunk : K;
     direct_f4 acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = direct_f4{0.0f, 0.0f, 0.0f, 0.0f};
     if (m0 < M) {  // the same for the whole wavefront
-        DirectOperand<MT, A_K_CONTIG> oa;
+        DirectOperand<MT, true> oa;
         DirectOperand<NT, B_K_CONTIG> ob;
         oa.init(A, lda, m0, M, x, q);
         ob.init(B, ldb, n0, N, x, q);
         // whole groups of 16 steps are dealt out evenly to the KS wavefronts, the partial group goes to the last of them
-        const int groups = (ke - kb) / 16;
+        const int groups = K / 16;
         const int g0 = (int)((long long)groups * share / KS), g1 = (int)((long long)groups * (share + 1) / KS);
         const auto multiply = [&](const float (&a)[MT][4], const float (&b)[NT][4]) {
 #pragma unroll
@@ -193,11 +190,11 @@ __global__ __launch_bounds__((KS > 4 ? KS : 4) * kWave) void sgemm_direct_kernel
         float a0[MT][4], b0[NT][4], a1[MT][4], b1[NT][4];
         // (Two forms of one loop, which the compiler schedules differently.  The first is for deep reductions: 2,708 x 1,433 x 64 13.2 ->
         // 11.4 us, 5,000 x 1,400 x 128 32.3 -> 29.0; blocks of a wavefront of their own lose by it, 15,003 x 100 x 50 7.7 -> 11.4.)
-        if constexpr (A_K_CONTIG && KS == 8) {
+        if constexpr (KS == 8) {
             if (g0 < g1) {
-                const auto group = [&](int g) { return kb + 16 * (g < g1 ? g : g1 - 1); };  // the last group again behind it
-                oa.load(kb + 16 * g0, a0);
-                ob.load(kb + 16 * g0, b0);
+                const auto group = [&](int g) { return 16 * (g < g1 ? g : g1 - 1); };  // the last group again behind it
+                oa.load(16 * g0, a0);
+                ob.load(16 * g0, b0);
                 for (int g = g0;;) {
                     bool over = false;
 #pragma unroll
@@ -214,50 +211,44 @@ __global__ __launch_bounds__((KS > 4 ? KS : 4) * kWave) void sgemm_direct_kernel
                 }
             }
         } else if (g0 < g1) {
-            oa.load(kb + 16 * g0, a0);
-            ob.load(kb + 16 * g0, b0);
+            oa.load(16 * g0, a0);
+            ob.load(16 * g0, b0);
             for (int g = g0;;) {
                 // the last group is fetched once more instead of the one behind it
                 int next = g + 1 < g1 ? g + 1 : g;
-                oa.load(kb + 16 * next, a1);
-                ob.load(kb + 16 * next, b1);
+                oa.load(16 * next, a1);
+                ob.load(16 * next, b1);
                 multiply(a0, b0);
                 if (++g >= g1) break;
                 next = g + 1 < g1 ? g + 1 : g;
-                oa.load(kb + 16 * next, a0);
-                ob.load(kb + 16 * next, b0);
+                oa.load(16 * next, a0);
+                ob.load(16 * next, b0);
                 multiply(a1, b1);
                 if (++g >= g1) break;
             }
         }
-        if (share == KS - 1 && kb + 16 * groups < ke) {
-            oa.load_tail(kb + 16 * groups, ke, q, a0);
-            ob.load_tail(kb + 16 * groups, ke, q, b0);
+        if (share == KS - 1 && 16 * groups < K) {
+            oa.load_tail(16 * groups, K, q, a0);
+            ob.load_tail(16 * groups, K, q, b0);
             multiply(a0, b0);
         }
     }
-    float *out = partial ? partial + (size_t)blockIdx.z * M * N : C;
-    const int ldo = partial ? N : ldc;
     const auto put = [&](int row, int col, float sum) {
-        float *dst = out + (size_t)row * ldo + col;
-        if (partial) {
-            *dst = sum;
-        } else {
-            float r = alpha * sum;
-            if (beta != 0.0f) r += beta * *dst;
-            *dst = r;
-        }
+        float *dst = C + (size_t)row * ldc + col;
+        float r = alpha * sum;
+        if (beta != 0.0f) r += beta * *dst;
+        *dst = r;
     };
     // Register v of lane x + 16 q of tile (i, t) is row position 4 q + v and column position x of the tile.
     if constexpr (KS == 1) {
         if (m0 >= M) return;
-        const bool wide = !partial && beta == 0.0f && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+        const bool wide = beta == 0.0f && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 bool own_row;
-                const int row = direct_outer<MT, A_K_CONTIG>(m0, M, i, 4 * q + v, own_row);
+                const int row = direct_outer<MT, true>(m0, M, i, 4 * q + v, own_row);
                 if (!own_row) continue;
 #pragma unroll
                 for (int t = 0; t < NT;) {
@@ -296,7 +287,7 @@ __global__ __launch_bounds__((KS > 4 ? KS : 4) * kWave) void sgemm_direct_kernel
             const int row = (row_group * kBlocks + blk) * RP + pr, col = n0 + pc;
             if (row >= M || col >= N) continue;
             int i, xr, t, xc;
-            direct_place<MT, A_K_CONTIG>((row_group * kBlocks + blk) * RP, M, row, i, xr);
+            direct_place<MT, true>((row_group * kBlocks + blk) * RP, M, row, i, xr);
             direct_place<NT, B_K_CONTIG>(n0, N, col, t, xc);
             const int at = ((i * NT + t) * 4 + xr % 4) * kWave + (xr / 4) * 16 + xc;
             float sum = 0.0f;
