@@ -48,6 +48,14 @@
 #include "spmm_bits.h"
 #include "spmm_slices.h"
 
+namespace drone {
+// The rows of a chunk (at most 63, with at most 64 entries together), from its first row and its first entry on.
+struct alignas(16) ChunkRows {
+    unsigned long long heads;  // bit e: entry e is the first of its row
+    unsigned long long some;   // bit j: row j has entries
+};
+}  // namespace drone
+
 struct drone_spmm_plan {
     int n_rows = 0, n_cols = 0;
     int64_t nnz = 0;
@@ -55,6 +63,7 @@ struct drone_spmm_plan {
     // short rows in chunks: consecutive rows of at most 64 entries together (or one row of any length up to the split)
     int num_chunks = 0;
     int4 *chunk = nullptr;  // device [num_chunks]: {first row, last + 1, first entry, last + 1}
+    drone::ChunkRows *chunk_rows = nullptr;  // device [num_chunks]
     // long rows, cut into band pieces
     int num_long = 0, num_pieces = 0;
     int64_t long_nnz = 0;
@@ -201,10 +210,30 @@ __device__ __forceinline__ void load_vec(const float *p, float (&x)[VEC])
     else { x[0] = *p; }
 }
 
+// The (col, val) pairs that a wavefront has fetched, one a lane, for its lane groups to read: an LDS read of a pair is one instruction where two
+// cross-lane reads (ds_bpermute) were.  A wavefront writes and reads its own.
+struct alignas(8) Pair {
+    int col;
+    float val;
+};
+struct WavePairs {
+    Pair at[kWave];
+    unsigned char row[kWave];  // of a chunk: place among its rows of the n-th row with entries
+};
+
+// Feature-row loads in flight per lane group in the launch that takes pieces and chunks together: eight of wide lane groups, of which a
+// wavefront has few, and four of narrow ones, where eight cost more registers than they bring.  us with 8 / 4: 30,011 vertices at K = 100 28.4 / 31.4,
+// at K = 23 14.8 / 12.5; 300,007 at K = 32 62.9 / 53.4; 71,791 at K = 62 31.5 / 33.1.
+constexpr int gather_rows(int lanes) { return lanes >= 16 ? 8 : 4; }
+
 // Accumulates sum_e val[e] * B[col[e], cols.at .. cols.at+VEC) for e in [e0, e1) into acc (per lane), then
-// folds the P lane groups together so that group 0 holds the totals.
-template <int G, int VEC>
-__device__ __forceinline__ void row_segment(int e0, int e1, const int *__restrict__ ci, const float *__restrict__ val,
+// folds the P lane groups together so that group 0 holds the totals.  MOST: feature-row loads in flight per lane group.  With `pairs`
+// they are handed out through LDS, and of narrow lane groups fetched a batch ahead: a row of several batches is then a round trip a
+// batch faster (wide groups take several steps a batch, and pay the registers with a wavefront a SIMD: 150,001 vertices at K = 128 88.9 / 90.7
+// us, 71,791 at K = 62 31.9 / 32.8).  Band pieces, mostly of one or two batches and in launches that wait for the fabric, do
+// without (null; 1,000,003 vertices at K = 41 340 / 376).
+template <int G, int VEC, int MOST>
+__device__ __forceinline__ void row_segment(WavePairs *pairs, int e0, int e1, const int *__restrict__ ci, const float *__restrict__ val,
                                             const float *__restrict__ B, int ldb, const LaneColumns<VEC> &cols,
                                             float (&acc)[VEC])
 {
@@ -218,12 +247,26 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
     // Software-pipelining the steps (slot u of the next step loaded as soon as slot u of this one is added, the
     // pairs read a batch ahead) needs 88 registers, leaves 5 wavefronts per SIMD and took 6.88 / 3.76 ms for K = 128 /
     // 41 on the 229 M-entry graph against 4.31 / 2.45; held to 64 registers it spills.
-    constexpr int U = (kWave / P) < 8 ? (kWave / P) : 8;
-    for (int base = e0; base < e1; base += kWave) {
+    constexpr int U = (kWave / P) < MOST ? (kWave / P) : MOST;
+    int c_next = 0;
+    float a_next = 0.0f;
+    const auto fetch = [&](int base) {
         const int e = base + lane;
-        const int c = e < e1 ? ci[e] : 0;
-        const float a = e < e1 ? val[e] : 0.0f;
+        c_next = e < e1 ? ci[e] : 0;
+        a_next = e < e1 ? val[e] : 0.0f;
+    };
+    const bool ahead = pairs && G < 16;
+    if (ahead) fetch(e0);
+    for (int base = e0; base < e1; base += kWave) {
+        if (!ahead) fetch(base);
+        const int c = c_next;
+        const float a = a_next;
+        if (ahead && base + kWave < e1) fetch(base + kWave);
         const int cnt = (e1 - base) < kWave ? (e1 - base) : kWave;
+        if (P > 1 && pairs) {
+            pairs->at[lane] = Pair{c, a};
+            __builtin_amdgcn_wave_barrier();
+        }
         for (int q = 0; q < cnt; q += P * U) {
             int cc[U];
             float aa[U];
@@ -232,9 +275,13 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
                 if constexpr (P == 1) {
                     cc[u] = __builtin_amdgcn_readlane(c, q + u);
                     aa[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), q + u));
-                } else {
+                } else if (!pairs) {
                     cc[u] = __shfl(c, q + u * P + sub, kWave);
                     aa[u] = __shfl(a, q + u * P + sub, kWave);
+                } else {
+                    const Pair at = pairs->at[q + u * P + sub];
+                    cc[u] = at.col;
+                    aa[u] = at.val;
                 }
             }
             if (cols.active()) {
@@ -253,6 +300,7 @@ __device__ __forceinline__ void row_segment(int e0, int e1, const int *__restric
                     for (int v = 0; v < VEC; ++v) acc[v] = fmaf(aa[u], b[u][v], acc[v]);
             }
         }
+        if (pairs) __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll
     for (int off = G; off < kWave; off <<= 1)
@@ -284,23 +332,24 @@ __device__ __forceinline__ void store_row(float *__restrict__ dst, const LaneCol
 // a handful of feature-row loads in flight at the end of it; a chunk pays the first two round trips once for ten rows
 // or so and then keeps U feature-row loads per lane group in flight across the row boundaries.  The P lane groups
 // take contiguous row ranges of the chunk (cut where the entries divide evenly); a group walks its entries in order
-// and stores a row whenever the next entry belongs to another one.  Control flow is kept uniform over the wavefront
-// (the cross-lane reads must see every lane), the groups differ in predicates only.
-// Where a chunk's segments (rows of the matrix) begin and end, and where their sums go.  (The band pieces were run
+// and stores a row whenever the next entry belongs to another one.  Where rows begin comes as a bit per entry with the chunk
+// (ChunkRows): as positions in the first lanes it took thirteen dependent cross-lane reads to place the groups, and twelve a step to hand out
+// columns, values and rows.  Bound, in a matrix that the GPU holds at once, by the chain descriptor, pairs, feature rows, store, and by its
+// vector instructions (half of the time at K = 8).  us before / with bits and pairs through LDS: 30,011 vertices and 0.65 M entries at K = 100
+// 30.0 / 28.5, K = 23 15.2 / 12.5; 71,791 and 1.4 M at K = 62 32.7 / 31.9, K = 8 21.8 / 18.4; 20,003 and 0.44 M at K = 48 14.3 / 12.1; 300,007 and 3.9 M at
+// K = 32 61 / 51; 2,400,011 and 21 M at K = 32 393 / 369; epoch on 2,708 vertices 135 / 129.  (The band pieces were run
 // through the same kernel, consecutive pieces of the work list with at most 64 entries together: no gain, 9.85 against
 // 9.79 ms per training step on the 229 M-entry graph - what is left in pieces waits for the fabric, not for round trips.)
-struct RowSegments {
-    const int *__restrict__ rp;
+struct RowSums {  // where they go
     float *__restrict__ C;
     int ldc;
     float alpha, beta;
-    __device__ __forceinline__ int start(int first, int j) const { return rp[first + j]; }  // j <= count
-    __device__ __forceinline__ float *out(int first, int j) const { return C + (size_t)(first + j) * ldc; }
+    __device__ __forceinline__ float *row(int r) const { return C + (size_t)r * ldc; }
 };
-template <int G, int VEC, typename Segments>
-__device__ __forceinline__ void sum_chunk(int block, int slice, int slices, int num_chunks, const int4 *__restrict__ chunk,
-                                          Segments seg, const int *__restrict__ ci, const float *__restrict__ val,
-                                          const float *__restrict__ B, int ldb, int K)
+template <int G, int VEC, int MOST>
+__device__ __forceinline__ void sum_chunk(WavePairs &pairs, int block, int slice, int slices, int num_chunks, const int4 *__restrict__ chunk,
+                                          const ChunkRows *__restrict__ chunk_rows, const RowSums &to, const int *__restrict__ ci,
+                                          const float *__restrict__ val, const float *__restrict__ B, int ldb, int K)
 {
     constexpr int P = kWave / G;
     // Feature-row loads in flight per lane group.  With 8 the kernels take 84 registers, 5 or 6 wavefronts a SIMD; with 4 at most
@@ -313,104 +362,67 @@ __device__ __forceinline__ void sum_chunk(int block, int slice, int slices, int 
     const int li = lane % G, sub = lane / G;
     const int4 mine = chunk[c];
     const int r0 = mine.x, nrows = mine.y - mine.x, e0 = mine.z, n = mine.w - mine.z;
-    const float alpha = seg.alpha, beta = seg.beta;
     if (nrows == 1) {
-        float *dst = seg.out(r0, 0);
         for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
             const LaneColumns<VEC> cols{k0 + li * VEC, K};
             float acc[VEC];
-            row_segment<G, VEC>(e0, e0 + n, ci, val, B, ldb, cols, acc);
-            if (sub == 0 && cols.active()) store_row<VEC>(dst, cols, acc, alpha, beta);
+            row_segment<G, VEC, MOST>(&pairs, e0, e0 + n, ci, val, B, ldb, cols, acc);
+            if (sub == 0 && cols.active()) store_row<VEC>(to.row(r0), cols, acc, to.alpha, to.beta);
         }
         return;
     }
-    // lane j holds where segment r0 + j starts; lanes nrows .. 63 hold where the chunk ends.  (Its entries are fetched meanwhile:
-    // their bounds come with the chunk's.)
-    const int start = seg.start(r0, lane < nrows ? lane : nrows);
-    const int col = lane < n ? ci[e0 + lane] : 0;
-    const float a = lane < n ? val[e0 + lane] : 0.0f;
-    // the segment of entry `lane`: the last one that starts at or before it
-    int row_of = 0;
-    {
-        int lo = 0, hi = nrows - 1;
-#pragma unroll
-        for (int it = 0; it < 6; ++it) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (__shfl(start, mid, kWave) <= e0 + lane) lo = mid; else hi = mid - 1;
-        }
-        row_of = lo;
-    }
-    // group `sub` takes the segments from the first one that starts at or after its share of the entries
-    const auto first_row_at = [&](int target) {  // smallest j in [0, nrows] with start_j >= target (start_nrows = end)
-        int lo = 0, hi = nrows;
-#pragma unroll
-        for (int it = 0; it < 7; ++it) {
-            const int mid = (lo + hi) >> 1;
-            const int at = __shfl(start, mid, kWave);  // by every lane, whatever its own search still needs
-            if (lo < hi) {
-                if (at >= target) hi = mid; else lo = mid + 1;
-            }
-        }
-        return lo;
+    const unsigned long long heads = chunk_rows[c].heads, some = chunk_rows[c].some;
+    pairs.at[lane] = Pair{lane < n ? ci[e0 + lane] : 0, lane < n ? val[e0 + lane] : 0.0f};
+    const bool gaps = (some & (some + 1)) != 0;  // rows without entries before others (a chunk's last rows may have none without a gap)
+    if (gaps && (some >> lane & 1)) pairs.row[__popcll(some & ((1ull << lane) - 1))] = (unsigned char)lane;
+    __builtin_amdgcn_wave_barrier();
+    // group `sub` takes the rows from the first one that starts at or after its share of the entries
+    const auto first_head_at = [&](int target) {
+        const unsigned long long left = target < kWave ? heads >> target : 0ull;
+        return left ? target + __ffsll((long long)left) - 1 : n;
     };
-    // (both searches by every lane: the starts they read sit in the first lanes, which must not be masked off)
-    const int ra = first_row_at(e0 + (n * sub + P - 1) / P);
-    const int rb_search = first_row_at(e0 + (n * (sub + 1) + P - 1) / P);
-    const int rb = sub == P - 1 ? nrows : rb_search;
-    const int qa = __shfl(start, ra, kWave) - e0, qb = __shfl(start, rb, kWave) - e0;
-    int steps = (qb - qa + U - 1) / U;
-#pragma unroll
-    for (int off = G; off < kWave; off <<= 1) {
-        const int other = __shfl_xor(steps, off, kWave);
-        steps = other > steps ? other : steps;
-    }
-    // segments without entries: out = beta * out, by the first lane group
-    const int next_start = __shfl_down(start, 1, kWave);
-    const unsigned long long empty = __ballot(lane < nrows && next_start == start);
+    const int qa = first_head_at((n * sub + P - 1) / P), qb = sub == P - 1 ? n : first_head_at((n * (sub + 1) + P - 1) / P);
     for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
         const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-        int cur = -1;
-        for (int step = 0; step < steps; ++step) {
-            const int q0 = qa + step * U;
-            int cc[U], rr[U];
-            float aa[U];
+        if (cols.active() && qa < qb) {
+            int cur = __popcll(heads & ((1ull << qa) - 1));  // the n-th row with entries
+            const auto store = [&]() { store_row<VEC>(to.row(r0 + (gaps ? (int)pairs.row[cur] : cur)), cols, acc, to.alpha, to.beta); };
+            for (int q0 = qa; q0 < qb; q0 += U) {
+                Pair at[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int q = q0 + u < qb ? q0 + u : 0;
-                cc[u] = __shfl(col, q, kWave);
-                aa[u] = __shfl(a, q, kWave);
-                rr[u] = __shfl(row_of, q, kWave);
-            }
-            float b[U][VEC];
+                for (int u = 0; u < U; ++u) at[u] = pairs.at[q0 + u < kWave ? q0 + u : kWave - 1];
+                float b[U][VEC];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+                for (int u = 0; u < U; ++u) {
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) b[u][v] = 0.0f;
-                if (cols.active() && q0 + u < qb) load_vec<VEC>(B + (size_t)cc[u] * ldb + cols.at(), b[u]);
-            }
+                    for (int v = 0; v < VEC; ++v) b[u][v] = 0.0f;
+                    if (q0 + u < qb) load_vec<VEC>(B + (size_t)at[u].col * ldb + cols.at(), b[u]);
+                }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (q0 + u < qb) {
-                    if (rr[u] != cur) {
-                        if (cur >= 0 && cols.active()) store_row<VEC>(seg.out(r0, cur), cols, acc, alpha, beta);
-                        cur = rr[u];
+                for (int u = 0; u < U; ++u) {
+                    if (q0 + u < qb) {
+                        if ((heads >> (q0 + u) & 1) && q0 + u > qa) {
+                            store();
+                            ++cur;
 #pragma unroll
-                        for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
+                            for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
+                        }
+#pragma unroll
+                        for (int v = 0; v < VEC; ++v) acc[v] = fmaf(at[u].val, b[u][v], acc[v]);
                     }
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) acc[v] = fmaf(aa[u], b[u][v], acc[v]);
                 }
             }
+            store();
         }
-        if (cur >= 0 && cols.active()) store_row<VEC>(seg.out(r0, cur), cols, acc, alpha, beta);
-        for (unsigned long long left = empty; left; left &= left - 1) {
-            const int j = __ffsll((long long)left) - 1;
+        // rows without entries: out = beta * out, by the first lane group
+        if (sub == 0 && cols.active()) {
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[v] = 0.0f;
-            if (sub == 0 && cols.active()) store_row<VEC>(seg.out(r0, j), cols, acc, alpha, beta);
+            for (unsigned long long left = ~some & ((1ull << nrows) - 1); left; left &= left - 1)
+                store_row<VEC>(to.row(r0 + __ffsll((long long)left) - 1), cols, acc, to.alpha, to.beta);
         }
     }
 }
@@ -425,8 +437,8 @@ __device__ __forceinline__ void sum_chunk(int block, int slice, int slices, int 
 // occupancy (76 VGPRs, 6 instead of 8 wavefronts per SIMD; capped at 64 VGPRs it spills, 5.17 ms).
 // One piece per lane group (two or four pieces side by side in a wavefront, nothing folded across groups) lost too:
 // 4.78 / 3.00 ms for K = 128 / 41 against 4.44 / 2.60 - the wavefront runs as long as its longest piece.
-template <int G, int VEC>
-__device__ __forceinline__ void sum_piece(int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
+template <int G, int VEC, int MOST>
+__device__ __forceinline__ void sum_piece(WavePairs *pairs, int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
                                           const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
                                           const int *__restrict__ ci, const float *__restrict__ val,
                                           const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K)
@@ -438,7 +450,7 @@ __device__ __forceinline__ void sum_piece(int block, int slice, int slices, int 
     for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
         const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
-        row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
+        row_segment<G, VEC, MOST>(pairs, piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
         if (sub == 0 && cols.active()) store_row<VEC>(partial + (size_t)piece_slot[s] * ldp, cols, acc, 1.0f, 0.0f);
     }
 }
@@ -456,11 +468,11 @@ struct JoinRows {
     unsigned *ticket;
 };
 template <int G, int VEC>
-__device__ __forceinline__ void join_piece(int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
+__device__ __forceinline__ void join_piece(WavePairs &pairs, int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
                                            const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
                                            const int *__restrict__ ci, const float *__restrict__ val,
                                            const float *__restrict__ B, int ldb, float *partial, int ldp, int K, const JoinRows &rows,
-                                           const RowSegments &to)
+                                           const RowSums &to)
 {
     const int s = block * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (s >= num_pieces) return;
@@ -471,7 +483,7 @@ __device__ __forceinline__ void join_piece(int block, int slice, int slices, int
     for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
         const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
-        row_segment<G, VEC>(piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
+        row_segment<G, VEC, gather_rows(G)>(&pairs, piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
         if (sub == 0 && cols.active()) {
             float *mine = partial + (size_t)piece_slot[s] * ldp + cols.at();
             unsigned before[VEC];
@@ -519,16 +531,17 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock, G == 8 ? 6 : 8) void spmm_pi
     const float *__restrict__ B, int ldb, float *__restrict__ partial, int ldp, int K, int slice_bits)
 {
     const int slices = 1 << slice_bits;
-    sum_piece<G, VEC>(blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
+    sum_piece<G, VEC, 8>(nullptr, blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
 }
 
-template <int G, int VEC, typename Segments>
+template <int G, int VEC>
 __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_chunks_kernel(
-    int num_chunks, const int4 *__restrict__ chunk, Segments seg, const int *__restrict__ ci, const float *__restrict__ val,
-    const float *__restrict__ B, int ldb, int K, int slice_bits)
+    int num_chunks, const int4 *__restrict__ chunk, const ChunkRows *__restrict__ chunk_rows, RowSums to, const int *__restrict__ ci,
+    const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
+    __shared__ WavePairs s_pairs[kRowsPerBlock];
     const int slices = 1 << slice_bits;
-    sum_chunk<G, VEC>(blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_chunks, chunk, seg, ci, val, B, ldb, K);
+    sum_chunk<G, VEC, 4>(s_pairs[threadIdx.x / kWave], blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
 }
 
 // Both in one launch, the pieces first: the chunks fill the GPU while the last pieces end, and a launch is saved.  us
@@ -539,17 +552,19 @@ template <int G, int VEC, bool JOIN>
 __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_gather_kernel(
     int num_pieces, int piece_blocks, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
     const int *__restrict__ piece_slot, const int *__restrict__ ci2, const float *__restrict__ val2,
-    float *partial, int ldp, JoinRows join, int num_chunks, const int4 *__restrict__ chunk, RowSegments seg,
-    const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
+    float *partial, int ldp, JoinRows join, int num_chunks, const int4 *__restrict__ chunk, const ChunkRows *__restrict__ chunk_rows,
+    RowSums to, const int *__restrict__ ci, const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
+    __shared__ WavePairs s_pairs[kRowsPerBlock];
+    WavePairs &pairs = s_pairs[threadIdx.x / kWave];
     const int slices = 1 << slice_bits, block = blockIdx.x >> slice_bits, slice = blockIdx.x & (slices - 1);
     if (block < piece_blocks) {
         if constexpr (JOIN)
-            join_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K, join, seg);
+            join_piece<G, VEC>(pairs, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K, join, to);
         else
-            sum_piece<G, VEC>(block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
+            sum_piece<G, VEC, gather_rows(G)>(nullptr, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
     } else {
-        sum_chunk<G, VEC>(block - piece_blocks, slice, slices, num_chunks, chunk, seg, ci, val, B, ldb, K);
+        sum_chunk<G, VEC, gather_rows(G)>(pairs, block - piece_blocks, slice, slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
     }
 }
 
@@ -841,17 +856,17 @@ __global__ void gather_sorted_kernel(int64_t count, const unsigned *__restrict__
 }
 
 template <int G, int VEC>
-void launch_spmm(const drone_spmm_plan *plan, const int *rp, const int *ci, const float *v, const float *B, int ldb,
+void launch_spmm(const drone_spmm_plan *plan, const int *ci, const float *v, const float *B, int ldb,
                  float *C, int ldc, int K, float alpha, float beta, int slice_bits, hipStream_t s)
 {
     const int piece_blocks = (int)ceil_div(plan->num_pieces, kRowsPerBlock), chunk_blocks = (int)ceil_div(plan->num_chunks, kRowsPerBlock);
-    const RowSegments rows{rp, C, ldc, alpha, beta};
+    const RowSums rows{C, ldc, alpha, beta};
     if (piece_blocks > 0 && chunk_blocks > 0 && plan->bits.tiles == 0) {
         const JoinRows join{plan->piece_long, plan->long_row, plan->first_slot, plan->ticket};
         const auto launch = [&](auto kernel) {
             kernel<<<((unsigned)piece_blocks + (unsigned)chunk_blocks) << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
                 plan->num_pieces, piece_blocks, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2,
-                plan->partial, plan->ldp, join, plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
+                plan->partial, plan->ldp, join, plan->num_chunks, plan->chunk, plan->chunk_rows, rows, ci, v, B, ldb, K, slice_bits);
         };
         if (plan->ticket) {
             launch(spmm_gather_kernel<G, VEC, true>);
@@ -864,8 +879,8 @@ void launch_spmm(const drone_spmm_plan *plan, const int *rp, const int *ci, cons
                 plan->num_pieces, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2, B, ldb,
                 plan->partial, plan->ldp, K, slice_bits);
         if (chunk_blocks > 0)
-            spmm_chunks_kernel<G, VEC, RowSegments><<<(unsigned)chunk_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
-                plan->num_chunks, plan->chunk, rows, ci, v, B, ldb, K, slice_bits);
+            spmm_chunks_kernel<G, VEC><<<(unsigned)chunk_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
+                plan->num_chunks, plan->chunk, plan->chunk_rows, rows, ci, v, B, ldb, K, slice_bits);
     }
     if (plan->num_long > 0) {  // also when every entry of the long rows went to the dense part: C = beta * C there
         const auto launch = [&](auto kernel, int lanes) {
@@ -1228,11 +1243,17 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
     }
     // chunks of the short rows
     std::vector<int4> h_chunk;
+    std::vector<ChunkRows> h_chunk_rows;
     const int most = chunk_entries(n_rows, nnz);
     {
         int first = -1, entries = 0;
+        ChunkRows open{};
         const auto close = [&](int end) {
-            if (first >= 0) h_chunk.push_back(make_int4(first, end, h_rp[first], h_rp[end]));
+            if (first >= 0) {
+                h_chunk.push_back(make_int4(first, end, h_rp[first], h_rp[end]));
+                h_chunk_rows.push_back(open);
+            }
+            open = ChunkRows{};
             first = -1;
             entries = 0;
         };
@@ -1243,9 +1264,14 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
             } else if (len > kWave) {  // more than one load of pairs: a chunk of its own
                 close(r);
                 h_chunk.push_back(make_int4(r, r + 1, h_rp[r], h_rp[r + 1]));
+                h_chunk_rows.push_back(ChunkRows{});
             } else {
                 if (first >= 0 && (entries + len > most || r - first >= kWave - 1)) close(r);
                 if (first < 0) first = r;
+                if (len > 0) {
+                    open.heads |= 1ull << entries;
+                    open.some |= 1ull << (r - first);
+                }
                 entries += len;
             }
         }
@@ -1279,6 +1305,8 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
             const auto upload = [&]() -> int {
                 DRONE_HIP_TRY(hipMalloc(&p->chunk, sizeof(int4) * h_chunk.size()));
                 DRONE_HIP_TRY(hipMemcpy(p->chunk, h_chunk.data(), sizeof(int4) * h_chunk.size(), hipMemcpyHostToDevice));
+                DRONE_HIP_TRY(hipMalloc(&p->chunk_rows, sizeof(ChunkRows) * h_chunk_rows.size()));
+                DRONE_HIP_TRY(hipMemcpy(p->chunk_rows, h_chunk_rows.data(), sizeof(ChunkRows) * h_chunk_rows.size(), hipMemcpyHostToDevice));
                 return DRONE_OK;
             };
             const int urc = upload();
@@ -1349,6 +1377,7 @@ extern "C" int drone_spmm_plan_destroy(drone_spmm_plan *p)
 {
     if (!p) return DRONE_OK;
     (void)hipFree(p->chunk);
+    (void)hipFree(p->chunk_rows);
     (void)hipFree(p->long_row);
     (void)hipFree(p->first_slot);
     (void)hipFree(p->piece_begin);
@@ -1433,12 +1462,12 @@ extern "C" int drone_spmm_csr_f32(const drone_spmm_plan *plan, const int *rp, co
         DRONE_HIP_TRY(hipEventRecord(plan->bits.join, plan->bits.side));
     }
     if (K < 4) {
-        launch_spmm<4, 1>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
+        launch_spmm<4, 1>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
     } else {
         const bool whole_lines = ldb % kLineFloats == 0 && (uintptr_t)B % (4 * kLineFloats) == 0;
         const Slicing by = slicing(K, plan->n_cols, whole_lines, (int64_t)plan->num_pieces + plan->num_chunks,
                                    ceil_div(plan->num_pieces, kRowsPerBlock) + ceil_div(plan->num_chunks, kRowsPerBlock), kWave * kRowsPerBlock);
-        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, rp, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s); };
+        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s); };
         if (by.lanes == 4) launch(std::integral_constant<int, 4>());
         else if (by.lanes == 8) launch(std::integral_constant<int, 8>());
         else if (by.lanes == 16) launch(std::integral_constant<int, 16>());
