@@ -28,6 +28,7 @@
 #include "common.h"
 #include "gemm_direct.h"
 #include "gemm_grad.h"
+#include "gemm_strip.h"
 
 namespace drone {
 namespace {
@@ -740,6 +741,11 @@ int sgemm_entry(bool may_allocate, KeptSums *kept, int transA, int transB, int M
     }
     if (!transA) {
         const DirectShape direct = direct_shape(M, N, K);
+        if (direct.ks <= 1 && strip_covers(M, N, K)) {
+            sgemm_strip(transB != 0, direct.ks == 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
+            DRONE_HIP_TRY(hipGetLastError());
+            return DRONE_OK;
+        }
         if (direct.ks > 0) return sgemm_direct(direct, transB != 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
     }
     const bool narrow = N <= 64;
