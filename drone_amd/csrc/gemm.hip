@@ -633,6 +633,8 @@ DirectShape direct_shape(int M, int N, int K)
         if (K < 256 && d.nt > 2 && waves < 512) d.nt = 2;
         d.ks = K >= 384 ? 8 : K >= 64 ? 4 : 1;
     }
+    // half of the CUs at least (1,884 x 137 x 25 4.1 -> 3.3 us, its transposed B 1,927 x 218 x 28 3.9 -> 3.4)
+    while (d.ks == 4 && d.nt > 1 && blocks() < 128) d.nt = (d.nt + 1) / 2;
     // Deep reductions (384 steps and more) bring the tiled kernel's streams up to speed - 2.8 instead of 2.0 TB/s, and two of
     // its work-groups on a CU take 0.85 of two rounds -, and the direct kernel, whose row blocks each read all of op(B), reaches
     // 60 instead of 75 TFLOP/s there.  us direct / tiled: dense rectangles of an SpMM plan, 4,096 x 32,768 x 41 336 / 196 and
@@ -663,12 +665,48 @@ void launch_direct(int M, int N, int K, float alpha, const float *A, int lda, co
     sgemm_direct_kernel<MT, NT, BK, KS><<<grid, kWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 
+// Tiles a block of sgemm_twin_kernel, or 0 to leave the product to sgemm_direct_kernel<., ., ., 8>: as few as leave no CU a second block, whose
+// wavefronts would have to share its SIMDs (us by that kernel / this: 1,726 x 1,440 x 25 8.8 / 5.9, 1,052 x 972 x 100 9.5 / 8.1 and with more
+// blocks than CUs 10.6, 5,000 x 1,400 x 128 32.4 / 33.0, 16,227 x 667 x 61 23.4 / 26.1).  Eight tiles want a long reduction (2,748 x 1,452 x 117 23.5 / 18.8,
+// 2,640 x 508 x 113 10.7 / 11.1), and B transposed, which takes a quarter of the loads, gains by the smaller blocks alone (1,233 x 591 x 21 4.9 / 4.2, but
+// 2,708 x 1,440 x 64 16.0 / 16.5 and 3,977 x 514 x 29 5.3 / 6.0).
+int twin_width(const DirectShape &d, bool tb, int M, int N, int K)
+{
+    if (d.ks != 8 || d.mt != 1) return 0;
+    for (const int nt : {1, 2, 3, 4, 5, 6, 8})
+        if (ceil_div(M, 16) * ceil_div(N, 16 * nt) <= kTwinBlocks) return (nt == 8 && K < 768) || (tb && nt == d.nt) ? 0 : nt;
+    return 0;
+}
+
+template <int NT>
+void launch_twin(bool tb, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta, float *C, int ldc, hipStream_t s)
+{
+    const unsigned grid = (unsigned)(ceil_div(N, 16 * NT) * ceil_div(M, 16));
+    const size_t lds = sizeof(float) * kTwinShares * NT * 4 * kWave;
+    if (tb) sgemm_twin_kernel<NT, true><<<grid, kTwinWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+    else sgemm_twin_kernel<NT, false><<<grid, kTwinWaves * kWave, lds, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+}
+
 int sgemm_direct(const DirectShape &d, bool tb, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
                  float *C, int ldc, hipStream_t s)
 {
     bool done = false;
+    const int twin = twin_width(d, tb, M, N, K);
+#define DRONE_TWIN(NT_)                                                                    \
+    if (twin == NT_) {                                                                     \
+        launch_twin<NT_>(tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);             \
+        done = true;                                                                       \
+    }
+    DRONE_TWIN(1)
+    DRONE_TWIN(2)
+    DRONE_TWIN(3)
+    DRONE_TWIN(4)
+    DRONE_TWIN(5)
+    DRONE_TWIN(6)
+    DRONE_TWIN(8)
+#undef DRONE_TWIN
 #define DRONE_DIRECT(MT_, NT_, KS_)                                                                   \
-    if (d.mt == MT_ && d.nt == NT_ && d.ks == KS_) {                                                  \
+    if (!twin && d.mt == MT_ && d.nt == NT_ && d.ks == KS_) {                                         \
         if (tb) launch_direct<MT_, NT_, true, KS_>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);  \
         else launch_direct<MT_, NT_, false, KS_>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);    \
         done = true;                                                                                  \
