@@ -27,6 +27,7 @@
 
 #include "common.h"
 #include "gemm_direct.h"
+#include "gemm_flat.h"
 #include "gemm_grad.h"
 #include "gemm_strip.h"
 
@@ -779,6 +780,11 @@ int sgemm_entry(bool may_allocate, KeptSums *kept, int transA, int transB, int M
     }
     if (!transA) {
         const DirectShape direct = direct_shape(M, N, K);
+        if (direct.ks <= 1 && beta == 0.0f && flat_covers(direct.ks == 0, M, N, K)) {
+            sgemm_flat(transB != 0, direct.ks == 0, M, N, K, alpha, A, lda, B, ldb, C, ldc, s);
+            DRONE_HIP_TRY(hipGetLastError());
+            return DRONE_OK;
+        }
         if (direct.ks <= 1 && strip_covers(M, N, K)) {
             sgemm_strip(transB != 0, direct.ks == 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, s);
             DRONE_HIP_TRY(hipGetLastError());

@@ -10,7 +10,7 @@
 // over 100 shapes, several worse.
 //
 // us by the kernels that it stands in for / here: 30,011 x 320 x 100 33.0 / 30.9, 64,530 x 96 x 93 28.5 / 22.0, 103,955 x 288 x 84 96 / 69, 121,197 x 192 x 38
-// 42.1 / 32.6, 196,368 x 352 x 30 98 / 63, 208,773 x 576 x 62 208 / 162, 227,087 x 92 x 23 34.6 / 28.5 and its transposed B, 23 x 92, 48.5 / 34.1.  Bound by
+// 42.1 / 32.6, 196,368 x 352 x 30 98 / 63, 208,773 x 576 x 62 208 / 162, 227,087 x 92 x 23 34.6 / 28.5.  Bound by
 // op(B)'s fetch (a launch and 7 us in front of 140 KB) on few rows, by memory (3.9 TB/s of A and C) or the matrix pipe on many.
 //
 // Sums: one accumulator per output takes the reduction's steps one after the other, as v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 both do (their
@@ -162,9 +162,8 @@ __global__ __launch_bounds__(kStripWaves * kWave) void sgemm_strip_kernel(int M,
     }
 }
 
-// Enough rows, and enough to multiply, to pay for op(B) in every CU's LDS (us by the other kernels / here, in millions of multiply-adds: 38,055 x 30 x 16
-// (18) 3.9 / 6.7, 28,784 x 29 x 49 (41) 5.6 / 6.6, 55,760 x 24 x 54 (72) 11.3 / 11.2, 66,816 x 70 x 30 (140) 13.2 / 11.1, 28,200 x 224 x 32 (202)
-// 11.6 / 8.7).
+// Enough rows, and enough to multiply, to pay for op(B) in every CU's LDS (us by the other kernels / here, in millions of multiply-adds: 30,647 x 90 x 5
+// (14) 5.1 / 6.4, 46,375 x 119 x 4 (22) 7.7 / 8.4, 81,311 x 131 x 7 (75) 13.4 / 13.9, 28,200 x 224 x 32 (202) 11.6 / 8.7).
 bool strip_covers(int M, int N, int K)
 {
     return M >= 28000 && N <= 128 && K >= 16 && (int64_t)M * N * K >= 80'000'000 && strip_lds(N, K) <= kStripLds;
