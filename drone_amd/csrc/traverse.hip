@@ -67,7 +67,7 @@ struct SsspUnitEpi : SsspEpi {
     __device__ __forceinline__ MinF32 load(int c, int64_t) const { return MinF32{dist[c] + 1.0f}; }
 };
 
-constexpr double kNotWhole = (double)(1ll << 32);
+constexpr double kNegative = 0x1p32, kNotWhole = 0x1p64;  // more than there are edges, more than kNegative times that
 
 // Where a traversal stands.  Its launches hand it on in device memory, so that several rounds can be enqueued before the host
 // has to know how the first of them went: every kernel that runs rounds looks at `listed` and leaves lists that are not for
@@ -77,9 +77,12 @@ struct TraverseState {
     int mark;                   // of the next round, cc.cu:37 `active[v] = step + 1`: positive, and different in every round
     int rounds;                 // rounds completed
     int which;                  // which of the two list buffers holds the list
-    double not_one;             // lengths other than 1.0, and kNotWhole for each that is no whole number
+    double not_one;             // lengths other than 1.0, and kNotWhole for each that is no whole number, kNegative for each below zero
+    int hold;                   // rounds before n + 2 at which push_rounds_small_kernel stops, for near_rounds_kernel to look at the list
     // All lengths are whole numbers, some not 1.0: every improvement is past the tolerance.
     __host__ __device__ bool other_whole() const { return not_one > 0.0 && not_one < kNotWhole; }
+    // ... and none is below zero.
+    __host__ __device__ bool other_natural() const { return not_one > 0.0 && not_one < kNegative; }
 };
 // Pinned memory; `state` is as the last launch before the wait left it.
 struct Report {
@@ -94,15 +97,20 @@ struct Lists {
 // A list of no vertices that no round may take for its own: all of them still have to propagate.
 __host__ __device__ __forceinline__ unsigned long long everything() { return (1ull << 32) + 0xFFFFFFFFull; }
 
-// Ends a counting kernel: the last work-group adds the work-groups' counts and leaves the sum in *out.
-__device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
+// Ends a counting kernel: the last work-group adds the work-groups' counts and hands the sum to `finish` (thread 0).
+template <typename Finish>
+__device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, Finish finish)
 {
     const double total = block_sum_256(mine, s_red);
     unsigned int one = 0;
     if (threadIdx.x == 0) one = publish_part(block_part + blockIdx.x, total);
     if (!last_block_done(ticket, one)) return;
     const double all = block_sum_of_parts(block_part, (int)gridDim.x, s_red);
-    if (threadIdx.x == 0) *out = all;
+    if (threadIdx.x == 0) finish(all);
+}
+__device__ __forceinline__ void publish_sum(double mine, double *s_red, double *block_part, unsigned int *ticket, double *out)
+{
+    publish_sum(mine, s_red, block_part, ticket, [out](double all) { *out = all; });
 }
 
 // ---- labels by joining trees -------------------------------------------------------------------------------
@@ -421,12 +429,12 @@ __global__ void iota_kernel(int *out, int n)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = i;
 }
 
-// Lengths other than 1.0, and kNotWhole for each that is no whole number: this lane's share (len is 16-byte aligned).
+// Lengths other than 1.0, and kNotWhole or kNegative for some: this lane's share of TraverseState::not_one (len is 16-byte aligned).
 __device__ __forceinline__ double count_other_lengths(int n, const float *__restrict__ len)
 {
     constexpr int kInFlight = 2;  // more, or more work-groups: the same within 2 %
     double cnt = 0.0;
-    const auto other = [](float v) { return v == 1.0f ? 0.0 : v == rintf(v) && fabsf(v) < 0x1p24f ? 1.0 : 1.0 + kNotWhole; };
+    const auto other = [](float v) { return v == 1.0f ? 0.0 : !(v == rintf(v) && fabsf(v) < 0x1p24f) ? 1.0 + kNotWhole : v < 0.0f ? 1.0 + kNegative : 1.0; };
     const float4 *len4 = reinterpret_cast<const float4 *>(len);
     const int quads = n / 4, stride = gridDim.x * kSpmvBlock;
     for (int64_t i = blockIdx.x * kSpmvBlock + threadIdx.x; i < quads; i += (int64_t)kInFlight * stride) {
@@ -454,7 +462,7 @@ __global__ __launch_bounds__(kSpmvBlock) void sssp_begin_kernel(int n, const int
                                                                 float *__restrict__ dist, int *__restrict__ ubm, const int *__restrict__ index,
                                                                 int *__restrict__ list, int *__restrict__ offset, int edges,
                                                                 const float *__restrict__ len, double *block_part, unsigned int *ticket,
-                                                                TraverseState *state)
+                                                                TraverseState *state, int hold)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
     const int start = global_to_local[start_id];
@@ -471,7 +479,10 @@ __global__ __launch_bounds__(kSpmvBlock) void sssp_begin_kernel(int n, const int
         state->mark = 1;
         state->rounds = state->which = 0;
     }
-    publish_sum(count_other_lengths(edges, len), s_red, block_part, ticket, &state->not_one);
+    publish_sum(count_other_lengths(edges, len), s_red, block_part, ticket, [&](double all) {
+        state->not_one = all;
+        state->hold = state->other_natural() ? hold : 0;
+    });
 }
 
 __global__ void gather_len_kernel(int n, const int *__restrict__ eid, const float *__restrict__ len,
@@ -623,7 +634,7 @@ struct SsspPush {
 // agent-scope atomics (see publish_part in spmv_merge.h); the list itself is plain stores, read by the next launch.
 // Every work-group has read *state by the time the last one gets here.
 __device__ __forceinline__ void end_round(TraverseState *state, int mark, int rounds, int which, unsigned long long *counters,
-                                          unsigned int *ticket)
+                                          unsigned int *ticket, int hold = -1)
 {
     __syncthreads();  // every wavefront of the work-group has issued its appends (their atomics return before they go on)
     if (!last_block_done(ticket, 1u) || threadIdx.x != 0) return;
@@ -631,6 +642,7 @@ __device__ __forceinline__ void end_round(TraverseState *state, int mark, int ro
     state->mark = mark;
     state->rounds = rounds;
     state->which = which;
+    if (hold >= 0) state->hold = hold;
 }
 
 // A work-group's part of the next list: vertices and their out-degrees gathered in LDS, appended with ONE atomic on the
@@ -703,7 +715,7 @@ __global__ __launch_bounds__(kSpmvBlock) void collect_frontier_kernel(int n, con
         __syncthreads();  // everyone has read it before anyone adds again
         if (full) s_buf.flush(lists.vertex[0], lists.offset[0], counters);
     }
-    end_round(state, next_mark, rounds, 0, counters, ticket);
+    end_round(state, next_mark, rounds, 0, counters, ticket, 0);
 }
 
 // One push round over a list: a work-group takes kChunk consecutive edges of the list's concatenated out-edges at a time,
@@ -1040,8 +1052,47 @@ __global__ void first_edges_kernel(int n, const int *__restrict__ index, const i
 constexpr int kSmallEdges = 4096, kSmallThreads = 1024;
 constexpr int kSmallSlots = 2 * kSmallEdges;  // of the hash table: at most half full
 constexpr size_t kSmallLds = sizeof(int) * (5 * kSmallEdges + 2 * kSmallSlots);
+constexpr int kNearEdges = 2048, kNearFrom = 64;  // of NearRounds
+static_assert(sizeof(int) * (8 * kNearEdges + 2 * kSmallSlots + kNearEdges / 2) <= kSmallLds, "NearRounds' arrays lie where SmallRounds' do");
 
 constexpr int kWarmBytes = 3 << 20;  // of the 4 MB of an XCD's L2
+constexpr int64_t kNearBytes = 3 << 20;
+constexpr int kFirstEdgesPer = 8;  // see ensure_first_edges
+
+// Inclusive sum over the wavefront's lanes, all of them active.
+__device__ __forceinline__ int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // from 1, 2, 4, 8 lanes below in the row of 16
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of the row below to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
+    return v;
+}
+// A place in a list in LDS for each lane that wants one, with one addition per wavefront: those of a round's lanes on one address are carried out one
+// after the other, which took most of the time of a round of some hundred edges.  All lanes take part.
+__device__ __forceinline__ int lanes_take(int *count, bool wants)
+{
+    const unsigned long long who = __ballot(wants);
+    if (who == 0) return 0;
+    int base = 0;
+    if ((threadIdx.x & (kWave - 1)) == 0) base = atomicAdd(count, __popcll(who));
+    base = __builtin_amdgcn_readfirstlane(base);
+    return base + __builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u));
+}
+// ... and for `degree` > 0 edges of it: place << 32 | first edge
+__device__ __forceinline__ unsigned long long lanes_take_edges(unsigned long long *listed, bool wants, int degree)
+{
+    const unsigned long long who = __ballot(wants);
+    if (who == 0) return 0;
+    const int mine = wants ? degree : 0, upto = wave_scan(mine);
+    unsigned long long base = 0;
+    if ((threadIdx.x & (kWave - 1)) == kWave - 1) base = atomicAdd(listed, ((unsigned long long)__popcll(who) << 32) + (unsigned long long)(unsigned)upto);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)base, kWave - 1), hi = __builtin_amdgcn_readlane((unsigned)(base >> 32), kWave - 1);
+    const unsigned place = hi + __builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u));
+    return ((unsigned long long)place << 32) + lo + (unsigned)(upto - mine);
+}
 
 struct LoneShared {
     int4 edge[kWave];  // {target or -1, edge, place of the value it starts from, -} of the next round's lanes
@@ -1174,17 +1225,6 @@ struct SmallRounds {
         }
     }
 
-    // Inclusive sum over the wavefront's lanes, all of them active.
-    static __device__ __forceinline__ int wave_scan(int v)
-    {
-        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // from 1, 2, 4, 8 lanes below in the row of 16
-        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of the row below to rows 1 and 3
-        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 to rows 2 and 3
-        return v;
-    }
     // Orders the lanes' accesses to LDS and memory, which the hardware carries out in a wavefront's program order.
     static __device__ __forceinline__ void lanes_meet()
     {
@@ -1226,6 +1266,8 @@ struct SmallRounds {
             pending = false;
         }
         lanes_meet();
+        // Where the loop's branches lie within 32 bytes decides 3 % of a hop (a 5 x 2,000 grid 1.84 ms at an offset of 0 or 4 bytes, 1.85 at 20, 1.89 at the others).
+        asm volatile(".p2align 6");
         for (;;) {
             Value old{};
             FirstEdges f{0, 0, {-1, -1, -1, -1}, {0, 0}};
@@ -1341,6 +1383,313 @@ struct SmallRounds {
     }
 };
 
+// Rounds of distances over natural lengths, inside one launch as SmallRounds', but nearest vertices first.  Rounds over all that was lowered lower
+// most vertices many times over: on a 23 x 846 grid with lengths 1 ... 16 they relax every edge 51 times, 3,600 a round.  Here a lowered vertex whose
+// distance is below a threshold goes on the list, the others wait; when the list is empty the threshold moves past the nearest of them (near and far
+// piles, as Davidson, Baxter, Garland and Owens, 2014, split delta-stepping's buckets), by a step that is doubled while lists are shorter than a quarter of the
+// lanes and halved when one is longer than the lanes: 1.4 times every edge, 100 a round.  Sums of whole numbers have the same least fixed point in any order, so the distances
+// are the same bits.  Every move of the threshold settles the nearest waiting vertex, as no length is negative: it ends.
+// A list that would be too long is cut, and what it leaves waits too.  A vertex with more edges than a list may have ends it: all go back on the
+// call's list, and the launch ends.  What bounds a round (2 us) is its chain of loads - target and length, then value, row bounds and flag - and two
+// barriers.  ms by rounds over all / this, lengths 1 ... 16: a 23 x 846 grid 9.8 / 2.4, 50 x 900 12.0 / 3.1, 100 x 500 7.1 / 2.5, 5 x 2,000 14.3 / 4.6, 12 x 200
+// 0.78 / 0.58, 200 x 300 4.7 / 3.6; where a lone wavefront suffices it stays with it (a path of 10,000 3.96 / 4.03).
+struct NearRounds {
+    int *s_start, *s_edge, *s_vertex, *s_val;           // the list
+    int *s_low, *s_slot, *s_low_edge, *s_low_degree;    // lowered vertices, and 2 * out-edges + whether they wait already
+    int *s_slot_vertex, *s_slot_val;                    // hash table of the round's targets, kSmallSlots
+    unsigned short *s_owner;                            // list entry of an edge of the list, if that entry's edges are few
+    unsigned long long *s_list;                         // [2] vertices << 32 | out-edges, of the current list and of the one being built, by turns
+    unsigned long long *s_cut;                          // [2] the first entry that found no room: its place << 32 | its first edge, or ~0
+    int *s_lows;                                        // [2]
+    int *s_fars, *s_fars_kept, *s_least, *s_most;       // s_fars: entries of `far`
+    const int *__restrict__ index;
+    const int *__restrict__ dst;
+    SsspPush push;
+    int *active;
+    int *far, *waits;                                   // device [n] each: waiting vertices, some no longer or again; waits[v]: v's valid place there + 1, or 0
+    int first_mark, n_all;
+
+    static __device__ __forceinline__ unsigned int hash(int v) { return ((unsigned int)v * 0x9E3779B1u) >> 19; }
+
+    // On the list that is being built, if there is room.  All lanes of the wavefront take part.
+    __device__ __forceinline__ bool append(int which, bool wants, int v, int edge, int degree, float value) const
+    {
+        const unsigned long long p = lanes_take_edges(&s_list[which], wants, degree);
+        if (!wants) return false;
+        const int i = (int)(p >> 32), start = (int)(p & 0xFFFFFFFFull);
+        if (i >= kNearEdges || start + degree > kNearEdges) {
+            atomicMin(&s_cut[which], p);
+            return false;
+        }
+        s_start[i] = start;
+        s_edge[i] = edge;
+        s_vertex[i] = v;
+        s_val[i] = order_of(value);
+        constexpr int kFew = 16;
+        if (degree <= kFew)
+            for (int k = 0; k < degree; ++k) s_owner[start + k] = (unsigned short)i;
+        return true;
+    }
+    __device__ __forceinline__ unsigned long long listed(int which) const { return s_cut[which] != ~0ull ? s_cut[which] : s_list[which]; }
+
+    // Of the first `fars` waiting places those that are valid: on the list that is being built if their distance is below the threshold and there is room, the others
+    // move down to the first *s_fars_kept places.  Begins and ends behind a barrier.
+    __device__ __forceinline__ void sift(int fars, int which, float threshold) const
+    {
+        for (int base = 0; base < fars; base += kSmallThreads) {
+            const int i = base + (int)threadIdx.x;
+            bool there = i < fars;
+            int v = 0, edge = 0, degree = 0;
+            float d = 0.0f;
+            if (there) {
+                v = far[i];
+                there = waits[v] == i + 1;
+                d = push.at(v);
+                edge = index[v];
+                degree = index[v + 1] - edge;
+            }
+            __syncthreads();  // these have been read: places below them may be written
+            const bool goes = append(which, there && d < threshold, v, edge, degree, d);
+            const int place = lanes_take(s_fars_kept, there && !goes);
+            if (there && !goes) far[place] = v;
+            if (there) waits[v] = goes ? 0 : place + 1;
+        }
+        __syncthreads();
+    }
+
+    // From a list in s_start ... s_val, s_list[0].  Returns the rounds done; the list and the waiting vertices are left in list, offset and *out.
+    __device__ __forceinline__ int run(int *list, int *offset, unsigned long long *out) const
+    {
+        constexpr int T = kSmallThreads, PER = kNearEdges / T;
+        const int tid = threadIdx.x;
+        float threshold = -1.0f, step = 0.0f;
+        int rounds = 0, flips = 0, longest = 0;  // flips: lists built
+        for (;;) {
+            const int now = flips & 1, next = now ^ 1;
+            const unsigned long long all = listed(now);
+            const int n = (int)(all >> 32), m = (int)(all & 0xFFFFFFFFull), fars = *s_fars;
+            if (n == 0 && fars == 0) break;
+            if (n > 0 && fars + m > n_all) {
+                // A place for each vertex that may come to wait: those that no longer hold are taken out, and what is left and comes are different vertices.
+                if (tid == 0) *s_fars_kept = 0;
+                __syncthreads();
+                sift(fars, next, -1.0f);
+                if (tid == 0) *s_fars = *s_fars_kept;
+                __syncthreads();
+            }
+            if (n > 0) {
+                longest = max(longest, m);
+                int t[PER], e[PER], r0[PER], r1[PER], waiting[PER];
+                float nv[PER], old[PER];
+#pragma unroll
+                for (int k = 0; k < PER; ++k) {
+                    const int j = tid + k * T;
+                    if (j < m) {
+                        int lo = s_owner[j] < n ? s_owner[j] : 0;
+                        if (!(s_start[lo] <= j && (lo + 1 < n ? s_start[lo + 1] : m) > j)) {  // the entry has many edges
+                            lo = 0;
+                            int hi = n;
+                            while (hi - lo > 1) {
+                                const int mid = (lo + hi) >> 1;
+                                if (s_start[mid] <= j) lo = mid; else hi = mid;
+                            }
+                        }
+                        e[k] = s_edge[lo] + (j - s_start[lo]);
+                        t[k] = dst[e[k]];
+                        nv[k] = push.relax(value_of_order(s_val[lo], 0.0f), e[k]);
+                    }
+                }
+                if (tid == 0) s_lows[next] = 0;
+#pragma unroll
+                for (int k = 0; k < PER; ++k)
+                    if (tid + k * T < m) {
+                        old[k] = push.at(t[k]);
+                        r0[k] = index[t[k]];
+                        r1[k] = index[t[k] + 1];
+                        waiting[k] = waits[t[k]];
+                    }
+#pragma unroll
+                for (int k = 0; k < PER; ++k) {
+                    if (k * T >= m) break;
+                    unsigned int slot = 0;
+                    bool first = false;  // edge to lower its target
+                    if (tid + k * T < m && nv[k] < old[k]) {
+                        slot = hash(t[k]);
+                        int found;
+                        while ((found = atomicCAS(&s_slot_vertex[slot], -1, t[k])) != -1 && found != t[k]) slot = (slot + 1) & (kSmallSlots - 1);
+                        first = found == -1;
+                        atomicMin(&s_slot_val[slot], order_of(nv[k]));
+                    }
+                    const int i = lanes_take(&s_lows[now], first);
+                    if (first) {
+                        s_low[i] = t[k];
+                        s_slot[i] = (int)slot;
+                        s_low_edge[i] = r0[k];
+                        s_low_degree[i] = 2 * (r1[k] - r0[k]) + (waiting[k] != 0);
+                    }
+                }
+                __syncthreads();  // the list has been read, the lowered vertices are complete
+                const int lows = s_lows[now];
+                if (tid == 0) {
+                    s_list[now] = 0ull;
+                    s_cut[now] = ~0ull;
+                }
+                for (int base = 0; base < lows; base += T) {
+                    const int i = base + tid;
+                    int v = 0, degree = 0, edge = 0;
+                    bool waited = false;
+                    float value = 0.0f;
+                    if (i < lows) {
+                        const int slot = s_slot[i];
+                        v = s_low[i];
+                        edge = s_low_edge[i];
+                        degree = s_low_degree[i] >> 1;
+                        waited = s_low_degree[i] & 1;
+                        value = value_of_order(s_slot_val[slot], 0.0f);
+                        s_slot_val[slot] = INT_MAX;
+                        s_slot_vertex[slot] = -1;
+                        push.store(v, value);
+                        active[v] = first_mark + rounds;
+                    }
+                    const bool goes = append(next, degree > 0 && value < threshold, v, edge, degree, value);
+                    if (goes && waited) waits[v] = 0;
+                    const bool stays = degree > 0 && !goes && !waited;
+                    const int place = lanes_take(s_fars, stays);
+                    if (stays) {
+                        waits[v] = place + 1;
+                        far[place] = v;
+                    }
+                }
+                ++rounds;
+                ++flips;
+                __syncthreads();
+                continue;
+            }
+            // The threshold moves on.
+            if (tid == 0) {
+                *s_least = INT_MAX;
+                *s_most = INT_MIN;
+                *s_fars_kept = 0;
+                s_list[next] = 0ull;
+                s_cut[next] = ~0ull;
+                s_lows[next] = 0;
+            }
+            __syncthreads();
+            for (int i = tid; i < fars; i += T) {
+                const int v = far[i];
+                if (waits[v] != i + 1) continue;
+                const int d = order_of(push.at(v));
+                atomicMin(s_least, d);
+                atomicMax(s_most, d);
+            }
+            __syncthreads();
+            const float least = value_of_order(*s_least, 0.0f), most = value_of_order(*s_most, 0.0f);
+            step = step == 0.0f ? most - least : longest * 4 < T ? 2.0f * step : longest > T ? 0.5f * step : step;
+            step = fmaxf(step, 1.0f);
+            longest = 0;
+            threshold = least + step;
+            if (!(threshold > least)) threshold = nextafterf(least, INFINITY);
+            sift(fars, next, threshold);
+            const bool stuck = (listed(next) >> 32) == 0 && *s_fars_kept > 0;
+            if (tid == 0) *s_fars = *s_fars_kept;
+            ++flips;
+            __syncthreads();
+            if (stuck) break;
+        }
+        // What is left goes back.
+        const unsigned long long all = listed(flips & 1);
+        const int n = (int)(all >> 32), fars = *s_fars;
+        if (tid == 0) *out = all;
+        __syncthreads();
+        for (int i = tid; i < n; i += T) {
+            list[i] = s_vertex[i];
+            offset[i] = s_start[i];
+        }
+        for (int i = tid; i < fars; i += T) {
+            const int v = far[i];
+            if (waits[v] != i + 1) continue;
+            const unsigned long long p = atomicAdd(out, (1ull << 32) + (unsigned long long)(unsigned int)(index[v + 1] - index[v]));
+            list[p >> 32] = v;
+            offset[p >> 32] = (int)(p & 0xFFFFFFFFull);
+        }
+        __syncthreads();
+        return rounds;
+    }
+};
+
+// A list of any length: all of it waits at first.  One work-group.
+__global__ __launch_bounds__(kSmallThreads) void near_rounds_kernel(TraverseState *state, Lists lists, const int *__restrict__ index,
+                                                                   const int *__restrict__ dst, SsspPush push, int *active, int n_all)
+{
+    extern __shared__ int s_small[];
+    __shared__ unsigned long long s_list[2], s_cut[2], s_out;
+    __shared__ int s_lows[2], s_fars, s_fars_kept, s_least, s_most;
+    const TraverseState start = *state;
+    const int tid = threadIdx.x;
+    if (start.listed == 0 || start.hold <= 0 || start.rounds < n_all + 2 - start.hold) return;
+    if ((start.listed & 0xFFFFFFFFull) <= (unsigned long long)kWave) {  // a lone wavefront's: to be looked at when as many rounds more have run
+        if (tid == 0) state->hold = max(n_all + 2 - 4 * start.rounds, 0);
+        return;
+    }
+    int *list = lists.vertex[start.which & 1], *offset = lists.offset[start.which & 1];
+    int *at = s_small;
+    const auto take = [&](int words) { int *p = at; at += words; return p; };
+    NearRounds nr;
+    nr.s_start = take(kNearEdges);
+    nr.s_edge = take(kNearEdges);
+    nr.s_vertex = take(kNearEdges);
+    nr.s_val = take(kNearEdges);
+    nr.s_low = take(kNearEdges);
+    nr.s_slot = take(kNearEdges);
+    nr.s_low_edge = take(kNearEdges);
+    nr.s_low_degree = take(kNearEdges);
+    nr.s_slot_vertex = take(kSmallSlots);
+    nr.s_slot_val = take(kSmallSlots);
+    nr.s_owner = reinterpret_cast<unsigned short *>(take(kNearEdges / 2));
+    nr.s_list = s_list;
+    nr.s_cut = s_cut;
+    nr.s_lows = s_lows;
+    nr.s_fars = &s_fars;
+    nr.s_fars_kept = &s_fars_kept;
+    nr.s_least = &s_least;
+    nr.s_most = &s_most;
+    nr.index = index;
+    nr.dst = dst;
+    nr.push = push;
+    nr.active = active;
+    nr.far = lists.vertex[(start.which & 1) ^ 1];
+    nr.waits = lists.offset[(start.which & 1) ^ 1];
+    nr.first_mark = start.mark;
+    nr.n_all = n_all;
+    const int n = (int)(start.listed >> 32);
+    for (int v = tid; v < n_all; v += kSmallThreads) nr.waits[v] = 0;
+    for (int j = tid; j < kNearEdges; j += kSmallThreads) nr.s_owner[j] = 0xFFFF;
+    for (int i = tid; i < kSmallSlots; i += kSmallThreads) {
+        nr.s_slot_vertex[i] = -1;
+        nr.s_slot_val[i] = INT_MAX;
+    }
+    if (tid == 0) {
+        s_list[0] = s_list[1] = 0ull;
+        s_cut[0] = s_cut[1] = ~0ull;
+        s_lows[0] = s_lows[1] = 0;
+        s_fars = n;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kSmallThreads) {  // all of them wait
+        const int v = list[i];
+        nr.far[i] = v;
+        nr.waits[v] = i + 1;
+    }
+    __syncthreads();
+    const int rounds = nr.run(list, offset, &s_out);
+    if (tid == 0) {
+        state->listed = s_out;
+        state->mark = start.mark + rounds;
+        state->rounds = min(start.rounds + rounds, n_all);  // no cycle of negative length, however many they were
+        state->hold = 0;                                    // whatever is left is the other rounds'
+    }
+}
+
 template <typename Push>
 __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(TraverseState *state, Lists lists, const int *__restrict__ index,
                                                                          const int *__restrict__ dst, const FirstEdges *__restrict__ first,
@@ -1371,7 +1720,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
     const TraverseState start = *state;
     if ((start.listed & 0xFFFFFFFFull) > (unsigned long long)kSmallEdges || start.listed == 0) return;
     const int count = (int)(start.listed >> 32), edges = (int)(start.listed & 0xFFFFFFFFull), mark = start.mark;
-    const int max_rounds = n_all + 2 - start.rounds;  // the host tells a cycle of negative length by n + 2
+    const int max_rounds = n_all + 2 - start.hold - start.rounds;  // the host tells a cycle of negative length by n + 2
     int *list = lists.vertex[start.which & 1], *offset = lists.offset[start.which & 1];
     sr.first_mark = mark;
     for (int i = tid; i < kSmallSlots; i += kSmallThreads) {
@@ -1436,7 +1785,7 @@ __global__ __launch_bounds__(kSmallThreads) void push_rounds_small_kernel(Traver
 void allow_small_lds()
 {
     for (const void *kernel : {reinterpret_cast<const void *>(&push_rounds_small_kernel<CcPush>),
-                               reinterpret_cast<const void *>(&push_rounds_small_kernel<SsspPush>)})
+                               reinterpret_cast<const void *>(&push_rounds_small_kernel<SsspPush>), reinterpret_cast<const void *>(&near_rounds_kernel)})
         DRONE_HIP_OR_DIE(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
 }
 
@@ -1465,6 +1814,16 @@ void launch_pull(Graph *g, TraverseExt *t, Pull pull, hipStream_t s)
     GraphExt *x = static_cast<GraphExt *>(g->ext);
     pull_open_kernel<Pull><<<(unsigned)std::min<int64_t>(ceil_div(x->n, kPullThreads), kPullBlocks), kPullThreads, 0, s>>>(
         t->state, push_limit(x), x->n, x->in_index, x->in_src, pull, g->active, g->index, t->lists, t->counters, t->ticket);
+}
+
+// TraverseState::hold for natural lengths: where rounds of the nearest vertices pay.  For lists that reach a hundred edges or so at a time for hundreds of rounds, on roads
+// and grids: at most kFirstEdgesPer edges a vertex, and kNearFrom rounds gone by (a graph with hubs is done after a few tens; 3,000 vertices and 18,000 edges
+// 85 -> 221 us from the first round on).  And what a round's targets need - values, flags, row bounds, edges, lengths - within an XCD's L2: beyond,
+// one CU waits for each of them (ms before / with them: 100 x 500 7.1 / 2.4, 200 x 300 4.7 / 3.6, but 300 x 400 7.3 / 8.1, 1,000 x 1,000 30 / 93).
+int near_hold(const GraphExt *x)
+{
+    const bool pays = (int64_t)x->edges <= (int64_t)kFirstEdgesPer * x->n && 8ll * x->edges + 12ll * x->n <= kNearBytes;
+    return pays ? std::max(x->n + 2 - kNearFrom, 0) : 0;
 }
 
 // Runs rounds until nothing changes, from what *t->state says is left to propagate (`now`, if known).  What it takes of `run`:
@@ -1515,6 +1874,13 @@ int run_to_fixed_point(Graph *g, TraverseExt *t, Run &run, TraverseState now, bo
             if constexpr (Run::kSweeps) return run.can_pull(now);
             else return true;
         };
+        if constexpr (Run::kSweeps)
+            if (known && now.hold > 0 && now.rounds >= n + 2 - now.hold) {
+                for (int i = 0; i < 3; ++i) {  // they take turns while a lone wavefront suffices
+                    if (i > 0) small();
+                    near_rounds_kernel<<<1, kSmallThreads, kSmallLds, s>>>(t->state, t->lists, g->index, g->dst, run.push, g->active, n);
+                }
+            }
         if (!known || edges <= (unsigned long long)kSmallEdges) {
             small();
             push(1);
@@ -1706,7 +2072,6 @@ void exchange_values(Graph *g, T *vals, int **send_id, int **recv_id, T **send_v
 // 0.49 / 0.72 / 0.78 us instead of 0.40 / 0.53 / 0.54; lists too long for a lone wavefront do not read them.  They are made
 // before the first launch, which often runs all the rounds there are; 256 MB (8 Mi vertices) is the Infinity Cache, beyond
 // which the one access goes to HBM.
-constexpr int kFirstEdgesPer = 8;
 constexpr int64_t kFirstEdgesMost = 256 << 20;
 void ensure_first_edges(Graph *g, hipStream_t s)
 {
@@ -1897,7 +2262,7 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
     const auto begin = [&] {
         sssp_begin_kernel<<<std::max(sum_blocks(n), sum_blocks(x->edges, 16)), kSpmvBlock, 0, s>>>(
             n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage, g->index, t->lists.vertex[0], t->lists.offset[0], x->edges,
-            g->edgeLen, t->block_part, t->ticket, t->state);
+            g->edgeLen, t->block_part, t->ticket, t->state, near_hold(x));
         run.counted = true;
     };
     const bool chains = ensure_chains(g, t, s) && !x->chains.other_lengths;

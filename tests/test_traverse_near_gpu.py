@@ -1,0 +1,59 @@
+"""Distances over natural lengths by rounds of the nearest vertices first (NearRounds), where its lists, thresholds and waiting vertices are at their
+limits: grids, a vertex with more edges than a list may have, one with just as many, more waiting vertices than there is room for, lists that are cut,
+lengths of zero and near 2^24 (distances that round and that pass the unreached one), and lengths below zero, which take the other rounds.
+They begin after 64 rounds.  Against the oracle, exactly: sums of whole numbers in float have one least fixed point, in whatever order they are made."""
+import numpy as np
+import pytest
+
+from test_traverse_rounds_gpu import _layers
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(w, h):
+    at = np.arange(w * h).reshape(h, w)
+    s = np.concatenate([at[:-1].ravel(), at[:, :-1].ravel()])
+    d = np.concatenate([at[1:].ravel(), at[:, 1:].ravel()])
+    return np.concatenate([s, d]).astype(np.int32), np.concatenate([d, s]).astype(np.int32)
+
+
+def _hub(before, edges, tail):
+    """A path to a vertex with `edges` out-edges, each leading to a path of `tail` vertices."""
+    ends = before + 1 + np.arange(edges)[:, None] + edges * np.arange(tail)[None, :]
+    u = np.concatenate([np.arange(before), np.full(edges, before), ends[:, :-1].ravel()])
+    v = np.concatenate([np.arange(1, before + 1), ends[:, 0], ends[:, 1:].ravel()])
+    return u.astype(np.int32), v.astype(np.int32)
+
+
+CASES = {
+    "grid_3": (lambda: _grid(3, 300), 1, 17), "grid_23": (lambda: _grid(23, 211), 1, 17), "grid_120": (lambda: _grid(120, 130), 1, 17),
+    "grid_600": (lambda: _grid(600, 60), 1, 17),           # lists that are cut
+    "ones_and_two": (lambda: _grid(40, 50), 1, 3), "zeros": (lambda: _grid(31, 57), 0, 4), "far": (lambda: _grid(17, 40), 1, 1 << 24),
+    "hub_2048": (lambda: _hub(99, 2048, 3), 1, 5), "hub_2049": (lambda: _hub(99, 2049, 3), 1, 5), "hub_late": (lambda: _hub(700, 3000, 2), 1, 5),
+    "waiting": (lambda: _layers([1] * 70 + [500, 2047, 4000, 4100, 300, 2], 1, 3), 1, 400), "waiting_more": (lambda: _layers([1] * 70 + [60, 1900, 3900, 3900, 40], 2, 8), 1, 60),
+    "places": (lambda: _layers([1] * 70 + [40, 900, 1000, 1000, 900, 900] + [30, 900, 1000, 600] * 3, 3, 9), 1, 17),  # more entries than vertices, but for the sifting
+    "negative": (lambda: _layers([1] * 70 + [30, 300, 300, 50, 2], 2, 4), -3, 9), "path": (lambda: (np.arange(3000, dtype=np.int32), np.arange(1, 3001, dtype=np.int32)), 1, 9),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_nearest_first(oracle, name):
+    from drone_amd.traverse import SSSPWorkerCUDA
+    make, low, high = CASES[name]
+    u, v = make()
+    nglobal = int(max(u.max(), v.max())) + 1
+    n, g2l, l2g, index, dst = oracle.build_graph(nglobal, u, v)
+    length = np.random.default_rng(len(u)).integers(low, high, len(dst)).astype(np.float32)
+    if name == "waiting":
+        length[::7] = 1.0
+    st = oracle.SSSPState(index, dst, length)
+    st.peval(int(g2l[0]))
+    w = SSSPWorkerCUDA(nglobal, u, v, startId=0)
+    try:
+        w.set_edge_len(length)
+        for _ in range(2):
+            assert w.peval().VisitedSize == st.visited()
+            np.testing.assert_array_equal(w.read(), st.val)
+            np.testing.assert_array_equal(np.sign(w.flags()["active"]), np.sign(st.active))
+    finally:
+        w.close()
