@@ -1226,6 +1226,25 @@ __global__ __launch_bounds__(256) void check_scaled_values_kernel(int n_rows, co
     if (bad) atomicAdd(mismatches, bad);
 }
 
+// Where the rows of a chunk begin, a wavefront per chunk and a lane per row.  (Made on the host, two million short rows took 7 ms of a plan's 35.)
+__global__ __launch_bounds__(kWave * kRowsPerBlock) void chunk_rows_kernel(int num_chunks, const int4 *__restrict__ chunk, const int *__restrict__ rp,
+                                                                         ChunkRows *__restrict__ out)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int c = blockIdx.x * kRowsPerBlock + threadIdx.x / kWave; c < num_chunks; c += gridDim.x * kRowsPerBlock) {
+        const int4 d = chunk[c];  // {first row, row past the last, first entry, entry past the last}
+        unsigned long long head = 0;
+        if (d.w - d.z <= kWave && lane < d.y - d.x) {  // a longer chunk is a row of its own, which needs no bits
+            const int start = rp[d.x + lane] - d.z, end = rp[d.x + lane + 1] - d.z;
+            if (end > start) head = 1ull << start;
+        }
+        const unsigned long long some = __ballot(head != 0);
+#pragma unroll
+        for (int m = kWave / 2; m > 0; m >>= 1) head |= __shfl_xor(head, m, kWave);
+        if (lane == 0) out[c] = ChunkRows{head, some};
+    }
+}
+
 int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, const int *rp, const int *ci, const float *v,
                 const float *row_scale, const float *col_scale, int max_k, hipStream_t s)
 {
@@ -1243,17 +1262,11 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
     }
     // chunks of the short rows
     std::vector<int4> h_chunk;
-    std::vector<ChunkRows> h_chunk_rows;
     const int most = chunk_entries(n_rows, nnz);
     {
         int first = -1, entries = 0;
-        ChunkRows open{};
         const auto close = [&](int end) {
-            if (first >= 0) {
-                h_chunk.push_back(make_int4(first, end, h_rp[first], h_rp[end]));
-                h_chunk_rows.push_back(open);
-            }
-            open = ChunkRows{};
+            if (first >= 0) h_chunk.push_back(make_int4(first, end, h_rp[first], h_rp[end]));
             first = -1;
             entries = 0;
         };
@@ -1264,14 +1277,9 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
             } else if (len > kWave) {  // more than one load of pairs: a chunk of its own
                 close(r);
                 h_chunk.push_back(make_int4(r, r + 1, h_rp[r], h_rp[r + 1]));
-                h_chunk_rows.push_back(ChunkRows{});
             } else {
                 if (first >= 0 && (entries + len > most || r - first >= kWave - 1)) close(r);
                 if (first < 0) first = r;
-                if (len > 0) {
-                    open.heads |= 1ull << entries;
-                    open.some |= 1ull << (r - first);
-                }
                 entries += len;
             }
         }
@@ -1305,8 +1313,10 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
             const auto upload = [&]() -> int {
                 DRONE_HIP_TRY(hipMalloc(&p->chunk, sizeof(int4) * h_chunk.size()));
                 DRONE_HIP_TRY(hipMemcpy(p->chunk, h_chunk.data(), sizeof(int4) * h_chunk.size(), hipMemcpyHostToDevice));
-                DRONE_HIP_TRY(hipMalloc(&p->chunk_rows, sizeof(ChunkRows) * h_chunk_rows.size()));
-                DRONE_HIP_TRY(hipMemcpy(p->chunk_rows, h_chunk_rows.data(), sizeof(ChunkRows) * h_chunk_rows.size(), hipMemcpyHostToDevice));
+                DRONE_HIP_TRY(hipMalloc(&p->chunk_rows, sizeof(ChunkRows) * h_chunk.size()));
+                chunk_rows_kernel<<<(unsigned)std::min<int64_t>(ceil_div(p->num_chunks, kRowsPerBlock), 4096), kWave * kRowsPerBlock, 0, s>>>(
+                    p->num_chunks, p->chunk, rp, p->chunk_rows);
+                DRONE_HIP_TRY(hipGetLastError());
                 return DRONE_OK;
             };
             const int urc = upload();
