@@ -1389,8 +1389,8 @@ struct SmallRounds {
 // piles, as Davidson, Baxter, Garland and Owens, 2014, split delta-stepping's buckets), by a step that is doubled while lists are shorter than a quarter of the
 // lanes and halved when one is longer than the lanes: 1.4 times every edge, 100 a round.  Sums of whole numbers have the same least fixed point in any order, so the distances
 // are the same bits.  Every move of the threshold settles the nearest waiting vertex, as no length is negative: it ends.
-// A list that would be too long is cut, and what it leaves waits too.  A vertex with more edges than a list may have ends it: all go back on the
-// call's list, and the launch ends.  What bounds a round (2 us) is its chain of loads - target and length, then value, row bounds and flag - and two
+// A list that would be too long is cut, and what it leaves waits too.  A vertex with more edges than a list may have ends it, and so do n rounds: all go
+// back on the call's list, and the launch ends.  What bounds a round (2 us) is its chain of loads - target and length, then value, row bounds and flag - and two
 // barriers.  ms by rounds over all / this, lengths 1 ... 16: a 23 x 846 grid 9.8 / 2.4, 50 x 900 12.0 / 3.1, 100 x 500 7.1 / 2.5, 5 x 2,000 14.3 / 4.6, 12 x 200
 // 0.78 / 0.58, 200 x 300 4.7 / 3.6; where a lone wavefront suffices it stays with it (a path of 10,000 3.96 / 4.03).
 struct NearRounds {
@@ -1468,7 +1468,7 @@ struct NearRounds {
             const int now = flips & 1, next = now ^ 1;
             const unsigned long long all = listed(now);
             const int n = (int)(all >> 32), m = (int)(all & 0xFFFFFFFFull), fars = *s_fars;
-            if (n == 0 && fars == 0) break;
+            if ((n == 0 && fars == 0) || rounds >= n_all) break;
             if (n > 0 && fars + m > n_all) {
                 // A place for each vertex that may come to wait: those that no longer hold are taken out, and what is left and comes are different vertices.
                 if (tid == 0) *s_fars_kept = 0;
@@ -1685,8 +1685,9 @@ __global__ __launch_bounds__(kSmallThreads) void near_rounds_kernel(TraverseStat
     if (tid == 0) {
         state->listed = s_out;
         state->mark = start.mark + rounds;
-        state->rounds = min(start.rounds + rounds, n_all);  // no cycle of negative length, however many they were
-        state->hold = 0;                                    // whatever is left is the other rounds'
+        // Whatever is left is the other rounds', which have n to go from any distances: no length is negative, so a call may make more than n + 1 in all.
+        state->rounds = s_out == 0ull ? min(start.rounds + rounds, n_all) : 0;
+        state->hold = 0;
     }
 }
 

@@ -25,6 +25,44 @@ def _hub(before, edges, tail):
     return u.astype(np.int32), v.astype(np.int32)
 
 
+def _detour(edges, tail):
+    """A path to a fan of 100; one of the fan leads to a path of `tail` vertices by a long edge, and by two short ones through a vertex with `edges` out-edges, which finds no room on a list beside the path's first."""
+    fan, hub, leaf = 64 + np.arange(100), 164, 165 + np.arange(edges - 1)
+    path = 165 + edges - 1 + np.arange(tail + 1)
+    u = np.concatenate([np.arange(63), np.full(100, 63), [64], fan, [hub], np.full(edges - 1, hub), path[:-1]])
+    v = np.concatenate([np.arange(1, 64), fan, [path[0]], np.where(fan == 64, hub, 0), [path[0]], leaf, path[1:]])
+    return u.astype(np.int32), v.astype(np.int32)
+
+
+def _detour_lengths(n, g2l, l2g, index, dst):
+    length = np.ones(len(dst), np.float32)
+    at = lambda u, v: [e for e in range(index[g2l[u]], index[g2l[u] + 1]) if l2g[dst[e]] == v]
+    head = max(l2g[dst[e]] for e in range(index[g2l[64]], index[g2l[64] + 1]))
+    length[at(64, head)] = 100.0
+    length[at(63, 65)] = 1 << 20  # the first threshold lies beyond the path
+    return length
+
+
+@pytest.mark.parametrize("edges", [2048, 2100])
+def test_long_path_lowered_twice(oracle, edges):
+    """More rounds than there are vertices, some by the nearest vertices first and some not: no cycle of negative length."""
+    from drone_amd.traverse import SSSPWorkerCUDA
+    u, v = _detour(edges, 5000)
+    nglobal = int(max(u.max(), v.max())) + 1
+    n, g2l, l2g, index, dst = oracle.build_graph(nglobal, u, v)
+    length = _detour_lengths(n, g2l, l2g, index, dst)
+    st = oracle.SSSPState(index, dst, length)
+    st.peval(int(g2l[0]))
+    assert st.val[g2l[nglobal - 1]] == 63 + 1 + 1 + 1 + 5000
+    w = SSSPWorkerCUDA(nglobal, u, v, startId=0)
+    try:
+        w.set_edge_len(length)
+        assert w.peval().VisitedSize == st.visited()
+        np.testing.assert_array_equal(w.read(), st.val)
+    finally:
+        w.close()
+
+
 CASES = {
     "grid_3": (lambda: _grid(3, 300), 1, 17), "grid_23": (lambda: _grid(23, 211), 1, 17), "grid_120": (lambda: _grid(120, 130), 1, 17),
     "grid_600": (lambda: _grid(600, 60), 1, 17),           # lists that are cut
