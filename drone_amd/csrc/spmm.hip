@@ -1335,12 +1335,15 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
             rc = copy();
         }
         if (rc == DRONE_OK && !long_row.empty()) rc = build_band_pieces(p, h_rp, long_row, rp, ci, v, s, &duplicates);
-        if (rc == DRONE_OK && !duplicates) {
+        // A plan is whole when it is handed out, for products on any stream, and the caller's arrays have been read.
+        const hipError_t whole = rc == DRONE_OK && !duplicates ? hipStreamSynchronize(s) : hipSuccess;
+        if (rc == DRONE_OK && !duplicates && whole == hipSuccess) {
             *out = p;
             return DRONE_OK;
         }
         drone_spmm_plan_destroy(p);
         if (rc != DRONE_OK) return rc;
+        DRONE_HIP_TRY(whole);
         scaled = false;  // a multigraph: cells with several entries need the fp32 rectangles
     }
     return DRONE_OK;  // not reached: the unscaled build reports no duplicates

@@ -46,3 +46,29 @@ def test_chunks(name, lengths):
             assert np.all(np.abs(got[:, :K] - (alpha * want + before)) <= bound), (K, beta)
             assert np.array_equal(got[:, K:], C0[:, K:]), (K, beta)
         plan.close()
+
+
+@pytest.mark.parametrize("longest", [3, 1_500])
+def test_plan_is_whole_when_it_is_handed_out(longest):
+    """Nothing of a plan is still being made on its stream when the call returns, with and without long rows: products may be on any other."""
+    import torch
+    from drone_amd import gcn
+    n, K = 2_000_003, 8
+    lengths = torch.arange(n, device="cuda", dtype=torch.int32) % 3
+    lengths[n // 2] = longest
+    rp = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    rp[1:] = torch.cumsum(lengths, 0)
+    nnz = int(rp[-1])
+    ci = (torch.arange(nnz, device="cuda") * 7919 % 1_000).to(torch.int32)
+    val = (torch.arange(nnz, device="cuda") % 5 + 1).float()
+    H = (torch.arange(1_000 * K, device="cuda").reshape(1_000, K) % 11).float()
+    # whole numbers far below 2^24: exact in any order
+    want = torch.zeros(n, K, device="cuda").index_add_(0, torch.repeat_interleave(torch.arange(n, device="cuda"), lengths), val[:, None] * H[ci.long()])
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        plan = gcn.SpmmPlan(rp, ci, val, 1_000, K, stream=side.cuda_stream)
+        assert side.query()
+        got = gcn.spmm(plan, rp, ci, val, H)
+        assert torch.equal(got, want)
+        plan.close()
