@@ -62,6 +62,7 @@ struct drone_spmm_plan {
     int max_k = 0;
     // short rows in chunks: consecutive rows of at most 64 entries together (or one row of any length up to the split)
     int num_chunks = 0;
+    int longest = 0;        // entries of the longest row among them
     int4 *chunk = nullptr;  // device [num_chunks]: {first row, last + 1, first entry, last + 1}
     drone::ChunkRows *chunk_rows = nullptr;  // device [num_chunks]
     // long rows, cut into band pieces
@@ -225,6 +226,14 @@ struct WavePairs {
 // wavefront has few, and four of narrow ones, where eight cost more registers than they bring.  us with 8 / 4: 30,011 vertices at K = 100 28.4 / 31.4,
 // at K = 23 14.8 / 12.5; 300,007 at K = 32 62.9 / 53.4; 71,791 at K = 62 31.5 / 33.1.
 constexpr int gather_rows(int lanes) { return lanes >= 16 ? 8 : 4; }
+// But a row that is not split is one wavefront's chain of steps, for which a launch that the GPU holds at once waits: where the longest has this many
+// entries, lane groups of 8 in sliced launches have eight in flight too, a step of 64 entries instead of 32 (then without a batch of pairs ahead, which would spill).  us a
+// product with 4 / 8 by the longest row: 234 (12,007 rows at K = 37) 6.80 / 7.23, 284 (9,001 at K = 100) 6.96 / 7.26, 317 (16,001 at K = 37) 8.51 / 9.22, 324 (14,009)
+// 7.93 / 7.75, 340 (12,007 of twice the entries) 8.04 / 7.38, 384 (7,001 at K = 100) 8.68 / 7.54, 417 (20,011 at K = 37) 8.18 / 7.62, 511 (10,411) 8.83 / 7.38.  (Unsliced ones have several times the entries:
+// 30,011 vertices at K = 23, whose longest has 380, in a training step of 199 / 204.)
+// In the launch of chunks alone it is wide groups that gain by eight: rows of 400 entries, 8,009 of them, at K = 100 61.1 / 58.1, at K = 37 32.6 / 31.8; 2,000 at K = 100,
+// lane groups of 8, 23.2 / 23.7; of 100 entries, 4,001 at K = 37 6.8 / 7.3.
+constexpr int kDeepRow = 340;
 
 // Accumulates sum_e val[e] * B[col[e], cols.at .. cols.at+VEC) for e in [e0, e1) into acc (per lane), then
 // folds the P lane groups together so that group 0 holds the totals.  MOST: feature-row loads in flight per lane group.  With `pairs`
@@ -255,7 +264,7 @@ __device__ __forceinline__ void row_segment(WavePairs *pairs, int e0, int e1, co
         c_next = e < e1 ? ci[e] : 0;
         a_next = e < e1 ? val[e] : 0.0f;
     };
-    const bool ahead = pairs && G < 16;
+    const bool ahead = pairs && G < 16 && MOST < 8;
     if (ahead) fetch(e0);
     for (int base = e0; base < e1; base += kWave) {
         if (!ahead) fetch(base);
@@ -467,7 +476,7 @@ struct JoinRows {
     const int *__restrict__ first_slot;
     unsigned *ticket;
 };
-template <int G, int VEC>
+template <int G, int VEC, int MOST>
 __device__ __forceinline__ void join_piece(WavePairs &pairs, int block, int slice, int slices, int num_pieces, const int *__restrict__ piece_begin,
                                            const int *__restrict__ piece_end, const int *__restrict__ piece_slot,
                                            const int *__restrict__ ci, const float *__restrict__ val,
@@ -483,7 +492,7 @@ __device__ __forceinline__ void join_piece(WavePairs &pairs, int block, int slic
     for (int k0 = slice * G * VEC; k0 < K; k0 += slices * G * VEC) {
         const LaneColumns<VEC> cols{k0 + li * VEC, K};
         float acc[VEC];
-        row_segment<G, VEC, gather_rows(G)>(&pairs, piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
+        row_segment<G, VEC, MOST>(&pairs, piece_begin[s], piece_end[s], ci, val, B, ldb, cols, acc);
         if (sub == 0 && cols.active()) {
             float *mine = partial + (size_t)piece_slot[s] * ldp + cols.at();
             unsigned before[VEC];
@@ -534,22 +543,22 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock, G == 8 ? 6 : 8) void spmm_pi
     sum_piece<G, VEC, 8>(nullptr, blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_pieces, piece_begin, piece_end, piece_slot, ci, val, B, ldb, partial, ldp, K);
 }
 
-template <int G, int VEC>
+template <int G, int VEC, int MOST>
 __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_chunks_kernel(
     int num_chunks, const int4 *__restrict__ chunk, const ChunkRows *__restrict__ chunk_rows, RowSums to, const int *__restrict__ ci,
     const float *__restrict__ val, const float *__restrict__ B, int ldb, int K, int slice_bits)
 {
     __shared__ WavePairs s_pairs[kRowsPerBlock];
     const int slices = 1 << slice_bits;
-    sum_chunk<G, VEC, 4>(s_pairs[threadIdx.x / kWave], blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
+    sum_chunk<G, VEC, MOST>(s_pairs[threadIdx.x / kWave], blockIdx.x >> slice_bits, blockIdx.x & (slices - 1), slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
 }
 
 // Both in one launch, the pieces first: the chunks fill the GPU while the last pieces end, and a launch is saved.  us
 // against one launch each: training step on 30,011 vertices 280 / 263, 20 K vertices and 0.3 M entries at K = 128 74 / 57,
 // 1 M vertices and 15 M entries at K = 41 678 / 619, forward and backward over a vertex cut 757 / 715.  Not beside a bit
 // core, where a launch costs nothing and the product of 3 M vertices at K = 64 took 2,369 / 2,442.
-template <int G, int VEC, bool JOIN>
-__global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_gather_kernel(
+template <int G, int VEC, int MOST, bool JOIN>
+__global__ __launch_bounds__(kWave * kRowsPerBlock, G == 8 && MOST == 8 ? 6 : 7) void spmm_gather_kernel(
     int num_pieces, int piece_blocks, const int *__restrict__ piece_begin, const int *__restrict__ piece_end,
     const int *__restrict__ piece_slot, const int *__restrict__ ci2, const float *__restrict__ val2,
     float *partial, int ldp, JoinRows join, int num_chunks, const int4 *__restrict__ chunk, const ChunkRows *__restrict__ chunk_rows,
@@ -560,11 +569,11 @@ __global__ __launch_bounds__(kWave * kRowsPerBlock, 7) void spmm_gather_kernel(
     const int slices = 1 << slice_bits, block = blockIdx.x >> slice_bits, slice = blockIdx.x & (slices - 1);
     if (block < piece_blocks) {
         if constexpr (JOIN)
-            join_piece<G, VEC>(pairs, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K, join, to);
+            join_piece<G, VEC, MOST>(pairs, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K, join, to);
         else
-            sum_piece<G, VEC, gather_rows(G)>(nullptr, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
+            sum_piece<G, VEC, MOST>(nullptr, block, slice, slices, num_pieces, piece_begin, piece_end, piece_slot, ci2, val2, B, ldb, partial, ldp, K);
     } else {
-        sum_chunk<G, VEC, gather_rows(G)>(pairs, block - piece_blocks, slice, slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
+        sum_chunk<G, VEC, MOST>(pairs, block - piece_blocks, slice, slices, num_chunks, chunk, chunk_rows, to, ci, val, B, ldb, K);
     }
 }
 
@@ -855,12 +864,14 @@ __global__ void gather_sorted_kernel(int64_t count, const unsigned *__restrict__
     }
 }
 
-template <int G, int VEC>
+// DEEP: see kDeepRow.
+template <int G, int VEC, bool DEEP>
 void launch_spmm(const drone_spmm_plan *plan, const int *ci, const float *v, const float *B, int ldb,
                  float *C, int ldc, int K, float alpha, float beta, int slice_bits, hipStream_t s)
 {
     const int piece_blocks = (int)ceil_div(plan->num_pieces, kRowsPerBlock), chunk_blocks = (int)ceil_div(plan->num_chunks, kRowsPerBlock);
     const RowSums rows{C, ldc, alpha, beta};
+    constexpr int kMost = DEEP ? 8 : gather_rows(G);
     if (piece_blocks > 0 && chunk_blocks > 0 && plan->bits.tiles == 0) {
         const JoinRows join{plan->piece_long, plan->long_row, plan->first_slot, plan->ticket};
         const auto launch = [&](auto kernel) {
@@ -869,17 +880,17 @@ void launch_spmm(const drone_spmm_plan *plan, const int *ci, const float *v, con
                 plan->partial, plan->ldp, join, plan->num_chunks, plan->chunk, plan->chunk_rows, rows, ci, v, B, ldb, K, slice_bits);
         };
         if (plan->ticket) {
-            launch(spmm_gather_kernel<G, VEC, true>);
+            launch(spmm_gather_kernel<G, VEC, kMost, true>);
             return;
         }
-        launch(spmm_gather_kernel<G, VEC, false>);
+        launch(spmm_gather_kernel<G, VEC, kMost, false>);
     } else {
         if (piece_blocks > 0)
             spmm_pieces_kernel<G, VEC><<<(unsigned)piece_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
                 plan->num_pieces, plan->piece_begin, plan->piece_end, plan->piece_slot, plan->ci2, plan->val2, B, ldb,
                 plan->partial, plan->ldp, K, slice_bits);
         if (chunk_blocks > 0)
-            spmm_chunks_kernel<G, VEC><<<(unsigned)chunk_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
+            spmm_chunks_kernel<G, VEC, DEEP && G >= 16 ? 8 : 4><<<(unsigned)chunk_blocks << slice_bits, kWave * kRowsPerBlock, 0, s>>>(
                 plan->num_chunks, plan->chunk, plan->chunk_rows, rows, ci, v, B, ldb, K, slice_bits);
     }
     if (plan->num_long > 0) {  // also when every entry of the long rows went to the dense part: C = beta * C there
@@ -1255,10 +1266,12 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
     DRONE_HIP_TRY(hipStreamSynchronize(s));
     DRONE_REQUIRE(h_rp[0] == 0 && h_rp[n_rows] == nnz, "row_ptr does not span [0, nnz]");
     std::vector<int> long_row;
+    int longest = 0;  // of the others
     for (int r = 0; r < n_rows; ++r) {
         const int len = h_rp[r + 1] - h_rp[r];
         DRONE_REQUIRE(len >= 0, "row_ptr must be non-decreasing");
         if (len > kSplitRow) long_row.push_back(r);
+        else longest = std::max(longest, len);
     }
     // chunks of the short rows
     std::vector<int4> h_chunk;
@@ -1308,6 +1321,7 @@ int plan_create(drone_spmm_plan **out, int n_rows, int n_cols, int64_t nnz, cons
         p->max_k = max_k;
         p->scaled = scaled;
         p->num_chunks = (int)h_chunk.size();
+        p->longest = longest;
         p->ldp = (max_k + 3) / 4 * 4;
         if (p->num_chunks > 0) {
             const auto upload = [&]() -> int {
@@ -1475,12 +1489,18 @@ extern "C" int drone_spmm_csr_f32(const drone_spmm_plan *plan, const int *rp, co
         DRONE_HIP_TRY(hipEventRecord(plan->bits.join, plan->bits.side));
     }
     if (K < 4) {
-        launch_spmm<4, 1>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
+        launch_spmm<4, 1, false>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, 0, s);
     } else {
         const bool whole_lines = ldb % kLineFloats == 0 && (uintptr_t)B % (4 * kLineFloats) == 0;
-        const Slicing by = slicing(K, plan->n_cols, whole_lines, (int64_t)plan->num_pieces + plan->num_chunks,
+        const int64_t waves = (int64_t)plan->num_pieces + plan->num_chunks;
+        const Slicing by = slicing(K, plan->n_cols, whole_lines, waves,
                                    ceil_div(plan->num_pieces, kRowsPerBlock) + ceil_div(plan->num_chunks, kRowsPerBlock), kWave * kRowsPerBlock);
-        const auto launch = [&](auto group) { launch_spmm<decltype(group)::value, 4>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s); };
+        const bool deep = plan->longest >= kDeepRow && (waves << by.bits) <= kResidentWaves && (by.lanes > 8 || by.bits > 0);
+        const auto launch = [&](auto group) {
+            constexpr int G = decltype(group)::value;
+            if (G > 4 && deep) launch_spmm<G, 4, (G > 4)>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s);
+            else launch_spmm<G, 4, false>(plan, ci, v, B, ldb, C, ldc, K, alpha, beta, by.bits, s);
+        };
         if (by.lanes == 4) launch(std::integral_constant<int, 4>());
         else if (by.lanes == 8) launch(std::integral_constant<int, 8>());
         else if (by.lanes == 16) launch(std::integral_constant<int, 16>());

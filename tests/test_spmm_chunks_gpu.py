@@ -48,6 +48,41 @@ def test_chunks(name, lengths):
         plan.close()
 
 
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("rows", [4_500, 12_000, 24_000])
+@pytest.mark.parametrize("longest", [339, 340, 512])
+def test_longest_unsplit_row(longest, rows, split):
+    """Either side of the line at which unsplit rows have more loads in flight, with and without split rows beside them, in lane groups of 8 to 32: a row's sum is
+    taken in the same order either way, so the rows that two matrices share come out the same, bit by bit, and all of them right."""
+    import scipy.sparse
+    import torch
+    from drone_amd import gcn
+    rng = np.random.default_rng(rows)
+    n_cols = 2_000
+    lengths = rng.integers(0, 30, rows)
+    lengths[::29] = rng.integers(65, 338, len(lengths[::29]))
+    lengths[3], lengths[7], lengths[11] = 0, 64, 1_100 if split else 5
+    at = lengths[:3].sum()
+    ci, val = rng.integers(0, n_cols, lengths.sum()).astype(np.int32), rng.uniform(-1, 1, lengths.sum()).astype(np.float32)
+    row_ci, row_val = rng.integers(0, n_cols, 512).astype(np.int32), rng.uniform(-1, 1, 512).astype(np.float32)
+    for K in (23, 37, 64, 100, 128):
+        H = rng.uniform(-1, 1, (n_cols, K)).astype(np.float32)
+        got = []
+        for lengths[3] in (longest, 338):
+            rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+            c = np.insert(ci, at, row_ci[:lengths[3]])
+            v = np.insert(val, at, row_val[:lengths[3]])
+            dev = [torch.from_numpy(a).cuda() for a in (rp, c, v)]
+            plan = gcn.SpmmPlan(*dev, n_cols, K)
+            got.append(gcn.spmm(plan, *dev, torch.from_numpy(H).cuda()).cpu().numpy())
+            plan.close()
+            want = scipy.sparse.csr_matrix((v.astype(np.float64), c, rp), (rows, n_cols)) @ H.astype(np.float64)
+            size = scipy.sparse.csr_matrix((np.abs(v).astype(np.float64), c, rp), (rows, n_cols)) @ np.abs(H).astype(np.float64)
+            assert np.all(np.abs(got[-1] - want) <= (lengths[:, None] + 12) * 2.0 ** -24 * size), K  # as above
+        others = np.arange(rows) != 3
+        np.testing.assert_array_equal(got[0][others], got[1][others])
+
+
 @pytest.mark.parametrize("longest", [3, 1_500])
 def test_plan_is_whole_when_it_is_handed_out(longest):
     """Nothing of a plan is still being made on its stream when the call returns, with and without long rows: products may be on any other."""
