@@ -10,17 +10,19 @@
 //  * One wavefront a SIMD: with two the same loops, which then issue the same loads and matrix instructions in all, take 1.6 times as long
 //    (18.8 / 30.8 us per 30,720 rows of 320 x 100; the matrix instructions alone 17.3).
 //  * With the rows in the L2 a block may be small, which leaves few splits and partial sums: 6 of 32 x 32 blocks against 25 of 64 x 64.
-//  * Three groups of 16 rows in flight (two: 5 % slower on blocks of up to 8 tiles).
+//  * Three groups of 16 rows in flight (two: 5 % slower on blocks of up to 8 tiles), two of the larger blocks, as the registers allow.
 // us with the sum of the splits, before (four kernels, the reduction of a block shared by 8 or 16 wavefronts, or staged through LDS) / now: 320 x 100
 // over 30,011 rows 36.6 / 32.2, 1,536 x 64 over 2,708 17.2 / 12.4, 480 x 40 over 189,106 148 / 96, 128 x 41 over 232,965 47 / 36,
-// 640 x 128 over 232,965 337 / 341, 62 x 8 over 71,791 17.8 / 9.7, 100 x 50 over 45,000 25.2 / 14.7, 602 x 300 over 100,000 437 / 339, 1,000 x
+// 640 x 128 over 232,965 324 / 297, 62 x 8 over 71,791 17.8 / 9.7, 100 x 50 over 45,000 25.2 / 14.7, 602 x 300 over 100,000 432 / 316, 1,000 x
 // 1,000 over 5,000 106 / 94; 94 shapes, mostly of two-layer models, 1.27 times as fast in the mean.  Bound by the matrix pipe and by the L1, which
 // overlap in part (the estimate below); small ones by a launch and a few round trips.
 //
 // Sums: a wavefront's matrix instructions add row after row to one accumulator, whose rounding errors grow with the length of such a chain.  Every
-// 16, 48 or 64 rows the accumulators are added to a second set and the next chain starts from zero (not in the largest blocks, which
-// leave no registers for it, and whose reductions had chains as long before).  Error against double, before / now: 2.4e-7 / 1.7e-7, 1.6e-7 / 1.5e-7,
-// 5.0e-7 / 1.8e-7, 2.6e-7 / 1.8e-7, 8.6e-7 / 8.8e-7, 1.9e-7 / 1.4e-7, 1.8e-7 / 1.6e-7, 9.8e-7 / 9.0e-7, 4.5e-7 / 1.7e-7 for the shapes above.
+// 16, 48 or 64 rows the accumulators are added to a second set and the next chain starts from zero; in blocks of 32 tiles, whose loop is not unrolled
+// that far, every 384 rows, as a pass of its own that takes a 100th of their matrix instructions' time.  (These blocks had one chain of all rows of a split's
+// quarter, 2,336 for 640 x 128 over 232,965, and three groups in flight, of which the second set leaves two: 310 / 297 us, and with the second set in
+// LDS 321).  Error against double, before / now, normal operands: 2.4e-7 / 1.7e-7, 1.6e-7 / 1.5e-7, 5.0e-7 / 1.8e-7, 2.6e-7 / 1.8e-7, 8.6e-7 / 3.6e-7, 1.9e-7 / 1.4e-7,
+// 1.8e-7 / 1.6e-7, 9.7e-7 / 3.6e-7, 4.5e-7 / 1.7e-7 for the shapes above; 1,358 x 235 over 73,123 1.0e-6 / 3.6e-7, operands of one sign 1.8e-7 / 4.9e-8.
 #pragma once
 #include "gemm_direct.h"
 
@@ -28,19 +30,20 @@ namespace drone {
 namespace {
 
 constexpr int kGradWaves = 4;
-constexpr int grad_depth(int tiles) { return tiles == 16 ? 2 : 3; }  // groups of 16 rows in flight, as the registers allow
-constexpr bool grad_chains(int tiles) { return tiles <= 16; }         // a second set of accumulators fits
+constexpr int grad_depth(int tiles) { return tiles >= 16 ? 2 : 3; }  // groups of 16 rows in flight, as the registers allow
+constexpr int grad_waves(int tiles) { return tiles <= 16 ? 2 : 1; }   // a SIMD, as the registers allow
 constexpr int kGradXcds = 8;
+constexpr int kGradChain = 24;  // groups a chain in blocks of 32 tiles
 
 // (Registers for two wavefronts a SIMD where they suffice: with more of them the compiler keeps the sums in accumulation registers, and adding to
 // them takes three instructions.)
 template <int MT, int NT>
-__global__ __launch_bounds__(kGradWaves * kWave) __attribute__((amdgpu_waves_per_eu(grad_chains(MT * NT) ? 2 : 1, grad_chains(MT * NT) ? 2 : 1))) void
+__global__ __launch_bounds__(kGradWaves * kWave) __attribute__((amdgpu_waves_per_eu(grad_waves(MT * NT), grad_waves(MT * NT)))) void
 sgemm_grad_kernel(int M, int N, int K, float alpha, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb, float beta,
                   float *__restrict__ C, int ldc, int k_chunk, int splits, float *__restrict__ partial)
 {
     constexpr int RP = 16 * MT, CP = 16 * NT, D = grad_depth(MT * NT);
-    constexpr bool kChains = grad_chains(MT * NT);
+    constexpr bool kShortChains = MT * NT <= 16;  // which end inside a round of the unrolled loop
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int x = lane & 15, q = lane >> 4;
     // work-group blockIdx.x runs on XCD blockIdx.x % 8, which takes `per` consecutive (split, block)
@@ -51,14 +54,11 @@ sgemm_grad_kernel(int M, int N, int K, float alpha, const float *__restrict__ A,
     const int split = at / blocks, block = at - split * blocks;
     const int m0 = block / col_blocks * RP, n0 = block % col_blocks * CP;
     const int kb = split * k_chunk, ke = kb + k_chunk < K ? kb + k_chunk : K;
-    direct_f4 acc[MT][NT], sum[kChains ? MT : 1][kChains ? NT : 1];
+    direct_f4 acc[MT][NT], sum[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            acc[i][t] = direct_f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (kChains) sum[i][t] = acc[i][t];
-        }
+        for (int t = 0; t < NT; ++t) acc[i][t] = sum[i][t] = direct_f4{0.0f, 0.0f, 0.0f, 0.0f};
     DirectOperand<MT, false> oa;
     DirectOperand<NT, false> ob;
     oa.init(A, lda, m0, M, x, q);
@@ -74,28 +74,27 @@ sgemm_grad_kernel(int M, int N, int K, float alpha, const float *__restrict__ A,
                     acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][j], b[t][j], first && j == 0 ? direct_f4{0.0f, 0.0f, 0.0f, 0.0f} : acc[i][t], 0, 0, 0);
     };
     const auto end_chain = [&]() {
-        if constexpr (kChains)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int t = 0; t < NT; ++t) sum[i][t] += acc[i][t];
+            for (int t = 0; t < NT; ++t) sum[i][t] += acc[i][t];
     };
     // whole groups of 16 rows are dealt out evenly to the wavefronts, the partial group goes to the last of them
     const int groups = (ke - kb) / 16;
     const int g0 = (int)((long long)groups * wave / kGradWaves), g1 = (int)((long long)groups * (wave + 1) / kGradWaves);
     float a[D][MT][4], b[D][NT][4];
     const auto reduce = [&](auto length) {  // of a chain, in groups
-        constexpr int kRound = kChains ? (D + decltype(length)::value - 1) / decltype(length)::value * decltype(length)::value : D;
-        const auto starts = [](int r) { return kChains && r % decltype(length)::value == 0; };
+        constexpr int kRound = kShortChains ? (D + decltype(length)::value - 1) / decltype(length)::value * decltype(length)::value : D;
+        const auto starts = [](int r) { return kShortChains && r % decltype(length)::value == 0; };
         const auto fetch = [&](int d, int g) {  // the last group once more instead of one behind it
             oa.load(kb + 16 * (g < g1 ? g : g1 - 1), a[d]);
             ob.load(kb + 16 * (g < g1 ? g : g1 - 1), b[d]);
         };
 #pragma unroll
         for (int d = 0; d < D; ++d) fetch(d, g0 + d);
-        static_assert(kRound % D == 0, "a group's registers are the same in every round");
+        static_assert(kRound % D == 0 && kGradChain % D == 0, "a group's registers are the same in every round");
         int g = g0;
-        for (; g + kRound <= g1; g += kRound) {
+        const auto round = [&]() {
 #pragma unroll
             for (int r = 0; r < kRound; ++r) {
                 // (the barriers keep the compiler from moving a group's loads down to their use)
@@ -105,17 +104,30 @@ sgemm_grad_kernel(int M, int N, int K, float alpha, const float *__restrict__ A,
                 fetch(r % D, g + r + D);
                 if (starts(r + 1)) end_chain();
             }
+        };
+        if constexpr (kShortChains) {
+            for (; g + kRound <= g1; g += kRound) round();
+        } else {
+            while (g + kRound <= g1) {
+                const int end = g + kGradChain < g1 ? g + kGradChain : g1;
+                for (; g + kRound <= end; g += kRound) round();
+                end_chain();
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[i][t] = direct_f4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
         }
 #pragma unroll
         for (int r = 0; r < kRound; ++r)
             if (g + r < g1) {
                 multiply(a[r % D], b[r % D], starts(r));
                 if (r + D < kRound) fetch(r % D, g + r + D);
-                if (starts(r + 1) || g + r + 1 == g1) end_chain();
+                if (kShortChains && (starts(r + 1) || g + r + 1 == g1)) end_chain();
             }
     };
-    // A chain is a group where a wavefront has a dozen of them or fewer, else three or four, whose end takes a twentieth of the time of their
-    // matrix instructions.
+    // A short chain is a group where a wavefront has a dozen of them or fewer, else three or four, whose end takes a twentieth of the time of
+    // their matrix instructions.
     if (g0 < g1) {
         constexpr int kChain = D == 2 ? 4 : 3, kShort = MT * NT <= 8 ? 1 : kChain;
         if (kShort < kChain && g1 - g0 <= 12) reduce(std::integral_constant<int, kShort>());
@@ -124,16 +136,17 @@ sgemm_grad_kernel(int M, int N, int K, float alpha, const float *__restrict__ A,
     if (wave == kGradWaves - 1 && kb + 16 * groups < ke) {
         oa.load_tail(kb + 16 * groups, ke, q, a[0]);
         ob.load_tail(kb + 16 * groups, ke, q, b[0]);
-        multiply(a[0], b[0], kChains);
-        end_chain();
+        multiply(a[0], b[0], kShortChains);
+        if (kShortChains) end_chain();
     }
+    if (!kShortChains) end_chain();
     extern __shared__ float s_tile[];  // [wavefront][MT * NT][4][64]: the sums as they lie
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) s_tile[((wave * MT * NT + i * NT + t) * 4 + v) * kWave + lane] = kChains ? sum[kChains ? i : 0][kChains ? t : 0][v] : acc[i][t][v];
+            for (int v = 0; v < 4; ++v) s_tile[((wave * MT * NT + i * NT + t) * 4 + v) * kWave + lane] = sum[i][t][v];
     __syncthreads();
     // Register v of lane x + 16 q of tile (i, t) is row position 4 q + v and column position x of the tile.  Columns fastest, so
     // that C is written in runs of consecutive lanes.
