@@ -1389,8 +1389,8 @@ struct SmallRounds {
 // piles, as Davidson, Baxter, Garland and Owens, 2014, split delta-stepping's buckets), by a step that is doubled while lists are shorter than a quarter of the
 // lanes and halved when one is longer than the lanes: 1.4 times every edge, 100 a round.  Sums of whole numbers have the same least fixed point in any order, so the distances
 // are the same bits.  Every move of the threshold settles the nearest waiting vertex, as no length is negative: it ends.
-// A list that would be too long is cut, and what it leaves waits too.  A vertex with more edges than a list may have ends it, and so do n rounds: all go
-// back on the call's list, and the launch ends.  What bounds a round (2 us) is its chain of loads - target and length, then value, row bounds and flag - and two
+// A list that would be too long is cut, and what it leaves waits too.  A vertex with more edges than a list may have waits until no other goes on the list in
+// front of it, which ends it, and so do n rounds: all go back on the call's list, and the launch ends.  What bounds a round (2 us) is its chain of loads - target and length, then value, row bounds and flag - and two
 // barriers.  ms by rounds over all / this, lengths 1 ... 16: a 23 x 846 grid 9.8 / 2.4, 50 x 900 12.0 / 3.1, 100 x 500 7.1 / 2.5, 5 x 2,000 14.3 / 4.6, 12 x 200
 // 0.78 / 0.58, 200 x 300 4.7 / 3.6; where a lone wavefront suffices it stays with it (a path of 10,000 3.96 / 4.03).
 struct NearRounds {
@@ -1575,6 +1575,10 @@ struct NearRounds {
                 s_lows[next] = 0;
             }
             __syncthreads();
+            if (tid == 0) {  // the empty list too (everyone has seen that it is): one that is cut before its first entry has counted what found no room
+                s_list[now] = 0ull;
+                s_cut[now] = ~0ull;
+            }
             for (int i = tid; i < fars; i += T) {
                 const int v = far[i];
                 if (waits[v] != i + 1) continue;

@@ -63,6 +63,33 @@ def test_long_path_lowered_twice(oracle, edges):
         w.close()
 
 
+def test_list_cut_before_its_first_entry(oracle):
+    """A vertex with more edges than a list may have, lowered alone while another waits, leaves a list of none.  The rounds of the nearest go on with the other one's path, a round a
+    hop, and the large vertex comes last, by the other rounds: a list that still counted it would have no room for the path, and the large vertex's turn would come first."""
+    from drone_amd.traverse import SSSPWorkerCUDA
+    fan, way, tail, leaves = 64 + np.arange(100), 164 + np.arange(6), 170 + np.arange(500), 670 + np.arange(2_100)
+    hub, far = way[-1], fan[-1]
+    u = np.concatenate([np.arange(63), np.full(100, 63), fan, way[:-1], np.full(2_100, hub), tail[:-1]]).astype(np.int32)
+    v = np.concatenate([np.arange(1, 64), fan, [way[0]], np.zeros(98), [tail[0]], way[1:], leaves, tail[1:]]).astype(np.int32)
+    nglobal = 670 + 2_100
+    n, g2l, l2g, index, dst = oracle.build_graph(nglobal, u, v)
+    length = np.ones(len(dst), np.float32)
+    length[[e for e in range(index[g2l[63]], index[g2l[63] + 1]) if l2g[dst[e]] == far]] = 1 << 20  # waits while the others are done
+    length[index[g2l[0]]] = 2.0  # (not all are 1)
+    st = oracle.SSSPState(index, dst, length)
+    st.peval(int(g2l[0]))
+    w = SSSPWorkerCUDA(nglobal, u, v, startId=0)
+    try:
+        w.set_edge_len(length)
+        for _ in range(2):
+            w.peval()
+            np.testing.assert_array_equal(w.read(), st.val)
+            round_of = w.flags()["active"]
+            assert round_of[g2l[leaves]].min() > round_of[g2l[tail[-1]]]
+    finally:
+        w.close()
+
+
 CASES = {
     "grid_3": (lambda: _grid(3, 300), 1, 17), "grid_23": (lambda: _grid(23, 211), 1, 17), "grid_120": (lambda: _grid(120, 130), 1, 17),
     "grid_600": (lambda: _grid(600, 60), 1, 17),           # lists that are cut
