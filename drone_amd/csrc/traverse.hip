@@ -1803,6 +1803,9 @@ unsigned long long push_limit(const GraphExt *x) { return std::max((unsigned lon
 // grid 16.5 -> 13.2 ms; 100,000 vertices, 1.3 M edges 204 -> 228 us, where a list of most edges costs more in atomics.  (Over other
 // lengths a sweep takes improvements along that a push leaves, so there what was swept stays swept.)
 constexpr unsigned long long kPushAll = 1ull << 19;
+// near_rounds_kernel may change the list and its mark behind the host's back, in front of rounds that the host has chosen by what it knew: pushes and the small rounds
+// look for themselves, a sweep would run with a mark that has passed.  No list of a graph that near_hold() takes is too long to be pushed, so none is chosen.
+static_assert(kNearBytes / 8 < (int64_t)kPushAll, "graphs whose nearest vertices go first have lists that are pushed");
 unsigned long long push_limit_whole(const GraphExt *x) { return (unsigned long long)x->edges <= kPushAll ? kPushAll : push_limit(x); }
 
 // List 0 <- the vertices with active == value.
