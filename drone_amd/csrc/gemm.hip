@@ -440,10 +440,13 @@ __global__ __launch_bounds__(tall_waves(KQ, NT) * kWave) void sgemm_tall_kernel(
 }
 
 // Grow-only scratch for split-K partials, one per (device, stream): calls on one stream are ordered, so they can
-// share a buffer; calls on different streams may overlap and get their own.
+// share a buffer; calls on different streams may overlap and get their own.  It grows under stream capture too: there nothing may be waited
+// for, so what earlier calls may still read stays allocated, and a buffer that a graph was given stays for the graph's replays.  Such growth at least
+// doubles, so what stays is less than what is in use.
 struct SplitScratch {
     float *ptr = nullptr;
     size_t bytes = 0;
+    bool recorded = false;  // allocated under capture
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, SplitScratch> g_ws;
@@ -455,13 +458,24 @@ int workspace(size_t bytes, hipStream_t s, float **out)
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     SplitScratch &w = g_ws[std::make_pair(dev, s)];
     if (w.bytes < bytes) {
-        if (w.ptr) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();  // the null stream beside another's capture: not recorded itself
+        const bool capturing = status != hipStreamCaptureStatusNone;
+        if (capturing || w.recorded) {
+            bytes = std::max(bytes, 2 * w.bytes);
+        } else if (w.ptr) {
             DRONE_HIP_TRY(hipStreamSynchronize(s));  // earlier calls on this stream may still read it
             (void)hipFree(w.ptr);
             w = SplitScratch{};
         }
-        DRONE_HIP_TRY(hipMalloc(&w.ptr, bytes));
-        w.bytes = bytes;
+        float *p = nullptr;
+        // an allocation is no part of the graph: the thread's mode lets it through while others record in theirs
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (capturing) DRONE_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t allocated = hipMalloc(&p, bytes);
+        if (capturing) DRONE_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        DRONE_HIP_TRY(allocated);
+        w = SplitScratch{p, bytes, capturing};
     }
     *out = w.ptr;
     return DRONE_OK;

@@ -213,8 +213,9 @@ int drone_pr_run_workers_f64(Graph *g, PRValues *values, int workerId, int worke
  * drone_cross_entropy_f32 / drone_loss_pass_f32, nothing allocates; calls on different streams may overlap, except that two products with
  * the SAME plan share the plan's partial-row scratch and must not run at the same time.  drone_spmm_csr_f32 only
  * launches kernels and records / waits for events between `stream` and the plan's own side stream, so it can be
- * recorded into a HIP graph on a capturing stream (drone_sgemm_rm_f32 as well once its scratch has grown to the
- * shape, drone_sgemm_rm_f32_noalloc always). */
+ * recorded into a HIP graph on a capturing stream (drone_sgemm_rm_f32 as well, whose scratch then grows by an allocation
+ * that stays for the graph's replays; where it has grown before the capture, let no larger product run on the stream while the
+ * graph is in use: that would replace the scratch). */
 
 /* cuda_gcn/src/cuda/cuda_kernel.cu:145-155 (launched at cuda_module.cu:163):
  * v[e(u->col)] = 1 / sqrtf(1.0 * out_deg[u] * in_deg[col]) for every entry of row u. */

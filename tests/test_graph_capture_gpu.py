@@ -119,3 +119,37 @@ def test_first_loss_on_a_stream_is_recorded(T):
         result()
         graph.replay()
         result()
+
+
+@pytest.mark.parametrize("M,N,K", [(1_317, 194, 1_792), (128, 41, 60_001)])
+def test_first_split_product_on_a_stream_is_recorded(T, M, N, K):
+    """The first product of a stream whose reduction is split is recorded: its scratch is allocated under the capture, and stays where it is when a larger product
+    asks for more."""
+    from drone_amd import gcn
+    gen = T.Generator(device="cuda").manual_seed(M)
+    A, B = T.randn(K, M, generator=gen, device="cuda"), T.randn(K, N, generator=gen, device="cuda")
+    A2, B2 = T.randn(30_011, 640, generator=gen, device="cuda"), T.randn(30_011, 200, generator=gen, device="cuda")
+    A3, B3 = T.cat([A2, A2], 1), T.cat([B2, B2], 1)
+    want, want2, want3 = (gcn.sgemm(True, False, *ab) for ab in ((A, B), (A2, B2), (A3, B3)))
+    out, out2 = T.zeros(M, N, device="cuda"), T.zeros(640, 200, device="cuda")
+    out3 = T.zeros(1_280, 400, device="cuda")
+    T.cuda.synchronize()
+    side, graph, second = T.cuda.Stream(), T.cuda.CUDAGraph(), T.cuda.CUDAGraph()
+    with T.cuda.graph(graph, stream=side):
+        gcn.sgemm(True, False, A, B, out=out, stream=side.cuda_stream)
+    with T.cuda.graph(second, stream=side):
+        gcn.sgemm(True, False, A2, B2, out=out2, stream=side.cuda_stream)
+    with T.cuda.stream(side):  # all of it in order
+        for _ in range(3):
+            graph.replay()
+            side.synchronize()
+            assert T.equal(out, want)
+            out.zero_()
+            second.replay()
+            gcn.sgemm(True, False, A, B, out=out, stream=side.cuda_stream)
+            side.synchronize()
+            assert T.equal(out2, want2) and T.equal(out, want)
+            out.zero_(), out2.zero_()
+            gcn.sgemm(True, False, A3, B3, out=out3, stream=side.cuda_stream)
+            side.synchronize()
+            assert T.equal(out3, want3)
