@@ -457,12 +457,13 @@ __global__ __launch_bounds__(kSpmvBlock) void count_not_one_kernel(int n, const 
 
 // sssp.cu:23-38, the list of the first round - the start vertex if this subgraph holds it (sssp.cu:30) and it has out-edges -, and the
 // count of the lengths, which the stores do not wait for.  Distances of 1 M vertices and
-// 13 M edges 129 us with two launches, 121 with one; 20,000 vertices 77 and 69.
-__global__ __launch_bounds__(kSpmvBlock) void sssp_begin_kernel(int n, const int *__restrict__ global_to_local, int start_id, int *__restrict__ active,
-                                                                float *__restrict__ dist, int *__restrict__ ubm, const int *__restrict__ index,
-                                                                int *__restrict__ list, int *__restrict__ offset, int edges,
+// 13 M edges 129 us with two launches, 121 with one; 20,000 vertices 77 and 69.  (The arguments and the launch's size take two lines of 64 bytes, the numbers
+// side by side: a third, which every work-group's last steps read, took 0.2 us of 4.7.)
+__global__ __launch_bounds__(kSpmvBlock) void sssp_begin_kernel(int n, int hold, const int *__restrict__ global_to_local, int start_id, int edges,
+                                                                int *__restrict__ active, float *__restrict__ dist, int *__restrict__ ubm,
+                                                                const int *__restrict__ index, int *__restrict__ list, int *__restrict__ offset,
                                                                 const float *__restrict__ len, double *block_part, unsigned int *ticket,
-                                                                TraverseState *state, int hold)
+                                                                TraverseState *state)
 {
     __shared__ double s_red[kSpmvBlock / kWave];
     const int start = global_to_local[start_id];
@@ -2269,8 +2270,8 @@ extern "C" Response SSSP_PEVal(Graph *g, SSSPValues *values, int startId, int wo
     SsspRun run{g, t, values->distance, s, true};
     const auto begin = [&] {
         sssp_begin_kernel<<<std::max(sum_blocks(n), sum_blocks(x->edges, 16)), kSpmvBlock, 0, s>>>(
-            n, g->Global2Local, startId, g->active, values->distance, g->updateByMessage, g->index, t->lists.vertex[0], t->lists.offset[0], x->edges,
-            g->edgeLen, t->block_part, t->ticket, t->state, near_hold(x));
+            n, near_hold(x), g->Global2Local, startId, x->edges, g->active, values->distance, g->updateByMessage, g->index, t->lists.vertex[0],
+            t->lists.offset[0], g->edgeLen, t->block_part, t->ticket, t->state);
         run.counted = true;
     };
     const bool chains = ensure_chains(g, t, s) && !x->chains.other_lengths;
