@@ -18,7 +18,7 @@
 namespace drone {
 namespace {
 
-constexpr int kFlatWaves = 4;
+constexpr int kFlatWaves = 4, kFlatMost = 24;  // kFlatMost: groups of steps times tiles are fewer
 
 template <int KG, int NT>
 __global__ __launch_bounds__(kFlatWaves * kWave) void sgemm_flat_kernel(int M, int N, int K, bool ascending, float alpha, const float *__restrict__ A,
@@ -130,7 +130,7 @@ bool flat_covers(bool tiled, int M, int N, int K)
 {
     if (K < 1 || K > 64 || N > 128) return false;
     const int n16 = (int)ceil_div(N, 16), tiles = n16 <= 4 ? n16 : n16 <= 6 ? 6 : 8;
-    if (ceil_div(K, 16) * tiles >= 24) return false;
+    if (ceil_div(K, 16) * tiles >= kFlatMost) return false;
     return tiled ? M >= 8000 : M >= 24000 && !(K % 16 == 0 && N <= 16);
 }
 
@@ -140,15 +140,17 @@ void launch_flat(bool tb, bool ascending, int M, int N, int K, float alpha, cons
 {
     const unsigned grid = (unsigned)std::min<int64_t>(KG == 1 ? 1024 : 512, ceil_div(ceil_div(M, 16), kFlatWaves));
     const int n16 = (int)ceil_div(N, 16);
-    const auto go = [&](auto kernel) {
-        kernel<<<grid, kFlatWaves * kWave, 0, s>>>(M, N, K, ascending, alpha, A, lda, B, tb ? 1 : ldb, tb ? ldb : 1, C, ldc);
+    const auto go = [&](auto tiles) {
+        constexpr int NT = decltype(tiles)::value;
+        if constexpr (KG * NT < kFlatMost)
+            sgemm_flat_kernel<KG, NT><<<grid, kFlatWaves * kWave, 0, s>>>(M, N, K, ascending, alpha, A, lda, B, tb ? 1 : ldb, tb ? ldb : 1, C, ldc);
     };
-    if (n16 == 1) go(sgemm_flat_kernel<KG, 1>);
-    else if (n16 == 2) go(sgemm_flat_kernel<KG, 2>);
-    else if (n16 == 3) go(sgemm_flat_kernel<KG, 3>);
-    else if (n16 == 4) go(sgemm_flat_kernel<KG, 4>);
-    else if (n16 <= 6) go(sgemm_flat_kernel<KG, 6>);
-    else go(sgemm_flat_kernel<KG, 8>);
+    if (n16 == 1) go(std::integral_constant<int, 1>());
+    else if (n16 == 2) go(std::integral_constant<int, 2>());
+    else if (n16 == 3) go(std::integral_constant<int, 3>());
+    else if (n16 == 4) go(std::integral_constant<int, 4>());
+    else if (n16 <= 6) go(std::integral_constant<int, 6>());
+    else go(std::integral_constant<int, 8>());
 }
 void sgemm_flat(bool tb, bool ascending, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float *C, int ldc,
                 hipStream_t s)
