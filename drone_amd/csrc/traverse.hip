@@ -1632,7 +1632,7 @@ __global__ __launch_bounds__(kSmallThreads) void near_rounds_kernel(TraverseStat
     const TraverseState start = *state;
     const int tid = threadIdx.x;
     if (start.listed == 0 || start.hold <= 0 || start.rounds < n_all + 2 - start.hold) return;
-    if ((start.listed & 0xFFFFFFFFull) <= (unsigned long long)kWave) {  // a lone wavefront's: to be looked at when as many rounds more have run
+    if ((start.listed & 0xFFFFFFFFull) <= (unsigned long long)kWave) {  // a lone wavefront's: to be looked at when four times as many rounds have run
         if (tid == 0) state->hold = max(n_all + 2 - 4 * start.rounds, 0);
         return;
     }

@@ -1,5 +1,5 @@
-"""Weight gradients (A transposed) on both sides of every line at which their blocks and splits change: 16, 32, 64 and 96 columns, 32
-and 64 rows, 1.5e8 and 5e8 multiply-adds, reductions of a group of 16 steps per wavefront and one more or less."""
+"""Weight gradients (A transposed) from single blocks to many and over short and long reductions, with outputs and reductions of one more or less than
+whole tiles and groups of 16; and forward products in 64-row tiles and over deep reductions."""
 import pytest
 
 from test_gemm_direct_gpu import test_sgemm_direct_edges as _edges
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (64, 30, 255), (64, 17, 256), (65, 32, 127), (65, 31, 129), (65, 32, 4097),      # 16 and 8 wavefronts' shares
+    (64, 30, 255), (64, 17, 256), (65, 32, 127), (65, 31, 129), (65, 32, 4097),
     (32, 33, 2000), (33, 64, 2001), (63, 64, 128), (64, 64, 36_621), (64, 64, 36_622), (64, 63, 36_000),
     (32, 128, 122_071), (33, 128, 118_372), (301, 127, 13_080), (301, 127, 13_079), (317, 115, 13_717), (67, 65, 9_001), (61, 96, 9_000),
     (1400, 100, 3_572), (1400, 128, 127), (16, 16, 257), (17, 16, 255)])
