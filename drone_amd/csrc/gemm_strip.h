@@ -4,13 +4,16 @@
 // the reduction has no barrier and reads it once per 16 rows with 16 bytes a lane; a wavefront owns 16 rows and all columns, padded to 16 and not
 // to 64 or 128, and reads its rows straight from memory, 16 bytes a lane, four groups of 16 steps ahead.  What it took: the fetch of op(B)
 // addressed by scalar registers, a wavefront a block of 16 x 16 at a time (one index per lane took 12 us for 140 KB, this 6), beginning at
-// another place in every work-group, as all ask for the same lines at once; and LDS reads a group ahead of the matrix instructions, kept there
+// another place in every work-group, as all ask for the same lines at once; no branch for columns past op(B) (with N no multiple of 16 all blocks of the last tile,
+// which are one wavefront's where there are eight tiles, took a path of single loads: 31,465 x 224 x 113 28.8 / 22.7); op(B) transposed by 16-byte loads for either order of
+// sums (31,465 x 312 x 116 48.9 / 31.6, by the tiled kernel 31.0); and LDS reads a group ahead of the matrix instructions, kept there
 // by scheduling barriers (21 -> 20 us per 32,768 rows of 320 x 100, of which the matrix instructions are 15).  Two strips a wavefront, 4, 12 or 16
 // wavefronts, 8 groups ahead, op(B) by rows (four times the LDS instructions), one run of groups over the seams between strips: none better
 // over 100 shapes, several worse.
 //
-// us by the kernels that it stands in for / here: 30,011 x 320 x 100 33.0 / 30.9, 64,530 x 96 x 93 28.5 / 22.0, 103,955 x 288 x 84 96 / 69, 121,197 x 192 x 38
-// 42.1 / 32.6, 196,368 x 352 x 30 98 / 63, 208,773 x 576 x 62 208 / 162, 227,087 x 92 x 23 34.6 / 28.5.  Bound by
+// us by the kernels that it stands in for / here: 30,011 x 320 x 100 30.5 / 27.8, 64,530 x 96 x 93 27.2 / 19.5, 103,955 x 288 x 84 90 / 63, 121,197 x 192 x 38
+// 39.5 / 28.7, 196,368 x 352 x 30 91 / 55, 208,773 x 576 x 62 187 / 147, 227,087 x 92 x 23 31.6 / 24.3, transposed 64,593 x 244 x 110 45.7 / 42.0; 680 shapes 1.32 times as fast in the
+// mean, six slower by 2.5 to 5 % (mostly 38,000 to 49,000 rows, where the tiled kernel's rounds come out even, and its 128 columns are all used).  Bound by
 // op(B)'s fetch (a launch and 7 us in front of 140 KB) on few rows, by memory (3.9 TB/s of A and C) or the matrix pipe on many.
 //
 // Sums: one accumulator per output takes the reduction's steps one after the other, as v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 both do (their
@@ -65,11 +68,14 @@ __global__ __launch_bounds__(kStripWaves * kWave) void sgemm_strip_kernel(int M,
     };
     if (first < end) begin(first);  // in flight while op(B) comes
     {
+        // Columns past op(B) read its last one: nobody stores their sums.  Transposed, four steps of a lane are one 16-byte load, brought into order as A's are.
         constexpr int U = 4;
         const int blocks = groups * NT, turn = (int)((blockIdx.x / 8) % 32) * blocks / 32;
-        const int lane_k = ASC ? q : 4 * q;
-        constexpr int kStep = ASC ? 4 : 1;
+        const int lane_k = ASC && !TB ? q : 4 * q;
+        constexpr int kStep = ASC && !TB ? 4 : 1;
+        const int x_last = 16 * (NT - 1) + x < N ? x : N - 1 - 16 * (NT - 1);  // of the last tile
         const float *lane_b = TB ? B + (size_t)x * ldb + lane_k : B + (size_t)lane_k * ldb + x;
+        const float *lane_b_last = TB ? B + (ptrdiff_t)x_last * ldb + lane_k : B + (size_t)lane_k * ldb + x_last;
         for (int b0 = wave; b0 < blocks; b0 += U * kStripWaves) {
             direct_f4 v[U];
             int at[U];
@@ -79,20 +85,27 @@ __global__ __launch_bounds__(kStripWaves * kWave) void sgemm_strip_kernel(int M,
                 b = b + turn < blocks ? b + turn : b + turn - blocks;
                 at[u] = b;
                 const int g = b / NT, t = b - g * NT;
-                if (16 * g + 16 <= K && 16 * t + 16 <= N) {
-                    const float *src = TB ? lane_b + (size_t)(16 * t) * ldb + 16 * g : lane_b + (size_t)(16 * g) * ldb + 16 * t;
+                const float *src = (t < NT - 1 ? lane_b : lane_b_last) + (TB ? (size_t)(16 * t) * ldb + 16 * g : (size_t)(16 * g) * ldb + 16 * t);
+                if (16 * g + 16 <= K) {
+                    if constexpr (TB) {
+                        const DirectF4U r = *reinterpret_cast<const DirectF4U *>(src);
+                        v[u] = direct_f4{r.v[0], r.v[1], r.v[2], r.v[3]};
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[u][j] = src[TB ? (size_t)(kStep * j) : (size_t)(kStep * j) * ldb];
-                } else {
+                        for (int j = 0; j < 4; ++j) v[u][j] = src[(size_t)(kStep * j) * ldb];
+                    }
+                } else {  // the partial group: zeros past the reduction, the last step's element read again instead
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int k = 16 * g + lane_k + kStep * j, n = 16 * t + x;
-                        const int kc = k < K ? k : K - 1, nc = n < N ? n : N - 1;
-                        const float e = TB ? B[(size_t)nc * ldb + kc] : B[(size_t)kc * ldb + nc];
-                        v[u][j] = k < K && n < N ? e : 0.0f;
+                        const int k = 16 * g + lane_k + kStep * j, over = k < K ? 0 : k - (K - 1);
+                        const float e = TB ? src[kStep * j - over] : src[(ptrdiff_t)(kStep * j - over) * ldb];
+                        v[u][j] = k < K ? e : 0.0f;
                     }
                 }
             }
+            if constexpr (TB && ASC)
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = strip_ascending(v[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u) s_strip[at[u] * kWave + lane] = v[u];
         }

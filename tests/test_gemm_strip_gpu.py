@@ -15,3 +15,21 @@ pytestmark = pytest.mark.gpu
     (33_333, 64, 640), (33_333, 64, 641)])
 def test_strips_and_pieces(tb, M, N, K):
     _edges(0, tb, M, N, K)
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(28_001, 113, 353), (64_530, 93, 99)])
+def test_infinities_and_nan_stay_where_they_are(M, N, K, tb):
+    """In op(B)'s first and last step and column, which the kernel reads again in place of what lies past them."""
+    import torch
+    from drone_amd import gcn
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    A, B = torch.rand(M, K, generator=gen, device="cuda") + 0.5, torch.rand(K, N, generator=gen, device="cuda") + 0.5
+    B[K - 1, 3], B[0, 5], B[K - 1, N - 1], B[7, N - 2] = float("inf"), float("nan"), float("-inf"), float("inf")
+    got = gcn.sgemm(0, tb, A, B.t().contiguous() if tb else B)
+    want = torch.full((N,), 1.0, device="cuda")
+    want[3], want[5], want[N - 1], want[N - 2] = float("inf"), float("nan"), float("-inf"), float("inf")
+    special = ~torch.isfinite(want)
+    assert torch.isfinite(got[:, ~special]).all()
+    for j in torch.nonzero(special).view(-1).tolist():
+        assert torch.equal(torch.nan_to_num(got[:, j], nan=1.0, posinf=2.0, neginf=3.0), torch.nan_to_num(want[j], nan=1.0, posinf=2.0, neginf=3.0).expand(M))
